@@ -3,239 +3,362 @@
 // and 8x8x8 vector contracts (ModernTile.cpp:289-296, PrepareModernVec.cpp:43-48) and for which
 // its unfinished CUDA kernel intended a 128x128x8 shared-memory tiling
 // (src/libnncv/kernel/sgemm.cu:13-100).  Nothing of either is reused.
-//
-// Workgroup tile GBM x GBN = 128x128 (four waves of 64x64, 2x2 accumulators of v_mfma_f32_32x32x2_f32) for
-// large problems, 64x64 (four waves of 32x32) when that is what it takes to give each of the 256 CUs a
-// workgroup; K walked 16 at a time through two LDS buffers.
-//  * A 1024^3 product is 256 tiles of 64x64 with 512 dependent 64-cycle MFMAs per wave: one wave per SIMD and
-//    nothing to hide its loads, stores and barriers behind.  Small grids therefore run KG = 2 or 4 "K groups"
-//    per workgroup (512 / 1024 threads): group g takes every KG-th K tile through LDS buffers of its own, the
-//    groups' partial tiles meet in LDS at the end and all threads add them to C in whole 256-byte rows.
-//    The order of that sum is fixed (group 0, 1, ...), so results do not change from run to run.
-//  * A (M x K, K contiguous) is kept in LDS as rows of four 16-byte chunks + one chunk of padding;
-//    a lane reads one chunk (4 consecutive k of its row) per two MFMAs' worth of k.
-//  * B (K x N, N contiguous) is kept k-major exactly as it lies in memory, so the global loads are
-//    coalesced along n and the MFMA operand read (one float per lane, lanes along n) is a
-//    conflict-free 128-byte LDS row segment.
-//  * MFMA k-slot h of lane-half h takes k = 4*(2*kk + h) + j for both operands.
-//  * VEC: K and N multiples of 4 and 16-byte aligned operands -> 16-byte global loads; otherwise element
-//    loads with a bounds check each (any M, N, K; linalg.matmul puts no condition on them).
-#include "common.hpp"
+#include <algorithm>
+
+#include "mfma_tile.hpp"
 
 namespace nncv_hip {
 
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
+using mt::floatx16;
+using mt::floatx4;
+using mt::u32x4;
 
+namespace {
 
-// K tile of a round: 16 without K groups; 32 with them (a round then ends at a barrier of up to sixteen waves that all
-// start the next one by waiting for their first operands: fewer, longer rounds)
-constexpr int gemm_bk(int kg) { return kg > 1 ? 32 : 16; }
-constexpr int gemm_arow(int kg) { return (gemm_bk(kg) + 4) * 4; }  // bytes of an A row in LDS: the K tile + 16 bytes of padding
-constexpr int gemm_group_lds(int gbm, int gbn, int kg) { return 2 * gbm * gemm_arow(kg) + 2 * gemm_bk(kg) * (gbn + 4) * 4; }
-constexpr int gemm_lds(int gbm, int gbn, int kg) {
-  const int tiles = kg * gemm_group_lds(gbm, gbn, kg), red = kg > 1 ? kg * gbm * gbn * 4 : 0;
-  return tiles > red ? tiles : red;
+// One wave owns TM x TN accumulators of BT x BT (BT = 32: v_mfma_f32_32x32x2_f32, 16: v_mfma_f32_16x16x4_f32, both 256
+// flops a cycle and CU) and feeds them straight from memory: fp32 matrix instructions are so slow (64 / 32 cycles) that a wave
+// needs only 4-5 KB of operands per 1024 cycles (a fifth of the CU's 64 B/clk), and with no LDS tile there is no
+// barrier, no store pass and no wave that waits for another.
+//  * A (K contiguous): lane l holds row l % BT; a 16-byte load along k is the operand of four MFMAs (lane group h = l / BT
+//    takes k = QK q + 4 h + e, QK = 256 / BT).  The loads that cover a row's 128-byte line go out together, one round (32 k) ahead.
+//  * B (N contiguous): the MFMA columns are dealt to lanes so that lane l holds columns TN l .. TN l + TN - 1: one 4 or 8
+//    byte load of row k is the operand of TN accumulators, whole rows of 4 BT TN contiguous bytes per lane group.  C is
+//    read and written the same way.
+//  * Nothing asks for alignment beyond 4 bytes, so odd K and N (rows that do not start on 16 bytes) take the same loads.
+//    Only the last 32 k of the matrix can hold k >= K or leave the buffers; the group that owns them walks them FIRST,
+//    with A masked (B's rows past the end come back as zeros from the range check), so the main loop masks nothing.
+//    Rows m >= M read row M - 1 and columns n >= N read the next row: both only reach results that are not stored.
+//  * KG "K groups": waves of a workgroup that share a tile of C and split K.  Their sums meet in LDS, in a fixed order
+//    (results do not change from run to run), and every wave adds its share of rows to C, requested before the loop.
+template <int BT, int TM, int TN, int WM, int WN, int KG>
+struct GemmCfg {
+  static constexpr int kWaves = WM * WN * KG, kRows = BT * TM * WM, kCols = BT * TN * WN;
+  static constexpr int kAcc = BT * BT / 64;  // accumulator registers of a BT x BT block
+  static constexpr int kLds = KG > 1 ? KG * WM * WN * TM * TN * BT * BT * 4 : 0;
+};
+
+template <int TN>
+struct Vec { typedef float type __attribute__((ext_vector_type(TN))); };
+template <>
+struct Vec<1> { typedef float type; };
+
+template <int BT>
+struct Mma32;
+template <>
+struct Mma32<32> {
+  typedef floatx16 acc;
+  static __device__ __forceinline__ acc run(float a, float b, acc c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
+};
+template <>
+struct Mma32<16> {
+  typedef floatx4 acc;
+  static __device__ __forceinline__ acc run(float a, float b, acc c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+};
+
+template <int TN>
+__device__ __forceinline__ void load_row(__amdgpu_buffer_rsrc_t rs, unsigned voff, float (&b)[TN]) {
+  if constexpr (TN == 1) {
+    b[0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, voff, 0, 0));
+  } else {
+    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+    static_assert(TN == 2, "a lane holds one or two columns");
+    const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rs, voff, 0, 0);
+    const typename Vec<2>::type f = __builtin_bit_cast(typename Vec<2>::type, v);
+    b[0] = f[0];
+    b[1] = f[1];
+  }
 }
 
-template <int GBM, int GBN, int KG, bool VEC>
-__global__ __launch_bounds__(256 * KG) void gemm_nn_f32_kernel(const float* __restrict__ A, const float* __restrict__ B,
-                                                               float* __restrict__ C, int M, int N, int K) {
-  constexpr int GBK = gemm_bk(KG), kARow = gemm_arow(KG);
-  constexpr int kBRow = (GBN + 4) * 4;  // bytes: GBN floats + 4 pad (keeps 16-byte alignment)
-  constexpr int TM = GBM / 64, TN = GBN / 64;
-  constexpr int KQ = GBK / 16;  // 16-wide K quarters of a tile: the loader and the MFMA loop walk them one by one
-  constexpr int WTM = GBM / 2, WTN = GBN / 2;  // wave tile
-  constexpr int BROWS = 256 / (GBN / 4);       // B rows covered by one pass of the loader
-  static_assert(KG == 1 || (GBM == 64 && GBN == 64), "K groups go with the 64x64 tile");
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int grp = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8);
-  const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
-  unsigned char* sA = smem + grp * gemm_group_lds(GBM, GBN, KG);  // [2][GBM * kARow]
-  unsigned char* sB = sA + 2 * GBM * kARow;                   // [2][GBK * kBRow]
-  const int wm = wave & 1, wn = wave >> 1;
-  const int m0 = blockIdx.y * GBM, n0 = blockIdx.x * GBN;
+// bytes from element `at` to the end of an `elems`-element array, as a buffer descriptor's size
+__device__ __forceinline__ unsigned bytes_left(long long elems, long long at) {
+  const long long b = (elems - at) * 4;
+  return b > 0xffffffffll ? 0xffffffffu : (unsigned)b;
+}
 
-  // loader mapping. A: GBM rows x 4 chunks, TM per thread (rows ar + 64 i).
-  const int ack = tid & 3, ar = tid >> 2;
-  // B: 16 rows x GBN/4 float4, TN per thread (rows br + BROWS i).
-  const int bc4 = tid % (GBN / 4), br = tid / (GBN / 4);
-
-  floatx4 ra[KQ][TM], rb[KQ][TN];
-  auto load = [&](int k00) {
-#pragma unroll
-    for (int q = 0; q < KQ; ++q) {
-      const int k0 = k00 + 16 * q;
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int m = m0 + ar + 64 * i, k = k0 + ack * 4;
-        if constexpr (VEC) {
-          ra[q][i] = (m < M && k < K) ? *reinterpret_cast<const floatx4*>(A + (long long)m * K + k) : floatx4{0, 0, 0, 0};
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) ra[q][i][e] = (m < M && k + e < K) ? A[(long long)m * K + k + e] : 0.0f;
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < TN; ++i) {
-        const int kb = k0 + br + BROWS * i, n = n0 + bc4 * 4;
-        if constexpr (VEC) {
-          rb[q][i] = (kb < K && n < N) ? *reinterpret_cast<const floatx4*>(B + (long long)kb * N + n) : floatx4{0, 0, 0, 0};
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) rb[q][i][e] = (kb < K && n + e < N) ? B[(long long)kb * N + n + e] : 0.0f;
-        }
-      }
-    }
-  };
-  auto store = [&](int buf) {
-#pragma unroll
-    for (int q = 0; q < KQ; ++q) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i) *reinterpret_cast<floatx4*>(sA + buf * GBM * kARow + (ar + 64 * i) * kARow + q * 64 + ack * 16) = ra[q][i];
-#pragma unroll
-      for (int i = 0; i < TN; ++i)
-        *reinterpret_cast<floatx4*>(sB + buf * GBK * kBRow + (16 * q + br + BROWS * i) * kBRow + bc4 * 16) = rb[q][i];
-    }
-  };
-
-  // K groups: the four values of C this thread adds to at the end are requested now
-  floatx4 cpre = {0, 0, 0, 0};
-  if constexpr (KG > 1 && VEC) {
-    const int e = threadIdx.x;
-    if (e < 64 * 16) {
-      const int gm = m0 + (e >> 4), gn = n0 + (e & 15) * 4;
-      if (gm < M && gn + 3 < N) cpre = *reinterpret_cast<const floatx4*>(C + (long long)gm * N + gn);
-    }
+template <int BT, int TM, int TN, int WM, int WN, int KG>
+__global__ __launch_bounds__(64 * WM * WN * KG) void gemm_nn_f32_kernel(const float* __restrict__ A, const float* __restrict__ B,
+                                                                        float* __restrict__ C, int M, int N, int K, int tiles_m,
+                                                                        int tiles_n) {
+  using Cfg = GemmCfg<BT, TM, TN, WM, WN, KG>;
+  constexpr int QK = 256 / BT, NQ = 32 / QK, kAcc = Cfg::kAcc;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int grp = wave / (WM * WN), wmn = wave % (WM * WN);
+  const int lrow = lane & (BT - 1), lh = lane / BT;
+  // XCD x (workgroups x, x + 8, ...) takes a contiguous run of tiles, walked in bands of eight tile rows
+  int tm, tn;
+  {
+    const int tiles = tiles_m * tiles_n, per = (tiles + 7) >> 3, rem = tiles & 7;
+    const int x = blockIdx.x & 7, i = blockIdx.x >> 3;
+    const int t = rem == 0 ? x * per + i : (x < rem ? x * per : rem * per + (x - rem) * (per - 1)) + i;
+    const int band = t / (8 * tiles_n), in = t - band * 8 * tiles_n, h = min(8, tiles_m - 8 * band);
+    tn = in / h;
+    tm = 8 * band + (in - tn * h);
   }
-  floatx16 acc[TM][TN];
+  const int m0 = tm * Cfg::kRows + (wmn % WM) * BT * TM, n0 = tn * Cfg::kCols + (wmn / WM) * BT * TN;
+  const bool live = m0 < M && n0 < N;  // a wave of a multi-wave tile may lie outside the matrix altogether
+  // accumulator register v of block row i: matrix row of this lane's result
+  auto row_of = [&](int i, int v) { return BT * i + (BT == 32 ? 8 * (v >> 2) + 4 * lh + (v & 3) : 4 * lh + v); };
+  typedef typename Vec<TN>::type vec;
+  auto c_row = [&](int row, bool* whole) -> float* {
+    const int m = m0 + row, n = n0 + TN * lrow;
+    *whole = n + TN <= N;
+    return live && m < M && n < N ? C + (long long)m * N + n : nullptr;
+  };
+  auto fetch = [&](const float* c, bool whole) {
+    vec v;
+    if constexpr (TN == 1) {
+      v = c ? *c : 0.0f;
+    } else {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) v[j] = 0.0f;
+      if (c && whole) {
+        __builtin_memcpy(&v, c, sizeof(v));
+      } else if (c) {
+        v[0] = c[0];  // TN = 2: the last column of an odd row
+      }
+    }
+    return v;
+  };
+  auto put = [&](float* c, bool whole, vec v) {
+    if (!c) return;
+    if constexpr (TN == 1) {
+      *c = v;
+    } else {
+      if (whole) __builtin_memcpy(c, &v, sizeof(v));
+      else c[0] = v[0];
+    }
+  };
+
+  typename Mma32<BT>::acc acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+      for (int v = 0; v < kAcc; ++v) acc[i][j][v] = 0.0f;
 
-  // K tile kt of group g in round r is r * KG + g; a group past the end of K loads zeros (same barriers for all)
-  const int nk = (K + GBK - 1) / GBK, rounds = (nk + KG - 1) / KG;
-  load(grp * GBK);
-  store(0);
-  __syncthreads();
-  const int lrow = lane & 31, lh = lane >> 5;
-  for (int r = 0; r < rounds; ++r) {
-    const bool more = r + 1 < rounds;
-    if (more) load(((r + 1) * KG + grp) * GBK);
-    const unsigned char* pa = sA + (r & 1) * GBM * kARow + (wm * WTM + lrow) * kARow;
-    const unsigned char* pb = sB + (r & 1) * GBK * kBRow + (wn * WTN + lrow) * 4;
+  // row units (i, v) of the tile this wave adds to C
+  constexpr int kUnits = TM * kAcc, kMine = kUnits / KG;
+  static_assert(kUnits % KG == 0, "every wave of a tile takes the same number of row units");
+  vec cpre[KG > 1 ? kMine : 1];
+
+  // rounds of 32 k: group g owns [begin, end)
+  const int nk = (K + 31) >> 5;
+  const int begin = (int)((long long)nk * grp / KG), end = (int)((long long)nk * (grp + 1) / KG);
+  if (live && begin < end) {
+    unsigned aoff[TM];
 #pragma unroll
-    for (int kk = 0; kk < 2 * KQ; ++kk) {
-      const int chunk = 2 * kk + lh;
-      floatx4 fa[TM];
-      float fb[TN][4];
+    for (int i = 0; i < TM; ++i) aoff[i] = ((unsigned)min(BT * i + lrow, M - 1 - m0) * (unsigned)K + 4u * lh) * 4u;
+    const unsigned boff = (4u * lh * (unsigned)N + (unsigned)(TN * lrow)) * 4u, brow = (unsigned)N * 4u;
+    // A is one round ahead in a second buffer, requested in one burst per round; B's registers are refilled for the next
+    // round as each quarter's products are issued (three rounds in flight measured slower: fewer waves per SIMD)
+    floatx4 fa[2][TM][NQ];
+    float fb[NQ][4][TN];
+    auto load_a = [&](int r, floatx4 (&f)[TM][NQ]) {
+      const long long at = (long long)m0 * K + 32ll * r;
+      const __amdgpu_buffer_rsrc_t rs = mt::make_rsrc(A + at, bytes_left((long long)M * K, at));
 #pragma unroll
-      for (int i = 0; i < TM; ++i) fa[i] = *reinterpret_cast<const floatx4*>(pa + i * 32 * kARow + chunk * 16);
+      for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
+        for (int q = 0; q < NQ; ++q)
+          f[i][q] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs, aoff[i] + 4 * QK * q, 0, 0));
+    };
+    auto rsrc_b = [&](int r) {
+      const long long at = 32ll * r * N + n0;
+      return mt::make_rsrc(B + at, bytes_left((long long)K * N, at));
+    };
+    auto load_b = [&](__amdgpu_buffer_rsrc_t rs, int q) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) fb[j][e] = *reinterpret_cast<const float*>(pb + (chunk * 4 + e) * kBRow + j * 32 * 4);
+      for (int e = 0; e < 4; ++e) load_row<TN>(rs, boff + (unsigned)(QK * q + e) * brow, fb[q][e]);
+    };
+    auto mma = [&](const floatx4 (&f)[TM][NQ], int q) {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][e], fb[j][e], acc[i][j], 0, 0, 0);
-    }
-    if (more) store((r + 1) & 1);
-    __syncthreads();
-  }
-
-  if constexpr (KG > 1) {
-    // partial tiles [group][64][64] in LDS (the operand buffers are free after the last barrier), then every thread
-    // sums KG values for four consecutive n and adds them to C: 16 lanes per 256-byte row
-    float* red = reinterpret_cast<float*>(smem);
+          for (int j = 0; j < TN; ++j) acc[i][j] = Mma32<BT>::run(f[i][q][e], fb[q][e][j], acc[i][j]);
+    };
+    // the group's last round first
+    load_a(end - 1, fa[0]);
+    {
+      const __amdgpu_buffer_rsrc_t rb = rsrc_b(end - 1);
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int m = wm * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
-      red[(grp * 64 + m) * 64 + wn * 32 + lrow] = acc[0][0][v];
+      for (int q = 0; q < NQ; ++q) load_b(rb, q);
     }
-    __syncthreads();
-    const int t = threadIdx.x;
-    for (int e = t; e < 64 * 16; e += 256 * KG) {
-      const int m = e >> 4, nq = (e & 15) * 4;
-      floatx4 sum = *reinterpret_cast<const floatx4*>(red + m * 64 + nq);
+    if constexpr (KG > 1) {
 #pragma unroll
-      for (int g = 1; g < KG; ++g) {
-        const floatx4 p = *reinterpret_cast<const floatx4*>(red + (g * 64 + m) * 64 + nq);
-        sum += p;
+      for (int u = 0; u < kMine; ++u) {
+        bool whole;
+        const float* c = c_row(row_of((grp * kMine + u) / kAcc, (grp * kMine + u) % kAcc), &whole);
+        cpre[u] = fetch(c, whole);
       }
-      const int gm = m0 + m, gn = n0 + nq;
-      if (gm >= M) continue;
-      float* c = C + (long long)gm * N + gn;
-      if (VEC && gn + 3 < N) {
-        floatx4 cv = e == t ? cpre : *reinterpret_cast<floatx4*>(c);  // the thread's first element is the prefetched one
-        cv += sum;
-        *reinterpret_cast<floatx4*>(c) = cv;
+    }
+    if (const int left = K - 32 * (end - 1); left < 32) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) fa[0][i][q][e] = QK * q + 4 * lh + e < left ? fa[0][i][q][e] : 0.0f;
+    }
+    // one round: its products, and behind each part of it the loads of the round after it
+    auto round = [&](const floatx4 (&cur)[TM][NQ], floatx4 (&nxt)[TM][NQ], int next, bool more) {
+      if (more) {
+        load_a(next, nxt);
+        const __amdgpu_buffer_rsrc_t rb = rsrc_b(next);
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+          mma(cur, q);
+          __builtin_amdgcn_sched_barrier(0);
+          load_b(rb, q);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       } else {
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          if (gn + q < N) c[q] += sum[q];
+        for (int q = 0; q < NQ; ++q) mma(cur, q);
       }
+    };
+    int r = begin;
+    const int last = end - 1;
+    for (; r + 1 < last; r += 2) {
+      round(fa[0], fa[1], r, true);
+      round(fa[1], fa[0], r + 1, true);
     }
-    return;
+    if (r < last) {
+      round(fa[0], fa[1], r, true);
+      round(fa[1], fa[0], 0, false);
+    } else {
+      round(fa[0], fa[1], 0, false);
+    }
+  } else if constexpr (KG > 1) {
+#pragma unroll
+    for (int u = 0; u < kMine; ++u) {
+      bool whole;
+      const float* c = c_row(row_of((grp * kMine + u) / kAcc, (grp * kMine + u) % kAcc), &whole);
+      cpre[u] = fetch(c, whole);
+    }
   }
 
-  // D[i][j]: lane holds column n = lane%32, rows m = 8g + 4*(lane/32) + e
+  if constexpr (KG == 1) {
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int n = n0 + wn * WTN + j * 32 + lrow;
-      if (n >= N) continue;
+      for (int v = 0; v < kAcc; ++v) {
+        bool whole;
+        float* c = c_row(row_of(i, v), &whole);
+        vec y = fetch(c, whole);
+        if constexpr (TN == 1) {
+          y += acc[i][0][v];
+        } else {
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int m = m0 + wm * WTM + i * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
-        if (m < M) {
-          float* c = C + (long long)m * N + n;
-          *c = *c + acc[i][j][v];
+          for (int j = 0; j < TN; ++j) y[j] += acc[i][j][v];
         }
+        put(c, whole, y);
       }
+  } else {
+    // [group][tile][row unit][lane][TN]: lane-linear, no bank conflicts
+    extern __shared__ __align__(16) float red[];
+    vec* mine = reinterpret_cast<vec*>(red) + (size_t)(grp * WM * WN + wmn) * kUnits * 64 + lane;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int v = 0; v < kAcc; ++v) {
+        vec y;
+        if constexpr (TN == 1) {
+          y = acc[i][0][v];
+        } else {
+#pragma unroll
+          for (int j = 0; j < TN; ++j) y[j] = acc[i][j][v];
+        }
+        mine[(kAcc * i + v) * 64] = y;
+      }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kMine; ++u) {
+      const int unit = grp * kMine + u;
+      const vec* p = reinterpret_cast<const vec*>(red) + ((size_t)wmn * kUnits + unit) * 64 + lane;
+      vec sum = p[0];
+#pragma unroll
+      for (int g = 1; g < KG; ++g) sum += p[(size_t)g * WM * WN * kUnits * 64];
+      bool whole;
+      float* c = c_row(row_of(unit / kAcc, unit % kAcc), &whole);
+      put(c, whole, cpre[u] + sum);
     }
+  }
 }
 
-template <int GBM, int GBN, int KG, bool VEC>
-static void launch_gemm_cfg(const float* A, const float* B, float* C, int M, int N, int K, hipStream_t s) {
-  auto kern = gemm_nn_f32_kernel<GBM, GBN, KG, VEC>;
-  constexpr int smem = gemm_lds(GBM, GBN, KG);
+// Rows too long for 32-bit byte offsets over a tile (N or K from 2^24 up): one thread per element of C.
+__global__ void gemm_nn_f32_any_kernel(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, int M, int N, int K) {
+  const long long total = (long long)M * N;
+  for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += (long long)gridDim.x * blockDim.x) {
+    const long long m = t / N, n = t - m * N;
+    float part[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (long long k = 0; k < K; ++k) part[k & 7] += A[m * K + k] * B[k * N + n];
+    C[t] += ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
+  }
+}
+
+template <int BT, int TM, int TN, int WM, int WN, int KG>
+void launch_gemm_cfg(const float* A, const float* B, float* C, int M, int N, int K, hipStream_t s) {
+  using Cfg = GemmCfg<BT, TM, TN, WM, WN, KG>;
+  auto kern = gemm_nn_f32_kernel<BT, TM, TN, WM, WN, KG>;
   static const bool attr = [&] {
-    NNCV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
+    if (Cfg::kLds) NNCV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::kLds));
     return true;
   }();
   (void)attr;
-  dim3 grid((N + GBN - 1) / GBN, (M + GBM - 1) / GBM);
-  hipLaunchKernelGGL(kern, grid, dim3(256 * KG), smem, s, A, B, C, M, N, K);
+  const long long tm = (M + Cfg::kRows - 1) / Cfg::kRows, tn = (N + Cfg::kCols - 1) / Cfg::kCols;
+  NNCV_REQUIRE(tm * tn < (1ll << 31), "matmul: too many tiles");
+  hipLaunchKernelGGL(kern, dim3((unsigned)(tm * tn)), dim3(64 * Cfg::kWaves), Cfg::kLds, s, A, B, C, M, N, K, (int)tm, (int)tn);
 }
+
+}  // namespace
+
+namespace {
+
+// The forms of the kernel, and what a launch of each takes:
+//   us = fixed + rounds * (k_us * 32 x 32 blocks of a tile * K + tile_us),   rounds = ceil(tiles / 256 CUs)
+// with K rounded up to whole rounds of 32.  The coefficients are least-squares fits over 24 shapes from 16x16x4096 to 4096^3
+// (launches back to back, clocks warm; the fit is within 5-15 % of every time, and the form it picks is on average 3 %
+// slower than the best one).  k_us at the matrix rate is 0.0033: large tiles come close, 16-wide ones are bound by the
+// number of operand loads (their MFMAs take half as long on the same loads), but split a small C over more CUs.
+//   1024^3 26.7 -> 21.1 us, 4096^3 1120 -> 960 (143 TFLOP/s), 1500x1001x777 69.4 -> 27.6, 20x488x536 14.6 -> 3.2,
+//   64x64x4096 81 -> 11, 92x3260x2312 52 -> 22 (against the LDS-tiled kernel with 128x128 / 64x64 tiles that this replaces)
+struct GemmForm {
+  int rows, cols;
+  double fixed_us, k_us, tile_us;
+  void (*launch)(const float*, const float*, float*, int, int, int, hipStream_t);
+};
+const GemmForm kForms[] = {
+    {128, 128, 5.7, 0.00367, 9.0, launch_gemm_cfg<32, 2, 2, 2, 2, 1>},
+    {64, 128, 0.0, 0.00377, 5.3, launch_gemm_cfg<32, 1, 2, 2, 2, 2>},
+    {32, 64, 2.3, 0.00407, 1.0, launch_gemm_cfg<32, 1, 2, 1, 1, 4>},
+    {32, 32, 2.4, 0.00477, 0.56, launch_gemm_cfg<32, 1, 1, 1, 1, 4>},
+    {32, 32, 2.1, 0.00440, 1.2, launch_gemm_cfg<32, 1, 1, 1, 1, 8>},
+    {16, 32, 2.95, 0.00623, 0.13, launch_gemm_cfg<16, 1, 2, 1, 1, 4>},
+    {16, 16, 2.95, 0.00847, 0.11, launch_gemm_cfg<16, 1, 1, 1, 1, 4>},
+};
+
+}  // namespace
 
 void launch_gemm_nn_f32(const float* A, const float* B, float* C, int M, int N, int K, hipStream_t s) {
   NNCV_REQUIRE(M > 0 && N > 0 && K > 0, "matmul: empty operand");
   ProfScope prof("gemm_nn_f32", 2.0 * M * N * K, 4.0 * ((double)M * K + (double)K * N + 2.0 * M * N), s);
-  const bool vec = K % 4 == 0 && N % 4 == 0 && (reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(C)) % 16 == 0;
-  const long long big = (long long)((N + 127) / 128) * ((M + 127) / 128);
-  const long long small = (long long)((N + 63) / 64) * ((M + 63) / 64);
-  // K groups while the 64x64 grid leaves SIMDs with one wave (or none) and K is long enough to share
-  const int kg = big >= 256 ? 1 : (small <= 384 && K >= 256) ? 4 : (small <= 768 && K >= 128) ? 2 : 1;
-  if (big >= 256) {
-    if (vec) launch_gemm_cfg<128, 128, 1, true>(A, B, C, M, N, K, s);
-    else launch_gemm_cfg<128, 128, 1, false>(A, B, C, M, N, K, s);
-  } else if (kg == 4) {
-    if (vec) launch_gemm_cfg<64, 64, 4, true>(A, B, C, M, N, K, s);
-    else launch_gemm_cfg<64, 64, 4, false>(A, B, C, M, N, K, s);
-  } else if (kg == 2) {
-    if (vec) launch_gemm_cfg<64, 64, 2, true>(A, B, C, M, N, K, s);
-    else launch_gemm_cfg<64, 64, 2, false>(A, B, C, M, N, K, s);
-  } else {
-    if (vec) launch_gemm_cfg<64, 64, 1, true>(A, B, C, M, N, K, s);
-    else launch_gemm_cfg<64, 64, 1, false>(A, B, C, M, N, K, s);
+  if (N >= 1 << 24 || K >= 1 << 24) {  // 64 rows of A or 32 of B beyond 32-bit byte offsets
+    const long long blocks = ((long long)M * N + 255) / 256;
+    hipLaunchKernelGGL(gemm_nn_f32_any_kernel, dim3((unsigned)std::min(blocks, 1ll << 20)), dim3(256), 0, s, A, B, C, M, N, K);
+    NNCV_HIP_CHECK(hipGetLastError());
+    return;
   }
+  const GemmForm* best = nullptr;
+  double best_us = 0;
+  for (const GemmForm& f : kForms) {
+    const long long tiles = (long long)((M + f.rows - 1) / f.rows) * ((N + f.cols - 1) / f.cols), rounds = (tiles + 255) / 256;
+    const double us = f.fixed_us + (double)rounds * (f.k_us * (f.rows * f.cols / 1024.0) * ((K + 31) / 32 * 32) + f.tile_us);
+    if (!best || us < best_us) best = &f, best_us = us;
+  }
+  best->launch(A, B, C, M, N, K, s);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 

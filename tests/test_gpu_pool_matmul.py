@@ -101,3 +101,24 @@ def test_matmul_k_groups_are_deterministic():
         abi.check(abi.lib().nncv_hip_matmul_f32(ad.data_ptr(), bd.data_ptr(), c.data_ptr(), 1024, 1024, 1024, None))
         outs.append(host(c))
     assert np.array_equal(outs[0], outs[1])
+
+
+# one shape for every form the dispatch can pick (tiles 16x16 ... 128x128, K groups or none) with every dimension one off a
+# tile or a 32-wide K round, fewer rounds than K groups, and rows too long for 32-bit offsets; one row of A holds infinities
+# and the K tail reads past row ends, so nothing of a neighbouring row may reach a result
+@pytest.mark.parametrize("M,N,K", [(15, 31, 4097), (129, 33, 31), (63, 470, 33), (1025, 260, 65), (65, 4001, 95), (31, 2999, 1001),
+                                   (1400, 999, 129), (513, 2049, 1063), (2300, 2190, 33), (3000, 2945, 161), (2, 3, (1 << 24) + 3)])
+def test_matmul_forms_and_tails(M, N, K):
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.rand((M, K), generator=g) * 2 - 1
+    b = torch.rand((K, N), generator=g) * 2 - 1
+    c0 = torch.rand((M, N), generator=g) * 2 - 1
+    a[M // 2] = float("inf")
+    keep = [m for m in range(M) if m != M // 2]
+    want = c0.double() + a.double() @ b.double()
+    ad, bd, c = a.cuda(), b.cuda(), c0.cuda()
+    abi.check(abi.lib().nncv_hip_matmul_f32(ad.data_ptr(), bd.data_ptr(), c.data_ptr(), M, N, K, None))
+    got = c.cpu()
+    assert not torch.isfinite(got[M // 2]).any()
+    err = ((got[keep].double() - want[keep]).abs().max() / want[keep].abs().max()).item()
+    assert err < 2e-6 * max(1.0, (K / 4096) ** 0.5), err
