@@ -35,24 +35,32 @@ void Context::init(int device) {
   // the code objects in this library exist for gfx950 only; anything else cannot run them
   NNCV_REQUIRE(arch_.rfind("gfx950", 0) == 0, "this library is built for gfx950 (MI355X); found " + arch_);
   NNCV_HIP_CHECK(hipStreamCreate(&stream_));  // default priority
-  NNCV_HIP_CHECK(hipEventCreateWithFlags(&tail_event_, hipEventDisableTiming));
   device_ = device;
   ready_ = true;
   (void)noalloc_scratch();  // the scratch array's address on this device, resolved with the device current
 }
 
-// The event is recorded by the call that leaves work pending, on its own (then certainly live) stream; a later call on
-// another stream only waits for the event, so a caller stream destroyed in between is never touched again.
-void Context::order_after_previous(hipStream_t s) {
-  if (!tail_pending_ || tail_stream_ == s) return;
-  NNCV_HIP_CHECK(hipStreamWaitEvent(s, tail_event_, 0));
-  tail_pending_ = false;
+StreamOrder::~StreamOrder() {
+  if (ev_) (void)hipEventDestroy(ev_);
 }
 
-void Context::note_stream(hipStream_t s, bool pending) {
-  tail_stream_ = s;
-  tail_pending_ = pending;
-  if (pending) NNCV_HIP_CHECK(hipEventRecord(tail_event_, s));
+void StreamOrder::after_previous(hipStream_t s) {
+  if (!pending_ || tail_ == s) return;
+  if (many_) {
+    NNCV_HIP_CHECK(hipStreamWaitEvent(s, ev_, 0));
+  } else {
+    NNCV_HIP_CHECK(hipDeviceSynchronize());
+    many_ = true;
+  }
+  pending_ = false;
+}
+
+void StreamOrder::note(hipStream_t s, bool pending) {
+  tail_ = s;
+  pending_ = pending;
+  if (!pending || !many_) return;
+  if (!ev_) NNCV_HIP_CHECK(hipEventCreateWithFlags(&ev_, hipEventDisableTiming));
+  NNCV_HIP_CHECK(hipEventRecord(ev_, s));
 }
 
 }  // namespace nncv_hip
@@ -89,8 +97,7 @@ void guarded_abort(const char* what, const std::function<void()>& fn) {
 // pinned staging buffers are shared by every call, and the mutex only serialises the enqueueing: work
 // left pending on one caller stream must not overlap work enqueued next on another.  So a call that
 // arrives on a different stream than the previous one first makes its stream wait for everything the
-// previous stream was given (an event recorded there now: the mutex is held, so that is exactly the
-// earlier calls' work).  Calls that stay on one stream pay nothing.
+// previous stream was given (StreamOrder, runtime.hpp).  Calls that stay on one stream pay nothing.
 // A caller stream that is being captured into a HIP graph takes neither the wait nor the event: both would reach
 // outside the capture and end it.  The captured launches then run whenever the caller's graph does, and ordering
 // them against other users of the library's shared workspace is the caller's business, as for the graph itself.
@@ -109,18 +116,18 @@ struct Sync {
   bool capturing;
   explicit Sync(void* user) : s(user ? static_cast<hipStream_t>(user) : Context::get().stream()), own(user == nullptr) {
     capturing = !own && stream_is_capturing(s);
-    if (!capturing) Context::get().order_after_previous(s);
+    if (!capturing) Context::get().order.after_previous(s);
   }
   bool done = false;
   void finish() {
     if (own) NNCV_HIP_CHECK(hipStreamSynchronize(s));
-    if (!capturing) Context::get().note_stream(s, /*pending=*/!own);
+    if (!capturing) Context::get().order.note(s, /*pending=*/!own);
     done = true;
   }
   ~Sync() {  // left early by an exception: whatever was enqueued may still be running
     if (!done && !capturing) {
       try {
-        Context::get().note_stream(s, true);
+        Context::get().order.note(s, true);
       } catch (...) {
       }
     }
@@ -134,12 +141,7 @@ struct Sync {
 // previous one first makes its stream wait for that one, as Sync does for the library-wide arena.
 struct HandleState {
   Arena arena;
-  hipStream_t tail = nullptr;
-  bool pending = false;
-  hipEvent_t ev = nullptr;
-  ~HandleState() {
-    if (ev) (void)hipEventDestroy(ev);
-  }
+  StreamOrder order;
 };
 
 struct HandleSync {
@@ -148,29 +150,17 @@ struct HandleSync {
   bool own;
   bool done = false;
   HandleSync(HandleState& hs, void* user) : h(hs), s(user ? static_cast<hipStream_t>(user) : Context::get().stream()), own(user == nullptr) {
-    // the event was recorded when the previous call ended, on its stream: that stream is not touched again here
-    if (h.pending && h.tail != s) {
-      NNCV_HIP_CHECK(hipStreamWaitEvent(s, h.ev, 0));
-      h.pending = false;
-    }
-  }
-  void leave(bool pending) {
-    h.tail = s;
-    h.pending = pending;
-    if (pending) {
-      if (!h.ev) NNCV_HIP_CHECK(hipEventCreateWithFlags(&h.ev, hipEventDisableTiming));
-      NNCV_HIP_CHECK(hipEventRecord(h.ev, s));
-    }
+    h.order.after_previous(s);
   }
   void finish() {
     if (own) NNCV_HIP_CHECK(hipStreamSynchronize(s));
-    leave(!own);
+    h.order.note(s, /*pending=*/!own);
     done = true;
   }
   ~HandleSync() {  // left early by an exception: whatever was enqueued may still be running
     if (!done) {
       try {
-        leave(true);
+        h.order.note(s, true);
       } catch (...) {
       }
     }
@@ -491,7 +481,7 @@ void forward_abi(nncv_memref2d* dst, nncv_memref4d* src, void* params, int dt) {
   Context& ctx = Context::get();
   ctx.init(-1);
   hipStream_t s = ctx.stream();
-  ctx.order_after_previous(s);
+  ctx.order.after_previous(s);
   const size_t es = dtype_size(dt);
   const nncv_memref1d* p = static_cast<const nncv_memref1d*>(params);
   NNCV_REQUIRE(p->aligned && p->strides[0] == 1, "params must be a dense rank-1 memref");
@@ -583,7 +573,7 @@ void _mlir_ciface_matmul(nncv_memref2d* res, nncv_memref2d* a, nncv_memref2d* b,
     Context& ctx = Context::get();
     ctx.init(-1);
     hipStream_t s = ctx.stream();
-    ctx.order_after_previous(s);
+    ctx.order.after_previous(s);
     const int M = (int)a->sizes[0], K = (int)a->sizes[1], N = (int)b->sizes[1];
     NNCV_REQUIRE(b->sizes[0] == K && c->sizes[0] == M && c->sizes[1] == N, "matmul: shapes do not agree");
     const size_t ab = align256((size_t)M * K * 4), bb = align256((size_t)K * N * 4), cb = align256((size_t)M * N * 4);
@@ -606,7 +596,7 @@ void _mlir_ciface_batch_nchw_conv(nncv_memref4d* res, nncv_memref4d* in, nncv_me
     Context& ctx = Context::get();
     ctx.init(-1);
     hipStream_t s = ctx.stream();
-    ctx.order_after_previous(s);
+    ctx.order.after_previous(s);
     const int N = (int)in->sizes[0], C = (int)in->sizes[1], H = (int)in->sizes[2], W = (int)in->sizes[3];
     const int F = (int)filter->sizes[0], R = (int)filter->sizes[2], S = (int)filter->sizes[3];
     const int OH = (int)out->sizes[2], OW = (int)out->sizes[3];
