@@ -40,6 +40,15 @@ void Context::init(int device) {
   (void)noalloc_scratch();  // the scratch array's address on this device, resolved with the device current
 }
 
+hipEvent_t Context::event(size_t i) {
+  while (events_.size() <= i) {
+    hipEvent_t e = nullptr;
+    NNCV_HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    events_.push_back(e);
+  }
+  return events_[i];
+}
+
 StreamOrder::~StreamOrder() {
   if (ev_) (void)hipEventDestroy(ev_);
 }
@@ -185,12 +194,14 @@ void strided_copy(char* base, intptr_t offset, const intptr_t* sizes, const intp
   intptr_t idx[R] = {0};
   long long total = 1;
   for (int i = 0; i < R; ++i) total *= sizes[i];
-  for (long long lin = 0; lin < total; ++lin) {
+  const bool rows = R > 1 && strides[R - 1] == 1;  // whole rows of the last dimension at once
+  const intptr_t step = rows ? sizes[R - 1] : 1;
+  for (long long lin = 0; lin < total; lin += step) {
     intptr_t off = offset;
     for (int i = 0; i < R; ++i) off += idx[i] * strides[i];
-    if (to_dense) memcpy(dense + lin * es, base + off * es, es);
-    else memcpy(base + off * es, dense + lin * es, es);
-    for (int i = R - 1; i >= 0; --i) {
+    if (to_dense) memcpy(dense + lin * es, base + off * es, es * step);
+    else memcpy(base + off * es, dense + lin * es, es * step);
+    for (int i = rows ? R - 2 : R - 1; i >= 0; --i) {
       if (++idx[i] < sizes[i]) break;
       idx[i] = 0;
     }
@@ -230,6 +241,41 @@ void download(void* aligned, intptr_t offset, const intptr_t* sizes, const intpt
     strided_copy<R>(base, offset, sizes, strides, es, p, false);
   }
 }
+
+// ---- pinned staging of the host-buffer calls --------------------------------------------------------------------------
+// The runtime's copies of pageable memory are slow where these calls live (measured: 4 MB up 130 us and down 237 us, 256 KB
+// up 108 us, against 81 / 81 / 12 us from pinned memory; one thread copies 4 MB to pinned memory in 54 us).  Up to this
+// many bytes a call stages everything in pinned memory, in pieces that the DMA engine or a kernel reads while the next
+// one is being copied; larger calls, whose time is the bus either way, go through the runtime and keep no such block.
+constexpr size_t kStageMost = size_t(64) << 20, kStagePiece = size_t(1) << 20;
+
+// rows [r0, r1) of the outermost dimension of a host memref, dense, to or from `stage`
+template <int R>
+void stage_rows(const void* aligned, intptr_t offset, const intptr_t* sizes, const intptr_t* strides, size_t es, intptr_t r0, intptr_t r1,
+                char* stage, bool in) {
+  intptr_t sz[R];
+  long long row = 1;
+  for (int i = 0; i < R; ++i) sz[i] = sizes[i];
+  for (int i = 1; i < R; ++i) row *= sizes[i];
+  sz[0] = r1 - r0;
+  char* base = static_cast<char*>(const_cast<void*>(aligned));
+  const intptr_t off = offset + r0 * strides[0];
+  if (contiguous<R>(sz, strides)) {
+    const size_t bytes = (size_t)(sz[0] * row) * es;
+    if (in) parallel_copy(stage, base + off * (intptr_t)es, bytes);
+    else parallel_copy(base + off * (intptr_t)es, stage, bytes);
+  } else {
+    strided_copy<R>(base, off, sz, strides, es, stage, in);
+  }
+}
+
+// rows of `row_bytes` per piece of about kStagePiece
+intptr_t rows_per_piece(size_t row_bytes) { return (intptr_t)std::max<size_t>(1, kStagePiece / std::max<size_t>(1, row_bytes)); }
+
+// A copy out of pinned memory as a kernel: 64 workgroups keep the bus as busy as the DMA engine does with copies of 4 MB
+// (52-56 GB/s; the engine's 1 MB copies run at 44), a launch costs the host 3 us, and a kernel behind it in the stream
+// starts without the 5-10 us that a signal from the engine takes.
+RideCopy from_pinned(const void* src, void* dst, size_t bytes) { return RideCopy{src, dst, align256(bytes), 64}; }
 
 // ---- model cache for the handle-less reference ABI ---------------------------------------
 struct CachedModel {
@@ -286,21 +332,16 @@ std::unique_ptr<ResNet18> build_model(const void* host, long long n, int dt, int
   return m;
 }
 
-ResNet18& cached_model(const void* host, long long n, int dt, hipStream_t s) {
-  const uint64_t fp = fingerprint(host, n, dtype_size(dt));
+// The cached entry of a blob, built on first sight.  Whether its contents are still those it was built from is asked
+// separately (refresh), while the device is already running the pass: the 4096 samples are as many cache misses.
+CachedModel& cached_model(const void* host, long long n, int dt, hipStream_t s) {
   auto& cache = model_cache();
   for (auto& e : cache)
-    if (e.host_ptr == host && e.n == n && e.dt == dt) {
-      if (e.fingerprint != fp) {  // same address, new contents: rebuild
-        e.model.reset();
-        e.model = build_model(host, n, dt, kAlgoAuto, s);
-        e.fingerprint = fp;
-      }
-      return *e.model;
-    }
+    if (e.host_ptr == host && e.n == n && e.dt == dt) return e;
+  const uint64_t fp = fingerprint(host, n, dtype_size(dt));
   if (cache.size() >= 4) cache.erase(cache.begin());
   cache.push_back(CachedModel{host, n, dt, fp, build_model(host, n, dt, kAlgoAuto, s)});
-  return *cache.back().model;
+  return cache.back();
 }
 
 // ---- HIP-graph replay of the forward pass --------------------------------------------------
@@ -420,33 +461,25 @@ std::unique_ptr<Graph> build_graph(const GraphOp* ops, int n_ops, int c_in, cons
   NNCV_HIP_CHECK(hipStreamSynchronize(s));  // the staging blob dies here
   return g;
 }
-Graph& cached_mobilenetv3(const void* host, long long n, int dt, hipStream_t s) {
-  const uint64_t fp = fingerprint(host, n, dtype_size(dt));
+std::unique_ptr<Graph> build_mobilenetv3(const void* host, long long n, int dt, hipStream_t s) {
+  long long k = 0;
+  const std::vector<GraphOp> ops = mobilenetv3_small_ops(&k);
+  return build_graph(ops.data(), (int)ops.size(), 3, host, n, dt, s);
+}
+CachedGraph& cached_mobilenetv3(const void* host, long long n, int dt, hipStream_t s) {
   auto& cache = graph_model_cache();
-  auto make = [&] {
-    long long k = 0;
-    const std::vector<GraphOp> ops = mobilenetv3_small_ops(&k);
-    return build_graph(ops.data(), (int)ops.size(), 3, host, n, dt, s);
-  };
   for (auto& e : cache)
-    if (e.host_ptr == host && e.n == n && e.dt == dt) {
-      if (e.fingerprint != fp) {
-        e.graph.reset();
-        e.graph = make();
-        e.fingerprint = fp;
-      }
-      return *e.graph;
-    }
+    if (e.host_ptr == host && e.n == n && e.dt == dt) return e;
+  const uint64_t fp = fingerprint(host, n, dtype_size(dt));
   if (cache.size() >= 4) cache.erase(cache.begin());
-  cache.push_back(CachedGraph{host, n, dt, fp, make()});
-  return *cache.back().graph;
+  cache.push_back(CachedGraph{host, n, dt, fp, build_mobilenetv3(host, n, dt, s)});
+  return cache.back();
 }
 
-// ---- the host-buffer call: the upload of a large dense input ---------------------------------------------------------
-// _mlir_ciface_forward hands over pageable host memory (examples/Res18/main.cpp:79-99).  The DMA engine moves config 4's
-// 9.6 MB in 0.23 ms from pinned memory; through the runtime's own staging of pageable memory the same copy takes 0.34 ms.
-// So the input goes to pinned staging memory in pieces, each copied by a few host threads while the DMA engine moves the
-// piece before it; a caller buffer that is pinned already is handed to the DMA engine as it is.
+// ---- the host-buffer call: the upload of a dense input -----------------------------------------------------------------
+// _mlir_ciface_forward hands over pageable host memory (examples/Res18/main.cpp:79-99).  The input goes to pinned staging
+// memory in pieces, each copied by a few host threads while a kernel fetches the piece before it; a caller buffer that is
+// pinned already is handed to the DMA engine as it is.  Config 4's 9.6 MB: 0.47 ms a call, 0.51 with DMA copies of the pieces.
 // Tried and not kept: cutting the batch into two halves (or a quarter, a quarter and a half) whose forward passes start
 // as soon as their bytes have landed, on streams and workspaces of their own.  The passes of 8-16 images are launch-bound
 // (8 + 8 + 16 images one after the other: 0.41 ms against 0.26 for the 32 at once), submitting a pass costs the host
@@ -463,16 +496,21 @@ bool host_pointer_is_pinned(const void* p) {
 
 void upload_dense(const char* hsrc, size_t bytes, void* dev, PinnedBuffer& pin, hipStream_t s) {
   static const bool plain = getenv("NNCV_HIP_NO_STAGED_UPLOAD") != nullptr;
-  if (plain || bytes < (size_t(1) << 20) || host_pointer_is_pinned(hsrc)) {
+  if (plain || host_pointer_is_pinned(hsrc)) {
     NNCV_HIP_CHECK(hipMemcpyAsync(dev, hsrc, bytes, hipMemcpyHostToDevice, s));
     return;
   }
-  char* stage = static_cast<char*>(pin.ensure(bytes));
-  const size_t piece = size_t(2) << 20;
-  for (size_t off = 0; off < bytes; off += piece) {
+  constexpr size_t piece = 2 * kStagePiece, slots = kStageMost / piece;  // a longer input goes round a ring of pieces
+  char* stage = static_cast<char*>(pin.ensure(align256(std::min(bytes, kStageMost))));
+  Context& ctx = Context::get();
+  size_t k = 0;
+  for (size_t off = 0; off < bytes; off += piece, ++k) {
     const size_t n = std::min(piece, bytes - off);
-    parallel_copy(stage + off, hsrc + off, n);
-    NNCV_HIP_CHECK(hipMemcpyAsync(static_cast<char*>(dev) + off, stage + off, n, hipMemcpyHostToDevice, s));
+    char* at = stage + (k % slots) * piece;
+    if (k >= slots) NNCV_HIP_CHECK(hipEventSynchronize(ctx.event(k % slots)));
+    parallel_copy(at, hsrc + off, n);
+    launch_copy16(from_pinned(at, static_cast<char*>(dev) + off, n), s);
+    if (bytes > kStageMost) NNCV_HIP_CHECK(hipEventRecord(ctx.event(k % slots), s));
   }
 }
 
@@ -492,12 +530,12 @@ void forward_abi(nncv_memref2d* dst, nncv_memref4d* src, void* params, int dt) {
   // (tests/Nets/Res18.mlir) or MobileNetV3-small (tests/Nets/MobileNetV3.mlir); both map
   // [N,3,H,W] to [N,1000].
   const bool mobilenet = p->sizes[0] == mobilenetv3_elems();
-  ResNet18* model = mobilenet ? nullptr : &cached_model(blob, p->sizes[0], dt, s);
-  Graph* graph = mobilenet ? &cached_mobilenetv3(blob, p->sizes[0], dt, s) : nullptr;
+  CachedModel* model = mobilenet ? nullptr : &cached_model(blob, p->sizes[0], dt, s);
+  CachedGraph* graph = mobilenet ? &cached_mobilenetv3(blob, p->sizes[0], dt, s) : nullptr;
 
   const size_t in_bytes = align256((size_t)N * 3 * H * W * es), out_bytes = align256((size_t)N * 1000 * 4);
-  const size_t ws_bytes = mobilenet ? graph->workspace_bytes(N, H, W) : model->workspace_bytes(N, H, W);
-  ctx.arena.reserve(in_bytes + 2 * out_bytes + ws_bytes + 2048, s);
+  const size_t ws_bytes = mobilenet ? graph->graph->workspace_bytes(N, H, W) : model->model->workspace_bytes(N, H, W);
+  ctx.arena.reserve(in_bytes + out_bytes + ws_bytes + 2048, s);
   void* d_in = ctx.arena.take(in_bytes);
   float* d_out = static_cast<float*>(ctx.arena.take(out_bytes));
   void* ws = ctx.arena.take(ws_bytes);
@@ -507,25 +545,33 @@ void forward_abi(nncv_memref2d* dst, nncv_memref4d* src, void* params, int dt) {
     upload_dense(static_cast<const char*>(src->aligned) + src->offset * (intptr_t)es, (size_t)N * 3 * H * W * es, d_in, ctx.pin_in, s);
   else
     upload<4>(src->aligned, src->offset, src->sizes, src->strides, es, d_in, ctx.pin_in, s);
-  if (mobilenet) graph->forward(d_in, N, H, W, d_out, ws, s);
-  else model->forward(d_in, N, H, W, d_out, ws, s);
-
+  // The last kernel writes the logits to pinned memory itself: no copy command behind the pass.  fp16 logits are rounded on
+  // the device (one round-to-nearest-even conversion, what the host's would be).
+  void* logits = ctx.pin_out.ensure((size_t)N * 1000 * 4);
+  auto enqueue = [&] {
+    float* y = dt == kF32 ? static_cast<float*>(logits) : d_out;
+    if (mobilenet) graph->graph->forward(d_in, N, H, W, y, ws, s);
+    else model->model->forward(d_in, N, H, W, y, ws, s);
+    if (dt == kF16) launch_cast(d_out, kF32, logits, kF16, (long long)N * 1000, s);
+  };
+  enqueue();
   // MLIR C-interface convention: the callee allocates the result and overwrites *dst.
   void* result = nullptr;
   NNCV_REQUIRE(posix_memalign(&result, 64, std::max<size_t>(64, (size_t)N * 1000 * es)) == 0, "out of host memory");
-  if (dt == kF32) {
-    NNCV_HIP_CHECK(hipMemcpyAsync(result, d_out, (size_t)N * 1000 * 4, hipMemcpyDeviceToHost, s));
+  const uint64_t fp = fingerprint(blob, p->sizes[0], es);
+  NNCV_HIP_CHECK(hipStreamSynchronize(s));
+  if (fp != (mobilenet ? graph->fingerprint : model->fingerprint)) {  // same address, new contents: rebuild and run again
+    if (mobilenet) {
+      graph->graph = build_mobilenetv3(blob, p->sizes[0], dt, s);
+      graph->fingerprint = fp;
+    } else {
+      model->model = build_model(blob, p->sizes[0], dt, kAlgoAuto, s);
+      model->fingerprint = fp;
+    }
+    enqueue();
     NNCV_HIP_CHECK(hipStreamSynchronize(s));
-  } else {
-    // rounded to half on the device (one round-to-nearest-even conversion, what the host's would be): half the bytes over
-    // the bus and no conversion loop on the host
-    void* d_half = ctx.arena.take(align256((size_t)N * 1000 * 2));
-    launch_cast(d_out, kF32, d_half, kF16, (long long)N * 1000, s);
-    void* tmp = ctx.pin_out.ensure((size_t)N * 1000 * 2);
-    NNCV_HIP_CHECK(hipMemcpyAsync(tmp, d_half, (size_t)N * 1000 * 2, hipMemcpyDeviceToHost, s));
-    NNCV_HIP_CHECK(hipStreamSynchronize(s));
-    memcpy(result, tmp, (size_t)N * 1000 * 2);
   }
+  memcpy(result, logits, (size_t)N * 1000 * es);
   dst->allocated = result;
   dst->aligned = result;
   dst->offset = 0;
@@ -533,6 +579,146 @@ void forward_abi(nncv_memref2d* dst, nncv_memref4d* src, void* params, int dt) {
   dst->sizes[1] = 1000;
   dst->strides[0] = 1000;
   dst->strides[1] = 1;
+}
+
+// ---- linalg.matmul on host memory ------------------------------------------------------------------------------------
+// What the call cannot do without is the bus: A, B and C up, C down (1024^3: 12 MB and 4 MB, 220 + 75 us at 57 GB/s each way,
+// against 21 us of product).  B goes up first, then A and C in bands of rows, A's and C's part of a band side by side.
+// The launch that multiplies a band also fetches the next one, in workgroups of its own (two streams with events between
+// copies and products cost the host 20 us per band and the device a signal each), and writes its result to pinned memory
+// itself: both directions of the bus run at once, and the host copies a band out while later ones are under way.
+// 1024^3: 740 us a call through pageable copies, 384 with DMA copies on a second stream, then this.
+void matmul_host(Context& ctx, nncv_memref2d* a, nncv_memref2d* b, nncv_memref2d* c, int M, int N, int K, hipStream_t s) {
+  const size_t row_a = (size_t)K * 4, row_b = (size_t)N * 4, row_c = row_b;
+  const size_t bb = align256(row_b * K);
+  const int bands = (int)std::min<size_t>(std::min(M, 16), std::max<size_t>(1, (row_a + row_c) * M / (2 * kStagePiece)));
+  auto band_row = [&](int i) { return (int)((long long)M * i / bands); };
+  std::vector<size_t> at_a, at_c;  // byte offsets of A's and C's part of a band, on the host and on the device alike
+  size_t total = bb;
+  for (int i = 0; i < bands; ++i) {
+    const size_t rows = (size_t)(band_row(i + 1) - band_row(i));
+    at_a.push_back(total);
+    at_c.push_back(total + align256(rows * row_a));
+    total = at_c.back() + align256(rows * row_c);
+  }
+  at_a.push_back(total);
+  ctx.order.after_previous(s);
+  ctx.arena.reserve(total + 1024, s);
+  char* dev = static_cast<char*>(ctx.arena.take(total));
+  auto f32 = [](char* p) { return reinterpret_cast<float*>(p); };
+  if (total > kStageMost) {
+    char *dA = dev + bb, *dC = dA + align256(row_a * M);
+    upload<2>(b->aligned, b->offset, b->sizes, b->strides, 4, dev, ctx.pin_in, s);
+    upload<2>(a->aligned, a->offset, a->sizes, a->strides, 4, dA, ctx.pin_in, s);
+    upload<2>(c->aligned, c->offset, c->sizes, c->strides, 4, dC, ctx.pin_in, s);
+    launch_gemm_nn_f32(f32(dA), f32(dev), f32(dC), f32(dC), M, N, K, s);
+    download<2>(c->aligned, c->offset, c->sizes, c->strides, 4, dC, ctx.pin_out, s);
+    return;
+  }
+  char* host = static_cast<char*>(ctx.pin_in.ensure(total));
+  auto stage = [&](nncv_memref2d* m, char* to, int r0, int r1, bool in) {
+    stage_rows<2>(m->aligned, m->offset, m->sizes, m->strides, 4, r0, r1, to, in);
+  };
+  auto stage_band = [&](int i) {
+    stage(a, host + at_a[i], band_row(i), band_row(i + 1), true);
+    stage(c, host + at_c[i], band_row(i), band_row(i + 1), true);
+  };
+  size_t sent = 0;
+  // A launch of 1 MB takes 27 us, 19 of them for the bytes: the pieces of B start small, to get the bus going, and double
+  size_t piece = kStagePiece / 2;
+  for (intptr_t r = 0; r < K; piece *= 2) {
+    const intptr_t e = std::min<intptr_t>(K, r + (intptr_t)std::max<size_t>(1, piece / row_b));
+    stage(b, host + r * row_b, (int)r, (int)e, true);
+    const size_t end = e * row_b & ~size_t(255);
+    if (end - sent >= kStagePiece / 2) {
+      launch_copy16(from_pinned(host + sent, dev + sent, end - sent), s);
+      sent = end;
+    }
+    r = e;
+  }
+  stage_band(0);
+  launch_copy16(from_pinned(host + sent, dev + sent, at_a[1] - sent), s);  // what is left of B, and the first band
+  for (int i = 0; i < bands; ++i) {
+    RideCopy next{};
+    if (i + 1 < bands) {
+      stage_band(i + 1);
+      next = from_pinned(host + at_a[i + 1], dev + at_a[i + 1], at_a[i + 2] - at_a[i + 1]);
+    }
+    launch_gemm_nn_f32(f32(dev + at_a[i]), f32(dev), f32(dev + at_c[i]), f32(host + at_c[i]), band_row(i + 1) - band_row(i), N, K, s, &next);
+    if (i % 2 == 1 && i + 1 < bands) NNCV_HIP_CHECK(hipEventRecord(ctx.event(i / 2), s));
+  }
+  for (int i = 0; i < bands; ++i) {
+    if (i % 2 == 0) {
+      if (i + 2 < bands) NNCV_HIP_CHECK(hipEventSynchronize(ctx.event(i / 2)));
+      else NNCV_HIP_CHECK(hipStreamSynchronize(s));
+    }
+    stage(c, host + at_c[i], band_row(i), band_row(i + 1), false);
+  }
+}
+
+// ---- linalg.conv_2d_nchw_fchw on host memory -------------------------------------------------------------------------
+// Up to kStageMost bytes no copy command runs at all: the kernels that re-lay the filter, the input and the result for the
+// NHWC convolution read and write the pinned staging memory over the bus, every byte once, so each is its own transfer, and
+// reading and adding to `out` use both directions of the bus at once.  The caller's arrays are staged in ranges of
+// images, each range's kernel running while the next range is copied.
+void conv_host(Context& ctx, nncv_memref4d* in, nncv_memref4d* filter, nncv_memref4d* out, int N, int C, int H, int W, int F, int R, int S,
+               int stride, int OH, int OW, hipStream_t s) {
+  const int Cp = (C + 3) / 4 * 4, Fp = (F + 3) / 4 * 4;
+  const size_t img_i = (size_t)C * H * W * 4, img_o = (size_t)F * OH * OW * 4, fb = align256((size_t)F * C * R * S * 4);
+  const size_t ib = align256(img_i * N), ob = align256(img_o * N);
+  const size_t wt_b = align256((size_t)Fp * R * S * Cp * 4), x_b = align256((size_t)N * H * W * Cp * 4), y_b = align256((size_t)N * OH * OW * Fp * 4);
+  const bool staged = fb + ib + ob <= kStageMost;
+  ctx.order.after_previous(s);
+  ctx.arena.reserve(wt_b + x_b + y_b + (staged ? 0 : fb + ib + ob) + 2048, s);
+  char* wt = static_cast<char*>(ctx.arena.take(wt_b));
+  char* x = static_cast<char*>(ctx.arena.take(x_b));
+  char* y = static_cast<char*>(ctx.arena.take(y_b));
+  char *hF, *hI, *hO;  // what the re-laying kernels read: pinned memory, or device copies of the caller's arrays
+  if (staged) {
+    hF = static_cast<char*>(ctx.pin_in.ensure(fb + ib + ob));
+    hI = hF + fb;
+    hO = hI + ib;
+    stage_rows<4>(filter->aligned, filter->offset, filter->sizes, filter->strides, 4, 0, F, hF, true);
+  } else {
+    hF = static_cast<char*>(ctx.arena.take(fb));
+    hI = static_cast<char*>(ctx.arena.take(ib));
+    hO = static_cast<char*>(ctx.arena.take(ob));
+    upload<4>(filter->aligned, filter->offset, filter->sizes, filter->strides, 4, hF, ctx.pin_in, s);
+    upload<4>(in->aligned, in->offset, in->sizes, in->strides, 4, hI, ctx.pin_in, s);
+    upload<4>(out->aligned, out->offset, out->sizes, out->strides, 4, hO, ctx.pin_in, s);
+  }
+  launch_weight_frsc(hF, kF32, wt, kF32, F, C, R, S, Cp, s);
+  if (Fp > F) launch_fill_f32(reinterpret_cast<float*>(wt) + (size_t)F * R * S * Cp, 0.0f, (long long)(Fp - F) * R * S * Cp, s);
+  const intptr_t step_i = staged ? rows_per_piece(img_i) : N, step_o = staged ? rows_per_piece(img_o) : N;
+  for (intptr_t n = 0; n < N; n += step_i) {
+    const int k = (int)std::min<intptr_t>(step_i, N - n);
+    if (staged) stage_rows<4>(in->aligned, in->offset, in->sizes, in->strides, 4, n, n + k, hI + n * img_i, true);
+    launch_relayout(hI + n * img_i, kF32, strides_of(kNCHW, C, H, W), x + (size_t)n * H * W * Cp * 4, kF32, strides_of(kNHWC, Cp, H, W), k, C, Cp,
+                    H, W, false, s);
+  }
+  IgemmArgs g{};
+  g.in = x; g.wt = wt; g.out = y;
+  g.N = N; g.H = H; g.W = W; g.C = Cp; g.F = Fp; g.R = R; g.S = S; g.OH = OH; g.OW = OW;
+  g.stride_h = g.stride_w = stride; g.ldo = Fp; g.batch = 1;
+  launch_igemm(g, kF32, kF32, s);
+  size_t k_ev = 0;
+  for (intptr_t n = 0; n < N; n += step_o) {
+    const int k = (int)std::min<intptr_t>(step_o, N - n);
+    if (staged) stage_rows<4>(out->aligned, out->offset, out->sizes, out->strides, 4, n, n + k, hO + n * img_o, true);
+    launch_relayout(y + (size_t)n * OH * OW * Fp * 4, kF32, strides_of(kNHWC, Fp, OH, OW), hO + n * img_o, kF32, strides_of(kNCHW, F, OH, OW), k, F,
+                    F, OH, OW, true, s);
+    if (n + step_o < N) NNCV_HIP_CHECK(hipEventRecord(ctx.event(k_ev++), s));
+  }
+  if (!staged) {
+    download<4>(out->aligned, out->offset, out->sizes, out->strides, 4, hO, ctx.pin_out, s);
+    return;
+  }
+  k_ev = 0;
+  for (intptr_t n = 0; n < N; n += step_o) {
+    if (n + step_o < N) NNCV_HIP_CHECK(hipEventSynchronize(ctx.event(k_ev++)));
+    else NNCV_HIP_CHECK(hipStreamSynchronize(s));
+    stage_rows<4>(out->aligned, out->offset, out->sizes, out->strides, 4, n, std::min<intptr_t>(N, n + step_o), hO + n * img_o, false);
+  }
 }
 
 struct nncv_hip_model_impl {
@@ -573,19 +759,10 @@ void _mlir_ciface_matmul(nncv_memref2d* res, nncv_memref2d* a, nncv_memref2d* b,
     Context& ctx = Context::get();
     ctx.init(-1);
     hipStream_t s = ctx.stream();
-    ctx.order.after_previous(s);
     const int M = (int)a->sizes[0], K = (int)a->sizes[1], N = (int)b->sizes[1];
     NNCV_REQUIRE(b->sizes[0] == K && c->sizes[0] == M && c->sizes[1] == N, "matmul: shapes do not agree");
-    const size_t ab = align256((size_t)M * K * 4), bb = align256((size_t)K * N * 4), cb = align256((size_t)M * N * 4);
-    ctx.arena.reserve(ab + bb + cb + 1024, s);
-    float* dA = static_cast<float*>(ctx.arena.take(ab));
-    float* dB = static_cast<float*>(ctx.arena.take(bb));
-    float* dC = static_cast<float*>(ctx.arena.take(cb));
-    upload<2>(a->aligned, a->offset, a->sizes, a->strides, 4, dA, ctx.pin_in, s);
-    upload<2>(b->aligned, b->offset, b->sizes, b->strides, 4, dB, ctx.pin_in, s);
-    upload<2>(c->aligned, c->offset, c->sizes, c->strides, 4, dC, ctx.pin_in, s);
-    launch_gemm_nn_f32(dA, dB, dC, M, N, K, s);
-    download<2>(c->aligned, c->offset, c->sizes, c->strides, 4, dC, ctx.pin_out, s);
+    NNCV_REQUIRE(M > 0 && N > 0 && K > 0, "matmul: empty operand");
+    matmul_host(ctx, a, b, c, M, N, K, s);
     *res = *c;  // in-place bufferization: the result aliases `outs`
   });
 }
@@ -596,7 +773,6 @@ void _mlir_ciface_batch_nchw_conv(nncv_memref4d* res, nncv_memref4d* in, nncv_me
     Context& ctx = Context::get();
     ctx.init(-1);
     hipStream_t s = ctx.stream();
-    ctx.order.after_previous(s);
     const int N = (int)in->sizes[0], C = (int)in->sizes[1], H = (int)in->sizes[2], W = (int)in->sizes[3];
     const int F = (int)filter->sizes[0], R = (int)filter->sizes[2], S = (int)filter->sizes[3];
     const int OH = (int)out->sizes[2], OW = (int)out->sizes[3];
@@ -608,22 +784,8 @@ void _mlir_ciface_batch_nchw_conv(nncv_memref4d* res, nncv_memref4d* in, nncv_me
     else if (OW > 1) stride = (W - S) / (OW - 1);
     NNCV_REQUIRE(stride >= 1 && (H - R) / stride + 1 == OH && (W - S) / stride + 1 == OW,
                  "conv: output shape is not (in - filter)/stride + 1 for any stride");
-    const size_t ib = align256((size_t)N * C * H * W * 4), fb = align256((size_t)F * C * R * S * 4),
-                 ob = align256((size_t)N * F * OH * OW * 4);
-    ConvLayer::Desc d;
-    d.dt = kF32; d.C = C; d.F = F; d.R = R; d.S = S; d.stride = stride; d.pad = 0; d.relu = kActNone; d.algo = kAlgoAuto;
-    DeviceBuffer dF(fb);
-    upload<4>(filter->aligned, filter->offset, filter->sizes, filter->strides, 4, dF.get(), ctx.pin_in, s);
-    ConvLayer layer(d, dF.get(), nullptr, nullptr, nullptr, nullptr, s);
-    const size_t wsb = layer.workspace_bytes(N, H, W, true);
-    ctx.arena.reserve(ib + ob + wsb + 1024, s);
-    void* dI = ctx.arena.take(ib);
-    void* dO = ctx.arena.take(ob);
-    void* ws = ctx.arena.take(wsb);
-    upload<4>(in->aligned, in->offset, in->sizes, in->strides, 4, dI, ctx.pin_in, s);
-    upload<4>(out->aligned, out->offset, out->sizes, out->strides, 4, dO, ctx.pin_in, s);
-    layer.forward_strided(dI, strides_of(kNCHW, C, H, W), N, H, W, nullptr, dO, strides_of(kNCHW, F, OH, OW), true, ws, s);
-    download<4>(out->aligned, out->offset, out->sizes, out->strides, 4, dO, ctx.pin_out, s);
+    NNCV_REQUIRE(N > 0 && C > 0 && F > 0, "conv: empty tensor");
+    conv_host(ctx, in, filter, out, N, C, H, W, F, R, S, stride, OH, OW, s);
     *res = *out;
   });
 }
@@ -967,9 +1129,9 @@ int nncv_hip_matmul_time(const float* A, const float* B, float* C, int M, int N,
     hipEvent_t e0, e1;
     NNCV_HIP_CHECK(hipEventCreate(&e0));
     NNCV_HIP_CHECK(hipEventCreate(&e1));
-    for (int i = 0; i < 5; ++i) launch_gemm_nn_f32(A, B, C, M, N, K, sy.s);
+    for (int i = 0; i < 5; ++i) launch_gemm_nn_f32(A, B, C, C, M, N, K, sy.s);
     NNCV_HIP_CHECK(hipEventRecord(e0, sy.s));
-    for (int i = 0; i < reps; ++i) launch_gemm_nn_f32(A, B, C, M, N, K, sy.s);
+    for (int i = 0; i < reps; ++i) launch_gemm_nn_f32(A, B, C, C, M, N, K, sy.s);
     NNCV_HIP_CHECK(hipEventRecord(e1, sy.s));
     NNCV_HIP_CHECK(hipEventSynchronize(e1));
     float ms = 0.0f;
@@ -986,7 +1148,7 @@ int nncv_hip_matmul_f32(const float* A, const float* B, float* C, int M, int N, 
     NNCV_REQUIRE(A && B && C, "null argument");
     Context::get().init(-1);
     Sync sy(stream);
-    launch_gemm_nn_f32(A, B, C, M, N, K, sy.s);
+    launch_gemm_nn_f32(A, B, C, C, M, N, K, sy.s);
     sy.finish();
   });
 }

@@ -211,8 +211,12 @@ void launch_conv_pairs(const IgemmArgs& a, hipStream_t s);
 bool igemm_fast_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 void launch_igemm_fast(const IgemmArgs& a, int in_dt, int out_dt, hipStream_t s);
 
-// fp32 row-major C += A.B  (linalg.matmul)
-void launch_gemm_nn_f32(const float* A, const float* B, float* C, int M, int N, int K, hipStream_t s);
+// fp32 row-major D = C + A.B  (linalg.matmul); D may be C
+// (`ride`: a copy that the launch carries in workgroups of its own, for operands of the next launch)
+struct RideCopy { const void* src; void* dst; size_t bytes; int blocks; };  // 16-byte aligned, bytes a multiple of 16
+void launch_gemm_nn_f32(const float* A, const float* B, const float* C, float* D, int M, int N, int K, hipStream_t s,
+                        const RideCopy* ride = nullptr);
+void launch_copy16(const RideCopy& r, hipStream_t s);  // the copy alone
 
 // ---------------------------------------------------------------------------------------------
 // Winograd F(4x4,3x3)

@@ -1,4 +1,4 @@
-// fp32 row-major C += A.B on gfx950 MFMA — the linalg.matmul of
+// fp32 row-major D = C + A.B on gfx950 MFMA (D may be C) — the linalg.matmul of
 // tests/MatMulOptimization/MatMulDeafult.mlir:6-9, which the reference lowers with 16/8/k8 tiles
 // and 8x8x8 vector contracts (ModernTile.cpp:289-296, PrepareModernVec.cpp:43-48) and for which
 // its unfinished CUDA kernel intended a 128x128x8 shared-memory tiling
@@ -75,12 +75,38 @@ __device__ __forceinline__ unsigned bytes_left(long long elems, long long at) {
   return b > 0xffffffffll ? 0xffffffffu : (unsigned)b;
 }
 
-template <int BT, int TM, int TN, int WM, int WN, int KG>
+// A copy that rides in front of a launch: its first `blocks` workgroups move `bytes` (a multiple of 16) and are done.
+__device__ __forceinline__ void ride_along_copy(const RideCopy& r, int block, int threads) {
+  const u32x4* src = static_cast<const u32x4*>(r.src);
+  u32x4* dst = static_cast<u32x4*>(r.dst);
+  const size_t n = r.bytes >> 4, step = (size_t)r.blocks * threads;
+  size_t i = (size_t)block * threads + threadIdx.x;
+  for (; i + 3 * step < n; i += 4 * step) {
+    u32x4 v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = src[i + k * step];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) dst[i + k * step] = v[k];
+  }
+  for (; i < n; i += step) dst[i] = src[i];
+}
+
+__global__ __launch_bounds__(256) void copy16_kernel(RideCopy r) { ride_along_copy(r, blockIdx.x, 256); }
+
+template <int BT, int TM, int TN, int WM, int WN, int KG, bool RIDE = false>
 __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_nn_f32_kernel(const float* __restrict__ A, const float* __restrict__ B,
-                                                                        float* __restrict__ C, int M, int N, int K, int tiles_m,
-                                                                        int tiles_n) {
+                                                                        const float* C, float* D, int M, int N, int K, int tiles_m,
+                                                                        int tiles_n, RideCopy ride) {
   using Cfg = GemmCfg<BT, TM, TN, WM, WN, KG>;
   constexpr int QK = 256 / BT, NQ = 32 / QK, kAcc = Cfg::kAcc;
+  int block = blockIdx.x;
+  if constexpr (RIDE) {
+    if (block < ride.blocks) {
+      ride_along_copy(ride, block, 64 * Cfg::kWaves);
+      return;
+    }
+    block -= ride.blocks;
+  }
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int grp = wave / (WM * WN), wmn = wave % (WM * WN);
   const int lrow = lane & (BT - 1), lh = lane / BT;
@@ -88,7 +114,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_nn_f32_kernel(const fl
   int tm, tn;
   {
     const int tiles = tiles_m * tiles_n, per = (tiles + 7) >> 3, rem = tiles & 7;
-    const int x = blockIdx.x & 7, i = blockIdx.x >> 3;
+    const int x = block & 7, i = block >> 3;
     const int t = rem == 0 ? x * per + i : (x < rem ? x * per : rem * per + (x - rem) * (per - 1)) + i;
     const int band = t / (8 * tiles_n), in = t - band * 8 * tiles_n, h = min(8, tiles_m - 8 * band);
     tn = in / h;
@@ -99,12 +125,13 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_nn_f32_kernel(const fl
   // accumulator register v of block row i: matrix row of this lane's result
   auto row_of = [&](int i, int v) { return BT * i + (BT == 32 ? 8 * (v >> 2) + 4 * lh + (v & 3) : 4 * lh + v); };
   typedef typename Vec<TN>::type vec;
-  auto c_row = [&](int row, bool* whole) -> float* {
+  auto c_row = [&](int row, bool* whole) -> long long {  // element of C and D, -1 outside the matrix
     const int m = m0 + row, n = n0 + TN * lrow;
     *whole = n + TN <= N;
-    return live && m < M && n < N ? C + (long long)m * N + n : nullptr;
+    return live && m < M && n < N ? (long long)m * N + n : -1;
   };
-  auto fetch = [&](const float* c, bool whole) {
+  auto fetch = [&](long long at, bool whole) {
+    const float* c = at >= 0 ? C + at : nullptr;
     vec v;
     if constexpr (TN == 1) {
       v = c ? *c : 0.0f;
@@ -119,8 +146,9 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_nn_f32_kernel(const fl
     }
     return v;
   };
-  auto put = [&](float* c, bool whole, vec v) {
-    if (!c) return;
+  auto put = [&](long long at, bool whole, vec v) {
+    if (at < 0) return;
+    float* c = D + at;
     if constexpr (TN == 1) {
       *c = v;
     } else {
@@ -190,7 +218,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_nn_f32_kernel(const fl
 #pragma unroll
       for (int u = 0; u < kMine; ++u) {
         bool whole;
-        const float* c = c_row(row_of((grp * kMine + u) / kAcc, (grp * kMine + u) % kAcc), &whole);
+        const long long c = c_row(row_of((grp * kMine + u) / kAcc, (grp * kMine + u) % kAcc), &whole);
         cpre[u] = fetch(c, whole);
       }
     }
@@ -235,7 +263,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_nn_f32_kernel(const fl
 #pragma unroll
     for (int u = 0; u < kMine; ++u) {
       bool whole;
-      const float* c = c_row(row_of((grp * kMine + u) / kAcc, (grp * kMine + u) % kAcc), &whole);
+      const long long c = c_row(row_of((grp * kMine + u) / kAcc, (grp * kMine + u) % kAcc), &whole);
       cpre[u] = fetch(c, whole);
     }
   }
@@ -246,7 +274,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_nn_f32_kernel(const fl
 #pragma unroll
       for (int v = 0; v < kAcc; ++v) {
         bool whole;
-        float* c = c_row(row_of(i, v), &whole);
+        const long long c = c_row(row_of(i, v), &whole);
         vec y = fetch(c, whole);
         if constexpr (TN == 1) {
           y += acc[i][0][v];
@@ -282,27 +310,27 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_nn_f32_kernel(const fl
 #pragma unroll
       for (int g = 1; g < KG; ++g) sum += p[(size_t)g * WM * WN * kUnits * 64];
       bool whole;
-      float* c = c_row(row_of(unit / kAcc, unit % kAcc), &whole);
+      const long long c = c_row(row_of(unit / kAcc, unit % kAcc), &whole);
       put(c, whole, cpre[u] + sum);
     }
   }
 }
 
 // Rows too long for 32-bit byte offsets over a tile (N or K from 2^24 up): one thread per element of C.
-__global__ void gemm_nn_f32_any_kernel(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, int M, int N, int K) {
+__global__ void gemm_nn_f32_any_kernel(const float* __restrict__ A, const float* __restrict__ B, const float* C, float* D, int M, int N, int K) {
   const long long total = (long long)M * N;
   for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += (long long)gridDim.x * blockDim.x) {
     const long long m = t / N, n = t - m * N;
     float part[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (long long k = 0; k < K; ++k) part[k & 7] += A[m * K + k] * B[k * N + n];
-    C[t] += ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
+    D[t] = C[t] + ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
   }
 }
 
-template <int BT, int TM, int TN, int WM, int WN, int KG>
-void launch_gemm_cfg(const float* A, const float* B, float* C, int M, int N, int K, hipStream_t s) {
+template <int BT, int TM, int TN, int WM, int WN, int KG, bool RIDE = false>
+void launch_gemm_cfg(const float* A, const float* B, const float* C, float* D, int M, int N, int K, const RideCopy& ride, hipStream_t s) {
   using Cfg = GemmCfg<BT, TM, TN, WM, WN, KG>;
-  auto kern = gemm_nn_f32_kernel<BT, TM, TN, WM, WN, KG>;
+  auto kern = gemm_nn_f32_kernel<BT, TM, TN, WM, WN, KG, RIDE>;
   static const bool attr = [&] {
     if (Cfg::kLds) NNCV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::kLds));
     return true;
@@ -310,7 +338,7 @@ void launch_gemm_cfg(const float* A, const float* B, float* C, int M, int N, int
   (void)attr;
   const long long tm = (M + Cfg::kRows - 1) / Cfg::kRows, tn = (N + Cfg::kCols - 1) / Cfg::kCols;
   NNCV_REQUIRE(tm * tn < (1ll << 31), "matmul: too many tiles");
-  hipLaunchKernelGGL(kern, dim3((unsigned)(tm * tn)), dim3(64 * Cfg::kWaves), Cfg::kLds, s, A, B, C, M, N, K, (int)tm, (int)tn);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(tm * tn + ride.blocks)), dim3(64 * Cfg::kWaves), Cfg::kLds, s, A, B, C, D, M, N, K, (int)tm, (int)tn, ride);
 }
 
 }  // namespace
@@ -328,7 +356,7 @@ namespace {
 struct GemmForm {
   int rows, cols;
   double fixed_us, k_us, tile_us;
-  void (*launch)(const float*, const float*, float*, int, int, int, hipStream_t);
+  void (*launch)(const float*, const float*, const float*, float*, int, int, int, const RideCopy&, hipStream_t);
 };
 const GemmForm kForms[] = {
     {128, 128, 5.7, 0.00367, 9.0, launch_gemm_cfg<32, 2, 2, 2, 2, 1>},
@@ -342,12 +370,27 @@ const GemmForm kForms[] = {
 
 }  // namespace
 
-void launch_gemm_nn_f32(const float* A, const float* B, float* C, int M, int N, int K, hipStream_t s) {
+void launch_copy16(const RideCopy& r, hipStream_t s) {
+  if (r.bytes == 0) return;
+  hipLaunchKernelGGL(copy16_kernel, dim3((unsigned)r.blocks), dim3(256), 0, s, r);
+  NNCV_HIP_CHECK(hipGetLastError());
+}
+
+void launch_gemm_nn_f32(const float* A, const float* B, const float* C, float* D, int M, int N, int K, hipStream_t s, const RideCopy* ride) {
   NNCV_REQUIRE(M > 0 && N > 0 && K > 0, "matmul: empty operand");
   ProfScope prof("gemm_nn_f32", 2.0 * M * N * K, 4.0 * ((double)M * K + (double)K * N + 2.0 * M * N), s);
+  if (ride && ride->bytes) {
+    if (N < 1 << 24 && K < 1 << 24) {
+      // one form only: these launches are bands of a product whose operands arrive over the bus
+      launch_gemm_cfg<32, 1, 2, 1, 1, 4, true>(A, B, C, D, M, N, K, *ride, s);
+      NNCV_HIP_CHECK(hipGetLastError());
+      return;
+    }
+    launch_copy16(*ride, s);
+  }
   if (N >= 1 << 24 || K >= 1 << 24) {  // 64 rows of A or 32 of B beyond 32-bit byte offsets
     const long long blocks = ((long long)M * N + 255) / 256;
-    hipLaunchKernelGGL(gemm_nn_f32_any_kernel, dim3((unsigned)std::min(blocks, 1ll << 20)), dim3(256), 0, s, A, B, C, M, N, K);
+    hipLaunchKernelGGL(gemm_nn_f32_any_kernel, dim3((unsigned)std::min(blocks, 1ll << 20)), dim3(256), 0, s, A, B, C, D, M, N, K);
     NNCV_HIP_CHECK(hipGetLastError());
     return;
   }
@@ -358,7 +401,7 @@ void launch_gemm_nn_f32(const float* A, const float* B, float* C, int M, int N, 
     const double us = f.fixed_us + (double)rounds * (f.k_us * (f.rows * f.cols / 1024.0) * ((K + 31) / 32 * 32) + f.tile_us);
     if (!best || us < best_us) best = &f, best_us = us;
   }
-  best->launch(A, B, C, M, N, K, s);
+  best->launch(A, B, C, D, M, N, K, RideCopy{}, s);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 

@@ -118,7 +118,7 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
         const void* w = param(op.w, (long long)op.F * Cl * op.K * op.K, where + "w");
         if (dry_) break;
         nd.wt.reset((size_t)Cstored * op.K * op.K * C * es);
-        NNCV_HIP_CHECK(hipMemsetAsync(nd.wt.get(), 0, nd.wt.bytes(), s));
+        if (Cstored > op.F) NNCV_HIP_CHECK(hipMemsetAsync(nd.wt.get(), 0, nd.wt.bytes(), s));
         launch_weight_frsc(w, dt, nd.wt.get(), dt, op.F, Cl, op.K, op.K, C, s);
         if (op.K == 3 && (op.stride == 1 || op.stride == 2) && op.pad == 1 && Cl == C && Cstored == op.F && C % (128 / (int)es) == 0) {
           nd.wfrag.reset((size_t)((op.F + 63) / 64) * 64 * 9 * C * es);

@@ -63,7 +63,7 @@ ConvLayer::ConvLayer(const Desc& d, const void* w, const void* gamma, const void
   } else {
     const int Cp = round_up(d.C, ce), Fp = round_up(d.F, 4);
     wt_.reset((size_t)Fp * d.R * d.S * Cp * es);
-    NNCV_HIP_CHECK(hipMemsetAsync(wt_.get(), 0, wt_.bytes(), s));
+    if (Fp > d.F) NNCV_HIP_CHECK(hipMemsetAsync(wt_.get(), 0, wt_.bytes(), s));  // padding filters; padding channels are written
     launch_weight_frsc(w, d.dt, wt_.get(), d.dt, d.F, d.C, d.R, d.S, Cp, s);
     if (d.R == 3 && d.S == 3 && (d.stride == 1 || d.stride == 2) && d.pad == 1 && d.C % (128 / (int)es) == 0) {
       wfrag_.reset((size_t)((d.F + 63) / 64) * 64 * 9 * d.C * es);
@@ -102,7 +102,7 @@ size_t ConvLayer::workspace_bytes(int N, int H, int W, bool strided) const {
   // strided (operator-level) form of the igemm path stages NHWC copies of input and output
   if (strided && !d_.stem && algo_ == kAlgoIgemm)
     b += align256((size_t)N * H * W * round_up(d_.C, ce) * es) + 2 * align256((size_t)N * OH * OW * round_up(d_.F, 4) * es);
-  if (!strided && splitk_counters_.get()) b += kSplitKWsBytes;
+  if (splitk_counters_.get()) b += kSplitKWsBytes;
   return b;
 }
 
@@ -240,11 +240,16 @@ void ConvLayer::forward_strided(const void* in, Strides4 in_st, int N, int H, in
     launch_relayout(residual, d_.dt, out_st, rin, d_.dt, strides_of(kNHWC, Fp, OH, OW), N, d_.F, Fp, OH, OW, false, s);
   IgemmArgs a{};
   a.in = xin; a.wt = wt_.get(); a.out = yout; a.residual = rin;
+  if (Cp == d_.C && Fp == d_.F) { a.wt_frag = wfrag_.get(); a.wt_frag32 = wfrag32_.get(); }  // the staged tensors are the layer's own
   a.scale = scale_.as<float>(); a.shift = shift_.as<float>();
   a.N = N; a.H = H; a.W = W; a.C = Cp; a.F = Fp; a.R = d_.R; a.S = d_.S; a.OH = OH; a.OW = OW;
   a.stride_h = a.stride_w = d_.stride; a.pad_h = a.pad_w = d_.pad;
   a.relu = d_.relu; a.ldo = Fp; a.batch = 1;
   NNCV_REQUIRE(!(accumulate && (d_.relu || residual)), "conv: accumulate form has no epilogue");
+  if (splitk_counters_.get()) {
+    a.splitk_ws = wsp + in_b + 2 * out_b; a.splitk_ws_bytes = kSplitKWsBytes;
+    a.splitk_counters = splitk_counters_.as<int>(); a.splitk_counters_n = kSplitKCounters;
+  }
   launch_igemm(a, d_.dt, d_.dt, s);
   // out (+)= y : y is NHWC with Fp channels; only the first F are copied
   launch_relayout(yout, d_.dt, strides_of(kNHWC, Fp, OH, OW), out, d_.dt, out_st, N, d_.F, d_.F, OH, OW, accumulate, s);

@@ -1,9 +1,10 @@
 // Bandwidth-bound helpers of the ResNet-18 path: pooling, layout packing and one-time parameter
 // preparation.  Activations are NHWC inside the library (channels contiguous), so every kernel
 // here maps lanes to the channel axis and moves 16 bytes per lane where the shape allows.
+#include <algorithm>
 #include <type_traits>
 
-#include "common.hpp"
+#include "mfma_tile.hpp"
 
 namespace nncv_hip {
 
@@ -541,6 +542,107 @@ __global__ void relayout_kernel(const Ts* __restrict__ src, Strides4 ss, Td* __r
   *d = accumulate ? (Td)((float)*d + v) : (Td)v;
 }
 
+// NCHW <-> NHWC: per image a transposition of [C][P] (P = H * W pixels), 64 channels x 64 pixels through LDS so that both
+// sides move whole rows (the element-wise kernel above walks one side with a stride of a plane, and divides 64-bit
+// indices four times per element).  CFAST: the destination's channels are contiguous (dc = 1, sp = 1), otherwise its
+// pixels are (dp = 1, sc = 1).  The side with contiguous channels is walked flat over (pixel, channel), which keeps
+// tensors of a few channels contiguous as well.  Either side may be pinned host memory: every byte is touched once.
+template <typename Ts, typename Td, bool CFAST>
+__global__ __launch_bounds__(256) void relayout_tile_kernel(const Ts* __restrict__ src, long long sn, long long sc, long long sp,
+                                                            Td* __restrict__ dst, long long dn, long long dc, long long dp, int Cs, int Cd,
+                                                            int P, int accumulate) {
+  __shared__ float tile[64][65];  // [channel][pixel]
+  const int p0 = blockIdx.x * 64, c0 = blockIdx.y * 64, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int pw = min(64, P - p0), cw = min(64, Cd - c0), cr = min(64, Cs - c0);  // cr: channels the source has (the rest are zero)
+  const Ts* s = src + blockIdx.z * sn + p0 * sp + c0 * sc;
+  Td* d = dst + blockIdx.z * dn + p0 * dp + c0 * dc;
+  const float inv_cw = 1.0f / (float)cw, inv_cr = 1.0f / (float)max(cr, 1);
+  // the side with contiguous pixels: four of them per lane, sixteen lanes to a row of the tile (4-byte aligned vectors; over
+  // the bus one-element lanes reach 30 GB/s, these 45)
+  const int px = (t & 15) * 4, row = t >> 4;
+  if constexpr (CFAST) {
+    float v[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int c = row + 16 * i;
+      const Ts* q = s + c * sc + px;
+      typedef Ts T4 __attribute__((ext_vector_type(4)));
+      if (c < cr && px + 4 <= pw) {
+        T4 x;
+        __builtin_memcpy(&x, q, sizeof(x));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[i][e] = (float)x[e];
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[i][e] = c < cr && px + e < pw ? (float)q[e] : 0.0f;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) tile[row + 16 * i][px + e] = v[i][e];
+    __syncthreads();
+    for (int e = t; e < pw * cw; e += 256) {
+      int c;
+      const int p = mt::fast_div(e, cw, inv_cw, &c);
+      Td* q = d + p * dp + c;
+      *q = accumulate ? (Td)((float)*q + tile[c][p]) : (Td)tile[c][p];
+    }
+  } else {
+    typedef Td T4 __attribute__((ext_vector_type(4)));
+    T4 old[4] = {};
+    if (accumulate) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int c = row + 16 * i;
+        const Td* q = d + c * dc + px;
+        if (c < cw && px + 4 <= pw) {
+          __builtin_memcpy(&old[i], q, sizeof(T4));
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (c < cw && px + e < pw) old[i][e] = q[e];
+        }
+      }
+    }
+    if (cr > 0) {
+      float v[16];
+      int at[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int e = t + 256 * i;
+        int c;
+        const int p = mt::fast_div(e, cr, inv_cr, &c);
+        at[i] = e < pw * cr ? c * 65 + p : -1;
+        v[i] = e < pw * cr ? (float)s[p * sp + c] : 0.0f;
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (at[i] >= 0) (&tile[0][0])[at[i]] = v[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int c = row + 16 * i;
+      if (c >= cw) continue;
+      Td* q = d + c * dc + px;
+      T4 y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float x = c < cr ? tile[c][px + e] : 0.0f;
+        y[e] = accumulate ? (Td)((float)old[i][e] + x) : (Td)x;
+      }
+      if (px + 4 <= pw) {
+        __builtin_memcpy(q, &y, sizeof(T4));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (px + e < pw) q[e] = y[e];
+      }
+    }
+  }
+}
+
 void launch_relayout(const void* src, int src_dt, Strides4 ss, void* dst, int dst_dt, Strides4 ds, int N, int Cs, int Cd,
                      int H, int W, bool accumulate, hipStream_t s) {
   const long long work = (long long)N * Cd * H * W;
@@ -548,6 +650,33 @@ void launch_relayout(const void* src, int src_dt, Strides4 ss, void* dst, int ds
   const long long grid = (work + 255) / 256;
   NNCV_REQUIRE(grid < (1ll << 31), "relayout: grid too large");
   const int cf = ds.c == 1;
+  // whole planes on one side, whole pixels on the other: through LDS.  (A plane of up to 2^31 pixels; grid.z holds 65535.)
+  if (ss.h == W * ss.w && ds.h == W * ds.w && N <= 65535 && (long long)H * W < (1ll << 31) - 64 &&
+      ((ss.w == 1 && ds.c == 1) || (ss.c == 1 && ds.w == 1))) {
+    int P = H * W;
+    if (P == 1 && Cs == Cd && ss.c == 1 && ds.c == 1) {  // one pixel per image: its channels are the row that is moved
+      P = Cd;
+      Cs = Cd = 1;
+      ss.w = ds.w = 1;
+      ds.c = 0;  // (any value but 1: the rows form below)
+    }
+    const dim3 grid((unsigned)((P + 63) / 64), (unsigned)((Cd + 63) / 64), (unsigned)N);
+    ProfScope prof("relayout", 0.0, (double)N * P * ((double)Cs * dtype_size(src_dt) + (double)Cd * dtype_size(dst_dt) * (accumulate ? 2 : 1)), s);
+#define LAUNCH(TS, TD)                                                                                                              \
+  if (ss.w == 1 && ds.c == 1)                                                                                                       \
+    hipLaunchKernelGGL((relayout_tile_kernel<TS, TD, true>), grid, dim3(256), 0, s, (const TS*)src, ss.n, ss.c, ss.w, (TD*)dst,     \
+                       ds.n, ds.c, ds.w, Cs, Cd, P, accumulate ? 1 : 0);                                                            \
+  else                                                                                                                              \
+    hipLaunchKernelGGL((relayout_tile_kernel<TS, TD, false>), grid, dim3(256), 0, s, (const TS*)src, ss.n, ss.c, ss.w, (TD*)dst,    \
+                       ds.n, ds.c, ds.w, Cs, Cd, P, accumulate ? 1 : 0)
+    if (src_dt == kF32 && dst_dt == kF32) { LAUNCH(float, float); }
+    else if (src_dt == kF32 && dst_dt == kF16) { LAUNCH(float, half_t); }
+    else if (src_dt == kF16 && dst_dt == kF16) { LAUNCH(half_t, half_t); }
+    else if (src_dt == kF16 && dst_dt == kF32) { LAUNCH(half_t, float); }
+#undef LAUNCH
+    NNCV_HIP_CHECK(hipGetLastError());
+    return;
+  }
 #define LAUNCH(TS, TD) \
   hipLaunchKernelGGL((relayout_kernel<TS, TD>), dim3((unsigned)grid), dim3(256), 0, s, (const TS*)src, ss, (TD*)dst, ds, N, Cs, Cd, H, W, cf, accumulate ? 1 : 0)
   if (src_dt == kF32 && dst_dt == kF32) LAUNCH(float, float);
@@ -684,22 +813,33 @@ void launch_stem_pack(const void* src, int src_dt, void* dst, int dst_dt, int N,
 // ---------------------------------------------------------------------------------------------
 // one-time parameter preparation
 // ---------------------------------------------------------------------------------------------
+// One workgroup per filter: its [C][R*S] values are read once, in order (they may lie in pinned host memory), a chunk of
+// channels at a time through LDS, and written as [R*S][Cp] rows.
 template <typename Ts, typename Td>
-__global__ void weight_frsc_kernel(const Ts* __restrict__ w, Td* __restrict__ dst, int F, int C, int R, int S, int Cp) {
-  const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long long)F * R * S * Cp) return;
-  const int c = (int)(idx % Cp);
-  long long r = idx / Cp;
-  const int s = (int)(r % S); r /= S;
-  const int rr = (int)(r % R);
-  const int f = (int)(r / R);
-  dst[idx] = c < C ? (Td)(float)w[(((long long)f * C + c) * R + rr) * S + s] : (Td)0.0f;
+__global__ __launch_bounds__(256) void weight_frsc_kernel(const Ts* __restrict__ w, Td* __restrict__ dst, int C, int RS, int Cp, int cc,
+                                                          int staged) {
+  extern __shared__ float stage[];  // [cc][RS]
+  const long long f = blockIdx.x;
+  const Ts* src = w + f * C * RS;
+  Td* out = dst + f * RS * Cp;
+  for (int c0 = 0; c0 < Cp; c0 += cc) {
+    const int have = max(0, min(cc, C - c0)), width = min(cc, Cp - c0);
+    if (staged)
+      for (int e = threadIdx.x; e < have * RS; e += 256) stage[e] = (float)src[(long long)c0 * RS + e];
+    __syncthreads();
+    for (int e = threadIdx.x; e < width * RS; e += 256) {
+      const int k = e / width, c = e - k * width;
+      out[(long long)k * Cp + c0 + c] = c >= have ? (Td)0.0f : staged ? (Td)stage[c * RS + k] : (Td)(float)src[(long long)(c0 + c) * RS + k];
+    }
+    __syncthreads();
+  }
 }
 
 void launch_weight_frsc(const void* w, int w_dt, void* dst, int dst_dt, int F, int C, int R, int S, int Cp, hipStream_t s) {
-  const long long work = (long long)F * R * S * Cp;
-  const unsigned grid = (unsigned)((work + 255) / 256);
-#define LAUNCH(TS, TD) hipLaunchKernelGGL((weight_frsc_kernel<TS, TD>), dim3(grid), dim3(256), 0, s, (const TS*)w, (TD*)dst, F, C, R, S, Cp)
+  const int RS = R * S;
+  const int staged = RS <= 8192, cc = staged ? std::min(Cp, 8192 / RS) : Cp;  // 32 KB of LDS hold one channel's window at least
+  const size_t lds = staged ? (size_t)cc * RS * 4 : 0;
+#define LAUNCH(TS, TD) hipLaunchKernelGGL((weight_frsc_kernel<TS, TD>), dim3((unsigned)F), dim3(256), lds, s, (const TS*)w, (TD*)dst, C, RS, Cp, cc, staged)
   if (w_dt == kF32 && dst_dt == kF32) LAUNCH(float, float);
   else if (w_dt == kF16 && dst_dt == kF16) LAUNCH(half_t, half_t);
   else if (w_dt == kF32 && dst_dt == kF16) LAUNCH(float, half_t);

@@ -129,6 +129,7 @@ class Context {
   static Context& get();
   void init(int device);  // idempotent; device < 0 keeps the current one
   hipStream_t stream() const { return stream_; }
+  hipEvent_t event(size_t i);  // kept events of the host-buffer calls
   int device() const { return device_; }
   const std::string& arch() const { return arch_; }
   Arena arena;
@@ -140,6 +141,7 @@ class Context {
   bool ready_ = false;
   int device_ = -1;
   hipStream_t stream_ = nullptr;
+  std::vector<hipEvent_t> events_;
   std::string arch_;
 };
 
