@@ -277,6 +277,46 @@ intptr_t rows_per_piece(size_t row_bytes) { return (intptr_t)std::max<size_t>(1,
 // starts without the 5-10 us that a signal from the engine takes.
 RideCopy from_pinned(const void* src, void* dst, size_t bytes) { return RideCopy{src, dst, align256(bytes), 64}; }
 
+// ---- the host-buffer call: the upload of a dense input -----------------------------------------------------------------
+// _mlir_ciface_forward hands over pageable host memory (examples/Res18/main.cpp:79-99).  The input goes to pinned staging
+// memory in pieces, each copied by a few host threads while a kernel fetches the piece before it; a caller buffer that is
+// pinned already is handed to the DMA engine as it is.  Config 4's 9.6 MB: 0.47 ms a call, 0.51 with DMA copies of the pieces.
+// Tried and not kept: cutting the batch into two halves (or a quarter, a quarter and a half) whose forward passes start
+// as soon as their bytes have landed, on streams and workspaces of their own.  The passes of 8-16 images are launch-bound
+// (8 + 8 + 16 images one after the other: 0.41 ms against 0.26 for the 32 at once), submitting a pass costs the host
+// 50-100 us during which the DMA queue ran dry, and the call measured 0.63-0.77 ms against 0.68 before and 0.59 for this
+// form with a pinned buffer.
+// (the runtime copies straight from what it knows)
+bool pointer_is_plain(const void* p) {
+  hipPointerAttribute_t at;
+  if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+    (void)hipGetLastError();  // plain malloc memory is unknown to the runtime: an error, not a fault
+    return true;
+  }
+  return at.type == hipMemoryTypeUnregistered;
+}
+
+// `most`: staging memory to use; a longer input goes round a ring of pieces.  dev has room up to the next 256 bytes.
+void upload_dense(const char* hsrc, size_t bytes, void* dev, PinnedBuffer& pin, hipStream_t s, size_t most = kStageMost) {
+  static const bool plain = getenv("NNCV_HIP_NO_STAGED_UPLOAD") != nullptr;
+  if (plain || !pointer_is_plain(hsrc)) {
+    NNCV_HIP_CHECK(hipMemcpyAsync(dev, hsrc, bytes, hipMemcpyHostToDevice, s));
+    return;
+  }
+  const size_t piece = 2 * kStagePiece, slots = most / piece;
+  char* stage = static_cast<char*>(pin.ensure(align256(std::min(bytes, most))));
+  Context& ctx = Context::get();
+  size_t k = 0;
+  for (size_t off = 0; off < bytes; off += piece, ++k) {
+    const size_t n = std::min(piece, bytes - off);
+    char* at = stage + (k % slots) * piece;
+    if (k >= slots) NNCV_HIP_CHECK(hipEventSynchronize(ctx.event(k % slots)));
+    parallel_copy(at, hsrc + off, n);
+    launch_copy16(from_pinned(at, static_cast<char*>(dev) + off, n), s);
+    if (bytes > most) NNCV_HIP_CHECK(hipEventRecord(ctx.event(k % slots), s));
+  }
+}
+
 // ---- model cache for the handle-less reference ABI ---------------------------------------
 struct CachedModel {
   const void* host_ptr;
@@ -324,10 +364,18 @@ uint64_t fingerprint(const void* p, long long n, size_t es) {
   return h;
 }
 
-std::unique_ptr<ResNet18> build_model(const void* host, long long n, int dt, int algo, hipStream_t s) {
-  DeviceBuffer blob((size_t)n * dtype_size(dt));
-  NNCV_HIP_CHECK(hipMemcpyAsync(blob.get(), host, blob.bytes(), hipMemcpyHostToDevice, s));
-  auto m = std::make_unique<ResNet18>(blob.get(), n, dt, algo, s);
+// A parameter blob on the device, for as long as a network is built from it (47 MB from pageable memory: 1.0 ms through the
+// staging ring, 2.7 through the runtime's own copy).
+constexpr size_t kParamsRing = size_t(16) << 20;
+DeviceBuffer upload_params(const void* host, size_t bytes, hipStream_t s) {
+  DeviceBuffer blob(align256(bytes));
+  upload_dense(static_cast<const char*>(host), bytes, blob.get(), Context::get().pin_in, s, kParamsRing);
+  return blob;
+}
+
+std::unique_ptr<ResNet18> build_model(const void* host, long long n, int dt, int algo, hipStream_t s, DevicePool pool = {}) {
+  const DeviceBuffer blob = upload_params(host, (size_t)n * dtype_size(dt), s);
+  auto m = std::make_unique<ResNet18>(blob.get(), n, dt, algo, s, std::move(pool));
   NNCV_HIP_CHECK(hipStreamSynchronize(s));  // the staging blob dies here
   return m;
 }
@@ -339,8 +387,12 @@ CachedModel& cached_model(const void* host, long long n, int dt, hipStream_t s) 
   for (auto& e : cache)
     if (e.host_ptr == host && e.n == n && e.dt == dt) return e;
   const uint64_t fp = fingerprint(host, n, dtype_size(dt));
-  if (cache.size() >= 4) cache.erase(cache.begin());
-  cache.push_back(CachedModel{host, n, dt, fp, build_model(host, n, dt, kAlgoAuto, s)});
+  DevicePool pool;
+  if (cache.size() >= 4) {  // its passes have ended: these calls wait for theirs
+    if (cache.front().dt == dt && cache.front().model) pool = cache.front().model->take_pool();
+    cache.erase(cache.begin());
+  }
+  cache.push_back(CachedModel{host, n, dt, fp, build_model(host, n, dt, kAlgoAuto, s, std::move(pool))});
   return cache.back();
 }
 
@@ -455,8 +507,7 @@ long long mobilenetv3_elems() {
   return n;
 }
 std::unique_ptr<Graph> build_graph(const GraphOp* ops, int n_ops, int c_in, const void* host, long long n, int dt, hipStream_t s) {
-  DeviceBuffer blob((size_t)n * dtype_size(dt));
-  NNCV_HIP_CHECK(hipMemcpyAsync(blob.get(), host, blob.bytes(), hipMemcpyHostToDevice, s));
+  const DeviceBuffer blob = upload_params(host, (size_t)n * dtype_size(dt), s);
   auto g = std::make_unique<Graph>(ops, n_ops, c_in, blob.get(), n, dt, s);
   NNCV_HIP_CHECK(hipStreamSynchronize(s));  // the staging blob dies here
   return g;
@@ -474,44 +525,6 @@ CachedGraph& cached_mobilenetv3(const void* host, long long n, int dt, hipStream
   if (cache.size() >= 4) cache.erase(cache.begin());
   cache.push_back(CachedGraph{host, n, dt, fp, build_mobilenetv3(host, n, dt, s)});
   return cache.back();
-}
-
-// ---- the host-buffer call: the upload of a dense input -----------------------------------------------------------------
-// _mlir_ciface_forward hands over pageable host memory (examples/Res18/main.cpp:79-99).  The input goes to pinned staging
-// memory in pieces, each copied by a few host threads while a kernel fetches the piece before it; a caller buffer that is
-// pinned already is handed to the DMA engine as it is.  Config 4's 9.6 MB: 0.47 ms a call, 0.51 with DMA copies of the pieces.
-// Tried and not kept: cutting the batch into two halves (or a quarter, a quarter and a half) whose forward passes start
-// as soon as their bytes have landed, on streams and workspaces of their own.  The passes of 8-16 images are launch-bound
-// (8 + 8 + 16 images one after the other: 0.41 ms against 0.26 for the 32 at once), submitting a pass costs the host
-// 50-100 us during which the DMA queue ran dry, and the call measured 0.63-0.77 ms against 0.68 before and 0.59 for this
-// form with a pinned buffer.
-bool host_pointer_is_pinned(const void* p) {
-  hipPointerAttribute_t at;
-  if (hipPointerGetAttributes(&at, p) != hipSuccess) {
-    (void)hipGetLastError();  // plain malloc memory is unknown to the runtime: an error, not a fault
-    return false;
-  }
-  return at.type == hipMemoryTypeHost;
-}
-
-void upload_dense(const char* hsrc, size_t bytes, void* dev, PinnedBuffer& pin, hipStream_t s) {
-  static const bool plain = getenv("NNCV_HIP_NO_STAGED_UPLOAD") != nullptr;
-  if (plain || host_pointer_is_pinned(hsrc)) {
-    NNCV_HIP_CHECK(hipMemcpyAsync(dev, hsrc, bytes, hipMemcpyHostToDevice, s));
-    return;
-  }
-  constexpr size_t piece = 2 * kStagePiece, slots = kStageMost / piece;  // a longer input goes round a ring of pieces
-  char* stage = static_cast<char*>(pin.ensure(align256(std::min(bytes, kStageMost))));
-  Context& ctx = Context::get();
-  size_t k = 0;
-  for (size_t off = 0; off < bytes; off += piece, ++k) {
-    const size_t n = std::min(piece, bytes - off);
-    char* at = stage + (k % slots) * piece;
-    if (k >= slots) NNCV_HIP_CHECK(hipEventSynchronize(ctx.event(k % slots)));
-    parallel_copy(at, hsrc + off, n);
-    launch_copy16(from_pinned(at, static_cast<char*>(dev) + off, n), s);
-    if (bytes > kStageMost) NNCV_HIP_CHECK(hipEventRecord(ctx.event(k % slots), s));
-  }
 }
 
 void forward_abi(nncv_memref2d* dst, nncv_memref4d* src, void* params, int dt) {
@@ -565,7 +578,7 @@ void forward_abi(nncv_memref2d* dst, nncv_memref4d* src, void* params, int dt) {
       graph->graph = build_mobilenetv3(blob, p->sizes[0], dt, s);
       graph->fingerprint = fp;
     } else {
-      model->model = build_model(blob, p->sizes[0], dt, kAlgoAuto, s);
+      model->model = build_model(blob, p->sizes[0], dt, kAlgoAuto, s, model->model->take_pool());
       model->fingerprint = fp;
     }
     enqueue();
@@ -666,11 +679,12 @@ void conv_host(Context& ctx, nncv_memref4d* in, nncv_memref4d* filter, nncv_memr
   const int Cp = (C + 3) / 4 * 4, Fp = (F + 3) / 4 * 4;
   const size_t img_i = (size_t)C * H * W * 4, img_o = (size_t)F * OH * OW * 4, fb = align256((size_t)F * C * R * S * 4);
   const size_t ib = align256(img_i * N), ob = align256(img_o * N);
-  const size_t wt_b = align256((size_t)Fp * R * S * Cp * 4), x_b = align256((size_t)N * H * W * Cp * 4), y_b = align256((size_t)N * OH * OW * Fp * 4);
+  const size_t wt_b = align256((size_t)Fp * R * S * Cp * 4), wf_b = align256(weight_flat_bytes(kF32, Fp, R * S, Cp)), x_b = align256((size_t)N * H * W * Cp * 4), y_b = align256((size_t)N * OH * OW * Fp * 4);
   const bool staged = fb + ib + ob <= kStageMost;
   ctx.order.after_previous(s);
-  ctx.arena.reserve(wt_b + x_b + y_b + (staged ? 0 : fb + ib + ob) + 2048, s);
+  ctx.arena.reserve(wt_b + wf_b + x_b + y_b + (staged ? 0 : fb + ib + ob) + 2048, s);
   char* wt = static_cast<char*>(ctx.arena.take(wt_b));
+  char* wf = static_cast<char*>(ctx.arena.take(wf_b));
   char* x = static_cast<char*>(ctx.arena.take(x_b));
   char* y = static_cast<char*>(ctx.arena.take(y_b));
   char *hF, *hI, *hO;  // what the re-laying kernels read: pinned memory, or device copies of the caller's arrays
@@ -687,8 +701,19 @@ void conv_host(Context& ctx, nncv_memref4d* in, nncv_memref4d* filter, nncv_memr
     upload<4>(in->aligned, in->offset, in->sizes, in->strides, 4, hI, ctx.pin_in, s);
     upload<4>(out->aligned, out->offset, out->sizes, out->strides, 4, hO, ctx.pin_in, s);
   }
-  launch_weight_frsc(hF, kF32, wt, kF32, F, C, R, S, Cp, s);
-  if (Fp > F) launch_fill_f32(reinterpret_cast<float*>(wt) + (size_t)F * R * S * Cp, 0.0f, (long long)(Fp - F) * R * S * Cp, s);
+  IgemmArgs g{};
+  g.in = x; g.wt_flat = wf; g.out = y;
+  g.N = N; g.H = H; g.W = W; g.C = Cp; g.F = Fp; g.R = R; g.S = S; g.OH = OH; g.OW = OW;
+  g.stride_h = g.stride_w = stride; g.ldo = Fp; g.batch = 1;
+  // the filter in the order of the kernel that will read it
+  if (igemm_takes_direct(g, kF32, kF32)) {
+    launch_weight_flat(hF, wf, kF32, F, C, R * S, Cp, s);
+  } else {
+    g.wt = wt;
+    g.wt_flat = nullptr;
+    launch_weight_frsc(hF, kF32, wt, kF32, F, C, R, S, Cp, s);
+    if (Fp > F) launch_fill_f32(reinterpret_cast<float*>(wt) + (size_t)F * R * S * Cp, 0.0f, (long long)(Fp - F) * R * S * Cp, s);
+  }
   const intptr_t step_i = staged ? rows_per_piece(img_i) : N, step_o = staged ? rows_per_piece(img_o) : N;
   for (intptr_t n = 0; n < N; n += step_i) {
     const int k = (int)std::min<intptr_t>(step_i, N - n);
@@ -696,10 +721,6 @@ void conv_host(Context& ctx, nncv_memref4d* in, nncv_memref4d* filter, nncv_memr
     launch_relayout(hI + n * img_i, kF32, strides_of(kNCHW, C, H, W), x + (size_t)n * H * W * Cp * 4, kF32, strides_of(kNHWC, Cp, H, W), k, C, Cp,
                     H, W, false, s);
   }
-  IgemmArgs g{};
-  g.in = x; g.wt = wt; g.out = y;
-  g.N = N; g.H = H; g.W = W; g.C = Cp; g.F = Fp; g.R = R; g.S = S; g.OH = OH; g.OW = OW;
-  g.stride_h = g.stride_w = stride; g.ldo = Fp; g.batch = 1;
   launch_igemm(g, kF32, kF32, s);
   size_t k_ev = 0;
   for (intptr_t n = 0; n < N; n += step_o) {

@@ -180,11 +180,16 @@ struct IgemmArgs {
   size_t splitk_ws_bytes;
   int* splitk_counters;
   int splitk_counters_n;
+  // What conv_direct.hip reads instead of wt and wt_frag: the filters (launch_weight_flat), and the auxiliary filters alone
+  // (the same with one tap); or null.  Behind the fields that the other kernels load.
+  const void *wt_flat, *aux_wt_flat;
 };
 // in_dt: element type of in/wt (kF32 | kF16); out_dt: element type of out/residual.
 // Dispatches to the fast kernel (igemm_fast.hip) when C is a multiple of one K step and the
 // tensors are below 2 GiB, else to the generic one (igemm.hip).
 void launch_igemm(const IgemmArgs& a, int in_dt, int out_dt, hipStream_t s);
+// whether it would launch the kernel of conv_direct.hip, i.e. reads wt_flat (which must be set, as must be what it points to later)
+bool igemm_takes_direct(const IgemmArgs& a, int in_dt, int out_dt);
 // 3x3 pad-1 layers at stride 1 or 2: direct convolution with the haloed input patch resident in LDS
 // (conv3x3_patch.hip); same arguments and epilogue as the igemm kernels.
 bool conv3x3_patch_applicable(const IgemmArgs& a, int in_dt);
@@ -208,6 +213,16 @@ void launch_weight_frag32(const void* w, int w_dt, void* dst, int F, int C, hipS
 // the whole K axis in one step (conv_pairs.hip); same arguments and epilogue as the igemm kernels.
 bool conv_pairs_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 void launch_conv_pairs(const IgemmArgs& a, hipStream_t s);
+// Barrier-free implicit GEMM for fp32 layers and small fp16 layers (conv_direct.hip); `wins`: its modelled time against
+// that of the kernel which would run the layer otherwise.
+enum DirectRival : int { kRivalPatch = 0, kRivalPatchS2 = 1, kRivalIgemmFast = 2, kRivalIgemm = 3, kRivalShortK = 4 };
+bool conv_direct_applicable(const IgemmArgs& a, int in_dt, int out_dt);
+bool conv_direct_wins(const IgemmArgs& a, int dt, DirectRival rival);
+void launch_conv_direct(const IgemmArgs& a, int dt, hipStream_t s);
+size_t weight_flat_bytes(int dt, int F, int RS, int Cp);
+// (rows: the filters are [F][K] already, K contiguous)
+void launch_weight_flat_rows(const void* w, void* dst, int dt, int F, int K, hipStream_t s);
+void launch_weight_flat(const void* w_fcrs, void* dst, int dt, int F, int C, int RS, int Cp, hipStream_t s);
 bool igemm_fast_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 void launch_igemm_fast(const IgemmArgs& a, int in_dt, int out_dt, hipStream_t s);
 

@@ -117,14 +117,16 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
         const int Cl = logical_[op.in[0]];  // channels the filters really have
         const void* w = param(op.w, (long long)op.F * Cl * op.K * op.K, where + "w");
         if (dry_) break;
-        nd.wt.reset((size_t)Cstored * op.K * op.K * C * es);
+        nd.wt.reset((size_t)Cstored * op.K * op.K * C * es, &pool_);
         if (Cstored > op.F) NNCV_HIP_CHECK(hipMemsetAsync(nd.wt.get(), 0, nd.wt.bytes(), s));
         launch_weight_frsc(w, dt, nd.wt.get(), dt, op.F, Cl, op.K, op.K, C, s);
+        nd.wflat.reset(weight_flat_bytes(dt, Cstored, op.K * op.K, C), &pool_);
+        launch_weight_flat(w, nd.wflat.get(), dt, op.F, Cl, op.K * op.K, C, s);
         if (op.K == 3 && (op.stride == 1 || op.stride == 2) && op.pad == 1 && Cl == C && Cstored == op.F && C % (128 / (int)es) == 0) {
-          nd.wfrag.reset((size_t)((op.F + 63) / 64) * 64 * 9 * C * es);
+          nd.wfrag.reset((size_t)((op.F + 63) / 64) * 64 * 9 * C * es, &pool_);
           launch_weight_frag3x3(w, dt, nd.wfrag.get(), dt, op.F, C, s);
           if (dt == kF16 && op.stride == 1 && C % 64 == 0 && op.F % 32 == 0) {
-            nd.wfrag32.reset(weight_frag32_bytes(op.F, C));
+            nd.wfrag32.reset(weight_frag32_bytes(op.F, C), &pool_);
             launch_weight_frag32(w, dt, nd.wfrag32.get(), op.F, C, s);
           }
         }
@@ -135,7 +137,7 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
         NNCV_REQUIRE(op.stride >= 1 && op.pad >= 0, where + "bad geometry");
         const void* w = param(op.w, (long long)C * op.K * op.K, where + "w");
         if (dry_) break;
-        nd.wt.reset((size_t)C * op.K * op.K * es);
+        nd.wt.reset((size_t)C * op.K * op.K * es, &pool_);
         launch_weight_dw(w, dt, nd.wt.get(), dt, C, op.K, s);
         break;
       }
@@ -184,8 +186,8 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
       const int F = Cout, Fs = Cstored > 0 ? Cstored : Cout;
       if (op.gamma >= 0) {
         NNCV_REQUIRE(op.beta >= 0 && op.mean >= 0 && op.var >= 0, where + "BatchNorm needs gamma, beta, mean and var");
-        nd.scale.reset((size_t)Fs * 4);
-        nd.shift.reset((size_t)Fs * 4);
+        nd.scale.reset((size_t)Fs * 4, &pool_);
+        nd.shift.reset((size_t)Fs * 4, &pool_);
         launch_fill_f32(nd.scale.as<float>(), 0.0f, Fs, s);
         launch_fill_f32(nd.shift.as<float>(), 0.0f, Fs, s);
         launch_bn_fold(param(op.gamma, F, where + "gamma"), param(op.beta, F, where + "beta"), param(op.mean, F, where + "mean"),
@@ -195,7 +197,7 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
         const void* b = param(op.bias, F, where + "bias");
         const bool had = nd.shift.get() != nullptr;
         if (!had) {
-          nd.shift.reset((size_t)Fs * 4);
+          nd.shift.reset((size_t)Fs * 4, &pool_);
           launch_fill_f32(nd.shift.as<float>(), 0.0f, Fs, s);
         }
         const unsigned grid = (unsigned)((F + 255) / 256);
@@ -245,7 +247,7 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
         const int Fp = channels_[o.out], S2 = (o.K + (o.pad & 1) + 1) / 2;
         pair_stem_ = i;
         if (dry_) continue;
-        nodes_[i].wt_pairs.reset((size_t)Fp * o.K * S2 * 8 * es);
+        nodes_[i].wt_pairs.reset((size_t)Fp * o.K * S2 * 8 * es, &pool_);
         launch_weight_pairs(param(o.w, (long long)o.F * c_in_ * o.K * o.K, "pair stem w"), dt, nodes_[i].wt_pairs.get(), o.F, Fp, c_in_,
                             o.K, o.pad, s);
       }
@@ -569,7 +571,7 @@ void Graph::forward(const void* src, int N, int H, int W, float* out, void* ws, 
       case NNCV_HIP_OP_CONV: {
         IgemmArgs g{};
         const int dst = nd.add_out >= 0 ? nd.add_out : op.out;
-        g.in = at(op.in[0]); g.wt = nd.wt.get(); g.wt_frag = nd.wfrag.get(); g.wt_frag32 = nd.wfrag32.get(); g.out = at(dst);
+        g.in = at(op.in[0]); g.wt = nd.wt.get(); g.wt_frag = nd.wfrag.get(); g.wt_frag32 = nd.wfrag32.get(); g.wt_flat = nd.wflat.get(); g.out = at(dst);
         g.scale = nd.scale.as<float>(); g.shift = nd.shift.as<float>();
         g.residual = nd.add_res >= 0 ? at(nd.add_res) : (op.in[1] >= 0 ? at(op.in[1]) : nullptr);
         // padding filters (zero rows, zero scale/shift) are computed like any other: o.C >= op.F
@@ -579,6 +581,7 @@ void Graph::forward(const void* src, int N, int H, int W, float* out, void* ws, 
         g.ldo = pitch(dst); g.batch = 1;
         if (pairs && (int)i == pair_stem_) {  // the image as [N][H][W/2][2 pixels x 4 channels]
           g.wt = nd.wt_pairs.get();
+          g.wt_flat = nullptr;
           g.W = a.W / 2; g.C = 8; g.S = (op.K + (op.pad & 1) + 1) / 2;
           g.stride_w = 1; g.pad_w = (op.pad + 1) / 2;
         }

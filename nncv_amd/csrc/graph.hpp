@@ -43,7 +43,7 @@ class Graph {
   struct Node {
     GraphOp op;
     int C = 0;  // channels of in[0] as stored (the network input is padded to a whole vector)
-    DeviceBuffer wt, wfrag, wfrag32, scale, shift;
+    DeviceBuffer wt, wfrag, wfrag32, wflat, scale, shift;
     // Set on a GAVGPOOL that starts "pool -> 1x1 conv + bias -> 1x1 conv + bias -> SCALE of the pooled
     // tensor" whose three intermediate tensors have no other reader: the four operators run as one
     // squeeze-excitation launch and the next three nodes are skipped.
@@ -68,6 +68,7 @@ class Graph {
 
   int dt_, c_in_, n_tensors_ = 0;
   bool dry_ = false;
+  DevicePool pool_;  // the nodes' weights
   std::vector<Node> nodes_;
   std::vector<int> channels_;  // per tensor, as stored (padded to a whole 16-byte vector)
   std::vector<int> logical_;   // per tensor, as the network defines it

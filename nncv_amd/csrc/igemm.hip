@@ -266,14 +266,28 @@ static void launch_typed(const IgemmArgs& a, hipStream_t s) {
   }
 }
 
-void launch_igemm(const IgemmArgs& a_in, int in_dt, int out_dt, hipStream_t s) {
-  IgemmArgs a = a_in;
-  const int ce = in_dt == kF16 ? 8 : 4;
+static IgemmArgs with_bytes(IgemmArgs a, int in_dt) {
   const int pix = a.pix_stride ? a.pix_stride : a.C;
   const unsigned long long in_b = (unsigned long long)a.N * a.H * a.W * pix * dtype_size(in_dt);
   const unsigned long long wt_b = (unsigned long long)a.F * a.R * a.S * a.C * dtype_size(in_dt);
   if (!a.in_bytes) a.in_bytes = in_b < 0xffffffffull ? (unsigned)in_b : 0xffffffffu;
   if (!a.wt_bytes) a.wt_bytes = wt_b < 0xffffffffull ? (unsigned)wt_b : 0xffffffffu;
+  return a;
+}
+
+bool igemm_takes_direct(const IgemmArgs& a_in, int in_dt, int out_dt) {
+  const IgemmArgs a = with_bytes(a_in, in_dt);
+  if (!conv_direct_applicable(a, in_dt, out_dt)) return false;
+  DirectRival rival = kRivalIgemm;
+  if (conv_pairs_applicable(a, in_dt, out_dt)) rival = kRivalShortK;
+  else if (conv3x3_stream_applicable(a, in_dt, out_dt) || conv3x3_patch_applicable(a, in_dt)) rival = a.stride_h == 1 ? kRivalPatch : kRivalPatchS2;
+  else if (igemm_fast_applicable(a, in_dt, out_dt)) rival = kRivalIgemmFast;
+  return conv_direct_wins(a, in_dt, rival);
+}
+
+void launch_igemm(const IgemmArgs& a_in, int in_dt, int out_dt, hipStream_t s) {
+  const IgemmArgs a = with_bytes(a_in, in_dt);
+  const int ce = in_dt == kF16 ? 8 : 4;
   NNCV_REQUIRE(a.C % ce == 0, "igemm: C must be a multiple of the 16-byte chunk");
   NNCV_REQUIRE(a.F % 4 == 0 && a.ldo % 4 == 0, "igemm: F and ldo must be multiples of 4");
   NNCV_REQUIRE(a.batch >= 1 && a.batch <= 65535, "igemm: batch out of range");
@@ -283,6 +297,10 @@ void launch_igemm(const IgemmArgs& a_in, int in_dt, int out_dt, hipStream_t s) {
   NNCV_REQUIRE(a.OH >= 1 && a.OW >= 1 && a.OH <= (a.H + 2 * a.pad_h - a.R) / a.stride_h + 1 &&
                    a.OW <= (a.W + 2 * a.pad_w - a.S) / a.stride_w + 1,
                "igemm: output size does not match input/filter/stride/pad");
+  if (igemm_takes_direct(a, in_dt, out_dt)) {
+    launch_conv_direct(a, in_dt, s);
+    return;
+  }
   if (conv_pairs_applicable(a, in_dt, out_dt)) {
     launch_conv_pairs(a, s);
     return;

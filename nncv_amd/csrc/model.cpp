@@ -53,27 +53,31 @@ ConvLayer::ConvLayer(const Desc& d, const void* w, const void* gamma, const void
   if (d.stem) {
     NNCV_REQUIRE(d.C == 3 && d.R == 7 && d.S == 7 && d.stride == 2 && d.pad == 3, "stem: must be 7x7 s2 p3 over 3 channels");
     NNCV_REQUIRE(d.F % 4 == 0, "stem: F must be a multiple of 4");
-    wt_.reset((size_t)d.F * 224 * es);
+    wt_.reset((size_t)d.F * 224 * es, d.pool);
     launch_stem_weight(w, d.dt, wt_.get(), d.dt, d.F, 0, s);
-    wt_shift_.reset((size_t)d.F * 224 * es);  // pairs start one column further left (fused stem)
+    wflat_.reset(weight_flat_bytes(d.dt, d.F, 7, 32), d.pool);
+    launch_weight_flat_rows(wt_.get(), wflat_.get(), d.dt, d.F, 224, s);
+    wt_shift_.reset((size_t)d.F * 224 * es, d.pool);  // pairs start one column further left (fused stem)
     launch_stem_weight(w, d.dt, wt_shift_.get(), d.dt, d.F, 1, s);
   } else if (algo_ == kAlgoWinograd) {
-    U_.reset((size_t)36 * d.F * d.C * es);
+    U_.reset((size_t)36 * d.F * d.C * es, d.pool);
     launch_wino43_filter(w, d.dt, U_.get(), d.dt, d.F, d.C, s);
   } else {
     const int Cp = round_up(d.C, ce), Fp = round_up(d.F, 4);
-    wt_.reset((size_t)Fp * d.R * d.S * Cp * es);
+    wt_.reset((size_t)Fp * d.R * d.S * Cp * es, d.pool);
     if (Fp > d.F) NNCV_HIP_CHECK(hipMemsetAsync(wt_.get(), 0, wt_.bytes(), s));  // padding filters; padding channels are written
     launch_weight_frsc(w, d.dt, wt_.get(), d.dt, d.F, d.C, d.R, d.S, Cp, s);
+    wflat_.reset(weight_flat_bytes(d.dt, Fp, d.R * d.S, Cp), d.pool);
+    launch_weight_flat(w, wflat_.get(), d.dt, d.F, d.C, d.R * d.S, Cp, s);
     if (d.R == 3 && d.S == 3 && (d.stride == 1 || d.stride == 2) && d.pad == 1 && d.C % (128 / (int)es) == 0) {
-      wfrag_.reset((size_t)((d.F + 63) / 64) * 64 * 9 * d.C * es);
+      wfrag_.reset((size_t)((d.F + 63) / 64) * 64 * 9 * d.C * es, d.pool);
       launch_weight_frag3x3(w, d.dt, wfrag_.get(), d.dt, d.F, d.C, s);
       if (d.dt == kF16 && d.stride == 1 && d.C % 64 == 0 && d.F % 32 == 0) {
-        wfrag32_.reset(weight_frag32_bytes(d.F, d.C));
+        wfrag32_.reset(weight_frag32_bytes(d.F, d.C), d.pool);
         launch_weight_frag32(w, d.dt, wfrag32_.get(), d.F, d.C, s);
       }
       if (d.dt == kF32) {
-        splitk_counters_.reset(kSplitKCounters * sizeof(int));
+        splitk_counters_.reset(kSplitKCounters * sizeof(int), d.pool);
         NNCV_HIP_CHECK(hipMemsetAsync(splitk_counters_.get(), 0, splitk_counters_.bytes(), s));
       }
     }
@@ -81,8 +85,8 @@ ConvLayer::ConvLayer(const Desc& d, const void* w, const void* gamma, const void
   if (gamma) {
     NNCV_REQUIRE(beta && mean && var, "conv: BN needs gamma, beta, mean and var");
     const int Fp = round_up(d.F, 4);
-    scale_.reset((size_t)Fp * 4);
-    shift_.reset((size_t)Fp * 4);
+    scale_.reset((size_t)Fp * 4, d.pool);
+    shift_.reset((size_t)Fp * 4, d.pool);
     launch_fill_f32(scale_.as<float>(), 0.0f, Fp, s);
     launch_fill_f32(shift_.as<float>(), 0.0f, Fp, s);
     launch_bn_fold(gamma, beta, mean, var, d.dt, scale_.as<float>(), shift_.as<float>(), d.F, s);
@@ -116,7 +120,7 @@ void ConvLayer::forward(const void* in, int N, int H, int W, const void* residua
     const int HP = H + 6, WP = (W + 9) / 2;
     launch_stem_pack(in, d_.dt, wsp, d_.dt, N, H, W, s);
     IgemmArgs a{};
-    a.in = wsp; a.wt = wt_.get(); a.out = out;
+    a.in = wsp; a.wt = wt_.get(); a.wt_flat = wflat_.get(); a.out = out;
     a.scale = scale_.as<float>(); a.shift = shift_.as<float>(); a.residual = residual;
     // a filter row is 4 consecutive pixel pairs = 32 contiguous elements: one K step
     a.N = N; a.H = HP; a.W = WP; a.C = 32; a.pix_stride = 8; a.F = d_.F; a.R = 7; a.S = 1; a.OH = OH; a.OW = OW;
@@ -132,7 +136,7 @@ void ConvLayer::forward(const void* in, int N, int H, int W, const void* residua
   }
   NNCV_REQUIRE(d_.C % (16 / (int)es) == 0 && d_.F % 4 == 0, "conv: NHWC igemm needs C %% chunk == 0 and F %% 4 == 0");
   IgemmArgs a{};
-  a.in = in; a.wt = wt_.get(); a.wt_frag = wfrag_.get(); a.wt_frag32 = wfrag32_.get(); a.out = out;
+  a.in = in; a.wt = wt_.get(); a.wt_frag = wfrag_.get(); a.wt_frag32 = wfrag32_.get(); a.wt_flat = wflat_.get(); a.out = out;
   a.scale = scale_.as<float>(); a.shift = shift_.as<float>(); a.residual = residual;
   a.N = N; a.H = H; a.W = W; a.C = d_.C; a.F = d_.F; a.R = d_.R; a.S = d_.S; a.OH = OH; a.OW = OW;
   a.stride_h = a.stride_w = d_.stride; a.pad_h = a.pad_w = d_.pad;
@@ -159,22 +163,23 @@ bool ConvLayer::fuse_shortcut(const ConvLayer& ds, hipStream_t s) {
       d_.C % ce != 0 || !scale_.get() || !ds.scale_.get())
     return false;
   const size_t row = (size_t)9 * d_.C * es;
-  wt_cat_.reset((size_t)(d_.F + q.F) * row);
+  wt_cat_.reset((size_t)(d_.F + q.F) * row, d_.pool);
   NNCV_HIP_CHECK(hipMemsetAsync(wt_cat_.get(), 0, wt_cat_.bytes(), s));
   NNCV_HIP_CHECK(hipMemcpyAsync(wt_cat_.get(), wt_.get(), (size_t)d_.F * row, hipMemcpyDeviceToDevice, s));
   // the shortcut's [F][C] rows become the centre tap (r = s = 1) of otherwise zero 3x3 filters
   NNCV_HIP_CHECK(hipMemcpy2DAsync(wt_cat_.as<char>() + (size_t)d_.F * row + (size_t)4 * d_.C * es, row, ds.wt_.get(),
                                   (size_t)d_.C * es, (size_t)d_.C * es, q.F, hipMemcpyDeviceToDevice, s));
-  scale_cat_.reset((size_t)(d_.F + q.F) * 4);
-  shift_cat_.reset((size_t)(d_.F + q.F) * 4);
+  scale_cat_.reset((size_t)(d_.F + q.F) * 4, d_.pool);
+  shift_cat_.reset((size_t)(d_.F + q.F) * 4, d_.pool);
   NNCV_HIP_CHECK(hipMemcpyAsync(scale_cat_.get(), scale_.get(), (size_t)d_.F * 4, hipMemcpyDeviceToDevice, s));
   NNCV_HIP_CHECK(hipMemcpyAsync(shift_cat_.get(), shift_.get(), (size_t)d_.F * 4, hipMemcpyDeviceToDevice, s));
   NNCV_HIP_CHECK(hipMemcpyAsync(scale_cat_.as<float>() + d_.F, ds.scale_.get(), (size_t)q.F * 4, hipMemcpyDeviceToDevice, s));
   NNCV_HIP_CHECK(hipMemcpyAsync(shift_cat_.as<float>() + d_.F, ds.shift_.get(), (size_t)q.F * 4, hipMemcpyDeviceToDevice, s));
   if (wfrag_.get() && d_.C % (128 / (int)es) == 0) {
-    aux_wfrag_.reset((size_t)((q.F + 63) / 64) * 64 * d_.C * es);
+    aux_wfrag_.reset((size_t)((q.F + 63) / 64) * 64 * d_.C * es, d_.pool);
     launch_weight_frag1x1(ds.wt_.get(), d_.dt, aux_wfrag_.get(), d_.dt, q.F, d_.C, s);  // [F][1][1][C] rows
   }
+  aux_wflat_ = ds.wflat_.get();
   aux_F_ = q.F;
   aux_relu_ = q.relu;
   aux_flops_per_pixel_ = 2.0 * q.F * q.C;
@@ -188,6 +193,7 @@ void ConvLayer::forward_with_shortcut(const void* in, int N, int H, int W, void*
   NNCV_REQUIRE(N > 0 && OH > 0 && OW > 0, "conv: empty tensor");
   IgemmArgs a{};
   a.in = in; a.wt = wt_cat_.get(); a.wt_frag = wfrag_.get(); a.aux_wt_frag = aux_wfrag_.get(); a.out = out;
+  a.wt_flat = wflat_.get(); a.aux_wt_flat = aux_wflat_;
   a.scale = scale_cat_.as<float>(); a.shift = shift_cat_.as<float>();
   a.N = N; a.H = H; a.W = W; a.C = d_.C; a.F = d_.F + aux_F_; a.R = 3; a.S = 3; a.OH = OH; a.OW = OW;
   a.stride_h = a.stride_w = d_.stride; a.pad_h = a.pad_w = 1;
@@ -239,7 +245,7 @@ void ConvLayer::forward_strided(const void* in, Strides4 in_st, int N, int H, in
   if (residual)
     launch_relayout(residual, d_.dt, out_st, rin, d_.dt, strides_of(kNHWC, Fp, OH, OW), N, d_.F, Fp, OH, OW, false, s);
   IgemmArgs a{};
-  a.in = xin; a.wt = wt_.get(); a.out = yout; a.residual = rin;
+  a.in = xin; a.wt = wt_.get(); a.wt_flat = wflat_.get(); a.out = yout; a.residual = rin;
   if (Cp == d_.C && Fp == d_.F) { a.wt_frag = wfrag_.get(); a.wt_frag32 = wfrag32_.get(); }  // the staged tensors are the layer's own
   a.scale = scale_.as<float>(); a.shift = shift_.as<float>();
   a.N = N; a.H = H; a.W = W; a.C = Cp; a.F = Fp; a.R = d_.R; a.S = d_.S; a.OH = OH; a.OW = OW;
@@ -257,7 +263,9 @@ void ConvLayer::forward_strided(const void* in, Strides4 in_st, int N, int H, in
 
 // ---------------------------------------------------------------------------------------------
 
-ResNet18::ResNet18(const void* params, long long n_elems, int dt, int algo3x3, hipStream_t s) : dt_(dt) {
+ResNet18::ResNet18(const void* params, long long n_elems, int dt, int algo3x3, hipStream_t s, DevicePool pool)
+    : dt_(dt), pool_(std::move(pool)) {
+  pool_.rewind();
   NNCV_REQUIRE(n_elems == kResNet18Elems,
                "ResNet-18 params: expected 11699112 elements in the canonical model.bin order, got " + std::to_string(n_elems));
   const size_t es = dtype_size(dt);
@@ -267,6 +275,7 @@ ResNet18::ResNet18(const void* params, long long n_elems, int dt, int algo3x3, h
     ConvLayer::Desc d;
     d.dt = dt; d.C = C; d.F = F; d.R = d.S = R; d.stride = stride; d.pad = pad; d.relu = relu; d.stem = stem;
     d.algo = (R == 3 && stride == 1) ? algo3x3 : kAlgoIgemm;
+    d.pool = &pool_;
     const void* w = take((long long)F * C * R * R);
     const void* g = take(F); const void* b = take(F); const void* m = take(F); const void* v = take(F);
     return std::make_unique<ConvLayer>(d, w, g, b, m, v, s);
@@ -290,9 +299,9 @@ ResNet18::ResNet18(const void* params, long long n_elems, int dt, int algo3x3, h
     }
   const void* fw = take(1000 * 512);
   const void* fb = take(1000);
-  fc_w_.reset((size_t)1000 * 512 * es);
+  fc_w_.reset((size_t)1000 * 512 * es, &pool_);
   NNCV_HIP_CHECK(hipMemcpyAsync(fc_w_.get(), fw, fc_w_.bytes(), hipMemcpyDeviceToDevice, s));
-  fc_b_.reset(1000 * 4);
+  fc_b_.reset(1000 * 4, &pool_);
   launch_cast(fb, dt, fc_b_.get(), kF32, 1000, s);
   NNCV_REQUIRE((p - static_cast<const char*>(params)) == (long long)(kResNet18Elems * es), "ResNet-18 params: table walk mismatch");
 }

@@ -23,6 +23,7 @@ class ConvLayer {
     int C = 0, F = 0, R = 0, S = 0, stride = 1, pad = 0;
     int relu = 0;  // activation applied last (enum Act); 1 = ReLU
     int algo = kAlgoAuto;
+    DevicePool* pool = nullptr;  // where the weights live (it outlives the layer); null = allocations of their own
     bool stem = false;  // 7x7 s2 p3 over 3 channels read from NCHW (pixel-pair packing)
   };
   // w: device pointer to FCHW weights of type `dt`; bn: device pointers gamma,beta,mean,var of
@@ -58,8 +59,9 @@ class ConvLayer {
  private:
   Desc d_;
   int algo_;
-  DeviceBuffer wt_, wfrag_, wfrag32_, U_, scale_, shift_, wt_shift_;
+  DeviceBuffer wt_, wfrag_, wfrag32_, wflat_, U_, scale_, shift_, wt_shift_;
   DeviceBuffer wt_cat_, scale_cat_, shift_cat_;  // this layer's filters followed by the fused shortcut's
+  const void* aux_wflat_ = nullptr;  // the fused shortcut layer's own wflat_
   DeviceBuffer aux_wfrag_;  // the fused shortcut's filters alone, fragment-major (stride-2 patch kernel)
   DeviceBuffer splitk_counters_;  // tickets of the patch kernel's K split (fp32); zero between launches
   int aux_F_ = 0;
@@ -70,7 +72,9 @@ class ConvLayer {
 class ResNet18 {
  public:
   // params_dev: flat device blob of `n_elems` elements of type dt in the canonical tensor order.
-  ResNet18(const void* params_dev, long long n_elems, int dt, int algo3x3, hipStream_t s);
+  // pool: device memory to build in first, of a network that is gone.
+  ResNet18(const void* params_dev, long long n_elems, int dt, int algo3x3, hipStream_t s, DevicePool pool = {});
+  DevicePool take_pool() { return std::move(pool_); }  // the network is not used after this
   int dtype() const { return dt_; }
   size_t workspace_bytes(int N, int H, int W) const;
   // src: NCHW [N,3,H,W] of type dt (device); logits: [N,1000] of type dt (device).
@@ -85,6 +89,7 @@ class ResNet18 {
 
  private:
   int dt_;
+  DevicePool pool_;
   std::unique_ptr<ConvLayer> stem_;
   std::vector<Block> blocks_;
   DeviceBuffer fc_w_, fc_b_;  // [1000][512] dt ; [1000] f32

@@ -552,7 +552,7 @@ __global__ __launch_bounds__(256) void relayout_tile_kernel(const Ts* __restrict
                                                             Td* __restrict__ dst, long long dn, long long dc, long long dp, int Cs, int Cd,
                                                             int P, int accumulate) {
   __shared__ float tile[64][65];  // [channel][pixel]
-  const int p0 = blockIdx.x * 64, c0 = blockIdx.y * 64, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int p0 = blockIdx.x * 64, c0 = blockIdx.y * 64, t = threadIdx.x;
   const int pw = min(64, P - p0), cw = min(64, Cd - c0), cr = min(64, Cs - c0);  // cr: channels the source has (the rest are zero)
   const Ts* s = src + blockIdx.z * sn + p0 * sp + c0 * sc;
   Td* d = dst + blockIdx.z * dn + p0 * dp + c0 * dc;

@@ -3,6 +3,7 @@
 // The reference has no counterpart (its object runs in host memory); the only device code it
 // contains are cudaMalloc/cudaFree wrappers (src/nncv/vm/cuda/vm_alloc_cuda.cu:6-10).
 #pragma once
+#include <algorithm>
 #include <memory>
 #include <mutex>
 #include <vector>
@@ -11,15 +12,17 @@
 
 namespace nncv_hip {
 
+class DevicePool;
+
 class DeviceBuffer {
  public:
   DeviceBuffer() = default;
   explicit DeviceBuffer(size_t bytes) { reset(bytes); }
   DeviceBuffer(const DeviceBuffer&) = delete;
   DeviceBuffer& operator=(const DeviceBuffer&) = delete;
-  DeviceBuffer(DeviceBuffer&& o) noexcept : p_(o.p_), n_(o.n_) { o.p_ = nullptr; o.n_ = 0; }
+  DeviceBuffer(DeviceBuffer&& o) noexcept : p_(o.p_), n_(o.n_), owned_(o.owned_) { o.p_ = nullptr; o.n_ = 0; }
   DeviceBuffer& operator=(DeviceBuffer&& o) noexcept {
-    if (this != &o) { release(); p_ = o.p_; n_ = o.n_; o.p_ = nullptr; o.n_ = 0; }
+    if (this != &o) { release(); p_ = o.p_; n_ = o.n_; owned_ = o.owned_; o.p_ = nullptr; o.n_ = 0; }
     return *this;
   }
   ~DeviceBuffer() { release(); }
@@ -27,9 +30,12 @@ class DeviceBuffer {
     release();
     if (bytes) NNCV_HIP_CHECK(hipMalloc(&p_, bytes));
     n_ = bytes;
+    owned_ = true;
   }
+  // from `pool` (which outlives this), or an allocation of its own where there is none
+  void reset(size_t bytes, DevicePool* pool);
   void release() {
-    if (p_) (void)hipFree(p_);
+    if (p_ && owned_) (void)hipFree(p_);
     p_ = nullptr;
     n_ = 0;
   }
@@ -40,7 +46,35 @@ class DeviceBuffer {
  private:
   void* p_ = nullptr;
   size_t n_ = 0;
+  bool owned_ = true;
 };
+
+// Device memory for the weights of one network: handed out from a few large blocks, freed with the network.  A network has
+// several hundred small arrays, and creating one spent most of its time in as many hipMalloc calls.  A network that takes
+// the place of an idle one can take over its blocks (rewind): mapping and unmapping 100 MB costs the host 4 ms.
+class DevicePool {
+ public:
+  void* take(size_t bytes) {
+    bytes = (bytes + 255) & ~size_t(255);
+    while (cur_ < blocks_.size() && off_ + bytes > blocks_[cur_].bytes()) ++cur_, off_ = 0;
+    if (cur_ == blocks_.size()) blocks_.emplace_back(std::max(bytes, size_t(8) << 20));
+    off_ += bytes;
+    return blocks_[cur_].as<char>() + off_ - bytes;
+  }
+  void rewind() { cur_ = off_ = 0; }  // nothing handed out so far is used any more
+
+ private:
+  std::vector<DeviceBuffer> blocks_;
+  size_t cur_ = 0, off_ = 0;
+};
+
+inline void DeviceBuffer::reset(size_t bytes, DevicePool* pool) {
+  if (!pool || bytes == 0) return reset(bytes);
+  release();
+  p_ = pool->take(bytes);
+  n_ = bytes;
+  owned_ = false;
+}
 
 class PinnedBuffer {
  public:
