@@ -53,13 +53,13 @@ StreamOrder::~StreamOrder() {
   if (ev_) (void)hipEventDestroy(ev_);
 }
 
-void StreamOrder::after_previous(hipStream_t s) {
+void StreamOrder::after_previous(hipStream_t s, bool blocking) {
   if (!pending_ || tail_ == s) return;
   if (many_) {
     NNCV_HIP_CHECK(hipStreamWaitEvent(s, ev_, 0));
   } else {
     NNCV_HIP_CHECK(hipDeviceSynchronize());
-    many_ = true;
+    many_ = !blocking;
   }
   pending_ = false;
 }
@@ -125,7 +125,7 @@ struct Sync {
   bool capturing;
   explicit Sync(void* user) : s(user ? static_cast<hipStream_t>(user) : Context::get().stream()), own(user == nullptr) {
     capturing = !own && stream_is_capturing(s);
-    if (!capturing) Context::get().order.after_previous(s);
+    if (!capturing) Context::get().order.after_previous(s, own);
   }
   bool done = false;
   void finish() {
@@ -159,7 +159,7 @@ struct HandleSync {
   bool own;
   bool done = false;
   HandleSync(HandleState& hs, void* user) : h(hs), s(user ? static_cast<hipStream_t>(user) : Context::get().stream()), own(user == nullptr) {
-    h.order.after_previous(s);
+    h.order.after_previous(s, own);
   }
   void finish() {
     if (own) NNCV_HIP_CHECK(hipStreamSynchronize(s));
@@ -532,7 +532,7 @@ void forward_abi(nncv_memref2d* dst, nncv_memref4d* src, void* params, int dt) {
   Context& ctx = Context::get();
   ctx.init(-1);
   hipStream_t s = ctx.stream();
-  ctx.order.after_previous(s);
+  ctx.order.after_previous(s, true);
   const size_t es = dtype_size(dt);
   const nncv_memref1d* p = static_cast<const nncv_memref1d*>(params);
   NNCV_REQUIRE(p->aligned && p->strides[0] == 1, "params must be a dense rank-1 memref");
@@ -615,7 +615,7 @@ void matmul_host(Context& ctx, nncv_memref2d* a, nncv_memref2d* b, nncv_memref2d
     total = at_c.back() + align256(rows * row_c);
   }
   at_a.push_back(total);
-  ctx.order.after_previous(s);
+  ctx.order.after_previous(s, true);
   ctx.arena.reserve(total + 1024, s);
   char* dev = static_cast<char*>(ctx.arena.take(total));
   auto f32 = [](char* p) { return reinterpret_cast<float*>(p); };
@@ -681,7 +681,7 @@ void conv_host(Context& ctx, nncv_memref4d* in, nncv_memref4d* filter, nncv_memr
   const size_t ib = align256(img_i * N), ob = align256(img_o * N);
   const size_t wt_b = align256((size_t)Fp * R * S * Cp * 4), wf_b = align256(weight_flat_bytes(kF32, Fp, R * S, Cp)), x_b = align256((size_t)N * H * W * Cp * 4), y_b = align256((size_t)N * OH * OW * Fp * 4);
   const bool staged = fb + ib + ob <= kStageMost;
-  ctx.order.after_previous(s);
+  ctx.order.after_previous(s, true);
   ctx.arena.reserve(wt_b + wf_b + x_b + y_b + (staged ? 0 : fb + ib + ob) + 2048, s);
   char* wt = static_cast<char*>(ctx.arena.take(wt_b));
   char* wf = static_cast<char*>(ctx.arena.take(wf_b));
@@ -748,6 +748,8 @@ struct nncv_hip_model_impl {
   int passes = 0;  // forward passes the caller keeps in flight next to this handle's; 0 = the process-wide default
 };
 struct nncv_hip_conv_impl {
+  explicit nncv_hip_conv_impl(size_t block) : pool(block) {}
+  DevicePool pool;
   std::unique_ptr<ConvLayer> c;
 };
 struct nncv_hip_graph_impl {
@@ -758,7 +760,9 @@ struct nncv_hip_graph_impl {
 }  // namespace
 
 struct nncv_hip_model : nncv_hip_model_impl {};
-struct nncv_hip_conv : nncv_hip_conv_impl {};
+struct nncv_hip_conv : nncv_hip_conv_impl {
+  using nncv_hip_conv_impl::nncv_hip_conv_impl;
+};
 struct nncv_hip_graph : nncv_hip_graph_impl {};
 
 extern "C" {
@@ -1020,23 +1024,28 @@ nncv_hip_conv* nncv_hip_conv_create(int dtype, const void* weights, int F, int C
     ctx.init(-1);
     hipStream_t s = ctx.stream();
     const size_t es = dtype_size(dtype);
-    DeviceBuffer w((size_t)F * C * R * S * es), bn;
-    NNCV_HIP_CHECK(hipMemcpyAsync(w.get(), weights, w.bytes(), hipMemcpyHostToDevice, s));
-    const char* g = nullptr;
-    if (gamma) {
-      NNCV_REQUIRE(beta && mean && var, "conv: BN needs gamma, beta, mean and var");
-      bn.reset((size_t)4 * F * es);
-      const void* srcs[4] = {gamma, beta, mean, var};
-      for (int i = 0; i < 4; ++i)
-        NNCV_HIP_CHECK(hipMemcpyAsync(bn.as<char>() + (size_t)i * F * es, srcs[i], (size_t)F * es, hipMemcpyHostToDevice, s));
-      g = bn.as<char>();
+    NNCV_REQUIRE(!gamma || (beta && mean && var), "conv: BN needs gamma, beta, mean and var");
+    // the filters and the batch-norm rows go up as one piece of staging memory; what the layer keeps is one allocation
+    const void* srcs[5] = {weights, gamma, beta, mean, var};
+    const size_t row = align256((size_t)F * es), wb = (size_t)F * C * R * S * es, n_src = gamma ? 5 : 1;
+    const DeviceBuffer blob(align256(wb) + 4 * row);
+    auto at = [&](size_t i) { return i == 0 ? 0 : align256(wb) + (i - 1) * row; };
+    bool plain = blob.bytes() <= kParamsRing;
+    for (size_t i = 0; i < n_src; ++i) plain = plain && pointer_is_plain(srcs[i]);
+    char* stage = plain ? static_cast<char*>(ctx.pin_in.ensure(blob.bytes())) : nullptr;
+    for (size_t i = 0; i < n_src; ++i) {
+      const size_t bytes = i == 0 ? wb : (size_t)F * es;
+      if (plain) parallel_copy(stage + at(i), static_cast<const char*>(srcs[i]), bytes);
+      else NNCV_HIP_CHECK(hipMemcpyAsync(blob.as<char>() + at(i), srcs[i], bytes, hipMemcpyHostToDevice, s));
     }
+    if (plain) launch_copy16(from_pinned(stage, blob.get(), at(n_src)), s);
+    const char* g = gamma ? blob.as<char>() + at(1) : nullptr;
     ConvLayer::Desc d;
     d.dt = dtype; d.C = C; d.F = F; d.R = R; d.S = S; d.stride = stride; d.pad = pad; d.relu = relu; d.algo = algo;
-    h = new nncv_hip_conv();
+    h = new nncv_hip_conv(4 * ((size_t)F + 64) * ((size_t)R * S * (C + 8) * es + 128) + (size_t(64) << 10));
+    d.pool = &h->pool;
     try {
-      h->c = std::make_unique<ConvLayer>(d, w.get(), g, g ? g + (size_t)F * es : nullptr, g ? g + (size_t)2 * F * es : nullptr,
-                                         g ? g + (size_t)3 * F * es : nullptr, s);
+      h->c = std::make_unique<ConvLayer>(d, blob.get(), g, g ? g + row : nullptr, g ? g + 2 * row : nullptr, g ? g + 3 * row : nullptr, s);
       NNCV_HIP_CHECK(hipStreamSynchronize(s));
     } catch (...) {
       delete h;

@@ -54,10 +54,11 @@ class DeviceBuffer {
 // the place of an idle one can take over its blocks (rewind): mapping and unmapping 100 MB costs the host 4 ms.
 class DevicePool {
  public:
+  DevicePool(size_t block = size_t(8) << 20) : block_(block) {}
   void* take(size_t bytes) {
     bytes = (bytes + 255) & ~size_t(255);
     while (cur_ < blocks_.size() && off_ + bytes > blocks_[cur_].bytes()) ++cur_, off_ = 0;
-    if (cur_ == blocks_.size()) blocks_.emplace_back(std::max(bytes, size_t(8) << 20));
+    if (cur_ == blocks_.size()) blocks_.emplace_back(std::max(bytes, block_));
     off_ += bytes;
     return blocks_[cur_].as<char>() + off_ - bytes;
   }
@@ -65,7 +66,7 @@ class DevicePool {
 
  private:
   std::vector<DeviceBuffer> blocks_;
-  size_t cur_ = 0, off_ = 0;
+  size_t block_, cur_ = 0, off_ = 0;
 };
 
 inline void DeviceBuffer::reset(size_t bytes, DevicePool* pool) {
@@ -140,14 +141,15 @@ std::vector<hipStream_t> pick_streams(int want, int* found);
 // record behind every call costs 4 us of queue time between two kernels (16.7 against 20.7 us per launch of a 16 us kernel,
 // 2.7 against 8.4 of a short one).  The first call on a second stream waits for the device once, and from then on every
 // call that leaves work pending records an event on its own (then certainly live) stream, for a later call on another
-// stream to wait on: a caller stream destroyed in between is never touched again.
+// stream to wait on: a caller stream destroyed in between is never touched again.  A call that waits for its own work
+// before it returns (host buffers, or no stream given) is no second stream: it waits for the device first.
 class StreamOrder {
  public:
   StreamOrder() = default;
   StreamOrder(const StreamOrder&) = delete;
   StreamOrder& operator=(const StreamOrder&) = delete;
   ~StreamOrder();
-  void after_previous(hipStream_t s);
+  void after_previous(hipStream_t s, bool blocking);  // blocking: the call that begins waits for its work before it returns
   void note(hipStream_t s, bool pending);  // the call that ends here left work in flight on s, or none
 
  private:
