@@ -215,7 +215,7 @@ bool conv_pairs_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 void launch_conv_pairs(const IgemmArgs& a, hipStream_t s);
 // Barrier-free implicit GEMM for fp32 layers and small fp16 layers (conv_direct.hip); `wins`: its modelled time against
 // that of the kernel which would run the layer otherwise.
-enum DirectRival : int { kRivalPatch = 0, kRivalPatchS2 = 1, kRivalIgemmFast = 2, kRivalIgemm = 3, kRivalShortK = 4 };
+enum DirectRival : int { kRivalPatch = 0, kRivalPatchS2 = 1, kRivalIgemmFast = 2, kRivalIgemm = 3, kRivalShortK = 4, kRivalRing = 5 };
 bool conv_direct_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 bool conv_direct_wins(const IgemmArgs& a, int dt, DirectRival rival);
 void launch_conv_direct(const IgemmArgs& a, int dt, hipStream_t s);
@@ -223,6 +223,10 @@ size_t weight_flat_bytes(int dt, int F, int RS, int Cp);
 // (rows: the filters are [F][K] already, K contiguous)
 void launch_weight_flat_rows(const void* w, void* dst, int dt, int F, int K, hipStream_t s);
 void launch_weight_flat(const void* w_fcrs, void* dst, int dt, int F, int C, int RS, int Cp, hipStream_t s);
+// fp16 implicit GEMM through an LDS ring filled straight from memory (conv_ring.hip); us: its modelled time
+bool conv_ring_applicable(const IgemmArgs& a, int in_dt, int out_dt);
+double conv_ring_us(const IgemmArgs& a);
+void launch_conv_ring(const IgemmArgs& a, hipStream_t s);
 bool igemm_fast_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 void launch_igemm_fast(const IgemmArgs& a, int in_dt, int out_dt, hipStream_t s);
 

@@ -482,9 +482,10 @@ bool conv_direct_wins(const IgemmArgs& a, int dt, DirectRival rival) {
       ((long long)((a.F + 31) / 32) * (((long long)a.N * a.OH * a.OW + 63) / 64) >= 64 || (a.N > 1 && a.OH * a.OW < 32)))
     return false;
   // fp16 implicit GEMMs stay with the LDS kernel once its 128 x 128 tiles fill the chip: the models below end there.
-  if (rival == kRivalIgemmFast && dt == kF16 && (long long)((a.F + 127) / 128) * (((long long)a.N * a.OH * a.OW + 127) / 128) >= 256) return false;
+  if ((rival == kRivalIgemmFast || rival == kRivalRing) && dt == kF16 && (long long)((a.F + 127) / 128) * (((long long)a.N * a.OH * a.OW + 127) / 128) >= 256) return false;
   double us = 0;
   if (!best_form(a, dt, &us)) return false;
+  if (rival == kRivalRing) return us < 0.97 * conv_ring_us(a);
   // margins cover the fits' errors: the fp16 3x3 stride-1 kernels' times are the least well fitted
   const double margin = dt == kF32 ? 0.97 : rival == kRivalPatch ? 0.85 : 0.9;
   return us < margin * other_us(a, dt, rival);

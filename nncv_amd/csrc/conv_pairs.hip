@@ -186,12 +186,12 @@ bool conv_pairs_applicable(const IgemmArgs& a, int in_dt, int out_dt) {
   if (window)
     return !off && a.C == 8 && pix == 8 && a.F <= 64 && a.residual == nullptr && (a.relu & ~0xff) == 0 &&
            (long long)a.N * a.H * a.W * 16 < (long long)kOOBc;
-  // 1x1, stride 1, no padding: the output pixel is the input pixel.  Channel counts that the pipelined
-  // kernel takes as well (multiples of 32) come here only for small launches, where its barriers per K
-  // step are all latency (MobileNetV3's 96-channel layers at 14x14 and 7x7: 0.449 -> 0.444 ms per
-  // batch of 32); on YOLOv5s' large 1x1 layers it is the faster one (1.27 against 1.32 ms).
+  // 1x1, stride 1, no padding: the output pixel is the input pixel.  The LDS ring (conv_ring.hip) is the better one for whole
+  // multiples of 32 channels (64 -> 32 at 5880 pixels: 2.9 against 3.2 us), and from 24 channels on where its 64 x 64 tiles
+  // give every CU one and more than 32 filters share a pixel's line (40 -> 240 at 6272 pixels: 3.5 against 4.7).
+  const bool ring = a.C % 32 == 0 || (a.C > 16 && a.F > 32 && (P + 63) / 64 * ((a.F + 63) / 64) >= 256);
   return !off_pw && a.R == 1 && a.S == 1 && a.stride_h == 1 && a.stride_w == 1 && a.pad_h == 0 && a.pad_w == 0 && a.OH == a.H &&
-         a.OW == a.W && a.C % 8 == 0 && (a.C % 32 != 0 || P <= 8192) && a.C <= 144 && pix % 8 == 0 && P * pix * 2 < (long long)kOOBc;
+         a.OW == a.W && a.C % 8 == 0 && !ring && a.C <= 144 && pix % 8 == 0 && P * pix * 2 < (long long)kOOBc;
 }
 
 template <bool PW, int R, int S, int KST, int NI>
@@ -223,15 +223,15 @@ void launch_conv_pairs(const IgemmArgs& a, hipStream_t s) {
     if (a.F > 32) launch_pairs_cfg<false, 3, 2, 3, 2>(a, "conv_pairs<f16,3x2,64>", s);
     else launch_pairs_cfg<false, 3, 2, 3, 1>(a, "conv_pairs<f16,3x2,32>", s);
   } else {
-    // K steps in registers: 1 (16 channels), 3 (..48), 6 (..96), 9 (..144); 64 filters per wave tile
-    // while the registers allow it
+    // K steps in registers: 1 (16 channels), 3 (..48), 6 (..96), 9 (..144).  64 filters per wave tile only for launches that
+    // fill the chip all the same (24 -> 112 at 1440 pixels: 4.1 us with 64, 3.1 with 32)
     const int kst = (a.C / 8 + 1) / 2;
+    const bool many = ((long long)a.N * a.OH * a.OW + 63) / 64 * ((a.F + 63) / 64) >= 1024;
     if (kst <= 1) {
-      if (a.F > 32) launch_pairs_cfg<true, 1, 1, 1, 2>(a, "conv1x1_shortk<f16,16,64>", s);
+      if (a.F > 32 && many) launch_pairs_cfg<true, 1, 1, 1, 2>(a, "conv1x1_shortk<f16,16,64>", s);
       else launch_pairs_cfg<true, 1, 1, 1, 1>(a, "conv1x1_shortk<f16,16,32>", s);
     } else if (kst <= 3) {
-      if (a.F > 32) launch_pairs_cfg<true, 1, 1, 3, 2>(a, "conv1x1_shortk<f16,48,64>", s);
-      else launch_pairs_cfg<true, 1, 1, 3, 1>(a, "conv1x1_shortk<f16,48,32>", s);
+      launch_pairs_cfg<true, 1, 1, 3, 1>(a, "conv1x1_shortk<f16,48,32>", s);
     } else if (kst <= 6) {
       launch_pairs_cfg<true, 1, 1, 6, 1>(a, "conv1x1_shortk<f16,96,32>", s);
     } else {

@@ -1,0 +1,46 @@
+"""The fp16 implicit GEMM through an LDS ring (conv_ring.hip) where it can go wrong: every tile form, pixel and filter counts that
+end inside a tile, K axes that end inside a slab, taps that share a slab, strides and padding, one slab, residual before and
+after the activation; against torch on the CPU."""
+import pytest
+import torch
+
+from nncv_amd import abi
+from gpu_util import Conv, FP16_REL_L2, dev, host, nchw, nhwc, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+def rand(seed, *shape):
+    return torch.rand(shape, generator=torch.Generator().manual_seed(seed)).mul_(2).sub_(1).half().float()
+
+
+@pytest.mark.parametrize("N,C,F,H,W,R,stride,pad,act", [
+    (2, 64, 32, 91, 93, 1, 1, 0, "silu"),     # one slab, pixels end inside a tile
+    (3, 96, 136, 37, 41, 1, 1, 0, None),      # the second slab is half full, filters end inside a block
+    (20, 256, 120, 40, 40, 1, 2, 0, "relu"),  # strided pixels
+    (8, 40, 264, 28, 28, 1, 1, 0, "relu"),    # less than one slab
+    (64, 64, 24, 40, 41, 1, 1, 0, "silu"),    # the narrow form
+    (20, 64, 72, 61, 62, 5, 2, 1, "relu"),    # taps of one slab, and halo on every side
+    (2, 16, 40, 70, 61, 3, 1, 1, "silu"),     # four taps to a slab
+    (9, 24, 72, 61, 62, 3, 2, 1, None),       # taps that straddle slabs
+    (8, 40, 72, 64, 64, 5, 1, 4, "relu"),     # the large form, padding wider than the centre
+    (16, 512, 256, 20, 20, 1, 1, 0, "relu"),  # two buffers
+    (8, 512, 128, 60, 60, 1, 1, 0, "relu"),   # the wide form
+])
+def test_ring_kernel_matches_torch(N, C, F, H, W, R, stride, pad, act):
+    oh, ow = (H + 2 * pad - R) // stride + 1, (W + 2 * pad - R) // stride + 1
+    x, w, r = rand(1, N, C, H, W), (rand(2, F, C, R, R) * (2.0 / (R * R * C)) ** 0.5).half().float(), rand(3, N, F, oh, ow)
+    y = torch.nn.functional.conv2d(x, w, stride=stride, padding=pad)
+    f = {None: lambda v: v, "relu": torch.relu, "silu": torch.nn.functional.silu}[act]
+    code = {None: abi.ACT_NONE, "relu": abi.ACT_RELU, "silu": abi.ACT_SILU}[act]
+    layer, xd, rd = Conv(abi.F16, w.numpy(), stride, pad, relu=code), dev(nhwc(x.numpy()), abi.F16), dev(nhwc(r.numpy()), abi.F16)
+    abi.profile_enable(True)
+    try:
+        abi.profile_report()
+        plain, added = host(layer(xd, abi.NHWC)), host(layer(xd, abi.NHWC, residual=rd))
+        tags = list(abi.profile_report())
+    finally:
+        abi.profile_enable(False)
+    assert all(t.startswith("conv_ring<") for t in tags), tags
+    print(tags, flush=True)
+    assert rel_l2(nchw(plain), f(y).numpy()) < 2e-3 < FP16_REL_L2
+    assert rel_l2(nchw(added), f(y + r).numpy()) < 2e-3
