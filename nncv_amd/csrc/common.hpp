@@ -226,6 +226,7 @@ void launch_weight_flat(const void* w_fcrs, void* dst, int dt, int F, int C, int
 // fp16 implicit GEMM through an LDS ring filled straight from memory (conv_ring.hip); us: its modelled time
 bool conv_ring_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 double conv_ring_us(const IgemmArgs& a);
+bool conv_ring_beats_patch_s2(const IgemmArgs& a);
 void launch_conv_ring(const IgemmArgs& a, hipStream_t s);
 bool igemm_fast_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 void launch_igemm_fast(const IgemmArgs& a, int in_dt, int out_dt, hipStream_t s);

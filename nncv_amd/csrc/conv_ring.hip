@@ -38,6 +38,8 @@ struct RingArgs {
   int stride_h, stride_w, pad_h, pad_w, S;
   int act, ldo, chunks, cpt;                          // 16-byte chunks of K, and of one tap
   int tiles_f, tiles_p, pixels_first;
+  int aux_tiles, aux_f0, aux_tap, aux_act, aux_ldo;              // filters from aux_f0 on walk one tap only and go to aux_out; 0: none
+  void* aux_out; unsigned aux_out_bytes;
   float inv_ohw, inv_ow, inv_tiles;
 };
 
@@ -54,16 +56,31 @@ __global__ __launch_bounds__(64 * WP * WF) void conv_ring_kernel(const RingArgs 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int wp = wave % WP, wf = wave / WP;
   int tf, tp;
-  {  // XCD x takes a contiguous run of tiles: its L2 holds a part of the larger operand only
+  bool aux = false;
+  if (MODE == kLines && a.aux_f0 > 0) {
+    // XCD x takes a run of pixel tiles: all filters of the convolution over them, then the auxiliary ones, whose tiles are
+    // short (in between they kept the long ones waiting: 94.6 us instead of 66.5 for 256x56x56x64 -> 128 + 128)
+    const int per = (a.tiles_p + 7) >> 3, x = blockIdx.x & 7;
+    int i = blockIdx.x >> 3;
+    aux = i >= per * a.tiles_f;
+    const int nf = aux ? a.aux_tiles : a.tiles_f;
+    if (aux) i -= per * a.tiles_f;
+    tp = i / nf;
+    tf = i - tp * nf + (aux ? a.tiles_f : 0);
+    tp += x * per;
+    if (tp >= a.tiles_p) return;  // (uniform; before any barrier)
+  } else {  // XCD x takes a contiguous run of tiles: its L2 holds a part of the larger operand only
     const int tiles = a.tiles_f * a.tiles_p, per = (tiles + 7) >> 3, rem = tiles & 7;
     const int x = blockIdx.x & 7, i = blockIdx.x >> 3;
     const int t = rem == 0 ? x * per + i : (x < rem ? x * per : rem * per + (x - rem) * (per - 1)) + i;
     if (a.pixels_first) tf = fast_div(t, a.tiles_p, a.inv_tiles, &tp);
     else tp = fast_div(t, a.tiles_f, a.inv_tiles, &tf);
-    tf = __builtin_amdgcn_readfirstlane(tf);
-    tp = __builtin_amdgcn_readfirstlane(tp);
   }
+  tf = __builtin_amdgcn_readfirstlane(tf);
+  tp = __builtin_amdgcn_readfirstlane(tp);
   const int p0 = tp * BP, f0 = tf * BF;
+  const int fend = MODE == kLines && a.aux_f0 > 0 && !aux ? a.aux_f0 : a.F;
+  const int act = aux ? a.aux_act : a.act;
   const __amdgpu_buffer_rsrc_t rs_in = make_rsrc(a.in, a.in_bytes);
   const __amdgpu_buffer_rsrc_t rs_wt = make_rsrc(a.wt, a.wt_bytes);
 
@@ -113,7 +130,14 @@ __global__ __launch_bounds__(64 * WP * WF) void conv_ring_kernel(const RingArgs 
     for (int v = 0; v < 2; ++v) kc[v] = column(v), settle(v);
   }
   int slab = 0, skr = 0, sks = 0, skc = 0;  // the slab to fetch next, and its tap (kLines)
-  const int nslab = (a.chunks + 7) >> 3;
+  int nslab = (a.chunks + 7) >> 3;
+  if (aux) {
+    slab = a.aux_tap * (a.cpt >> 3);
+    nslab = slab + (a.cpt >> 3);
+    skr = a.aux_tap / a.S;
+    sks = a.aux_tap - skr * a.S;
+  }
+  const int first = slab;
   auto fetch = [&](int buf) {
     unsigned char* dst = smem + buf * kStage;
     const bool tail = 8 * slab + 8 > a.chunks;
@@ -157,16 +181,17 @@ __global__ __launch_bounds__(64 * WP * WF) void conv_ring_kernel(const RingArgs 
 
   // ---- rows of the outgoing tile: 4 * FB lanes to a row; the residual's rows are requested now ----
   constexpr int kLanesRow = 4 * FB, kRowsInstr = 64 / kLanesRow, kOut = PB * 32 / kRowsInstr;
-  const __amdgpu_buffer_rsrc_t rs_out = make_rsrc(a.out, a.out_bytes);
+  const __amdgpu_buffer_rsrc_t rs_out = aux ? make_rsrc(a.aux_out, a.aux_out_bytes) : make_rsrc(a.out, a.out_bytes);
+  const bool residual = a.residual != nullptr && !aux;
   const int orow = lane / kLanesRow, ochan = (lane % kLanesRow) * 8;
   unsigned oofs[kOut];
   u32x4 rv[kOut];
 #pragma unroll
   for (int o = 0; o < kOut; ++o) {
     const int p = p0 + wp * PB * 32 + o * kRowsInstr + orow, f = f0 + wf * FB * 32 + ochan;
-    oofs[o] = p < a.P && f < a.F ? (unsigned)(p * a.ldo + f) * 2u : kOOBr;
+    oofs[o] = p < a.P && f < fend ? (unsigned)(aux ? p * a.aux_ldo + f - a.aux_f0 : p * a.ldo + f) * 2u : kOOBr;
   }
-  if (a.residual) {
+  if (residual) {
     const __amdgpu_buffer_rsrc_t rs_res = make_rsrc(a.residual, a.out_bytes);
 #pragma unroll
     for (int o = 0; o < kOut; ++o) rv[o] = __builtin_amdgcn_raw_buffer_load_b128(rs_res, oofs[o], 0, 0);
@@ -186,8 +211,8 @@ __global__ __launch_bounds__(64 * WP * WF) void conv_ring_kernel(const RingArgs 
   const int lrow = lane & 31, lh = lane >> 5, key = (lrow >> 1) & 7;
   const unsigned char* prow = smem + (wp * PB * 32 + lrow) * 128;
   const unsigned char* wrow = smem + (BP + wf * FB * 32 + lrow) * 128;
-  for (int s = 0; s < nslab; ++s) {
-    const int buf = S == 2 ? s & 1 : 0;
+  for (int s = first; s < nslab; ++s) {
+    const int buf = S == 2 ? (s - first) & 1 : 0;
     __builtin_amdgcn_s_waitcnt(kAllLanded);
     __syncthreads();
     if (S == 2 && s + 1 < nslab) fetch(buf ^ 1);
@@ -213,7 +238,7 @@ __global__ __launch_bounds__(64 * WP * WF) void conv_ring_kernel(const RingArgs 
 
   // ---- out: this wave's tile [PB * 32 pixels][FB * 32 channels] ----
   unsigned char* tile = smem + wave * (PB * 32 * kPitch);
-  if (a.residual) {
+  if (residual) {
 #pragma unroll
     for (int o = 0; o < kOut; ++o) *reinterpret_cast<u32x4*>(tile + (o * kRowsInstr + orow) * kPitch + ochan * 2) = rv[o];
   }
@@ -230,20 +255,20 @@ __global__ __launch_bounds__(64 * WP * WF) void conv_ring_kernel(const RingArgs 
         for (int e = 0; e < 4; ++e) y[4 * q + e] = acc[i][j][4 * q + e] * m[e] + h[e];
       }
       unsigned char* at = tile + (j * 32 + lrow) * kPitch + i * 64 + lh * 8;
-      if (a.residual) {
+      if (residual) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const half4 x = *reinterpret_cast<const half4*>(at + q * 16);
 #pragma unroll
           for (int e = 0; e < 4; ++e) r[4 * q + e] = (float)x[e];
         }
-        if (!(a.act & kActResidualAfter)) {
+        if (!(act & kActResidualAfter)) {
 #pragma unroll
           for (int e = 0; e < 16; ++e) y[e] += r[e];
         }
       }
-      act_apply_n<true>(y, a.act & 0xff);
-      if (a.residual && (a.act & kActResidualAfter)) {
+      act_apply_n<true>(y, act & 0xff);
+      if (residual && (act & kActResidualAfter)) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) y[e] += r[e];
       }
@@ -268,7 +293,9 @@ template <int WP, int WF, int PB, int FB, int S>
 void launch_cfg(RingArgs d, int mode, hipStream_t s) {
   constexpr int NW = WP * WF, BP = 32 * WP * PB, BF = 32 * WF * FB, ring = S * (BP + BF) * 128, tile = NW * PB * 32 * (FB * 64 + 16);
   constexpr int lds = (ring > tile ? ring : tile) + BF * 8;
-  d.tiles_f = (d.F + BF - 1) / BF;
+  const int main_f = d.aux_f0 ? d.aux_f0 : d.F;
+  d.tiles_f = (main_f + BF - 1) / BF;
+  d.aux_tiles = (d.F - main_f + BF - 1) / BF;
   d.tiles_p = (d.P + BP - 1) / BP;
   d.inv_tiles = 1.0f / (float)(d.pixels_first ? d.tiles_p : d.tiles_f);
   auto go = [&](auto kern) {
@@ -277,7 +304,7 @@ void launch_cfg(RingArgs d, int mode, hipStream_t s) {
       return true;
     }();
     (void)attr;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(d.tiles_f * d.tiles_p)), dim3(64 * NW), lds, s, d);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(d.aux_f0 ? (d.tiles_p + 7) / 8 * 8 * (d.tiles_f + d.aux_tiles) : d.tiles_f * d.tiles_p)), dim3(64 * NW), lds, s, d);
   };
   if (mode == kPoint) go(conv_ring_kernel<WP, WF, PB, FB, S, kPoint>);
   else if (mode == kLines) go(conv_ring_kernel<WP, WF, PB, FB, S, kLines>);
@@ -301,6 +328,7 @@ const Form kForms[] = {
     {64, 32, 13, 2.71, 0.144, 0.180, 0.423, 0.24, 0.26, launch_cfg<2, 1, 1, 1, 1>, "conv_ring<64x32>"},
     {64, 128, 3, 3.04, 0.353, 0.620, 0.434, 0.11, 0.37, launch_cfg<2, 2, 1, 2, 2>, "conv_ring<64x128,2>"},
     {128, 128, 2, 2.94, 0.626, 1.086, 0.631, 0.11, 0.11, launch_cfg<4, 2, 1, 2, 1>, "conv_ring<128x128>"},
+    {128, 128, 2, 3.08, 0.583, 1.142, 0.515, 0.21, 0.48, launch_cfg<4, 2, 1, 2, 2>, "conv_ring<128x128,2>"},
 };
 
 const Form* best_form(const IgemmArgs& a, double* us) {
@@ -308,7 +336,8 @@ const Form* best_form(const IgemmArgs& a, double* us) {
   const bool any = a.R * a.S > 1 && a.C % 64 != 0;
   const Form* best = nullptr;
   for (const Form& f : kForms) {
-    const double x = std::ceil(P / f.bp) * std::ceil((double)a.F / f.bf) / 256;
+    const double fs = a.aux_f0 ? a.aux_f0 + (double)(a.F - a.aux_f0) / (a.R * a.S) : a.F;  // auxiliary filters walk one tap
+    const double x = std::ceil(P / f.bp) * std::ceil(fs / f.bf) / 256;
     const double busy = x * (f.slab_us * slabs * (any ? 1 + f.slab_any : 1) + f.tile_us);
     const double chain = std::ceil(x / f.resident) * f.chain_us * slabs * (any ? 1 + f.chain_any : 1);
     const double v = f.fixed_us + std::cbrt(busy * busy * busy + chain * chain * chain);
@@ -324,10 +353,20 @@ const Form* best_form(const IgemmArgs& a, double* us) {
 bool conv_ring_applicable(const IgemmArgs& a, int in_dt, int out_dt) {
   const int pix = a.pix_stride ? a.pix_stride : a.C;
   const long long P = (long long)a.N * a.OH * a.OW, k = (long long)a.R * a.S * a.C, lim = 1 << 24;  // fast_div's range
-  return in_dt == kF16 && out_dt == kF16 && a.batch == 1 && a.aux_f0 == 0 && a.C % 8 == 0 && (a.R * a.S == 1 || a.C >= 16) && pix % 8 == 0 &&
+  const bool aux_ok = a.aux_f0 == 0 || (a.aux_f0 % 128 == 0 && a.C % 64 == 0 && a.R * a.S > 1 && a.aux_tap >= 0 && a.aux_tap < a.R * a.S && a.aux_out &&
+                                        a.aux_ldo % 8 == 0 && P * a.aux_ldo * 2 < (long long)kOOBr);
+  return in_dt == kF16 && out_dt == kF16 && a.batch == 1 && aux_ok && a.C % 8 == 0 && (a.R * a.S == 1 || a.C >= 16) && pix % 8 == 0 &&
          a.F % 8 == 0 && a.ldo % 8 == 0 && P < lim && k < lim && a.in_bytes > 0 && a.in_bytes < kOOBr &&
          (long long)a.N * a.H * a.W * pix * 2 < (long long)kOOBr && (long long)a.F * k * 2 < (long long)kOOBr &&
          P * a.ldo * 2 < (long long)kOOBr && ((P + 63) / 64) * ((a.F + 31) / 32) < lim && (a.relu & ~(0xff | kActResidualAfter)) == 0;
+}
+
+// Stride-2 3x3 layers leave the patch kernel where 128 x 128 tiles keep three quarters of the CUs busy: it is bound by its
+// patch reads (64x56x56x64 -> 128: 18.4 -> 14.7 us, 256x28x28x128 -> 256 with its shortcut 59.9 -> 47.7), while below that its
+// smaller tiles and K groups fill the chip better (32x28x28x128 -> 256: 9.1 against 10.6).
+bool conv_ring_beats_patch_s2(const IgemmArgs& a) {
+  const long long P = (long long)a.N * a.OH * a.OW, main_f = a.aux_f0 ? a.aux_f0 : a.F;
+  return a.stride_h == 2 && (P + 127) / 128 * ((main_f + 127) / 128) >= 200;
 }
 
 double conv_ring_us(const IgemmArgs& a) {
@@ -345,6 +384,10 @@ void launch_conv_ring(const IgemmArgs& a, hipStream_t s) {
   d.in_bytes = a.in_bytes; d.wt_bytes = (unsigned)d.F * d.chunks * 16u; d.out_bytes = (unsigned)d.P * a.ldo * 2u;
   d.stride_h = a.stride_h; d.stride_w = a.stride_w; d.pad_h = a.pad_h; d.pad_w = a.pad_w;
   d.act = a.relu; d.ldo = a.ldo;
+  if (a.aux_f0) {
+    d.aux_f0 = a.aux_f0; d.aux_tap = a.aux_tap; d.aux_act = a.aux_relu; d.aux_ldo = a.aux_ldo; d.aux_out = a.aux_out;
+    d.aux_out_bytes = (unsigned)d.P * a.aux_ldo * 2u;
+  }
   d.inv_ohw = 1.0f / (float)d.OHW; d.inv_ow = 1.0f / (float)d.OW;
   d.pixels_first = d.wt_bytes > d.in_bytes;
   double us = 0;

@@ -280,6 +280,7 @@ bool igemm_takes_direct(const IgemmArgs& a_in, int in_dt, int out_dt) {
   if (!conv_direct_applicable(a, in_dt, out_dt)) return false;
   DirectRival rival = kRivalIgemm;
   if (conv_pairs_applicable(a, in_dt, out_dt)) rival = kRivalShortK;
+  else if (conv_ring_applicable(a, in_dt, out_dt) && conv_ring_beats_patch_s2(a)) rival = kRivalRing;
   else if (conv3x3_stream_applicable(a, in_dt, out_dt) || conv3x3_patch_applicable(a, in_dt)) rival = a.stride_h == 1 ? kRivalPatch : kRivalPatchS2;
   else if (conv_ring_applicable(a, in_dt, out_dt)) rival = kRivalRing;
   else if (igemm_fast_applicable(a, in_dt, out_dt)) rival = kRivalIgemmFast;
@@ -307,11 +308,12 @@ void launch_igemm(const IgemmArgs& a_in, int in_dt, int out_dt, hipStream_t s) {
     return;
   }
   if (conv3x3_stream_applicable(a, in_dt, out_dt) && launch_conv3x3_stream(a, s)) return;
-  if (in_dt == out_dt && conv3x3_patch_applicable(a, in_dt)) {
+  const bool ring = conv_ring_applicable(a, in_dt, out_dt);
+  if (in_dt == out_dt && conv3x3_patch_applicable(a, in_dt) && !(ring && conv_ring_beats_patch_s2(a))) {
     launch_conv3x3_patch(a, in_dt, out_dt, s);
     return;
   }
-  if (conv_ring_applicable(a, in_dt, out_dt)) {
+  if (ring) {
     launch_conv_ring(a, s);
     return;
   }

@@ -24,6 +24,7 @@ def rand(seed, *shape):
     (9, 24, 72, 61, 62, 3, 2, 1, None),       # taps that straddle slabs
     (8, 40, 72, 64, 64, 5, 1, 4, "relu"),     # the large form, padding wider than the centre
     (16, 512, 256, 20, 20, 1, 1, 0, "relu"),  # two buffers
+    (33, 64, 136, 57, 55, 3, 2, 1, None),     # 3x3 stride 2: the large form with two buffers
     (8, 512, 128, 60, 60, 1, 1, 0, "relu"),   # the wide form
 ])
 def test_ring_kernel_matches_torch(N, C, F, H, W, R, stride, pad, act):
@@ -44,3 +45,28 @@ def test_ring_kernel_matches_torch(N, C, F, H, W, R, stride, pad, act):
     print(tags, flush=True)
     assert rel_l2(nchw(plain), f(y).numpy()) < 2e-3 < FP16_REL_L2
     assert rel_l2(nchw(added), f(y + r).numpy()) < 2e-3
+
+
+def test_shortcut_filters_ride_along():
+    """A ResNet-18 pass whose stride-2 layers are large enough to come here: their 1x1 shortcuts are further tiles of the same
+    launch.  Stage outputs of three images, spread over the batch, against the oracle's."""
+    import numpy as np
+    import oracle
+    from nncv_amd import synth
+    from gpu_util import Model
+    n, pick = 37, [0, 17, 36]
+    blob = synth.round_fp16(synth.resnet18_params())
+    x = synth.round_fp16(synth.uniform(4005, (n, 3, 219, 227), 0.0, 1.0))
+    m = Model(blob, abi.F16, abi.ALGO_IGEMM)
+    abi.profile_enable(True)
+    try:
+        abi.profile_report()
+        got = host(m(dev(x, abi.F16)))
+        tags = {k: v["launches"] for k, v in abi.profile_report().items()}
+    finally:
+        abi.profile_enable(False)
+    print(tags, flush=True)
+    assert sum(v for k, v in tags.items() if k.startswith("conv_ring<")) >= 1, tags
+    want = oracle.resnet18_forward(np.ascontiguousarray(x[pick]), blob)
+    assert rel_l2(got[pick], want) < FP16_REL_L2
+    assert (got[pick].argmax(1) == want.argmax(1)).all()
