@@ -265,6 +265,37 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
     nodes_[i + 1].skip = true;
   }
 
+  // inverted-residual blocks
+  if (dt == kF16) {
+    std::vector<int> uses(n_tensors_, 0);
+    for (int i = 0; i < n; ++i)
+      for (int k = 0; k < 4; ++k)
+        if (ops[i].in[k] >= 0) ++uses[ops[i].in[k]];
+    for (int i = 0; i < n; ++i) {
+      const GraphOp& d = ops[i];
+      if (d.kind == NNCV_HIP_OP_DWCONV && i > 0) {
+        const GraphOp& e = ops[i - 1];
+        if (e.kind == NNCV_HIP_OP_CONV && e.out == d.in[0] && e.K == 1 && e.stride == 1 && e.pad == 0 && e.in[1] < 0 && e.in[0] != 0 && uses[e.out] == 1 &&
+            nodes_[i - 1].add_out < 0 && logical_[e.out] == channels_[e.out])
+          nodes_[i].expands = i - 1;
+      }
+      // (the pooled tensor must be the depthwise convolution right before it, read by the pool and the gate alone)
+      if (nodes_[i].se_head && i > 0 && i + 4 < n && ops[i - 1].kind == NNCV_HIP_OP_DWCONV && ops[i - 1].out == d.in[0] && uses[d.in[0]] == 2) {
+        const GraphOp &g = ops[i + 3], &pr = ops[i + 4];
+        if (pr.kind == NNCV_HIP_OP_CONV && pr.in[0] == g.out && pr.in[1] != g.out && uses[g.out] == 1 && pr.K == 1 && pr.stride == 1 && pr.pad == 0 &&
+            nodes_[i + 4].add_out < 0 && logical_[pr.out] == channels_[pr.out] && se_project_applicable(1, g.in[0] >= 0 ? channels_[g.in[0]] : 0, ops[i + 1].F, pr.F))
+        {
+          nodes_[i].projects = i + 4;
+          for (int k = 1; k <= 2 && !dry_; ++k) {
+            Node& f = nodes_[i + k];
+            f.wt_t.reset(f.wt.bytes(), &pool_);
+            launch_transpose_half(f.wt.get(), f.wt_t.get(), f.op.F, f.C, s);
+          }
+        }
+      }
+    }
+  }
+
   // concatenation views
   view_of_.assign(n_tensors_, -1);
   view_c0_.assign(n_tensors_, 0);
@@ -283,7 +314,8 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
       if (nodes_[i].skip)  // merged into its predecessor: the residual of a conv + ADD pair shares the result's pitch
         return i > 0 && nodes_[i - 1].add_out >= 0 && nodes_[i - 1].add_res != t;
       switch (o.kind) {
-        case NNCV_HIP_OP_CONV: return o.in[1] != t;  // not as the residual
+        case NNCV_HIP_OP_CONV:  // not as the residual, nor as the input of a projection
+          return o.in[1] != t && !(i >= 4 && nodes_[i - 4].projects == i);
         case NNCV_HIP_OP_MAXPOOL:
         case NNCV_HIP_OP_UPSAMPLE2X:
         case NNCV_HIP_OP_ADD:
@@ -297,7 +329,8 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
       const GraphOp& o = ops[i];
       if (nodes_[i].se_head || nodes_[i].skip) return false;
       switch (o.kind) {
-        case NNCV_HIP_OP_CONV: return o.in[1] < 0 && nodes_[i].add_res < 0;  // residual and result share one pitch
+        case NNCV_HIP_OP_CONV:  // residual and result share one pitch; so do the results of the merged blocks
+          return o.in[1] < 0 && nodes_[i].add_res < 0 && !(i >= 4 && nodes_[i - 4].projects == i) && !(i + 1 < n && nodes_[i + 1].expands == i);
         case NNCV_HIP_OP_MAXPOOL:
         case NNCV_HIP_OP_UPSAMPLE2X:
         case NNCV_HIP_OP_ADD:
@@ -386,6 +419,21 @@ const Graph::Plan& Graph::plan_of(int N, int H, int W) const {
     NNCV_REQUIRE((long long)N * o.H * o.W * o.C < (1ll << 31), where + "tensor too large");
     p.dims[op.out] = o;
   }
+  p.dw.assign(n, 0);
+  p.se.assign(n, 0);
+  if (dt_ == kF16)
+    for (int i = 0; i < n; ++i) {
+      const GraphOp& op = nodes_[i].op;
+      if (op.kind != NNCV_HIP_OP_DWCONV) continue;
+      const bool expands = nodes_[i].expands >= 0, projects = i + 1 < n && nodes_[i + 1].projects >= 0;
+      if (!expands && !projects) continue;
+      const Dims a = p.dims[op.in[0]], o = p.dims[op.out];
+      const int Cin = expands ? p.dims[nodes_[i - 1].op.in[0]].C : 0;
+      p.dw[i] = dw_block_bands(N, a.H, a.W, Cin, a.C, op.K, op.stride, op.pad);
+      if (p.dw[i] && projects)
+        p.se[i + 1] = se_project_applicable(o.H * o.W, a.C, nodes_[i + 2].op.F, nodes_[i + 5].op.F);
+      if (!expands && !p.se[i + 1]) p.dw[i] = 0;
+    }
   // Lifetimes in operator steps: step 0 lays the input out as NHWC, step i + 1 is operator i,
   // step n + 1 converts the output.  A tensor is live from the step that writes it to the last
   // step that reads it, so an operator's output never shares memory with any of its inputs.
@@ -406,6 +454,15 @@ const Graph::Plan& Graph::plan_of(int N, int H, int W) const {
   // time and may lay one over the other.
   for (int i = 0; i < n; ++i) {
     if (nodes_[i].se_head && i + 3 < n) life[nodes_[i + 3].op.out].first_op = i + 1;
+    if (p.dw[i] && nodes_[i].expands >= 0) {  // one launch, at the expansion's step; the expanded tensor is never stored
+      life[nodes_[i].op.out].first_op = i;
+      life[nodes_[i - 1].op.out] = TensorLife{i, i, 0, 0};
+    }
+    if (p.se[i]) {  // the channel sums, from the depthwise launch on; the gated tensor is never stored
+      life[nodes_[i].op.out] = TensorLife{nodes_[i - 1].expands >= 0 ? i - 1 : i, i + 1, (size_t)N * p.dw[i - 1] * p.dims[nodes_[i].op.in[0]].C * 4, 0};
+      life[nodes_[i + 3].op.out] = TensorLife{i + 1, i + 1, 0, 0};
+      life[nodes_[i + 4].op.out].first_op = i + 1;
+    }
     if (nodes_[i].add_out >= 0) life[nodes_[i].add_out].first_op = std::min(life[nodes_[i].add_out].first_op, i + 1);
   }
   {
@@ -452,13 +509,35 @@ const Graph::Plan& Graph::plan_of(int N, int H, int W) const {
 }
 
 // The tensors one launch of forward() touches: what it writes and what it reads.
-void Graph::launch_io(int i, std::vector<int>* writes, std::vector<int>* reads) const {
+void Graph::launch_io(const Plan& p, int i, std::vector<int>* writes, std::vector<int>* reads) const {
   writes->clear();
   reads->clear();
   const int n = (int)nodes_.size();
   const Node& nd = nodes_[i];
   const GraphOp& op = nd.op;
   if (nd.skip) return;
+  if (op.kind == NNCV_HIP_OP_CONV && i + 1 < n && nodes_[i + 1].expands == i && p.dw[i + 1]) {
+    reads->push_back(op.in[0]);
+    writes->push_back(nodes_[i + 1].op.out);
+    if (i + 2 < n && p.se[i + 2]) writes->push_back(nodes_[i + 2].op.out);
+    return;
+  }
+  if (op.kind == NNCV_HIP_OP_DWCONV && p.dw[i]) {
+    if (nd.expands >= 0) return;
+    reads->push_back(op.in[0]);
+    writes->push_back(op.out);
+    writes->push_back(nodes_[i + 1].op.out);
+    return;
+  }
+  if (p.se[i]) {
+    const GraphOp& pr = nodes_[i + 4].op;
+    reads->push_back(op.in[0]);
+    reads->push_back(op.out);
+    if (pr.in[1] >= 0) reads->push_back(pr.in[1]);
+    writes->push_back(pr.out);
+    return;
+  }
+  if (op.kind == NNCV_HIP_OP_CONV && i >= 4 && p.se[i - 4]) return;
   if (nd.se_head) {
     reads->push_back(op.in[0]);
     writes->push_back(nodes_[i + 3].op.out);
@@ -495,7 +574,7 @@ void Graph::check_plan(const Plan& p) const {
   };
   std::vector<int> w, r;
   for (int i = 0; i < (int)nodes_.size(); ++i) {
-    launch_io(i, &w, &r);
+    launch_io(p, i, &w, &r);
     for (size_t x = 0; x < w.size(); ++x) {
       for (int t : r)
         NNCV_REQUIRE(!clash(w[x], t), "graph: workspace plan lays the result of operator " + std::to_string(i) + " (tensor " +
@@ -518,7 +597,7 @@ size_t Graph::describe_plan(int N, int H, int W, long long* tensor_info, int* la
   }
   std::vector<int> w, r;
   for (int i = 0; i < (int)nodes_.size(); ++i) {
-    launch_io(i, &w, &r);
+    launch_io(p, i, &w, &r);
     launch_dst[i] = w.empty() ? -1 : w[0];
   }
   return p.total;
@@ -558,6 +637,33 @@ void Graph::forward(const void* src, int N, int H, int W, float* out, void* ws, 
     const GraphOp& op = nd.op;
     const Dims a = p.dims[op.in[0]], o = p.dims[op.out];
     if (nd.skip) continue;
+    if (op.kind == NNCV_HIP_OP_CONV && i + 1 < nodes_.size() && nodes_[i + 1].expands == (int)i && p.dw[i + 1]) continue;  // rides below
+    if (op.kind == NNCV_HIP_OP_DWCONV && p.dw[i]) {
+      DwBlockArgs d{};
+      const Node* e = nd.expands >= 0 ? &nodes_[i - 1] : nullptr;
+      const int src = e ? e->op.in[0] : op.in[0];
+      d.in = at(src); d.pix = pitch(src); d.wt = nd.wt.get(); d.scale = nd.scale.as<float>(); d.shift = nd.shift.as<float>(); d.out = at(op.out);
+      if (e) {
+        d.w1 = e->wt.get(); d.scale1 = e->scale.as<float>(); d.shift1 = e->shift.as<float>();
+        d.Cin = p.dims[src].C; d.act1 = e->op.act;
+      }
+      d.sums = i + 1 < nodes_.size() && p.se[i + 1] ? static_cast<float*>(at(nodes_[i + 1].op.out)) : nullptr;
+      d.N = N; d.H = a.H; d.W = a.W; d.C = a.C; d.K = op.K; d.stride = op.stride; d.pad = op.pad; d.OH = o.H; d.OW = o.W; d.act = op.act;
+      launch_dw_block(d, s);
+      continue;
+    }
+    if (p.se[i]) {
+      const Node &f1 = nodes_[i + 1], &f2 = nodes_[i + 2], &pr = nodes_[i + 4];
+      SeProjectArgs e{};
+      e.x = at(op.in[0]); e.sums = static_cast<const float*>(at(op.out)); e.bands = p.dw[i - 1];
+      e.w1t = f1.wt_t.get(); e.b1 = f1.shift.as<float>(); e.w2t = f2.wt_t.get(); e.b2 = f2.shift.as<float>(); e.act1 = f1.op.act; e.act2 = f2.op.act;
+      e.wp_flat = pr.wflat.get(); e.scale = pr.scale.as<float>(); e.shift = pr.shift.as<float>(); e.out = at(pr.op.out);
+      e.residual = pr.op.in[1] >= 0 ? at(pr.op.in[1]) : nullptr;
+      e.N = N; e.HW = a.H * a.W; e.C = a.C; e.SQ = f1.op.F; e.F = pr.op.F; e.act = pr.op.act;
+      launch_se_project(e, s);
+      i += 4;
+      continue;
+    }
     if (nd.se_head) {
       const Node &f1 = nodes_[i + 1], &f2 = nodes_[i + 2];
       SeArgs e{};

@@ -53,6 +53,12 @@ class Graph {
     // output tensor `add_out`; the ADD node is skipped.
     int add_res = -1, add_out = -1;
     DeviceBuffer wt_pairs;  // see pair_stem_
+    // fp16 inverted-residual blocks (mobile_block.hip), where the image size allows it (Plan::dw, Plan::se): on a DWCONV,
+    // the 1x1 CONV before it that nothing else reads rides in its launch (expands = that node's index) and, when a
+    // squeeze-excitation block follows, the launch leaves the channel sums in the memory of the pooling operator's tensor;
+    // on that GAVGPOOL, projects = the 1x1 CONV that is the only reader of the gated tensor.
+    int expands = -1, projects = -1;
+    DeviceBuffer wt_t;  // the two vectors' weights of such a block, [in][out]
   };
   struct Dims { int C, H, W; };
   struct Plan {
@@ -60,10 +66,12 @@ class Graph {
     std::vector<Dims> dims;      // per tensor
     std::vector<size_t> offset;  // per tensor, in the workspace (tensor 0: its NHWC copy)
     std::vector<size_t> root_bytes;  // per tensor: size of the memory block it lives in
+    std::vector<int> dw;             // per operator: bands of a DWCONV that runs as a dw_block, 0: as its own operators
+    std::vector<char> se;            // per operator: this GAVGPOOL starts a se_project launch
     size_t total;
   };
   const Plan& plan_of(int N, int H, int W) const;
-  void launch_io(int i, std::vector<int>* writes, std::vector<int>* reads) const;
+  void launch_io(const Plan& p, int i, std::vector<int>* writes, std::vector<int>* reads) const;
   void check_plan(const Plan& p) const;
 
   int dt_, c_in_, n_tensors_ = 0;
