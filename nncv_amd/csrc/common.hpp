@@ -183,6 +183,10 @@ struct IgemmArgs {
   // What conv_direct.hip reads instead of wt and wt_frag: the filters (launch_weight_flat), and the auxiliary filters alone
   // (the same with one tap); or null.  Behind the fields that the other kernels load.
   const void *wt_flat, *aux_wt_flat;
+  // Two results (conv_ring.hip only): filters from split_f on go to another tensor of row pitch split_ldo, split_ofs bytes from
+  // `out`.  split_f = 0: none; otherwise a multiple of 8, and no residual.
+  int split_f, split_ldo;
+  long long split_ofs;
 };
 // in_dt: element type of in/wt (kF32 | kF16); out_dt: element type of out/residual.
 // Dispatches to the fast kernel (igemm_fast.hip) when C is a multiple of one K step and the

@@ -40,6 +40,7 @@ struct RingArgs {
   int tiles_f, tiles_p, pixels_first;
   int aux_tiles, aux_f0, aux_tap, aux_act, aux_ldo;              // filters from aux_f0 on walk one tap only and go to aux_out; 0: none
   void* aux_out; unsigned aux_out_bytes;
+  int split_f, split_ldo; unsigned ofs, split_ofs;    // filters from split_f on (F: none) go to rows of their own; bytes from `out`
   float inv_ohw, inv_ow, inv_tiles;
 };
 
@@ -190,6 +191,7 @@ __global__ __launch_bounds__(64 * WP * WF) void conv_ring_kernel(const RingArgs 
   for (int o = 0; o < kOut; ++o) {
     const int p = p0 + wp * PB * 32 + o * kRowsInstr + orow, f = f0 + wf * FB * 32 + ochan;
     oofs[o] = p < a.P && f < fend ? (unsigned)(aux ? p * a.aux_ldo + f - a.aux_f0 : p * a.ldo + f) * 2u : kOOBr;
+    if (MODE == kPoint && p < a.P && f < fend) oofs[o] = f < a.split_f ? oofs[o] + a.ofs : (unsigned)(p * a.split_ldo + f - a.split_f) * 2u + a.split_ofs;
   }
   if (residual) {
     const __amdgpu_buffer_rsrc_t rs_res = make_rsrc(a.residual, a.out_bytes);
@@ -355,7 +357,11 @@ bool conv_ring_applicable(const IgemmArgs& a, int in_dt, int out_dt) {
   const long long P = (long long)a.N * a.OH * a.OW, k = (long long)a.R * a.S * a.C, lim = 1 << 24;  // fast_div's range
   const bool aux_ok = a.aux_f0 == 0 || (a.aux_f0 % 128 == 0 && a.C % 64 == 0 && a.R * a.S > 1 && a.aux_tap >= 0 && a.aux_tap < a.R * a.S && a.aux_out &&
                                         a.aux_ldo % 8 == 0 && P * a.aux_ldo * 2 < (long long)kOOBr);
-  return in_dt == kF16 && out_dt == kF16 && a.batch == 1 && aux_ok && a.C % 8 == 0 && (a.R * a.S == 1 || a.C >= 16) && pix % 8 == 0 &&
+  // (two results: one range of bytes that holds both)
+  const long long reach = (a.split_ofs < 0 ? -a.split_ofs : a.split_ofs) + P * (a.ldo > a.split_ldo ? a.ldo : a.split_ldo) * 2;
+  const bool split_ok = a.split_f == 0 || (a.split_f % 8 == 0 && a.split_ldo % 8 == 0 && a.split_ofs % 16 == 0 && reach < (long long)kOOBr && !a.residual &&
+                                           a.aux_f0 == 0 && a.R * a.S == 1 && a.pad_h == 0 && a.pad_w == 0);
+  return in_dt == kF16 && out_dt == kF16 && a.batch == 1 && aux_ok && split_ok && a.C % 8 == 0 && (a.R * a.S == 1 || a.C >= 16) && pix % 8 == 0 &&
          a.F % 8 == 0 && a.ldo % 8 == 0 && P < lim && k < lim && a.in_bytes > 0 && a.in_bytes < kOOBr &&
          (long long)a.N * a.H * a.W * pix * 2 < (long long)kOOBr && (long long)a.F * k * 2 < (long long)kOOBr &&
          P * a.ldo * 2 < (long long)kOOBr && ((P + 63) / 64) * ((a.F + 31) / 32) < lim && (a.relu & ~(0xff | kActResidualAfter)) == 0;
@@ -384,6 +390,14 @@ void launch_conv_ring(const IgemmArgs& a, hipStream_t s) {
   d.in_bytes = a.in_bytes; d.wt_bytes = (unsigned)d.F * d.chunks * 16u; d.out_bytes = (unsigned)d.P * a.ldo * 2u;
   d.stride_h = a.stride_h; d.stride_w = a.stride_w; d.pad_h = a.pad_h; d.pad_w = a.pad_w;
   d.act = a.relu; d.ldo = a.ldo;
+  d.split_f = a.F;
+  if (a.split_f) {
+    const long long low = a.split_ofs < 0 ? a.split_ofs : 0;
+    d.split_f = a.split_f; d.split_ldo = a.split_ldo; d.ofs = (unsigned)-low; d.split_ofs = (unsigned)(a.split_ofs - low);
+    d.out = static_cast<char*>(a.out) + low;
+    const unsigned e0 = d.ofs + (unsigned)d.P * a.ldo * 2u, e1 = d.split_ofs + (unsigned)d.P * a.split_ldo * 2u;
+    d.out_bytes = e0 > e1 ? e0 : e1;
+  }
   if (a.aux_f0) {
     d.aux_f0 = a.aux_f0; d.aux_tap = a.aux_tap; d.aux_act = a.aux_relu; d.aux_ldo = a.aux_ldo; d.aux_out = a.aux_out;
     d.aux_out_bytes = (unsigned)d.P * a.aux_ldo * 2u;

@@ -69,6 +69,32 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
   logical_[0] = in_channels;
   nodes_.resize(n);
 
+  // Two 1x1 convolutions of one tensor, equal but for their filters (cv1 and cv2 of a YOLOv5 C3 block): the second one's
+  // parameters lie behind the first one's, so that one launch can compute both where the shape is the LDS ring's (plan_of).
+  for (int i = 0; i < n && dt == kF16; ++i) {
+    auto point = [&](const GraphOp& o) {
+      return o.kind == NNCV_HIP_OP_CONV && o.K == 1 && o.stride == 1 && o.pad == 0 && o.in[0] > 0 && o.in[1] < 0 && o.F > 0 && o.F % vn == 0;
+    };
+    if (!point(ops[i]) || nodes_[i].joined) continue;
+    for (int j = i + 1; j < n; ++j)
+      if (point(ops[j]) && ops[j].in[0] == ops[i].in[0] && ops[j].F == ops[i].F && ops[j].act == ops[i].act &&
+          (ops[j].gamma < 0) == (ops[i].gamma < 0) && (ops[j].bias < 0) == (ops[i].bias < 0) && !nodes_[j].joined) {
+        nodes_[i].joins = j;
+        nodes_[j].joined = true;
+        break;
+      }
+  }
+  auto joined_by = [&](int i) -> Node* {
+    for (int k = 0; nodes_[i].joined && k < i; ++k)
+      if (nodes_[k].joins == i) return &nodes_[k];
+    return nullptr;
+  };
+  // a buffer of node i, with room behind it for the node it joins, or the second half of its joiner's
+  auto take = [&](int i, DeviceBuffer Node::*b, size_t bytes) {
+    if (const Node* first = joined_by(i)) (nodes_[i].*b).borrow((first->*b).as<char>() + bytes, bytes);
+    else (nodes_[i].*b).reset(bytes * (nodes_[i].joins >= 0 ? 2 : 1), &pool_);
+  };
+
   auto param = [&](long long off, long long count, const std::string& what) -> const void* {
     NNCV_REQUIRE(off >= 0 && (dry_ || off + count <= n_elems), "graph: " + what + " lies outside the parameter blob");
     return blob + (size_t)off * es;
@@ -117,8 +143,8 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
         const int Cl = logical_[op.in[0]];  // channels the filters really have
         const void* w = param(op.w, (long long)op.F * Cl * op.K * op.K, where + "w");
         if (dry_) break;
-        nd.wt.reset((size_t)Cstored * op.K * op.K * C * es, &pool_);
-        if (Cstored > op.F) NNCV_HIP_CHECK(hipMemsetAsync(nd.wt.get(), 0, nd.wt.bytes(), s));
+        take(i, &Node::wt, (size_t)Cstored * op.K * op.K * C * es);
+        if (Cstored > op.F) NNCV_HIP_CHECK(hipMemsetAsync(nd.wt.get(), 0, (size_t)Cstored * op.K * op.K * C * es, s));
         launch_weight_frsc(w, dt, nd.wt.get(), dt, op.F, Cl, op.K, op.K, C, s);
         nd.wflat.reset(weight_flat_bytes(dt, Cstored, op.K * op.K, C), &pool_);
         launch_weight_flat(w, nd.wflat.get(), dt, op.F, Cl, op.K * op.K, C, s);
@@ -186,8 +212,8 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
       const int F = Cout, Fs = Cstored > 0 ? Cstored : Cout;
       if (op.gamma >= 0) {
         NNCV_REQUIRE(op.beta >= 0 && op.mean >= 0 && op.var >= 0, where + "BatchNorm needs gamma, beta, mean and var");
-        nd.scale.reset((size_t)Fs * 4, &pool_);
-        nd.shift.reset((size_t)Fs * 4, &pool_);
+        take(i, &Node::scale, (size_t)Fs * 4);
+        take(i, &Node::shift, (size_t)Fs * 4);
         launch_fill_f32(nd.scale.as<float>(), 0.0f, Fs, s);
         launch_fill_f32(nd.shift.as<float>(), 0.0f, Fs, s);
         launch_bn_fold(param(op.gamma, F, where + "gamma"), param(op.beta, F, where + "beta"), param(op.mean, F, where + "mean"),
@@ -197,7 +223,7 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
         const void* b = param(op.bias, F, where + "bias");
         const bool had = nd.shift.get() != nullptr;
         if (!had) {
-          nd.shift.reset((size_t)Fs * 4, &pool_);
+          take(i, &Node::shift, (size_t)Fs * 4);
           launch_fill_f32(nd.shift.as<float>(), 0.0f, Fs, s);
         }
         const unsigned grid = (unsigned)((F + 255) / 256);
@@ -288,7 +314,7 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
           nodes_[i].projects = i + 4;
           for (int k = 1; k <= 2 && !dry_; ++k) {
             Node& f = nodes_[i + k];
-            f.wt_t.reset(f.wt.bytes(), &pool_);
+            f.wt_t.reset((size_t)f.op.F * f.C * es, &pool_);
             launch_transpose_half(f.wt.get(), f.wt_t.get(), f.op.F, f.C, s);
           }
         }
@@ -296,14 +322,22 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
     }
   }
 
+  for (int i = 0; i < n; ++i) {  // what rides in another launch, or carries one, does not join
+    auto single = [&](int k) {
+      return !nodes_[k].skip && nodes_[k].add_out < 0 && !(k >= 4 && nodes_[k - 4].projects == k) && !(k + 1 < n && nodes_[k + 1].expands == k);
+    };
+    if (nodes_[i].joins >= 0 && !(single(i) && single(nodes_[i].joins))) nodes_[nodes_[i].joins].joined = false, nodes_[i].joins = -1;
+  }
+
   // concatenation views
+  row_ = channels_;
   view_of_.assign(n_tensors_, -1);
   view_c0_.assign(n_tensors_, 0);
   static const bool no_views = getenv("NNCV_HIP_NO_CONCAT_VIEWS") != nullptr;
   if (!no_views) {
     std::vector<int> producer(n_tensors_, -1), cat_uses(n_tensors_, 0);
     for (int i = 0; i < n; ++i) {
-      producer[nodes_[i].add_out >= 0 ? nodes_[i].add_out : ops[i].out] = i;
+      if (i == 0 || nodes_[i - 1].add_out != ops[i].out) producer[nodes_[i].add_out >= 0 ? nodes_[i].add_out : ops[i].out] = i;
       if (ops[i].kind == NNCV_HIP_OP_CONCAT)
         for (int k = 0; k < 4; ++k)
           if (ops[i].in[k] >= 0) ++cat_uses[ops[i].in[k]];
@@ -339,16 +373,33 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
         default: return false;
       }
     };
+    // The result of conv + ADD shares its pitch with the residual.  To put it into a concatenated tensor, the residual (and
+    // what was added to that, and so on) is given rows of the same width, the rest of them unused: that costs memory but no
+    // traffic, where copying the result into its slice cost a read and a write of it (10 us for 16x160x160x32).
+    auto widen = [&](int t, int to, int reader, auto& self) -> bool {
+      const int pr = t > 0 ? producer[t] : -1;
+      if (pr < 0 || view_of_[t] >= 0 || cat_uses[t] > 0 || logical_[t] != channels_[t] || row_[t] != channels_[t] || row_[t] > to) return false;
+      const int res = nodes_[pr].add_res;
+      if (ops[pr].kind != NNCV_HIP_OP_CONV || (res < 0 && !writes_pitched(pr))) return false;
+      for (int j = 0; j < n; ++j)
+        for (int q = 0; q < 4; ++q)
+          if (ops[j].in[q] == t && !(j == reader + 1 && nodes_[j].skip) && !reads_pitched(j, t)) return false;
+      if (res >= 0 && !self(res, to, pr, self)) return false;
+      row_[t] = to;
+      return true;
+    };
     for (int i = 0; i < n; ++i) {
       if (ops[i].kind != NNCV_HIP_OP_CONCAT) continue;
       int c0 = 0;
       for (int k = 0; k < 4; ++k) {
         const int t = ops[i].in[k];
         if (t < 0) continue;
-        bool ok = t != 0 && cat_uses[t] == 1 && producer[t] >= 0 && writes_pitched(producer[t]) && logical_[t] == channels_[t];
+        const int res = producer[t] >= 0 ? nodes_[producer[t]].add_res : -1;
+        bool ok = t != 0 && cat_uses[t] == 1 && producer[t] >= 0 && (res >= 0 || writes_pitched(producer[t])) && logical_[t] == channels_[t];
         for (int j = 0; ok && j < n; ++j)
           for (int q = 0; q < 4; ++q)
             if (ops[j].in[q] == t && !reads_pitched(j, t)) ok = false;
+        if (ok && res >= 0) ok = cat_uses[ops[i].out] == 0 && widen(res, channels_[ops[i].out], producer[t], widen);
         if (ok) {
           view_of_[t] = ops[i].out;
           view_c0_[t] = c0;
@@ -443,7 +494,7 @@ const Graph::Plan& Graph::plan_of(int N, int H, int W) const {
   for (int i = 0; i < n; ++i) {
     const int t = nodes_[i].op.out;
     const Dims d = p.dims[t];
-    life[t] = TensorLife{i + 1, std::max(i + 1, last_use_[t] + 1), (size_t)N * d.H * d.W * d.C * es, 0};
+    life[t] = TensorLife{i + 1, std::max(i + 1, last_use_[t] + 1), (size_t)N * d.H * d.W * (nodes_[i].op.kind == NNCV_HIP_OP_YOLO_DETECT ? d.C : row_[t]) * es, 0};
     if (nodes_[i].op.kind == NNCV_HIP_OP_YOLO_DETECT) life[t].bytes = 256;  // written straight to the caller's buffer
   }
   // Operators that were merged into an earlier launch write their result at that launch's step, so the
@@ -464,6 +515,7 @@ const Graph::Plan& Graph::plan_of(int N, int H, int W) const {
       life[nodes_[i + 4].op.out].first_op = i + 1;
     }
     if (nodes_[i].add_out >= 0) life[nodes_[i].add_out].first_op = std::min(life[nodes_[i].add_out].first_op, i + 1);
+    if (nodes_[i].joins >= 0) life[nodes_[nodes_[i].joins].op.out].first_op = i + 1;  // (also where the shape is not joined)
   }
   {
     auto pool5 = [&](int k, int in) {
@@ -502,10 +554,48 @@ const Graph::Plan& Graph::plan_of(int N, int H, int W) const {
     p.offset[t] = life[root].offset + (size_t)c0 * es;
     p.root_bytes[t] = life[root].bytes;
   }
+  // Joined convolutions: one launch where the LDS ring takes the doubled filters and both results lie within its reach.
+  p.joint.assign(n, 0);
+  for (int i = 0; i < n; ++i) {
+    if (nodes_[i].joins < 0) continue;
+    const IgemmArgs g = joint_args(p, i, nullptr);
+    p.joint[i] = g.in_bytes < 0x7fffff00u && !igemm_takes_direct(g, dt_, dt_) && conv_ring_applicable(g, dt_, dt_);
+  }
   check_plan(p);
   if (plans_.size() >= 8) plans_.erase(plans_.begin());
   plans_.push_back(std::move(p));
   return plans_.back();
+}
+
+bool Graph::joint_second(const Plan& p, int i) const {
+  for (int k = 0; k < i; ++k)
+    if (nodes_[k].joins == i) return p.joint[k];
+  return false;
+}
+
+int Graph::pitch(int t) const {
+  int root, c0;
+  root_of(t, &root, &c0);
+  return row_[root];
+}
+
+// The launch that computes operator i and the one it joins: filters of both, results to two tensors.
+IgemmArgs Graph::joint_args(const Plan& p, int i, char* base) const {
+  const Node &nd = nodes_[i], &nj = nodes_[nd.joins];
+  const Dims a = p.dims[nd.op.in[0]];
+  const int F = nd.op.F, t = nd.op.out, u = nj.op.out, ldi = pitch(nd.op.in[0]);
+  IgemmArgs g{};
+  g.in = base + p.offset[nd.op.in[0]]; g.wt = nd.wt.get(); g.wt_flat = nd.wflat.get();
+  g.scale = nd.scale.as<float>(); g.shift = nd.shift.as<float>();
+  g.N = p.N; g.H = g.OH = a.H; g.W = g.OW = a.W; g.C = a.C; g.F = 2 * F; g.R = g.S = 1;
+  g.stride_h = g.stride_w = 1; g.relu = nd.op.act; g.batch = 1;
+  g.pix_stride = ldi;
+  const unsigned long long span = (unsigned long long)p.N * a.H * a.W * ldi * dtype_size(dt_);
+  g.in_bytes = span < 0xffffffffull ? (unsigned)span : 0xffffffffu;
+  g.out = base + p.offset[t]; g.ldo = pitch(t);
+  g.split_f = F; g.split_ldo = pitch(u); g.split_ofs = (long long)p.offset[u] - (long long)p.offset[t];
+  g.alg_flops = 2.0 * p.N * a.H * a.W * 2 * F * (double)logical_[nd.op.in[0]];
+  return g;
 }
 
 // The tensors one launch of forward() touches: what it writes and what it reads.
@@ -516,6 +606,13 @@ void Graph::launch_io(const Plan& p, int i, std::vector<int>* writes, std::vecto
   const Node& nd = nodes_[i];
   const GraphOp& op = nd.op;
   if (nd.skip) return;
+  if (nd.joined && joint_second(p, i)) return;
+  if (nd.joins >= 0 && p.joint[i]) {
+    reads->push_back(op.in[0]);
+    writes->push_back(op.out);
+    writes->push_back(nodes_[nd.joins].op.out);
+    return;
+  }
   if (op.kind == NNCV_HIP_OP_CONV && i + 1 < n && nodes_[i + 1].expands == i && p.dw[i + 1]) {
     reads->push_back(op.in[0]);
     writes->push_back(nodes_[i + 1].op.out);
@@ -617,13 +714,6 @@ void Graph::forward(const void* src, int N, int H, int W, float* out, void* ws, 
   const Plan& p = plan_of(N, H, W);
   char* base = static_cast<char*>(ws);
   auto at = [&](int t) -> void* { return base + p.offset[t]; };
-  // elements between consecutive pixels of tensor t: its own channel count, or that of the
-  // concatenated tensor it lives in
-  auto pitch = [&](int t) {
-    int root, c0;
-    root_of(t, &root, &c0);
-    return channels_[root];
-  };
   const bool pairs = pair_stem_ >= 0 && W % 2 == 0;
   if (pairs)
     launch_image_to_nhwc(src, at(0), dt_, N, c_in_, H, W, s, 4);
@@ -636,7 +726,11 @@ void Graph::forward(const void* src, int N, int H, int W, float* out, void* ws, 
     const Node& nd = nodes_[i];
     const GraphOp& op = nd.op;
     const Dims a = p.dims[op.in[0]], o = p.dims[op.out];
-    if (nd.skip) continue;
+    if (nd.skip || (nd.joined && joint_second(p, (int)i))) continue;
+    if (nd.joins >= 0 && p.joint[i]) {
+      launch_conv_ring(joint_args(p, (int)i, base), s);
+      continue;
+    }
     if (op.kind == NNCV_HIP_OP_CONV && i + 1 < nodes_.size() && nodes_[i + 1].expands == (int)i && p.dw[i + 1]) continue;  // rides below
     if (op.kind == NNCV_HIP_OP_DWCONV && p.dw[i]) {
       DwBlockArgs d{};

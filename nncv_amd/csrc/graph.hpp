@@ -58,6 +58,9 @@ class Graph {
     // squeeze-excitation block follows, the launch leaves the channel sums in the memory of the pooling operator's tensor;
     // on that GAVGPOOL, projects = the 1x1 CONV that is the only reader of the gated tensor.
     int expands = -1, projects = -1;
+    // 1x1 convolutions that may run as one launch (Plan::joint): on the first one, the index of the second
+    int joins = -1;
+    bool joined = false;
     DeviceBuffer wt_t;  // the two vectors' weights of such a block, [in][out]
   };
   struct Dims { int C, H, W; };
@@ -68,6 +71,7 @@ class Graph {
     std::vector<size_t> root_bytes;  // per tensor: size of the memory block it lives in
     std::vector<int> dw;             // per operator: bands of a DWCONV that runs as a dw_block, 0: as its own operators
     std::vector<char> se;            // per operator: this GAVGPOOL starts a se_project launch
+    std::vector<char> joint;         // per operator: its launch computes the one it joins as well
     size_t total;
   };
   const Plan& plan_of(int N, int H, int W) const;
@@ -89,6 +93,10 @@ class Graph {
   // per pixel) and that convolution walks pairs (launch_weight_pairs); -1 otherwise.
   int pair_stem_ = -1;
   void root_of(int t, int* root, int* c0) const;
+  std::vector<int> row_;  // per tensor that is no view: elements between consecutive pixels, its channel count or more
+  int pitch(int t) const;  // the same for any tensor
+  IgemmArgs joint_args(const Plan& p, int i, char* base) const;
+  bool joint_second(const Plan& p, int i) const;  // operator i is computed by the one that joins it
   std::vector<float> detect_anchor_wh_, detect_stride_;  // YOLO_DETECT: host copies of anchors * stride, strides
   std::vector<int> last_use_;  // per tensor: index of the last operator that reads it
   mutable std::vector<Plan> plans_;

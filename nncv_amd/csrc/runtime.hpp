@@ -34,6 +34,12 @@ class DeviceBuffer {
   }
   // from `pool` (which outlives this), or an allocation of its own where there is none
   void reset(size_t bytes, DevicePool* pool);
+  void borrow(void* p, size_t bytes) {  // memory of another buffer, which outlives this one
+    release();
+    p_ = p;
+    n_ = bytes;
+    owned_ = false;
+  }
   void release() {
     if (p_ && owned_) (void)hipFree(p_);
     p_ = nullptr;
