@@ -329,6 +329,24 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
     if (nodes_[i].joins >= 0 && !(single(i) && single(nodes_[i].joins))) nodes_[nodes_[i].joins].joined = false, nodes_[i].joins = -1;
   }
 
+  // detection heads
+  if (dt == kF16 && ops[n - 1].kind == NNCV_HIP_OP_YOLO_DETECT) {
+    const GraphOp& d = ops[n - 1];
+    std::vector<int> made;
+    bool ok = true;
+    for (int k = 0; k < 3 && d.in[k] >= 0; ++k) {
+      int h = -1;
+      for (int i = 0; i < n; ++i)
+        if (ops[i].out == d.in[k]) h = i;
+      const GraphOp& c = ops[std::max(h, 0)];
+      ok = ok && h >= 0 && c.kind == NNCV_HIP_OP_CONV && c.K == 1 && c.stride == 1 && c.pad == 0 && c.in[0] > 0 && c.in[1] < 0 && c.act == kActNone &&
+           readers[d.in[k]] == 1 && !nodes_[h].skip && !nodes_[h].joined && nodes_[h].joins < 0 && logical_[c.in[0]] == channels_[c.in[0]] &&
+           detect_head_applicable(d.K, d.F, channels_[c.in[0]], 0);
+      made.push_back(h);
+    }
+    for (int h : made) nodes_[std::max(h, 0)].head = ok;
+  }
+
   // concatenation views
   row_ = channels_;
   view_of_.assign(n_tensors_, -1);
@@ -528,6 +546,17 @@ const Graph::Plan& Graph::plan_of(int N, int H, int W) const {
         life[nodes_[i + 2].op.out].first_op = i + 1;
       }
   }
+  p.head = nodes_[n - 1].op.kind == NNCV_HIP_OP_YOLO_DETECT;
+  for (int k = 0; p.head && k < 3 && nodes_[n - 1].op.in[k] >= 0; ++k) {
+    const Node* c = maker(nodes_[n - 1].op.in[k]);
+    const int t = c ? c->op.in[0] : 0;
+    p.head = c && c->head && detect_head_applicable(nodes_[n - 1].op.K, nodes_[n - 1].op.F, channels_[t], (long long)N * p.dims[t].H * p.dims[t].W * pitch(t) * (long long)es);
+  }
+  for (int k = 0; p.head && k < 3 && nodes_[n - 1].op.in[k] >= 0; ++k) {  // the heads are never stored, what they read lives on
+    const int h = nodes_[n - 1].op.in[k], t = maker(h)->op.in[0];
+    life[t].last_op = std::max(life[t].last_op, n);
+    life[h] = TensorLife{n, n, 0, 0};
+  }
   life[nodes_[n - 1].op.out].last_op = n + 1;
   // a tensor that lives inside a concatenated one has no memory of its own; the concatenated
   // tensor is live from its first such input to the last reader of any of them
@@ -565,6 +594,12 @@ const Graph::Plan& Graph::plan_of(int N, int H, int W) const {
   if (plans_.size() >= 8) plans_.erase(plans_.begin());
   plans_.push_back(std::move(p));
   return plans_.back();
+}
+
+const Graph::Node* Graph::maker(int t) const {
+  for (const Node& nd : nodes_)
+    if (nd.op.out == t) return &nd;
+  return nullptr;
 }
 
 bool Graph::joint_second(const Plan& p, int i) const {
@@ -605,7 +640,12 @@ void Graph::launch_io(const Plan& p, int i, std::vector<int>* writes, std::vecto
   const int n = (int)nodes_.size();
   const Node& nd = nodes_[i];
   const GraphOp& op = nd.op;
-  if (nd.skip) return;
+  if (nd.skip || (nd.head && p.head)) return;
+  if (op.kind == NNCV_HIP_OP_YOLO_DETECT && p.head) {
+    for (int k = 0; k < 3; ++k)
+      if (op.in[k] >= 0) reads->push_back(maker(op.in[k])->op.in[0]);
+    return;
+  }
   if (nd.joined && joint_second(p, i)) return;
   if (nd.joins >= 0 && p.joint[i]) {
     reads->push_back(op.in[0]);
@@ -726,7 +766,7 @@ void Graph::forward(const void* src, int N, int H, int W, float* out, void* ws, 
     const Node& nd = nodes_[i];
     const GraphOp& op = nd.op;
     const Dims a = p.dims[op.in[0]], o = p.dims[op.out];
-    if (nd.skip || (nd.joined && joint_second(p, (int)i))) continue;
+    if (nd.skip || (nd.head && p.head) || (nd.joined && joint_second(p, (int)i))) continue;
     if (nd.joins >= 0 && p.joint[i]) {
       launch_conv_ring(joint_args(p, (int)i, base), s);
       continue;
@@ -852,6 +892,23 @@ void Graph::forward(const void* src, int N, int H, int W, float* out, void* ws, 
         break;
       case NNCV_HIP_OP_YOLO_DETECT: {
         long long box0 = 0;
+        if (p.head) {
+          DetectHeadArgs d{};
+          d.out = out; d.N = N; d.A = op.K; d.F = op.F; d.boxes_total = o.C;
+          while (d.levels < 3 && op.in[d.levels] >= 0) ++d.levels;
+          for (int k = 0; k < d.levels; ++k) {
+            const Node& c = *maker(op.in[k]);
+            const int t = c.op.in[0];
+            const Dims h = p.dims[t];
+            DetectHeadLevel& v = d.lv[d.levels - 1 - k];  // (the later levels are the ones with more channels)
+            v.in = at(t); v.wt = c.wt.get(); v.scale = c.scale.as<float>(); v.shift = c.shift.as<float>();
+            v.HW = h.H * h.W; v.W = h.W; v.pix = pitch(t); v.C = h.C; v.rows = channels_[c.op.out]; v.box0 = box0; v.stride = detect_stride_[k];
+            for (int q = 0; q < op.K * 2; ++q) v.anchor_wh[q] = detect_anchor_wh_[k * op.K * 2 + q];
+            box0 += (long long)op.K * h.H * h.W;
+          }
+          launch_detect_head(d, s);
+          break;
+        }
         for (int k = 0; k < 3 && op.in[k] >= 0; ++k) {
           const Dims h = p.dims[op.in[k]];
           DetectArgs d{};

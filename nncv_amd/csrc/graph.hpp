@@ -60,6 +60,7 @@ class Graph {
     int expands = -1, projects = -1;
     // 1x1 convolutions that may run as one launch (Plan::joint): on the first one, the index of the second
     int joins = -1;
+    bool head = false;  // a 1x1 CONV that only the YOLO_DETECT reads and whose launch may compute it (Plan::head)
     bool joined = false;
     DeviceBuffer wt_t;  // the two vectors' weights of such a block, [in][out]
   };
@@ -71,6 +72,7 @@ class Graph {
     std::vector<size_t> root_bytes;  // per tensor: size of the memory block it lives in
     std::vector<int> dw;             // per operator: bands of a DWCONV that runs as a dw_block, 0: as its own operators
     std::vector<char> se;            // per operator: this GAVGPOOL starts a se_project launch
+    bool head = false;               // the YOLO_DETECT launch computes the convolutions that it reads
     std::vector<char> joint;         // per operator: its launch computes the one it joins as well
     size_t total;
   };
@@ -96,6 +98,7 @@ class Graph {
   std::vector<int> row_;  // per tensor that is no view: elements between consecutive pixels, its channel count or more
   int pitch(int t) const;  // the same for any tensor
   IgemmArgs joint_args(const Plan& p, int i, char* base) const;
+  const Node* maker(int t) const;  // the operator whose result t is
   bool joint_second(const Plan& p, int i) const;  // operator i is computed by the one that joins it
   std::vector<float> detect_anchor_wh_, detect_stride_;  // YOLO_DETECT: host copies of anchors * stride, strides
   std::vector<int> last_use_;  // per tensor: index of the last operator that reads it
