@@ -213,10 +213,20 @@ bool launch_conv3x3_stream(const IgemmArgs& a, hipStream_t s);
 bool conv3x3_stream_plan(int N, int H, int W, int C, int F, int out[14]);
 size_t weight_frag32_bytes(int F, int C);
 void launch_weight_frag32(const void* w, int w_dt, void* dst, int F, int C, hipStream_t s);
-// Stride-2 image convolutions over pixel pairs (C = 8, fp16, 6x3 and 3x2 windows, at most 64 filters):
-// the whole K axis in one step (conv_pairs.hip); same arguments and epilogue as the igemm kernels.
+// 1x1 convolutions of few channels (fp16), the whole K axis in one step (conv_pairs.hip); same arguments and epilogue as the
+// igemm kernels.
 bool conv_pairs_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 void launch_conv_pairs(const IgemmArgs& a, hipStream_t s);
+// Stride-2 convolutions of an fp16 NCHW image of at most four channels, over pairs of pixels: 6x3 and 3x2 windows of pairs (R, S,
+// pad_w count pairs; wt from launch_weight_pairs), at most 64 filters, even W.  NHWC out.
+struct ImagePairsArgs {
+  const void* in; const void* wt; const float* scale; const float* shift; void* out;
+  int N, C, H, W, F, R, S, OH, OW, pad_h, pad_w, ldo, act;
+  double alg_flops;
+  unsigned in_bytes, wt_bytes; int tiles_x, tiles_y; float inv_tx, inv_ty;  // filled in by the launcher
+};
+bool image_pairs_applicable(const ImagePairsArgs& a);
+void launch_image_pairs(const ImagePairsArgs& a, hipStream_t s);
 // Barrier-free implicit GEMM for fp32 layers and small fp16 layers (conv_direct.hip); `wins`: its modelled time against
 // that of the kernel which would run the layer otherwise.
 enum DirectRival : int { kRivalPatch = 0, kRivalPatchS2 = 1, kRivalIgemmFast = 2, kRivalIgemm = 3, kRivalShortK = 4, kRivalRing = 5 };

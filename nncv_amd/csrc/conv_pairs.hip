@@ -1,15 +1,14 @@
 // Convolutions whose whole K axis is a handful of 16-byte chunks (fp16), in two forms:
-//  * the stride-2 first layer of a network whose input has at most four channels, once the graph
-//    executor has packed the image as [N][H][W/2][2 pixels x 4 channels]: the horizontal walk is
-//    stride 1 over S pairs, every filter tap is one chunk and K is R*S chunks, 18 for YOLOv5s'
-//    6x6 window, 6 for MobileNetV3's 3x3 (tests/Nets/Yolov5s.mlir, tests/Nets/MobileNetV3.mlir);
-//  * 1x1 convolutions over at most 144 channels in multiples of 8 (MobileNetV3's expansion and
+//  * image_pairs: the stride-2 first layer of a network whose image has at most four channels, straight from the NCHW image:
+//    two horizontally adjacent pixels x 4 channels are one chunk, the horizontal walk is stride 1 over S pairs and K is R*S
+//    chunks, 18 for YOLOv5s' 6x6 window, 6 for MobileNetV3's 3x3 (tests/Nets/Yolov5s.mlir, tests/Nets/MobileNetV3.mlir);
+//  * conv1x1_shortk: 1x1 convolutions over at most 144 channels in multiples of 8 (MobileNetV3's expansion and
 //    projection layers, 16..144 channels: none of them a multiple of the 64-byte K step of the
 //    pipelined kernel), with the residual add of an inverted-residual block.
 // Replaces the compiler's tiling of linalg.conv_2d_nchw_fchw for those layers
 // (src/nncv/compiler/Conversion/CodeGen/LlvmCpu/ModernTile.cpp:124-286).
 //
-// K is so short that a pipelined K walk through LDS only adds barriers.  A wave owns 64 pixels x 32
+// K is so short that a pipelined K walk through LDS only adds barriers.  In the 1x1 form a wave owns 64 pixels x 32
 // or 64 filters and needs no staging at all: lane (pixel l%32, chunk half l/32) of MFMA step kk reads
 // chunk 2*kk + l/32 of its pixel straight from global memory, ALL steps requested back to back (one
 // latency), the filters sit in registers.  The epilogue (scale/shift, residual, activation, one
@@ -27,14 +26,12 @@ namespace {
 constexpr unsigned kOOBc = 0x7fff0000u;  // byte offset beyond any buffer this kernel accepts
 }
 
-// PW = false: R x S window over pixel pairs (C = 8), KST = R*S/2.
-// PW = true : 1x1 window over C = 8*nch channels, nch <= 2*KST chunks (chunks past nch read as zero).
+// 1x1 window over C = 8*nch channels, nch <= 2*KST chunks (chunks past nch read as zero).
 // WV waves per workgroup, 64 pixels each (1 for small launches: more, smaller workgroups).
 // RES: the launch has a residual input (instances without one carry no registers or code for it).
-template <bool PW, int R, int S, int KST, int NI, int WV, bool RES>
+template <int KST, int NI, int WV, bool RES>
 __global__ __launch_bounds__(64 * WV) void conv_pairs_kernel(const IgemmArgs a) {
   constexpr int TP = 64 * NI + 16;  // bytes per pixel row of the output tile: 32*NI halves + pad
-  static_assert(PW || R * S == 2 * KST, "an MFMA step takes two chunks");
   __shared__ __align__(16) unsigned char smem[WV * 64 * TP];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -42,44 +39,21 @@ __global__ __launch_bounds__(64 * WV) void conv_pairs_kernel(const IgemmArgs a) 
   const int P = a.N * a.OH * a.OW;
   const int f0 = blockIdx.y * (32 * NI);
   const int p0 = blockIdx.x * (64 * WV) + wave * 64;
-  const int nch = PW ? a.C / 8 : R * S;  // chunks per pixel = chunks per filter row
+  const int nch = a.C / 8;  // chunks per pixel = chunks per filter row
   const __amdgpu_buffer_rsrc_t rs_in = make_rsrc(a.in, a.in_bytes);
   const __amdgpu_buffer_rsrc_t rs_wt = make_rsrc(a.wt, a.wt_bytes);
 
   // ---- this lane's two pixels and its chunk of every step, requested back to back ----
   u32x4 b[KST][2];
-  if constexpr (PW) {
-    const int pix = a.pix_stride ? a.pix_stride : a.C;
+  const int pix = a.pix_stride ? a.pix_stride : a.C;
 #pragma unroll
-    for (int kk = 0; kk < KST; ++kk) {
-      const int c = 2 * kk + lchunk;
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int p = p0 + j * 32 + lrow;
-        const bool ok = (p < P) & (c < nch);
-        b[kk][j] = __builtin_amdgcn_raw_buffer_load_b128(rs_in, ok ? (unsigned)(p * pix + c * 8) * 2u : kOOBc, 0, 0);
-      }
-    }
-  } else {
-    int base[2], iy0[2], ix0[2];
-    const int ohow = a.OH * a.OW;
+  for (int kk = 0; kk < KST; ++kk) {
+    const int c = 2 * kk + lchunk;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int p = p0 + j * 32 + lrow;
-      const int n = p / ohow, rem = p - n * ohow;
-      const int oy = rem / a.OW, ox = rem - oy * a.OW;
-      iy0[j] = p < P ? oy * a.stride_h - a.pad_h : -(1 << 28);  // pixels past the end: never inside the image
-      ix0[j] = ox * a.stride_w - a.pad_w;
-      base[j] = (n * a.H + iy0[j]) * a.W + ix0[j];  // in pairs; only used when the tap is in bounds
-    }
-#pragma unroll
-    for (int kk = 0; kk < KST; ++kk) {
-      const int c = 2 * kk + lchunk, r = c / S, s = c - r * S;
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const bool ok = ((unsigned)(iy0[j] + r) < (unsigned)a.H) & ((unsigned)(ix0[j] + s) < (unsigned)a.W);
-        b[kk][j] = __builtin_amdgcn_raw_buffer_load_b128(rs_in, ok ? (unsigned)(base[j] + r * a.W + s) * 16u : kOOBc, 0, 0);
-      }
+      const bool ok = (p < P) & (c < nch);
+      b[kk][j] = __builtin_amdgcn_raw_buffer_load_b128(rs_in, ok ? (unsigned)(p * pix + c * 8) * 2u : kOOBc, 0, 0);
     }
   }
   // ---- the filters: row f is nch chunks; lane (filter l%32, chunk half l/32) of step kk holds
@@ -174,7 +148,6 @@ __global__ __launch_bounds__(64 * WV) void conv_pairs_kernel(const IgemmArgs a) 
 }
 
 bool conv_pairs_applicable(const IgemmArgs& a, int in_dt, int out_dt) {
-  static const bool off = getenv("NNCV_HIP_NO_CONV_PAIRS") != nullptr;
   static const bool off_pw = getenv("NNCV_HIP_NO_CONV_SHORTK") != nullptr;
   const int pix = a.pix_stride ? a.pix_stride : a.C;
   const long long P = (long long)a.N * a.OH * a.OW;
@@ -182,10 +155,6 @@ bool conv_pairs_applicable(const IgemmArgs& a, int in_dt, int out_dt) {
                       P * a.ldo < (1ll << 31) && a.in_bytes > 0 && a.in_bytes < kOOBc && a.wt_bytes > 0 && a.wt_bytes < kOOBc &&
                       (a.relu & ~(0xff | kActResidualAfter)) == 0;
   if (!common) return false;
-  const bool window = (a.R == 6 && a.S == 3) || (a.R == 3 && a.S == 2);
-  if (window)
-    return !off && a.C == 8 && pix == 8 && a.F <= 64 && a.residual == nullptr && (a.relu & ~0xff) == 0 &&
-           (long long)a.N * a.H * a.W * 16 < (long long)kOOBc;
   // 1x1, stride 1, no padding: the output pixel is the input pixel.  The LDS ring (conv_ring.hip) is the better one for whole
   // multiples of 32 channels (64 -> 32 at 5880 pixels: 2.9 against 3.2 us), and from 24 channels on where its 64 x 64 tiles
   // give every CU one and more than 32 filters share a pixel's line (40 -> 240 at 6272 pixels: 3.5 against 4.7).
@@ -194,7 +163,7 @@ bool conv_pairs_applicable(const IgemmArgs& a, int in_dt, int out_dt) {
          a.OW == a.W && a.C % 8 == 0 && !ring && a.C <= 144 && pix % 8 == 0 && P * pix * 2 < (long long)kOOBc;
 }
 
-template <bool PW, int R, int S, int KST, int NI>
+template <int KST, int NI>
 static void launch_pairs_cfg(const IgemmArgs& a, const char* tag, hipStream_t s) {
   const long long P = (long long)a.N * a.OH * a.OW;
   const double flops = a.alg_flops > 0 ? a.alg_flops : 2.0 * P * a.F * a.R * a.S * a.C;
@@ -204,41 +173,169 @@ static void launch_pairs_cfg(const IgemmArgs& a, const char* tag, hipStream_t s)
   // fewer four-wave workgroups than CUs: one wave per workgroup instead
   const bool small = (P + 255) / 256 * gy < 256;
   const dim3 grid(small ? (unsigned)((P + 63) / 64) : (unsigned)((P + 255) / 256), gy), block(small ? 64 : 256);
-  if constexpr (PW) {
-    if (a.residual && small) hipLaunchKernelGGL((conv_pairs_kernel<PW, R, S, KST, NI, 1, true>), grid, block, 0, s, a);
-    else if (a.residual) hipLaunchKernelGGL((conv_pairs_kernel<PW, R, S, KST, NI, 4, true>), grid, block, 0, s, a);
-    else if (small) hipLaunchKernelGGL((conv_pairs_kernel<PW, R, S, KST, NI, 1, false>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((conv_pairs_kernel<PW, R, S, KST, NI, 4, false>), grid, block, 0, s, a);
-  } else {  // the image layers have no residual input (conv_pairs_applicable)
-    if (small) hipLaunchKernelGGL((conv_pairs_kernel<PW, R, S, KST, NI, 1, false>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((conv_pairs_kernel<PW, R, S, KST, NI, 4, false>), grid, block, 0, s, a);
-  }
+  if (a.residual && small) hipLaunchKernelGGL((conv_pairs_kernel<KST, NI, 1, true>), grid, block, 0, s, a);
+  else if (a.residual) hipLaunchKernelGGL((conv_pairs_kernel<KST, NI, 4, true>), grid, block, 0, s, a);
+  else if (small) hipLaunchKernelGGL((conv_pairs_kernel<KST, NI, 1, false>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((conv_pairs_kernel<KST, NI, 4, false>), grid, block, 0, s, a);
 }
 
 void launch_conv_pairs(const IgemmArgs& a, hipStream_t s) {
-  if (a.R == 6) {
-    if (a.F > 32) launch_pairs_cfg<false, 6, 3, 9, 2>(a, "conv_pairs<f16,6x3,64>", s);
-    else launch_pairs_cfg<false, 6, 3, 9, 1>(a, "conv_pairs<f16,6x3,32>", s);
-  } else if (a.R == 3) {
-    if (a.F > 32) launch_pairs_cfg<false, 3, 2, 3, 2>(a, "conv_pairs<f16,3x2,64>", s);
-    else launch_pairs_cfg<false, 3, 2, 3, 1>(a, "conv_pairs<f16,3x2,32>", s);
+  // K steps in registers: 1 (16 channels), 3 (..48), 6 (..96), 9 (..144).  64 filters per wave tile only for launches that
+  // fill the chip all the same (24 -> 112 at 1440 pixels: 4.1 us with 64, 3.1 with 32)
+  const int kst = (a.C / 8 + 1) / 2;
+  const bool many = ((long long)a.N * a.OH * a.OW + 63) / 64 * ((a.F + 63) / 64) >= 1024;
+  if (kst <= 1) {
+    if (a.F > 32 && many) launch_pairs_cfg<1, 2>(a, "conv1x1_shortk<f16,16,64>", s);
+    else launch_pairs_cfg<1, 1>(a, "conv1x1_shortk<f16,16,32>", s);
+  } else if (kst <= 3) {
+    launch_pairs_cfg<3, 1>(a, "conv1x1_shortk<f16,48,32>", s);
+  } else if (kst <= 6) {
+    launch_pairs_cfg<6, 1>(a, "conv1x1_shortk<f16,96,32>", s);
   } else {
-    // K steps in registers: 1 (16 channels), 3 (..48), 6 (..96), 9 (..144).  64 filters per wave tile only for launches that
-    // fill the chip all the same (24 -> 112 at 1440 pixels: 4.1 us with 64, 3.1 with 32)
-    const int kst = (a.C / 8 + 1) / 2;
-    const bool many = ((long long)a.N * a.OH * a.OW + 63) / 64 * ((a.F + 63) / 64) >= 1024;
-    if (kst <= 1) {
-      if (a.F > 32 && many) launch_pairs_cfg<true, 1, 1, 1, 2>(a, "conv1x1_shortk<f16,16,64>", s);
-      else launch_pairs_cfg<true, 1, 1, 1, 1>(a, "conv1x1_shortk<f16,16,32>", s);
-    } else if (kst <= 3) {
-      launch_pairs_cfg<true, 1, 1, 3, 1>(a, "conv1x1_shortk<f16,48,32>", s);
-    } else if (kst <= 6) {
-      launch_pairs_cfg<true, 1, 1, 6, 1>(a, "conv1x1_shortk<f16,96,32>", s);
-    } else {
-      launch_pairs_cfg<true, 1, 1, 9, 1>(a, "conv1x1_shortk<f16,144,32>", s);
-    }
+    launch_pairs_cfg<9, 1>(a, "conv1x1_shortk<f16,144,32>", s);
   }
   NNCV_HIP_CHECK(hipGetLastError());
+}
+
+// ---------------------------------------------------------------------------------------------
+// The image layer.  A workgroup makes 2*WV rows x 32 columns of the result: it reads the haloed rectangle of its image from
+// the channel planes (a dword is two pixels of a row; lanes walk a row's pairs), packs pairs of pixels into chunks on the
+// way into LDS, and a wave takes its operands for two rows from there, 32 consecutive chunks per read and half.
+// What bounds it: its bytes (16x640x640: 39 MB in, 105 out) and the SiLU of 52 million results (a quarter-rate exp and rcp
+// each).  Packing the image in a launch of its own wrote 52 MB that the convolution read again, every chunk nine times
+// through the vector caches: 23 + 56 us for YOLOv5s (F = 32), 52 now; 6.6 + 10.5 for MobileNetV3 (F = 16, 32x224x224), 10.2 now.
+// ---------------------------------------------------------------------------------------------
+template <int R, int S, int NI, int WV>
+__global__ __launch_bounds__(64 * WV) void image_pairs_kernel(const ImagePairsArgs a) {
+  constexpr int KST = R * S / 2, TP = 64 * NI + 16, kRows = 2 * (2 * WV - 1) + R, kCols = 32 + S - 1, kPitch = kCols * 16;
+  static_assert(R * S % 2 == 0, "an MFMA step takes two chunks");
+  constexpr int kLds = kRows * kPitch > WV * 64 * TP ? kRows * kPitch : WV * 64 * TP, kEach = (kRows * kCols + 64 * WV - 1) / (64 * WV);
+  __shared__ __align__(16) unsigned char smem[kLds];  // the packed rectangle, then the waves' outgoing tiles
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lrow = lane & 31, lh = lane >> 5;
+  // XCD x takes a run of tiles: neighbours share halo lines in its L2
+  const int tiles = a.N * a.tiles_y * a.tiles_x, t = (blockIdx.x & 7) * ((tiles + 7) >> 3) + (blockIdx.x >> 3);
+  if (t >= tiles) return;  // (uniform; before any barrier)
+  int tx, ty;
+  const int rowt = fast_div(t, a.tiles_x, a.inv_tx, &tx), n = fast_div(rowt, a.tiles_y, a.inv_ty, &ty);
+  const int oy0 = __builtin_amdgcn_readfirstlane(ty * 2 * WV), ox0 = __builtin_amdgcn_readfirstlane(tx * 32), img = __builtin_amdgcn_readfirstlane(n);
+  const __amdgpu_buffer_rsrc_t rs_in = make_rsrc(a.in, a.in_bytes), rs_wt = make_rsrc(a.wt, a.wt_bytes);
+
+  unsigned d[kEach][4];
+  const unsigned plane = (unsigned)(a.H * a.W) * 2u;
+#pragma unroll
+  for (int i = 0; i < kEach; ++i) {
+    const int e = i * 64 * WV + tid, row = e / kCols, col = e - row * kCols, iy = 2 * oy0 - a.pad_h + row, ip = ox0 - a.pad_w + col;
+    const bool ok = (e < kRows * kCols) & ((unsigned)iy < (unsigned)a.H) & ((unsigned)ip < (unsigned)(a.W >> 1));
+    const unsigned off = ok ? (unsigned)(iy * a.W + 2 * ip) * 2u : kOOBc;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) d[i][c] = c < a.C ? __builtin_amdgcn_raw_buffer_load_b32(rs_in, off, (unsigned)(img * a.C + c) * plane, 0) : 0u;
+  }
+  u32x4 w[KST][NI];
+#pragma unroll
+  for (int kk = 0; kk < KST; ++kk)
+#pragma unroll
+    for (int i = 0; i < NI; ++i) w[kk][i] = __builtin_amdgcn_raw_buffer_load_b128(rs_wt, (unsigned)(((i * 32 + lrow) * R * S + 2 * kk + lh) * 16), 0, 0);
+#pragma unroll
+  for (int i = 0; i < kEach; ++i) {
+    const int e = i * 64 * WV + tid;
+    if (e < kRows * kCols)
+      *reinterpret_cast<u32x4*>(smem + e * 16) = u32x4{(d[i][0] & 0xffffu) | (d[i][1] << 16), (d[i][2] & 0xffffu) | (d[i][3] << 16),
+                                                      (d[i][0] >> 16) | (d[i][1] & 0xffff0000u), (d[i][2] >> 16) | (d[i][3] & 0xffff0000u)};
+  }
+  __syncthreads();
+
+  floatx16 acc[NI][2];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+  // chunks 2 kk and 2 kk + 1 of the window: neighbours of a row, or the last of one and the first of the next
+  const unsigned char* base = smem + 4 * wave * kPitch + lrow * 16;
+  const unsigned char *next = base + lh * 16, *wrap = base + lh * (kPitch - (S - 1) * 16);
+#pragma unroll
+  for (int kk = 0; kk < KST; ++kk) {
+    const int r = 2 * kk / S, c = 2 * kk - r * S;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const u32x4 b = *reinterpret_cast<const u32x4*>((c == S - 1 ? wrap : next) + (2 * j + r) * kPitch + c * 16);
+#pragma unroll
+      for (int i = 0; i < NI; ++i) Mma<half_t>::run(w[kk][i], b, acc[i][j]);
+    }
+  }
+  __syncthreads();
+
+  unsigned char* tile = smem + wave * (64 * TP);
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    floatx4 sc[4], sh[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int f = i * 32 + 8 * q + 4 * lh;
+      sc[q] = a.scale && f < a.F ? *reinterpret_cast<const floatx4*>(a.scale + f) : floatx4{1.f, 1.f, 1.f, 1.f};
+      sh[q] = a.shift && f < a.F ? *reinterpret_cast<const floatx4*>(a.shift + f) : floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      float y[16];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) y[e] = acc[i][j][e] * sc[e >> 2][e & 3] + sh[e >> 2][e & 3];
+      act_apply_n<true>(y, a.act);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        half4 h;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) h[e] = (half_t)y[4 * q + e];
+        *reinterpret_cast<half4*>(tile + (j * 32 + lrow) * TP + (i * 32 + 8 * q + 4 * lh) * 2) = h;
+      }
+    }
+  }
+  // whole pixel rows out: 4*NI lanes cover the 32*NI channels of one pixel (a wave's own tile: no barrier)
+  constexpr int LPR = 4 * NI, RPI = 64 / LPR;
+  const int fc = (lane % LPR) * 8;
+  half_t* out = static_cast<half_t*>(a.out);
+#pragma unroll
+  for (int it = 0; it < 64 / RPI; ++it) {
+    const int row = it * RPI + lane / LPR, oy = oy0 + 2 * wave + (row >> 5), ox = ox0 + (row & 31);
+    const u32x4 v = *reinterpret_cast<const u32x4*>(tile + row * TP + fc * 2);
+    if (oy < a.OH && ox < a.OW && fc < a.F) *reinterpret_cast<u32x4*>(out + ((long long)(img * a.OH + oy) * a.OW + ox) * a.ldo + fc) = v;
+  }
+}
+
+bool image_pairs_applicable(const ImagePairsArgs& a) {
+  static const bool off = getenv("NNCV_HIP_NO_CONV_PAIRS") != nullptr;
+  const bool window = (a.R == 6 && a.S == 3) || (a.R == 3 && a.S == 2);
+  return !off && window && a.C >= 1 && a.C <= 4 && a.W % 2 == 0 && a.F % 8 == 0 && a.F <= 64 && a.ldo % 8 == 0 &&
+         (long long)a.N * a.C * a.H * a.W * 2 < (long long)kOOBc && (long long)a.N * ((a.OH + 1) / 2) * ((a.OW + 31) / 32) < (1 << 24) &&
+         reinterpret_cast<uintptr_t>(a.in) % 4 == 0;
+}
+
+template <int R, int S, int NI>
+static void launch_image_cfg(ImagePairsArgs a, const char* tag, hipStream_t s) {
+  // tiles of 8 rows; of 2 where those would leave CUs without a workgroup
+  const bool small = (long long)a.N * ((a.OH + 7) / 8) * ((a.OW + 31) / 32) < 256;
+  const int th = small ? 2 : 8;
+  a.tiles_y = (a.OH + th - 1) / th; a.tiles_x = (a.OW + 31) / 32;
+  a.inv_tx = 1.0f / (float)a.tiles_x; a.inv_ty = 1.0f / (float)a.tiles_y;
+  a.in_bytes = (unsigned)((long long)a.N * a.C * a.H * a.W * 2);
+  a.wt_bytes = (unsigned)(a.F * a.R * a.S * 16);
+  const double px = (double)a.N * a.OH * a.OW;
+  ProfScope prof(tag, a.alg_flops, 2.0 * ((double)a.N * a.C * a.H * a.W + (double)a.F * a.R * a.S * 8 + px * a.F), s);
+  const dim3 grid((unsigned)((a.N * a.tiles_y * a.tiles_x + 7) / 8 * 8));
+  if (small) hipLaunchKernelGGL((image_pairs_kernel<R, S, NI, 1>), grid, dim3(64), 0, s, a);
+  else hipLaunchKernelGGL((image_pairs_kernel<R, S, NI, 4>), grid, dim3(256), 0, s, a);
+  NNCV_HIP_CHECK(hipGetLastError());
+}
+
+void launch_image_pairs(const ImagePairsArgs& a, hipStream_t s) {
+  if (a.R == 6) {
+    if (a.F > 32) launch_image_cfg<6, 3, 2>(a, "conv_pairs<f16,6x3,64>", s);
+    else launch_image_cfg<6, 3, 1>(a, "conv_pairs<f16,6x3,32>", s);
+  } else {
+    if (a.F > 32) launch_image_cfg<3, 2, 2>(a, "conv_pairs<f16,3x2,64>", s);
+    else launch_image_cfg<3, 2, 1>(a, "conv_pairs<f16,3x2,32>", s);
+  }
 }
 
 }  // namespace nncv_hip

@@ -755,7 +755,20 @@ void Graph::forward(const void* src, int N, int H, int W, float* out, void* ws, 
   char* base = static_cast<char*>(ws);
   auto at = [&](int t) -> void* { return base + p.offset[t]; };
   const bool pairs = pair_stem_ >= 0 && W % 2 == 0;
-  if (pairs)
+  ImagePairsArgs image{};
+  if (pairs) {
+    const Node& nd = nodes_[pair_stem_];
+    const Dims o = p.dims[nd.op.out];
+    image.in = src; image.wt = nd.wt_pairs.get(); image.scale = nd.scale.as<float>(); image.shift = nd.shift.as<float>(); image.out = at(nd.op.out);
+    image.N = N; image.C = c_in_; image.H = H; image.W = W; image.F = o.C; image.OH = o.H; image.OW = o.W;
+    image.R = nd.op.K; image.S = (nd.op.K + (nd.op.pad & 1) + 1) / 2; image.pad_h = nd.op.pad; image.pad_w = (nd.op.pad + 1) / 2;
+    image.ldo = pitch(nd.op.out); image.act = nd.op.act;
+    image.alg_flops = 2.0 * N * o.H * o.W * nd.op.F * (double)nd.op.K * nd.op.K * c_in_;
+  }
+  const bool direct = pairs && nodes_[pair_stem_].add_out < 0 && image_pairs_applicable(image);
+  if (direct) {
+    // its one reader takes the image as it is
+  } else if (pairs)
     launch_image_to_nhwc(src, at(0), dt_, N, c_in_, H, W, s, 4);
   else if (image_to_nhwc_applicable(dt_, c_in_))
     launch_image_to_nhwc(src, at(0), dt_, N, c_in_, H, W, s);
@@ -766,6 +779,10 @@ void Graph::forward(const void* src, int N, int H, int W, float* out, void* ws, 
     const Node& nd = nodes_[i];
     const GraphOp& op = nd.op;
     const Dims a = p.dims[op.in[0]], o = p.dims[op.out];
+    if (direct && (int)i == pair_stem_) {
+      launch_image_pairs(image, s);
+      continue;
+    }
     if (nd.skip || (nd.head && p.head) || (nd.joined && joint_second(p, (int)i))) continue;
     if (nd.joins >= 0 && p.joint[i]) {
       launch_conv_ring(joint_args(p, (int)i, base), s);
