@@ -35,6 +35,7 @@ void Context::init(int device) {
   // the code objects in this library exist for gfx950 only; anything else cannot run them
   NNCV_REQUIRE(arch_.rfind("gfx950", 0) == 0, "this library is built for gfx950 (MI355X); found " + arch_);
   NNCV_HIP_CHECK(hipStreamCreate(&stream_));  // default priority
+  order.create();
   device_ = device;
   ready_ = true;
   (void)noalloc_scratch();  // the scratch array's address on this device, resolved with the device current
@@ -49,27 +50,29 @@ hipEvent_t Context::event(size_t i) {
   return events_[i];
 }
 
+TailEvent*& tail_event() {
+  static thread_local TailEvent* t = nullptr;
+  return t;
+}
+
 StreamOrder::~StreamOrder() {
   if (ev_) (void)hipEventDestroy(ev_);
 }
 
-void StreamOrder::after_previous(hipStream_t s, bool blocking) {
+void StreamOrder::create() {
+  if (!ev_) NNCV_HIP_CHECK(hipEventCreateWithFlags(&ev_, hipEventDisableTiming));
+}
+
+void StreamOrder::after_previous(hipStream_t s) {
   if (!pending_ || tail_ == s) return;
-  if (many_) {
-    NNCV_HIP_CHECK(hipStreamWaitEvent(s, ev_, 0));
-  } else {
-    NNCV_HIP_CHECK(hipDeviceSynchronize());
-    many_ = !blocking;
-  }
+  NNCV_HIP_CHECK(hipStreamWaitEvent(s, ev_, 0));
   pending_ = false;
 }
 
-void StreamOrder::note(hipStream_t s, bool pending) {
+void StreamOrder::note(hipStream_t s, bool pending, bool covered) {
   tail_ = s;
   pending_ = pending;
-  if (!pending || !many_) return;
-  if (!ev_) NNCV_HIP_CHECK(hipEventCreateWithFlags(&ev_, hipEventDisableTiming));
-  NNCV_HIP_CHECK(hipEventRecord(ev_, s));
+  if (pending && !covered) NNCV_HIP_CHECK(hipEventRecord(ev_, s));
 }
 
 }  // namespace nncv_hip
@@ -102,11 +105,30 @@ void guarded_abort(const char* what, const std::function<void()>& fn) {
   }
 }
 
+// The launches of a call, or of its last part, complete the event of the order the call belongs to.  No two of these are
+// open at once on a thread; a call that waits for its own work, or is being captured, opens none.
+class TailScope {
+ public:
+  explicit TailScope(hipEvent_t e) : t_{e, false} {
+    if (e) tail_event() = &t_;
+  }
+  TailScope(const TailScope&) = delete;
+  TailScope& operator=(const TailScope&) = delete;
+  ~TailScope() { close(); }
+  bool close() {  // whether a launch completes the event
+    if (tail_event() == &t_) tail_event() = nullptr;
+    return t_.bound;
+  }
+
+ private:
+  TailEvent t_;
+};
+
 // NULL stream -> library stream + synchronise on exit.  Workspace (one arena), split-K tickets and the
 // pinned staging buffers are shared by every call, and the mutex only serialises the enqueueing: work
 // left pending on one caller stream must not overlap work enqueued next on another.  So a call that
-// arrives on a different stream than the previous one first makes its stream wait for everything the
-// previous stream was given (StreamOrder, runtime.hpp).  Calls that stay on one stream pay nothing.
+// arrives on a different stream than the previous one first makes its stream wait for what the
+// previous call left behind (StreamOrder, runtime.hpp).
 // A caller stream that is being captured into a HIP graph takes neither the wait nor the event: both would reach
 // outside the capture and end it.  The captured launches then run whenever the caller's graph does, and ordering
 // them against other users of the library's shared workspace is the caller's business, as for the graph itself.
@@ -123,20 +145,27 @@ struct Sync {
   hipStream_t s;
   bool own;
   bool capturing;
-  explicit Sync(void* user) : s(user ? static_cast<hipStream_t>(user) : Context::get().stream()), own(user == nullptr) {
-    capturing = !own && stream_is_capturing(s);
-    if (!capturing) Context::get().order.after_previous(s, own);
-  }
   bool done = false;
+  TailScope tail;
+  // timed: the launches are being measured, and complete nothing
+  explicit Sync(void* user, bool timed = false)
+      : s(user ? static_cast<hipStream_t>(user) : Context::get().stream()),
+        own(user == nullptr),
+        capturing(!own && stream_is_capturing(s)),
+        tail(own || capturing || timed ? nullptr : Context::get().order.event()) {
+    if (!capturing) Context::get().order.after_previous(s);
+  }
   void finish() {
+    const bool covered = tail.close();
     if (own) NNCV_HIP_CHECK(hipStreamSynchronize(s));
-    if (!capturing) Context::get().order.note(s, /*pending=*/!own);
+    if (!capturing) Context::get().order.note(s, /*pending=*/!own, covered);
     done = true;
   }
   ~Sync() {  // left early by an exception: whatever was enqueued may still be running
+    tail.close();
     if (!done && !capturing) {
       try {
-        Context::get().order.note(s, true);
+        Context::get().order.note(s, true, false);
       } catch (...) {
       }
     }
@@ -149,6 +178,7 @@ struct Sync {
 // workspace (and the K-split tickets of its layers), so a call that arrives on another stream than the handle's
 // previous one first makes its stream wait for that one, as Sync does for the library-wide arena.
 struct HandleState {
+  HandleState() { order.create(); }
   Arena arena;
   StreamOrder order;
 };
@@ -156,20 +186,27 @@ struct HandleState {
 struct HandleSync {
   HandleState& h;
   hipStream_t s;
-  bool own;
-  bool done = false;
-  HandleSync(HandleState& hs, void* user) : h(hs), s(user ? static_cast<hipStream_t>(user) : Context::get().stream()), own(user == nullptr) {
-    h.order.after_previous(s, own);
+  bool own, capturing;
+  bool done = false, covered = false;
+  HandleSync(HandleState& hs, void* user)
+      : h(hs), s(user ? static_cast<hipStream_t>(user) : Context::get().stream()), own(user == nullptr), capturing(!own && stream_is_capturing(s)) {
+    if (!capturing) h.order.after_previous(s);
+  }
+  // the last launches of the call
+  void last(const std::function<void()>& launches) {
+    TailScope tail(own || capturing ? nullptr : h.order.event());
+    launches();
+    covered = tail.close();
   }
   void finish() {
     if (own) NNCV_HIP_CHECK(hipStreamSynchronize(s));
-    h.order.note(s, /*pending=*/!own);
+    if (!capturing) h.order.note(s, /*pending=*/!own, covered);
     done = true;
   }
   ~HandleSync() {  // left early by an exception: whatever was enqueued may still be running
-    if (!done) {
+    if (!done && !capturing) {
       try {
-        h.order.note(s, true);
+        h.order.note(s, true, false);
       } catch (...) {
       }
     }
@@ -399,7 +436,8 @@ CachedModel& cached_model(const void* host, long long n, int dt, hipStream_t s) 
 // ---- HIP-graph replay of the forward pass --------------------------------------------------
 // A forward pass is 18-73 kernel launches on one stream with fixed arguments for a given (model,
 // input pointer, output pointer, shape, workspace).  The second call with the same combination captures
-// the launches into a graph and every later call replays it: one submission instead of 18-73.  That is
+// the launches but for the last into a graph and every later call replays it: one submission instead of 18-73 (the last
+// one completes the call's event, which behind a graph would cost 3.3 us more: StreamOrder, runtime.hpp).  That is
 // what batch-1 latency is made of (MobileNetV3 at batch 1: 0.308 ms against 0.323), and it is what lets
 // the host keep two passes in flight on two streams (ResNet-18 at batch 32: 0.184 ms per pass replayed
 // against 0.196 with plain launches; MobileNetV3 at batch 32: 0.269 against 0.326).  With one pass at a
@@ -438,16 +476,17 @@ void drop_graphs_of(const void* m) {
   }
 }
 
-// `run` enqueues the whole pass on `s`; `owner` identifies the handle it belongs to.
-void replay(const void* owner, const std::function<void()>& run, const void* src, int N, int H, int W, const float* logits, void* ws,
-            hipStream_t s, bool launch_bound) {
+// `body` enqueues the pass on `s` but for its last launches, which the caller enqueues after this; `owner` identifies the
+// handle it belongs to.
+void replay(const void* owner, const std::function<void()>& body, const void* src, int N, int H, int W, const float* logits, void* ws,
+            hipStream_t s, bool launch_bound, bool capturing) {
   static const int mode = [] {  // -1 by size, 0 never, 1 always (the default)
     const char* e = getenv("NNCV_HIP_GRAPH");
     return !e ? 1 : (!strcmp(e, "size") ? -1 : (atoi(e) != 0 ? 1 : 0));
   }();
   const bool use = mode == 1 || (mode == -1 && launch_bound);
-  if (!use || profiler_enabled()) {
-    run();
+  if (!use || profiler_enabled() || capturing) {  // (capturing: the caller's own graph takes the launches)
+    body();
     return;
   }
   auto& cache = graph_cache();
@@ -462,13 +501,13 @@ void replay(const void* owner, const std::function<void()>& run, const void* src
       cache.erase(cache.begin());
     }
     cache.push_back(GraphEntry{owner, src, logits, N, H, W, ws, s, nullptr, nullptr});
-    run();
+    body();
     return;
   }
   if (!hit->exec) {  // second sighting: capture
     NNCV_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
     try {
-      run();
+      body();
     } catch (...) {
       hipGraph_t g = nullptr;
       (void)hipStreamEndCapture(s, &g);
@@ -479,11 +518,6 @@ void replay(const void* owner, const std::function<void()>& run, const void* src
     NNCV_HIP_CHECK(hipGraphInstantiate(&hit->exec, hit->graph, nullptr, nullptr, 0));
   }
   NNCV_HIP_CHECK(hipGraphLaunch(hit->exec, s));
-}
-
-void forward_replay(const void* owner, const ResNet18& m, const void* src, int N, int H, int W, float* logits, void* ws, hipStream_t s) {
-  // 18 launches: launch-bound up to about two 224x224 images
-  replay(owner, [&] { m.forward(src, N, H, W, logits, ws, s); }, src, N, H, W, logits, ws, s, (long long)N * H * W <= 2ll * 224 * 224);
 }
 
 // ---- the MobileNetV3 object behind the handle-less reference ABI ----------------------------
@@ -532,7 +566,7 @@ void forward_abi(nncv_memref2d* dst, nncv_memref4d* src, void* params, int dt) {
   Context& ctx = Context::get();
   ctx.init(-1);
   hipStream_t s = ctx.stream();
-  ctx.order.after_previous(s, true);
+  ctx.order.after_previous(s);
   const size_t es = dtype_size(dt);
   const nncv_memref1d* p = static_cast<const nncv_memref1d*>(params);
   NNCV_REQUIRE(p->aligned && p->strides[0] == 1, "params must be a dense rank-1 memref");
@@ -615,7 +649,7 @@ void matmul_host(Context& ctx, nncv_memref2d* a, nncv_memref2d* b, nncv_memref2d
     total = at_c.back() + align256(rows * row_c);
   }
   at_a.push_back(total);
-  ctx.order.after_previous(s, true);
+  ctx.order.after_previous(s);
   ctx.arena.reserve(total + 1024, s);
   char* dev = static_cast<char*>(ctx.arena.take(total));
   auto f32 = [](char* p) { return reinterpret_cast<float*>(p); };
@@ -681,7 +715,7 @@ void conv_host(Context& ctx, nncv_memref4d* in, nncv_memref4d* filter, nncv_memr
   const size_t ib = align256(img_i * N), ob = align256(img_o * N);
   const size_t wt_b = align256((size_t)Fp * R * S * Cp * 4), wf_b = align256(weight_flat_bytes(kF32, Fp, R * S, Cp)), x_b = align256((size_t)N * H * W * Cp * 4), y_b = align256((size_t)N * OH * OW * Fp * 4);
   const bool staged = fb + ib + ob <= kStageMost;
-  ctx.order.after_previous(s, true);
+  ctx.order.after_previous(s);
   ctx.arena.reserve(wt_b + wf_b + x_b + y_b + (staged ? 0 : fb + ib + ob) + 2048, s);
   char* wt = static_cast<char*>(ctx.arena.take(wt_b));
   char* wf = static_cast<char*>(ctx.arena.take(wf_b));
@@ -954,7 +988,10 @@ int nncv_hip_resnet18_forward(nncv_hip_model* m, const void* src, int N, int H, 
     OverlapScope hint(m->passes);
     const size_t wsb = m->m->workspace_bytes(N, H, W);
     if (m->st.arena.reserve(wsb + 1024, sy.s)) drop_graphs_of(&m->st);  // captured against the old workspace
-    forward_replay(&m->st, *m->m, src, N, H, W, logits, m->st.arena.take(wsb), sy.s);
+    void* ws = m->st.arena.take(wsb);
+    // 18 launches: launch-bound up to about two 224x224 images
+    replay(&m->st, [&] { m->m->forward_body(src, N, H, W, ws, sy.s); }, src, N, H, W, logits, ws, sy.s, (long long)N * H * W <= 2ll * 224 * 224, sy.capturing);
+    sy.last([&] { m->m->forward_head(N, H, W, logits, ws, sy.s); });
     sy.finish();
   });
 }
@@ -993,7 +1030,7 @@ int nncv_hip_resnet18_classify_u8(nncv_hip_model* m, const void* hwc_u8, int N, 
     void* x = m->st.arena.take(in_b);
     launch_preprocess_u8(hwc_u8, x, dt, N, H, W, channels, sy.s);
     m->m->forward(x, N, H, W, logits, m->st.arena.take(wsb), sy.s);
-    launch_argmax_rows(logits, top1, N, 1000, sy.s);
+    sy.last([&] { launch_argmax_rows(logits, top1, N, 1000, sy.s); });
     sy.finish();
   });
 }
@@ -1112,7 +1149,7 @@ int nncv_hip_conv_time(nncv_hip_conv* c, const void* in, int N, int H, int W, co
   return guarded([&] {
     NNCV_REQUIRE(c && c->c && in && out && avg_us && reps > 0, "null argument");
     Context& ctx = Context::get();
-    Sync sy(stream);
+    Sync sy(stream, /*timed=*/true);
     const ConvLayer& L = *c->c;
     const size_t wsb = L.workspace_bytes(N, H, W, false);
     ctx.arena.reserve(wsb + 1024, sy.s);
@@ -1155,7 +1192,7 @@ int nncv_hip_matmul_time(const float* A, const float* B, float* C, int M, int N,
   return guarded([&] {
     NNCV_REQUIRE(A && B && C && avg_us && reps > 0, "null argument");
     Context::get().init(-1);
-    Sync sy(stream);
+    Sync sy(stream, /*timed=*/true);
     hipEvent_t e0, e1;
     NNCV_HIP_CHECK(hipEventCreate(&e0));
     NNCV_HIP_CHECK(hipEventCreate(&e1));
@@ -1304,7 +1341,8 @@ int nncv_hip_graph_forward(nncv_hip_graph* g, const void* src, int N, int H, int
     if (g->st.arena.reserve(wsb + 1024, sy.s)) drop_graphs_of(&g->st);  // captured against the old workspace
     void* ws = g->st.arena.take(wsb);
     // 49-73 launches: launch-bound up to about four 224x224 images
-    replay(&g->st, [&] { gr.forward(src, N, H, W, out, ws, sy.s); }, src, N, H, W, out, ws, sy.s, (long long)N * H * W <= 4ll * 224 * 224);
+    replay(&g->st, [&] { gr.forward_body(src, N, H, W, ws, sy.s); }, src, N, H, W, out, ws, sy.s, (long long)N * H * W <= 4ll * 224 * 224, sy.capturing);
+    sy.last([&] { gr.forward_tail(N, H, W, out, ws, sy.s); });
     sy.finish();
   });
 }

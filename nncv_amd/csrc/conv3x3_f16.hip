@@ -729,8 +729,8 @@ void launch_weight_frag32(const void* w, int w_dt, void* dst, int F, int C, hipS
   const int Fp = (F + 31) / 32 * 32;
   const long long total = (long long)(Fp / 32) * (C / 64) * 9 * 4 * 64;
   const unsigned grid = (unsigned)((total + 255) / 256);
-  if (w_dt == kF16) hipLaunchKernelGGL((weight_frag32_kernel<half_t>), dim3(grid), dim3(256), 0, s, (const half_t*)w, (half_t*)dst, F, C, Fp);
-  else hipLaunchKernelGGL((weight_frag32_kernel<float>), dim3(grid), dim3(256), 0, s, (const float*)w, (half_t*)dst, F, C, Fp);
+  if (w_dt == kF16) launch_kernel((weight_frag32_kernel<half_t>), dim3(grid), dim3(256), 0, s, (const half_t*)w, (half_t*)dst, F, C, Fp);
+  else launch_kernel((weight_frag32_kernel<float>), dim3(grid), dim3(256), 0, s, (const float*)w, (half_t*)dst, F, C, Fp);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 
@@ -783,7 +783,7 @@ static void launch_stream_cfg(const StreamArgs& a, int grid, double flops, doubl
   }();
   (void)attr;
   ProfScope prof(tag, flops, bytes, s);
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * NW), smem, s, a.in, a.wf, a.G, a.div, a.mdiv, a.mS32, a.n_tiles, a.tstep_nslab_flags, a.N_TH, a.geom,
+  launch_kernel(kern, dim3(grid), dim3(64 * NW), smem, s, a.in, a.wf, a.G, a.div, a.mdiv, a.mS32, a.n_tiles, a.tstep_nslab_flags, a.N_TH, a.geom,
                      a.pixB, a.rowx_rnseg, a.t);
 }
 

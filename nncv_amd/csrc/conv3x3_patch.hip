@@ -870,7 +870,7 @@ static void launch_patch_cfg(const PatchArgs& a, double flops, double bytes, con
   const int fblocks = b.aux_fb0 + (b.aux_inline ? 0 : (a.aux_F + 32 * NI - 1) / (32 * NI));
   if (b.xcd_by_filter && fblocks % kXcdsP != 0) b.xcd_by_filter = 0;
   dim3 grid((a.tiles + kXcdsP - 1) / kXcdsP * kXcdsP, fblocks, SK ? a.ksplit : 1);
-  hipLaunchKernelGGL(kern, grid, dim3(Cfg::NT), Cfg::smem, s, b.in, b.tiles, b.tiles_y, b.TN, b.TH, b.N, b.H, b.W, b.C, b.rw_log,
+  launch_kernel(kern, grid, dim3(Cfg::NT), Cfg::smem, s, b.in, b.tiles, b.tiles_y, b.TN, b.TH, b.N, b.H, b.W, b.C, b.rw_log,
                      b.xcd_by_filter, b.in_bytes, b.txw, b);
 }
 

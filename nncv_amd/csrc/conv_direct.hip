@@ -326,7 +326,7 @@ void launch_cfg(DirectArgs d, int batch, hipStream_t s) {
       return true;
     }();
     (void)attr;
-    hipLaunchKernelGGL(kern, dim3((unsigned)((long long)d.tiles_f * d.tiles_p), (unsigned)batch), dim3(64 * KG), lds, s, d);
+    launch_kernel(kern, dim3((unsigned)((long long)d.tiles_f * d.tiles_p), (unsigned)batch), dim3(64 * KG), lds, s, d);
   };
   if (d.cpt % 8 == 0) go(conv_direct_kernel<T, OutT, BT, TM, TN, KG, true>);
   else go(conv_direct_kernel<T, OutT, BT, TM, TN, KG, false>);
@@ -450,10 +450,10 @@ void launch_weight_flat(const void* w_fcrs, void* dst, int dt, int F, int C, int
   const size_t lds = staged ? (size_t)cc * RS * es : 0;
   const dim3 grid((unsigned)((F + 31) / 32 * 32));
   if (dt == kF16)
-    hipLaunchKernelGGL((weight_flat_kernel<half_t>), grid, dim3(256), lds, s, static_cast<const half_t*>(w_fcrs), static_cast<half_t*>(dst), F, C, RS,
+    launch_kernel((weight_flat_kernel<half_t>), grid, dim3(256), lds, s, static_cast<const half_t*>(w_fcrs), static_cast<half_t*>(dst), F, C, RS,
                        Cp, units, cc, staged);
   else
-    hipLaunchKernelGGL((weight_flat_kernel<float>), grid, dim3(256), lds, s, static_cast<const float*>(w_fcrs), static_cast<float*>(dst), F, C, RS, Cp,
+    launch_kernel((weight_flat_kernel<float>), grid, dim3(256), lds, s, static_cast<const float*>(w_fcrs), static_cast<float*>(dst), F, C, RS, Cp,
                        units, cc, staged);
   NNCV_HIP_CHECK(hipGetLastError());
 }

@@ -173,10 +173,10 @@ static void launch_pairs_cfg(const IgemmArgs& a, const char* tag, hipStream_t s)
   // fewer four-wave workgroups than CUs: one wave per workgroup instead
   const bool small = (P + 255) / 256 * gy < 256;
   const dim3 grid(small ? (unsigned)((P + 63) / 64) : (unsigned)((P + 255) / 256), gy), block(small ? 64 : 256);
-  if (a.residual && small) hipLaunchKernelGGL((conv_pairs_kernel<KST, NI, 1, true>), grid, block, 0, s, a);
-  else if (a.residual) hipLaunchKernelGGL((conv_pairs_kernel<KST, NI, 4, true>), grid, block, 0, s, a);
-  else if (small) hipLaunchKernelGGL((conv_pairs_kernel<KST, NI, 1, false>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((conv_pairs_kernel<KST, NI, 4, false>), grid, block, 0, s, a);
+  if (a.residual && small) launch_kernel((conv_pairs_kernel<KST, NI, 1, true>), grid, block, 0, s, a);
+  else if (a.residual) launch_kernel((conv_pairs_kernel<KST, NI, 4, true>), grid, block, 0, s, a);
+  else if (small) launch_kernel((conv_pairs_kernel<KST, NI, 1, false>), grid, block, 0, s, a);
+  else launch_kernel((conv_pairs_kernel<KST, NI, 4, false>), grid, block, 0, s, a);
 }
 
 void launch_conv_pairs(const IgemmArgs& a, hipStream_t s) {
@@ -323,8 +323,8 @@ static void launch_image_cfg(ImagePairsArgs a, const char* tag, hipStream_t s) {
   const double px = (double)a.N * a.OH * a.OW;
   ProfScope prof(tag, a.alg_flops, 2.0 * ((double)a.N * a.C * a.H * a.W + (double)a.F * a.R * a.S * 8 + px * a.F), s);
   const dim3 grid((unsigned)((a.N * a.tiles_y * a.tiles_x + 7) / 8 * 8));
-  if (small) hipLaunchKernelGGL((image_pairs_kernel<R, S, NI, 1>), grid, dim3(64), 0, s, a);
-  else hipLaunchKernelGGL((image_pairs_kernel<R, S, NI, 4>), grid, dim3(256), 0, s, a);
+  if (small) launch_kernel((image_pairs_kernel<R, S, NI, 1>), grid, dim3(64), 0, s, a);
+  else launch_kernel((image_pairs_kernel<R, S, NI, 4>), grid, dim3(256), 0, s, a);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 

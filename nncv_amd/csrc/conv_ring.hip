@@ -306,7 +306,7 @@ void launch_cfg(RingArgs d, int mode, hipStream_t s) {
       return true;
     }();
     (void)attr;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(d.aux_f0 ? (d.tiles_p + 7) / 8 * 8 * (d.tiles_f + d.aux_tiles) : d.tiles_f * d.tiles_p)), dim3(64 * NW), lds, s, d);
+    launch_kernel(kern, dim3((unsigned)(d.aux_f0 ? (d.tiles_p + 7) / 8 * 8 * (d.tiles_f + d.aux_tiles) : d.tiles_f * d.tiles_p)), dim3(64 * NW), lds, s, d);
   };
   if (mode == kPoint) go(conv_ring_kernel<WP, WF, PB, FB, S, kPoint>);
   else if (mode == kLines) go(conv_ring_kernel<WP, WF, PB, FB, S, kLines>);

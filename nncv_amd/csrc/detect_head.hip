@@ -148,8 +148,8 @@ void launch_detect_head(const DetectHeadArgs& a_in, hipStream_t s) {
   NNCV_REQUIRE(blocks < (1 << 24), "detect_head: too many boxes");
   constexpr int lds = kStageH;  // (at least kPix * kFil floats)
   ProfScope prof("detect_head", flops, bytes, s);
-  if (vec) hipLaunchKernelGGL(detect_head_kernel<true>, dim3((unsigned)blocks), dim3(512), lds, s, a);
-  else hipLaunchKernelGGL(detect_head_kernel<false>, dim3((unsigned)blocks), dim3(512), lds, s, a);
+  if (vec) launch_kernel(detect_head_kernel<true>, dim3((unsigned)blocks), dim3(512), lds, s, a);
+  else launch_kernel(detect_head_kernel<false>, dim3((unsigned)blocks), dim3(512), lds, s, a);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 

@@ -123,7 +123,7 @@ static void launch_dwconv_oxt(const DwConvArgs& a, hipStream_t s) {
   const long long work = (long long)a.N * a.OH * strips * (a.C / V16<T>::n);
   const long long grid = (work + 127) / 128;
   NNCV_REQUIRE(grid >= 1 && grid < (1ll << 31), "dwconv: grid out of range");
-  hipLaunchKernelGGL((dwconv_kernel<T, K, S, OXT>), dim3((unsigned)grid), dim3(128), 0, s, a, strips);
+  launch_kernel((dwconv_kernel<T, K, S, OXT>), dim3((unsigned)grid), dim3(128), 0, s, a, strips);
 }
 
 // A lane-FMA is all the arithmetic there is (a wave retires one per 4 cycles), so the launch is as
@@ -176,7 +176,7 @@ __global__ void weight_dw_kernel(const Ts* __restrict__ w, Td* __restrict__ dst,
 void launch_weight_dw(const void* w, int w_dt, void* dst, int dst_dt, int C, int K, hipStream_t s) {
   const int n = C * K * K;
   const unsigned grid = grid_for(n);
-#define LAUNCH(TS, TD) hipLaunchKernelGGL((weight_dw_kernel<TS, TD>), dim3(grid), dim3(256), 0, s, (const TS*)w, (TD*)dst, C, K * K)
+#define LAUNCH(TS, TD) launch_kernel((weight_dw_kernel<TS, TD>), dim3(grid), dim3(256), 0, s, (const TS*)w, (TD*)dst, C, K * K)
   if (w_dt == kF32 && dst_dt == kF32) LAUNCH(float, float);
   else if (w_dt == kF16 && dst_dt == kF16) LAUNCH(half_t, half_t);
   else if (w_dt == kF32 && dst_dt == kF16) LAUNCH(float, half_t);
@@ -214,10 +214,10 @@ void launch_scale_channels(const void* x, const void* g, void* out, int dt, int 
   if (total == 0) return;
   ProfScope prof("scale_channels", (double)total * vn, (double)dtype_size(dt) * (2.0 * total * vn + (double)N * C), s);
   if (dt == kF16)
-    hipLaunchKernelGGL((scale_channels_kernel<half_t>), dim3(grid_for(total)), dim3(256), 0, s, (const half_t*)x, (const half_t*)g,
+    launch_kernel((scale_channels_kernel<half_t>), dim3(grid_for(total)), dim3(256), 0, s, (const half_t*)x, (const half_t*)g,
                        (half_t*)out, total, HW * CG, CG);
   else
-    hipLaunchKernelGGL((scale_channels_kernel<float>), dim3(grid_for(total)), dim3(256), 0, s, (const float*)x, (const float*)g,
+    launch_kernel((scale_channels_kernel<float>), dim3(grid_for(total)), dim3(256), 0, s, (const float*)x, (const float*)g,
                        (float*)out, total, HW * CG, CG);
   NNCV_HIP_CHECK(hipGetLastError());
 }
@@ -371,9 +371,9 @@ void launch_se_block(const SeArgs& a, int dt, hipStream_t s) {
   const double es = (double)dtype_size(dt);
   ProfScope prof("se_block", 4.0 * a.N * a.C * a.SQ + 2.0 * a.N * a.HW * a.C, es * (2.0 * a.N * a.HW * a.C + 2.0 * a.C * a.SQ), s);
   if (dt == kF16)
-    hipLaunchKernelGGL((se_block_kernel<half_t>), dim3(a.N), dim3(kSeThreads), 0, s, a);
+    launch_kernel((se_block_kernel<half_t>), dim3(a.N), dim3(kSeThreads), 0, s, a);
   else
-    hipLaunchKernelGGL((se_block_kernel<float>), dim3(a.N), dim3(kSeThreads), 0, s, a);
+    launch_kernel((se_block_kernel<float>), dim3(a.N), dim3(kSeThreads), 0, s, a);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 
@@ -416,10 +416,10 @@ void launch_eltwise_pitched(const void* a, int lda, const void* b, int ldb, void
   if (n == 0) return;
   ProfScope prof(b ? "eltwise_add" : "eltwise_act", (double)n, (double)dtype_size(dt) * n * (b ? 3 : 2), s);
   if (dt == kF16)
-    hipLaunchKernelGGL((eltwise_kernel<half_t>), dim3(grid_for(n / vn)), dim3(256), 0, s, (const half_t*)a, (const half_t*)b,
+    launch_kernel((eltwise_kernel<half_t>), dim3(grid_for(n / vn)), dim3(256), 0, s, (const half_t*)a, (const half_t*)b,
                        (half_t*)out, n / vn, C / vn, lda, ldb, ldo, act);
   else
-    hipLaunchKernelGGL((eltwise_kernel<float>), dim3(grid_for(n / vn)), dim3(256), 0, s, (const float*)a, (const float*)b,
+    launch_kernel((eltwise_kernel<float>), dim3(grid_for(n / vn)), dim3(256), 0, s, (const float*)a, (const float*)b,
                        (float*)out, n / vn, C / vn, lda, ldb, ldo, act);
   NNCV_HIP_CHECK(hipGetLastError());
 }
@@ -451,7 +451,7 @@ void launch_concat_slice(const void* x, void* out, int dt, long long P, int C, i
   const long long total = P * (C / vn);
   if (total == 0) return;
   ProfScope prof("concat_slice", 0.0, 2.0 * dtype_size(dt) * P * C, s);
-  hipLaunchKernelGGL(concat_slice_kernel, dim3(grid_for(total)), dim3(256), 0, s, (const uint4*)x, (uint4*)out, total, C / vn,
+  launch_kernel(concat_slice_kernel, dim3(grid_for(total)), dim3(256), 0, s, (const uint4*)x, (uint4*)out, total, C / vn,
                      ldi / vn, ldo / vn, c0 / vn);
   NNCV_HIP_CHECK(hipGetLastError());
 }
@@ -477,7 +477,7 @@ void launch_upsample2x(const void* x, void* out, int dt, int N, int H, int W, in
   const long long total = (long long)N * 4 * H * W * (C / vn);
   if (total == 0) return;
   ProfScope prof("upsample2x", 0.0, 5.0 * dtype_size(dt) * N * H * W * C, s);
-  hipLaunchKernelGGL(upsample2x_kernel, dim3(grid_for(total)), dim3(256), 0, s, (const uint4*)x, (uint4*)out, total, H, W, C / vn,
+  launch_kernel(upsample2x_kernel, dim3(grid_for(total)), dim3(256), 0, s, (const uint4*)x, (uint4*)out, total, H, W, C / vn,
                      ldi / vn, ldo / vn, c0 / vn);
   NNCV_HIP_CHECK(hipGetLastError());
 }
@@ -533,10 +533,10 @@ void launch_maxpool_nhwc(const void* in, void* out, int dt, int N, int H, int W,
   if (work == 0) return;
   ProfScope prof("maxpool", 0.0, (double)dtype_size(dt) * N * C * ((double)H * W + (double)OH * OW), s);
   if (dt == kF16)
-    hipLaunchKernelGGL((maxpool_kernel<half_t>), dim3(grid_for(work)), dim3(256), 0, s, (const half_t*)in, (half_t*)out, N, H, W, C,
+    launch_kernel((maxpool_kernel<half_t>), dim3(grid_for(work)), dim3(256), 0, s, (const half_t*)in, (half_t*)out, N, H, W, C,
                        K, stride, pad, OH, OW, ldi, ldo);
   else
-    hipLaunchKernelGGL((maxpool_kernel<float>), dim3(grid_for(work)), dim3(256), 0, s, (const float*)in, (float*)out, N, H, W, C, K,
+    launch_kernel((maxpool_kernel<float>), dim3(grid_for(work)), dim3(256), 0, s, (const float*)in, (float*)out, N, H, W, C, K,
                        stride, pad, OH, OW, ldi, ldo);
   NNCV_HIP_CHECK(hipGetLastError());
 }
@@ -636,10 +636,10 @@ void launch_maxpool5_chain3(const void* in, void* o1, void* o2, void* o3, int dt
   (void)once;
   const size_t smem = (size_t)3 * H * W * 16;
   if (dt == kF16)
-    hipLaunchKernelGGL((maxpool5_chain3_kernel<half_t>), grid, dim3(256), smem, s, (const half_t*)in, (half_t*)o1, (half_t*)o2, (half_t*)o3,
+    launch_kernel((maxpool5_chain3_kernel<half_t>), grid, dim3(256), smem, s, (const half_t*)in, (half_t*)o1, (half_t*)o2, (half_t*)o3,
                        H, W, C / vn, ldi, ld1, ld2, ld3);
   else
-    hipLaunchKernelGGL((maxpool5_chain3_kernel<float>), grid, dim3(256), smem, s, (const float*)in, (float*)o1, (float*)o2, (float*)o3, H, W,
+    launch_kernel((maxpool5_chain3_kernel<float>), grid, dim3(256), smem, s, (const float*)in, (float*)o1, (float*)o2, (float*)o3, H, W,
                        C / vn, ldi, ld1, ld2, ld3);
   NNCV_HIP_CHECK(hipGetLastError());
 }
@@ -741,17 +741,17 @@ void launch_yolo_detect(const DetectArgs& a, int dt, hipStream_t s) {
   if (vec4) {
     dim3 grid4((unsigned)((hwf / 4 + 255) / 256), (unsigned)(a.N * a.A));
     if (dt == kF16)
-      hipLaunchKernelGGL((yolo_detect4_kernel<half_t>), grid4, dim3(256), 0, s, b);
+      launch_kernel((yolo_detect4_kernel<half_t>), grid4, dim3(256), 0, s, b);
     else
-      hipLaunchKernelGGL((yolo_detect4_kernel<float>), grid4, dim3(256), 0, s, b);
+      launch_kernel((yolo_detect4_kernel<float>), grid4, dim3(256), 0, s, b);
     NNCV_HIP_CHECK(hipGetLastError());
     return;
   }
   dim3 grid((unsigned)(((long long)a.H * a.W * a.F + 255) / 256), (unsigned)(a.N * a.A));
   if (dt == kF16)
-    hipLaunchKernelGGL((yolo_detect_kernel<half_t>), grid, dim3(256), 0, s, b);
+    launch_kernel((yolo_detect_kernel<half_t>), grid, dim3(256), 0, s, b);
   else
-    hipLaunchKernelGGL((yolo_detect_kernel<float>), grid, dim3(256), 0, s, b);
+    launch_kernel((yolo_detect_kernel<float>), grid, dim3(256), 0, s, b);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 

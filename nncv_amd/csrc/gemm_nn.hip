@@ -338,7 +338,7 @@ void launch_gemm_cfg(const float* A, const float* B, const float* C, float* D, i
   (void)attr;
   const long long tm = (M + Cfg::kRows - 1) / Cfg::kRows, tn = (N + Cfg::kCols - 1) / Cfg::kCols;
   NNCV_REQUIRE(tm * tn < (1ll << 31), "matmul: too many tiles");
-  hipLaunchKernelGGL(kern, dim3((unsigned)(tm * tn + ride.blocks)), dim3(64 * Cfg::kWaves), Cfg::kLds, s, A, B, C, D, M, N, K, (int)tm, (int)tn, ride);
+  launch_kernel(kern, dim3((unsigned)(tm * tn + ride.blocks)), dim3(64 * Cfg::kWaves), Cfg::kLds, s, A, B, C, D, M, N, K, (int)tm, (int)tn, ride);
 }
 
 }  // namespace
@@ -372,7 +372,7 @@ const GemmForm kForms[] = {
 
 void launch_copy16(const RideCopy& r, hipStream_t s) {
   if (r.bytes == 0) return;
-  hipLaunchKernelGGL(copy16_kernel, dim3((unsigned)r.blocks), dim3(256), 0, s, r);
+  launch_kernel(copy16_kernel, dim3((unsigned)r.blocks), dim3(256), 0, s, r);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 
@@ -390,7 +390,7 @@ void launch_gemm_nn_f32(const float* A, const float* B, const float* C, float* D
   }
   if (N >= 1 << 24 || K >= 1 << 24) {  // 64 rows of A or 32 of B beyond 32-bit byte offsets
     const long long blocks = ((long long)M * N + 255) / 256;
-    hipLaunchKernelGGL(gemm_nn_f32_any_kernel, dim3((unsigned)std::min(blocks, 1ll << 20)), dim3(256), 0, s, A, B, C, D, M, N, K);
+    launch_kernel(gemm_nn_f32_any_kernel, dim3((unsigned)std::min(blocks, 1ll << 20)), dim3(256), 0, s, A, B, C, D, M, N, K);
     NNCV_HIP_CHECK(hipGetLastError());
     return;
   }

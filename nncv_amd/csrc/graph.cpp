@@ -228,10 +228,10 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
         }
         const unsigned grid = (unsigned)((F + 255) / 256);
         if (dt == kF16)
-          hipLaunchKernelGGL((fold_bias_kernel<half_t>), dim3(grid), dim3(256), 0, s, (const half_t*)b, nd.scale.as<float>(),
+          launch_kernel((fold_bias_kernel<half_t>), dim3(grid), dim3(256), 0, s, (const half_t*)b, nd.scale.as<float>(),
                              nd.shift.as<float>(), had ? 1 : 0, F);
         else
-          hipLaunchKernelGGL((fold_bias_kernel<float>), dim3(grid), dim3(256), 0, s, (const float*)b, nd.scale.as<float>(),
+          launch_kernel((fold_bias_kernel<float>), dim3(grid), dim3(256), 0, s, (const float*)b, nd.scale.as<float>(),
                              nd.shift.as<float>(), had ? 1 : 0, F);
         NNCV_HIP_CHECK(hipGetLastError());
       }
@@ -750,7 +750,7 @@ void Graph::output_shape(int H, int W, int* C, int* OH, int* OW) const {
 
 size_t Graph::workspace_bytes(int N, int H, int W) const { return plan_of(N, H, W).total; }
 
-void Graph::forward(const void* src, int N, int H, int W, float* out, void* ws, hipStream_t s) const {
+void Graph::forward_body(const void* src, int N, int H, int W, void* ws, hipStream_t s) const {
   const Plan& p = plan_of(N, H, W);
   char* base = static_cast<char*>(ws);
   auto at = [&](int t) -> void* { return base + p.offset[t]; };
@@ -907,44 +907,50 @@ void Graph::forward(const void* src, int N, int H, int W, float* out, void* ws, 
       case NNCV_HIP_OP_UPSAMPLE2X:
         launch_upsample2x(at(op.in[0]), at(op.out), dt_, N, a.H, a.W, a.C, pitch(op.out), 0, s, pitch(op.in[0]));
         break;
-      case NNCV_HIP_OP_YOLO_DETECT: {
-        long long box0 = 0;
-        if (p.head) {
-          DetectHeadArgs d{};
-          d.out = out; d.N = N; d.A = op.K; d.F = op.F; d.boxes_total = o.C;
-          while (d.levels < 3 && op.in[d.levels] >= 0) ++d.levels;
-          for (int k = 0; k < d.levels; ++k) {
-            const Node& c = *maker(op.in[k]);
-            const int t = c.op.in[0];
-            const Dims h = p.dims[t];
-            DetectHeadLevel& v = d.lv[d.levels - 1 - k];  // (the later levels are the ones with more channels)
-            v.in = at(t); v.wt = c.wt.get(); v.scale = c.scale.as<float>(); v.shift = c.shift.as<float>();
-            v.HW = h.H * h.W; v.W = h.W; v.pix = pitch(t); v.C = h.C; v.rows = channels_[c.op.out]; v.box0 = box0; v.stride = detect_stride_[k];
-            for (int q = 0; q < op.K * 2; ++q) v.anchor_wh[q] = detect_anchor_wh_[k * op.K * 2 + q];
-            box0 += (long long)op.K * h.H * h.W;
-          }
-          launch_detect_head(d, s);
-          break;
-        }
-        for (int k = 0; k < 3 && op.in[k] >= 0; ++k) {
-          const Dims h = p.dims[op.in[k]];
-          DetectArgs d{};
-          d.head = at(op.in[k]); d.out = out; d.N = N; d.H = h.H; d.W = h.W; d.A = op.K; d.F = op.F; d.ldc = pitch(op.in[k]);
-          d.box0 = box0; d.boxes_total = o.C; d.stride = detect_stride_[k];
-          for (int q = 0; q < op.K * 2; ++q) d.anchor_wh[q] = detect_anchor_wh_[k * op.K * 2 + q];
-          launch_yolo_detect(d, dt_, s);
-          box0 += (long long)op.K * h.H * h.W;
-        }
-        break;
-      }
+      case NNCV_HIP_OP_YOLO_DETECT: break;  // the last operator: forward_tail
       default: fail("graph: unknown operator kind");
     }
   }
-  if (nodes_.back().op.kind == NNCV_HIP_OP_YOLO_DETECT) return;  // already in the caller's buffer, fp32
-  const int t = nodes_.back().op.out;
-  const Dims d = p.dims[t];
-  const int Cl = logical_[t];
-  launch_relayout(at(t), dt_, strides_of(kNHWC, d.C, d.H, d.W), out, kF32, strides_of(kNCHW, Cl, d.H, d.W), N, Cl, Cl, d.H, d.W,
+}
+
+void Graph::forward_tail(int N, int H, int W, float* out, void* ws, hipStream_t s) const {
+  const Plan& p = plan_of(N, H, W);
+  char* base = static_cast<char*>(ws);
+  auto at = [&](int t) -> void* { return base + p.offset[t]; };
+  const GraphOp& op = nodes_.back().op;
+  const Dims o = p.dims[op.out];
+  if (op.kind == NNCV_HIP_OP_YOLO_DETECT) {  // decoded straight into the caller's buffer, fp32
+    long long box0 = 0;
+    if (p.head) {
+      DetectHeadArgs d{};
+      d.out = out; d.N = N; d.A = op.K; d.F = op.F; d.boxes_total = o.C;
+      while (d.levels < 3 && op.in[d.levels] >= 0) ++d.levels;
+      for (int k = 0; k < d.levels; ++k) {
+        const Node& c = *maker(op.in[k]);
+        const int t = c.op.in[0];
+        const Dims h = p.dims[t];
+        DetectHeadLevel& v = d.lv[d.levels - 1 - k];  // (the later levels are the ones with more channels)
+        v.in = at(t); v.wt = c.wt.get(); v.scale = c.scale.as<float>(); v.shift = c.shift.as<float>();
+        v.HW = h.H * h.W; v.W = h.W; v.pix = pitch(t); v.C = h.C; v.rows = channels_[c.op.out]; v.box0 = box0; v.stride = detect_stride_[k];
+        for (int q = 0; q < op.K * 2; ++q) v.anchor_wh[q] = detect_anchor_wh_[k * op.K * 2 + q];
+        box0 += (long long)op.K * h.H * h.W;
+      }
+      launch_detect_head(d, s);
+      return;
+    }
+    for (int k = 0; k < 3 && op.in[k] >= 0; ++k) {
+      const Dims h = p.dims[op.in[k]];
+      DetectArgs d{};
+      d.head = at(op.in[k]); d.out = out; d.N = N; d.H = h.H; d.W = h.W; d.A = op.K; d.F = op.F; d.ldc = pitch(op.in[k]);
+      d.box0 = box0; d.boxes_total = o.C; d.stride = detect_stride_[k];
+      for (int q = 0; q < op.K * 2; ++q) d.anchor_wh[q] = detect_anchor_wh_[k * op.K * 2 + q];
+      launch_yolo_detect(d, dt_, s);
+      box0 += (long long)op.K * h.H * h.W;
+    }
+    return;
+  }
+  const int Cl = logical_[op.out];
+  launch_relayout(at(op.out), dt_, strides_of(kNHWC, o.C, o.H, o.W), out, kF32, strides_of(kNCHW, Cl, o.H, o.W), N, Cl, Cl, o.H, o.W,
                   false, s);
 }
 

@@ -37,7 +37,13 @@ class Graph {
   // or writes no workspace tensor.  Returns the workspace size.  Host arithmetic only.
   size_t describe_plan(int N, int H, int W, long long* tensor_info, int* launch_dst) const;
   // src: NCHW [N,in_channels,H,W] of type dt; out: NCHW fp32 of the output shape (both device)
-  void forward(const void* src, int N, int H, int W, float* out, void* ws, hipStream_t s) const;
+  void forward(const void* src, int N, int H, int W, float* out, void* ws, hipStream_t s) const {
+    forward_body(src, N, H, W, ws, s);
+    forward_tail(N, H, W, out, ws, s);
+  }
+  // the pass but for the launches that write `out`, and those
+  void forward_body(const void* src, int N, int H, int W, void* ws, hipStream_t s) const;
+  void forward_tail(int N, int H, int W, float* out, void* ws, hipStream_t s) const;
 
  private:
   struct Node {

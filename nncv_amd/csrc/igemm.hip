@@ -239,7 +239,7 @@ static void launch_cfg(const IgemmArgs& a, hipStream_t s) {
                        sizeof(OutT) * (double)P * a.F * a.batch * (a.residual ? 2 : 1);
   ProfScope prof(tag.c_str(), flops, bytes, s);
   dim3 grid((P + BP - 1) / BP, (a.F + BF - 1) / BF, a.batch);
-  hipLaunchKernelGGL((igemm_kernel<T, OutT, BP, BF, WP, WF>), grid, dim3(kThreads), 0, s, a);
+  launch_kernel((igemm_kernel<T, OutT, BP, BF, WP, WF>), grid, dim3(kThreads), 0, s, a);
 }
 
 template <typename T, typename OutT>

@@ -251,7 +251,7 @@ void launch_fast_cfg(const IgemmArgs& a, hipStream_t s) {
   ProfScope prof(tag.c_str(), flops, bytes, s);
   const int tiles_x = (P + BP - 1) / BP;
   dim3 grid((tiles_x + kXcds - 1) / kXcds * kXcds, (a.F + BFE - 1) / BFE, a.batch);
-  hipLaunchKernelGGL(kern, grid, dim3(64 * WP * WF * WK), smem, s, a, tiles_x, 1.0f / (float)(a.OH * a.OW), 1.0f / (float)a.OW);
+  launch_kernel(kern, grid, dim3(64 * WP * WF * WK), smem, s, a, tiles_x, 1.0f / (float)(a.OH * a.OW), 1.0f / (float)a.OW);
 }
 
 template <typename T, typename OutT>

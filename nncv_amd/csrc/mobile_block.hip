@@ -443,7 +443,7 @@ void launch_dw_block(const DwBlockArgs& args, hipStream_t s) {
       return true;
     }();
     (void)attr;
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(kDwThreads), lds, s, a);
+    launch_kernel(kern, dim3(grid), dim3(kDwThreads), lds, s, a);
   };
   auto steps = [&](auto k, auto st, auto ox) {
     constexpr int K = decltype(k)::value, S = decltype(st)::value, OXT = decltype(ox)::value;
@@ -477,7 +477,7 @@ __global__ __launch_bounds__(256) void transpose_half_kernel(const half_t* __res
 }  // namespace
 
 void launch_transpose_half(const void* w, void* dst, int rows, int cols, hipStream_t s) {
-  hipLaunchKernelGGL(transpose_half_kernel, dim3((unsigned)((rows * cols + 255) / 256)), dim3(256), 0, s, static_cast<const half_t*>(w),
+  launch_kernel(transpose_half_kernel, dim3((unsigned)((rows * cols + 255) / 256)), dim3(256), 0, s, static_cast<const half_t*>(w),
                      static_cast<half_t*>(dst), rows, cols);
   NNCV_HIP_CHECK(hipGetLastError());
 }
@@ -509,7 +509,7 @@ void launch_se_project(const SeProjectArgs& args, hipStream_t s) {
       return true;
     }();
     (void)attr;
-    hipLaunchKernelGGL(kern, grid, dim3(kSpThreads), lds, s, a);
+    launch_kernel(kern, grid, dim3(kSpThreads), lds, s, a);
   };
   auto filters = [&](auto nsc, auto ptc, auto kc) {
     const int ft = (a.F + 15) / 16;

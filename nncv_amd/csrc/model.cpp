@@ -312,7 +312,7 @@ namespace {
 // convolution, 1 max-pool, then per BasicBlock k: 2+3k conv1, 3+3k shortcut conv, 4+3k conv2,
 // 26 average pool, 27 FC.
 struct Plan {
-  int h1, w1, h2, w2;            // after stem, after maxpool
+  int h1, w1, h2, w2, h_out, w_out;  // after stem, after maxpool, after the body
   size_t stem_out, pooled, cws;  // offsets
   size_t x[9];                   // x[k] = input of block k; x[8] = network body output
   size_t y1[8], idn[8];
@@ -349,6 +349,7 @@ static Plan make_plan(const ConvLayer& stem, const std::vector<const ConvLayer*>
     ix[k + 1] = add(o + 2, o + 3, 0);
     h = oh; w = ow; ch = f;
   }
+  p.h_out = h; p.w_out = w;
   t[ix[nb]].bytes = (size_t)N * h * w * ch * es;
   t[ix[nb]].last_op = 26;
   const int i_pooled = add(26, 27, (size_t)N * 512 * es);
@@ -371,13 +372,11 @@ static Plan plan_of(const ConvLayer& stem, const std::vector<ResNet18::Block>& b
 
 size_t ResNet18::workspace_bytes(int N, int H, int W) const { return plan_of(*stem_, blocks_, dt_, N, H, W).total; }
 
-void ResNet18::forward(const void* src, int N, int H, int W, void* logits, void* ws, hipStream_t s, int tap_stage,
-                       void* tap) const {
+void ResNet18::forward_body(const void* src, int N, int H, int W, void* ws, hipStream_t s, int tap_stage, void* tap) const {
   NNCV_REQUIRE(N > 0 && H >= 32 && W >= 32, "ResNet-18: input must be at least 32x32");
   const Plan p = plan_of(*stem_, blocks_, dt_, N, H, W);
   char* base = static_cast<char*>(ws);
   char* stem_out = base + p.stem_out;
-  char* pooled = base + p.pooled;
   char* cws = base + p.cws;
   char* x0 = base + p.x[0];
 
@@ -414,7 +413,13 @@ void ResNet18::forward(const void* src, int N, int H, int W, void* logits, void*
     if (nblk % 2 == 0 && tap_stage == nblk / 2)
       NNCV_HIP_CHECK(hipMemcpyAsync(tap, y2, (size_t)N * h * w * ch * es, hipMemcpyDeviceToDevice, s));
   }
-  char* body_out = base + p.x[8];
+}
+
+void ResNet18::forward_head(int N, int H, int W, void* logits, void* ws, hipStream_t s) const {
+  const Plan p = plan_of(*stem_, blocks_, dt_, N, H, W);
+  char* body_out = static_cast<char*>(ws) + p.x[8];
+  char* pooled = static_cast<char*>(ws) + p.pooled;
+  const int h = p.h_out, w = p.w_out;
   // head: global average pool (sum, one divide), FC with bias (Res18.mlir:609-628)
   static const bool never_fused = getenv("NNCV_HIP_NO_HEAD_FUSION") != nullptr;
   // see overlap_hint (arena_plan.hpp); at small batches the fused head is a few dozen workgroups and one launch less

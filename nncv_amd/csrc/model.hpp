@@ -81,7 +81,13 @@ class ResNet18 {
   // tap_stage >= 0 also copies the NHWC activation after that stage to `tap`
   // (0: after the max-pool, 1..4: after layer1..layer4).
   void forward(const void* src, int N, int H, int W, void* logits, void* ws, hipStream_t s, int tap_stage = -1,
-               void* tap = nullptr) const;
+               void* tap = nullptr) const {
+    forward_body(src, N, H, W, ws, s, tap_stage, tap);
+    forward_head(N, H, W, logits, ws, s);
+  }
+  // the pass up to the last activation (left in `ws`), and average pool and FC from there
+  void forward_body(const void* src, int N, int H, int W, void* ws, hipStream_t s, int tap_stage = -1, void* tap = nullptr) const;
+  void forward_head(int N, int H, int W, void* logits, void* ws, hipStream_t s) const;
 
   struct Block {
     std::unique_ptr<ConvLayer> c1, c2, ds;

@@ -44,7 +44,7 @@ void* noalloc_scratch() {
 
 // A fill kernel, not hipMemsetAsync: a caller may be capturing the stream into a graph.
 void launch_clear_words(void* p, int n_words, hipStream_t s) {
-  hipLaunchKernelGGL(clear_words_kernel, dim3((n_words + 255) / 256), dim3(256), 0, s, static_cast<unsigned*>(p), n_words);
+  launch_kernel(clear_words_kernel, dim3((n_words + 255) / 256), dim3(256), 0, s, static_cast<unsigned*>(p), n_words);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 

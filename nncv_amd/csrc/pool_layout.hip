@@ -190,18 +190,18 @@ void launch_maxpool3x3s2_nhwc(const void* in, void* out, int dt, int N, int H, i
     const unsigned inv_cg = C / vn == 1 ? 0u : (unsigned)(0xffffffffull / (unsigned)(C / vn) + 1);
     const unsigned grid_rows = ((unsigned)(N * OH) + 7u) / 8u * 8u;
     if (dt == kF16)
-      hipLaunchKernelGGL((maxpool3x3s2_rows_kernel<half_t>), dim3(grid_rows), dim3(256), 0, s, (const half_t*)in, (half_t*)out, H, W, C, OH, OW,
+      launch_kernel((maxpool3x3s2_rows_kernel<half_t>), dim3(grid_rows), dim3(256), 0, s, (const half_t*)in, (half_t*)out, H, W, C, OH, OW,
                          (unsigned)in_bytes, inv_cg, (unsigned)(N * OH));
     else
-      hipLaunchKernelGGL((maxpool3x3s2_rows_kernel<float>), dim3(grid_rows), dim3(256), 0, s, (const float*)in, (float*)out, H, W, C, OH, OW,
+      launch_kernel((maxpool3x3s2_rows_kernel<float>), dim3(grid_rows), dim3(256), 0, s, (const float*)in, (float*)out, H, W, C, OH, OW,
                          (unsigned)in_bytes, inv_cg, (unsigned)(N * OH));
     NNCV_HIP_CHECK(hipGetLastError());
     return;
   }
   if (dt == kF16)
-    hipLaunchKernelGGL((maxpool3x3s2_kernel<half_t>), dim3((unsigned)grid), dim3(256), 0, s, (const half_t*)in, (half_t*)out, N, H, W, C, OH, OW);
+    launch_kernel((maxpool3x3s2_kernel<half_t>), dim3((unsigned)grid), dim3(256), 0, s, (const half_t*)in, (half_t*)out, N, H, W, C, OH, OW);
   else
-    hipLaunchKernelGGL((maxpool3x3s2_kernel<float>), dim3((unsigned)grid), dim3(256), 0, s, (const float*)in, (float*)out, N, H, W, C, OH, OW);
+    launch_kernel((maxpool3x3s2_kernel<float>), dim3((unsigned)grid), dim3(256), 0, s, (const float*)in, (float*)out, N, H, W, C, OH, OW);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 
@@ -285,17 +285,17 @@ void launch_global_avgpool_nhwc(const void* in, void* out, int dt, int N, int HW
     while (cgb > 2 && (long long)((CG + cgb - 1) / cgb) * N < 256) cgb >>= 1;
     dim3 grid((CG + cgb - 1) / cgb, N);
     if (dt == kF16)
-      hipLaunchKernelGGL((global_avgpool_vec_kernel<half_t>), grid, dim3(256), 0, s, (const half_t*)in, (half_t*)out, HW, C, cgb);
+      launch_kernel((global_avgpool_vec_kernel<half_t>), grid, dim3(256), 0, s, (const half_t*)in, (half_t*)out, HW, C, cgb);
     else
-      hipLaunchKernelGGL((global_avgpool_vec_kernel<float>), grid, dim3(256), 0, s, (const float*)in, (float*)out, HW, C, cgb);
+      launch_kernel((global_avgpool_vec_kernel<float>), grid, dim3(256), 0, s, (const float*)in, (float*)out, HW, C, cgb);
     NNCV_HIP_CHECK(hipGetLastError());
     return;
   }
   dim3 grid((C + 63) / 64, N);
   if (dt == kF16)
-    hipLaunchKernelGGL((global_avgpool_kernel<half_t>), grid, dim3(256), 0, s, (const half_t*)in, (half_t*)out, HW, C);
+    launch_kernel((global_avgpool_kernel<half_t>), grid, dim3(256), 0, s, (const half_t*)in, (half_t*)out, HW, C);
   else
-    hipLaunchKernelGGL((global_avgpool_kernel<float>), grid, dim3(256), 0, s, (const float*)in, (float*)out, HW, C);
+    launch_kernel((global_avgpool_kernel<float>), grid, dim3(256), 0, s, (const float*)in, (float*)out, HW, C);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 
@@ -446,9 +446,9 @@ void launch_avgpool_fc(const void* in, const void* w, const float* bias, float* 
   const double es = (double)dtype_size(dt);
   ProfScope prof("avgpool_fc", 2.0 * N * F * 512.0, es * ((double)N * HW * 512 + (double)F * 512) + 4.0 * N * F, s);
   if (dt == kF16)
-    hipLaunchKernelGGL((avgpool_fc_kernel<half_t>), grid, dim3(256), 0, s, (const half_t*)in, (const half_t*)w, bias, out, N, HW, F, fpb);
+    launch_kernel((avgpool_fc_kernel<half_t>), grid, dim3(256), 0, s, (const half_t*)in, (const half_t*)w, bias, out, N, HW, F, fpb);
   else
-    hipLaunchKernelGGL((avgpool_fc_kernel<float>), grid, dim3(256), 0, s, (const float*)in, (const float*)w, bias, out, N, HW, F, fpb);
+    launch_kernel((avgpool_fc_kernel<float>), grid, dim3(256), 0, s, (const float*)in, (const float*)w, bias, out, N, HW, F, fpb);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 
@@ -482,9 +482,9 @@ void launch_preprocess_u8(const void* src, void* dst, int dst_dt, int N, int H, 
   NNCV_REQUIRE(work > 0 && grid < (1ll << 31), "preprocess: bad size");
   ProfScope prof("preprocess_u8", 0.0, (double)work * (channels + 3.0 * dtype_size(dst_dt)), s);
   if (dst_dt == kF16)
-    hipLaunchKernelGGL((preprocess_u8_kernel<half_t>), dim3((unsigned)grid), dim3(256), 0, s, (const unsigned char*)src, (half_t*)dst, N, H * W, channels);
+    launch_kernel((preprocess_u8_kernel<half_t>), dim3((unsigned)grid), dim3(256), 0, s, (const unsigned char*)src, (half_t*)dst, N, H * W, channels);
   else
-    hipLaunchKernelGGL((preprocess_u8_kernel<float>), dim3((unsigned)grid), dim3(256), 0, s, (const unsigned char*)src, (float*)dst, N, H * W, channels);
+    launch_kernel((preprocess_u8_kernel<float>), dim3((unsigned)grid), dim3(256), 0, s, (const unsigned char*)src, (float*)dst, N, H * W, channels);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 
@@ -518,7 +518,7 @@ __global__ __launch_bounds__(256) void argmax_rows_kernel(const float* __restric
 void launch_argmax_rows(const float* x, int* idx, int N, int F, hipStream_t s) {
   NNCV_REQUIRE(N > 0 && F > 0, "argmax: empty");
   ProfScope prof("argmax_rows", 0.0, 4.0 * N * (F + 1.0), s);
-  hipLaunchKernelGGL(argmax_rows_kernel, dim3(N), dim3(256), 0, s, x, idx, F);
+  launch_kernel(argmax_rows_kernel, dim3(N), dim3(256), 0, s, x, idx, F);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 
@@ -664,10 +664,10 @@ void launch_relayout(const void* src, int src_dt, Strides4 ss, void* dst, int ds
     ProfScope prof("relayout", 0.0, (double)N * P * ((double)Cs * dtype_size(src_dt) + (double)Cd * dtype_size(dst_dt) * (accumulate ? 2 : 1)), s);
 #define LAUNCH(TS, TD)                                                                                                              \
   if (ss.w == 1 && ds.c == 1)                                                                                                       \
-    hipLaunchKernelGGL((relayout_tile_kernel<TS, TD, true>), grid, dim3(256), 0, s, (const TS*)src, ss.n, ss.c, ss.w, (TD*)dst,     \
+    launch_kernel((relayout_tile_kernel<TS, TD, true>), grid, dim3(256), 0, s, (const TS*)src, ss.n, ss.c, ss.w, (TD*)dst,     \
                        ds.n, ds.c, ds.w, Cs, Cd, P, accumulate ? 1 : 0);                                                            \
   else                                                                                                                              \
-    hipLaunchKernelGGL((relayout_tile_kernel<TS, TD, false>), grid, dim3(256), 0, s, (const TS*)src, ss.n, ss.c, ss.w, (TD*)dst,    \
+    launch_kernel((relayout_tile_kernel<TS, TD, false>), grid, dim3(256), 0, s, (const TS*)src, ss.n, ss.c, ss.w, (TD*)dst,    \
                        ds.n, ds.c, ds.w, Cs, Cd, P, accumulate ? 1 : 0)
     if (src_dt == kF32 && dst_dt == kF32) { LAUNCH(float, float); }
     else if (src_dt == kF32 && dst_dt == kF16) { LAUNCH(float, half_t); }
@@ -678,7 +678,7 @@ void launch_relayout(const void* src, int src_dt, Strides4 ss, void* dst, int ds
     return;
   }
 #define LAUNCH(TS, TD) \
-  hipLaunchKernelGGL((relayout_kernel<TS, TD>), dim3((unsigned)grid), dim3(256), 0, s, (const TS*)src, ss, (TD*)dst, ds, N, Cs, Cd, H, W, cf, accumulate ? 1 : 0)
+  launch_kernel((relayout_kernel<TS, TD>), dim3((unsigned)grid), dim3(256), 0, s, (const TS*)src, ss, (TD*)dst, ds, N, Cs, Cd, H, W, cf, accumulate ? 1 : 0)
   if (src_dt == kF32 && dst_dt == kF32) LAUNCH(float, float);
   else if (src_dt == kF32 && dst_dt == kF16) LAUNCH(float, half_t);
   else if (src_dt == kF16 && dst_dt == kF16) LAUNCH(half_t, half_t);
@@ -720,11 +720,11 @@ void launch_image_to_nhwc(const void* src, void* dst, int dt, int N, int C, int 
   NNCV_REQUIRE(grid < (1ll << 31), "image_to_nhwc: grid too large");
   ProfScope prof("image_to_nhwc", 0.0, (double)dtype_size(dt) * total * (C + Cp), s);
   if (dt == kF16 && Cp == 8)
-    hipLaunchKernelGGL((image_to_nhwc_kernel<half_t, 8>), dim3((unsigned)grid), dim3(256), 0, s, (const half_t*)src, (half_t*)dst, C, HW, total);
+    launch_kernel((image_to_nhwc_kernel<half_t, 8>), dim3((unsigned)grid), dim3(256), 0, s, (const half_t*)src, (half_t*)dst, C, HW, total);
   else if (dt == kF16)
-    hipLaunchKernelGGL((image_to_nhwc_kernel<half_t, 4>), dim3((unsigned)grid), dim3(256), 0, s, (const half_t*)src, (half_t*)dst, C, HW, total);
+    launch_kernel((image_to_nhwc_kernel<half_t, 4>), dim3((unsigned)grid), dim3(256), 0, s, (const half_t*)src, (half_t*)dst, C, HW, total);
   else
-    hipLaunchKernelGGL((image_to_nhwc_kernel<float, 4>), dim3((unsigned)grid), dim3(256), 0, s, (const float*)src, (float*)dst, C, HW, total);
+    launch_kernel((image_to_nhwc_kernel<float, 4>), dim3((unsigned)grid), dim3(256), 0, s, (const float*)src, (float*)dst, C, HW, total);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 
@@ -757,9 +757,9 @@ void launch_weight_pairs(const void* w, int w_dt, void* dst, int F, int Fp, int 
   const int total = Fp * K * S2 * 8;
   const unsigned grid = (unsigned)((total + 255) / 256);
   if (w_dt == kF16)
-    hipLaunchKernelGGL((weight_pairs_kernel<half_t>), dim3(grid), dim3(256), 0, s, (const half_t*)w, (half_t*)dst, F, C, K, S2, shift, total);
+    launch_kernel((weight_pairs_kernel<half_t>), dim3(grid), dim3(256), 0, s, (const half_t*)w, (half_t*)dst, F, C, K, S2, shift, total);
   else
-    hipLaunchKernelGGL((weight_pairs_kernel<float>), dim3(grid), dim3(256), 0, s, (const float*)w, (half_t*)dst, F, C, K, S2, shift, total);
+    launch_kernel((weight_pairs_kernel<float>), dim3(grid), dim3(256), 0, s, (const float*)w, (half_t*)dst, F, C, K, S2, shift, total);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 
@@ -801,7 +801,7 @@ void launch_stem_pack(const void* src, int src_dt, void* dst, int dst_dt, int N,
   NNCV_REQUIRE(grid < (1ll << 31), "stem_pack: grid too large");
   ProfScope prof("stem_pack", 0.0, (double)dtype_size(src_dt) * N * 3 * H * W + (double)dtype_size(dst_dt) * work * 8, s);
 #define LAUNCH(TS, TD) \
-  hipLaunchKernelGGL((stem_pack_kernel<TS, TD>), dim3((unsigned)grid), dim3(256), 0, s, (const TS*)src, (TD*)dst, N, H, W, HP, WP)
+  launch_kernel((stem_pack_kernel<TS, TD>), dim3((unsigned)grid), dim3(256), 0, s, (const TS*)src, (TD*)dst, N, H, W, HP, WP)
   if (src_dt == kF32 && dst_dt == kF32) LAUNCH(float, float);
   else if (src_dt == kF16 && dst_dt == kF16) LAUNCH(half_t, half_t);
   else if (src_dt == kF32 && dst_dt == kF16) LAUNCH(float, half_t);
@@ -839,7 +839,7 @@ void launch_weight_frsc(const void* w, int w_dt, void* dst, int dst_dt, int F, i
   const int RS = R * S;
   const int staged = RS <= 8192, cc = staged ? std::min(Cp, 8192 / RS) : Cp;  // 32 KB of LDS hold one channel's window at least
   const size_t lds = staged ? (size_t)cc * RS * 4 : 0;
-#define LAUNCH(TS, TD) hipLaunchKernelGGL((weight_frsc_kernel<TS, TD>), dim3((unsigned)F), dim3(256), lds, s, (const TS*)w, (TD*)dst, C, RS, Cp, cc, staged)
+#define LAUNCH(TS, TD) launch_kernel((weight_frsc_kernel<TS, TD>), dim3((unsigned)F), dim3(256), lds, s, (const TS*)w, (TD*)dst, C, RS, Cp, cc, staged)
   if (w_dt == kF32 && dst_dt == kF32) LAUNCH(float, float);
   else if (w_dt == kF16 && dst_dt == kF16) LAUNCH(half_t, half_t);
   else if (w_dt == kF32 && dst_dt == kF16) LAUNCH(float, half_t);
@@ -883,7 +883,7 @@ static void launch_weight_frag(const void* w, int w_dt, void* dst, int dst_dt, i
   const int Fp = (F + 63) / 64 * 64;
   const long long total = (long long)(Fp / 64) * (C / (8 * ce)) * TAPS * 4 * 2 * 64;
   const unsigned grid = (unsigned)((total + 255) / 256);
-#define LAUNCH(TS, TD) hipLaunchKernelGGL((weight_frag3x3_kernel<TS, TD, TAPS>), dim3(grid), dim3(256), 0, s, (const TS*)w, (TD*)dst, F, C, Fp)
+#define LAUNCH(TS, TD) launch_kernel((weight_frag3x3_kernel<TS, TD, TAPS>), dim3(grid), dim3(256), 0, s, (const TS*)w, (TD*)dst, F, C, Fp)
   if (w_dt == kF32 && dst_dt == kF32) LAUNCH(float, float);
   else if (w_dt == kF16 && dst_dt == kF16) LAUNCH(half_t, half_t);
   else fail("weight_frag: unsupported dtype combination");
@@ -910,7 +910,7 @@ __global__ void stem_weight_kernel(const Ts* __restrict__ w, Td* __restrict__ ds
 void launch_stem_weight(const void* w, int w_dt, void* dst, int dst_dt, int F, int col_shift, hipStream_t s) {
   const unsigned grid = (unsigned)((F * 224 + 255) / 256);
 #define LAUNCH(TS, TD) \
-  hipLaunchKernelGGL((stem_weight_kernel<TS, TD>), dim3(grid), dim3(256), 0, s, (const TS*)w, (TD*)dst, F, col_shift)
+  launch_kernel((stem_weight_kernel<TS, TD>), dim3(grid), dim3(256), 0, s, (const TS*)w, (TD*)dst, F, col_shift)
   if (w_dt == kF32 && dst_dt == kF32) LAUNCH(float, float);
   else if (w_dt == kF16 && dst_dt == kF16) LAUNCH(half_t, half_t);
   else if (w_dt == kF32 && dst_dt == kF16) LAUNCH(float, half_t);
@@ -937,9 +937,9 @@ void launch_bn_fold(const void* g, const void* b, const void* m, const void* v, 
                     hipStream_t s, float eps) {
   const unsigned grid = (unsigned)((C + 255) / 256);
   if (dt == kF16)
-    hipLaunchKernelGGL((bn_fold_kernel<half_t>), dim3(grid), dim3(256), 0, s, (const half_t*)g, (const half_t*)b, (const half_t*)m, (const half_t*)v, scale, shift, C, eps);
+    launch_kernel((bn_fold_kernel<half_t>), dim3(grid), dim3(256), 0, s, (const half_t*)g, (const half_t*)b, (const half_t*)m, (const half_t*)v, scale, shift, C, eps);
   else
-    hipLaunchKernelGGL((bn_fold_kernel<float>), dim3(grid), dim3(256), 0, s, (const float*)g, (const float*)b, (const float*)m, (const float*)v, scale, shift, C, eps);
+    launch_kernel((bn_fold_kernel<float>), dim3(grid), dim3(256), 0, s, (const float*)g, (const float*)b, (const float*)m, (const float*)v, scale, shift, C, eps);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 
@@ -952,7 +952,7 @@ __global__ void cast_kernel(const Ts* __restrict__ src, Td* __restrict__ dst, lo
 void launch_cast(const void* src, int src_dt, void* dst, int dst_dt, long long n, hipStream_t s) {
   if (n == 0) return;
   const unsigned grid = (unsigned)((n + 255) / 256);
-#define LAUNCH(TS, TD) hipLaunchKernelGGL((cast_kernel<TS, TD>), dim3(grid), dim3(256), 0, s, (const TS*)src, (TD*)dst, n)
+#define LAUNCH(TS, TD) launch_kernel((cast_kernel<TS, TD>), dim3(grid), dim3(256), 0, s, (const TS*)src, (TD*)dst, n)
   if (src_dt == kF32 && dst_dt == kF32) LAUNCH(float, float);
   else if (src_dt == kF16 && dst_dt == kF16) LAUNCH(half_t, half_t);
   else if (src_dt == kF32 && dst_dt == kF16) LAUNCH(float, half_t);
@@ -967,7 +967,7 @@ __global__ void fill_f32_kernel(float* dst, float v, long long n) {
 }
 void launch_fill_f32(float* dst, float v, long long n, hipStream_t s) {
   if (n == 0) return;
-  hipLaunchKernelGGL(fill_f32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, dst, v, n);
+  launch_kernel(fill_f32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, dst, v, n);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 

@@ -405,7 +405,7 @@ void launch_stem_pool(const void* in, const void* wt, const float* scale, const 
   const double bytes = 2.0 * ((double)N * 3 * H * W + (double)N * a.PH * a.PW * 64 + 64.0 * 224);
   ProfScope prof("stem_conv7x7_bn_relu_maxpool<f16>", flops, bytes, s);
   const int grid = a.ntiles < 512 ? a.ntiles : 512;  // two persistent workgroups per CU
-  hipLaunchKernelGGL(stem_pool_kernel, dim3(grid), dim3(256), smem, s, a);
+  launch_kernel(stem_pool_kernel, dim3(grid), dim3(256), smem, s, a);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 

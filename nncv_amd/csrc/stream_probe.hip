@@ -26,7 +26,7 @@ constexpr int kChain = 8;       // kernels per chain
 constexpr int kSpin = 12000;    // about 25 us per kernel
 
 void enqueue_chain(hipStream_t s, float* sink) {
-  for (int k = 0; k < kChain; ++k) hipLaunchKernelGGL(probe_spin_kernel, dim3(1), dim3(64), 0, s, kSpin, sink);
+  for (int k = 0; k < kChain; ++k) launch_kernel(probe_spin_kernel, dim3(1), dim3(64), 0, s, kSpin, sink);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 

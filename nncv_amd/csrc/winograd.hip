@@ -428,11 +428,11 @@ __global__ __launch_bounds__(256) void wino43_output_lds_kernel(const WinoOutArg
 void launch_wino43_filter(const void* w, int w_dt, void* U, int u_dt, int F, int C, hipStream_t s) {
   const int n = F * C, blk = 256, grid = (n + blk - 1) / blk;
   if (w_dt == kF32 && u_dt == kF32)
-    hipLaunchKernelGGL((wino43_filter_kernel<float, float>), dim3(grid), dim3(blk), 0, s, (const float*)w, (float*)U, F, C);
+    launch_kernel((wino43_filter_kernel<float, float>), dim3(grid), dim3(blk), 0, s, (const float*)w, (float*)U, F, C);
   else if (w_dt == kF16 && u_dt == kF16)
-    hipLaunchKernelGGL((wino43_filter_kernel<half_t, half_t>), dim3(grid), dim3(blk), 0, s, (const half_t*)w, (half_t*)U, F, C);
+    launch_kernel((wino43_filter_kernel<half_t, half_t>), dim3(grid), dim3(blk), 0, s, (const half_t*)w, (half_t*)U, F, C);
   else if (w_dt == kF32 && u_dt == kF16)
-    hipLaunchKernelGGL((wino43_filter_kernel<float, half_t>), dim3(grid), dim3(blk), 0, s, (const float*)w, (half_t*)U, F, C);
+    launch_kernel((wino43_filter_kernel<float, half_t>), dim3(grid), dim3(blk), 0, s, (const float*)w, (half_t*)U, F, C);
   else
     fail("wino43_filter: unsupported dtype combination");
   NNCV_HIP_CHECK(hipGetLastError());
@@ -458,16 +458,16 @@ void launch_wino43_input(const void* in, int in_dt, Strides4 st, void* V, int v_
     const long long tiles = (long long)N * TH * TW;
     if (in_dt == kF16) {
       dim3 g((unsigned)(((tiles + WinoLds<half_t>::kTiles - 1) / WinoLds<half_t>::kTiles + 7) / 8 * 8), C / 64);
-      hipLaunchKernelGGL((wino43_input_lds_kernel<half_t>), g, dim3(256), 0, s, (const half_t*)in, (half_t*)V, N, C, H, W, pad, TH, TW);
+      launch_kernel((wino43_input_lds_kernel<half_t>), g, dim3(256), 0, s, (const half_t*)in, (half_t*)V, N, C, H, W, pad, TH, TW);
     } else {
       dim3 g((unsigned)(((tiles + WinoLds<float>::kTiles - 1) / WinoLds<float>::kTiles + 7) / 8 * 8), C / 64);
-      hipLaunchKernelGGL((wino43_input_lds_kernel<float>), g, dim3(256), 0, s, (const float*)in, (float*)V, N, C, H, W, pad, TH, TW);
+      launch_kernel((wino43_input_lds_kernel<float>), g, dim3(256), 0, s, (const float*)in, (float*)V, N, C, H, W, pad, TH, TW);
     }
     NNCV_HIP_CHECK(hipGetLastError());
     return;
   }
 #define LAUNCH(TI, TV, CC)                                                                               \
-  hipLaunchKernelGGL((wino43_input_kernel<TI, TV, CC>), dim3((unsigned)grid), dim3(blk), 0, s, (const TI*)in, st, \
+  launch_kernel((wino43_input_kernel<TI, TV, CC>), dim3((unsigned)grid), dim3(blk), 0, s, (const TI*)in, st, \
                      (TV*)V, N, C, H, W, pad, TH, TW)
   if (in_dt == kF32 && v_dt == kF32) { if (contig) LAUNCH(float, float, true); else LAUNCH(float, float, false); }
   else if (in_dt == kF16 && v_dt == kF16) { if (contig) LAUNCH(half_t, half_t, true); else LAUNCH(half_t, half_t, false); }
@@ -492,16 +492,16 @@ void launch_wino43_output(const WinoOutArgs& a, int m_dt, int out_dt, hipStream_
     const long long tiles = (long long)a.N * TH * TW;
     if (m_dt == kF16) {
       dim3 g((unsigned)((tiles + WinoLds<half_t>::kTiles - 1) / WinoLds<half_t>::kTiles), a.F / 64);
-      hipLaunchKernelGGL((wino43_output_lds_kernel<half_t>), g, dim3(256), 0, s, a, TH, TW);
+      launch_kernel((wino43_output_lds_kernel<half_t>), g, dim3(256), 0, s, a, TH, TW);
     } else {
       dim3 g((unsigned)((tiles + WinoLds<float>::kTiles - 1) / WinoLds<float>::kTiles), a.F / 64);
-      hipLaunchKernelGGL((wino43_output_lds_kernel<float>), g, dim3(256), 0, s, a, TH, TW);
+      launch_kernel((wino43_output_lds_kernel<float>), g, dim3(256), 0, s, a, TH, TW);
     }
     NNCV_HIP_CHECK(hipGetLastError());
     return;
   }
 #define LAUNCH(TM, TO, CC) \
-  hipLaunchKernelGGL((wino43_output_kernel<TM, TO, CC>), dim3((unsigned)grid), dim3(blk), 0, s, a, TH, TW)
+  launch_kernel((wino43_output_kernel<TM, TO, CC>), dim3((unsigned)grid), dim3(blk), 0, s, a, TH, TW)
   if (m_dt == kF32 && out_dt == kF32) { if (contig) LAUNCH(float, float, true); else LAUNCH(float, float, false); }
   else if (m_dt == kF16 && out_dt == kF16) { if (contig) LAUNCH(half_t, half_t, true); else LAUNCH(half_t, half_t, false); }
   else if (m_dt == kF32 && out_dt == kF16) { if (contig) LAUNCH(float, half_t, true); else LAUNCH(float, half_t, false); }
