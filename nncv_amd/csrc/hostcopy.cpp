@@ -34,6 +34,7 @@ class CopyPool {
     }
     const uint64_t g = ++last_;
     gen_.store(0, std::memory_order_relaxed);
+    std::atomic_thread_fence(std::memory_order_release);  // with take()'s fence: whoever sees a field of job g sees that gen_ has left g - 1
     dst_.store(dst, std::memory_order_relaxed);
     src_.store(src, std::memory_order_relaxed);
     bytes_.store(bytes, std::memory_order_relaxed);
