@@ -48,7 +48,7 @@ class CopyPool {
     while (take()) {
     }
     const size_t chunks = (bytes + kChunk - 1) / kChunk;
-    while (done_.load(std::memory_order_acquire) < chunks) __builtin_ia32_pause();
+    for (int spins = 0; done_.load(std::memory_order_acquire) < chunks;) pause(spins);
   }
 
  private:
@@ -62,6 +62,11 @@ class CopyPool {
     if (hw > 0) n = std::min(n, hw);
     workers_ = std::max(1, std::min(n, 16)) - 1;
     for (int i = 0; i < workers_; ++i) std::thread([this] { loop(); }).detach();
+  }
+  // A wait of a chunk's length is spun through; in a longer one the thread that is waited for may need this CPU.
+  static void pause(int& spins) {
+    if (++spins & 255) __builtin_ia32_pause();
+    else std::this_thread::yield();
   }
   // Takes one chunk of the current job; false when none is left.  The counter carries the job's number: a chunk index that
   // lies inside job g keeps g from completing, so its fields stay as they are while the chunk is copied; fields that
@@ -85,8 +90,8 @@ class CopyPool {
       uint64_t g;
       int spins = 0;
       while ((g = next_.load(std::memory_order_acquire) >> 24) == seen) {
-        __builtin_ia32_pause();
-        if ((++spins & 63) == 0 && std::chrono::steady_clock::now() > until) break;
+        pause(spins);
+        if ((spins & 63) == 0 && std::chrono::steady_clock::now() > until) break;
       }
       if (g == seen) {
         std::unique_lock<std::mutex> lk(mu_);
