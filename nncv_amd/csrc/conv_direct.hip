@@ -4,7 +4,7 @@
 //
 // A wave owns TM x TN accumulators of BT x BT (filters x pixels).  K is the flat (r, s, c) axis in 16-byte chunks, eight of
 // them (one 128-byte line of a pixel) to a round.
-//  * Weights come fragment-major (launch_weight_frag_flat): an operand of a wave is one contiguous kilobyte, straight into
+//  * Weights come fragment-major (launch_weight_flat): an operand of a wave is one contiguous kilobyte, straight into
 //    registers a round ahead.
 //  * Pixels: an operand wants 32 (16) pixels x 2 (4) chunks, and read like that every lane of the load touches a line of
 //    its own, which the CU's address unit serves one lane a clock (58 cycles per load measured, against 16 for whole
@@ -69,7 +69,6 @@ struct Block<half_t, 16> {
 
 struct DirectArgs {
   const void* in; const void* wt; const void* aux_wt; void* out; const float* scale; const float* shift; const void* residual; void* aux_out;
-  long long in_bs, wt_bs, out_bs;
   unsigned in_bytes, wt_bytes, aux_wt_bytes;
   int H, W, F, S, OW, OHW, P, pix;
   int stride_h, stride_w, pad_h, pad_w;
@@ -106,8 +105,8 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
   const bool aux = tf >= a.main_tiles;
   const int f0 = aux ? a.main_f + (tf - a.main_tiles) * BT * TM : tf * BT * TM, p0 = tp * BT * TN;
   const int f_end = aux ? a.F : a.main_f;
-  const __amdgpu_buffer_rsrc_t rs_in = make_rsrc(static_cast<const T*>(a.in) + blockIdx.y * a.in_bs, a.in_bytes);
-  const __amdgpu_buffer_rsrc_t rs_wt = aux ? make_rsrc(a.aux_wt, a.aux_wt_bytes) : make_rsrc(static_cast<const T*>(a.wt) + blockIdx.y * a.wt_bs, a.wt_bytes);
+  const __amdgpu_buffer_rsrc_t rs_in = make_rsrc(a.in, a.in_bytes);
+  const __amdgpu_buffer_rsrc_t rs_wt = aux ? make_rsrc(a.aux_wt, a.aux_wt_bytes) : make_rsrc(a.wt, a.wt_bytes);
 
   // rounds of this group; an auxiliary tile walks the rounds of its tap (UNI)
   const int nr = (a.chunks + 7) >> 3, rpt = a.cpt >> 3;
@@ -207,7 +206,7 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
   // what this wave finishes: quads of four consecutive filters of a pixel.  Their residual and scale / shift are asked for
   // now; they arrive under the K walk.
   const OutT* res = aux ? nullptr : static_cast<const OutT*>(a.residual);
-  OutT* out = static_cast<OutT*>(aux ? a.aux_out : a.out) + blockIdx.y * a.out_bs;
+  OutT* out = static_cast<OutT*>(aux ? a.aux_out : a.out);
   const int ldo = aux ? a.aux_ldo : a.ldo, act = aux ? a.aux_act : a.act;
   typedef OutT out4 __attribute__((ext_vector_type(4)));
   struct Quad {
@@ -224,7 +223,7 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
     q.sc = a.scale && ok ? *reinterpret_cast<const floatx4*>(a.scale + f) : floatx4{1.f, 1.f, 1.f, 1.f};
     q.sh = a.shift && ok ? *reinterpret_cast<const floatx4*>(a.shift + f) : floatx4{0.f, 0.f, 0.f, 0.f};
     q.rv = out4{};
-    if (res && ok) q.rv = *reinterpret_cast<const out4*>(res + blockIdx.y * a.out_bs + q.at);
+    if (res && ok) q.rv = *reinterpret_cast<const out4*>(res + q.at);
     return q;
   };
   auto finish = [&](const Quad& q, const floatx4& sum) {
@@ -314,7 +313,7 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
 }
 
 template <typename T, typename OutT, int BT, int TM, int TN, int KG>
-void launch_cfg(DirectArgs d, int batch, hipStream_t s) {
+void launch_cfg(DirectArgs d, hipStream_t s) {
   constexpr int kBuf = 2 * BT * TN * 128, kPart = TM * TN * BT * BT * 4, lds = KG * (kBuf > kPart || KG == 1 ? kBuf : kPart);
   d.main_tiles = (d.main_f + BT * TM - 1) / (BT * TM);
   d.tiles_f = d.main_tiles + (d.F - d.main_f + BT * TM - 1) / (BT * TM);
@@ -326,7 +325,7 @@ void launch_cfg(DirectArgs d, int batch, hipStream_t s) {
       return true;
     }();
     (void)attr;
-    launch_kernel(kern, dim3((unsigned)((long long)d.tiles_f * d.tiles_p), (unsigned)batch), dim3(64 * KG), lds, s, d);
+    launch_kernel(kern, dim3((unsigned)((long long)d.tiles_f * d.tiles_p)), dim3(64 * KG), lds, s, d);
   };
   if (d.cpt % 8 == 0) go(conv_direct_kernel<T, OutT, BT, TM, TN, KG, true>);
   else go(conv_direct_kernel<T, OutT, BT, TM, TN, KG, false>);
@@ -371,7 +370,7 @@ __global__ __launch_bounds__(256) void weight_flat_kernel(const T* __restrict__ 
 struct Form {
   int rows, cols, kg;
   double fixed_us, round_us, tile_us, chain_us;
-  void (*launch)(DirectArgs, int, hipStream_t);
+  void (*launch)(DirectArgs, hipStream_t);
   const char* tags[3];  // 1x1, 3x3 and other windows
 };
 const Form kForms32[] = {
@@ -510,7 +509,7 @@ void launch_conv_direct(const IgemmArgs& a, int dt, hipStream_t s) {
   const double P = (double)d.P, flops = a.alg_flops > 0 ? a.alg_flops : 2.0 * P * a.F * a.R * a.S * a.C;
   ProfScope prof(f->tags[a.R == 1 && a.S == 1 ? 0 : a.R == 3 && a.S == 3 ? 1 : 2], flops,
                  (double)es * ((double)a.N * a.H * a.W * a.C + (double)a.F * a.R * a.S * a.C + P * a.F * (a.residual ? 2 : 1)), s);
-  f->launch(d, 1, s);
+  f->launch(d, s);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 
