@@ -366,6 +366,7 @@ __global__ __launch_bounds__(256) void weight_flat_kernel(const T* __restrict__ 
 //   us = fixed + t (round_us * rounds of a wave + tile_us) + chain_us * rounds of a wave
 // with t between tiles / 256 CUs and its ceiling, and a round = one 128-byte line of K.  Least-squares fits over 117 (fp32) and
 // 146 (fp16) layers of 1x1 to 7x7 windows, 8 to 1000 channels, one to 48 images, within 5-12 % of the measured times.
+// (fp32 64x64 tiles over four K groups are no form: 64x32 ones take less per area at every number of tiles.)
 #define TAGS(x) {"conv1x1_direct<" x ">", "conv3x3_direct<" x ">", "conv_direct<" x ">"}
 struct Form {
   int rows, cols, kg;
@@ -381,7 +382,6 @@ const Form kForms32[] = {
     {16, 16, 16, 2.1, 0.538, 1.24, 0.31, launch_cfg<float, float, 16, 1, 1, 16>, TAGS("f32,16x16,splitk16")},
     {32, 16, 8, 2.6, 0.543, 0.51, 0.12, launch_cfg<float, float, 16, 2, 1, 8>, TAGS("f32,32x16,splitk8")},
     {64, 32, 4, 3.3, 1.061, 0.53, 0.22, launch_cfg<float, float, 32, 2, 1, 4>, TAGS("f32,64x32,splitk4")},
-    {64, 64, 4, 3.6, 2.368, 1.08, 0.0, launch_cfg<float, float, 32, 2, 2, 4>, TAGS("f32,64x64,splitk4")},
     {64, 64, 1, 6.0, 0.297, 1.44, 1.89, launch_cfg<float, float, 32, 2, 2, 1>, TAGS("f32,64x64")},
 };
 const Form kForms16[] = {
