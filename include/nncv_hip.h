@@ -109,8 +109,7 @@ int nncv_hip_resnet18_passes_in_flight(const nncv_hip_model* m);
  * the reference. */
 int nncv_hip_pick_streams(int want, void** streams, int* overlapping);
 void nncv_hip_resnet18_destroy(nncv_hip_model* m);
-/* A second handle on the SAME device weights (fp16 models only; an fp32 model keeps the tickets of its K-split launches
- * with its layers, which two passes at once would share): its own workspace, so its passes overlap with those of
+/* A second handle on the SAME device weights (fp16 models only): its own workspace, so its passes overlap with those of
  * `m` and of other clones on other streams like those of separately created models do, without a second copy of the
  * 23 MB of filters in memory and in the caches (four passes in flight: 0.160 against 0.163 ms per pass).  The weights
  * live until the last handle on them is destroyed.  NULL on error.  No counterpart in the reference, whose compiled
@@ -143,8 +142,8 @@ int nncv_hip_conv_forward(nncv_hip_conv* c, const void* in, int N, int H, int W,
                           void* out, void* stream);
 /* The same as nncv_hip_conv_forward with layout = 1 (NHWC), for callers that cannot allocate: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the reference.  The
- * workspace the layer's kernels need (the partial sums and ticket counters of the K split of fp32 3x3 layers) is a
- * device array of the library, 4 MiB + 1 KiB on every GPU it runs on, held until the process ends; the call allocates
+ * workspace the layer's kernels need (a Winograd layer's transformed tensors; the direct convolutions need none) is a
+ * device array of the library, 4 MiB on every GPU it runs on, held until the process ends; the call allocates
  * and frees nothing.  A layer/shape whose workspace is larger fails with an error that says so.  All calls on one GPU
  * share the array.  Outside a capture the library orders them itself: a call on another stream than the previous one
  * first waits for the event that call left behind.  On a stream that is being captured it neither waits nor records

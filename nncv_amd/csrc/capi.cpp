@@ -124,8 +124,8 @@ class TailScope {
   TailEvent t_;
 };
 
-// NULL stream -> library stream + synchronise on exit.  Workspace (one arena), split-K tickets and the
-// pinned staging buffers are shared by every call, and the mutex only serialises the enqueueing: work
+// NULL stream -> library stream + synchronise on exit.  The workspace (one arena) and the pinned
+// staging buffers are shared by every call, and the mutex only serialises the enqueueing: work
 // left pending on one caller stream must not overlap work enqueued next on another.  So a call that
 // arrives on a different stream than the previous one first makes its stream wait for what the
 // previous call left behind (StreamOrder, runtime.hpp).
@@ -175,7 +175,7 @@ struct Sync {
 // A network handle (nncv_hip_resnet18 / nncv_hip_graph) owns its workspace, so passes of DIFFERENT handles on
 // different streams run concurrently: two passes in flight fill each other's launch gaps, prologues and tails
 // (ResNet-18 at batch 32: 0.18-0.19 ms per pass against 0.24 one after the other).  Calls on ONE handle share that
-// workspace (and the K-split tickets of its layers), so a call that arrives on another stream than the handle's
+// workspace, so a call that arrives on another stream than the handle's
 // previous one first makes its stream wait for that one, as Sync does for the library-wide arena.
 struct HandleState {
   HandleState() { order.create(); }
@@ -950,7 +950,7 @@ nncv_hip_model* nncv_hip_resnet18_clone(nncv_hip_model* m) {
   nncv_hip_model* h = nullptr;
   const int rc = guarded([&] {
     NNCV_REQUIRE(m && m->m, "null argument");
-    NNCV_REQUIRE(m->m->dtype() == kF16, "clone: fp16 models only (an fp32 model's K-split tickets belong to its layers)");
+    NNCV_REQUIRE(m->m->dtype() == kF16, "clone: fp16 models only");
     h = new nncv_hip_model();
     h->m = m->m;
     h->passes = m->passes;
@@ -1134,12 +1134,8 @@ int nncv_hip_conv_forward_noalloc(nncv_hip_conv* c, const void* in, int N, int H
     NNCV_REQUIRE(wsb <= kNoAllocWorkspaceBytes,
                  "nncv_hip_conv_forward_noalloc: this layer and shape need " + std::to_string(wsb) + " bytes of workspace, the "
                  "scratch array holds " + std::to_string(kNoAllocWorkspaceBytes) + "; use nncv_hip_conv_forward");
-    static_assert(ConvLayer::kSplitKCounterInts * sizeof(int) <= kNoAllocCounterBytes, "ticket counters outgrow their slot");
     Sync sy(stream);
-    char* scratch = static_cast<char*>(noalloc_scratch());
-    // the array keeps the previous call's contents: the tickets must start at zero (the workspace is written before it is read)
-    launch_clear_words(scratch, ConvLayer::kSplitKCounterInts, sy.s);
-    L.forward(in, N, H, W, residual, out, scratch + kNoAllocCounterBytes, sy.s, reinterpret_cast<int*>(scratch));
+    L.forward(in, N, H, W, residual, out, noalloc_scratch(), sy.s);
     sy.finish();
   });
 }

@@ -207,13 +207,6 @@ struct IgemmArgs {
   int aux_f0, aux_tap, aux_relu, aux_ldo;
   void* aux_out;
   const void* aux_wt_frag;  // the auxiliary 1x1 filters alone, fragment-major (launch_weight_frag1x1), or null
-  // Optional scratch for splitting K over workgroups (conv3x3_patch.hip, small fp32 launches only):
-  // splitk_ws holds fp32 partial tiles for the duration of the launch; splitk_counters are
-  // splitk_counters_n ints that are zero before the launch and zero again after it.  Null: no split.
-  void* splitk_ws;
-  size_t splitk_ws_bytes;
-  int* splitk_counters;
-  int splitk_counters_n;
   // What conv_direct.hip reads instead of wt and wt_frag: the filters (launch_weight_flat), and the auxiliary filters alone
   // (the same with one tap); or null.  Behind the fields that the other kernels load.
   const void *wt_flat, *aux_wt_flat;
@@ -228,7 +221,7 @@ struct IgemmArgs {
 void launch_igemm(const IgemmArgs& a, int in_dt, int out_dt, hipStream_t s);
 // whether it would launch the kernel of conv_direct.hip, i.e. reads wt_flat (which must be set, as must be what it points to later)
 bool igemm_takes_direct(const IgemmArgs& a, int in_dt, int out_dt);
-// 3x3 pad-1 layers at stride 1 or 2: direct convolution with the haloed input patch resident in LDS
+// 3x3 pad-1 layers at stride 1, or 2 in fp16: direct convolution with the haloed input patch resident in LDS
 // (conv3x3_patch.hip); same arguments and epilogue as the igemm kernels.
 bool conv3x3_patch_applicable(const IgemmArgs& a, int in_dt);
 // The tile plan that kernel would use for N x OH x OW output pixels, F filters and `slabs` 128-byte

@@ -417,7 +417,7 @@ const Form* best_form(const IgemmArgs& a, int dt, double* us) {
 
 // The same for the kernel that would run the layer otherwise.  Implicit GEMM: fits over its 64 x 64 tiles, within 7-16 %.
 // fp32 3x3 stride-1 patch kernel: 0.5 us per 32 channels and tap for every 64 slots x 64 filters of a CU's workgroups, half
-// of it where a half-filled launch runs 32-filter blocks or splits K.  (Its waves share pixels through LDS, so it stays
+// of it where a half-filled launch runs 32-filter blocks.  (Its waves share pixels through LDS, so it stays
 // ahead where its tiles fill the CUs evenly, 6x29x39x128: 22.1 against 24.5 us, and falls behind where they do not.)
 double other_us(const IgemmArgs& a, int dt, DirectRival rival) {
   struct Fit { double fixed, round, tile, chain; };
@@ -472,7 +472,10 @@ bool conv_direct_applicable(const IgemmArgs& a, int in_dt, int out_dt) {
 
 bool conv_direct_wins(const IgemmArgs& a, int dt, DirectRival rival) {
   if (rival == kRivalShortK) return false;  // already one latency long (3.0-4.5 us either way)
-  if (rival == kRivalPatchS2 && dt == kF32) return true;  // 5-60 % faster at every size measured (6x58x78x64 -> 128: 23.2 -> 15.1 us)
+  // fp32 3x3 stride-2 layers of up to 8 GFLOP: the model below flatters igemm_fast there.  Of 40 random shapes that it would
+  // give to that kernel 38 are 2-60 % faster here (3x56x80x64 -> 640: 31.3 against 45.3 us, 1x154x199x64 -> 240: 26.9 against 28.1).
+  const double main_flops = 2.0 * a.N * a.OH * a.OW * (a.aux_f0 ? a.aux_f0 : a.F) * a.R * a.S * (double)a.C;
+  if (dt == kF32 && a.R == 3 && a.S == 3 && a.stride_h == 2 && a.stride_w == 2 && a.pad_h == 1 && a.pad_w == 1 && a.C % 32 == 0 && main_flops <= 8e9) return true;
   const bool patch = rival == kRivalPatch || rival == kRivalPatchS2;
   // fp16 3x3 layers leave the patch kernels only where those have less than a quarter of the chip to work with (blocks of 64
   // pixels x 32 filters): there the layer is bound by how many CUs stream its weights (7x7x512, one image: 8.4 -> 6.0 us).

@@ -148,7 +148,7 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
         launch_weight_frsc(w, dt, nd.wt.get(), dt, op.F, Cl, op.K, op.K, C, s);
         nd.wflat.reset(weight_flat_bytes(dt, Cstored, op.K * op.K, C), &pool_);
         launch_weight_flat(w, nd.wflat.get(), dt, op.F, Cl, op.K * op.K, C, s);
-        if (op.K == 3 && (op.stride == 1 || op.stride == 2) && op.pad == 1 && Cl == C && Cstored == op.F && C % (128 / (int)es) == 0) {
+        if (op.K == 3 && (op.stride == 1 || (op.stride == 2 && dt == kF16)) && op.pad == 1 && Cl == C && Cstored == op.F && C % (128 / (int)es) == 0) {
           nd.wfrag.reset((size_t)((op.F + 63) / 64) * 64 * 9 * C * es, &pool_);
           launch_weight_frag3x3(w, dt, nd.wfrag.get(), dt, op.F, C, s);
           if (dt == kF16 && op.stride == 1 && C % 64 == 0 && op.F % 32 == 0) {

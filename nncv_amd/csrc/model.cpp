@@ -16,10 +16,6 @@ static int env_algo3x3() {
 
 static int round_up(int v, int m) { return (v + m - 1) / m * m; }
 
-// scratch of the patch kernel's K split: at most 256 workgroups' 64x64 fp32 partial tiles
-constexpr size_t kSplitKWsBytes = 256 * 4096 * sizeof(float);
-constexpr int kSplitKCounters = ConvLayer::kSplitKCounterInts;
-
 ConvLayer::ConvLayer(const Desc& d, const void* w, const void* gamma, const void* beta, const void* mean, const void* var,
                      hipStream_t s)
     : d_(d) {
@@ -69,16 +65,12 @@ ConvLayer::ConvLayer(const Desc& d, const void* w, const void* gamma, const void
     launch_weight_frsc(w, d.dt, wt_.get(), d.dt, d.F, d.C, d.R, d.S, Cp, s);
     wflat_.reset(weight_flat_bytes(d.dt, Fp, d.R * d.S, Cp), d.pool);
     launch_weight_flat(w, wflat_.get(), d.dt, d.F, d.C, d.R * d.S, Cp, s);
-    if (d.R == 3 && d.S == 3 && (d.stride == 1 || d.stride == 2) && d.pad == 1 && d.C % (128 / (int)es) == 0) {
+    if (d.R == 3 && d.S == 3 && (d.stride == 1 || (d.stride == 2 && d.dt == kF16)) && d.pad == 1 && d.C % (128 / (int)es) == 0) {
       wfrag_.reset((size_t)((d.F + 63) / 64) * 64 * 9 * d.C * es, d.pool);
       launch_weight_frag3x3(w, d.dt, wfrag_.get(), d.dt, d.F, d.C, s);
       if (d.dt == kF16 && d.stride == 1 && d.C % 64 == 0 && d.F % 32 == 0) {
         wfrag32_.reset(weight_frag32_bytes(d.F, d.C), d.pool);
         launch_weight_frag32(w, d.dt, wfrag32_.get(), d.F, d.C, s);
-      }
-      if (d.dt == kF32) {
-        splitk_counters_.reset(kSplitKCounters * sizeof(int), d.pool);
-        NNCV_HIP_CHECK(hipMemsetAsync(splitk_counters_.get(), 0, splitk_counters_.bytes(), s));
       }
     }
   }
@@ -106,12 +98,10 @@ size_t ConvLayer::workspace_bytes(int N, int H, int W, bool strided) const {
   // strided (operator-level) form of the igemm path stages NHWC copies of input and output
   if (strided && !d_.stem && algo_ == kAlgoIgemm)
     b += align256((size_t)N * H * W * round_up(d_.C, ce) * es) + 2 * align256((size_t)N * OH * OW * round_up(d_.F, 4) * es);
-  if (splitk_counters_.get()) b += kSplitKWsBytes;
   return b;
 }
 
-void ConvLayer::forward(const void* in, int N, int H, int W, const void* residual, void* out, void* ws, hipStream_t s,
-                        int* counters) const {
+void ConvLayer::forward(const void* in, int N, int H, int W, const void* residual, void* out, void* ws, hipStream_t s) const {
   const int OH = out_h(H), OW = out_w(W);
   NNCV_REQUIRE(N > 0 && OH > 0 && OW > 0, "conv: empty tensor");
   const size_t es = dtype_size(d_.dt);
@@ -141,10 +131,6 @@ void ConvLayer::forward(const void* in, int N, int H, int W, const void* residua
   a.N = N; a.H = H; a.W = W; a.C = d_.C; a.F = d_.F; a.R = d_.R; a.S = d_.S; a.OH = OH; a.OW = OW;
   a.stride_h = a.stride_w = d_.stride; a.pad_h = a.pad_w = d_.pad;
   a.relu = d_.relu; a.ldo = d_.F; a.batch = 1;
-  if (ws && splitk_counters_.get()) {
-    a.splitk_ws = ws; a.splitk_ws_bytes = kSplitKWsBytes;
-    a.splitk_counters = counters ? counters : splitk_counters_.as<int>(); a.splitk_counters_n = kSplitKCounters;
-  }
   launch_igemm(a, d_.dt, d_.dt, s);
 }
 
@@ -200,10 +186,6 @@ void ConvLayer::forward_with_shortcut(const void* in, int N, int H, int W, void*
   a.relu = d_.relu; a.ldo = d_.F; a.batch = 1;
   a.aux_f0 = d_.F; a.aux_tap = 4; a.aux_relu = aux_relu_; a.aux_ldo = aux_F_; a.aux_out = shortcut_out;
   a.alg_flops = (2.0 * d_.F * 9.0 * d_.C + aux_flops_per_pixel_) * N * OH * OW;
-  if (ws && splitk_counters_.get()) {
-    a.splitk_ws = ws; a.splitk_ws_bytes = kSplitKWsBytes;
-    a.splitk_counters = splitk_counters_.as<int>(); a.splitk_counters_n = kSplitKCounters;
-  }
   launch_igemm(a, d_.dt, d_.dt, s);
 }
 
@@ -252,10 +234,6 @@ void ConvLayer::forward_strided(const void* in, Strides4 in_st, int N, int H, in
   a.stride_h = a.stride_w = d_.stride; a.pad_h = a.pad_w = d_.pad;
   a.relu = d_.relu; a.ldo = Fp; a.batch = 1;
   NNCV_REQUIRE(!(accumulate && (d_.relu || residual)), "conv: accumulate form has no epilogue");
-  if (splitk_counters_.get()) {
-    a.splitk_ws = wsp + in_b + 2 * out_b; a.splitk_ws_bytes = kSplitKWsBytes;
-    a.splitk_counters = splitk_counters_.as<int>(); a.splitk_counters_n = kSplitKCounters;
-  }
   launch_igemm(a, d_.dt, d_.dt, s);
   // out (+)= y : y is NHWC with Fp channels; only the first F are copied
   launch_relayout(yout, d_.dt, strides_of(kNHWC, Fp, OH, OW), out, d_.dt, out_st, N, d_.F, d_.F, OH, OW, accumulate, s);

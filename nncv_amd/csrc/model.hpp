@@ -37,11 +37,8 @@ class ConvLayer {
   int out_w(int W) const { return (W + 2 * d_.pad - d_.S) / d_.stride + 1; }
   size_t workspace_bytes(int N, int H, int W, bool strided = false) const;
   // in/out/residual: NHWC device tensors of type dt (stem: `in` is NCHW [N,3,H,W]).
-  // `ws` must hold workspace_bytes().  `counters`: kSplitKCounterInts zeroed ints to use as the K split's tickets
-  // instead of the layer's own (null = the layer's own).
-  void forward(const void* in, int N, int H, int W, const void* residual, void* out, void* ws, hipStream_t s,
-               int* counters = nullptr) const;
-  static constexpr int kSplitKCounterInts = 256;
+  // `ws` must hold workspace_bytes().
+  void forward(const void* in, int N, int H, int W, const void* residual, void* out, void* ws, hipStream_t s) const;
   // generic-layout form used by the operator-level ABI: strides for in / out (residual shares out's)
   void forward_strided(const void* in, Strides4 in_st, int N, int H, int W, const void* residual, void* out, Strides4 out_st,
                        bool accumulate, void* ws, hipStream_t s) const;
@@ -63,7 +60,6 @@ class ConvLayer {
   DeviceBuffer wt_cat_, scale_cat_, shift_cat_;  // this layer's filters followed by the fused shortcut's
   const void* aux_wflat_ = nullptr;  // the fused shortcut layer's own wflat_
   DeviceBuffer aux_wfrag_;  // the fused shortcut's filters alone, fragment-major (stride-2 patch kernel)
-  DeviceBuffer splitk_counters_;  // tickets of the patch kernel's K split (fp32); zero between launches
   int aux_F_ = 0;
   int aux_relu_ = 0;
   double aux_flops_per_pixel_ = 0.0;

@@ -1,8 +1,8 @@
 // The scratch memory of the one entry point that allocates nothing (nncv_hip_conv_forward_noalloc): callers that
 // cannot call hipMalloc -- code under HIP graph capture, serving loops, harnesses that forbid it -- still need the
-// partial-sum workspace and the ticket counters of the K split that fp32 3x3 layers use
-// (conv3x3_patch.hip, tile_reduce_store_splitk).  Here that workspace is a file-scope device array: each GPU the
-// library runs on holds its own copy at its own address until the process ends.
+// workspace of the layer's kernels (the transformed tensors of a Winograd layer; the direct convolutions need none).
+// Here that workspace is a file-scope device array: each GPU the library runs on holds its own copy at its own address
+// until the process ends.
 //
 // In host code the array's name is a stand-in, not a device address; the address on the current device comes
 // from hipGetSymbolAddress, once per device, and everything else uses that pointer.
@@ -16,15 +16,10 @@ namespace {
 
 constexpr int kMaxDevices = 64;
 
-static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
+static __device__ __align__(256) unsigned char scratch[kNoAllocWorkspaceBytes];
 
 std::mutex g_mu;
 void* g_ptr[kMaxDevices] = {};
-
-__global__ void clear_words_kernel(unsigned* p, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0u;
-}
 
 }  // namespace
 
@@ -40,12 +35,6 @@ void* noalloc_scratch() {
     g_ptr[dev] = p;
   }
   return g_ptr[dev];
-}
-
-// A fill kernel, not hipMemsetAsync: a caller may be capturing the stream into a graph.
-void launch_clear_words(void* p, int n_words, hipStream_t s) {
-  launch_kernel(clear_words_kernel, dim3((n_words + 255) / 256), dim3(256), 0, s, static_cast<unsigned*>(p), n_words);
-  NNCV_HIP_CHECK(hipGetLastError());
 }
 
 }  // namespace nncv_hip

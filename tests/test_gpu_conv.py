@@ -184,9 +184,9 @@ def test_random_layers(dt):
 
 
 def test_fp32_k_split_over_workgroups_is_exact_and_repeatable():
-    """A deep fp32 3x3 layer at batch 1 has too few workgroups for the chip, so the patch kernel splits its K walk over
-    several per output tile; the last one to arrive adds the partial tiles in slab order.  Whichever arrives last, the bits
-    must be the same on every launch (the tickets return to zero each time), and they must match the oracle."""
+    """A deep fp32 3x3 layer at batch 1 has too few output tiles for the chip, so the waves of a workgroup split its K walk
+    (conv_direct.hip) and add their sums in a fixed order: the bits must be the same on every launch, and they must match
+    the oracle."""
     N, C, F, H = 1, 512, 512, 7
     x = synth.normal(7100, (N, C, H, H))
     w = synth.normal(7101, (F, C, 3, 3), std=float(np.sqrt(2.0 / (C * 9))))

@@ -186,8 +186,7 @@ def test_device_calls_on_two_streams_do_not_overlap_in_the_shared_workspace(blob
 def test_two_handles_on_two_streams_run_concurrently_and_stay_exact(blob, dt):
     """Every network handle owns its workspace: passes of two handles enqueued alternately on two caller streams, with
     nothing ordering them, overlap on the GPU and must still each give the bits of a pass run alone -- fp16 at the
-    measured batch and fp32 at batch 1, where the deep layers split K over workgroups (tickets and partial sums are
-    per handle too)."""
+    measured batch and fp32 at batch 1, where the deep layers split K over the waves of a workgroup."""
     import torch
     from gpu_util import Model, dev, host
     b = synth.round_fp16(blob) if dt == abi.F16 else blob
@@ -372,8 +371,7 @@ def test_pick_streams_returns_usable_streams(blob):
 
 def test_clones_share_the_weights_and_outlive_the_first_handle(blob):
     """nncv_hip_resnet18_clone: the clone gives the bits of the model it was made from, keeps working after that model's
-    handle is destroyed (the weights live until the last handle goes), and is refused for fp32 models, whose K-split
-    tickets belong to the layers."""
+    handle is destroyed (the weights live until the last handle goes), and is refused for fp32 models."""
     import pytest
     from gpu_util import Model, dev, host
     hb = synth.round_fp16(blob)

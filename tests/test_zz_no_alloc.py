@@ -1,8 +1,8 @@
 """The entry point that allocates nothing, nncv_hip_conv_forward_noalloc, against nncv_hip_conv_forward on the same
 inputs: two calls in a row through the C ABI, the second with a smaller input (the scratch array keeps the first
 call's contents), then a request beyond the scratch array's size, which must fail with a message and change nothing.
-The layers are fp32 3x3 ones of the K-split kind (the partial sums and tickets are what the scratch array holds) and
-one fp16 layer that needs no workspace at all."""
+The direct convolutions need no workspace, in fp32 or fp16; what the scratch array holds are the transformed tensors of a
+Winograd layer, small enough or too large for it."""
 import numpy as np
 import pytest
 import torch
@@ -47,7 +47,7 @@ def test_noalloc_matches_conv_forward_twice(dt):
     if dt == abi.F16:
         bn = tuple(synth.round_fp16(b) for b in bn)
     layer = Conv(dt, w, 1, 1, bn=bn, relu=True, algo=abi.ALGO_IGEMM)
-    for (N, H, W, seed) in ((1, 8, 8, 9200), (1, 4, 4, 9300)):  # the K-split shape of config 3's last stage, then a smaller one
+    for (N, H, W, seed) in ((1, 8, 8, 9200), (1, 4, 4, 9300)):  # the last stage of a 256x256 image, then a smaller input
         print("noalloc case", dt, N, H, W, flush=True)
         got, want = run_pair(layer, dt, N, H, W, seed)
         # against the CPU oracle as well, so that this file stands on its own: conv + BatchNorm + residual + ReLU
@@ -91,8 +91,8 @@ def test_noalloc_refuses_what_the_scratch_cannot_hold():
 
 @pytest.mark.parametrize("dt", [abi.F32, abi.F16])
 def test_noalloc_under_graph_capture(dt):
-    """Two calls of the entry point recorded into one HIP graph on a capturing stream (kernel nodes only: the tickets are
-    cleared by a fill kernel, the library neither waits for nor records events on a capturing stream), replayed three
+    """Two calls of the entry point recorded into one HIP graph on a capturing stream (kernel nodes only:
+    the library neither waits for nor completes events on a capturing stream), replayed three
     times with eager work and synchronisations in between; every replay gives the bits of nncv_hip_conv_forward."""
     C = F = 512
     w = synth.normal(9600, (F, C, 3, 3), std=float(np.sqrt(2.0 / (C * 9))))
