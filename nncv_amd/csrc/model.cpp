@@ -284,46 +284,39 @@ ResNet18::ResNet18(const void* params, long long n_elems, int dt, int algo3x3, h
   NNCV_REQUIRE((p - static_cast<const char*>(params)) == (long long)(kResNet18Elems * es), "ResNet-18 params: table walk mismatch");
 }
 
-namespace {
-// Workspace layout of one forward pass, planned with plan_offsets (arena_plan.hpp) from the
-// tensors' sizes and the operator range over which each one is live.  Operator numbering: 0 stem
-// convolution, 1 max-pool, then per BasicBlock k: 2+3k conv1, 3+3k shortcut conv, 4+3k conv2,
-// 26 average pool, 27 FC.
-struct Plan {
-  int h1, w1, h2, w2, h_out, w_out;  // after stem, after maxpool, after the body
-  size_t stem_out, pooled, cws;  // offsets
-  size_t x[9];                   // x[k] = input of block k; x[8] = network body output
-  size_t y1[8], idn[8];
-  size_t total;
-};
-}  // namespace
-
-static Plan make_plan(const ConvLayer& stem, const std::vector<const ConvLayer*>& c1s, const std::vector<const ConvLayer*>& c2s,
-                      const std::vector<const ConvLayer*>& dss, int dt, int N, int H, int W) {
+const ResNet18::Plan& ResNet18::plan_of(int N, int H, int W) const {
+  const int linger = (overlap_hint() >= 3 && N >= 16 && !arena_linger_forced()) ? 0 : arena_linger();  // see overlap_hint
+  for (const Plan& p : plans_)
+    if (p.N == N && p.H == H && p.W == W && p.linger == linger) return p;
+  NNCV_REQUIRE(blocks_.size() == 8, "ResNet-18 has eight BasicBlocks");
+  const ConvLayer& stem = *stem_;
   Plan p{};
-  const size_t es = dtype_size(dt);
+  p.N = N; p.H = H; p.W = W; p.linger = linger;
+  const size_t es = dtype_size(dt_);
   p.h1 = stem.out_h(H); p.w1 = stem.out_w(W);
   p.h2 = (p.h1 + 2 - 3) / 2 + 1; p.w2 = (p.w1 + 2 - 3) / 2 + 1;
   std::vector<TensorLife> t;
   auto add = [&](int first, int last, size_t bytes) { t.push_back(TensorLife{first, last, bytes, 0}); return (int)t.size() - 1; };
   // the fused stem kernel writes the pooled tensor directly: no stem output, no packed image
-  const bool fused_stem = stem.desc().relu == kActRelu && stem_pool_applicable(dt, N, H, W, stem.desc().F);
+  const bool fused_stem = stem.desc().relu == kActRelu && stem_pool_applicable(dt_, N, H, W, stem.desc().F);
   const int i_stem = add(0, 1, fused_stem ? 0 : (size_t)N * p.h1 * p.w1 * 64 * es);
   size_t cws = fused_stem ? 0 : stem.workspace_bytes(N, H, W);
   int h = p.h2, w = p.w2, ch = 64;
   int ix[9], iy1[8], iidn[8];
   ix[0] = add(1, 0, 0);  // last use filled in below
-  const int nb = (int)c1s.size();
+  const int nb = (int)blocks_.size();
   for (int k = 0; k < nb; ++k) {
+    const ConvLayer &c1 = *blocks_[k].c1, &c2 = *blocks_[k].c2;
+    const ConvLayer* ds = blocks_[k].ds.get();
     const int o = 2 + 3 * k;
-    const int oh = c1s[k]->out_h(h), ow = c1s[k]->out_w(w), f = c2s[k]->desc().F;
-    cws = std::max(cws, c1s[k]->workspace_bytes(N, h, w));
-    cws = std::max(cws, c2s[k]->workspace_bytes(N, oh, ow));
-    if (dss[k]) cws = std::max(cws, dss[k]->workspace_bytes(N, h, w));
+    const int oh = c1.out_h(h), ow = c1.out_w(w), f = c2.desc().F;
+    cws = std::max(cws, c1.workspace_bytes(N, h, w));
+    cws = std::max(cws, c2.workspace_bytes(N, oh, ow));
+    if (ds) cws = std::max(cws, ds->workspace_bytes(N, h, w));
     t[ix[k]].bytes = (size_t)N * h * w * ch * es;
-    t[ix[k]].last_op = dss[k] ? o + 1 : o + 2;  // identity shortcuts are read by conv2
+    t[ix[k]].last_op = ds ? o + 1 : o + 2;  // identity shortcuts are read by conv2
     iy1[k] = add(o, o + 2, (size_t)N * oh * ow * f * es);
-    iidn[k] = dss[k] ? add(o, o + 2, (size_t)N * oh * ow * f * es) : -1;
+    iidn[k] = ds ? add(o, o + 2, (size_t)N * oh * ow * f * es) : -1;
     ix[k + 1] = add(o + 2, o + 3, 0);
     h = oh; w = ow; ch = f;
   }
@@ -332,27 +325,21 @@ static Plan make_plan(const ConvLayer& stem, const std::vector<const ConvLayer*>
   t[ix[nb]].last_op = 26;
   const int i_pooled = add(26, 27, (size_t)N * 512 * es);
   const int i_cws = add(0, 27, cws);
-  const int linger = (overlap_hint() >= 3 && N >= 16 && !arena_linger_forced()) ? 0 : arena_linger();  // see overlap_hint
   for (auto& e : t) e.last_op = std::min(27, e.last_op + linger);
   p.total = plan_offsets(t, 256) + 4096;
   p.stem_out = t[i_stem].offset; p.pooled = t[i_pooled].offset; p.cws = t[i_cws].offset;
   for (int k = 0; k <= nb; ++k) p.x[k] = t[ix[k]].offset;
   for (int k = 0; k < nb; ++k) { p.y1[k] = t[iy1[k]].offset; p.idn[k] = iidn[k] >= 0 ? t[iidn[k]].offset : 0; }
-  return p;
+  if (plans_.size() >= 8) plans_.erase(plans_.begin());
+  plans_.push_back(p);
+  return plans_.back();
 }
 
-static Plan plan_of(const ConvLayer& stem, const std::vector<ResNet18::Block>& blocks, int dt, int N, int H, int W) {
-  std::vector<const ConvLayer*> c1s, c2s, dss;
-  for (const ResNet18::Block& b : blocks) { c1s.push_back(b.c1.get()); c2s.push_back(b.c2.get()); dss.push_back(b.ds.get()); }
-  NNCV_REQUIRE(c1s.size() == 8, "ResNet-18 has eight BasicBlocks");
-  return make_plan(stem, c1s, c2s, dss, dt, N, H, W);
-}
-
-size_t ResNet18::workspace_bytes(int N, int H, int W) const { return plan_of(*stem_, blocks_, dt_, N, H, W).total; }
+size_t ResNet18::workspace_bytes(int N, int H, int W) const { return plan_of(N, H, W).total; }
 
 void ResNet18::forward_body(const void* src, int N, int H, int W, void* ws, hipStream_t s, int tap_stage, void* tap) const {
   NNCV_REQUIRE(N > 0 && H >= 32 && W >= 32, "ResNet-18: input must be at least 32x32");
-  const Plan p = plan_of(*stem_, blocks_, dt_, N, H, W);
+  const Plan& p = plan_of(N, H, W);
   char* base = static_cast<char*>(ws);
   char* stem_out = base + p.stem_out;
   char* cws = base + p.cws;
@@ -394,7 +381,7 @@ void ResNet18::forward_body(const void* src, int N, int H, int W, void* ws, hipS
 }
 
 void ResNet18::forward_head(int N, int H, int W, void* logits, void* ws, hipStream_t s) const {
-  const Plan p = plan_of(*stem_, blocks_, dt_, N, H, W);
+  const Plan& p = plan_of(N, H, W);
   char* body_out = static_cast<char*>(ws) + p.x[8];
   char* pooled = static_cast<char*>(ws) + p.pooled;
   const int h = p.h_out, w = p.w_out;

@@ -90,10 +90,25 @@ class ResNet18 {
   };
 
  private:
+  // Workspace layout of one forward pass, planned with plan_offsets (arena_plan.hpp) from the
+  // tensors' sizes and the operator range over which each one is live.  Operator numbering: 0 stem
+  // convolution, 1 max-pool, then per BasicBlock k: 2+3k conv1, 3+3k shortcut conv, 4+3k conv2,
+  // 26 average pool, 27 FC.
+  struct Plan {
+    int N, H, W, linger;
+    int h1, w1, h2, w2, h_out, w_out;  // after stem, after maxpool, after the body
+    size_t stem_out, pooled, cws;      // offsets
+    size_t x[9];                       // x[k] = input of block k; x[8] = network body output
+    size_t y1[8], idn[8];
+    size_t total;
+  };
+  const Plan& plan_of(int N, int H, int W) const;
+
   int dt_;
   DevicePool pool_;
   std::unique_ptr<ConvLayer> stem_;
   std::vector<Block> blocks_;
+  mutable std::vector<Plan> plans_;  // of the last few sizes; callers hold the library's mutex
   DeviceBuffer fc_w_, fc_b_;  // [1000][512] dt ; [1000] f32
 };
 
