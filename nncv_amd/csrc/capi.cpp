@@ -1079,7 +1079,7 @@ nncv_hip_conv* nncv_hip_conv_create(int dtype, const void* weights, int F, int C
     const char* g = gamma ? blob.as<char>() + at(1) : nullptr;
     ConvLayer::Desc d;
     d.dt = dtype; d.C = C; d.F = F; d.R = R; d.S = S; d.stride = stride; d.pad = pad; d.relu = relu; d.algo = algo;
-    h = new nncv_hip_conv(4 * ((size_t)F + 64) * ((size_t)R * S * (C + 8) * es + 128) + (size_t(64) << 10));
+    h = new nncv_hip_conv(ConvLayer::device_bytes(d, gamma != nullptr));
     d.pool = &h->pool;
     try {
       h->c = std::make_unique<ConvLayer>(d, blob.get(), g, g ? g + row : nullptr, g ? g + 2 * row : nullptr, g ? g + 3 * row : nullptr, s);

@@ -257,6 +257,8 @@ void launch_image_pairs(const ImagePairsArgs& a, hipStream_t s);
 // Barrier-free implicit GEMM for fp32 layers and small fp16 layers (conv_direct.hip); `wins`: its modelled time against
 // that of the kernel which would run the layer otherwise.
 enum DirectRival : int { kRivalPatch = 0, kRivalPatchS2 = 1, kRivalIgemmFast = 2, kRivalIgemm = 3, kRivalShortK = 4, kRivalRing = 5 };
+// whether it is the kernel for a layer of F filters over RS taps of Cp channels at any size (else its order of the filters is not kept)
+bool conv_direct_serves(int dt, int F, int RS, int Cp);
 bool conv_direct_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 bool conv_direct_wins(const IgemmArgs& a, int dt, DirectRival rival);
 void launch_conv_direct(const IgemmArgs& a, int dt, hipStream_t s);

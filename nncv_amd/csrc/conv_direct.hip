@@ -460,6 +460,11 @@ void launch_weight_flat(const void* w_fcrs, void* dst, int dt, int F, int C, int
 // K values in memory order are the flat K axis: C = K channels of one tap
 void launch_weight_flat_rows(const void* w, void* dst, int dt, int F, int K, hipStream_t s) { launch_weight_flat(w, dst, dt, F, K, 1, K, s); }
 
+// fp16 1x1 layers of up to 64 channels have one round of K at most, which conv_pairs and one slab of the LDS ring do sooner at
+// every number of pixels: the models below never choose this kernel for them (88 combinations of channels and filters, one
+// pixel to a million).  Filter counts those kernels do not take, and every other layer, have sizes that come here.
+bool conv_direct_serves(int dt, int F, int RS, int Cp) { return dt != kF16 || RS > 1 || Cp > 64 || F % 8 != 0; }
+
 bool conv_direct_applicable(const IgemmArgs& a, int in_dt, int out_dt) {
   const int es = (int)dtype_size(in_dt), pix = a.pix_stride ? a.pix_stride : a.C;
   const long long P = (long long)a.N * a.OH * a.OW, k = (long long)a.R * a.S * a.C, lim = 1 << 24;  // fast_div's range

@@ -146,8 +146,6 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
         take(i, &Node::wt, (size_t)Cstored * op.K * op.K * C * es);
         if (Cstored > op.F) NNCV_HIP_CHECK(hipMemsetAsync(nd.wt.get(), 0, (size_t)Cstored * op.K * op.K * C * es, s));
         launch_weight_frsc(w, dt, nd.wt.get(), dt, op.F, Cl, op.K, op.K, C, s);
-        nd.wflat.reset(weight_flat_bytes(dt, Cstored, op.K * op.K, C), &pool_);
-        launch_weight_flat(w, nd.wflat.get(), dt, op.F, Cl, op.K * op.K, C, s);
         if (op.K == 3 && (op.stride == 1 || (op.stride == 2 && dt == kF16)) && op.pad == 1 && Cl == C && Cstored == op.F && C % (128 / (int)es) == 0) {
           nd.wfrag.reset((size_t)((op.F + 63) / 64) * 64 * 9 * C * es, &pool_);
           launch_weight_frag3x3(w, dt, nd.wfrag.get(), dt, op.F, C, s);
@@ -320,6 +318,18 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
         }
       }
     }
+  }
+
+  // The filters in conv_direct.hip's order, for the layers that may run there, and for projections (mobile_block.hip).  The two
+  // vectors of a squeeze-excitation block are never convolutions of their own.
+  for (int i = 0; i < n && !dry_; ++i) {
+    const GraphOp& o = ops[i];
+    const bool projection = i >= 4 && nodes_[i - 4].projects == i;
+    if (o.kind != NNCV_HIP_OP_CONV || nodes_[i].skip) continue;
+    const int C = nodes_[i].C, Fs = channels_[o.out];
+    if (!projection && !conv_direct_serves(dt, Fs, o.K * o.K, C)) continue;
+    nodes_[i].wflat.reset(weight_flat_bytes(dt, Fs, o.K * o.K, C), &pool_);
+    launch_weight_flat(blob + (size_t)o.w * es, nodes_[i].wflat.get(), dt, o.F, logical_[o.in[0]], o.K * o.K, C, s);
   }
 
   for (int i = 0; i < n; ++i) {  // what rides in another launch, or carries one, does not join

@@ -16,14 +16,8 @@ static int env_algo3x3() {
 
 static int round_up(int v, int m) { return (v + m - 1) / m * m; }
 
-ConvLayer::ConvLayer(const Desc& d, const void* w, const void* gamma, const void* beta, const void* mean, const void* var,
-                     hipStream_t s)
-    : d_(d) {
-  NNCV_REQUIRE(d.dt == kF32 || d.dt == kF16, "conv: dtype must be f32 or f16");
-  NNCV_REQUIRE(d.C > 0 && d.F > 0 && d.R > 0 && d.S > 0 && d.stride > 0 && d.pad >= 0, "conv: bad geometry");
-  NNCV_REQUIRE(d.relu >= kActNone && d.relu <= kActSigmoid, "conv: unknown activation");
+int ConvLayer::pick_algo(const Desc& d) {
   const int ce = d.dt == kF16 ? 8 : 4;
-  const size_t es = dtype_size(d.dt);
   const bool wino_ok = !d.stem && d.relu <= kActRelu && d.R == 3 && d.S == 3 && d.stride == 1 && d.C % ce == 0 && d.F % 4 == 0;
   int algo = d.algo;
   if (algo == kAlgoAuto) algo = env_algo3x3();
@@ -44,41 +38,72 @@ ConvLayer::ConvLayer(const Desc& d, const void* w, const void* gamma, const void
     }
     algo = kAlgoIgemm;
   }
-  algo_ = algo;
+  return algo;
+}
 
+ConvLayer::Sizes ConvLayer::sizes(const Desc& d, int algo, bool bn) {
+  const size_t es = dtype_size(d.dt);
+  const int Cp = round_up(d.C, d.dt == kF16 ? 8 : 4), Fp = round_up(d.F, 4), RS = d.R * d.S;
+  Sizes z{};
   if (d.stem) {
-    NNCV_REQUIRE(d.C == 3 && d.R == 7 && d.S == 7 && d.stride == 2 && d.pad == 3, "stem: must be 7x7 s2 p3 over 3 channels");
-    NNCV_REQUIRE(d.F % 4 == 0, "stem: F must be a multiple of 4");
-    wt_.reset((size_t)d.F * 224 * es, d.pool);
-    launch_stem_weight(w, d.dt, wt_.get(), d.dt, d.F, 0, s);
-    wflat_.reset(weight_flat_bytes(d.dt, d.F, 7, 32), d.pool);
-    launch_weight_flat_rows(wt_.get(), wflat_.get(), d.dt, d.F, 224, s);
-    wt_shift_.reset((size_t)d.F * 224 * es, d.pool);  // pairs start one column further left (fused stem)
-    launch_stem_weight(w, d.dt, wt_shift_.get(), d.dt, d.F, 1, s);
-  } else if (algo_ == kAlgoWinograd) {
-    U_.reset((size_t)36 * d.F * d.C * es, d.pool);
-    launch_wino43_filter(w, d.dt, U_.get(), d.dt, d.F, d.C, s);
+    z.wt = z.wt_shift = (size_t)d.F * 224 * es;
+    z.wflat = weight_flat_bytes(d.dt, d.F, 7, 32);
+  } else if (algo == kAlgoWinograd) {
+    z.U = (size_t)36 * d.F * d.C * es;
   } else {
-    const int Cp = round_up(d.C, ce), Fp = round_up(d.F, 4);
-    wt_.reset((size_t)Fp * d.R * d.S * Cp * es, d.pool);
-    if (Fp > d.F) NNCV_HIP_CHECK(hipMemsetAsync(wt_.get(), 0, wt_.bytes(), s));  // padding filters; padding channels are written
-    launch_weight_frsc(w, d.dt, wt_.get(), d.dt, d.F, d.C, d.R, d.S, Cp, s);
-    wflat_.reset(weight_flat_bytes(d.dt, Fp, d.R * d.S, Cp), d.pool);
-    launch_weight_flat(w, wflat_.get(), d.dt, d.F, d.C, d.R * d.S, Cp, s);
+    z.wt = (size_t)Fp * RS * Cp * es;
+    if (d.shortcut || conv_direct_serves(d.dt, Fp, RS, Cp)) z.wflat = weight_flat_bytes(d.dt, Fp, RS, Cp);
     if (d.R == 3 && d.S == 3 && (d.stride == 1 || (d.stride == 2 && d.dt == kF16)) && d.pad == 1 && d.C % (128 / (int)es) == 0) {
-      wfrag_.reset((size_t)((d.F + 63) / 64) * 64 * 9 * d.C * es, d.pool);
-      launch_weight_frag3x3(w, d.dt, wfrag_.get(), d.dt, d.F, d.C, s);
-      if (d.dt == kF16 && d.stride == 1 && d.C % 64 == 0 && d.F % 32 == 0) {
-        wfrag32_.reset(weight_frag32_bytes(d.F, d.C), d.pool);
-        launch_weight_frag32(w, d.dt, wfrag32_.get(), d.F, d.C, s);
-      }
+      z.wfrag = (size_t)((d.F + 63) / 64) * 64 * 9 * d.C * es;
+      if (d.dt == kF16 && d.stride == 1 && d.C % 64 == 0 && d.F % 32 == 0) z.wfrag32 = weight_frag32_bytes(d.F, d.C);
     }
   }
+  if (bn) z.scale = (size_t)Fp * 4;
+  return z;
+}
+
+size_t ConvLayer::device_bytes(const Desc& d, bool bn) {
+  const Sizes z = sizes(d, pick_algo(d), bn);
+  size_t total = 0;
+  for (const size_t b : {z.wt, z.wflat, z.wfrag, z.wfrag32, z.U, z.wt_shift, z.scale, z.scale}) total += align256(b);
+  return total;
+}
+
+ConvLayer::ConvLayer(const Desc& d, const void* w, const void* gamma, const void* beta, const void* mean, const void* var,
+                     hipStream_t s)
+    : d_(d) {
+  NNCV_REQUIRE(d.dt == kF32 || d.dt == kF16, "conv: dtype must be f32 or f16");
+  NNCV_REQUIRE(d.C > 0 && d.F > 0 && d.R > 0 && d.S > 0 && d.stride > 0 && d.pad >= 0, "conv: bad geometry");
+  NNCV_REQUIRE(d.relu >= kActNone && d.relu <= kActSigmoid, "conv: unknown activation");
+  NNCV_REQUIRE(!d.stem || (d.C == 3 && d.R == 7 && d.S == 7 && d.stride == 2 && d.pad == 3), "stem: must be 7x7 s2 p3 over 3 channels");
+  NNCV_REQUIRE(!d.stem || d.F % 4 == 0, "stem: F must be a multiple of 4");
+  NNCV_REQUIRE(!gamma || (beta && mean && var), "conv: BN needs gamma, beta, mean and var");
+  algo_ = pick_algo(d);
+  const Sizes z = sizes(d, algo_, gamma != nullptr);
+  wt_.reset(z.wt, d.pool);
+  wflat_.reset(z.wflat, d.pool);
+  wfrag_.reset(z.wfrag, d.pool);
+  wfrag32_.reset(z.wfrag32, d.pool);
+  U_.reset(z.U, d.pool);
+  wt_shift_.reset(z.wt_shift, d.pool);
+  scale_.reset(z.scale, d.pool);
+  shift_.reset(z.scale, d.pool);
+
+  const int Cp = round_up(d.C, d.dt == kF16 ? 8 : 4), Fp = round_up(d.F, 4);
+  if (d.stem) {
+    launch_stem_weight(w, d.dt, wt_.get(), d.dt, d.F, 0, s);
+    launch_weight_flat_rows(wt_.get(), wflat_.get(), d.dt, d.F, 224, s);
+    launch_stem_weight(w, d.dt, wt_shift_.get(), d.dt, d.F, 1, s);  // pairs start one column further left (fused stem)
+  } else if (algo_ == kAlgoWinograd) {
+    launch_wino43_filter(w, d.dt, U_.get(), d.dt, d.F, d.C, s);
+  } else {
+    if (Fp > d.F) NNCV_HIP_CHECK(hipMemsetAsync(wt_.get(), 0, wt_.bytes(), s));  // padding filters; padding channels are written
+    launch_weight_frsc(w, d.dt, wt_.get(), d.dt, d.F, d.C, d.R, d.S, Cp, s);
+    if (z.wflat) launch_weight_flat(w, wflat_.get(), d.dt, d.F, d.C, d.R * d.S, Cp, s);
+    if (z.wfrag) launch_weight_frag3x3(w, d.dt, wfrag_.get(), d.dt, d.F, d.C, s);
+    if (z.wfrag32) launch_weight_frag32(w, d.dt, wfrag32_.get(), d.F, d.C, s);
+  }
   if (gamma) {
-    NNCV_REQUIRE(beta && mean && var, "conv: BN needs gamma, beta, mean and var");
-    const int Fp = round_up(d.F, 4);
-    scale_.reset((size_t)Fp * 4, d.pool);
-    shift_.reset((size_t)Fp * 4, d.pool);
     launch_fill_f32(scale_.as<float>(), 0.0f, Fp, s);
     launch_fill_f32(shift_.as<float>(), 0.0f, Fp, s);
     launch_bn_fold(gamma, beta, mean, var, d.dt, scale_.as<float>(), shift_.as<float>(), d.F, s);
@@ -253,6 +278,7 @@ ResNet18::ResNet18(const void* params, long long n_elems, int dt, int algo3x3, h
     ConvLayer::Desc d;
     d.dt = dt; d.C = C; d.F = F; d.R = d.S = R; d.stride = stride; d.pad = pad; d.relu = relu; d.stem = stem;
     d.algo = (R == 3 && stride == 1) ? algo3x3 : kAlgoIgemm;
+    d.shortcut = R == 1;
     d.pool = &pool_;
     const void* w = take((long long)F * C * R * R);
     const void* g = take(F); const void* b = take(F); const void* m = take(F); const void* v = take(F);

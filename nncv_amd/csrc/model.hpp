@@ -12,8 +12,9 @@ enum ConvAlgo : int { kAlgoAuto = 0, kAlgoWinograd = 1, kAlgoIgemm = 2 };
 
 // linalg.conv_2d_nchw_fchw + BatchNorm + (residual add) + ReLU as one device operation.
 // Weights arrive in the reference's FCHW order; they are re-laid once at creation:
-//   igemm    : [F][R][S][C]   (K = (r,s,c) contiguous per filter); 3x3 stride-1 layers also keep
-//              a fragment-major copy for the LDS-patch kernel (conv3x3_patch.hip)
+//   igemm    : [F][R][S][C]   (K = (r,s,c) contiguous per filter), the same in conv_direct.hip's order
+//              where that kernel can be the one for a layer (conv_direct_serves), and for 3x3 layers
+//              fragment-major copies for the LDS-patch and the stream kernel (conv3x3_patch.hip, conv3x3_f16.hip)
 //   winograd : U[36][F][C]    (filter transform done here, like the reference folds it at
 //                              compile time, OptimizeConv2dUsingWinograd.cpp:106-150)
 class ConvLayer {
@@ -24,8 +25,11 @@ class ConvLayer {
     int relu = 0;  // activation applied last (enum Act); 1 = ReLU
     int algo = kAlgoAuto;
     DevicePool* pool = nullptr;  // where the weights live (it outlives the layer); null = allocations of their own
+    bool shortcut = false;  // 1x1 layer whose filters another layer's launches may read (fuse_shortcut)
     bool stem = false;  // 7x7 s2 p3 over 3 channels read from NCHW (pixel-pair packing)
   };
+  // bytes of everything a layer keeps on the device, in pieces as a DevicePool hands them out
+  static size_t device_bytes(const Desc& d, bool bn);
   // w: device pointer to FCHW weights of type `dt`; bn: device pointers gamma,beta,mean,var of
   // type `dt` (all null -> no scale/shift).
   ConvLayer(const Desc& d, const void* w_dev, const void* gamma, const void* beta, const void* mean, const void* var,
@@ -54,6 +58,11 @@ class ConvLayer {
   void forward_with_shortcut(const void* in, int N, int H, int W, void* out, void* shortcut_out, void* ws, hipStream_t s) const;
 
  private:
+  // bytes of each array a layer keeps, 0: not kept
+  struct Sizes { size_t wt, wflat, wfrag, wfrag32, U, wt_shift, scale; };
+  static Sizes sizes(const Desc& d, int algo, bool bn);
+  static int pick_algo(const Desc& d);
+
   Desc d_;
   int algo_;
   DeviceBuffer wt_, wfrag_, wfrag32_, wflat_, U_, scale_, shift_, wt_shift_;
