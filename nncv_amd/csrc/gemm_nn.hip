@@ -357,15 +357,16 @@ struct GemmForm {
   int rows, cols;
   double fixed_us, k_us, tile_us;
   void (*launch)(const float*, const float*, const float*, float*, int, int, int, const RideCopy&, hipStream_t);
+  const char* tag;
 };
 const GemmForm kForms[] = {
-    {128, 128, 5.7, 0.00367, 9.0, launch_gemm_cfg<32, 2, 2, 2, 2, 1>},
-    {64, 128, 0.0, 0.00377, 5.3, launch_gemm_cfg<32, 1, 2, 2, 2, 2>},
-    {32, 64, 2.3, 0.00407, 1.0, launch_gemm_cfg<32, 1, 2, 1, 1, 4>},
-    {32, 32, 2.4, 0.00477, 0.56, launch_gemm_cfg<32, 1, 1, 1, 1, 4>},
-    {32, 32, 2.1, 0.00440, 1.2, launch_gemm_cfg<32, 1, 1, 1, 1, 8>},
-    {16, 32, 2.95, 0.00623, 0.13, launch_gemm_cfg<16, 1, 2, 1, 1, 4>},
-    {16, 16, 2.95, 0.00847, 0.11, launch_gemm_cfg<16, 1, 1, 1, 1, 4>},
+    {128, 128, 5.7, 0.00367, 9.0, launch_gemm_cfg<32, 2, 2, 2, 2, 1>, "gemm_nn_f32<128x128>"},
+    {64, 128, 0.0, 0.00377, 5.3, launch_gemm_cfg<32, 1, 2, 2, 2, 2>, "gemm_nn_f32<64x128,splitk2>"},
+    {32, 64, 2.3, 0.00407, 1.0, launch_gemm_cfg<32, 1, 2, 1, 1, 4>, "gemm_nn_f32<32x64,splitk4>"},
+    {32, 32, 2.4, 0.00477, 0.56, launch_gemm_cfg<32, 1, 1, 1, 1, 4>, "gemm_nn_f32<32x32,splitk4>"},
+    {32, 32, 2.1, 0.00440, 1.2, launch_gemm_cfg<32, 1, 1, 1, 1, 8>, "gemm_nn_f32<32x32,splitk8>"},
+    {16, 32, 2.95, 0.00623, 0.13, launch_gemm_cfg<16, 1, 2, 1, 1, 4>, "gemm_nn_f32<16x32,splitk4>"},
+    {16, 16, 2.95, 0.00847, 0.11, launch_gemm_cfg<16, 1, 1, 1, 1, 4>, "gemm_nn_f32<16x16,splitk4>"},
 };
 
 }  // namespace
@@ -378,10 +379,11 @@ void launch_copy16(const RideCopy& r, hipStream_t s) {
 
 void launch_gemm_nn_f32(const float* A, const float* B, const float* C, float* D, int M, int N, int K, hipStream_t s, const RideCopy* ride) {
   NNCV_REQUIRE(M > 0 && N > 0 && K > 0, "matmul: empty operand");
-  ProfScope prof("gemm_nn_f32", 2.0 * M * N * K, 4.0 * ((double)M * K + (double)K * N + 2.0 * M * N), s);
+  const double flops = 2.0 * M * N * K, bytes = 4.0 * ((double)M * K + (double)K * N + 2.0 * M * N);
   if (ride && ride->bytes) {
     if (N < 1 << 24 && K < 1 << 24) {
       // one form only: these launches are bands of a product whose operands arrive over the bus
+      ProfScope prof("gemm_nn_f32<32x64,splitk4,ride>", flops, bytes, s);
       launch_gemm_cfg<32, 1, 2, 1, 1, 4, true>(A, B, C, D, M, N, K, *ride, s);
       NNCV_HIP_CHECK(hipGetLastError());
       return;
@@ -390,6 +392,7 @@ void launch_gemm_nn_f32(const float* A, const float* B, const float* C, float* D
   }
   if (N >= 1 << 24 || K >= 1 << 24) {  // 64 rows of A or 32 of B beyond 32-bit byte offsets
     const long long blocks = ((long long)M * N + 255) / 256;
+    ProfScope prof("gemm_nn_f32<any>", flops, bytes, s);
     launch_kernel(gemm_nn_f32_any_kernel, dim3((unsigned)std::min(blocks, 1ll << 20)), dim3(256), 0, s, A, B, C, D, M, N, K);
     NNCV_HIP_CHECK(hipGetLastError());
     return;
@@ -401,6 +404,7 @@ void launch_gemm_nn_f32(const float* A, const float* B, const float* C, float* D
     const double us = f.fixed_us + (double)rounds * (f.k_us * (f.rows * f.cols / 1024.0) * ((K + 31) / 32 * 32) + f.tile_us);
     if (!best || us < best_us) best = &f, best_us = us;
   }
+  ProfScope prof(best->tag, flops, bytes, s);
   best->launch(A, B, C, D, M, N, K, RideCopy{}, s);
   NNCV_HIP_CHECK(hipGetLastError());
 }

@@ -103,12 +103,32 @@ def test_matmul_k_groups_are_deterministic():
     assert np.array_equal(outs[0], outs[1])
 
 
-# one shape for every form the dispatch can pick (tiles 16x16 ... 128x128, K groups or none) with every dimension one off a
-# tile or a 32-wide K round, fewer rounds than K groups, and rows too long for 32-bit offsets; one row of A holds infinities
-# and the K tail reads past row ends, so nothing of a neighbouring row may reach a result
+# every dimension one off a tile or a 32-wide K round, fewer rounds than K groups, and rows too long for 32-bit offsets; one
+# row of A holds infinities and the K tail reads past row ends, so nothing of a neighbouring row may reach a result
 @pytest.mark.parametrize("M,N,K", [(15, 31, 4097), (129, 33, 31), (63, 470, 33), (1025, 260, 65), (65, 4001, 95), (31, 2999, 1001),
                                    (1400, 999, 129), (513, 2049, 1063), (2300, 2190, 33), (3000, 2945, 161), (2, 3, (1 << 24) + 3)])
 def test_matmul_forms_and_tails(M, N, K):
+    check_product(M, N, K)
+
+
+# one shape or two for every form of the kernel, M and N one off a tile and K one off a round of 32, on either side
+@pytest.mark.parametrize("M,N,K,form", [
+    (17, 17, 129, "16x16,splitk4"), (17, 17, 127, "16x16,splitk4"), (207, 353, 129, "16x32,splitk4"), (49, 1087, 191, "16x32,splitk4"),
+    (1377, 97, 65, "32x32,splitk4"), (1471, 97, 63, "32x32,splitk4"), (481, 289, 2655, "32x32,splitk8"), (383, 511, 3329, "32x32,splitk8"),
+    (705, 447, 129, "32x64,splitk4"), (2079, 127, 191, "32x64,splitk4"), (2559, 641, 33, "64x128,splitk2"), (2559, 641, 63, "64x128,splitk2"),
+    (4095, 4095, 321, "128x128"), (4095, 4095, 351, "128x128")])
+def test_matmul_every_form(M, N, K, form):
+    abi.profile_enable(True)
+    try:
+        abi.profile_report()
+        check_product(M, N, K)
+        tags = list(abi.profile_report())
+    finally:
+        abi.profile_enable(False)
+    assert tags == ["gemm_nn_f32<%s>" % form]
+
+
+def check_product(M, N, K):
     g = torch.Generator().manual_seed(M + N + K)
     a = torch.rand((M, K), generator=g) * 2 - 1
     b = torch.rand((K, N), generator=g) * 2 - 1
