@@ -367,9 +367,13 @@ bool conv_ring_applicable(const IgemmArgs& a, int in_dt, int out_dt) {
          P * a.ldo * 2 < (long long)kOOBr && ((P + 63) / 64) * ((a.F + 31) / 32) < lim && (a.relu & ~(0xff | kActResidualAfter)) == 0;
 }
 
-// Stride-2 3x3 layers leave the patch kernel where 128 x 128 tiles keep three quarters of the CUs busy: it is bound by its
-// patch reads (64x56x56x64 -> 128: 18.4 -> 14.7 us, 256x28x28x128 -> 256 with its shortcut 59.9 -> 47.7), while below that its
-// smaller tiles and K groups fill the chip better (32x28x28x128 -> 256: 9.1 against 10.6).
+// Stride-2 3x3 layers leave the patch kernel where 128 x 128 tiles keep three quarters of the CUs busy.  From 200 tiles to the
+// patch kernel's limit (8 GFLOP) that kernel is bound by its patch reads: 48x56x56x64 -> 128 14.3 against 13.3 us here, 64
+// images 17.4 against 14.1, 32x40x40x128 -> 256 20.0 against 15.9, 16x80x80x64 -> 128 10.2 against 10.3 at 200 tiles.  Below, its
+// smaller tiles and K groups mostly fill the chip better (32x28x28x128 -> 256, 98 tiles: 9.1 against 11.6; 24x40x40x128 -> 256,
+// 150 tiles, is the other way round: 16.5 against 15.1).  Larger launches used to be igemm_fast's: 23 of them take 1.14 to 1.35
+// times as long there (256x28x28x128 -> 256: 52.2 against 42.0).  In a ResNet-18 pass of 256 images the three such layers with
+// their shortcuts went from 78.1 + 58.4 + 52.2 us there to 65.4 + 46.6 + 43.6, the pass from 1162 to 1133 us of launches.
 bool conv_ring_beats_patch_s2(const IgemmArgs& a) {
   const long long P = (long long)a.N * a.OH * a.OW, main_f = a.aux_f0 ? a.aux_f0 : a.F;
   return a.stride_h == 2 && (P + 127) / 128 * ((main_f + 127) / 128) >= 200;
