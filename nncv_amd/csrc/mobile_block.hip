@@ -422,8 +422,6 @@ void launch_dw_block(const DwBlockArgs& args, hipStream_t s) {
   a.rows = p.rows; a.bands = p.bands; a.pitch = p.pitch; a.cells = p.cells;
   a.inv_w = 1.0f / (float)a.W;
   const double px_in = (double)a.N * a.H * a.W, px_out = (double)a.N * a.OH * a.OW;
-  ProfScope prof(a.Cin ? "dw_block<expand>" : "dw_block", 2.0 * px_out * a.C * a.K * a.K + 2.0 * px_in * a.C * a.Cin,
-                 2.0 * (px_in * (a.Cin ? a.Cin : a.C) + px_out * a.C + a.C * (a.K * a.K + a.Cin)), s);
   // Outputs a thread takes at a time, by the clocks that eight waves of a CU need for a round of them: LDS reads (a row of
   // taps and of pixels per filter row, shared by all) or multiply-adds (two waves a SIMD).  More share their operands, fewer
   // leave no thread of the last round idle.
@@ -435,6 +433,11 @@ void launch_dw_block(const DwBlockArgs& args, hipStream_t s) {
   for (int o : {2, 4})
     if (clocks(o) < clocks(oxt)) oxt = o;
   a.inv_strips = 1.0f / (float)((a.OW + oxt - 1) / oxt);
+  const int steps16 = (a.Cin + 15) / 16, kst = steps16 <= 1 ? steps16 : steps16 <= 3 ? 3 : 6;  // K steps of the expansion that are unrolled
+  char tag[40];
+  snprintf(tag, sizeof tag, "dw_block<%d,%d,%d,%d>", a.K, a.stride, oxt, kst);
+  ProfScope prof(tag, 2.0 * px_out * a.C * a.K * a.K + 2.0 * px_in * a.C * a.Cin,
+                 2.0 * (px_in * (a.Cin ? a.Cin : a.C) + px_out * a.C + a.C * (a.K * a.K + a.Cin)), s);
   const unsigned grid = (unsigned)((a.C + 31) / 32 * a.bands * a.N);
   const size_t lds = (size_t)a.cells * 64 + a.K * a.K * 64;
   auto go = [&](auto kern) {
@@ -447,10 +450,9 @@ void launch_dw_block(const DwBlockArgs& args, hipStream_t s) {
   };
   auto steps = [&](auto k, auto st, auto ox) {
     constexpr int K = decltype(k)::value, S = decltype(st)::value, OXT = decltype(ox)::value;
-    const int kst = (a.Cin + 15) / 16;
     if (kst == 0) go(dw_block_kernel<K, S, OXT, 0>);
     else if (kst == 1) go(dw_block_kernel<K, S, OXT, 1>);
-    else if (kst <= 3) go(dw_block_kernel<K, S, OXT, 3>);
+    else if (kst == 3) go(dw_block_kernel<K, S, OXT, 3>);
     else go(dw_block_kernel<K, S, OXT, 6>);
   };
   auto strips = [&](auto k, auto st) {

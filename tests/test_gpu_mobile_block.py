@@ -17,6 +17,49 @@ pytestmark = pytest.mark.gpu
     (32, 104, 56, 3, 1, 16, 130, 9, 9), (16, 64, 16, 5, 1, 16, 1, 6, 700)])
 def test_inverted_residual_block(case):
     cin, exp, cout, K, stride, sq, N, H, W = case
+    tags = check_block(case)
+    merged = exp != cin or sq > 0
+    assert sum(v for k, v in tags.items() if k.startswith("dw_block")) == int(merged and W < 700), tags
+    assert tags.get("se_project", 0) == int(sq > 0 and W < 700), tags
+
+
+# every instance of the depthwise kernel (window, stride, outputs a thread takes at a time, 16-channel steps of the expansion), and
+# between them every instance of the projection: one, two or three slices of 256 channels, 16, 48 or 96 filters, 16 or
+# 32 pixels a tile, and expanded tensors of up to 32 channels
+EVERY = [
+    (24, 24, 8, 3, 1, 200, 2, 6, 7, "3,1,1,0"), (8, 40, 56, 3, 1, 40, 70, 15, 15, "3,1,1,1"), (8, 40, 24, 3, 1, 136, 70, 19, 12, "3,1,1,1"),
+    (8, 40, 24, 3, 1, 136, 2, 7, 6, "3,1,1,1"), (32, 24, 8, 3, 1, 8, 3, 7, 6, "3,1,1,3"), (72, 24, 8, 3, 1, 40, 2, 6, 9, "3,1,1,6"),
+    (24, 24, 8, 3, 1, 40, 2, 6, 27, "3,1,2,0"), (8, 520, 8, 3, 1, 40, 70, 13, 18, "3,1,2,1"), (8, 264, 8, 3, 1, 24, 70, 11, 21, "3,1,2,1"),
+    (8, 40, 8, 3, 1, 8, 40, 15, 27, "3,1,2,1"), (32, 24, 8, 3, 1, 136, 2, 6, 25, "3,1,2,3"), (72, 24, 16, 3, 1, 72, 2, 6, 22, "3,1,2,6"),
+    (24, 24, 8, 3, 1, 40, 2, 7, 37, "3,1,4,0"), (8, 520, 56, 3, 1, 256, 70, 6, 39, "3,1,4,1"), (8, 520, 24, 3, 1, 256, 40, 14, 30, "3,1,4,1"),
+    (8, 264, 56, 3, 1, 8, 40, 16, 26, "3,1,4,1"), (8, 264, 24, 3, 1, 24, 40, 31, 13, "3,1,4,1"), (32, 24, 16, 3, 1, 200, 2, 8, 35, "3,1,4,3"),
+    (72, 24, 24, 3, 1, 8, 2, 7, 34, "3,1,4,6"), (24, 24, 24, 3, 2, 40, 2, 6, 6, "3,2,1,0"), (8, 520, 56, 3, 2, 24, 2, 7, 7, "3,2,1,1"),
+    (8, 520, 24, 3, 2, 200, 2, 6, 7, "3,2,1,1"), (8, 264, 56, 3, 2, 40, 2, 6, 7, "3,2,1,1"), (16, 584, 8, 3, 2, 40, 2, 6, 6, "3,2,1,1"),
+    (8, 264, 24, 3, 2, 200, 2, 6, 7, "3,2,1,1"), (8, 264, 8, 3, 2, 40, 3, 6, 7, "3,2,1,1"), (16, 40, 56, 3, 2, 256, 2, 6, 6, "3,2,1,1"),
+    (8, 24, 56, 3, 2, 8, 2, 6, 7, "3,2,1,1"), (8, 40, 16, 3, 2, 24, 2, 6, 7, "3,2,1,1"), (32, 24, 16, 3, 2, 136, 2, 6, 7, "3,2,1,3"),
+    (56, 24, 16, 3, 2, 136, 2, 7, 7, "3,2,1,6"), (24, 24, 8, 3, 2, 24, 2, 7, 37, "3,2,2,0"), (16, 24, 16, 3, 2, 8, 2, 7, 33, "3,2,2,1"),
+    (32, 24, 8, 3, 2, 40, 2, 7, 34, "3,2,2,3"), (56, 24, 8, 3, 2, 256, 2, 8, 33, "3,2,2,6"), (24, 24, 8, 3, 2, 24, 1, 3, 260, "3,2,4,0"),
+    (8, 24, 8, 3, 2, 40, 1, 3, 259, "3,2,4,1"), (32, 24, 8, 3, 2, 200, 1, 3, 284, "3,2,4,3"), (56, 24, 8, 3, 2, 24, 1, 3, 272, "3,2,4,6"),
+    (24, 24, 16, 5, 1, 24, 2, 7, 6, "5,1,1,0"), (8, 24, 8, 5, 1, 8, 2, 6, 7, "5,1,1,1"), (32, 24, 16, 5, 1, 256, 2, 6, 6, "5,1,1,3"),
+    (72, 24, 8, 5, 1, 200, 2, 6, 6, "5,1,1,6"), (24, 24, 24, 5, 1, 24, 2, 8, 18, "5,1,2,0"), (8, 24, 8, 5, 1, 136, 2, 7, 18, "5,1,2,1"),
+    (32, 24, 8, 5, 1, 40, 2, 7, 17, "5,1,2,3"), (72, 24, 8, 5, 1, 256, 2, 7, 17, "5,1,2,6"), (24, 24, 16, 5, 1, 8, 2, 7, 34, "5,1,4,0"),
+    (8, 24, 8, 5, 1, 136, 2, 7, 40, "5,1,4,1"), (40, 24, 16, 5, 1, 200, 2, 7, 34, "5,1,4,3"), (88, 24, 16, 5, 1, 72, 2, 7, 34, "5,1,4,6"),
+    (24, 24, 8, 5, 2, 136, 2, 6, 6, "5,2,1,0"), (8, 24, 8, 5, 2, 8, 2, 6, 8, "5,2,1,1"), (32, 24, 48, 5, 2, 72, 2, 6, 6, "5,2,1,3"),
+    (56, 24, 24, 5, 2, 40, 2, 8, 8, "5,2,1,6"), (24, 24, 16, 5, 2, 24, 2, 7, 33, "5,2,2,0"), (8, 24, 16, 5, 2, 24, 2, 7, 39, "5,2,2,1"),
+    (32, 24, 8, 5, 2, 136, 2, 7, 39, "5,2,2,3"), (56, 24, 16, 5, 2, 200, 2, 8, 33, "5,2,2,6"), (24, 24, 8, 5, 2, 40, 1, 3, 267, "5,2,4,0"),
+    (8, 24, 8, 5, 2, 200, 1, 3, 267, "5,2,4,1"), (32, 24, 8, 5, 2, 72, 1, 3, 270, "5,2,4,3"), (56, 24, 16, 5, 2, 72, 1, 3, 263, "5,2,4,6"),
+]
+
+
+@pytest.mark.parametrize("case", EVERY, ids=lambda c: "-".join(map(str, c)))
+def test_every_instance(case):
+    tags = check_block(case[:9])
+    assert tags.get("dw_block<%s>" % case[9]) == 1 and tags.get("se_project") == 1, tags
+
+
+def check_block(case):
+    """The block against the oracle's evaluator; launches by tag."""
+    cin, exp, cout, K, stride, sq, N, H, W = case
     sizes, ops = [], []
 
     def take(n):
@@ -64,9 +107,7 @@ def test_inverted_residual_block(case):
     finally:
         abi.profile_enable(False)
     print(case, tags, flush=True)
-    merged = exp != cin or sq > 0
-    assert sum(v for k, v in tags.items() if k.startswith("dw_block")) == int(merged and W < 700), tags
-    assert tags.get("se_project", 0) == int(sq > 0 and W < 700), tags
     want = oracle.run_graph(ops, x, blob, cin)
     assert rel_l2(got, want) < 3e-3 < FP16_REL_L2
     g.close()
+    return tags
