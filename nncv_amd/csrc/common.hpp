@@ -41,13 +41,14 @@ struct Error : std::runtime_error {
 
 // ---------------------------------------------------------------------------------------------
 // Launches.  A call that leaves work in flight for a later call on another stream to wait for (StreamOrder, runtime.hpp)
-// has its launches complete an event of their own: the last one's end is the call's.  That costs the queue nothing behind
-// a kernel of 13 us and 0.9 us behind one of 3, where an event recorded behind the launch costs 2.8 between two kernels
-// and 4.9 behind a replayed graph.  Every launch of the library goes through here, so that none can come after the event.
+// has its last launch complete an event.  That costs the queue nothing behind a kernel of 13 us or more, where an event
+// recorded behind the launch costs 2.8 us between two kernels and 4.9 behind a replayed graph; the host pays 1-3 us for
+// it.  Every launch of the library goes through here, so that none can come after the event.
 // ---------------------------------------------------------------------------------------------
 struct TailEvent {
   hipEvent_t event;
-  bool bound;  // a launch completes it
+  int skip;    // launches of this call that are known not to be its last
+  bool bound;  // a launch completes the event
 };
 TailEvent*& tail_event();  // of this thread's current call; null: launches complete nothing (capi.cpp)
 
@@ -56,6 +57,7 @@ template <typename Args, size_t... I>
 void launch_with(const void* kernel, dim3 grid, dim3 block, size_t lds, hipStream_t s, Args& args, std::index_sequence<I...>) {
   void* ptrs[] = {static_cast<void*>(&std::get<I>(args))...};
   TailEvent* tail = tail_event();
+  if (tail && tail->skip > 0) --tail->skip, tail = nullptr;
   if (tail) tail->bound = true;
   NNCV_HIP_CHECK(tail ? hipExtLaunchKernel(kernel, grid, block, ptrs, lds, s, nullptr, tail->event, 0)
                       : hipLaunchKernel(kernel, grid, block, ptrs, lds, s));

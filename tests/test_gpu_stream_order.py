@@ -180,3 +180,18 @@ def test_a_chain_of_layers_over_streams_without_waits(layout):
         b.zero_()
     torch.cuda.synchronize()
     assert torch.equal(chain([torch.cuda.Stream().cuda_stream for _ in range(4)]), want)
+
+
+@pytest.mark.parametrize("M,N,K", [(20, 30, 40), (700, 500, 64)])
+def test_products_accumulate_over_streams(M, N, K):
+    """C += A.B over and over, each call on another stream than the one before: every call reads what the previous one wrote, from
+    other compute units and caches than those that wrote it.  Whole numbers, so the sum is exact."""
+    g = torch.Generator().manual_seed(7)
+    a, b = (torch.randint(-3, 4, s, generator=g).float().cuda() for s in ((M, K), (K, N)))
+    c = torch.zeros((M, N), device="cuda")
+    streams = [torch.cuda.Stream().cuda_stream for _ in range(3)]
+    torch.cuda.synchronize()
+    for k in range(600):
+        abi.check(abi.lib().nncv_hip_matmul_f32(a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, streams[k % 3]))
+    torch.cuda.synchronize()
+    assert torch.equal(c.cpu(), 600 * (a.cpu() @ b.cpu()))
