@@ -686,9 +686,10 @@ bool conv3x3_patch_applicable(const IgemmArgs& a, int in_dt) {
                                              (a.relu & ~(0xff | kActResidualAfter)) == 0);
   const int pix = a.pix_stride ? a.pix_stride : a.C;
   // Stride 2 pays while the launch is small: its workgroups load four input pixels per output pixel
-  // in front of the same K walk, which the implicit-GEMM kernel overtakes once it has enough
-  // 128x128 tiles for several rounds per CU (measured at 15 GFLOP per launch: 29-34 us there, 35-38
-  // here; at 3.7 GFLOP: 13-17 us there, 10-11 here).
+  // in front of the same K walk, which implicit GEMM overtakes once it has enough 128x128 tiles for
+  // several rounds per CU (igemm_fast at 15 GFLOP per launch: 29-34 us there, 35-38 here; at 3.7
+  // GFLOP: 13-17 us there, 10-11 here).  Launches above the line go to conv_ring, whose own line
+  // (conv_ring_beats_patch_s2) lies lower for most of them.
   const double s2_flops = 2.0 * a.N * a.OH * a.OW * (double)fmain * 9.0 * a.C;
   if (st == 2 && s2_flops > 8e9) return false;
   return !off && aux_ok && act_ok && a.wt_frag && a.R == 3 && a.S == 3 && (st == 1 || (st == 2 && in_dt == kF16 && !off2)) && a.stride_w == st &&
