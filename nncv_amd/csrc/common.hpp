@@ -281,6 +281,9 @@ void launch_igemm_fast(const IgemmArgs& a, int in_dt, int out_dt, hipStream_t s)
 struct RideCopy { const void* src; void* dst; size_t bytes; int blocks; };  // 16-byte aligned, bytes a multiple of 16
 void launch_gemm_nn_f32(const float* A, const float* B, const float* C, float* D, int M, int N, int K, hipStream_t s,
                         const RideCopy* ride = nullptr);
+// the same through three-way bf16 splits (gemm_split.hip); `wins`: its modelled time against that of the fp32 instructions
+bool gemm_split_wins(int M, int N, int K, double other_us);
+void launch_gemm_split(const float* A, const float* B, const float* C, float* D, int M, int N, int K, hipStream_t s);
 void launch_copy16(const RideCopy& r, hipStream_t s);  // the copy alone
 
 // ---------------------------------------------------------------------------------------------

@@ -9,6 +9,7 @@
 
 namespace nncv_hip {
 
+using mt::bytes_left;
 using mt::floatx16;
 using mt::floatx4;
 using mt::u32x4;
@@ -67,12 +68,6 @@ __device__ __forceinline__ void load_row(__amdgpu_buffer_rsrc_t rs, unsigned vof
     b[0] = f[0];
     b[1] = f[1];
   }
-}
-
-// bytes from element `at` to the end of an `elems`-element array, as a buffer descriptor's size
-__device__ __forceinline__ unsigned bytes_left(long long elems, long long at) {
-  const long long b = (elems - at) * 4;
-  return b > 0xffffffffll ? 0xffffffffu : (unsigned)b;
 }
 
 // A copy that rides in front of a launch: its first `blocks` workgroups move `bytes` (a multiple of 16) and are done.
@@ -351,8 +346,8 @@ namespace {
 // (launches back to back, clocks warm; the fit is within 5-15 % of every time, and the form it picks is on average 3 %
 // slower than the best one).  k_us at the matrix rate is 0.0033: large tiles come close, 16-wide ones are bound by the
 // number of operand loads (their MFMAs take half as long on the same loads), but split a small C over more CUs.
-//   1024^3 26.7 -> 21.1 us, 4096^3 1120 -> 960 (143 TFLOP/s), 1500x1001x777 69.4 -> 27.6, 20x488x536 14.6 -> 3.2,
-//   64x64x4096 81 -> 11, 92x3260x2312 52 -> 22 (against the LDS-tiled kernel with 128x128 / 64x64 tiles that this replaces)
+//   20x488x536 14.6 -> 3.2 us, 64x64x4096 81 -> 11, 92x3260x2312 52 -> 22 (against the LDS-tiled kernel with 128x128 / 64x64
+//   tiles that this replaces).  From 352 k on the larger products go to gemm_split.hip, by its model against this one.
 struct GemmForm {
   int rows, cols;
   double fixed_us, k_us, tile_us;
@@ -403,6 +398,10 @@ void launch_gemm_nn_f32(const float* A, const float* B, const float* C, float* D
     const long long tiles = (long long)((M + f.rows - 1) / f.rows) * ((N + f.cols - 1) / f.cols), rounds = (tiles + 255) / 256;
     const double us = f.fixed_us + (double)rounds * (f.k_us * (f.rows * f.cols / 1024.0) * ((K + 31) / 32 * 32) + f.tile_us);
     if (!best || us < best_us) best = &f, best_us = us;
+  }
+  if (gemm_split_wins(M, N, K, best_us)) {
+    launch_gemm_split(A, B, C, D, M, N, K, s);
+    return;
   }
   ProfScope prof(best->tag, flops, bytes, s);
   best->launch(A, B, C, D, M, N, K, RideCopy{}, s);

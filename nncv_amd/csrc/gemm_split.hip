@@ -1,0 +1,280 @@
+// fp32 row-major D = C + A.B (D may be C) on the bf16 matrix pipes, operands split in three (split.hpp).
+//
+// One wave owns TM x TN accumulators of 32 x 32 and walks K in rounds of 32, on its own: no barrier before the sums meet.
+//  * A (K contiguous): whole 128-byte lines, eight lanes each, a round ahead, through an LDS buffer of the wave's own, because an
+//    operand wants 16 bytes of 32 rows and read like that every lane of a load touches a line of its own.
+//  * B (N contiguous): lane l holds columns TN l .. TN l + TN - 1, so a load of row k is whole lines again.
+//  * Both are split in registers, 7 vector instructions for two values: 112 of them feed the 24 products (768 clocks) of a
+//    64 x 64 tile and 16 k, and run under the products of the SIMD's other wave.
+//  * Nothing asks for alignment beyond 4 bytes.  Only the last round of the matrix can hold k >= K or leave the buffers; the
+//    group that owns it walks it first, with A masked (B's rows past the end come back as zeros from the range check).
+//    Rows m >= M read row M - 1 and columns n >= N read the next row: both only reach results that are not stored.
+//  * KG "K groups": waves of a workgroup that share a tile of C and take every KG-th round.  Their sums meet in LDS, in a
+//    fixed order.
+#include <cmath>
+
+#include "split.hpp"
+
+namespace nncv_hip {
+
+using namespace mt;
+
+namespace {
+
+template <int TM, int TN, int KG>
+struct SplitCfg {
+  static constexpr int kPitch = 144;  // of a row of 32 k in LDS
+  static constexpr int kStage = 32 * TM * kPitch, kPart = KG > 1 ? 32 * TM * 32 * TN * 4 : 0;
+  static constexpr int kWave = kStage > kPart ? kStage : kPart, kLds = KG * kWave;
+};
+
+// one element in plain fp32
+__device__ __attribute__((noinline)) float plain_dot(const float* a, const float* b, int K, int N) {
+  float s = 0.0f;
+#pragma unroll 8
+  for (int k = 0; k < K; ++k) s = __builtin_fmaf(a[k], b[(long long)k * N], s);
+  return s;
+}
+
+template <int TM, int TN, int KG>
+__global__ __launch_bounds__(64 * KG, TM * TN == 4 ? 2 : TM * TN == 2 ? 3 : 4) void gemm_split_kernel(const float* __restrict__ A, const float* __restrict__ B, const float* C, float* D, int M,
+                                                               int N, int K, int tiles_m, int tiles_n) {
+  typedef SplitCfg<TM, TN, KG> Cfg;
+  static_assert(TN == 1 || TN == 2, "a lane holds one or two columns");
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int lane = threadIdx.x & 63, grp = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int lrow = lane & 31, lh = lane >> 5;
+  unsigned char* lds = smem + grp * Cfg::kWave;
+  // XCD x (workgroups x, x + 8, ...) takes a contiguous run of tiles, walked in bands of eight tile rows
+  int tm, tn;
+  {
+    const int tiles = tiles_m * tiles_n, per = (tiles + 7) >> 3, rem = tiles & 7;
+    const int x = blockIdx.x & 7, i = blockIdx.x >> 3;
+    const int t = rem == 0 ? x * per + i : (x < rem ? x * per : rem * per + (x - rem) * (per - 1)) + i;
+    const int band = t / (8 * tiles_n), in = t - band * 8 * tiles_n, h = min(8, tiles_m - 8 * band);
+    tn = in / h;
+    tm = 8 * band + (in - tn * h);
+  }
+  const int m0 = tm * 32 * TM, n0 = tn * 32 * TN;
+
+  constexpr int kA = 4 * TM;  // loads of a round: eight rows each
+  unsigned aoff[kA];
+#pragma unroll
+  for (int i = 0; i < kA; ++i) aoff[i] = ((unsigned)min((lane >> 3) + 8 * i, M - 1 - m0) * (unsigned)K + 4u * (lane & 7)) * 4u;
+  const unsigned boff = (8u * lh * (unsigned)N + (unsigned)(TN * lrow)) * 4u, brow = (unsigned)N * 4u;
+  floatx4 ra[kA];
+  float rb[2][8][TN];
+  // (rounds below the first read nothing: descriptors of no bytes)
+  auto left = [&](long long elems, long long at, int r) { return r >= 0 ? bytes_left(elems, at) : 0u; };
+  auto load_a = [&](int r) {
+    const long long at = (long long)m0 * K + 32ll * r;
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(A + at, left((long long)M * K, at, r));
+#pragma unroll
+    for (int i = 0; i < kA; ++i) ra[i] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs, aoff[i], 0, 0));
+  };
+  auto load_b = [&](int r, int k) {
+    const long long at = (32ll * r + 16 * k) * N + n0;
+    const bool in = 32 * r + 16 * k < K;
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(B + at, in ? left((long long)K * N, at, r) : 0u);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      if constexpr (TN == 1) {
+        rb[k][e][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, boff, (int)(e * brow), 0));
+      } else {
+        const floatx2 v = __builtin_bit_cast(floatx2, __builtin_amdgcn_raw_buffer_load_b64(rs, boff, (int)(e * brow), 0));
+        rb[k][e][0] = v[0];
+        rb[k][e][1] = v[1];
+      }
+    }
+  };
+
+  floatx16 big[TM][TN], low[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) big[i][j][v] = low[i][j][v] = 0.0f;
+
+  // units of the tile: register u % 16 of block row u / 16, columns TN lrow .. ; the ones this wave adds to C are asked for now
+  typedef float vec __attribute__((ext_vector_type(TN)));
+  constexpr int kUnits = 16 * TM, kMine = kUnits / KG;
+  auto row_of = [&](int u) { return m0 + 32 * (u >> 4) + 8 * ((u & 15) >> 2) + 4 * lh + (u & 3); };
+  auto fetch = [&](int u) {
+    const int m = row_of(u), n = n0 + TN * lrow;
+    vec v = {};
+    if (m < M && n < N) {
+      const float* c = C + ((long long)m * N + n);
+      if (TN == 1 || n + 1 < N) __builtin_memcpy(&v, c, sizeof(v));
+      else v[0] = c[0];
+    }
+    return v;
+  };
+
+  const int nk = (K + 31) >> 5;
+  int r = nk - 1 - grp;  // this group's rounds, from the last one down
+  load_a(r);
+  load_b(r, 0);
+  load_b(r, 1);
+  constexpr bool kEarly = KG > 1 && TM * TN < 4;  // (the 64 x 64 forms have no registers to spare)
+  vec cpre[kEarly ? kMine : 1];
+  if constexpr (kEarly) {
+#pragma unroll
+    for (int q = 0; q < kMine; ++q) cpre[q] = fetch(grp * kMine + q);
+  }
+  if (grp == 0) {
+    const int kend = K - 32 * r - 4 * (lane & 7);  // of this lane's four k
+#pragma unroll
+    for (int i = 0; i < kA; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ra[i][e] = e < kend ? ra[i][e] : 0.0f;
+  }
+  unsigned char* put = lds + (lane >> 3) * Cfg::kPitch + (lane & 7) * 16;
+  const unsigned char* get = lds + lrow * Cfg::kPitch + lh * 32;
+  for (; r >= 0; r -= KG) {
+#pragma unroll
+    for (int i = 0; i < kA; ++i) *reinterpret_cast<floatx4*>(put + 8 * i * Cfg::kPitch) = ra[i];
+    load_a(r - KG);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      u32x4 a[TM][3], b[TN][3];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const floatx4 x = *reinterpret_cast<const floatx4*>(get + i * 32 * Cfg::kPitch + k * 64), y = *reinterpret_cast<const floatx4*>(get + i * 32 * Cfg::kPitch + k * 64 + 16);
+        unsigned p[4][3];
+        split_pair(x[0], x[1], p[0]);
+        split_pair(x[2], x[3], p[1]);
+        split_pair(y[0], y[1], p[2]);
+        split_pair(y[2], y[3], p[3]);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) a[i][c] = u32x4{p[0][c], p[1][c], p[2][c], p[3][c]};
+      }
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        unsigned p[4][3];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) split_pair(rb[k][2 * e][j], rb[k][2 * e + 1][j], p[e]);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) b[j][c] = u32x4{p[0][c], p[1][c], p[2][c], p[3][c]};
+      }
+      load_b(r - KG, k);
+      constexpr int kX[6] = {0, 0, 1, 0, 1, 2}, kY[6] = {0, 1, 0, 2, 1, 0};
+#pragma unroll
+      for (int c = 0; c < 6; ++c)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) {
+            floatx16& s = c == 0 ? big[i][j] : low[i][j];
+            s = mma_bf16(a[i][kX[c]], b[j][kY[c]], s);
+          }
+    }
+  }
+
+  // ---- D = C + sums ----
+  auto emit = [&](int unit, const vec& c, vec sum) {
+    const int m = row_of(unit), n = n0 + TN * lrow;
+    if (m >= M || n >= N) return;
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      if (n + j < N && !(__builtin_fabsf(sum[j]) < __builtin_inff())) sum[j] = plain_dot(A + (long long)m * K, B + n + j, K, N);
+    sum += c;
+    float* d = D + ((long long)m * N + n);
+    if (TN == 1 || n + 1 < N) __builtin_memcpy(d, &sum, sizeof(sum));
+    else d[0] = sum[0];
+  };
+  if constexpr (KG == 1) {
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u) {
+      vec y;
+#pragma unroll
+      for (int j = 0; j < TN; ++j) y[j] = big[u >> 4][j][u & 15] + low[u >> 4][j][u & 15];
+      emit(u, fetch(u), y);
+    }
+  } else {
+    // [group][unit][lane][TN]
+    vec* mine = reinterpret_cast<vec*>(lds) + lane;
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u) {
+      vec y;
+#pragma unroll
+      for (int j = 0; j < TN; ++j) y[j] = big[u >> 4][j][u & 15] + low[u >> 4][j][u & 15];
+      mine[u * 64] = y;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kMine; ++q) {
+      const int u = grp * kMine + q;
+      const vec* p = reinterpret_cast<const vec*>(smem) + u * 64 + lane;
+      vec sum = p[0];
+#pragma unroll
+      for (int g = 1; g < KG; ++g) sum += p[g * (Cfg::kWave / sizeof(vec))];
+      emit(u, kEarly ? cpre[kEarly ? q : 0] : fetch(u), sum);
+    }
+  }
+}
+
+template <int TM, int TN, int KG>
+void launch_cfg(const float* A, const float* B, const float* C, float* D, int M, int N, int K, hipStream_t s) {
+  typedef SplitCfg<TM, TN, KG> Cfg;
+  auto kern = gemm_split_kernel<TM, TN, KG>;
+  static const bool attr = [&] {
+    NNCV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::kLds));
+    return true;
+  }();
+  (void)attr;
+  const long long tm = (M + 32 * TM - 1) / (32 * TM), tn = (N + 32 * TN - 1) / (32 * TN);
+  NNCV_REQUIRE(tm * tn < (1ll << 31), "matmul: too many tiles");
+  launch_kernel(kern, dim3((unsigned)(tm * tn)), dim3(64 * KG), Cfg::kLds, s, A, B, C, D, M, N, K, (int)tm, (int)tn);
+}
+
+// The forms, and what a launch of each takes:
+//   us = fixed + x (round_us * rounds of a wave + tile_us) + turns (turn_round_us * rounds of a wave + turn_us)
+// with x = tiles / 256 CUs and turns = ceil(x / workgroups that a CU holds): the matrix pipes' share, and a workgroup's own length.
+// Least-squares fits over 115 shapes of 30 MFLOP to 137 GFLOP, within 4-8 % of the times; the form they choose, or the fp32
+// instructions where those are the sooner ones, takes 3 % longer than the best one on average and 15 % less than the fp32 ones.
+//   1024^3 23.9 -> 16.4 us (131 TFLOP/s), 1500x1001x777 31.6 -> 24.3, 4096^3 960 -> 726 (189 TFLOP/s), 676x1382x829 21.3 -> 15.6
+struct Form {
+  int rows, cols, kg, resident;
+  double fixed_us, round_us, tile_us, turn_round_us, turn_us;
+  void (*launch)(const float*, const float*, const float*, float*, int, int, int, hipStream_t);
+  const char* tag;
+};
+const Form kForms[] = {
+    {64, 64, 8, 1, 1.297, 0.938, 0.685, 2.075, 2.064, launch_cfg<2, 2, 8>, "gemm_split<64x64,splitk8>"},
+    {64, 64, 4, 2, 1.208, 0.631, 1.424, 1.550, 2.232, launch_cfg<2, 2, 4>, "gemm_split<64x64,splitk4>"},
+    {64, 64, 1, 8, 0.0, 0.115, 1.504, 1.534, 6.457, launch_cfg<2, 2, 1>, "gemm_split<64x64>"},
+    {32, 64, 8, 1, 1.696, 0.492, 0.0, 1.382, 1.533, launch_cfg<1, 2, 8>, "gemm_split<32x64,splitk8>"},
+    {32, 64, 4, 3, 2.922, 0.570, 0.798, 0.827, 0.0, launch_cfg<1, 2, 4>, "gemm_split<32x64,splitk4>"},
+};
+
+const Form* best_form(int M, int N, int K, double* us) {
+  const Form* best = nullptr;
+  for (const Form& f : kForms) {
+    const double x = (double)((M + f.rows - 1) / f.rows) * ((N + f.cols - 1) / f.cols) / 256, turns = std::ceil(x / f.resident);
+    const double rounds = ((K + 31) / 32 + f.kg - 1) / f.kg;
+    const double v = f.fixed_us + x * (f.round_us * rounds + f.tile_us) + turns * (f.turn_round_us * rounds + f.turn_us);
+    if (!best || v < *us) best = &f, *us = v;
+  }
+  return best;
+}
+
+}  // namespace
+
+// `other_us`: the modelled time of the fp32 kernel, which is 10 % short of what it takes on rows that are not whole lines (hence
+// the margin).  Below 352 k the first loads and the reading and writing of C are most of a launch: what is left to gain there
+// is under a quarter for large M and N and nothing for the rest.
+bool gemm_split_wins(int M, int N, int K, double other_us) {
+  double us = 0;
+  return K >= 352 && N < 1 << 24 && K < 1 << 24 && best_form(M, N, K, &us) && us < 1.06 * other_us;
+}
+
+void launch_gemm_split(const float* A, const float* B, const float* C, float* D, int M, int N, int K, hipStream_t s) {
+  double us = 0;
+  const Form* f = best_form(M, N, K, &us);
+  ProfScope prof(f->tag, 2.0 * M * N * K, 4.0 * ((double)M * K + (double)K * N + 2.0 * M * N), s);
+  f->launch(A, B, C, D, M, N, K, s);
+  NNCV_HIP_CHECK(hipGetLastError());
+}
+
+}  // namespace nncv_hip

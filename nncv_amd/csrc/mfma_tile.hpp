@@ -40,6 +40,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, unsig
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
 }
 
+// bytes from float `at` to the end of an `elems`-element array (at < elems), as a buffer descriptor's size
+__device__ __forceinline__ unsigned bytes_left(long long elems, long long at) {
+  const long long b = (elems - at) * 4;
+  return b > 0xffffffffll ? 0xffffffffu : (unsigned)b;
+}
+
 using ::nncv_hip::relu_ugt;
 
 // x / d for 0 <= x < 2^24 and 1 <= d, given inv = 1.0f / d computed on the host: one float

@@ -1,0 +1,45 @@
+// fp32 products on the bf16 matrix pipes (gfx950): an fp32 value is the exact sum of three bf16 pieces, and
+//   a b = ah bh + (ah bm + am bh) + (ah bl + am bm + al bh) + what is below 2^-24 of it.
+// The six products are v_mfma_f32_32x32x16_bf16, sixteen times the rate of the fp32 instructions for six times the
+// work; every one is exact and the sums are fp32.  The five small ones are summed in registers of their own, so the chain of
+// roundings that carries the result's magnitude has one link for 16 k, where the fp32 instructions have one for every k: against
+// 64 bits the error of a sum of normal products is 3.1e-8 at 16 of them (fp32 instructions 7.3e-8), 1.3e-7 at 576 (4.3e-7)
+// and 4.2e-7 at 4608 (1.2e-6).  The first piece rounds to nearest even: cutting it off as well gives the dropped products a
+// sign (a bias of 3e-8).
+// An infinity has a NaN for its second piece, and so has a finite value that rounds to infinity in bf16: every result such an
+// operand takes part in comes out as a NaN.  A kernel recomputes results that are not finite in plain fp32.
+#pragma once
+#include "mfma_tile.hpp"
+
+namespace nncv_hip {
+namespace mt {
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+
+// Two values -> their pieces, packed in pairs: eleven instructions.  The first piece is rounded to nearest even, the second is
+// cut off what is left, which has eight bits to go then: the third is exact.  (v_dot2_f32_bf16 would take a piece off in
+// one instruction instead of two, but it runs in the matrix pipe: the products wait for it.)
+__device__ __forceinline__ void split_pair(float x, float y, unsigned (&p)[3]) {
+  p[0] = __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2{x, y}), bf16x2));
+  x -= __builtin_bit_cast(float, p[0] << 16);
+  y -= __builtin_bit_cast(float, p[0] & 0xffff0000u);
+  const unsigned u = __builtin_bit_cast(unsigned, x), v = __builtin_bit_cast(unsigned, y);
+  p[1] = __builtin_amdgcn_perm(v, u, 0x07060302u);
+  x -= __builtin_bit_cast(float, u & 0xffff0000u);
+  y -= __builtin_bit_cast(float, v & 0xffff0000u);
+  p[2] = __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, y), __builtin_bit_cast(unsigned, x), 0x07060302u);
+}
+
+__device__ __forceinline__ floatx16 mma_bf16(const u32x4& a, const u32x4& b, const floatx16& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// Rows of operands in LDS: 32 k of one row as three runs of 64 bytes, one per piece.  At 13 units of 16 bytes a row, a 16-byte
+// read of one column of 16 neighbouring rows touches every bank once.
+constexpr int kSplitPitch = 208;
+
+}  // namespace mt
+}  // namespace nncv_hip
