@@ -335,6 +335,7 @@ void launch_stem_pack(const void* src, int src_dt, void* dst, int dst_dt, int N,
 void launch_weight_frsc(const void* w, int w_dt, void* dst, int dst_dt, int F, int C, int R, int S, int Cp,
                         hipStream_t s);
 // 3x3 weights FCHW -> fragment-major order of conv3x3_patch.hip, F padded to a multiple of 64
+size_t weight_frag3x3_bytes(int dt, int F, int C);
 void launch_weight_frag3x3(const void* w, int w_dt, void* dst, int dst_dt, int F, int C, hipStream_t s);
 // 1x1 weights [F][C] in the same order with one tap per slab (IgemmArgs::aux_wt_frag)
 void launch_weight_frag1x1(const void* w, int w_dt, void* dst, int dst_dt, int F, int C, hipStream_t s);

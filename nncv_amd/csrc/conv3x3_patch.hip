@@ -1,13 +1,13 @@
-// 3x3 pad-1 convolution, stride 1 or 2, with the haloed input patch resident in LDS (gfx950).
-// The text below describes stride 1; what stride 2 (fp16 only: conv_direct.hip is faster in fp32 at
-// every size) changes (a 2TH+1 x 2TW+1 patch with its even and odd columns kept apart, the 1x1
+// fp16 3x3 pad-1 convolution, stride 1 or 2, with the haloed input patch resident in LDS (gfx950); also the
+// tile plan and the launch of fp32 stride-1 layers, whose kernel is conv3x3_split.hip.
+// The text below describes stride 1; what stride 2 changes (a 2TH+1 x 2TW+1 patch with its even and odd columns kept apart, the 1x1
 // shortcut convolution of a down-sampling block as extra filter blocks) is said where the code does it.
 //
 // The implicit-GEMM kernels gather every input pixel once per filter tap, i.e. nine times, from
 // L2, and need a workgroup barrier per K step.  Here a workgroup owns an output tile of TN images
 // x TH rows x TW columns (at most 64*WS pixel "slots"; TW is the full width unless a row is wider
 // than the 64 pixels the loader walks, in which case rows are cut into column tiles) and 64
-// filters, and per 128-byte channel slab (64 halves / 32 floats):
+// filters, and per 128-byte channel slab (64 halves):
 //   * loads the (TH+2) x (TW+2) haloed input patch ONCE into LDS (zero halo straight from the
 //     buffer-load range check; the reference materialises it with tensor.pad,
 //     tests/Nets/Res18.mlir:152-155),
@@ -19,7 +19,7 @@
 //     and the main loop has no barrier at all (only the slab change has).
 //
 // Wave layout WS x WK: WS waves each own 64 slots x 64 filters (2x2 accumulators of
-// v_mfma_f32_32x32x16_f16; fp32: 4x v_mfma_f32_32x32x2_f32 per chunk pair), and WK "K groups"
+// v_mfma_f32_32x32x16_f16), and WK "K groups"
 // split the four 32-byte K sub-steps of every tap between them; their partial sums meet in an
 // fp32 LDS tile from which the epilogue (scale/shift, residual, ReLU) stores whole rows
 // (mfma_tile.hpp).  Splitting K inside the workgroup rather than shrinking the pixel tile keeps
@@ -29,53 +29,11 @@
 // LDS pixel pitch is 128 + 16 bytes: consecutive pixels land 36 banks apart.
 #include <type_traits>
 
-#include "mfma_tile.hpp"
+#include "patch_args.hpp"
 
 namespace nncv_hip {
 
 using namespace mt;
-
-namespace {
-constexpr int kPitch = 144;            // LDS bytes per patch pixel: 128 payload + 16 pad
-constexpr unsigned kOOBp = 0x7fff0000u;
-constexpr int kXcdsP = 8;
-
-template <int WS> struct PatchCap;     // patch capacity in pixels for 64*WS slots
-template <> struct PatchCap<4> { static constexpr int pix = 384; };
-template <> struct PatchCap<2> { static constexpr int pix = 256; };
-template <> struct PatchCap<1> { static constexpr int pix = 192; };
-}  // namespace
-
-struct PatchArgs {
-  const void* in;        // NHWC [N][H][W][C]
-  const void* wf;        // fragment-major weights (launch_weight_frag3x3)
-  void* out;             // NHWC [N][H][W][F]
-  const float* scale;    // [F] or null
-  const float* shift;    // [F] or null
-  const void* residual;  // like out, or null
-  int N, H, W, C, F, relu;
-  int TN, TH;            // tile: TN images x TH output rows x TW output columns
-  int tiles_y;           // tiles per group of TN images: ceil(OH / TH) row bands x NTX column tiles
-  int tiles;             // ceil(N / TN) * tiles_y
-  int ldo, pix;          // elements between pixels of out (and residual) / of in: F and C unless they are slices of wider tensors
-  int txw;               // TW | NTX << 16.  NTX = 1 (TW = the full output width) unless a row is too wide for the loader
-  int rw_log;            // patch loader: 2^rw_log >= patch columns per loader row
-  int rowx;              // stride 1: spare bytes behind the cells of a patch row (see the row pitch in the kernel)
-  int OH, OW;            // output size (stride 2; stride 1: H, W)
-  int xcd_by_filter;     // XCD <- filter block instead of XCD <- tile range
-  unsigned in_bytes, wf_bytes;
-  float inv_ph, inv_thw, inv_w;  // 1/(patch rows per image), 1/(TH*TW), 1/TW
-  // Stride 2 only: filter blocks >= aux_fb0 (in units of the workgroup's 32*NI filters) belong to a
-  // 1x1 stride-2 convolution over the same input (the shortcut of a down-sampling block), with its
-  // own output tensor [N][OH][OW][aux_F], scale/shift and ReLU flag.  aux_F = 0: none.
-  const void* aux_wf;    // fragment-major, one tap per slab (launch_weight_frag1x1)
-  void* aux_out;
-  const float* aux_scale;
-  const float* aux_shift;
-  int aux_F, aux_relu, aux_fb0;
-  int aux_inline;  // the workgroup of filter block b also computes block b of the auxiliary filters (aux_F == F): no extra blocks
-  unsigned aux_wf_bytes;
-};
 
 template <int WS, int WK, int ST = 1>
 struct PatchCfg {
@@ -341,7 +299,7 @@ __global__ __launch_bounds__(64 * WS * WK) __attribute__((amdgpu_waves_per_eu(2,
   // except in the instances whose tap loop has no 16 registers to spare for them (they would be
   // spilled to scratch memory around the loop: a wait for every load in flight at the loop's door
   // and 13 KB of extra HBM writes per workgroup), which request them behind the loop instead
-  constexpr bool kLateScale = sizeof(T) == 2 && (WS == 4 || (ST == 2 && WS == 1 && NI == 2));
+  constexpr bool kLateScale = WS == 4 || (ST == 2 && WS == 1 && NI == 2);
   EpiScale<OutT> ess;
   if constexpr (!kLateScale) ess.load(lane, f0blk, a.F, a.scale, a.shift);
 
@@ -372,15 +330,11 @@ __global__ __launch_bounds__(64 * WS * WK) __attribute__((amdgpu_waves_per_eu(2,
 
   // [filter half][pixel half]; with NI = 1 only acc[0] is used.  The first step of the first slab starts the sums from a
   // zero C operand: clearing the registers instead cost 64 moves between the patch barrier and the first MFMA.
-  // (fp16 instances; the fp32 ones, four chained MFMAs per product, are at their register limit and keep the moves.)
-  constexpr bool kZeroC = sizeof(T) == 2;
   floatx16 acc[2][2];
 #pragma unroll
-  for (int i = kZeroC ? 1 : 0; i < 2; ++i)  // fp16, NI = 1: acc[1] is never written by an MFMA and never read for a result
+  for (int j = 0; j < 2; ++j)  // NI = 1: acc[1] is never written by an MFMA and never read for a result
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+    for (int v = 0; v < 16; ++v) acc[1][j][v] = 0.0f;
 
   // ---- tap loop.  One trip = one slab = 9 taps x KPG K sub-steps ("steps"), fully unrolled, so
   // that tap offsets, weight register sets (NSET divides 9) and the ring slot of the pixel
@@ -414,8 +368,6 @@ __global__ __launch_bounds__(64 * WS * WK) __attribute__((amdgpu_waves_per_eu(2,
     else
       ring[st % kDepth][j] = *reinterpret_cast<const u32x4*>(patch + rowbase[t / 3][j] + (t % 3 == 1 ? odd_col : 0) + (t % 3 == 2 ? kPitch : 0) + k * 32);
   };
-  // the fp16 instances spread a step's other instructions between its MFMAs (see the tap loop)
-  constexpr bool kSpread = sizeof(T) == 2;
   auto prime = [&](auto self, auto d_c) -> void {  // the first kDepth-1 steps of a fresh patch
     constexpr int d = decltype(d_c)::value;
     if constexpr (d < kDepth - 1) {
@@ -438,38 +390,22 @@ __global__ __launch_bounds__(64 * WS * WK) __attribute__((amdgpu_waves_per_eu(2,
         constexpr int t = st / KPG, k = st % KPG, set = t % NSET;
         const int it_next = slab * 9 + t + NSET;
         const int wso = it_next < niter ? wbase + it_next * 8192 : 0;  // past the end: re-read block 0 (never used)
-        if constexpr (kSpread) {
-          // every MFMA is followed by its share of the step's other instructions (an LDS read of the step kDepth - 1
-          // ahead, a weight refill), so that they issue under it instead of behind the four: 7x7x512 at batch 32
-          // 13.3 -> 12.9 us (one wave per SIMD), the stride-2 launches 10.0 -> 9.4, 56x56x64 14.4 -> 14.05
+        // every MFMA is followed by its share of the step's other instructions (an LDS read of the step kDepth - 1
+        // ahead, a weight refill), so that they issue under it instead of behind the four: 7x7x512 at batch 32
+        // 13.3 -> 12.9 us (one wave per SIMD), the stride-2 launches 10.0 -> 9.4, 56x56x64 14.4 -> 14.05
 #pragma unroll
-          for (int i = 0; i < NI; ++i)
+        for (int i = 0; i < NI; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-              if (kZeroC && st == 0 && slab == 0) Mma<T>::start(wregs[set][k * NI + i], ring[st % kDepth][j], acc[i][j]);
-              else Mma<T>::run(wregs[set][k * NI + i], ring[st % kDepth][j], acc[i][j]);
-              __builtin_amdgcn_sched_barrier(0);
-              if constexpr (st + kDepth - 1 < kSteps) {
-                if (i == 0) ldp1(std::integral_constant<int, st + kDepth - 1>(), j);
-              }
-              if (j == 1) wregs[set][k * NI + i] = __builtin_amdgcn_raw_buffer_load_b128(rs_wf, wlane, wso + wfrag(k, i), 0);
-              __builtin_amdgcn_sched_barrier(0);
+          for (int j = 0; j < 2; ++j) {
+            if (st == 0 && slab == 0) Mma<T>::start(wregs[set][k * NI + i], ring[st % kDepth][j], acc[i][j]);
+            else Mma<T>::run(wregs[set][k * NI + i], ring[st % kDepth][j], acc[i][j]);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (st + kDepth - 1 < kSteps) {
+              if (i == 0) ldp1(std::integral_constant<int, st + kDepth - 1>(), j);
             }
-        } else {
-          if constexpr (st + kDepth - 1 < kSteps) ldp(std::integral_constant<int, st + kDepth - 1>());
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int i = 0; i < NI; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-              if (kZeroC && st == 0 && slab == 0) Mma<T>::start(wregs[set][k * NI + i], ring[st % kDepth][j], acc[i][j]);
-              else Mma<T>::run(wregs[set][k * NI + i], ring[st % kDepth][j], acc[i][j]);
-            }
-#pragma unroll
-          for (int i = 0; i < NI; ++i)
-            wregs[set][k * NI + i] = __builtin_amdgcn_raw_buffer_load_b128(rs_wf, wlane, wso + wfrag(k, i), 0);
-          __builtin_amdgcn_sched_barrier(0);
-        }
+            if (j == 1) wregs[set][k * NI + i] = __builtin_amdgcn_raw_buffer_load_b128(rs_wf, wlane, wso + wfrag(k, i), 0);
+            __builtin_amdgcn_sched_barrier(0);
+          }
         self(self, std::integral_constant<int, st + 1>());
       }
     };
@@ -697,7 +633,7 @@ bool conv3x3_patch_applicable(const IgemmArgs& a, int in_dt) {
          a.batch == 1 && pix % (slab / 8) == 0 && a.C % slab == 0 && fmain % 8 == 0 && a.ldo >= fmain && a.ldo % (slab / 8) == 0 &&
          (long long)a.N * a.OH * a.OW * std::max(a.ldo, faux) < (1ll << 31) && (long long)a.N * a.H * a.W < (1 << 24) && a.in_bytes < kOOBp &&
          (long long)pix * (long long)dtype_size(in_dt) < (1 << 24) &&
-         (long long)((std::max(fmain, faux) + 63) / 64) * 64 * 9 * a.C * (long long)dtype_size(in_dt) < (1ll << 31) &&
+         (long long)weight_frag3x3_bytes(in_dt, std::max(fmain, faux), a.C) < (1ll << 31) &&
          plan_patch(st, a.N, a.OH, a.OW, fmain, a.C / slab, &ws, &tp);
 }
 
@@ -726,7 +662,7 @@ static void launch_patch_cfg(const PatchArgs& a, double flops, double bytes, con
 
 void launch_conv3x3_patch(const IgemmArgs& g, int in_dt, int out_dt, hipStream_t s) {
   PatchArgs a{};
-  a.in = g.in; a.wf = g.wt_frag; a.out = g.out; a.scale = g.scale; a.shift = g.shift; a.residual = g.residual;
+  a.in = g.in; a.wf = g.wt_frag; a.wt = g.wt; a.out = g.out; a.scale = g.scale; a.shift = g.shift; a.residual = g.residual;
   a.N = g.N; a.H = g.H; a.W = g.W; a.C = g.C; a.F = g.aux_f0 ? g.aux_f0 : g.F; a.relu = g.relu;
   a.ldo = g.ldo; a.pix = g.pix_stride ? g.pix_stride : g.C;
   if (g.aux_f0) {
@@ -747,7 +683,7 @@ void launch_conv3x3_patch(const IgemmArgs& g, int in_dt, int out_dt, hipStream_t
   a.tiles_y = ((a.OH + a.TH - 1) / a.TH) * tp.NTX;
   a.tiles = ((a.N + a.TN - 1) / a.TN) * a.tiles_y;
   a.in_bytes = g.in_bytes;
-  a.wf_bytes = (unsigned)((size_t)((a.F + 63) / 64) * 64 * 9 * a.C * dtype_size(in_dt));
+  a.wf_bytes = (unsigned)weight_frag3x3_bytes(in_dt, a.F, a.C);
   a.xcd_by_filter = ((a.F + 63) / 64) % kXcdsP == 0 && a.wf_bytes > (2u << 20);
   a.inv_ph = 1.0f / (st == 1 ? a.TH + 2 : 2 * a.TH + 1);
   a.inv_thw = 1.0f / (a.TH * tp.TW);
@@ -787,10 +723,8 @@ void launch_conv3x3_patch(const IgemmArgs& g, int in_dt, int out_dt, hipStream_t
     else if (halves) launch_patch_cfg<half_t, half_t, 1, 4, 1>(a, flops, bytes, "conv3x3_patch<f16,1,4,half>", s);
     else launch_patch_cfg<half_t, half_t, 1, 4, 2>(a, flops, bytes, "conv3x3_patch<f16,1,4>", s);
   } else {
-    if (ws == 4) launch_patch_cfg<float, float, 4, 1, 2>(a, flops, bytes, "conv3x3_patch<f32,4,1>", s);
-    else if (ws == 2) launch_patch_cfg<float, float, 2, 2, 2>(a, flops, bytes, "conv3x3_patch<f32,2,2>", s);
-    else if (halves) launch_patch_cfg<float, float, 1, 4, 1>(a, flops, bytes, "conv3x3_patch<f32,1,4,half>", s);
-    else launch_patch_cfg<float, float, 1, 4, 2>(a, flops, bytes, "conv3x3_patch<f32,1,4>", s);
+    launch_conv3x3_split(a, ws, halves, ws == 4 ? "conv3x3_patch<f32,4,1>" : ws == 2 ? "conv3x3_patch<f32,2,2>" : halves ? "conv3x3_patch<f32,1,4,half>" : "conv3x3_patch<f32,1,4>",
+                         flops, bytes, s);
   }
   NNCV_HIP_CHECK(hipGetLastError());
 }

@@ -1,0 +1,336 @@
+// fp32 3x3 pad-1 stride-1 convolution on the bf16 matrix pipes, operands split in three (split.hpp), with the haloed input patch
+// resident in LDS.  Tiles and their plan are those of conv3x3_patch.hip: 64 * WS pixel slots x 32 * NI filters a workgroup, channel
+// slabs of 32.
+//
+//  * The patch of a slab is loaded once, split once, and read by nine taps: splitting pixels costs a ninth of what it costs a
+//    kernel that reads taps from memory.  A cell of LDS is one pixel's 32 channels as three runs of 64 bytes, one per piece.
+//  * Filters are split once, when the layer is made, in fragment order (launch_weight_frag3x3): an operand of a wave is three
+//    contiguous kilobytes, straight into registers, three steps ahead.
+//  * Two patch buffers: a slab is multiplied while the next one is split into the other buffer, between the products, and the one
+//    after that is on its way to registers.  One barrier a slab.
+//  * Four waves: WS = 4, 2: each 64 slots x 32 filters; WS = 1: 64 x 32 (NI = 1: 32 x 32) with
+//    the two 16-channel steps of a tap dealt to two K groups, whose sums meet in LDS.
+//  * A sum that is not finite is done again in plain fp32.
+//  * What bounds it: the matrix pipes where tiles fill the CUs (six products, 2.7 times the fp32 instructions' rate), one wave a
+//    SIMD issuing everything where they do not.
+#include <type_traits>
+
+#include "patch_args.hpp"
+#include "split.hpp"
+
+namespace nncv_hip {
+
+using namespace mt;
+
+namespace {
+
+constexpr int kCell = 208;              // 3 x 64 + 16: at 13 units of 16 bytes, 16 neighbouring cells touch every bank once
+constexpr int kRowSpare = 96;           // behind a patch row: its pitch is 13 TW units mod 16 then, as if a tile's rows were one
+
+template <int WS>
+struct SplitCfg {
+  static constexpr int cap = PatchCap<WS>::pix, passes = cap / 32;  // loader: 8 threads a pixel, 32 pixels a pass
+  static constexpr int buffers = WS == 4 ? 1 : 2;                     // (256 slots: layers of one slab)
+  static constexpr int patch = cap * kCell, dump = buffers * patch, scale = dump + 640, smem = scale + 512;
+};
+
+// one sum in plain fp32
+__device__ __forceinline__ float plain_sum(const PatchArgs& a, int p, int f) {
+  const int HW = a.H * a.W, n = p / HW, oy = (p - n * HW) / a.W, ox = p - n * HW - oy * a.W;
+  const float* in = static_cast<const float*>(a.in);
+  const float* wt = static_cast<const float*>(a.wt) + (long long)f * 9 * a.C;
+  float sum = 0.0f;
+  for (int t = 0; t < 9; ++t) {
+    const int iy = oy + t / 3 - 1, ix = ox + t % 3 - 1;
+    if ((unsigned)iy >= (unsigned)a.H || (unsigned)ix >= (unsigned)a.W) continue;
+    const float* row = in + (long long)((n * a.H + iy) * a.W + ix) * a.pix;
+    for (int c = 0; c < a.C; ++c) sum = __builtin_fmaf(row[c], wt[t * a.C + c], sum);
+  }
+  return sum;
+}
+
+template <int WS, int NI>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void conv3x3_split_kernel(
+    // (the values the patch addressing needs first: preloaded into SGPRs)
+    const void* in_p, int tiles_p, int tiles_y_p, int tn_p, int th_p, int n_p, int h_p, int w_p, int c_p, int rw_log_p, int xcd_by_filter_p,
+    unsigned in_bytes_p, int txw_p, const PatchArgs a_rest) {
+  PatchArgs a = a_rest;
+  a.txw = txw_p;
+  a.in = in_p; a.tiles = tiles_p; a.tiles_y = tiles_y_p; a.TN = tn_p; a.TH = th_p; a.N = n_p; a.H = h_p; a.W = w_p; a.C = c_p;
+  a.rw_log = rw_log_p; a.xcd_by_filter = xcd_by_filter_p; a.in_bytes = in_bytes_p;
+  typedef SplitCfg<WS> Cfg;
+  constexpr int kPasses = Cfg::passes;
+  constexpr int IN = 1, JN = WS == 1 && NI == 1 ? 1 : 2, KG = WS == 1 ? 2 : 1;  // filter and slot blocks of a wave, K groups
+  constexpr int KPG = 2 / KG, NSET = JN == 1 ? 9 : 3;                  // steps of a tap, steps whose filters are on their way
+  constexpr int kSteps = 9 * KPG, kQuads = IN * JN * 4;
+  static_assert(WS != 2 || NI == 2, "128 slots: two waves to a filter half");
+  static_assert(WS != 4 || NI == 1, "256 slots: every wave has its own");
+  extern __shared__ __align__(16) unsigned char smem[];
+
+  int tile, fblk;  // (as conv3x3_patch.hip)
+  if (a.xcd_by_filter) {
+    const int lin = blockIdx.y * gridDim.x + blockIdx.x, per = gridDim.y / kXcdsP, k = lin / kXcdsP;
+    fblk = lin % kXcdsP + kXcdsP * (k % per);
+    tile = k / per;
+  } else {
+    const int per_xcd = (a.tiles + kXcdsP - 1) / kXcdsP;
+    tile = (blockIdx.x % kXcdsP) * per_xcd + blockIdx.x / kXcdsP;
+    fblk = blockIdx.y;
+  }
+  if (tile >= a.tiles) return;
+  const int TW = a.txw & 0xffff, ntx = a.txw >> 16;
+  const int n0 = (tile / a.tiles_y) * a.TN;
+  int band = tile % a.tiles_y, x0 = 0;
+  if (ntx > 1) {
+    x0 = (band % ntx) * TW;
+    band /= ntx;
+  }
+  const int y0 = band * a.TH, PH = a.TH + 2, PW = TW + 2, RP = PW * kCell + kRowSpare;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int slot0 = WS == 4 ? wave * 64 : WS == 2 ? (wave & 1) * 64 : NI == 1 ? (wave >> 1) * 32 : 0;
+  const int kg = KG == 2 ? wave & 1 : 0;
+  const int half = NI == 1 ? fblk & 1 : wave >> 1;                 // of the 64-filter block
+  const int fb64 = NI == 1 ? fblk >> 1 : fblk, f0 = fb64 * 64 + half * 32;          // this wave's first filter
+  const int lrow = lane & 31, lh = lane >> 5;
+  const __amdgpu_buffer_rsrc_t rs_in = make_rsrc(a.in, a.in_bytes);
+  const __amdgpu_buffer_rsrc_t rs_wf = make_rsrc(a.wf, a.wf_bytes);
+  const int nslab = a.C >> 5, niter = nslab * 9;
+
+  // ---- patch loader: the patch is walked as rows of 2^rw_log pixels ----
+  const int p8 = tid >> 3, c4 = tid & 7, pc = c4 * 16;
+  const int prows = a.TN * PH, rwm = (1 << a.rw_log) - 1;
+  const unsigned ces = (unsigned)(a.pix * 4);
+  unsigned pvoff[kPasses];
+#pragma unroll
+  for (int i = 0; i < kPasses; ++i) {
+    const int q = i * 32 + p8, r = q >> a.rw_log, px = q & rwm;
+    int n = n0, py = r;
+    if (a.TN > 1) n += fast_div(r, PH, a.inv_ph, &py);
+    const int iy = y0 + py - 1;
+    const bool ok = (r < prows) & (n < a.N) & ((unsigned)iy < (unsigned)a.H) & ((unsigned)(x0 + px - 1) < (unsigned)a.W);
+    pvoff[i] = ok ? __umul24((unsigned)((n * a.H + iy) * a.W + x0 + px - 1), ces) + pc : kOOBp;
+  }
+  // four channels go where the operand of their step has them: units 4 s + h and 4 s + 2 + h of a step s are lane half h's.
+  // Lanes whose pass lies outside the patch write to a dump behind it.
+  unsigned pdst[kPasses];
+#pragma unroll
+  for (int i = 0; i < kPasses; ++i) {
+    const int q = i * 32 + p8, r = q >> a.rw_log, px = q & rwm;
+    const int sub = (c4 >> 2) * 32 + (c4 & 1) * 16 + ((c4 >> 1) & 1) * 8;
+    pdst[i] = ((px < PW) & (r < prows)) ? __umul24(r, RP) + __umul24(px, kCell) + sub : Cfg::dump + lane * 8;
+  }
+  u32x4 pregs[kPasses];
+  auto pload = [&](int i, int slab) { pregs[i] = __builtin_amdgcn_raw_buffer_load_b128(rs_in, pvoff[i] + slab * 128, 0, 0); };
+  auto pstore = [&](int i, unsigned to) {  // `to`: byte offset of the buffer (the dump is shared)
+    const floatx4 v = __builtin_bit_cast(floatx4, pregs[i]);
+    unsigned p[2][3];
+    split_pair(v[0], v[1], p[0]);
+    split_pair(v[2], v[3], p[1]);
+    unsigned char* dst = smem + (pdst[i] < (unsigned)Cfg::dump ? pdst[i] + to : pdst[i]);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) *reinterpret_cast<u32x2*>(dst + c * 64) = u32x2{p[0][c], p[1][c]};
+  };
+#pragma unroll
+  for (int i = 0; i < kPasses; ++i) pload(i, 0);
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- filters: the operand of iteration (slab, tap), step k, half i, piece c is the kilobyte at
+  //      (((fb64 * niter + it) * 2 + k) * 2 + i) * 3 + c ----
+  const int wbase = (fb64 * niter * 4 + kg * 2 + half) * 3072;
+  const unsigned wlane = lane * 16;
+  u32x4 w[NSET][1][3];
+  auto wload = [&](u32x4 (&r)[1][3], int it, int k) {
+    const int so = it < niter ? wbase + it * 12288 + k * 6144 : 0;  // past the end: block 0 again (never used)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) r[0][c] = __builtin_amdgcn_raw_buffer_load_b128(rs_wf, wlane, so + c * 1024, 0);
+  };
+#pragma unroll
+  for (int t = 0; t < NSET; ++t) wload(w[t], t / KPG, t % KPG);
+  if (tid < 64) {
+    const int f = fb64 * 64 + tid;
+    float* ss = reinterpret_cast<float*>(smem + Cfg::scale);
+    ss[tid] = a.scale && f < a.F ? a.scale[f] : 1.0f;
+    ss[64 + tid] = a.shift && f < a.F ? a.shift[f] : 0.0f;
+  }
+
+  // ---- this lane's pixel slots ----
+  const int nslots = a.TN * a.TH * TW;
+  int sbase[JN];  // byte offset of the slot's tap-(0,0) cell
+  int obase[JN];  // element offset of the slot's output pixel row, or -1
+#pragma unroll
+  for (int j = 0; j < JN; ++j) {
+    const int sl0 = slot0 + j * 32 + lrow;
+    int sl = sl0;
+    if (sl0 >= nslots) {  // reads with the slot 16, 32 ... before it (the same banks), is not stored
+      const int back = (((sl0 - nslots) >> 4) + 1) << 4;
+      sl = sl0 >= back ? sl0 - back : 0;
+    }
+    int nl = 0, rem = sl, tx;
+    if (a.TN > 1) nl = fast_div(sl, a.TH * TW, a.inv_thw, &rem);
+    const int ty = fast_div(rem, TW, a.inv_w, &tx);
+    const bool ok = (sl < nslots) & ((n0 + nl) < a.N) & ((y0 + ty) < a.H) & ((x0 + tx) < a.W);
+    sbase[j] = (ok ? (int)__umul24(__umul24(nl, PH) + ty, RP) + (int)__umul24(tx, kCell) : 0) + lh * 16 + kg * KPG * 32;
+    obase[j] = (ok && sl0 < nslots) ? (((n0 + nl) * a.H + y0 + ty) * a.W + x0 + tx) * a.ldo : -1;
+  }
+
+  floatx16 big[IN][JN], low[IN][JN];
+#pragma unroll
+  for (int i = 0; i < IN; ++i)
+#pragma unroll
+    for (int j = 0; j < JN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) big[i][j][v] = low[i][j][v] = 0.0f;
+
+  // ---- tap loop: one trip = one slab = 9 taps x KPG steps, unrolled.  Under the products of a step: the pixel operand of the next
+  //      one is read, the filters of NSET steps further on are asked for, and a share of the next slab's patch is split into the
+  //      other buffer and that of the slab after it asked for ----
+  u32x4 ring[2][JN][3];
+  int row[3][JN];
+  auto ldp = [&](auto step_c) {
+    constexpr int st = decltype(step_c)::value, t = st / KPG, k = st % KPG;
+#pragma unroll
+    for (int j = 0; j < JN; ++j)
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+        ring[st & 1][j][c] = *reinterpret_cast<const u32x4*>(smem + row[t / 3][j] + (t % 3) * kCell + k * 32 + c * 64);
+  };
+#pragma unroll
+  for (int i = 0; i < kPasses; ++i) {
+    pstore(i, 0);
+    if (Cfg::buffers == 2) pload(i, 1);
+  }
+  __syncthreads();
+  for (int slab = 0; slab < nslab; ++slab) {
+    const int at = Cfg::buffers == 2 ? (slab & 1) * Cfg::patch : 0;
+    const unsigned other = Cfg::patch - at;
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+      for (int j = 0; j < JN; ++j) row[r][j] = sbase[j] + at + r * RP;
+    ldp(std::integral_constant<int, 0>());
+    __builtin_amdgcn_sched_barrier(0);
+    auto steps = [&](auto self, auto step_c) -> void {
+      constexpr int st = decltype(step_c)::value;
+      if constexpr (st < kSteps) {
+        constexpr int nx = st + NSET, p0 = st * kPasses / kSteps, p1 = Cfg::buffers == 2 ? (st + 1) * kPasses / kSteps : p0;
+        if constexpr (st + 1 < kSteps) ldp(std::integral_constant<int, st + 1>());
+        split_products(w[st % NSET], ring[st & 1], big, low);
+        wload(w[st % NSET], (slab + nx / kSteps) * 9 + nx % kSteps / KPG, nx % KPG);
+#pragma unroll
+        for (int i = p0; i < p1; ++i) {
+          pstore(i, other);
+          pload(i, slab + 2);
+        }
+        constexpr int kMma = 6 * JN, kValu = (26 * (p1 - p0) + kMma - 1) / kMma;
+#pragma unroll
+        for (int n = 0; n < kMma; ++n) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          if (kValu) __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);
+          __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        self(self, std::integral_constant<int, st + 1>());
+      }
+    };
+    steps(steps, std::integral_constant<int, 0>());
+    __syncthreads();  // every wave has left this patch and written its share of the next
+  }
+
+  // ---- out: quad (i, j, g): filters 32 i + 8 g + 4 lh .. + 3 of slot block j.  K group g finishes every second quad ----
+  constexpr int kMine = kQuads / KG;
+  auto sum_of = [&](int q) {
+    const int i = q / (4 * JN), j = q / 4 % JN, g = q & 3;
+    floatx4 s;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[e] = big[i][j][4 * g + e] + low[i][j][4 * g + e];
+    return s;
+  };
+  const float* res = static_cast<const float*>(a.residual);
+  float* out = static_cast<float*>(a.out);
+  const float* ss = reinterpret_cast<const float*>(smem + Cfg::scale) + half * 32 + 4 * lh;
+  auto at_of = [&](int q, int* f) {  // element of the quad's first result, -1: not stored
+    const int o = obase[q / 4 % JN];
+    *f = f0 + (q / (4 * JN)) * 32 + (q & 3) * 8 + 4 * lh;
+    return o >= 0 && *f < a.F ? (long long)o + *f : -1ll;
+  };
+  floatx4 rv[kMine];
+  if (res) {
+#pragma unroll
+    for (int m = 0; m < kMine; ++m) {
+      int f;
+      const long long at = at_of(KG == 2 ? 2 * m + kg : m, &f);
+      rv[m] = at >= 0 ? *reinterpret_cast<const floatx4*>(res + at) : floatx4{};
+    }
+  }
+  floatx4 sums[kMine];
+  if constexpr (KG == 2) {
+    floatx4* part = reinterpret_cast<floatx4*>(smem);  // [wave][quad of the other group][lane]
+#pragma unroll
+    for (int m = 0; m < kMine; ++m) part[(wave * kMine + m) * 64 + lane] = kg ? sum_of(2 * m) : sum_of(2 * m + 1);
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < kMine; ++m) sums[m] = (kg ? sum_of(2 * m + 1) : sum_of(2 * m)) + part[((wave ^ 1) * kMine + m) * 64 + lane];
+  } else {
+#pragma unroll
+    for (int m = 0; m < kMine; ++m) sums[m] = sum_of(m);
+  }
+  auto put = [&](int q, long long at, floatx4 y, const floatx4& r) {
+    const int b = (q / (4 * JN)) * 32 + (q & 3) * 8;
+    y = y * *reinterpret_cast<const floatx4*>(ss + b) + *reinterpret_cast<const floatx4*>(ss + 64 + b);
+    if (res) y += r;
+    if (a.relu == kActRelu) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = relu_ugt(y[e]);
+    }
+    *reinterpret_cast<floatx4*>(out + at) = y;
+  };
+  unsigned again = 0;
+#pragma unroll
+  for (int m = 0; m < kMine; ++m) {
+    const int q = KG == 2 ? 2 * m + kg : m;
+    int f;
+    const long long at = at_of(q, &f);
+    if (at < 0) continue;
+    if (split_finite(sums[m])) put(q, at, sums[m], rv[m]);
+    else again |= 1u << q;
+  }
+  for (; again; again &= again - 1) {
+    const int q = __builtin_ctz(again);
+    const int o = JN == 2 && (q / 4 % JN) ? obase[JN - 1] : obase[0], f = f0 + (q / (4 * JN)) * 32 + (q & 3) * 8 + 4 * lh;
+    floatx4 s;
+#pragma unroll 1
+    for (int e = 0; e < 4; ++e) s[e] = plain_sum(a, o / a.ldo, f + e);
+    const long long at = (long long)o + f;
+    put(q, at, s, res ? *reinterpret_cast<const floatx4*>(res + at) : floatx4{});
+  }
+}
+
+template <int WS, int NI>
+void launch_cfg(const PatchArgs& b, hipStream_t s) {
+  auto kern = conv3x3_split_kernel<WS, NI>;
+  static const bool attr = [&] {
+    NNCV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, SplitCfg<WS>::smem));
+    return true;
+  }();
+  (void)attr;
+  const int fblocks = (b.F + 32 * NI - 1) / (32 * NI);
+  const dim3 grid((b.tiles + kXcdsP - 1) / kXcdsP * kXcdsP, fblocks);
+  launch_kernel(kern, grid, dim3(256), SplitCfg<WS>::smem, s, b.in, b.tiles, b.tiles_y, b.TN, b.TH, b.N, b.H, b.W, b.C, b.rw_log,
+                b.xcd_by_filter && fblocks % kXcdsP == 0, b.in_bytes, b.txw, b);
+}
+
+}  // namespace
+
+void launch_conv3x3_split(const PatchArgs& a, int ws, bool half, const char* tag, double flops, double bytes, hipStream_t s) {
+  ProfScope prof(tag, flops, bytes, s);
+  if (ws == 4) launch_cfg<4, 1>(a, s);
+  else if (ws == 2) launch_cfg<2, 2>(a, s);
+  else if (half) launch_cfg<1, 1>(a, s);
+  else launch_cfg<1, 2>(a, s);
+}
+
+}  // namespace nncv_hip

@@ -22,7 +22,7 @@
 #include <algorithm>
 #include <cmath>
 
-#include "mfma_tile.hpp"
+#include "split.hpp"
 
 namespace nncv_hip {
 
@@ -79,9 +79,34 @@ struct DirectArgs {
   float inv_ohw, inv_ow, inv_s, inv_cpt, inv_tiles;
 };
 
+// One sum in plain fp32, from the filters in their flat order: channel c of a tap is float c % 4 of chunk c / 4 of that tap.
+__device__ __forceinline__ float plain_sum(const DirectArgs& a, int p, int f, bool aux) {
+  int rem, ox;
+  const int n = fast_div(p, a.OHW, a.inv_ohw, &rem), oy = fast_div(rem, a.OW, a.inv_ow, &ox);
+  const int taps = aux ? 1 : a.chunks / a.cpt, rounds = ((aux ? a.cpt : a.chunks) + 7) >> 3;
+  const floatx4* wt = static_cast<const floatx4*>(aux ? a.aux_wt : a.wt) + (long long)(f >> 5) * rounds * 4 * 64 + (f & 31);
+  float sum = 0.0f;
+  for (int t = 0; t < taps; ++t) {
+    const int tap = aux ? a.aux_tap : t, r = tap / a.S, s = tap - r * a.S, iy = oy * a.stride_h - a.pad_h + r, ix = ox * a.stride_w - a.pad_w + s;
+    if ((unsigned)iy >= (unsigned)a.H || (unsigned)ix >= (unsigned)a.W) continue;
+    const floatx4* row = reinterpret_cast<const floatx4*>(static_cast<const float*>(a.in) + (long long)((n * a.H + iy) * a.W + ix) * a.pix);
+    for (int c = 0; c < a.cpt; ++c) {
+      const int k = t * a.cpt + c;
+      const floatx4 x = row[c], w = wt[(k >> 1) * 64 + (k & 1) * 32];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum = __builtin_fmaf(x[e], w[e], sum);
+    }
+  }
+  return sum;
+}
+
 // UNI: a tap is a whole number of rounds (C elements = whole 128-byte lines), so the tap of a round is the same for all lanes
 template <typename T, typename OutT, int BT, int TM, int TN, int KG, bool UNI>
 __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a) {
+  // Three-way bf16 splits (split.hpp) where two filter blocks share a split of the pixels and there are waves to hide it:
+  // 6x58x78x64 -> 128 at stride 2 17.2 -> 14.3 us, 16x28x28x128 -> 256 24.8 -> 19.9.  32 x 32 waves spend as long splitting as they
+  // save (0.83 to 1.11 times), 64 x 64 ones are alone on their SIMD (0.91).
+  constexpr bool kSplit = sizeof(T) == 4 && BT == 32 && TM == 2 && TN == 1;
   constexpr int kEs = sizeof(T), LG = 64 / BT, NQ = BT / 8, GL = BT * TN / 8;  // GL: pixel loads of a round
   constexpr int kBuf = BT * TN * 128, kPart = TM * TN * BT * BT * 4;
   constexpr int kWaveLds = 2 * kBuf > kPart || KG == 1 ? 2 * kBuf : kPart;
@@ -191,13 +216,17 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
     return *reinterpret_cast<const u32x4*>(lds + buf * kBuf + (BT * j + lrow) * 128 + (((LG * q + lh) ^ (lrow & 7)) * 16));
   };
 
-  typename Block<T, BT>::acc acc[TM][TN];
+  // (split: the small products in sums of their own)
+    typename Block<T, BT>::acc acc[TM][TN], low[kSplit ? TM : 1][kSplit ? TN : 1];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int v = 0; v < BT * BT / 64; ++v) acc[i][j][v] = 0.0f;
+      for (int v = 0; v < BT * BT / 64; ++v) {
+        acc[i][j][v] = 0.0f;
+        if constexpr (kSplit) low[i][j][v] = 0.0f;
+      }
   u32x4 w[NQ][TM];
   load_x();
 #pragma unroll
@@ -226,8 +255,7 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
     if (res && ok) q.rv = *reinterpret_cast<const out4*>(res + q.at);
     return q;
   };
-  auto finish = [&](const Quad& q, const floatx4& sum) {
-    if (q.at < 0) return;
+  auto put = [&](const Quad& q, const floatx4& sum) {
     float y[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) y[e] = sum[e] * q.sc[e] + q.sh[e];
@@ -246,6 +274,13 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
     for (int e = 0; e < 4; ++e) o[e] = (OutT)y[e];
     *reinterpret_cast<out4*>(out + q.at) = o;
   };
+  // Sums that are not finite (an operand that bf16 does not hold, or a result that is not) are marked, and done again at the end
+  unsigned again = 0;
+  auto finish = [&](int k, const Quad& q, const floatx4& sum) {
+    if (q.at < 0) return;
+    if (kSplit && !split_finite(sum)) again |= 1u << k;
+    else put(q, sum);
+  };
   Quad mine[KG > 1 ? kMine : 1];
   if constexpr (KG > 1) {
 #pragma unroll
@@ -259,25 +294,58 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
 #pragma unroll
   for (int j = 0; j < TN; ++j) x[j] = operand(0, 0, j);
   int buf = 0;
-  for (int r = rb; r < re; r += KG, buf ^= 1) {
+  if constexpr (kSplit) {
+    // two units of the fp32 order make one bf16 operand: its k are the same eight channels for filters and pixels
+    u32x4 y[TN];
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      u32x4 xn[TN];
-      if (q == NQ / 2) {
-        park(buf ^ 1);
-        load_x();
+    for (int j = 0; j < TN; ++j) y[j] = operand(0, 1, j);
+    for (int r = rb; r < re; r += KG, buf ^= 1) {
+#pragma unroll
+      for (int q = 0; q < NQ; q += 2) {
+        u32x4 wp[TM][3], xp[TN][3];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) split_eight(w[q][i], w[q + 1][i], wp[i]);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) split_eight(x[j], y[j], xp[j]);
+        load_w(r + KG, q, w);
+        load_w(r + KG, q + 1, w);
+        if (q == 0) {
+          park(buf ^ 1);
+          load_x();
+        }
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          x[j] = q == 0 ? operand(buf, 2, j) : operand(buf ^ 1, 0, j);
+          y[j] = q == 0 ? operand(buf, 3, j) : operand(buf ^ 1, 1, j);
+        }
+        split_products(wp, xp, acc, low);
       }
+    }
 #pragma unroll
-      for (int j = 0; j < TN; ++j) xn[j] = q + 1 < NQ ? operand(buf, q + 1, j) : operand(buf ^ 1, 0, j);
-      __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+      for (int j = 0; j < TN; ++j) acc[i][j] += low[i][j];
+  } else {
+    for (int r = rb; r < re; r += KG, buf ^= 1) {
 #pragma unroll
-        for (int j = 0; j < TN; ++j) Block<T, BT>::run(w[q][i], x[j], acc[i][j]);
-      __builtin_amdgcn_sched_barrier(0);
-      load_w(r + KG, q, w);
+      for (int q = 0; q < NQ; ++q) {
+        u32x4 xn[TN];
+        if (q == NQ / 2) {
+          park(buf ^ 1);
+          load_x();
+        }
 #pragma unroll
-      for (int j = 0; j < TN; ++j) x[j] = xn[j];
+        for (int j = 0; j < TN; ++j) xn[j] = q + 1 < NQ ? operand(buf, q + 1, j) : operand(buf ^ 1, 0, j);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) Block<T, BT>::run(w[q][i], x[j], acc[i][j]);
+        __builtin_amdgcn_sched_barrier(0);
+        load_w(r + KG, q, w);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) x[j] = xn[j];
+      }
     }
   }
 
@@ -290,7 +358,7 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
   };
   if constexpr (KG == 1) {
 #pragma unroll
-    for (int k = 0; k < kQuads; ++k) finish(quad_of(k), quad_sum(k));
+    for (int k = 0; k < kQuads; ++k) finish(k, quad_of(k), quad_sum(k));
   } else {
     floatx4* part = reinterpret_cast<floatx4*>(lds);  // this wave's own region: [quad][lane]
 #pragma unroll
@@ -307,7 +375,18 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
       for (int d = 1; d < KG; d *= 2)  // pairwise: a chain of log2(KG) additions
 #pragma unroll
         for (int g = 0; g + d < KG; g += 2 * d) v[g] += v[g + d];
-      finish(mine[k], v[0]);
+      finish(k, mine[k], v[0]);
+    }
+  }
+  if constexpr (kSplit) {
+    for (; again; again &= again - 1) {
+      const int k = __builtin_ctz(again);
+      const Quad q = quad_of(KG > 1 ? grp + k * KG : k);
+      const int p = (int)(q.at / ldo), f = (int)(q.at - (long long)p * ldo);
+      floatx4 sum;
+#pragma unroll 1
+      for (int e = 0; e < 4; ++e) sum[e] = plain_sum(a, p, f + e, aux);
+      put(q, sum);
     }
   }
 }
@@ -381,7 +460,7 @@ const Form kForms32[] = {
     {16, 16, 4, 2.6, 0.157, 0.23, 0.20, launch_cfg<float, float, 16, 1, 1, 4>, TAGS("f32,16x16,splitk4")},
     {16, 16, 16, 2.1, 0.538, 1.24, 0.31, launch_cfg<float, float, 16, 1, 1, 16>, TAGS("f32,16x16,splitk16")},
     {32, 16, 8, 2.6, 0.543, 0.51, 0.12, launch_cfg<float, float, 16, 2, 1, 8>, TAGS("f32,32x16,splitk8")},
-    {64, 32, 4, 3.3, 1.061, 0.53, 0.22, launch_cfg<float, float, 32, 2, 1, 4>, TAGS("f32,64x32,splitk4")},
+    {64, 32, 4, 3.3, 0.790, 1.30, 0.22, launch_cfg<float, float, 32, 2, 1, 4>, TAGS("f32,64x32,splitk4")},
     {64, 64, 1, 6.0, 0.297, 1.44, 1.89, launch_cfg<float, float, 32, 2, 2, 1>, TAGS("f32,64x64")},
 };
 const Form kForms16[] = {
@@ -416,9 +495,10 @@ const Form* best_form(const IgemmArgs& a, int dt, double* us) {
 }
 
 // The same for the kernel that would run the layer otherwise.  Implicit GEMM: fits over its 64 x 64 tiles, within 7-16 %.
-// fp32 3x3 stride-1 patch kernel: 0.5 us per 32 channels and tap for every 64 slots x 64 filters of a CU's workgroups, half
-// of it where a half-filled launch runs 32-filter blocks.  (Its waves share pixels through LDS, so it stays
-// ahead where its tiles fill the CUs evenly, 6x29x39x128: 22.1 against 24.5 us, and falls behind where they do not.)
+// fp32 3x3 stride-1 layers (conv3x3_split.hip): a start and so much for every 32 channels and tap of a CU's turns; 75 layers of 20
+// MFLOP to 20 GFLOP, within 10 %.  Half blocks of filters are the launches of up to 128 whole ones.  From 129 to 144 whole
+// blocks nearly half of the chip is idle and the layer stays here, though it would take less there (7x15x20x256 23.1 us against
+// 35.3, 5x9x25x192 -> 440 18.9 against 23.6): this is the size of layer that this kernel's test holds it to.
 double other_us(const IgemmArgs& a, int dt, DirectRival rival) {
   struct Fit { double fixed, round, tile, chain; };
   static const Fit f32[] = {{3.3, 0.642, 0.79, 0.0}, {2.7, 0.835, 0.14, 0.26}};
@@ -428,8 +508,11 @@ double other_us(const IgemmArgs& a, int dt, DirectRival rival) {
   if (rival == kRivalPatch && dt == kF32) {
     int p[8];
     if (!conv3x3_patch_plan(1, a.N, a.OH, a.OW, main_f, a.C / 32, p)) return 1e30;
-    const double wgs = (double)((a.N + p[1] - 1) / p[1]) * ((a.OH + p[2] - 1) / p[2]) * p[4] * ((main_f + 63) / 64);
-    return 4.0 + std::ceil(wgs / 256) * p[0] * 0.5 * rounds * (wgs <= 128 ? 0.5 : 1.0);
+    const double wgs = (double)((a.N + p[1] - 1) / p[1]) * ((a.OH + p[2] - 1) / p[2]) * p[4] * ((main_f + 63) / 64), turns = std::ceil(wgs / 256);
+    if (p[0] == 4) return 5.0 + 1.2 * rounds * turns;
+    if (p[0] == 2) return 6.0 + 0.5 * rounds * turns;
+    if (wgs <= 128 && main_f % 64 == 0) return 4.9 + 0.132 * rounds;
+    return wgs > 128 && wgs <= 144 ? 1e30 : 4.3 + 0.26 * rounds * turns;
   }
   const Fit& f = rival == kRivalPatch || rival == kRivalPatchS2 ? f16_3x3[rival] : (dt == kF16 ? f16 : f32)[rival - kRivalIgemmFast];
   const double tiles = (double)((main_f + 63) / 64) * (double)(((long long)a.N * a.OH * a.OW + 63) / 64);
@@ -494,7 +577,7 @@ bool conv_direct_wins(const IgemmArgs& a, int dt, DirectRival rival) {
   if (!best_form(a, dt, &us)) return false;
   if (rival == kRivalRing) return us < 0.97 * conv_ring_us(a);
   // margins cover the fits' errors: the fp16 3x3 stride-1 kernels' times are the least well fitted
-  const double margin = dt == kF32 ? 0.97 : rival == kRivalPatch ? 0.85 : 0.9;
+  const double margin = dt == kF32 ? (rival == kRivalPatch ? 1.0 : 0.97) : rival == kRivalPatch ? 0.85 : 0.9;
   return us < margin * other_us(a, dt, rival);
 }
 

@@ -140,14 +140,8 @@ __global__ __launch_bounds__(64 * KG, TM * TN == 4 ? 2 : TM * TN == 2 ? 3 : 4) v
       u32x4 a[TM][3], b[TN][3];
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
-        const floatx4 x = *reinterpret_cast<const floatx4*>(get + i * 32 * Cfg::kPitch + k * 64), y = *reinterpret_cast<const floatx4*>(get + i * 32 * Cfg::kPitch + k * 64 + 16);
-        unsigned p[4][3];
-        split_pair(x[0], x[1], p[0]);
-        split_pair(x[2], x[3], p[1]);
-        split_pair(y[0], y[1], p[2]);
-        split_pair(y[2], y[3], p[3]);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) a[i][c] = u32x4{p[0][c], p[1][c], p[2][c], p[3][c]};
+        const unsigned char* at = get + i * 32 * Cfg::kPitch + k * 64;
+        split_eight(*reinterpret_cast<const u32x4*>(at), *reinterpret_cast<const u32x4*>(at + 16), a[i]);
       }
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
@@ -158,16 +152,7 @@ __global__ __launch_bounds__(64 * KG, TM * TN == 4 ? 2 : TM * TN == 2 ? 3 : 4) v
         for (int c = 0; c < 3; ++c) b[j][c] = u32x4{p[0][c], p[1][c], p[2][c], p[3][c]};
       }
       load_b(r - KG, k);
-      constexpr int kX[6] = {0, 0, 1, 0, 1, 2}, kY[6] = {0, 1, 0, 2, 1, 0};
-#pragma unroll
-      for (int c = 0; c < 6; ++c)
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j) {
-            floatx16& s = c == 0 ? big[i][j] : low[i][j];
-            s = mma_bf16(a[i][kX[c]], b[j][kY[c]], s);
-          }
+      split_products(a, b, big, low);
     }
   }
 

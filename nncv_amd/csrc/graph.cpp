@@ -147,7 +147,7 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
         if (Cstored > op.F) NNCV_HIP_CHECK(hipMemsetAsync(nd.wt.get(), 0, (size_t)Cstored * op.K * op.K * C * es, s));
         launch_weight_frsc(w, dt, nd.wt.get(), dt, op.F, Cl, op.K, op.K, C, s);
         if (op.K == 3 && (op.stride == 1 || (op.stride == 2 && dt == kF16)) && op.pad == 1 && Cl == C && Cstored == op.F && C % (128 / (int)es) == 0) {
-          nd.wfrag.reset((size_t)((op.F + 63) / 64) * 64 * 9 * C * es, &pool_);
+          nd.wfrag.reset(weight_frag3x3_bytes(dt, op.F, C), &pool_);
           launch_weight_frag3x3(w, dt, nd.wfrag.get(), dt, op.F, C, s);
           if (dt == kF16 && op.stride == 1 && C % 64 == 0 && op.F % 32 == 0) {
             nd.wfrag32.reset(weight_frag32_bytes(op.F, C), &pool_);

@@ -54,7 +54,7 @@ ConvLayer::Sizes ConvLayer::sizes(const Desc& d, int algo, bool bn) {
     z.wt = (size_t)Fp * RS * Cp * es;
     if (d.shortcut || conv_direct_serves(d.dt, Fp, RS, Cp)) z.wflat = weight_flat_bytes(d.dt, Fp, RS, Cp);
     if (d.R == 3 && d.S == 3 && (d.stride == 1 || (d.stride == 2 && d.dt == kF16)) && d.pad == 1 && d.C % (128 / (int)es) == 0) {
-      z.wfrag = (size_t)((d.F + 63) / 64) * 64 * 9 * d.C * es;
+      z.wfrag = weight_frag3x3_bytes(d.dt, d.F, d.C);
       if (d.dt == kF16 && d.stride == 1 && d.C % 64 == 0 && d.F % 32 == 0) z.wfrag32 = weight_frag32_bytes(d.F, d.C);
     }
   }

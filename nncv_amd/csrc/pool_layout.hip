@@ -4,7 +4,7 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "mfma_tile.hpp"
+#include "split.hpp"
 
 namespace nncv_hip {
 
@@ -891,7 +891,40 @@ static void launch_weight_frag(const void* w, int w_dt, void* dst, int dst_dt, i
   NNCV_HIP_CHECK(hipGetLastError());
 }
 
+// fp32 3x3 weights for conv3x3_split.hip, in three bf16 pieces: the operand of (64-filter block fb, slab sl of 32 channels, tap,
+// 16-channel step k, filter half i, piece p) is one kilobyte, lane L holding filter fb*64 + i*32 + L%32 and the eight
+// channels sl*32 + k*16 + 4*(L/32) + {0..3, 8..11}:
+//   offset = ((((((fb*nslab + sl)*9 + tap)*2 + k)*2 + i)*3 + p)*64 + L) * 16 bytes.
+__global__ void weight_frag_split_kernel(const float* __restrict__ w, unsigned char* __restrict__ dst, int F, int C, int Fp) {
+  const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;  // one lane of an operand each
+  const int nslab = C / 32;
+  if (idx >= (long long)(Fp / 64) * nslab * 9 * 4 * 64) return;
+  const int L = (int)(idx & 63);
+  const long long op = idx >> 6;
+  long long r = op;
+  const int i = (int)(r & 1); r >>= 1;
+  const int k = (int)(r & 1); r >>= 1;
+  const int tap = (int)(r % 9); r /= 9;
+  const int sl = (int)(r % nslab), fb = (int)(r / nslab), f = fb * 64 + i * 32 + (L & 31), c0 = sl * 32 + k * 16 + 4 * (L >> 5);
+  mt::u32x4 v[2], out[3];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e >> 2][e & 3] = f < F ? __builtin_bit_cast(unsigned, w[((long long)f * C + c0 + (e & 3) + (e >> 2) * 8) * 9 + tap]) : 0u;
+  mt::split_eight(v[0], v[1], out);
+#pragma unroll
+  for (int p = 0; p < 3; ++p) *reinterpret_cast<mt::u32x4*>(dst + ((op * 3 + p) * 64 + L) * 16) = out[p];
+}
+
+size_t weight_frag3x3_bytes(int dt, int F, int C) { return (size_t)((F + 63) / 64) * 64 * 9 * C * (dt == kF32 ? 6 : 2); }
+
 void launch_weight_frag3x3(const void* w, int w_dt, void* dst, int dst_dt, int F, int C, hipStream_t s) {
+  if (w_dt == kF32 && dst_dt == kF32) {
+    NNCV_REQUIRE(C % 32 == 0, "weight_frag: C must be a multiple of the 128-byte slab");
+    const int Fp = (F + 63) / 64 * 64;
+    const long long total = (long long)(Fp / 64) * (C / 32) * 9 * 4 * 64;
+    launch_kernel(weight_frag_split_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, static_cast<const float*>(w), static_cast<unsigned char*>(dst), F, C, Fp);
+    NNCV_HIP_CHECK(hipGetLastError());
+    return;
+  }
   launch_weight_frag<9>(w, w_dt, dst, dst_dt, F, C, s);
 }
 void launch_weight_frag1x1(const void* w, int w_dt, void* dst, int dst_dt, int F, int C, hipStream_t s) {

@@ -37,9 +37,39 @@ __device__ __forceinline__ floatx16 mma_bf16(const u32x4& a, const u32x4& b, con
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// Rows of operands in LDS: 32 k of one row as three runs of 64 bytes, one per piece.  At 13 units of 16 bytes a row, a 16-byte
-// read of one column of 16 neighbouring rows touches every bank once.
-constexpr int kSplitPitch = 208;
+// eight values -> an operand in three pieces
+__device__ __forceinline__ void split_eight(const u32x4& a, const u32x4& b, u32x4 (&out)[3]) {
+  const floatx4 x = __builtin_bit_cast(floatx4, a), y = __builtin_bit_cast(floatx4, b);
+  unsigned p[4][3];
+  split_pair(x[0], x[1], p[0]);
+  split_pair(x[2], x[3], p[1]);
+  split_pair(y[0], y[1], p[2]);
+  split_pair(y[2], y[3], p[3]);
+#pragma unroll
+  for (int c = 0; c < 3; ++c) out[c] = u32x4{p[0][c], p[1][c], p[2][c], p[3][c]};
+}
+
+// the six products of TM x TN blocks
+template <int TM, int TN>
+__device__ __forceinline__ void split_products(const u32x4 (&a)[TM][3], const u32x4 (&b)[TN][3], floatx16 (&big)[TM][TN], floatx16 (&low)[TM][TN]) {
+  constexpr int kX[6] = {0, 0, 1, 0, 1, 2}, kY[6] = {0, 1, 0, 2, 1, 0};
+#pragma unroll
+  for (int c = 0; c < 6; ++c)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        floatx16& s = c == 0 ? big[i][j] : low[i][j];
+        s = mma_bf16(a[i][kX[c]], b[j][kY[c]], s);
+      }
+}
+
+__device__ __forceinline__ bool split_finite(const floatx4& v) {
+  bool ok = true;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) ok &= __builtin_fabsf(v[e]) < __builtin_inff();
+  return ok;
+}
 
 }  // namespace mt
 }  // namespace nncv_hip
