@@ -1,5 +1,5 @@
 // fp16 3x3 stride-1 pad-1 convolution + BN/residual/activation for gfx950: the stream form of the LDS-patch
-// kernel (conv3x3_patch.hip keeps every other case: fp32, stride 2, odd channel counts, wide rows, more than 256
+// kernel (conv3x3_patch.hip keeps every other case: stride 2, odd channel counts, wide rows, more than 512
 // channels, and launches too small to fill the CUs, where its shorter prologue wins).
 // Replaces what ModernTile.cpp:184-199 + ModernVec.cpp:54-62 emit for linalg.conv_2d_nchw_fchw
 // (tests/Nets/Res18.mlir:157 ...) together with the BN / add / ReLU generics behind it (:127-142, :193-203).
@@ -19,7 +19,8 @@
 //  * Rows of all images are stacked into one column of "virtual rows"; a tile is TH consecutive virtual
 //    rows.  Either every image takes a whole number of tiles (aligned form), or the images are one zero
 //    row apart and tiles run across image borders (gap form: that shared row is the halo of both images);
-//    14x14 and 7x7 images fill 126 of 128 slots that way instead of 98.
+//    14x14 images fill 126 of 128 slots that way instead of 98, and a tile of 7x7 ones is 16 rows of two images and more
+//    (112 slots instead of 49).
 //  * Patch cells (the 64 channels of one pixel, 128 bytes) are 144 bytes apart in LDS, which keeps the 16-byte
 //    reads of 16 neighbouring cells off each other's banks (64 banks of 4 bytes: a read is conflict-free when its
 //    16-byte units differ mod 16 within every 16 lanes, and 9 is odd).  Consecutive pixel slots wrap from the
@@ -493,14 +494,24 @@ __global__ __launch_bounds__(64 * PG * WF * WK) __attribute__((amdgpu_waves_per_
             if (j / NOWN == wk && (NR == 1 || j / 2 == round) && (PG == 1 || j < nrows)) {
               const int jx = NR == 1 ? j : (j & 1), nj = NR == 1 ? 4 : 2;
               const unsigned char* src = xb + ((((pg * WF + wf) * nj + jx) * (WK - 1)) * 4) * 1024 + lane * 16;
-#pragma unroll
-              for (int r = 0; r < WK - 1; ++r)
+              if constexpr (WK == 2) {
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                  const floatx4 p = *reinterpret_cast<const floatx4*>(src + (r * 4 + q) * 1024);
+                  const floatx4 p = *reinterpret_cast<const floatx4*>(src + q * 1024);
 #pragma unroll
                   for (int e = 0; e < 4; ++e) acc[j][4 * q + e] += p[e];
                 }
+              } else {
+                // (0 + 1) + (2 + 3) whoever adds: a pixel's bits do not depend on its slot, i.e. on where its image is in the batch
+                const int mate = wk < 2 ? 0 : 2, far = wk < 2 ? 1 : 0;  // ranks
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                  const floatx4 p = *reinterpret_cast<const floatx4*>(src + (mate * 4 + q) * 1024);
+                  const floatx4 x = *reinterpret_cast<const floatx4*>(src + (far * 4 + q) * 1024), y = *reinterpret_cast<const floatx4*>(src + ((far + 1) * 4 + q) * 1024);
+#pragma unroll
+                  for (int e = 0; e < 4; ++e) acc[j][4 * q + e] = (acc[j][4 * q + e] + p[e]) + (x[e] + y[e]);
+                }
+              }
             }
           }
         }
@@ -582,14 +593,12 @@ unsigned recip32(unsigned d) { return d == 1 ? 0u : (unsigned)(0xffffffffull / d
 // TH consecutive virtual rows of W columns per tile: at most `slots` pixels, and a patch of TH + 2 rows of
 // NSEG segments within `segcap`.  Aligned form: S = bands * TH >= H virtual rows per image, tiles never
 // leave their image.  Gap form: S = H + 1 (one shared zero row between images), tiles of the largest TH
-// that fits.  The form with fewer tiles wins; aligned on a tie (it wastes no slot on the zero rows).
+// that fits, be it several images.  The form with fewer tiles wins; aligned on a tie (it wastes no slot on the zero rows).
 bool stream_geometry(int N, int H, int W, int slots, int segcap, StreamGeom* g) {
   if (N < 1 || H < 1 || W < 1 || W > slots || H > 254 || N >= (1 << 24)) return false;
   const int NSEG = (W + 2 + kSegCells - 1) / kSegCells;
-  int thmax = 0;
-  for (int th = 1; th <= H + 1; ++th)
-    if (th * W <= slots && (th + 2) * NSEG <= segcap) thmax = th;
-  if (thmax == 0) return false;
+  const int thmax = std::min(slots / W, segcap / NSEG - 2);  // (in the gap form a tile may hold several small images)
+  if (thmax <= 0) return false;
   const int tha0 = std::min(thmax, H);
   const int bands = (H + tha0 - 1) / tha0, tha = (H + bands - 1) / bands;
   const long long tiles_a = (long long)N * bands;
@@ -746,10 +755,9 @@ bool conv3x3_stream_plan(int N, int H, int W, int C, int F, int out[14]) {
 
 bool conv3x3_stream_applicable(const IgemmArgs& a, int in_dt, int out_dt) {
   static const bool off = getenv("NNCV_HIP_NO_STREAM") != nullptr;
-  // The deepest layers (eight channel slabs per tile, few pixels) stay with the patch kernel unless asked for: 16.6 us
-  // here against 13.1 there on 7x7x512 at batch 32; up to 256 channels this kernel is 5-8 % ahead.
   static const bool all = getenv("NNCV_HIP_STREAM_ALL") != nullptr;
-  if (off || in_dt != kF16 || out_dt != kF16 || !a.wt_frag32 || (a.C > 256 && !all)) return false;
+  // (up to 512 channels is what the two kernels were compared on)
+  if (off || in_dt != kF16 || out_dt != kF16 || !a.wt_frag32 || (a.C > 512 && !all)) return false;
   const int pix = a.pix_stride ? a.pix_stride : a.C;
   const bool act_ok = a.relu <= kActRelu || ((a.relu & 0xff) <= kActSigmoid && (a.relu & ~(0xff | kActResidualAfter)) == 0);
   StreamConfig c;
@@ -769,7 +777,12 @@ bool conv3x3_stream_applicable(const IgemmArgs& a, int in_dt, int out_dt) {
   // layer, whose 64-filter form keeps the weights in registers (204.4 k images/s with layer1 on the patch kernel,
   // 212.6 k here, same box).
   if (!all && overlap_hint() >= 3 && a.relu <= kActRelu && c.WF != 4 && !(a.C == 64 && c.WF == 2 && c.PG == 1)) return false;
-  return all || (fine_wgs >= 160 && c.geo.TH * a.W >= 96);
+  // From five slabs up the line lies at 320: 1.04 to 1.5 times as fast here on 30 layers of 320 to 512 channels above it
+  // (256x7x7x512 79.4 -> 62.0 us, 48 of them 20.4 -> 16.8, 64x14x14x512 74.4 -> 58.5, 12x32x32x320 32.7 -> 23.0).  Below, where both
+  // kernels wait for the weights (32x7x7x512, 256: 12.2 against 13.1; seven others 1.02 to 1.1), the patch kernel keeps
+  // what ResNet-18 at batch 32 is checked to run.  A tile of 96 slots is too few there: 174x19x6x384 74 against 62.
+  const bool deep = a.C > 256;
+  return all || (fine_wgs >= (deep ? 320 : 144) && c.geo.TH * a.W >= (deep ? 100 : 96));
 }
 
 template <int PG, int WF, int WK, bool ACT, bool RES = false>
