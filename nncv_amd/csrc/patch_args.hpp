@@ -16,7 +16,6 @@ template <> struct PatchCap<1> { static constexpr int pix = 192; };
 struct PatchArgs {
   const void* in;        // NHWC [N][H][W][C]
   const void* wf;        // fragment-major weights (launch_weight_frag3x3)
-  const void* wt;        // the same as rows [F][9][C] (fp32 only)
   void* out;             // NHWC [N][H][W][F]
   const float* scale;    // [F] or null
   const float* shift;    // [F] or null
@@ -43,6 +42,7 @@ struct PatchArgs {
   int aux_F, aux_relu, aux_fb0;
   int aux_inline;  // the workgroup of filter block b also computes block b of the auxiliary filters (aux_F == F): no extra blocks
   unsigned aux_wf_bytes;
+  const void* wt;  // fp32 only: the filters as rows [F][9][C] (behind the fields that the fp16 kernel loads)
 };
 
 // The fp32 kernel (conv3x3_split.hip): 64 ws pixel slots, 64 filters (half: 32) a workgroup
