@@ -374,20 +374,22 @@ struct SeArgs {
 bool se_block_applicable(int dt, int HW, int C, int SQ);
 void launch_se_block(const SeArgs& a, int dt, hipStream_t s);
 // Inverted-residual blocks in fp16 (mobile_block.hip).  dw_block: out = act(dw(act1(w1 . in))), Cin = 0: no expansion (in has C
-// channels); sums (or null): fp32 channel sums of out, [N][bands][C], where dw_block_bands says how many (0: shape not
-// covered).  se_project: out = act(wp . (x * act2(w2 . act1(w1 . mean(x) + b1) + b2))), mean from those sums.
+// channels); parts (or null): sq_w . channel sums of out, fp32, [N][bands][groups of 32 channels][SQ], where dw_block_bands says
+// how many bands (0: shape not covered).  se_project: out = act(wp . (x * act2(w2 . act1(w1 . mean(x) + b1) + b2))), w1 . mean(x)
+// from those parts.
 struct DwBlockArgs {
   const void* in; const void* w1; const float* scale1; const float* shift1;  // [N][H][W] pixels of `pix` elements; [C][Cin]
   const void* wt; const float* scale; const float* shift;                    // [K*K][C]
-  void* out; float* sums;
+  void* out; float* parts;
   int N, H, W, pix, Cin, C, K, stride, pad, OH, OW, act1, act;
   int rows, bands, pitch, cells;  // filled in by the launcher, as are these
   float inv_w, inv_strips;
+  const void* sq_w; int SQ;       // [C][SQ]
 };
 int dw_block_bands(int N, int H, int W, int Cin, int C, int K, int S, int pad);
 void launch_dw_block(const DwBlockArgs& a, hipStream_t s);
 struct SeProjectArgs {
-  const void* x; const float* sums; const void* w1t; const float* b1; const void* w2t; const float* b2;  // transposed: [C][SQ], [SQ][C]
+  const void* x; const float* parts; const float* b1; const void* w2t; const float* b2;          // [SQ][C]
   const void* wp_flat; const float* scale; const float* shift; const void* residual; void* out;          // launch_weight_flat's order
   int N, HW, C, SQ, F, bands, act1, act2, act;  // act: may carry kActResidualAfter
   int tiles; float inv_sq, inv_c;               // filled in by the launcher

@@ -537,8 +537,9 @@ const Graph::Plan& Graph::plan_of(int N, int H, int W) const {
       life[nodes_[i].op.out].first_op = i;
       life[nodes_[i - 1].op.out] = TensorLife{i, i, 0, 0};
     }
-    if (p.se[i]) {  // the channel sums, from the depthwise launch on; the gated tensor is never stored
-      life[nodes_[i].op.out] = TensorLife{nodes_[i - 1].expands >= 0 ? i - 1 : i, i + 1, (size_t)N * p.dw[i - 1] * p.dims[nodes_[i].op.in[0]].C * 4, 0};
+    if (p.se[i]) {  // parts of the squeezed vector, from the depthwise launch on; the gated tensor is never stored
+      const size_t parts = (size_t)N * p.dw[i - 1] * ((p.dims[nodes_[i].op.in[0]].C + 31) / 32);
+      life[nodes_[i].op.out] = TensorLife{nodes_[i - 1].expands >= 0 ? i - 1 : i, i + 1, parts * nodes_[i + 1].op.F * 4, 0};
       life[nodes_[i + 3].op.out] = TensorLife{i + 1, i + 1, 0, 0};
       life[nodes_[i + 4].op.out].first_op = i + 1;
     }
@@ -808,7 +809,10 @@ void Graph::forward_body(const void* src, int N, int H, int W, void* ws, hipStre
         d.w1 = e->wt.get(); d.scale1 = e->scale.as<float>(); d.shift1 = e->shift.as<float>();
         d.Cin = p.dims[src].C; d.act1 = e->op.act;
       }
-      d.sums = i + 1 < nodes_.size() && p.se[i + 1] ? static_cast<float*>(at(nodes_[i + 1].op.out)) : nullptr;
+      if (i + 1 < nodes_.size() && p.se[i + 1]) {
+        d.parts = static_cast<float*>(at(nodes_[i + 1].op.out));
+        d.sq_w = nodes_[i + 2].wt_t.get(); d.SQ = nodes_[i + 2].op.F;
+      }
       d.N = N; d.H = a.H; d.W = a.W; d.C = a.C; d.K = op.K; d.stride = op.stride; d.pad = op.pad; d.OH = o.H; d.OW = o.W; d.act = op.act;
       launch_dw_block(d, s);
       continue;
@@ -816,8 +820,8 @@ void Graph::forward_body(const void* src, int N, int H, int W, void* ws, hipStre
     if (p.se[i]) {
       const Node &f1 = nodes_[i + 1], &f2 = nodes_[i + 2], &pr = nodes_[i + 4];
       SeProjectArgs e{};
-      e.x = at(op.in[0]); e.sums = static_cast<const float*>(at(op.out)); e.bands = p.dw[i - 1];
-      e.w1t = f1.wt_t.get(); e.b1 = f1.shift.as<float>(); e.w2t = f2.wt_t.get(); e.b2 = f2.shift.as<float>(); e.act1 = f1.op.act; e.act2 = f2.op.act;
+      e.x = at(op.in[0]); e.parts = static_cast<const float*>(at(op.out)); e.bands = p.dw[i - 1];
+      e.b1 = f1.shift.as<float>(); e.w2t = f2.wt_t.get(); e.b2 = f2.shift.as<float>(); e.act1 = f1.op.act; e.act2 = f2.op.act;
       e.wp_flat = pr.wflat.get(); e.scale = pr.scale.as<float>(); e.shift = pr.shift.as<float>(); e.out = at(pr.op.out);
       e.residual = pr.op.in[1] >= 0 ? at(pr.op.in[1]) : nullptr;
       e.N = N; e.HW = a.H * a.W; e.C = a.C; e.SQ = f1.op.F; e.F = pr.op.F; e.act = pr.op.act;

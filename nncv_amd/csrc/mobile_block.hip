@@ -1,14 +1,24 @@
 // fp16 inverted-residual blocks (MobileNetV3.mlir:260-420) in two launches instead of four or five.
 //
-//  1. dw_block: 1x1 expansion + BN + activation -> depthwise 3x3 / 5x5 + BN + activation, and the channel sums of the result.
-//  2. se_project: squeeze-excitation gate from those sums, gated 1x1 projection + BN, residual.
+//  1. dw_block: 1x1 expansion + BN + activation -> depthwise 3x3 / 5x5 + BN + activation, and what the workgroup's channel sums
+//     add to the squeezed vector.
+//  2. se_project: the squeezed vector from those parts, the gate, gated 1x1 projection + BN, residual.
 //
 // The layers are far too small to be bound by anything but launches and dependent loads: 14x14x240 at batch 32 is 3 MB and
-// 0.1 GFLOP and took 5.5 (expansion) + 15.5 (depthwise) + 11.4 (gate) + 5 us (projection) in a kernel each; it takes 9.0 + 8.7
-// here (7x7x576: 5.5 + 11.6 + 19.0 + 5.0 -> 9.4 + 15.0).  What is kept on chip is the expanded image (its values rounded to
+// 0.1 GFLOP and took 5.5 (expansion) + 15.5 (depthwise) + 11.4 (gate) + 5 us (projection) in a kernel each; it takes 9.3 + 6.9
+// here (7x7x576: 5.5 + 11.6 + 19.0 + 5.0 -> 10.2 + 9.3).  What is kept on chip is the expanded image (its values rounded to
 // fp16 as they were when they went through memory), the pooled and squeezed vectors and the gate (fp32), and the gated image
-// (fp16).  Of dw_block's 8.3 us, 2.4 are the launch, its first loads and zeros, 0.9 the expansion, 4 the depthwise part and
-// the stores, 1 the channel sums.
+// (fp16).
+//
+// The squeeze is linear in the pooled vector, so every dw_block workgroup puts its 32 channel sums through their 32 rows of
+// the squeeze weights (4 multiply-adds a thread at SQ = 32) and se_project adds up bands * C / 32 vectors of SQ elements.  With
+// the sums handed over instead, each of se_project's workgroups went through all C x SQ weights: 166 KB at 7x7x576, and
+// 9.4 + 15.0 us; 9.0 + 8.7 at 14x14x240.  (The vectors are as many bytes as the weights at 16 bands; an image has 1 to 4 where
+// C is above 200.)
+//
+// A 7x7x576 workgroup of dw_block spends 2200 clocks on its requests (mostly instruction and argument fetches: they are asked
+// for at once, and what is the same for all threads is not worked out by branches), 2200 until the operands are there, 1300 on
+// the expansion, 3700 on the depthwise part and the stores, 1400 on the sums and the squeeze.
 #include "mfma_tile.hpp"
 
 namespace nncv_hip {
@@ -19,12 +29,69 @@ namespace {
 
 constexpr unsigned kOOBm = 0x7fffff00u;  // byte offset beyond any buffer these kernels accept
 constexpr int kDwThreads = 256;
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
 __device__ __forceinline__ half8 as_half8(const u32x4& v) { return __builtin_bit_cast(half8, v); }
 
 // LDS cells of one pixel x 32 channels: 64 bytes, 16-byte chunk c at position c ^ (cell / 2) % 4, so that neither the
 // 16-byte reads of four lanes per pixel nor the 8-byte writes of one lane per pixel pile up on a few banks
 __device__ __forceinline__ int cell_at(int cell, int chunk) { return cell * 64 + ((chunk ^ ((cell >> 1) & 3)) << 4); }
+
+// Sums over lanes that each hold eight elements.  Every step hands half of the elements over to the lane that goes on with
+// them, by moves within the vector unit: seven exchanges where sums of all elements in all lanes take 24 trips through LDS.
+template <int CTRL>
+__device__ __forceinline__ float lane_move(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+constexpr int kQuadXor1 = 0xb1, kQuadXor2 = 0x4e, kQuadXor3 = 0x1b, kRowRor8 = 0x128, kHalfMirror = 0x141;
+// over lanes l, l ^ 1, .. l ^ 7: lane l returns element l & 7
+__device__ __forceinline__ float sum_of_eight(const float (&v)[8], int lane) {
+  float a[4], b[2];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float lo = v[e], hi = v[e + 4];
+    a[e] = (lane & 4 ? hi : lo) + lane_move<kHalfMirror>(lane & 4 ? lo : hi);
+  }
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const float lo = a[e], hi = a[e + 2];
+    b[e] = (lane & 2 ? hi : lo) + lane_move<kQuadXor2>(lane & 2 ? lo : hi);
+  }
+  const float lo = b[0], hi = b[1];
+  return (lane & 1 ? hi : lo) + lane_move<kQuadXor1>(lane & 1 ? lo : hi);
+}
+// over the sixteen lanes with the same l & 3: lane l returns element l >> 3
+__device__ __forceinline__ float sum_of_sixteen(const float (&v)[8], int lane) {
+  float a[4], b[2];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v[e]), __builtin_bit_cast(unsigned, v[e + 4]), false, false);
+    const unsigned r0 = r[0], r1 = r[1];  // (a bit_cast of r[1] itself takes element 0)
+    a[e] = __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1);
+  }
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a[e]), __builtin_bit_cast(unsigned, a[e + 2]), false, false);
+    const unsigned r0 = r[0], r1 = r[1];
+    b[e] = __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1);
+  }
+  const float lo = b[0], hi = b[1], s = (lane & 8 ? hi : lo) + lane_move<kRowRor8>(lane & 8 ? lo : hi);
+  return s + lane_move<kQuadXor3>(lane_move<kHalfMirror>(s));  // l ^ 7 ^ 3
+}
+
+// BatchNorm of channels c + STEP q .. + 3, q < Q
+template <int Q, int STEP>
+__device__ __forceinline__ void batch_norm(const float* scale, const float* shift, int C, int c, floatx4 (&sc)[Q], floatx4 (&sh)[Q]) {
+  const __amdgpu_buffer_rsrc_t rs_sc = make_rsrc(scale, scale ? (unsigned)C * 4u : 0u), rs_sh = make_rsrc(shift, shift ? (unsigned)C * 4u : 0u);
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    sc[q] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs_sc, (unsigned)(c + STEP * q) * 4u, 0, 0));
+    sh[q] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs_sh, (unsigned)(c + STEP * q) * 4u, 0, 0));
+  }
+  if (!scale)
+#pragma unroll
+    for (int q = 0; q < Q; ++q) sc[q] = floatx4{1.f, 1.f, 1.f, 1.f};
+}
 
 }  // namespace
 
@@ -36,24 +103,26 @@ template <int K, int S, int OXT, int KST>
 __global__ __launch_bounds__(kDwThreads) void dw_block_kernel(const DwBlockArgs a) {
   constexpr int LW = (OXT - 1) * S + K;
   extern __shared__ __align__(16) unsigned char smem[];  // cells, then the taps [K * K][32 channels]
+  // all arguments at once: fetched where they are first used, they are one wait after the other
+  asm volatile("" ::"s"(a.in), "s"(a.w1), "s"(a.scale1), "s"(a.shift1), "s"(a.wt), "s"(a.scale), "s"(a.shift), "s"(a.H), "s"(a.W), "s"(a.pix), "s"(a.Cin), "s"(a.C),
+               "s"(a.pad), "s"(a.OH), "s"(a.rows), "s"(a.pitch), "s"(a.cells), "s"(a.parts), "s"(a.sq_w), "s"(a.SQ), "s"(a.inv_w),
+               "s"(a.out), "s"(a.OW), "s"(a.act), "s"(a.act1), "s"(a.inv_strips), "s"(a.bands));
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int groups = (a.C + 31) >> 5;
-  const int g = blockIdx.x % groups, nb = blockIdx.x / groups, band = nb % a.bands, n = nb / a.bands;
+  const int n = blockIdx.x, g = blockIdx.y, band = blockIdx.z;
   const int c0 = g * 32, oy0 = band * a.rows, rows = min(a.rows, a.OH - oy0);
   const int iy0 = oy0 * S - a.pad, in_rows = (rows - 1) * S + K;
   unsigned char* taps = smem + a.cells * 64;
   const int chunk = tid & 3, ch = c0 + chunk * 8;  // the channels of this thread's depthwise work
   const bool live = ch < a.C;
 
-  // BatchNorm of this thread's depthwise channels and its share of the taps, requested first
-  floatx4 dsc[2], dsh[2];
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    dsc[q] = live && a.scale ? *reinterpret_cast<const floatx4*>(a.scale + ch + 4 * q) : floatx4{1.f, 1.f, 1.f, 1.f};
-    dsh[q] = live && a.shift ? *reinterpret_cast<const floatx4*>(a.shift + ch + 4 * q) : floatx4{0.f, 0.f, 0.f, 0.f};
-  }
-  u32x4 tap = {0, 0, 0, 0};
-  if (tid < K * K * 4 && live) tap = *reinterpret_cast<const u32x4*>(static_cast<const half_t*>(a.wt) + (tid >> 2) * a.C + ch);
+  // Squeeze weights of this group's channels, a run of 32 rows, by DMA into LDS: in registers they take the third workgroup
+  // from the CU (13.8 instead of 10.2 us at 7x7x576), and requested behind the stores they wait for the stores.
+  unsigned char* sqw = taps + K * K * 64;
+  auto request_squeeze = [&] {
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.sq_w, (unsigned)(a.C * a.SQ * 2));
+    for (int u = wave * 64; u < 4 * a.SQ; u += kDwThreads)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(sqw + u * 16), 16, (unsigned)(c0 * a.SQ * 2 + (u + lane) * 16), 0, 0, 0);
+  };
 
   // rows of the input that exist
   const int ya = max(iy0, 0), yb = min(iy0 + in_rows, a.H), npx = max(0, yb - ya) * a.W;
@@ -64,10 +133,19 @@ __global__ __launch_bounds__(kDwThreads) void dw_block_kernel(const DwBlockArgs 
     const int y = fast_div(q, a.W, a.inv_w, &x);
     return cell0 + y * a.pitch + x;
   };
+  // BatchNorm of this thread's depthwise channels and its share of the taps; what lies beyond channel C reads as zero
+  floatx4 dsc[2], dsh[2];
+  u32x4 tap;
+  auto request = [&] {
+    batch_norm<2, 4>(a.scale, a.shift, a.C, ch, dsc, dsh);
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.wt, (unsigned)(K * K * a.C * 2));
+    tap = __builtin_amdgcn_raw_buffer_load_b128(rs, live ? (unsigned)((tid >> 2) * a.C + ch) * 2u : kOOBm, 0, 0);
+  };
   auto prepare = [&] {  // zeros around the image, and the taps
     const u32x4 zero = {0, 0, 0, 0};
     for (int u = tid; u < in_rows * a.pitch * 4; u += kDwThreads) *reinterpret_cast<u32x4*>(smem + u * 16) = zero;
     if (tid < K * K * 4) *reinterpret_cast<u32x4*>(taps + tid * 16) = tap;
+    if (a.parts) request_squeeze();
     __syncthreads();
   };
 
@@ -76,22 +154,17 @@ __global__ __launch_bounds__(kDwThreads) void dw_block_kernel(const DwBlockArgs 
     const __amdgpu_buffer_rsrc_t rs_w = make_rsrc(a.w1, (unsigned)(a.C * a.Cin * 2));
     u32x4 w[KST], x[KST];
     floatx4 sc[4], sh[4];
-    auto load = [&](int blk) {
-      const int q = blk * 32 + lrow;
+    auto load = [&](int blk) {  // (pixels beyond npx and filters beyond C lie beyond their buffers)
+      const unsigned off = (unsigned)((blk * 32 + lrow) * a.pix + lh * 8) * 2u;
 #pragma unroll
-      for (int k = 0; k < KST; ++k)
-        x[k] = __builtin_amdgcn_raw_buffer_load_b128(rs_in, ((q < npx) & (2 * k + lh < nch)) ? (unsigned)(q * a.pix + (2 * k + lh) * 8) * 2u : kOOBm, 0, 0);
+      for (int k = 0; k < KST; ++k) x[k] = __builtin_amdgcn_raw_buffer_load_b128(rs_in, 2 * k + lh < nch ? off + 32u * k : kOOBm, 0, 0);
     };
     load(wave);
+    const unsigned off_w = (unsigned)((c0 + lrow) * a.Cin + lh * 8) * 2u;
 #pragma unroll
-    for (int k = 0; k < KST; ++k)
-      w[k] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, ((c0 + lrow < a.C) & (2 * k + lh < nch)) ? (unsigned)((c0 + lrow) * a.Cin + (2 * k + lh) * 8) * 2u : kOOBm, 0, 0);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {  // accumulator channels 8 q + 4 (lane / 32) .. + 3
-      const int f = c0 + 8 * q + 4 * lh;
-      sc[q] = f < a.C && a.scale1 ? *reinterpret_cast<const floatx4*>(a.scale1 + f) : floatx4{1.f, 1.f, 1.f, 1.f};
-      sh[q] = f < a.C && a.shift1 ? *reinterpret_cast<const floatx4*>(a.shift1 + f) : floatx4{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int k = 0; k < KST; ++k) w[k] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, 2 * k + lh < nch ? off_w + 32u * k : kOOBm, 0, 0);
+    batch_norm<4, 8>(a.scale1, a.shift1, a.C, c0 + 4 * lh, sc, sh);  // accumulator channels 8 q + 4 (lane / 32) .. + 3
+    request();
     prepare();
     constexpr int NW = kDwThreads / 64;
     for (int blk = wave; blk * 32 < npx; blk += NW) {
@@ -119,10 +192,12 @@ __global__ __launch_bounds__(kDwThreads) void dw_block_kernel(const DwBlockArgs 
       }
     }
   } else {
+    request();
     prepare();
     for (int u = tid; u < npx * 4; u += kDwThreads)
       if (live) *reinterpret_cast<u32x4*>(smem + cell_at(cell_of(u >> 2), chunk)) = __builtin_amdgcn_raw_buffer_load_b128(rs_in, (unsigned)((u >> 2) * a.pix + ch) * 2u, 0, 0);
   }
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the squeeze weights
   __syncthreads();
 
   // ---- depthwise: (kh, kw) order, fp32 ----
@@ -170,63 +245,83 @@ __global__ __launch_bounds__(kDwThreads) void dw_block_kernel(const DwBlockArgs 
       *reinterpret_cast<half8*>(out + ((long long)oy * a.OW + ox0 + j) * a.C) = h;
     }
   }
-  if (!a.sums) return;  // (uniform)
-  // ---- channel sums of the band, in a fixed order ----
-#pragma unroll
-  for (int o = 4; o < 64; o *= 2)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) sum[e] += __shfl_xor(sum[e], o);
+  if (!a.parts) return;  // (uniform)
+  // ---- channel sums of the band, in a fixed order, through the squeeze weights of these channels ----
+  const float total = sum_of_sixteen(sum, lane);
   __syncthreads();
   float* part = reinterpret_cast<float*>(smem);
-  if (lane < 4)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) part[wave * 32 + lane * 8 + e] = sum[e];
+  if (!(lane & 4)) part[wave * 32 + chunk * 8 + (lane >> 3)] = total;
   __syncthreads();
-  if (tid < 32 && c0 + tid < a.C)
-    a.sums[((long long)n * a.bands + band) * a.C + c0 + tid] = (part[tid] + part[32 + tid]) + (part[64 + tid] + part[96 + tid]);
+  const int sq_o = tid >> 3, sq_r = tid & 7;  // rows r, r + 8, ... of outputs 8 o .. 8 o + 7
+  if (8 * sq_o >= a.SQ) return;
+  float v[8];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int c = sq_r + 8 * u;
+    const float m = (part[c] + part[32 + c]) + (part[64 + c] + part[96 + c]);
+    const half8 w = *reinterpret_cast<const half8*>(sqw + (c * a.SQ + sq_o * 8) * 2);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = u ? v[e] + m * (float)w[e] : m * (float)w[e];
+  }
+  const float r = sum_of_eight(v, lane);
+  a.parts[(((long long)n * a.bands + band) * ((a.C + 31) >> 5) + g) * a.SQ + tid] = r;
 }
 
 namespace {
 
-// out[j] = act(b[j] + sum_c in[c] w[c][j]), both vectors fp32 in LDS.  Thread (g, o) takes rows c = g, g + G, ... of the eight
-// outputs of chunk o, so that a wave reads the weights in one run (a row of them per output instead, two lanes to a row,
-// took 22 us for 576 x 144); the G partial sums of an output meet in LDS (`part`, 8 floats a thread).
-template <int THREADS>
-__device__ __forceinline__ void fc_vector(const half_t* __restrict__ w, const float* __restrict__ b, const float* in, float* out, float* part, int n_out,
-                                          int n_in, float inv_oc, int act) {
-  constexpr int U = 8;
-  const int oc = n_out >> 3, groups = min(THREADS / oc, (n_in + U - 1) / U);
-  int o;
-  const int g = fast_div((int)threadIdx.x, oc, inv_oc, &o);
-  if (g < groups) {
+// The excitation: out[j] = act(b[j] + sum_c in[c] w[c][j]), both vectors fp32 in LDS.  Thread (g, o) takes rows c = g, g + G, ...
+// of the eight outputs of chunk o, so that a wave reads the weights in one run (a row of them per output instead, two lanes to
+// a row, took 22 us for 576 x 144); the G <= 8 partial sums of an output meet in LDS (`part`).  The first U rows of a thread
+// are requested long before the vector is there (`request`).
+template <int THREADS, int U>
+struct Excitation {
+  static constexpr int kGroups = 8;
+  __amdgpu_buffer_rsrc_t rs;
+  int n_out, n_in, groups, g, o, step;
+  unsigned first;
+  u32x4 x[U];
+  __device__ __forceinline__ Excitation(const void* w, int outs, int ins, float inv_oc) : rs(make_rsrc(w, (unsigned)(outs * ins) * 2u)), n_out(outs), n_in(ins) {
+    const int oc = outs >> 3;
+    groups = min(kGroups, min(THREADS / oc, (ins + 7) >> 3));
+    g = fast_div((int)threadIdx.x, oc, inv_oc, &o);
+    first = (unsigned)((g * oc + o) * 16);
+    step = groups * oc * 16;
+  }
+  // rows beyond the last read as zeros
+  __device__ __forceinline__ void request(int c0 = 0) {
+    unsigned off = first + (unsigned)(c0 * (n_out * 2));
+#pragma unroll
+    for (int u = 0; u < U; ++u, off += step) x[u] = __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0);
+  }
+  // `in` is followed by zeros up to the next multiple of U * kGroups
+  __device__ __forceinline__ void run(const float* in, float* part) {
+    if (g >= groups) return;
     float s[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) s[e] = 0.0f;
-    for (int c0 = g; c0 < n_in; c0 += U * groups) {
-      half8 x[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) x[u] = *reinterpret_cast<const half8*>(w + ((long long)min(c0 + u * groups, n_in - 1) * oc + o) * 8);
+    for (int c0 = 0; c0 < n_in; c0 += U * groups) {
+      if (c0) request(c0);
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const int c = c0 + u * groups;
-        if (c < n_in) {
-          const float m = in[c];
+        const float m = in[c0 + g + u * groups];
+        const half8 w = as_half8(x[u]);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) s[e] += m * (float)x[u][e];
-        }
+        for (int e = 0; e < 8; ++e) s[e] += m * (float)w[e];
       }
     }
-    *reinterpret_cast<floatx4*>(part + (g * oc + o) * 8) = floatx4{s[0], s[1], s[2], s[3]};
-    *reinterpret_cast<floatx4*>(part + (g * oc + o) * 8 + 4) = floatx4{s[4], s[5], s[6], s[7]};
+    float* at = part + (g * (n_out >> 3) + o) * 8;
+    *reinterpret_cast<floatx4*>(at) = floatx4{s[0], s[1], s[2], s[3]};
+    *reinterpret_cast<floatx4*>(at + 4) = floatx4{s[4], s[5], s[6], s[7]};
   }
-  __syncthreads();
-  for (int j = threadIdx.x; j < n_out; j += THREADS) {
-    float s = b[j];
-#pragma unroll 8
-    for (int k = 0; k < groups; ++k) s += part[k * n_out + j];
-    out[j] = act_apply<false>(s, act);
+  __device__ __forceinline__ float result(const float* part, int j, float bias) const {
+    float v[kGroups];
+#pragma unroll
+    for (int k = 0; k < kGroups; ++k) v[k] = part[min(k, groups - 1) * n_out + j];
+#pragma unroll
+    for (int k = 0; k < kGroups; ++k) bias += k < groups ? v[k] : 0.0f;
+    return bias;
   }
-}
+};
 
 constexpr int kSpThreads = 512, kSpMaxC = 768, kSpMaxSq = 256;
 
@@ -239,10 +334,13 @@ constexpr int kSpThreads = 512, kSpMaxC = 768, kSpMaxSq = 256;
 template <int NS, int FT, int PT, bool KSPLIT>
 __global__ __launch_bounds__(kSpThreads) void se_project_kernel(const SeProjectArgs a) {
   constexpr int NW = kSpThreads / 64;
-  __shared__ __align__(16) float mean[kSpMaxC];
-  __shared__ __align__(16) float hid[kSpMaxSq];
+  constexpr int U = NS == 3 ? 21 : 8;  // rows of the excitation weights that a thread holds
+  __shared__ __align__(16) float gate[kSpMaxC];
+  __shared__ __align__(16) float hid[kSpMaxSq + 8 * U];
   __shared__ __align__(16) float part_sum[kSpThreads * 8];
   extern __shared__ __align__(16) unsigned char smem[];  // partial sums of the K steps (KSPLIT)
+  asm volatile("" ::"s"(a.x), "s"(a.parts), "s"(a.b1), "s"(a.w2t), "s"(a.b2), "s"(a.wp_flat), "s"(a.scale), "s"(a.shift), "s"(a.residual), "s"(a.out), "s"(a.HW),
+               "s"(a.C), "s"(a.SQ), "s"(a.F), "s"(a.bands), "s"(a.tiles), "s"(a.inv_sq), "s"(a.inv_c));  // one wait for all, as above
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 15, lq = lane >> 4;
   const int tile = blockIdx.x % a.tiles, n = blockIdx.x / a.tiles;
@@ -252,21 +350,25 @@ __global__ __launch_bounds__(kSpThreads) void se_project_kernel(const SeProjectA
   // (filters in launch_weight_flat's order: blocks of 32, units of two chunks)
   const int units = ((a.C * 2 + 127) >> 7) * 4;
   const __amdgpu_buffer_rsrc_t rs_w = make_rsrc(a.wp_flat, (unsigned)((a.F + 31) / 32 * units) * 1024u);
-  // mean over the bands: thread (g, c) takes bands g, g + groups, ... of channel c.  Requested before everything else: results
-  // arrive in the order of the requests, and the whole chain hangs on these.
-  const int groups = max(1, kSpThreads / a.C);
-  float band_sum[(kSpMaxC + kSpThreads - 1) / kSpThreads];
+  // The squeezed vector's parts: thread (g, j) takes parts g, g + G, ... of element j.  Requested before everything else, and
+  // what the gate needs before what the projection does: results arrive in the order of the requests.
+  const int parts = a.bands * ((a.C + 31) >> 5), groups = min(8, kSpThreads / a.SQ);
+  int sj;
+  const int sg = fast_div(tid, a.SQ, a.inv_sq, &sj);
+  const __amdgpu_buffer_rsrc_t rs_p = make_rsrc(a.parts + (long long)n * parts * a.SQ, (unsigned)(parts * a.SQ) * 4u);
+  float hid_sum = 0.0f;
+  for (int b = sg < groups ? sg : parts; b < parts; b += 8 * groups) {
+    float v[8];
 #pragma unroll
-  for (int k = 0; k < (kSpMaxC + kSpThreads - 1) / kSpThreads; ++k) {
-    const int u = tid + k * kSpThreads;
-    float s = 0.0f;
-    if (u < a.C * groups) {
-      const int g = groups == 1 ? 0 : u / a.C, c = u - g * a.C;
-#pragma unroll 4
-      for (int b = g; b < a.bands; b += groups) s += a.sums[((long long)n * a.bands + b) * a.C + c];
-    }
-    band_sum[k] = s;
+    for (int k = 0; k < 8; ++k) v[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs_p, (unsigned)((b + k * groups) * a.SQ + sj) * 4u, 0, 0));
+    hid_sum += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
   }
+  const float bias1 = a.b1[min(tid, a.SQ - 1)];
+  float bias2[(kSpMaxC + kSpThreads - 1) / kSpThreads];
+#pragma unroll
+  for (int k = 0; k < (kSpMaxC + kSpThreads - 1) / kSpThreads; ++k) bias2[k] = a.b2[min(tid + k * kSpThreads, a.C - 1)];
+  Excitation<kSpThreads, U> excite(a.w2t, a.C, a.SQ, a.inv_c);
+  excite.request();
   u32x4 x[NS][PT], w[NS][FT];
 #pragma unroll
   for (int j = 0; j < NS; ++j) {
@@ -297,20 +399,24 @@ __global__ __launch_bounds__(kSpThreads) void se_project_kernel(const SeProjectA
     if (a.residual) tail[k].residual = *reinterpret_cast<const half4*>(static_cast<const half_t*>(a.residual) + ((long long)n * a.HW + p) * a.F + f);
   }
 
-#pragma unroll
-  for (int k = 0; k < (kSpMaxC + kSpThreads - 1) / kSpThreads; ++k)
-    if (tid + k * kSpThreads < a.C * groups) part_sum[tid + k * kSpThreads] = band_sum[k];
+  if (sg < groups) part_sum[tid] = hid_sum;
   __syncthreads();
-  for (int c = tid; c < a.C; c += kSpThreads) {
-    float s = 0.0f;
-#pragma unroll 8
-    for (int g = 0; g < groups; ++g) s += part_sum[g * a.C + c];
-    mean[c] = s / (float)a.HW;
+  if (tid < a.SQ) {
+    float v[8], s = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = part_sum[min(k, groups - 1) * a.SQ + tid];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) s += k < groups ? v[k] : 0.0f;
+    hid[tid] = act_apply<false>(s / (float)a.HW + bias1, a.act1);
+  } else if (tid < kSpMaxSq + 8 * U) {
+    hid[tid] = 0.0f;
   }
   __syncthreads();
-  fc_vector<kSpThreads>(static_cast<const half_t*>(a.w1t), a.b1, mean, hid, part_sum, a.SQ, a.C, a.inv_sq, a.act1);
+  excite.run(hid, part_sum);
   __syncthreads();
-  fc_vector<kSpThreads>(static_cast<const half_t*>(a.w2t), a.b2, hid, mean, part_sum, a.C, a.SQ, a.inv_c, a.act2);  // (mean was read long before)
+#pragma unroll
+  for (int k = 0; k < (kSpMaxC + kSpThreads - 1) / kSpThreads; ++k)
+    if (tid + k * kSpThreads < a.C) gate[tid + k * kSpThreads] = act_apply<false>(excite.result(part_sum, tid + k * kSpThreads, bias2[k]), a.act2);
   __syncthreads();
 
   floatx4 acc[FT][PT];
@@ -324,8 +430,8 @@ __global__ __launch_bounds__(kSpThreads) void se_project_kernel(const SeProjectA
     if (4 * ((KSPLIT ? wave : 0) + NW * j) >= nch) continue;  // (uniform)
     floatx4 g[2] = {};
     if (c < nch) {
-      g[0] = *reinterpret_cast<const floatx4*>(mean + c * 8);
-      g[1] = *reinterpret_cast<const floatx4*>(mean + c * 8 + 4);
+      g[0] = *reinterpret_cast<const floatx4*>(gate + c * 8);
+      g[1] = *reinterpret_cast<const floatx4*>(gate + c * 8 + 4);
     }
 #pragma unroll
     for (int q = 0; q < PT; ++q) {
@@ -410,7 +516,7 @@ int dw_block_bands(int N, int H, int W, int Cin, int C, int K, int S, int pad) {
   DwPlan p;
   const bool ok = (K == 3 || K == 5) && (S == 1 || S == 2) && pad >= 0 && pad < K && OH >= 1 && OW >= 1 && C % 8 == 0 &&
                   (Cin == 0 || (Cin % 8 == 0 && Cin <= 96)) && (long long)H * W * std::max(C, 96) * 2 < (1ll << 30) && (long long)H * W < (1 << 24) &&
-                  (long long)N * OH * ((C + 31) / 32) < (1ll << 30) && dw_plan(N, W, C, K, S, pad, OH, OW, &p);
+                  (long long)N * OH * ((C + 31) / 32) < (1ll << 30) && dw_plan(N, W, C, K, S, pad, OH, OW, &p) && p.bands < 65536 && C < (1 << 20);
   return ok ? p.bands : 0;
 }
 
@@ -438,15 +544,16 @@ void launch_dw_block(const DwBlockArgs& args, hipStream_t s) {
   snprintf(tag, sizeof tag, "dw_block<%d,%d,%d,%d>", a.K, a.stride, oxt, kst);
   ProfScope prof(tag, 2.0 * px_out * a.C * a.K * a.K + 2.0 * px_in * a.C * a.Cin,
                  2.0 * (px_in * (a.Cin ? a.Cin : a.C) + px_out * a.C + a.C * (a.K * a.K + a.Cin)), s);
-  const unsigned grid = (unsigned)((a.C + 31) / 32 * a.bands * a.N);
-  const size_t lds = (size_t)a.cells * 64 + a.K * a.K * 64;
+  // images first: where their number is a multiple of the eight chiplets, an image's groups of channels find it in one L2
+  const dim3 grid((unsigned)a.N, (unsigned)((a.C + 31) / 32), (unsigned)a.bands);
+  const size_t lds = (size_t)a.cells * 64 + a.K * a.K * 64 + (a.parts ? (size_t)(a.SQ + 15) / 16 * 1024 : 0);
   auto go = [&](auto kern) {
     static const bool attr = [&] {
-      NNCV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 100 << 10));
+      NNCV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 116 << 10));
       return true;
     }();
     (void)attr;
-    launch_kernel(kern, dim3(grid), dim3(kDwThreads), lds, s, a);
+    launch_kernel(kern, grid, dim3(kDwThreads), lds, s, a);
   };
   auto steps = [&](auto k, auto st, auto ox) {
     constexpr int K = decltype(k)::value, S = decltype(st)::value, OXT = decltype(ox)::value;
@@ -498,7 +605,7 @@ void launch_se_project(const SeProjectArgs& args, hipStream_t s) {
   // 32 pixels to a tile once 16 would be more than four workgroups a CU
   const int pt = !ksplit || (long long)a.N * ((a.HW + 15) / 16) > 1024 ? 2 : 1, px = pt * 16 * (ksplit ? 1 : kSpThreads / 64);
   a.tiles = (a.HW + px - 1) / px;
-  a.inv_sq = 1.0f / (float)(a.SQ / 8);
+  a.inv_sq = 1.0f / (float)a.SQ;
   a.inv_c = 1.0f / (float)(a.C / 8);
   const dim3 grid((unsigned)(a.tiles * a.N));
   auto go = [&](auto nsc, auto ftc, auto ptc, auto kc) {
