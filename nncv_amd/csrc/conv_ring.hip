@@ -42,6 +42,7 @@ struct RingArgs {
   void* aux_out; unsigned aux_out_bytes;
   int split_f, split_ldo; unsigned ofs, split_ofs;    // filters from split_f on (F: none) go to rows of their own; bytes from `out`
   float inv_ohw, inv_ow, inv_tiles;
+  const void* wfrag; const void* aux_wfrag; int groups, aux_groups, lead;  // the resident form's filters: 32-filter groups; bytes of padding
 };
 
 enum { kPoint = 0, kLines = 1, kAny = 2 };  // 1x1 without padding; taps of whole slabs (C % 64 == 0); any C % 8 == 0
@@ -289,6 +290,214 @@ __global__ __launch_bounds__(64 * WP * WF) void conv_ring_kernel(const RingArgs 
   }
 }
 
+// 3x3 windows over whole slabs of channels: the pixels go through a ring of four slabs, the filters straight from memory into
+// registers (fragments in weight_frag3x3's order, eight K steps ahead).  Four waves take 32 filters each of BP x 128 outputs, so a
+// K step is PB products on one fragment and PB LDS reads: per 128 x 128 x 64 products LDS takes 16 KB of pixels and gives 64 KB, where
+// the ring above takes 32 and gives 96 (LDS takes 80 and gives 256 bytes a clock).  A slab is fetched three stages ahead, and one
+// barrier a stage says both that it is there and that the one before it may go.
+//  * Slab outer, tap inner: of nine taps three or four bring lines that the others have not.
+//  * Whether a pixel has the tap is one bit per tap and row of the tile; the tap's offset is the scalar part of the address.
+//  * Auxiliary filters (AUX) are a second set of sums: the centre tap's pixels are their operands.
+//  * What bounds it: nothing alone.  22x49x58x512 -> 512 takes 75 us (1000 TFLOP/s; 88 in the ring above), 70 without the filters'
+//    loads, 62 without the pixels', 65 without the LDS reads, 50 without the products: a wave issues all of them in turn.
+// Times against the ring's 128 x 128 form or, below 200 tiles, conv3x3_patch.hip: 16x40x40x256 -> 512 27.1 -> 21.7 us, 16x160x160x64 ->
+// 128 29.0 -> 25.8, 16x40x40x256 -> 256 20.2 -> 13.3, 33x25x106x64 -> 128 14.0 -> 8.6.
+template <int PB, bool AUX>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PB == 4 ? 2 : 3, PB == 4 ? 2 : 4))) void conv_ring_frag_kernel(const RingArgs a) {
+  constexpr int BP = 32 * PB, BF = 128, kStage = BP * 128, kStages = 4, kRing = 8;
+  constexpr int kPitch = 272, kLds = kStages * kStage > BP * kPitch ? kStages * kStage : BP * kPitch;
+  constexpr int kWait = ((8 + 2 * PB) & 15) | (((8 + 2 * PB) >> 4) << 14) | 0x0f70;
+  extern __shared__ __align__(16) unsigned char smem[];  // ring, then scale[BF] and shift[BF]
+  asm volatile("" ::"s"(a.in), "s"(a.wfrag), "s"(a.aux_wfrag), "s"(a.scale), "s"(a.shift), "s"(a.H), "s"(a.W), "s"(a.OW), "s"(a.OHW), "s"(a.P), "s"(a.pix), "s"(a.F),
+               "s"(a.tiles_f), "s"(a.tiles_p), "s"(a.aux_tiles), "s"(a.aux_f0), "s"(a.groups), "s"(a.inv_ohw), "s"(a.inv_ow), "s"(a.inv_tiles), "s"(a.lead));
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  int tf, tp;
+  {
+    const int tiles = a.tiles_f * a.tiles_p, per = (tiles + 7) >> 3, rem = tiles & 7;
+    const int x = blockIdx.x & 7, i = blockIdx.x >> 3;
+    const int t = rem == 0 ? x * per + i : (x < rem ? x * per : rem * per + (x - rem) * (per - 1)) + i;
+    if (a.pixels_first) tf = fast_div(t, a.tiles_p, a.inv_tiles, &tp);
+    else tp = fast_div(t, a.tiles_f, a.inv_tiles, &tf);
+  }
+  tf = __builtin_amdgcn_readfirstlane(tf);
+  tp = __builtin_amdgcn_readfirstlane(tp);
+  const int p0 = tp * BP, f0 = tf * BF, fend = AUX ? a.aux_f0 : a.F;
+
+  // ---- filters: fragment (group g, stage st, sub-step kk) is the kilobyte ((g / 2 * stages + st) * 4 + kk) * 2 + g % 2 ----
+  const int nslab = a.cpt >> 3, T = nslab * 9;
+  const int g = min(tf * 4 + wave, a.groups - 1);  // (filters that are not there: the last ones again)
+  const __amdgpu_buffer_rsrc_t rs_w = make_rsrc(a.wfrag, (unsigned)(a.groups >> 1) * T * 8192u);
+  unsigned woff = (unsigned)((g >> 1) * T * 8192 + (g & 1) * 1024 + lane * 16);
+  u32x4 wring[kRing];
+  auto wload = [&](int step) __attribute__((always_inline)) { return __builtin_amdgcn_raw_buffer_load_b128(rs_w, woff + step * 2048, 0, 0); };  // step: from this stage on
+
+  // auxiliary filters: this slab's four fragments (their order is that of one-tap filters)
+  const int ga = AUX ? min(tf * 4 + wave, a.aux_groups - 1) : 0;
+  const __amdgpu_buffer_rsrc_t rs_a = make_rsrc(AUX ? a.aux_wfrag : a.wfrag, AUX ? (unsigned)(a.aux_groups >> 1) * nslab * 8192u : 0u);
+  unsigned aoff = (unsigned)((ga >> 1) * nslab * 8192 + (ga & 1) * 1024 + lane * 16);
+  u32x4 waux[4];
+  auto load_aux = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) waux[k] = __builtin_amdgcn_raw_buffer_load_b128(rs_a, aoff + k * 2048, 0, 0);
+    aoff += 8192;
+  };
+
+  // ---- pixels: of row (wave * PB + i) * 8 + lane / 8 the chunk at position lane % 8; bit 3 r + s of `valid`: tap (r, s) is inside ----
+  const int pos = lane & 7, sub = lane >> 3;
+  const __amdgpu_buffer_rsrc_t rs_in = make_rsrc(static_cast<const char*>(a.in) - a.lead, a.in_bytes + a.lead);
+  unsigned pbase[PB], valid[PB];
+#pragma unroll
+  for (int i = 0; i < PB; ++i) {
+    const int group = wave * PB + i, p = p0 + group * 8 + sub;
+    int rem, x;
+    const int n = fast_div(p < a.P ? p : 0, a.OHW, a.inv_ohw, &rem), y = fast_div(rem, a.OW, a.inv_ow, &x);
+    const int yy = y * a.stride_h, xx = x * a.stride_w;
+    pbase[i] = (unsigned)(((n * a.H + yy) * a.W + xx) * a.pix * 2 + (pos ^ (((group & 1) << 2) + (sub >> 1))) * 16);
+    const unsigned cols = (xx >= 1 ? 1u : 0u) | 2u | (xx + 1 < a.W ? 4u : 0u);
+    valid[i] = p < a.P ? (yy >= 1 ? cols : 0u) | cols << 3 | (yy + 1 < a.H ? cols << 6 : 0u) : 0u;
+  }
+  const int pixB = a.pix * 2, rowB = (a.W - 2) * pixB, turnB = 128 - (2 * a.W + 2) * pixB;
+  int ptap = 0, pleft = T, poff = 0;  // the stage to fetch next
+  auto fetch = [&](int buf) __attribute__((always_inline)) {
+    const unsigned bit = pleft > 0 ? 1u << ptap : 0u;
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+      const unsigned at = pbase[i], v = valid[i] & bit ? at : kOOBr;
+      fetch16(rs_in, smem + buf * kStage + (wave * PB + i) * 1024, v, (unsigned)poff);
+    }
+    --pleft;
+    // (locals: of captured variables hipcc 7.2 chooses the address, in scratch)
+    const int next = ptap + 1, row = rowB, pix = pixB, back = turnB;
+    int step = next == 3 || next == 6 ? row : pix;
+    step = next == 9 ? back : step;
+    poff = __builtin_amdgcn_readfirstlane(poff + step);
+    ptap = __builtin_amdgcn_readfirstlane(next == 9 ? 0 : next);
+  };
+
+  __builtin_amdgcn_sched_barrier(0);
+  fetch(0);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) wring[q] = wload(q);
+  fetch(1);
+#pragma unroll
+  for (int q = 4; q < 8; ++q) wring[q] = wload(q);
+  if constexpr (AUX) load_aux();
+  fetch(2);
+  // threads 0 .. 127: the filters' scale and shift; 128 .. 255: the auxiliary ones'
+  const bool second = (int)threadIdx.x >= BF;
+  const unsigned ssf = (unsigned)((second ? a.aux_f0 - BF : 0) + f0 + (int)threadIdx.x) * 4u;
+  const __amdgpu_buffer_rsrc_t rs_sc = make_rsrc(a.scale, a.scale ? (unsigned)a.F * 4u : 0u), rs_sh = make_rsrc(a.shift, a.shift ? (unsigned)a.F * 4u : 0u);
+  const unsigned scv = __builtin_amdgcn_raw_buffer_load_b32(rs_sc, ssf, 0, 0), shv = __builtin_amdgcn_raw_buffer_load_b32(rs_sh, ssf, 0, 0);
+  __builtin_amdgcn_sched_barrier(0);
+
+  floatx16 acc[PB], acc2[AUX ? PB : 1];
+#pragma unroll
+  for (int j = 0; j < PB; ++j)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      acc[j][e] = 0.0f;
+      if constexpr (AUX) acc2[j][e] = 0.0f;
+    }
+  int tap = 0;
+  const int lrow = lane & 31, lh = lane >> 5, key = (lrow >> 1) & 7;
+  const unsigned char* prow[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) prow[k] = smem + lrow * 128 + (((2 * k + lh) ^ key) * 16);
+  u32x4 pr[2][PB];
+  auto stage = [&](auto u_c) __attribute__((always_inline)) {
+    constexpr int u = decltype(u_c)::value;
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(kWait);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < PB; ++j) pr[0][j] = *reinterpret_cast<const u32x4*>(prow[0] + u * kStage + j * 4096);
+    fetch((u + 3) & 3);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      constexpr int base = (u * 4) % kRing;
+      const u32x4 wf = wring[base + k];
+#pragma unroll
+      for (int j = 0; j < PB; ++j) {
+        Mma<half_t>::run(wf, pr[k & 1][j], acc[j]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (k < 3) pr[(k + 1) & 1][j] = *reinterpret_cast<const u32x4*>(prow[k + 1] + u * kStage + j * 4096);
+        if (j == PB - 1) wring[base + k] = wload(8 + k);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    woff += 8192;
+    if constexpr (AUX) {  // the centre tap's pixels are the auxiliary filters' operands
+      if (tap == 4) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int j = 0; j < PB; ++j) {
+            const u32x4 x = *reinterpret_cast<const u32x4*>(prow[k] + u * kStage + j * 4096);
+            Mma<half_t>::run(waux[k], x, acc2[j]);
+          }
+        load_aux();  // (the next slab's; beyond the last one zeros)
+      }
+      tap = tap == 8 ? 0 : tap + 1;
+    }
+  };
+  for (int st = 0;;) {
+    stage(std::integral_constant<int, 0>());
+    if (++st >= T) break;
+    stage(std::integral_constant<int, 1>());
+    if (++st >= T) break;
+    stage(std::integral_constant<int, 2>());
+    if (++st >= T) break;
+    stage(std::integral_constant<int, 3>());
+    if (++st >= T) break;
+  }
+  float* ss = reinterpret_cast<float*>(smem + kLds);
+  if (AUX || !second) {
+    ss[threadIdx.x] = a.scale ? __builtin_bit_cast(float, scv) : 1.0f;
+    ss[(AUX ? 2 : 1) * BF + threadIdx.x] = __builtin_bit_cast(float, shv);
+  }
+  __builtin_amdgcn_s_waitcnt(kAllLanded);  // (also what was asked for beyond the last stage: the tile below takes its place)
+  __syncthreads();
+
+  // ---- out, through one tile [BP pixels][128 channels]: rows of 256 bytes leave as whole lines (64 bytes of a row a wave: 81
+  // instead of 66 us for 256x56x56x64 -> 128 + 128, which is bound by what it writes) ----
+  const int orow = wave * 4 + (lane >> 4), ochan = (lane & 15) * 8;
+  auto finish = [&](floatx16 (&sum)[PB], const float* sc, int act, __amdgpu_buffer_rsrc_t rs_out, int f, int filters, int ldo) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < PB; ++j) {
+      float y[16];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const floatx4 m = *reinterpret_cast<const floatx4*>(sc + 8 * q + 4 * lh), h = *reinterpret_cast<const floatx4*>(sc + (AUX ? 2 : 1) * BF + 8 * q + 4 * lh);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[4 * q + e] = sum[j][4 * q + e] * m[e] + h[e];
+      }
+      act_apply_n<true>(y, act & 0xff);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        half4 x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = (half_t)y[4 * q + e];
+        *reinterpret_cast<half4*>(smem + (j * 32 + lrow) * kPitch + wave * 64 + q * 16 + lh * 8) = x;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int o = 0; o < 2 * PB; ++o) {
+      const int p = p0 + o * 16 + orow;
+      const u32x4 v = *reinterpret_cast<const u32x4*>(smem + (o * 16 + orow) * kPitch + ochan * 2);
+      __builtin_amdgcn_raw_buffer_store_b128(v, rs_out, p < a.P && f < filters ? (unsigned)(p * ldo + f) * 2u : kOOBr, 0, 0);
+    }
+  };
+  finish(acc, ss + wave * 32, a.act, make_rsrc(a.out, a.out_bytes), f0 + ochan, fend, a.ldo);
+  if constexpr (AUX) {
+    __syncthreads();
+    finish(acc2, ss + BF + wave * 32, a.aux_act, make_rsrc(a.aux_out, a.aux_out_bytes), f0 + ochan, a.F - a.aux_f0, a.aux_ldo);
+  }
+}
+
 // ---- dispatch
 
 template <int WP, int WF, int PB, int FB, int S>
@@ -313,9 +522,38 @@ void launch_cfg(RingArgs d, int mode, hipStream_t s) {
   else go(conv_ring_kernel<WP, WF, PB, FB, S, kAny>);
 }
 
+template <int PB>
+void launch_frag(RingArgs d, int, hipStream_t s) {
+  constexpr int BP = 32 * PB, ring = 4 * BP * 128, tile = BP * 272, lds = (ring > tile ? ring : tile) + 128 * 16;
+  const int main_f = d.aux_f0 ? d.aux_f0 : d.F;
+  d.tiles_f = (main_f + 127) / 128;
+  d.tiles_p = (d.P + BP - 1) / BP;
+  d.inv_tiles = 1.0f / (float)(d.pixels_first ? d.tiles_p : d.tiles_f);
+  d.groups = (main_f + 63) / 64 * 2;
+  d.aux_groups = (d.F - main_f + 63) / 64 * 2;
+  d.lead = (d.W + 1) * d.pix * 2;
+  auto go = [&](auto kern) {
+    static const bool attr = [&] {
+      NNCV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+      return true;
+    }();
+    (void)attr;
+    launch_kernel(kern, dim3((unsigned)(d.tiles_f * d.tiles_p)), dim3(256), lds, s, d);
+  };
+  if (d.aux_f0) go(conv_ring_frag_kernel<PB, true>);
+  else go(conv_ring_frag_kernel<PB, false>);
+}
+
 // The forms, and what a launch of each takes: us = fixed + ((busy)^3 + (chain)^3)^(1/3) with
 //   busy  = tiles / 256 CUs * (slab_us * slabs + tile_us)            (LDS, matrix and memory pipes)
 //   chain = ceil(tiles / (256 * resident)) * chain_us * slabs        (a slab's latency, workgroups of a CU one after the other)
+// The fragment forms: us = fixed + t * (slab_us * slabs + tile_us), t halfway between tiles / 256 (at least 1) and its ceiling, or
+// chain_us + t * slab_any for 64 channels (nine slabs, bound by memory); within 6 % (1 sigma) over 112 stride-2 layers of 1 to 60
+// GFLOP, and in the choice between the two 0.8 % off the better one on average.  With 64 channels, 64 pixels to a tile are up to 8 %
+// ahead to 16 such tiles a CU (80x56x56 -> 128 17.1 against 18.3 us), 128 from there (241x77x91 -> 72 91.7 against 101.9).  The
+// ring's own forms of 128 filters are level with them at best, save for 64 channels and a fourth turn of the tiles of 64 pixels: the two
+// tiles of 128 x 128 of a CU then run side by side with 16 waves (64 to 80 images of 56x56x64 -> 128: 13.7 to 14.9 against 13.8 to 15.8 us
+// on one card, 15.5 to 17.4 against 15.9 to 17.1 on another).
 // slab_us and chain_us grow by slab_any and chain_any where the taps are not whole slabs.  Fits over 300 layers of 1x1 to 7x7
 // windows, 8 to 1024 channels; the form they choose is within 1.5 % of the best one on average.
 struct Form {
@@ -323,6 +561,7 @@ struct Form {
   double fixed_us, slab_us, tile_us, chain_us, slab_any, chain_any;
   void (*launch)(RingArgs, int, hipStream_t);
   const char* tag;
+  bool frag = false;
 };
 const Form kForms[] = {
     {64, 64, 7, 2.58, 0.220, 0.287, 0.405, 0.26, 0.18, launch_cfg<2, 2, 1, 1, 1>, "conv_ring<64x64>"},
@@ -331,18 +570,38 @@ const Form kForms[] = {
     {64, 128, 3, 3.04, 0.353, 0.620, 0.434, 0.11, 0.37, launch_cfg<2, 2, 1, 2, 2>, "conv_ring<64x128,2>"},
     {128, 128, 2, 2.94, 0.626, 1.086, 0.631, 0.11, 0.11, launch_cfg<4, 2, 1, 2, 1>, "conv_ring<128x128>"},
     {128, 128, 2, 3.08, 0.583, 1.142, 0.515, 0.21, 0.48, launch_cfg<4, 2, 1, 2, 2>, "conv_ring<128x128,2>"},
+    {64, 128, 4, 2.64, 0.293, 0.448, 2.98, 3.06, 0, launch_frag<2>, "conv_ring<64x128,frag>", true},
+    {128, 128, 2, 1.51, 0.472, 2.537, 2.41, 6.32, 0, launch_frag<4>, "conv_ring<128x128,frag>", true},
 };
 
+// What the fragment forms cover.  With auxiliary filters, whose sums take the registers of a third wave, from 256 channels on
+// (ResNet-18, 256 images: 44.3 -> 41.2 us; 47.2 -> 49.7 at 128 channels, 65.8 -> 67.8 at 64), and with 128 pixels to a tile (64: 77).
+bool frag_ok(const IgemmArgs& a) {
+  const long long pix = a.pix_stride ? a.pix_stride : a.C;
+  return a.wt_frag && a.R == 3 && a.S == 3 && a.pad_h == 1 && a.pad_w == 1 && a.C % 64 == 0 && !a.residual && (a.aux_f0 == 0 || (a.C >= 256 && a.aux_wt_frag && a.aux_tap == 4 && a.F <= 2 * a.aux_f0)) &&
+         (long long)a.in_bytes + (a.W + 1) * pix * 2 < (long long)kOOBr;
+}
+
 const Form* best_form(const IgemmArgs& a, double* us) {
-  const double P = (double)a.N * a.OH * a.OW, slabs = std::ceil(a.R * a.S * a.C / 64.0);
-  const bool any = a.R * a.S > 1 && a.C % 64 != 0;
+  const double P = (double)a.N * a.OH * a.OW, slabs = std::ceil(a.R * a.S * a.C / 64.0), main_f = a.aux_f0 ? a.aux_f0 : a.F;
+  const bool any = a.R * a.S > 1 && a.C % 64 != 0, nine = slabs <= 9;
+  auto per_cu = [&](const Form& f, double filters) { return std::ceil(P / f.bp) * std::ceil(filters / f.bf) / 256; };
+  const double quarters = std::ceil(P / 64) * std::ceil(main_f / 128) / 256;
+  const bool frag = frag_ok(a) && !(nine && quarters > 3 && quarters <= 4);
   const Form* best = nullptr;
   for (const Form& f : kForms) {
-    const double fs = a.aux_f0 ? a.aux_f0 + (double)(a.F - a.aux_f0) / (a.R * a.S) : a.F;  // auxiliary filters walk one tap
-    const double x = std::ceil(P / f.bp) * std::ceil(fs / f.bf) / 256;
-    const double busy = x * (f.slab_us * slabs * (any ? 1 + f.slab_any : 1) + f.tile_us);
-    const double chain = std::ceil(x / f.resident) * f.chain_us * slabs * (any ? 1 + f.chain_any : 1);
-    const double v = f.fixed_us + std::cbrt(busy * busy * busy + chain * chain * chain);
+    double v;
+    if (f.frag) {
+      if (!frag || (a.aux_f0 ? f.bp == 64 : nine && (quarters < 16) != (f.bp == 64))) continue;
+      const double x = per_cu(f, main_f), t = (0.5 * std::ceil(x) + 0.5 * std::max(1.0, x)) * (a.aux_f0 ? 10 / 9.0 : 1);
+      v = nine ? f.chain_us + t * f.slab_any : f.fixed_us + t * (f.slab_us * slabs + f.tile_us);
+    } else {
+      if (frag && f.bf == 128) continue;
+      const double x = per_cu(f, main_f + (a.F - main_f) / (a.R * a.S));  // auxiliary filters walk one tap
+      const double busy = x * (f.slab_us * slabs * (any ? 1 + f.slab_any : 1) + f.tile_us);
+      const double chain = std::ceil(x / f.resident) * f.chain_us * slabs * (any ? 1 + f.chain_any : 1);
+      v = f.fixed_us + std::cbrt(busy * busy * busy + chain * chain * chain);
+    }
     if (!best || v < *us) best = &f, *us = v;
   }
   return best;
@@ -367,7 +626,11 @@ bool conv_ring_applicable(const IgemmArgs& a, int in_dt, int out_dt) {
          P * a.ldo * 2 < (long long)kOOBr && ((P + 63) / 64) * ((a.F + 31) / 32) < lim && (a.relu & ~(0xff | kActResidualAfter)) == 0;
 }
 
-// Stride-2 3x3 layers leave the patch kernel where 128 x 128 tiles keep three quarters of the CUs busy.  From 200 tiles to the
+// Stride-2 3x3 layers without auxiliary filters leave the patch kernel for the fragment forms from 112 tiles of 64 x 128 on: of 41
+// layers between there and 400 tiles 38 take 0.5 to 0.96 times as long, the others 1.0 (24x19x16x256 -> 512, 120 tiles: 19.9 -> 12.7;
+// 19x31x77x64 -> 192, 372: 9.5 -> 9.1).  Below, its smaller tiles and K groups mostly fill the chip better (6x22x86x256 -> 256, 92
+// tiles: 9.1 against 12.3 us; 11x25x67x128, 73: 6.7 against 8.5), and 64 filters are half a tile (9x65x151x64 -> 64: 7.3 against 7.8).
+// The rest leaves it where 128 x 128 tiles keep three quarters of the CUs busy.  From 200 tiles to the
 // patch kernel's limit (8 GFLOP) that kernel is bound by its patch reads: 48x56x56x64 -> 128 14.3 against 13.3 us here, 64
 // images 17.4 against 14.1, 32x40x40x128 -> 256 20.0 against 15.9, 16x80x80x64 -> 128 10.2 against 10.3 at 200 tiles.  Below, its
 // smaller tiles and K groups mostly fill the chip better (32x28x28x128 -> 256, 98 tiles: 9.1 against 11.6; 24x40x40x128 -> 256,
@@ -376,6 +639,7 @@ bool conv_ring_applicable(const IgemmArgs& a, int in_dt, int out_dt) {
 // their shortcuts went from 78.1 + 58.4 + 52.2 us there to 65.4 + 46.6 + 43.6, the pass from 1162 to 1133 us of launches.
 bool conv_ring_beats_patch_s2(const IgemmArgs& a) {
   const long long P = (long long)a.N * a.OH * a.OW, main_f = a.aux_f0 ? a.aux_f0 : a.F;
+  if (a.stride_h == 2 && frag_ok(a) && a.aux_f0 == 0 && a.F > 64 && (P + 63) / 64 * ((main_f + 127) / 128) >= 112) return true;
   return a.stride_h == 2 && (P + 127) / 128 * ((main_f + 127) / 128) >= 200;
 }
 
@@ -410,6 +674,7 @@ void launch_conv_ring(const IgemmArgs& a, hipStream_t s) {
   d.pixels_first = d.wt_bytes > d.in_bytes;
   double us = 0;
   const Form* f = best_form(a, &us);
+  d.wfrag = a.wt_frag; d.aux_wfrag = a.aux_wt_frag;
   const double flops = a.alg_flops > 0 ? a.alg_flops : 2.0 * d.P * (double)a.F * a.R * a.S * a.C;
   ProfScope prof(f->tag, flops, 2.0 * ((double)a.N * a.H * a.W * a.C + (double)a.F * a.R * a.S * a.C + (double)d.P * a.F * (a.residual ? 2 : 1)), s);
   f->launch(d, a.R * a.S == 1 && a.pad_h == 0 && a.pad_w == 0 ? kPoint : a.C % 64 == 0 ? kLines : kAny, s);
