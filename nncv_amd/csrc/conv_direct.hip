@@ -101,7 +101,7 @@ __device__ __forceinline__ float plain_sum(const DirectArgs& a, int p, int f, bo
 }
 
 // UNI: a tap is a whole number of rounds (C elements = whole 128-byte lines), so the tap of a round is the same for all lanes
-template <typename T, typename OutT, int BT, int TM, int TN, int KG, bool UNI>
+template <typename T, typename OutT, int BT, int TM, int TN, int KG, bool UNI, int D>
 __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a) {
   // Three-way bf16 splits (split.hpp) where two filter blocks share a split of the pixels and there are waves to hide it:
   // 6x58x78x64 -> 128 at stride 2 17.2 -> 14.3 us, 16x28x28x128 -> 256 24.8 -> 19.9.  32 x 32 waves spend as long splitting as they
@@ -112,6 +112,10 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
   constexpr int kWaveLds = 2 * kBuf > kPart || KG == 1 ? 2 * kBuf : kPart;
   constexpr int kQuadsPerBlock = BT * BT / 256, kQuads = TM * TN * kQuadsPerBlock, kMine = (kQuads + KG - 1) / KG;
   extern __shared__ __align__(16) unsigned char smem[];
+  // all arguments at once: fetched where they are first used, they are one wait after the other
+  asm volatile("" ::"s"(a.in), "s"(a.wt), "s"(a.in_bytes), "s"(a.wt_bytes), "s"(a.H), "s"(a.W), "s"(a.F), "s"(a.S), "s"(a.OW), "s"(a.OHW), "s"(a.P), "s"(a.pix),
+               "s"(a.stride_h), "s"(a.stride_w), "s"(a.pad_h), "s"(a.pad_w), "s"(a.chunks), "s"(a.cpt), "s"(a.main_tiles), "s"(a.tiles_f), "s"(a.tiles_p), "s"(a.main_f),
+               "s"(a.inv_ohw), "s"(a.inv_ow), "s"(a.inv_s), "s"(a.inv_cpt), "s"(a.inv_tiles));
   const int lane = threadIdx.x & 63, grp = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int lrow = lane & (BT - 1), lh = lane / BT;
   unsigned char* lds = smem + grp * kWaveLds;
@@ -146,11 +150,16 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
     const unsigned fb = (unsigned)(f >> 5) * (unsigned)(r_n * 4);
     woff[i] = BT == 32 ? (fb * 64u + lane) * 16u : ((fb + (lh >> 1)) * 64u + (lh & 1) * 32u + (f & 16) + lrow) * 16u;
   }
-  auto load_w = [&](int r, int q, u32x4 (&w)[NQ][TM]) {
+  auto load_w = [&](int r, int q, u32x4 (&w)[NQ][TM]) __attribute__((always_inline)) {
     const unsigned at = (unsigned)(4 * (r - r_lo) + (BT == 32 ? q : 2 * q)) * 1024u;
 #pragma unroll
     for (int i = 0; i < TM; ++i) w[q][i] = __builtin_amdgcn_raw_buffer_load_b128(rs_wt, ((f0 + BT * i < f_end) & (r < re)) ? woff[i] + at : kOOBd, 0, 0);
   };
+  u32x4 w[D][NQ][TM];  // the first ones are asked for now: their addresses are there long before the pixels'
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) load_w(rb, q, w[0]);
+  __builtin_amdgcn_sched_barrier(0);
+
   // pixels: this lane loads chunk lane % 8 of the rows lane / 8, + 8, ...; pixels past the end read the last one (not stored)
   // (worked out once per row, a lane each, and handed round through the LDS buffer that is still empty)
   int base[GL], iy0[GL], ix0[GL];
@@ -181,8 +190,8 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
     dr = fast_div(tap, a.S, a.inv_s, &ds);
   }
   int rload = rb;
-  u32x4 gx[GL];
-  auto load_x = [&]() {
+  u32x4 gx[D][GL];
+  auto load_x = [&](u32x4 (&gx)[GL]) __attribute__((always_inline)) {
     int r = ur, s = us, at;
     bool in_k = rload < re;
     if constexpr (UNI) {
@@ -208,7 +217,7 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
     }
   };
   const int wr_at = (lane >> 3) * 128 + (((lane & 7) ^ (lane >> 3)) * 16);
-  auto park = [&](int buf) {
+  auto park = [&](int buf, const u32x4 (&gx)[GL]) __attribute__((always_inline)) {
 #pragma unroll
     for (int g = 0; g < GL; ++g) *reinterpret_cast<u32x4*>(lds + buf * kBuf + g * 1024 + wr_at) = gx[g];
   };
@@ -227,10 +236,14 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
         acc[i][j][v] = 0.0f;
         if constexpr (kSplit) low[i][j][v] = 0.0f;
       }
-  u32x4 w[NQ][TM];
-  load_x();
+  load_x(gx[0]);
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) load_w(rb, q, w);
+  for (int d = 1; d < D; ++d) {
+    __builtin_amdgcn_sched_barrier(0);  // (the first requests leave before the addresses of the others are there)
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) load_w(rb + d * KG, q, w[d]);
+    load_x(gx[d]);
+  }
 
   // what this wave finishes: quads of four consecutive filters of a pixel.  Their residual and scale / shift are asked for
   // now; they arrive under the K walk.
@@ -288,8 +301,8 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
       if (grp + k * KG < kQuads) mine[k] = quad_of(grp + k * KG);
   }
 
-  park(0);
-  load_x();
+  park(0, gx[0]);
+  load_x(gx[0]);
   u32x4 x[TN];  // the pixel operand is read one step ahead of its products
 #pragma unroll
   for (int j = 0; j < TN; ++j) x[j] = operand(0, 0, j);
@@ -304,14 +317,14 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
       for (int q = 0; q < NQ; q += 2) {
         u32x4 wp[TM][3], xp[TN][3];
 #pragma unroll
-        for (int i = 0; i < TM; ++i) split_eight(w[q][i], w[q + 1][i], wp[i]);
+        for (int i = 0; i < TM; ++i) split_eight(w[0][q][i], w[0][q + 1][i], wp[i]);
 #pragma unroll
         for (int j = 0; j < TN; ++j) split_eight(x[j], y[j], xp[j]);
-        load_w(r + KG, q, w);
-        load_w(r + KG, q + 1, w);
+        load_w(r + KG, q, w[0]);
+        load_w(r + KG, q + 1, w[0]);
         if (q == 0) {
-          park(buf ^ 1);
-          load_x();
+          park(buf ^ 1, gx[0]);
+          load_x(gx[0]);
         }
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
@@ -326,25 +339,30 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
 #pragma unroll
       for (int j = 0; j < TN; ++j) acc[i][j] += low[i][j];
   } else {
-    for (int r = rb; r < re; r += KG, buf ^= 1) {
+    for (int r = rb; r < re; r += D * KG, buf ^= D & 1) {
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) {
-        u32x4 xn[TN];
-        if (q == NQ / 2) {
-          park(buf ^ 1);
-          load_x();
+      for (int d = 0; d < D; ++d) {
+        if (d > 0 && r + d * KG >= re) break;  // (uniform)
+        const int here = buf ^ (d & 1);
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+          u32x4 xn[TN];
+          if (q == NQ / 2) {
+            park(here ^ 1, gx[(d + 1) % D]);
+            load_x(gx[(d + 1) % D]);
+          }
+#pragma unroll
+          for (int j = 0; j < TN; ++j) xn[j] = q + 1 < NQ ? operand(here, q + 1, j) : operand(here ^ 1, 0, j);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) Block<T, BT>::run(w[d][q][i], x[j], acc[i][j]);
+          __builtin_amdgcn_sched_barrier(0);
+          load_w(r + (d + D) * KG, q, w[d]);
+#pragma unroll
+          for (int j = 0; j < TN; ++j) x[j] = xn[j];
         }
-#pragma unroll
-        for (int j = 0; j < TN; ++j) xn[j] = q + 1 < NQ ? operand(buf, q + 1, j) : operand(buf ^ 1, 0, j);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j) Block<T, BT>::run(w[q][i], x[j], acc[i][j]);
-        __builtin_amdgcn_sched_barrier(0);
-        load_w(r + KG, q, w);
-#pragma unroll
-        for (int j = 0; j < TN; ++j) x[j] = xn[j];
       }
     }
   }
@@ -406,8 +424,21 @@ void launch_cfg(DirectArgs d, hipStream_t s) {
     (void)attr;
     launch_kernel(kern, dim3((unsigned)((long long)d.tiles_f * d.tiles_p)), dim3(64 * KG), lds, s, d);
   };
-  if (d.cpt % 8 == 0) go(conv_direct_kernel<T, OutT, BT, TM, TN, KG, true>);
-  else go(conv_direct_kernel<T, OutT, BT, TM, TN, KG, false>);
+  auto depth = [&](auto dc) {
+    if (d.cpt % 8 == 0) go(conv_direct_kernel<T, OutT, BT, TM, TN, KG, true, decltype(dc)::value>);
+    else go(conv_direct_kernel<T, OutT, BT, TM, TN, KG, false, decltype(dc)::value>);
+  };
+  // Three rounds of operands in flight for fp16 walks of nine rounds a wave and more, up to two workgroups a CU: the weights of a
+  // pass over one image come from beyond L2 (7x7x512 in such a pass: 8.1 -> 6.9 us, the pass 104.3 -> 101.2; alone, from L2, 6.4 either
+  // way).  Shorter walks lose up to 0.7 us to the longer start, fp32 ones 0.5 (twice the requests per round of products), and 32 x 32
+  // tiles the third wave of a SIMD (55x66x32x128 -> 32 at 7x7, stride 2: 34.1 -> 40.2).
+  if constexpr (sizeof(T) == 2 && BT == 16) {
+    if ((d.chunks + 7) / 8 >= 9 * KG && (long long)d.tiles_f * d.tiles_p <= 512) {
+      depth(std::integral_constant<int, 3>());
+      return;
+    }
+  }
+  depth(std::integral_constant<int, 1>());
 }
 
 // [F][C][RS] filters -> the order a wave reads its operands in: [ceil(F / 32)][rounds * 4 units][64 lanes][16 bytes], lane l of
