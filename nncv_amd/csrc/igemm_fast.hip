@@ -18,10 +18,12 @@
 //    two LDS buffers, one barrier per stage).
 //  * K groups meet in an fp32 LDS tile and the epilogue reads it back so that residual reads and
 //    result stores are whole 128-byte rows (mfma_tile.hpp).
+//  * fp32 blocks without K groups multiply on the bf16 matrix pipes (three-way splits, split.hpp): a 64x64 sub-tile's 16 k are 24
+//    instructions of 32 clocks instead of 32 of 64, and 176 to split its operands, which run beside them (two waves a SIMD).
 //  * Workgroups are renumbered so that each XCD (8 of them, round-robin over the linear workgroup
 //    id) gets a contiguous range of pixel tiles: neighbouring tiles share input rows, and each
 //    XCD has its own L2.
-#include "mfma_tile.hpp"
+#include "split.hpp"
 
 namespace nncv_hip {
 
@@ -33,13 +35,15 @@ constexpr unsigned kOOB = 0x7fffff00u;   // byte offset beyond any buffer this k
 constexpr int kXcds = 8;
 }  // namespace
 
-template <typename T, typename OutT, int WP, int WF, int WK, int KS, int NI>
-__global__ __launch_bounds__(64 * WP * WF * WK) void igemm_fast_kernel(const IgemmArgs a, const int tiles_x,
+template <typename T, typename OutT, int WP, int WF, int WK, int KS, int NI, bool kSplit>
+__global__ __launch_bounds__(64 * WP * WF * WK, kSplit ? 2 : 1) void igemm_fast_kernel(const IgemmArgs a, const int tiles_x,
                                                                        const float inv_ohow, const float inv_ow) {
   constexpr int NT = 64 * WP * WF * WK;
   static_assert(NT == 256, "loader mapping assumes 256 threads");
   constexpr int ES = sizeof(T);
   constexpr int CE = 16 / ES;       // elements per 16-byte chunk
+  // kSplit: three-way bf16 splits (split.hpp) of the operands as they leave LDS, for fp32 tiles without K groups
+  static_assert(!kSplit || (ES == 4 && WK == 1 && NI == 2), "the split form");
   constexpr int BKE = 4 * CE;       // elements per K step
   constexpr int BP = 64 * WP, BF = 64 * WF, ROWS = BP + BF;
   // NI = 1: a workgroup owns 32 filters instead of 64 (twice the workgroups for small problems).
@@ -143,13 +147,16 @@ __global__ __launch_bounds__(64 * WP * WF * WK) void igemm_fast_kernel(const Ige
         *reinterpret_cast<u32x4*>(base + (st * ROWS + 64 * g) * kRow) = r[st * R64 + g];
   };
 
-  floatx16 acc[2][2];  // [f sub-tile][pixel sub-tile]
+  floatx16 acc[2][2], low[kSplit ? 2 : 1][kSplit ? 2 : 1];  // [f sub-tile][pixel sub-tile]; split: the small products' sums
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+      for (int v = 0; v < 16; ++v) {
+        acc[i][j][v] = 0.0f;
+        if constexpr (kSplit) low[i][j][v] = 0.0f;
+      }
 
   const int lrow = lane & 31, lchunk = lane >> 5;
   auto compute = [&](int buf) {
@@ -157,6 +164,17 @@ __global__ __launch_bounds__(64 * WP * WF * WK) void igemm_fast_kernel(const Ige
     const unsigned char* sW = smem + buf * STAGE + (BP + wf * 64 + lrow) * kRow + lchunk * 16;
 #pragma unroll
     for (int st = wk; st < KS; st += WK) {
+      if constexpr (kSplit) {
+        u32x4 w[2][3], p[2][3];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          split_eight(*reinterpret_cast<const u32x4*>(sW + (st * ROWS + i * 32) * kRow), *reinterpret_cast<const u32x4*>(sW + (st * ROWS + i * 32) * kRow + 32), w[i]);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          split_eight(*reinterpret_cast<const u32x4*>(sP + (st * ROWS + j * 32) * kRow), *reinterpret_cast<const u32x4*>(sP + (st * ROWS + j * 32) * kRow + 32), p[j]);
+        split_products(w, p, acc, low);
+        continue;
+      }
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
         u32x4 fw[2], fp[2];
@@ -219,8 +237,42 @@ __global__ __launch_bounds__(64 * WP * WF * WK) void igemm_fast_kernel(const Ige
   const OutT* res = (a.residual && !aux) ? static_cast<const OutT*>(a.residual) + (long long)bz * a.out_bs : nullptr;
   const int fo = aux ? a.aux_f0 : 0;                     // first filter of this output tensor
   const int fend = (aux || a.aux_f0 == 0) ? a.F : a.aux_f0;  // one past its last filter
-  tile_reduce_store<OutT, WK, NI>(acc, smem + wpos * WK * kTileBytes, wk, lane, rowoff, by * BFE + wf * 64 - fo, fend - fo, ess, res, out,
-                              aux ? a.aux_relu : a.relu);
+  if constexpr (kSplit) {
+    // Sums that are not finite (an operand that bf16 does not hold, or a result that is not) are done again in plain fp32
+    unsigned long long again = 0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        acc[i][j] += low[i][j];
+#pragma unroll
+        for (int v = 0; v < 16; ++v) again |= __builtin_fabsf(acc[i][j][v]) < __builtin_inff() ? 0ull : 1ull << ((i * 2 + j) * 16 + v);
+      }
+    auto mend = [&](unsigned char* tile) {
+      for (; again; again &= again - 1) {
+        const int k = __builtin_ctzll(again), i = k >> 5, j = k >> 4 & 1, v = k & 15;
+        const int slot = j * 32 + lrow, chan = i * 32 + 8 * (v >> 2) + 4 * lchunk + (v & 3);
+        const int f = by * BFE + wf * 64 + chan, gp = bx * BP + wp * 64 + slot;
+        if (f >= a.F || gp >= P) continue;
+        int rem, ox;
+        const int n = fast_div(gp, a.OH * a.OW, inv_ohow, &rem), oy = fast_div(rem, a.OW, inv_ow, &ox);
+        float sum = 0.0f;
+        for (int t = aux ? a.aux_tap : 0; t < (aux ? a.aux_tap + 1 : a.R * a.S); ++t) {
+          const int iy = oy * a.stride_h - a.pad_h + t / a.S, ix = ox * a.stride_w - a.pad_w + t % a.S;
+          if ((unsigned)iy >= (unsigned)a.H || (unsigned)ix >= (unsigned)a.W) continue;
+          const float* x = static_cast<const float*>(a.in) + (long long)bz * a.in_bs + (long long)((n * a.H + iy) * a.W + ix) * pix;
+          const float* y = static_cast<const float*>(a.wt) + (long long)bz * a.wt_bs + ((long long)f * a.R * a.S + t) * a.C;
+          for (int c = 0; c < a.C; ++c) sum = __builtin_fmaf(x[c], y[c], sum);
+        }
+        *reinterpret_cast<float*>(tile + slot * kTilePitch + chan * 4) = sum;
+      }
+    };
+    tile_reduce_store<OutT, WK, NI>(acc, smem + wpos * WK * kTileBytes, wk, lane, rowoff, by * BFE + wf * 64 - fo, fend - fo, ess, res, out,
+                                    aux ? a.aux_relu : a.relu, mend);
+  } else {
+    tile_reduce_store<OutT, WK, NI>(acc, smem + wpos * WK * kTileBytes, wk, lane, rowoff, by * BFE + wf * 64 - fo, fend - fo, ess, res, out,
+                                    aux ? a.aux_relu : a.relu);
+  }
 }
 
 namespace {
@@ -229,7 +281,7 @@ template <typename T> constexpr const char* tn();
 template <> constexpr const char* tn<half_t>() { return "f16"; }
 template <> constexpr const char* tn<float>() { return "f32"; }
 
-template <typename T, typename OutT, int WP, int WF, int WK, int KS, int NI = 2>
+template <typename T, typename OutT, int WP, int WF, int WK, int KS, int NI = 2, bool SPLIT = false>
 void launch_fast_cfg(const IgemmArgs& a, hipStream_t s) {
   constexpr int BP = 64 * WP, BF = 64 * WF, BFE = NI == 2 ? BF : 32;
   constexpr int stage2 = 2 * KS * (BP + BF) * kRow;
@@ -237,7 +289,7 @@ void launch_fast_cfg(const IgemmArgs& a, hipStream_t s) {
   constexpr int smem = stage2 > epi ? stage2 : epi;
   static const std::string tag = std::string("igemm_fast<") + tn<T>() + "," + tn<OutT>() + "," + std::to_string(WP) + "," +
                                  std::to_string(WF) + "," + std::to_string(WK) + "," + std::to_string(KS) + (NI == 1 ? ",half>" : ">");
-  auto kern = igemm_fast_kernel<T, OutT, WP, WF, WK, KS, NI>;
+  auto kern = igemm_fast_kernel<T, OutT, WP, WF, WK, KS, NI, SPLIT>;
   static const bool attr_set = [&] {
     NNCV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
     return true;
@@ -271,6 +323,16 @@ void launch_fast_typed(const IgemmArgs& a, hipStream_t s) {
     else if (blocks(128, 64) >= 256) pick = 3;
     else if (blocks(64, 64) >= 128 || a.F % 32 != 0) pick = 4;
     else pick = 5;  // fewer than 128 workgroups of 64x64: halve the filter blocks
+  }
+  // fp32 blocks without K groups: on the bf16 matrix pipes from 32 k on (1.17 times at 64, 1.3 at 144, 1.4 to 1.6 at 400; the 7x7
+  // stem of 6x224x303 40.3 -> 30.8 us); a single step of 16 is bound by memory (55x9x90x16 -> 128 10.5 against 10.9).  Blocks with K
+  // groups have as many waves as their steps, and wait for memory.
+  if constexpr (sizeof(T) == 4) {
+    if (pick <= 2 && a.R * a.S * a.C >= 32) {
+      if (pick == 1) launch_fast_cfg<T, OutT, 2, 2, 1, 1, 2, true>(a, s);
+      else launch_fast_cfg<T, OutT, 4, 1, 1, 1, 2, true>(a, s);
+      return;
+    }
   }
   switch (pick) {
     case 1: launch_fast_cfg<T, OutT, 2, 2, 1, 1>(a, s); break;
