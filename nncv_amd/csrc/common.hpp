@@ -273,6 +273,7 @@ bool conv_ring_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 double conv_ring_us(const IgemmArgs& a);
 bool conv_ring_beats_patch_s2(const IgemmArgs& a);
 void launch_conv_ring(const IgemmArgs& a, hipStream_t s);
+double igemm_fast_split_us(const IgemmArgs& a);
 bool igemm_fast_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 void launch_igemm_fast(const IgemmArgs& a, int in_dt, int out_dt, hipStream_t s);
 

@@ -545,6 +545,10 @@ double other_us(const IgemmArgs& a, int dt, DirectRival rival) {
     if (wgs <= 128 && main_f % 64 == 0) return 4.9 + 0.132 * rounds;
     return wgs > 128 && wgs <= 144 ? 1e30 : 4.3 + 0.26 * rounds * turns;
   }
+  if (rival == kRivalIgemmFast && dt == kF32) {
+    const double split = igemm_fast_split_us(a);
+    if (split > 0) return split;
+  }
   const Fit& f = rival == kRivalPatch || rival == kRivalPatchS2 ? f16_3x3[rival] : (dt == kF16 ? f16 : f32)[rival - kRivalIgemmFast];
   const double tiles = (double)((main_f + 63) / 64) * (double)(((long long)a.N * a.OH * a.OW + 63) / 64);
   return f.fixed + std::max(1.0, tiles / 256) * (f.round * rounds + f.tile) + f.chain * rounds;
