@@ -8,11 +8,13 @@
 //    contiguous kilobytes, straight into registers, three steps ahead.
 //  * Two patch buffers: a slab is multiplied while the next one is split into the other buffer, between the products, and the one
 //    after that is on its way to registers.  One barrier a slab.
-//  * Four waves: WS = 4, 2: each 64 slots x 32 filters; WS = 1: 64 x 32 (NI = 1: 32 x 32) with
-//    the two 16-channel steps of a tap dealt to two K groups, whose sums meet in LDS.
+//  * Eight waves, or four where two workgroups share a CU (launch_ws1).  A wave's share of the tile is 64 slots x 32 filters (WS = 1,
+//    NI = 1: 32 x 32), its K groups take a 16-channel half of a slab each, four of them the even or the odd taps of a half; their
+//    sums meet in LDS.
 //  * A sum that is not finite is done again in plain fp32.
-//  * What bounds it: the matrix pipes where tiles fill the CUs (six products, 2.7 times the fp32 instructions' rate), one wave a
-//    SIMD issuing everything where they do not.
+//  * What bounds it: the matrix pipes where tiles fill the CUs (six products, 2.7 times the fp32 instructions' rate), a slab's
+//    barrier and the LDS reads behind it where they do not: two waves a SIMD cover each other there (six 224x224 images classified by an
+//    fp32 ResNet-18: 373 us with one, 353 with two).
 #include <type_traits>
 
 #include "patch_args.hpp"
@@ -27,9 +29,11 @@ namespace {
 constexpr int kCell = 208;              // 3 x 64 + 16: at 13 units of 16 bytes, 16 neighbouring cells touch every bank once
 constexpr int kRowSpare = 96;           // behind a patch row: its pitch is 13 TW units mod 16 then, as if a tile's rows were one
 
+constexpr int split_units(int ws) { return ws == 1 ? 2 : 4; }  // waves that a workgroup's tile is dealt to
+
 template <int WS>
 struct SplitCfg {
-  static constexpr int cap = PatchCap<WS>::pix, passes = cap / 32;  // loader: 8 threads a pixel, 32 pixels a pass
+  static constexpr int cap = PatchCap<WS>::pix;
   static constexpr int buffers = WS == 4 ? 1 : 2;                     // (256 slots: layers of one slab)
   static constexpr int patch = cap * kCell, dump = buffers * patch, scale = dump + 640, smem = scale + 512;
 };
@@ -49,8 +53,8 @@ __device__ __forceinline__ float plain_sum(const PatchArgs& a, int p, int f) {
   return sum;
 }
 
-template <int WS, int NI>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void conv3x3_split_kernel(
+template <int WS, int NI, int KG>  // KG: K groups, waves that share a tile's sums
+__global__ __launch_bounds__(64 * KG * split_units(WS)) __attribute__((amdgpu_waves_per_eu(2, 2))) void conv3x3_split_kernel(
     // (the values the patch addressing needs first: preloaded into SGPRs)
     const void* in_p, int tiles_p, int tiles_y_p, int tn_p, int th_p, int n_p, int h_p, int w_p, int c_p, int rw_log_p, int xcd_by_filter_p,
     unsigned in_bytes_p, int txw_p, const PatchArgs a_rest) {
@@ -59,10 +63,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   a.in = in_p; a.tiles = tiles_p; a.tiles_y = tiles_y_p; a.TN = tn_p; a.TH = th_p; a.N = n_p; a.H = h_p; a.W = w_p; a.C = c_p;
   a.rw_log = rw_log_p; a.xcd_by_filter = xcd_by_filter_p; a.in_bytes = in_bytes_p;
   typedef SplitCfg<WS> Cfg;
-  constexpr int kPasses = Cfg::passes;
-  constexpr int IN = 1, JN = WS == 1 && NI == 1 ? 1 : 2, KG = WS == 1 ? 2 : 1;  // filter and slot blocks of a wave, K groups
-  constexpr int KPG = 2 / KG, NSET = JN == 1 ? 9 : 3;                  // steps of a tap, steps whose filters are on their way
-  constexpr int kSteps = 9 * KPG, kQuads = IN * JN * 4;
+  constexpr int kThreads = 64 * KG * split_units(WS), kPass = kThreads / 8, kPasses = Cfg::cap / kPass;  // loader: 8 threads a pixel
+  constexpr int JN = WS == 1 && NI == 1 ? 1 : 2;  // slot blocks of a wave
+  constexpr int kQuads = JN * 4;
   static_assert(WS != 2 || NI == 2, "128 slots: two waves to a filter half");
   static_assert(WS != 4 || NI == 1, "256 slots: every wave has its own");
   extern __shared__ __align__(16) unsigned char smem[];
@@ -89,9 +92,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int slot0 = WS == 4 ? wave * 64 : WS == 2 ? (wave & 1) * 64 : NI == 1 ? (wave >> 1) * 32 : 0;
-  const int kg = KG == 2 ? wave & 1 : 0;
-  const int half = NI == 1 ? fblk & 1 : wave >> 1;                 // of the 64-filter block
+  // K group g: channels 16 (g % 2) .. of a slab, and with four groups the taps 2 i + g / 2.  Waves w and w + 4 share a SIMD: one
+  // of them has the five even taps, the other the four odd ones.
+  const int unit = wave / KG, kg = KG == 4 ? (wave & 3) ^ (unit << 1) : wave % KG;
+  auto wave_of = [&](int g) { return unit * KG + (KG == 4 ? g ^ (unit << 1) : g); };
+  const int slot0 = WS == 4 ? unit * 64 : WS == 2 ? (unit & 1) * 64 : NI == 1 ? unit * 32 : 0;
+  const int half = NI == 1 ? fblk & 1 : WS == 2 ? unit >> 1 : unit;                  // of the 64-filter block
   const int fb64 = NI == 1 ? fblk >> 1 : fblk, f0 = fb64 * 64 + half * 32;          // this wave's first filter
   const int lrow = lane & 31, lh = lane >> 5;
   const __amdgpu_buffer_rsrc_t rs_in = make_rsrc(a.in, a.in_bytes);
@@ -105,7 +111,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   unsigned pvoff[kPasses];
 #pragma unroll
   for (int i = 0; i < kPasses; ++i) {
-    const int q = i * 32 + p8, r = q >> a.rw_log, px = q & rwm;
+    const int q = i * kPass + p8, r = q >> a.rw_log, px = q & rwm;
     int n = n0, py = r;
     if (a.TN > 1) n += fast_div(r, PH, a.inv_ph, &py);
     const int iy = y0 + py - 1;
@@ -117,7 +123,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   unsigned pdst[kPasses];
 #pragma unroll
   for (int i = 0; i < kPasses; ++i) {
-    const int q = i * 32 + p8, r = q >> a.rw_log, px = q & rwm;
+    const int q = i * kPass + p8, r = q >> a.rw_log, px = q & rwm;
     const int sub = (c4 >> 2) * 32 + (c4 & 1) * 16 + ((c4 >> 1) & 1) * 8;
     pdst[i] = ((px < PW) & (r < prows)) ? __umul24(r, RP) + __umul24(px, kCell) + sub : Cfg::dump + lane * 8;
   }
@@ -138,16 +144,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
   // ---- filters: the operand of iteration (slab, tap), step k, half i, piece c is the kilobyte at
   //      (((fb64 * niter + it) * 2 + k) * 2 + i) * 3 + c ----
-  const int wbase = (fb64 * niter * 4 + kg * 2 + half) * 3072;
+  const int wbase = (fb64 * niter * 4 + (kg & 1) * 2 + half) * 3072;
   const unsigned wlane = lane * 16;
-  u32x4 w[NSET][1][3];
-  auto wload = [&](u32x4 (&r)[1][3], int it, int k) {
+  auto wload = [&](u32x4 (&r)[1][3], int it, int k) __attribute__((always_inline)) {
     const int so = it < niter ? wbase + it * 12288 + k * 6144 : 0;  // past the end: block 0 again (never used)
 #pragma unroll
     for (int c = 0; c < 3; ++c) r[0][c] = __builtin_amdgcn_raw_buffer_load_b128(rs_wf, wlane, so + c * 1024, 0);
   };
-#pragma unroll
-  for (int t = 0; t < NSET; ++t) wload(w[t], t / KPG, t % KPG);
   if (tid < 64) {
     const int f = fb64 * 64 + tid;
     float* ss = reinterpret_cast<float*>(smem + Cfg::scale);
@@ -171,90 +174,102 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     if (a.TN > 1) nl = fast_div(sl, a.TH * TW, a.inv_thw, &rem);
     const int ty = fast_div(rem, TW, a.inv_w, &tx);
     const bool ok = (sl < nslots) & ((n0 + nl) < a.N) & ((y0 + ty) < a.H) & ((x0 + tx) < a.W);
-    sbase[j] = (ok ? (int)__umul24(__umul24(nl, PH) + ty, RP) + (int)__umul24(tx, kCell) : 0) + lh * 16 + kg * KPG * 32;
+    sbase[j] = (ok ? (int)__umul24(__umul24(nl, PH) + ty, RP) + (int)__umul24(tx, kCell) : 0) + lh * 16 + (kg & 1) * 32;
     obase[j] = (ok && sl0 < nslots) ? (((n0 + nl) * a.H + y0 + ty) * a.W + x0 + tx) * a.ldo : -1;
   }
 
-  floatx16 big[IN][JN], low[IN][JN];
+  floatx16 big[1][JN], low[1][JN];
 #pragma unroll
-  for (int i = 0; i < IN; ++i)
+  for (int j = 0; j < JN; ++j)
 #pragma unroll
-    for (int j = 0; j < JN; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) big[i][j][v] = low[i][j][v] = 0.0f;
+    for (int v = 0; v < 16; ++v) big[0][j][v] = low[0][j][v] = 0.0f;
 
-  // ---- tap loop: one trip = one slab = 9 taps x KPG steps, unrolled.  Under the products of a step: the pixel operand of the next
+  // ---- tap loop: one trip = one slab = this wave's taps, unrolled.  Under the products of a step: the pixel operand of the next
   //      one is read, the filters of NSET steps further on are asked for, and a share of the next slab's patch is split into the
   //      other buffer and that of the slab after it asked for ----
-  u32x4 ring[2][JN][3];
-  int row[3][JN];
-  auto ldp = [&](auto step_c) {
-    constexpr int st = decltype(step_c)::value, t = st / KPG, k = st % KPG;
+  auto walk = [&](auto par_c) __attribute__((always_inline)) {
+    constexpr int PAR = decltype(par_c)::value;                                 // four K groups: odd taps
+    constexpr int kSteps = KG == 1 ? 18 : KG == 2 ? 9 : 5 - PAR, NSET = KG == 4 ? kSteps : JN == 1 ? 9 : 3;  // steps whose filters are on their way
+    auto tap_of = [](int st) constexpr { return KG == 1 ? st / 2 : KG == 2 ? st : 2 * st + PAR; };
+    auto k_of = [](int st) constexpr { return KG == 1 ? st & 1 : 0; };
+    u32x4 w[NSET][1][3];
 #pragma unroll
-    for (int j = 0; j < JN; ++j)
+    for (int t = 0; t < NSET; ++t) wload(w[t], tap_of(t), k_of(t));
+    u32x4 ring[2][JN][3];
+    int row[3][JN];
+    auto ldp = [&](auto step_c) __attribute__((always_inline)) {
+      constexpr int st = decltype(step_c)::value, t = tap_of(st), k = k_of(st);
 #pragma unroll
-      for (int c = 0; c < 3; ++c)
-        ring[st & 1][j][c] = *reinterpret_cast<const u32x4*>(smem + row[t / 3][j] + (t % 3) * kCell + k * 32 + c * 64);
-  };
+      for (int j = 0; j < JN; ++j)
 #pragma unroll
-  for (int i = 0; i < kPasses; ++i) {
-    pstore(i, 0);
-    if (Cfg::buffers == 2) pload(i, 1);
-  }
-  __syncthreads();
-  for (int slab = 0; slab < nslab; ++slab) {
-    const int at = Cfg::buffers == 2 ? (slab & 1) * Cfg::patch : 0;
-    const unsigned other = Cfg::patch - at;
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-      for (int j = 0; j < JN; ++j) row[r][j] = sbase[j] + at + r * RP;
-    ldp(std::integral_constant<int, 0>());
-    __builtin_amdgcn_sched_barrier(0);
-    auto steps = [&](auto self, auto step_c) -> void {
-      constexpr int st = decltype(step_c)::value;
-      if constexpr (st < kSteps) {
-        constexpr int nx = st + NSET, p0 = st * kPasses / kSteps, p1 = Cfg::buffers == 2 ? (st + 1) * kPasses / kSteps : p0;
-        if constexpr (st + 1 < kSteps) ldp(std::integral_constant<int, st + 1>());
-        split_products(w[st % NSET], ring[st & 1], big, low);
-        wload(w[st % NSET], (slab + nx / kSteps) * 9 + nx % kSteps / KPG, nx % KPG);
-#pragma unroll
-        for (int i = p0; i < p1; ++i) {
-          pstore(i, other);
-          pload(i, slab + 2);
-        }
-        constexpr int kMma = 6 * JN, kValu = (26 * (p1 - p0) + kMma - 1) / kMma;
-#pragma unroll
-        for (int n = 0; n < kMma; ++n) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          if (kValu) __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);
-          __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        self(self, std::integral_constant<int, st + 1>());
-      }
+        for (int c = 0; c < 3; ++c) ring[st & 1][j][c] = *reinterpret_cast<const u32x4*>(smem + row[t / 3][j] + (t % 3) * kCell + k * 32 + c * 64);
     };
-    steps(steps, std::integral_constant<int, 0>());
-    __syncthreads();  // every wave has left this patch and written its share of the next
+#pragma unroll
+    for (int i = 0; i < kPasses; ++i) {
+      pstore(i, 0);
+      if (Cfg::buffers == 2) pload(i, 1);
+    }
+    __syncthreads();
+    for (int slab = 0; slab < nslab; ++slab) {
+      const int at = Cfg::buffers == 2 ? (slab & 1) * Cfg::patch : 0;
+      const unsigned other = Cfg::patch - at;
+#pragma unroll
+      for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int j = 0; j < JN; ++j) row[r][j] = sbase[j] + at + r * RP;
+      ldp(std::integral_constant<int, 0>());
+      __builtin_amdgcn_sched_barrier(0);
+      auto steps = [&](auto self, auto step_c) __attribute__((always_inline)) -> void {
+        constexpr int st = decltype(step_c)::value;
+        if constexpr (st < kSteps) {
+          constexpr int nx = st + NSET, p0 = st * kPasses / kSteps, p1 = Cfg::buffers == 2 ? (st + 1) * kPasses / kSteps : p0;
+          if constexpr (st + 1 < kSteps) ldp(std::integral_constant<int, st + 1>());
+          split_products(w[st % NSET], ring[st & 1], big, low);
+          wload(w[st % NSET], (slab + nx / kSteps) * 9 + tap_of(nx % kSteps), k_of(nx % kSteps));
+#pragma unroll
+          for (int i = p0; i < p1; ++i) {
+            pstore(i, other);
+            pload(i, slab + 2);
+          }
+          constexpr int kMma = 6 * JN, kValu = (26 * (p1 - p0) + kMma - 1) / kMma;
+#pragma unroll
+          for (int n = 0; n < kMma; ++n) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            if (kValu) __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);
+            __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          self(self, std::integral_constant<int, st + 1>());
+        }
+      };
+      steps(steps, std::integral_constant<int, 0>());
+      __syncthreads();  // every wave has left this patch and written its share of the next
+    }
+  };
+  if constexpr (KG < 4) {
+    walk(std::integral_constant<int, 0>());
+  } else {  // (as many barriers on both sides)
+    if (kg < 2) walk(std::integral_constant<int, 0>());
+    else walk(std::integral_constant<int, 1>());
   }
 
-  // ---- out: quad (i, j, g): filters 32 i + 8 g + 4 lh .. + 3 of slot block j.  K group g finishes every second quad ----
+  // ---- out: quad (j, g): filters 8 g + 4 lh .. + 3 of slot block j.  K group g finishes quads g, g + KG ... ----
   constexpr int kMine = kQuads / KG;
   auto sum_of = [&](int q) {
-    const int i = q / (4 * JN), j = q / 4 % JN, g = q & 3;
+    const int j = q / 4, g = q & 3;
     floatx4 s;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) s[e] = big[i][j][4 * g + e] + low[i][j][4 * g + e];
+    for (int e = 0; e < 4; ++e) s[e] = big[0][j][4 * g + e] + low[0][j][4 * g + e];
     return s;
   };
   const float* res = static_cast<const float*>(a.residual);
   float* out = static_cast<float*>(a.out);
   const float* ss = reinterpret_cast<const float*>(smem + Cfg::scale) + half * 32 + 4 * lh;
   auto at_of = [&](int q, int* f) {  // element of the quad's first result, -1: not stored
-    const int o = obase[q / 4 % JN];
-    *f = f0 + (q / (4 * JN)) * 32 + (q & 3) * 8 + 4 * lh;
+    const int o = JN == 2 && q / 4 ? obase[JN - 1] : obase[0];
+    *f = f0 + (q & 3) * 8 + 4 * lh;
     return o >= 0 && *f < a.F ? (long long)o + *f : -1ll;
   };
   floatx4 rv[kMine];
@@ -262,24 +277,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int m = 0; m < kMine; ++m) {
       int f;
-      const long long at = at_of(KG == 2 ? 2 * m + kg : m, &f);
+      const long long at = at_of(KG * m + kg, &f);
       rv[m] = at >= 0 ? *reinterpret_cast<const floatx4*>(res + at) : floatx4{};
     }
   }
   floatx4 sums[kMine];
-  if constexpr (KG == 2) {
-    floatx4* part = reinterpret_cast<floatx4*>(smem);  // [wave][quad of the other group][lane]
-#pragma unroll
-    for (int m = 0; m < kMine; ++m) part[(wave * kMine + m) * 64 + lane] = kg ? sum_of(2 * m) : sum_of(2 * m + 1);
-    __syncthreads();
-#pragma unroll
-    for (int m = 0; m < kMine; ++m) sums[m] = (kg ? sum_of(2 * m + 1) : sum_of(2 * m)) + part[((wave ^ 1) * kMine + m) * 64 + lane];
-  } else {
+  if constexpr (KG == 1) {
 #pragma unroll
     for (int m = 0; m < kMine; ++m) sums[m] = sum_of(m);
+  } else {
+    floatx4* part = reinterpret_cast<floatx4*>(smem);  // [wave][quad][lane]
+#pragma unroll
+    for (int q = 0; q < kQuads; ++q) part[(wave * kQuads + q) * 64 + lane] = sum_of(q);
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < kMine; ++m) {
+      floatx4 v[KG];
+#pragma unroll
+      for (int g = 0; g < KG; ++g) v[g] = part[(wave_of(g) * kQuads + KG * m + kg) * 64 + lane];
+      sums[m] = KG == 2 ? v[0] + v[1] : (v[0] + v[1]) + (v[KG - 2] + v[KG - 1]);
+    }
   }
   auto put = [&](int q, long long at, floatx4 y, const floatx4& r) {
-    const int b = (q / (4 * JN)) * 32 + (q & 3) * 8;
+    const int b = (q & 3) * 8;
     y = y * *reinterpret_cast<const floatx4*>(ss + b) + *reinterpret_cast<const floatx4*>(ss + 64 + b);
     if (res) y += r;
     if (a.relu == kActRelu) {
@@ -291,7 +311,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   unsigned again = 0;
 #pragma unroll
   for (int m = 0; m < kMine; ++m) {
-    const int q = KG == 2 ? 2 * m + kg : m;
+    const int q = KG * m + kg;
     int f;
     const long long at = at_of(q, &f);
     if (at < 0) continue;
@@ -300,37 +320,51 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
   for (; again; again &= again - 1) {
     const int q = __builtin_ctz(again);
-    const int o = JN == 2 && (q / 4 % JN) ? obase[JN - 1] : obase[0], f = f0 + (q / (4 * JN)) * 32 + (q & 3) * 8 + 4 * lh;
+    int f;
+    const long long at = at_of(q, &f);
+    const int o = (int)(at - f);
     floatx4 s;
 #pragma unroll 1
     for (int e = 0; e < 4; ++e) s[e] = plain_sum(a, o / a.ldo, f + e);
-    const long long at = (long long)o + f;
     put(q, at, s, res ? *reinterpret_cast<const floatx4*>(res + at) : floatx4{});
   }
 }
 
-template <int WS, int NI>
-void launch_cfg(const PatchArgs& b, hipStream_t s) {
-  auto kern = conv3x3_split_kernel<WS, NI>;
+template <int WS, int NI, int KG>
+void launch_cfg(const PatchArgs& b, int fblocks, hipStream_t s) {
+  auto kern = conv3x3_split_kernel<WS, NI, KG>;
   static const bool attr = [&] {
     NNCV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, SplitCfg<WS>::smem));
     return true;
   }();
   (void)attr;
-  const int fblocks = (b.F + 32 * NI - 1) / (32 * NI);
   const dim3 grid((b.tiles + kXcdsP - 1) / kXcdsP * kXcdsP, fblocks);
-  launch_kernel(kern, grid, dim3(256), SplitCfg<WS>::smem, s, b.in, b.tiles, b.tiles_y, b.TN, b.TH, b.N, b.H, b.W, b.C, b.rw_log,
-                b.xcd_by_filter && fblocks % kXcdsP == 0, b.in_bytes, b.txw, b);
+  launch_kernel(kern, grid, dim3(64 * KG * split_units(WS)), SplitCfg<WS>::smem, s, b.in, b.tiles, b.tiles_y, b.TN, b.TH, b.N, b.H, b.W, b.C,
+                b.rw_log, b.xcd_by_filter && fblocks % kXcdsP == 0, b.in_bytes, b.txw, b);
+}
+
+// WS = 1: eight waves unless a CU gets a second workgroup beside its first (LDS has room for two): there are more of them than the 32
+// CUs of an XCD.  Four -> eight waves, us: one a CU 15.3 -> 14.8 (128 -> 128 channels, 29x39, 6 images), 17.6 -> 16.0 (256 -> 256,
+// 15x20, 6), 10.4 -> 9.0 (128 -> 128, 16x27, 6); two a CU 22.7 -> 25.2 (128 -> 64, 35x57, 9), 32.5 -> 35.6 (224 -> 152, 14x19, 17: 33
+// on an XCD).  WS = 2 leaves room for one only: eight, 29.1 -> 27.8 (64 -> 64, 56x56, 16).  WS = 4 comes with many workgroups, two a
+// CU: four, 36.3 -> 42.9 (32 -> 352, 53x47, 8).
+template <int NI>
+void launch_ws1(const PatchArgs& b, int fblocks, hipStream_t s) {
+  const bool by_filter = b.xcd_by_filter && fblocks % kXcdsP == 0;
+  const long long on_xcd = by_filter ? (long long)b.tiles * (fblocks / kXcdsP) : (long long)((b.tiles + kXcdsP - 1) / kXcdsP) * fblocks;
+  if (on_xcd > 32) launch_cfg<1, NI, 2>(b, fblocks, s);
+  else launch_cfg<1, NI, 4>(b, fblocks, s);
 }
 
 }  // namespace
 
 void launch_conv3x3_split(const PatchArgs& a, int ws, bool half, const char* tag, double flops, double bytes, hipStream_t s) {
   ProfScope prof(tag, flops, bytes, s);
-  if (ws == 4) launch_cfg<4, 1>(a, s);
-  else if (ws == 2) launch_cfg<2, 2>(a, s);
-  else if (half) launch_cfg<1, 1>(a, s);
-  else launch_cfg<1, 2>(a, s);
+  const int halves = (a.F + 31) / 32, blocks = (a.F + 63) / 64;
+  if (ws == 4) launch_cfg<4, 1, 1>(a, halves, s);
+  else if (ws == 2) launch_cfg<2, 2, 2>(a, blocks, s);
+  else if (half) launch_ws1<1>(a, halves, s);
+  else launch_ws1<2>(a, blocks, s);
 }
 
 }  // namespace nncv_hip

@@ -14,7 +14,9 @@ pytestmark = pytest.mark.gpu
 # tile, several images a tile, rows cut into column tiles, fewer pixels than a tile
 CASES = [(8, 32, 344, 53, 47, "4,1"), (15, 32, 480, 35, 17, "4,1"), (6, 64, 64, 58, 78, "2,2"), (25, 160, 152, 11, 22, "2,2"), (3, 128, 328, 51, 25, "2,2"),
          (12, 128, 200, 19, 13, "1,4"), (33, 96, 72, 31, 9, "1,4"), (5, 96, 456, 19, 13, "1,4"), (6, 256, 256, 15, 20, "1,4,half"),
-         (4, 224, 256, 40, 7, "1,4,half"), (16, 512, 512, 7, 7, "1,4,half"), (5, 128, 128, 25, 17, "1,4,half")]
+         (4, 224, 256, 40, 7, "1,4,half"), (16, 512, 512, 7, 7, "1,4,half"), (5, 128, 128, 25, 17, "1,4,half"),
+         # more workgroups on an XCD than it has CUs
+         (17, 224, 152, 14, 19, "1,4"), (9, 512, 896, 8, 8, "1,4,half")]
 
 
 def layer_and_reference(case, seed, spoil=None):
