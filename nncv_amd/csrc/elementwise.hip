@@ -546,25 +546,36 @@ void launch_maxpool_nhwc(const void* in, void* out, int dt, int N, int H, int W,
 // Yolov5s.mlir: y1 = m(x), y2 = m(y1), y3 = m(y2), all four concatenated): one launch instead of
 // three.  A workgroup owns one image x one 16-byte channel vector: the H*W map sits in LDS, each
 // stage takes five row maxima and then five of those down the column (the -inf halo is a skipped
-// tap) and writes its result both to memory and to the other LDS map.  The maps are 20x20 for a 640x640 input, so the three
-// stand-alone launches were nothing but latency (16 us each for 3 MB).
+// tap) and writes its result both to memory and to the other LDS map.  The maxima stay in the tensor's type: two
+// three-operand instructions (NaN goes through them) make five.
+// What bounds it: latency, its 13 MB (16 images of 20x20x256) are small.  A pixel's vectors share cache lines, so an XCD takes a run of
+// them: dealt out one by one they brought every line into eight L2s.
+// 17.1 us one by one with fp32 maxima and 256 threads, 7.6 now.
 // ---------------------------------------------------------------------------------------------
 constexpr int kPoolChainMaxHW = 1600;
 
+template <typename V>
+__device__ __forceinline__ V max5(const V& a, const V& b, const V& c, const V& d, const V& e) {
+  const V m = __builtin_elementwise_maximum(a, __builtin_elementwise_maximum(b, c));
+  return __builtin_elementwise_maximum(m, __builtin_elementwise_maximum(d, e));
+}
+
 template <typename T>
-__global__ __launch_bounds__(256) void maxpool5_chain3_kernel(const T* __restrict__ in, T* __restrict__ o1, T* __restrict__ o2,
+__global__ __launch_bounds__(512) void maxpool5_chain3_kernel(const T* __restrict__ in, T* __restrict__ o1, T* __restrict__ o2,
                                                               T* __restrict__ o3, int H, int W, int CG, int ldi, int ld1, int ld2,
-                                                              int ld3) {
+                                                              int ld3, int units) {
   constexpr int VN = V16<T>::n;
   typedef typename V16<T>::type V;
   extern __shared__ __align__(16) unsigned char pool_smem[];
-  const int HW = H * W, tid = threadIdx.x;
+  const int HW = H * W, tid = threadIdx.x, step = blockDim.x;
   V* bufs = reinterpret_cast<V*>(pool_smem);  // two maps that take turns + the row maxima of the current stage
   V* rowmax = bufs + 2 * HW;
-  const int n = blockIdx.x / CG, cg = blockIdx.x - n * CG;
+  const int unit = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  if (unit >= units) return;  // (uniform; before any barrier)
+  const int n = unit / CG, cg = unit - n * CG;
   const float inv_w = 1.0f / (float)W;
   in += (long long)n * HW * ldi + cg * VN;
-  for (int p = tid; p < HW; p += 256) bufs[p] = *reinterpret_cast<const V*>(in + (long long)p * ldi);
+  for (int p = tid; p < HW; p += step) bufs[p] = *reinterpret_cast<const V*>(in + (long long)p * ldi);
   __syncthreads();
 #pragma unroll
   for (int stage = 0; stage < 3; ++stage) {
@@ -573,38 +584,17 @@ __global__ __launch_bounds__(256) void maxpool5_chain3_kernel(const T* __restric
     const int ldo = stage == 0 ? ld1 : stage == 1 ? ld2 : ld3;
     T* out = (stage == 0 ? o1 : stage == 1 ? o2 : o3) + ((long long)n * HW * ldo + cg * VN);
     // the 5x5 maximum as five columns of row maxima (the maximum does not depend on the order, NaN included)
-    for (int p = tid; p < HW; p += 256) {
+    for (int p = tid; p < HW; p += step) {
       int y = (int)((float)p * inv_w), x = p - y * W;  // exact for p < 2^24 after the correction
       if (x >= W) { ++y; x -= W; }
       if (x < 0) { --y; x += W; }
-      float m[VN];
-#pragma unroll
-      for (int e = 0; e < VN; ++e) m[e] = -INFINITY;
-#pragma unroll
-      for (int q = -2; q <= 2; ++q) {
-        const V v = src[(unsigned)(x + q) < (unsigned)W ? p + q : p];  // outside the map: the centre again, which changes nothing
-#pragma unroll
-        for (int e = 0; e < VN; ++e) m[e] = max_nan(m[e], (float)v[e]);
-      }
-      V o;
-#pragma unroll
-      for (int e = 0; e < VN; ++e) o[e] = (T)m[e];
-      rowmax[p] = o;
+      auto at = [&](int q) { return src[(unsigned)(x + q) < (unsigned)W ? p + q : p]; };  // outside the map: the centre again, which changes nothing
+      rowmax[p] = max5(at(-2), at(-1), at(0), at(1), at(2));
     }
     __syncthreads();
-    for (int p = tid; p < HW; p += 256) {
-      float m[VN];
-#pragma unroll
-      for (int e = 0; e < VN; ++e) m[e] = -INFINITY;
-#pragma unroll
-      for (int r = -2; r <= 2; ++r) {
-        const V v = rowmax[(unsigned)(p + r * W) < (unsigned)HW ? p + r * W : p];
-#pragma unroll
-        for (int e = 0; e < VN; ++e) m[e] = max_nan(m[e], (float)v[e]);
-      }
-      V o;
-#pragma unroll
-      for (int e = 0; e < VN; ++e) o[e] = (T)m[e];
+    for (int p = tid; p < HW; p += step) {
+      auto at = [&](int r) { return rowmax[(unsigned)(p + r * W) < (unsigned)HW ? p + r * W : p]; };
+      const V o = max5(at(-2), at(-1), at(0), at(1), at(2));
       dst[p] = o;
       *reinterpret_cast<V*>(out + (long long)p * ldo) = o;
     }
@@ -622,10 +612,12 @@ void launch_maxpool5_chain3(const void* in, void* o1, void* o2, void* o3, int dt
                             int ld3, hipStream_t s) {
   const int vn = dt == kF16 ? 8 : 4;
   NNCV_REQUIRE(maxpool5_chain3_applicable(dt, H, W, C) && ldi % vn == 0 && ld1 % vn == 0 && ld2 % vn == 0 && ld3 % vn == 0 &&
-                   ldi >= C && ld1 >= C && ld2 >= C && ld3 >= C && (long long)N * (C / vn) < (1ll << 31),
+                   ldi >= C && ld1 >= C && ld2 >= C && ld3 >= C && (long long)N * (C / vn) < (1ll << 31) - 8,
                "maxpool chain: shape not covered");
   ProfScope prof("maxpool5_chain3", 0.0, (double)dtype_size(dt) * N * C * 4.0 * H * W, s);
-  const dim3 grid((unsigned)((long long)N * (C / vn)));
+  const long long units = (long long)N * (C / vn);
+  if (units == 0) return;
+  const dim3 grid((unsigned)((units + 7) / 8 * 8)), block(H * W > 256 ? 512 : 256);  // one pass over the map up to 512 pixels
   static const bool once = [] {
     NNCV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(maxpool5_chain3_kernel<half_t>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, 3 * kPoolChainMaxHW * 16));
@@ -636,11 +628,11 @@ void launch_maxpool5_chain3(const void* in, void* o1, void* o2, void* o3, int dt
   (void)once;
   const size_t smem = (size_t)3 * H * W * 16;
   if (dt == kF16)
-    launch_kernel((maxpool5_chain3_kernel<half_t>), grid, dim3(256), smem, s, (const half_t*)in, (half_t*)o1, (half_t*)o2, (half_t*)o3,
-                       H, W, C / vn, ldi, ld1, ld2, ld3);
+    launch_kernel((maxpool5_chain3_kernel<half_t>), grid, block, smem, s, (const half_t*)in, (half_t*)o1, (half_t*)o2, (half_t*)o3,
+                       H, W, C / vn, ldi, ld1, ld2, ld3, (int)units);
   else
-    launch_kernel((maxpool5_chain3_kernel<float>), grid, dim3(256), smem, s, (const float*)in, (float*)o1, (float*)o2, (float*)o3, H, W,
-                       C / vn, ldi, ld1, ld2, ld3);
+    launch_kernel((maxpool5_chain3_kernel<float>), grid, block, smem, s, (const float*)in, (float*)o1, (float*)o2, (float*)o3, H, W,
+                       C / vn, ldi, ld1, ld2, ld3, (int)units);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 
