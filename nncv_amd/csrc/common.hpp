@@ -258,7 +258,7 @@ bool image_pairs_applicable(const ImagePairsArgs& a);
 void launch_image_pairs(const ImagePairsArgs& a, hipStream_t s);
 // Barrier-free implicit GEMM for fp32 layers and small fp16 layers (conv_direct.hip); `wins`: its modelled time against
 // that of the kernel which would run the layer otherwise.
-enum DirectRival : int { kRivalPatch = 0, kRivalPatchS2 = 1, kRivalIgemmFast = 2, kRivalIgemm = 3, kRivalShortK = 4, kRivalRing = 5 };
+enum DirectRival : int { kRivalPatch = 0, kRivalPatchS2 = 1, kRivalIgemmFast = 2, kRivalIgemm = 3, kRivalShortK = 4, kRivalRing = 5, kRivalNarrow = 6 };
 // whether it is the kernel for a layer of F filters over RS taps of Cp channels at any size (else its order of the filters is not kept)
 bool conv_direct_serves(int dt, int F, int RS, int Cp);
 bool conv_direct_applicable(const IgemmArgs& a, int in_dt, int out_dt);
@@ -269,6 +269,10 @@ size_t weight_flat_bytes(int dt, int F, int RS, int Cp);
 void launch_weight_flat_rows(const void* w, void* dst, int dt, int F, int K, hipStream_t s);
 void launch_weight_flat(const void* w_fcrs, void* dst, int dt, int F, int C, int RS, int Cp, hipStream_t s);
 // fp16 implicit GEMM through an LDS ring filled straight from memory (conv_ring.hip); us: its modelled time
+// (conv3x3_narrow.hip: 32 channels, filters in registers)
+bool conv3x3_narrow_applicable(const IgemmArgs& a, int in_dt, int out_dt);
+double conv3x3_narrow_us(const IgemmArgs& a);
+void launch_conv3x3_narrow(const IgemmArgs& a, hipStream_t s);
 bool conv_ring_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 double conv_ring_us(const IgemmArgs& a);
 bool conv_ring_beats_patch_s2(const IgemmArgs& a);

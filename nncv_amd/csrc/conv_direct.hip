@@ -610,6 +610,7 @@ bool conv_direct_wins(const IgemmArgs& a, int dt, DirectRival rival) {
   if ((rival == kRivalIgemmFast || rival == kRivalRing) && dt == kF16 && (long long)((a.F + 127) / 128) * (((long long)a.N * a.OH * a.OW + 127) / 128) >= 256) return false;
   double us = 0;
   if (!best_form(a, dt, &us)) return false;
+  if (rival == kRivalNarrow) return us < 0.97 * conv3x3_narrow_us(a);
   if (rival == kRivalRing) return us < 0.97 * conv_ring_us(a);
   // margins cover the fits' errors: the fp16 3x3 stride-1 kernels' times are the least well fitted
   const double margin = dt == kF32 ? (rival == kRivalPatch ? 1.0 : 0.97) : rival == kRivalPatch ? 0.85 : 0.9;

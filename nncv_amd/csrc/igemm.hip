@@ -282,6 +282,7 @@ bool igemm_takes_direct(const IgemmArgs& a_in, int in_dt, int out_dt) {
   if (conv_pairs_applicable(a, in_dt, out_dt)) rival = kRivalShortK;
   else if (conv_ring_applicable(a, in_dt, out_dt) && conv_ring_beats_patch_s2(a)) rival = kRivalRing;
   else if (conv3x3_stream_applicable(a, in_dt, out_dt) || conv3x3_patch_applicable(a, in_dt)) rival = a.stride_h == 1 ? kRivalPatch : kRivalPatchS2;
+  else if (conv3x3_narrow_applicable(a, in_dt, out_dt)) rival = kRivalNarrow;
   else if (conv_ring_applicable(a, in_dt, out_dt)) rival = kRivalRing;
   else if (igemm_fast_applicable(a, in_dt, out_dt)) rival = kRivalIgemmFast;
   return conv_direct_wins(a, in_dt, rival);
@@ -305,6 +306,10 @@ void launch_igemm(const IgemmArgs& a_in, int in_dt, int out_dt, hipStream_t s) {
   }
   if (conv_pairs_applicable(a, in_dt, out_dt)) {
     launch_conv_pairs(a, s);
+    return;
+  }
+  if (conv3x3_narrow_applicable(a, in_dt, out_dt)) {
+    launch_conv3x3_narrow(a, s);
     return;
   }
   if (conv3x3_stream_applicable(a, in_dt, out_dt) && launch_conv3x3_stream(a, s)) return;
