@@ -201,105 +201,132 @@ void launch_conv_pairs(const IgemmArgs& a, hipStream_t s) {
 // The image layer.  A workgroup makes 2*WV rows x 32 columns of the result: it reads the haloed rectangle of its image from
 // the channel planes (a dword is two pixels of a row; lanes walk a row's pairs), packs pairs of pixels into chunks on the
 // way into LDS, and a wave takes its operands for two rows from there, 32 consecutive chunks per read and half.
+// It walks a run of such tiles, as many workgroups as the CUs hold: filters, scale and shift are fetched once, and a tile's pixels
+// are on their way under the products and stores of the one before (a workgroup a tile: 53.5 us for 16x640x640, 39.7 now).
 // What bounds it: its bytes (16x640x640: 39 MB in, 105 out) and the SiLU of 52 million results (a quarter-rate exp and rcp
 // each).  Packing the image in a launch of its own wrote 52 MB that the convolution read again, every chunk nine times
-// through the vector caches: 23 + 56 us for YOLOv5s (F = 32), 52 now; 6.6 + 10.5 for MobileNetV3 (F = 16, 32x224x224), 10.2 now.
+// through the vector caches: 23 + 56 us for YOLOv5s (F = 32); 6.6 + 10.5 for MobileNetV3 (F = 16, 32x224x224), 10.2 now.
 // ---------------------------------------------------------------------------------------------
 template <int R, int S, int NI, int WV>
-__global__ __launch_bounds__(64 * WV) void image_pairs_kernel(const ImagePairsArgs a) {
+__global__ __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(NI == 1 && WV == 4 ? 4 : 2))) void image_pairs_kernel(const ImagePairsArgs a) {
   constexpr int KST = R * S / 2, TP = 64 * NI + 16, kRows = 2 * (2 * WV - 1) + R, kCols = 32 + S - 1, kPitch = kCols * 16;
   static_assert(R * S % 2 == 0, "an MFMA step takes two chunks");
-  constexpr int kLds = kRows * kPitch > WV * 64 * TP ? kRows * kPitch : WV * 64 * TP, kEach = (kRows * kCols + 64 * WV - 1) / (64 * WV);
-  __shared__ __align__(16) unsigned char smem[kLds];  // the packed rectangle, then the waves' outgoing tiles
+  constexpr int kEach = (kRows * kCols + 64 * WV - 1) / (64 * WV);
+  __shared__ __align__(16) unsigned char smem[kRows * kPitch];  // the packed rectangle
+  __shared__ __align__(16) unsigned char outgoing[WV * 64 * TP];
+  __shared__ __align__(16) float ss[64 * NI];  // scale, shift
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lrow = lane & 31, lh = lane >> 5;
   // XCD x takes a run of tiles: neighbours share halo lines in its L2
-  const int tiles = a.N * a.tiles_y * a.tiles_x, t = (blockIdx.x & 7) * ((tiles + 7) >> 3) + (blockIdx.x >> 3);
-  if (t >= tiles) return;  // (uniform; before any barrier)
-  int tx, ty;
-  const int rowt = fast_div(t, a.tiles_x, a.inv_tx, &tx), n = fast_div(rowt, a.tiles_y, a.inv_ty, &ty);
-  const int oy0 = __builtin_amdgcn_readfirstlane(ty * 2 * WV), ox0 = __builtin_amdgcn_readfirstlane(tx * 32), img = __builtin_amdgcn_readfirstlane(n);
+  const int tiles = a.N * a.tiles_y * a.tiles_x, per = (tiles + 7) >> 3, from = (blockIdx.x & 7) * per, end = from + per < tiles ? from + per : tiles;
+  int t = from + (blockIdx.x >> 3);
+  if (t >= end) return;  // (uniform; before any barrier)
   const __amdgpu_buffer_rsrc_t rs_in = make_rsrc(a.in, a.in_bytes), rs_wt = make_rsrc(a.wt, a.wt_bytes);
 
   unsigned d[kEach][4];
   const unsigned plane = (unsigned)(a.H * a.W) * 2u;
+  int oy0, ox0, img;  // of the tile that d is for
+  auto request = [&](int tile) __attribute__((always_inline)) {
+    int tx, ty;
+    const int rowt = fast_div(tile, a.tiles_x, a.inv_tx, &tx), n = fast_div(rowt, a.tiles_y, a.inv_ty, &ty);
+    oy0 = __builtin_amdgcn_readfirstlane(ty * 2 * WV), ox0 = __builtin_amdgcn_readfirstlane(tx * 32), img = __builtin_amdgcn_readfirstlane(n);
 #pragma unroll
-  for (int i = 0; i < kEach; ++i) {
-    const int e = i * 64 * WV + tid, row = e / kCols, col = e - row * kCols, iy = 2 * oy0 - a.pad_h + row, ip = ox0 - a.pad_w + col;
-    const bool ok = (e < kRows * kCols) & ((unsigned)iy < (unsigned)a.H) & ((unsigned)ip < (unsigned)(a.W >> 1));
-    const unsigned off = ok ? (unsigned)(iy * a.W + 2 * ip) * 2u : kOOBc;
+    for (int i = 0; i < kEach; ++i) {
+      const int e = i * 64 * WV + tid, row = e / kCols, col = e - row * kCols, iy = 2 * oy0 - a.pad_h + row, ip = ox0 - a.pad_w + col;
+      const bool ok = (e < kRows * kCols) & ((unsigned)iy < (unsigned)a.H) & ((unsigned)ip < (unsigned)(a.W >> 1));
+      const unsigned off = ok ? (unsigned)(iy * a.W + 2 * ip) * 2u : kOOBc;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) d[i][c] = c < a.C ? __builtin_amdgcn_raw_buffer_load_b32(rs_in, off, (unsigned)(img * a.C + c) * plane, 0) : 0u;
+      for (int c = 0; c < 3; ++c) d[i][c] = __builtin_amdgcn_raw_buffer_load_b32(rs_in, c < a.C ? off : kOOBc, (unsigned)(img * a.C + c) * plane, 0);
+      d[i][3] = 0;
+      if (a.C == 4) d[i][3] = __builtin_amdgcn_raw_buffer_load_b32(rs_in, off, (unsigned)(img * 4 + 3) * plane, 0);
+    }
+  };
+  request(t);
+  for (int f = tid; f < 32 * NI; f += 64 * WV) {
+    ss[f] = a.scale && f < a.F ? a.scale[f] : 1.0f;
+    ss[32 * NI + f] = a.shift && f < a.F ? a.shift[f] : 0.0f;
   }
   u32x4 w[KST][NI];
 #pragma unroll
   for (int kk = 0; kk < KST; ++kk)
 #pragma unroll
     for (int i = 0; i < NI; ++i) w[kk][i] = __builtin_amdgcn_raw_buffer_load_b128(rs_wt, (unsigned)(((i * 32 + lrow) * R * S + 2 * kk + lh) * 16), 0, 0);
+  // all of it now: waited for where it is used, in the loop, every trip would wait for the next tile's pixels too
+  __builtin_amdgcn_s_waitcnt(0x0f70);
+  for (;;) {
 #pragma unroll
-  for (int i = 0; i < kEach; ++i) {
-    const int e = i * 64 * WV + tid;
-    if (e < kRows * kCols)
-      *reinterpret_cast<u32x4*>(smem + e * 16) = u32x4{(d[i][0] & 0xffffu) | (d[i][1] << 16), (d[i][2] & 0xffffu) | (d[i][3] << 16),
-                                                      (d[i][0] >> 16) | (d[i][1] & 0xffff0000u), (d[i][2] >> 16) | (d[i][3] & 0xffff0000u)};
-  }
-  __syncthreads();
-
-  floatx16 acc[NI][2];
-#pragma unroll
-  for (int i = 0; i < NI; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-  // chunks 2 kk and 2 kk + 1 of the window: neighbours of a row, or the last of one and the first of the next
-  const unsigned char* base = smem + 4 * wave * kPitch + lrow * 16;
-  const unsigned char *next = base + lh * 16, *wrap = base + lh * (kPitch - (S - 1) * 16);
-#pragma unroll
-  for (int kk = 0; kk < KST; ++kk) {
-    const int r = 2 * kk / S, c = 2 * kk - r * S;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const u32x4 b = *reinterpret_cast<const u32x4*>((c == S - 1 ? wrap : next) + (2 * j + r) * kPitch + c * 16);
-#pragma unroll
-      for (int i = 0; i < NI; ++i) Mma<half_t>::run(w[kk][i], b, acc[i][j]);
+    for (int i = 0; i < kEach; ++i) {
+      const int e = i * 64 * WV + tid;
+      if (e < kRows * kCols)
+        *reinterpret_cast<u32x4*>(smem + e * 16) = u32x4{(d[i][0] & 0xffffu) | (d[i][1] << 16), (d[i][2] & 0xffffu) | (d[i][3] << 16),
+                                                        (d[i][0] >> 16) | (d[i][1] & 0xffff0000u), (d[i][2] >> 16) | (d[i][3] & 0xffff0000u)};
     }
-  }
-  __syncthreads();
+    __syncthreads();
+    // the next tile's pixels are on their way under this one's products, activation and stores
+    const int row0 = oy0 + 2 * wave, col0 = ox0, at = img;
+    t += gridDim.x >> 3;
+    const bool more = t < end;
+    if (more) request(t);
 
-  unsigned char* tile = smem + wave * (64 * TP);
+    floatx16 acc[NI][2];
 #pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    floatx4 sc[4], sh[4];
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int f = i * 32 + 8 * q + 4 * lh;
-      sc[q] = a.scale && f < a.F ? *reinterpret_cast<const floatx4*>(a.scale + f) : floatx4{1.f, 1.f, 1.f, 1.f};
-      sh[q] = a.shift && f < a.F ? *reinterpret_cast<const floatx4*>(a.shift + f) : floatx4{0.f, 0.f, 0.f, 0.f};
-    }
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      float y[16];
+        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+    // chunks 2 kk and 2 kk + 1 of the window: neighbours of a row, or the last of one and the first of the next
+    const unsigned char* base = smem + 4 * wave * kPitch + lrow * 16;
+    const unsigned char *next = base + lh * 16, *wrap = base + lh * (kPitch - (S - 1) * 16);
 #pragma unroll
-      for (int e = 0; e < 16; ++e) y[e] = acc[i][j][e] * sc[e >> 2][e & 3] + sh[e >> 2][e & 3];
-      act_apply_n<true>(y, a.act);
+    for (int kk = 0; kk < KST; ++kk) {
+      const int r = 2 * kk / S, c = 2 * kk - r * S;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        half4 h;
+      for (int j = 0; j < 2; ++j) {
+        const u32x4 b = *reinterpret_cast<const u32x4*>((c == S - 1 ? wrap : next) + (2 * j + r) * kPitch + c * 16);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) h[e] = (half_t)y[4 * q + e];
-        *reinterpret_cast<half4*>(tile + (j * 32 + lrow) * TP + (i * 32 + 8 * q + 4 * lh) * 2) = h;
+        for (int i = 0; i < NI; ++i) Mma<half_t>::run(w[kk][i], b, acc[i][j]);
       }
     }
-  }
-  // whole pixel rows out: 4*NI lanes cover the 32*NI channels of one pixel (a wave's own tile: no barrier)
-  constexpr int LPR = 4 * NI, RPI = 64 / LPR;
-  const int fc = (lane % LPR) * 8;
-  half_t* out = static_cast<half_t*>(a.out);
+    __syncthreads();  // the rectangle has been read
+
+    unsigned char* tile = outgoing + wave * (64 * TP);
 #pragma unroll
-  for (int it = 0; it < 64 / RPI; ++it) {
-    const int row = it * RPI + lane / LPR, oy = oy0 + 2 * wave + (row >> 5), ox = ox0 + (row & 31);
-    const u32x4 v = *reinterpret_cast<const u32x4*>(tile + row * TP + fc * 2);
-    if (oy < a.OH && ox < a.OW && fc < a.F) *reinterpret_cast<u32x4*>(out + ((long long)(img * a.OH + oy) * a.OW + ox) * a.ldo + fc) = v;
+    for (int i = 0; i < NI; ++i) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        asm volatile("" ::: "memory");  // (scale and shift are read again for every block: registers)
+        float y[16];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const floatx4 m = *reinterpret_cast<const floatx4*>(ss + i * 32 + 8 * q + 4 * lh), h = *reinterpret_cast<const floatx4*>(ss + 32 * NI + i * 32 + 8 * q + 4 * lh);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) y[4 * q + e] = acc[i][j][4 * q + e] * m[e] + h[e];
+        }
+        act_apply_n<true>(y, a.act);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          half4 h;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) h[e] = (half_t)y[4 * q + e];
+          *reinterpret_cast<half4*>(tile + (j * 32 + lrow) * TP + (i * 32 + 8 * q + 4 * lh) * 2) = h;
+        }
+      }
+    }
+    // whole pixel rows out: 4*NI lanes cover the 32*NI channels of one pixel (a wave's own tile: no barrier)
+    constexpr int LPR = 4 * NI, RPI = 64 / LPR;
+    const int fc = (lane % LPR) * 8;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {  // (a row's own descriptor: the tensor may be larger than a buffer)
+      const __amdgpu_buffer_rsrc_t rs_out = make_rsrc(static_cast<half_t*>(a.out) + ((long long)(at * a.OH + row0 + j) * a.OW + col0) * a.ldo, kOOBc);
+#pragma unroll
+      for (int it = 0; it < 32 / RPI; ++it) {
+        const int px = it * RPI + lane / LPR;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(tile + (j * 32 + px) * TP + fc * 2);
+        const bool ok = (row0 + j < a.OH) & (col0 + px < a.OW) & (fc < a.F);
+        __builtin_amdgcn_raw_buffer_store_b128(v, rs_out, ok ? (unsigned)(px * a.ldo + fc) * 2u : kOOBc, 0, 0);
+      }
+    }
+    if (!more) break;
   }
 }
 
@@ -322,7 +349,9 @@ static void launch_image_cfg(ImagePairsArgs a, const char* tag, hipStream_t s) {
   a.wt_bytes = (unsigned)(a.F * a.R * a.S * 16);
   const double px = (double)a.N * a.OH * a.OW;
   ProfScope prof(tag, a.alg_flops, 2.0 * ((double)a.N * a.C * a.H * a.W + (double)a.F * a.R * a.S * 8 + px * a.F), s);
-  const dim3 grid((unsigned)((a.N * a.tiles_y * a.tiles_x + 7) / 8 * 8));
+  // as many workgroups as the CUs hold at most, each with a run of tiles (fewer than 1024 of the small ones)
+  const int tiles = a.N * a.tiles_y * a.tiles_x;
+  const dim3 grid((unsigned)(tiles < 1024 ? (tiles + 7) / 8 * 8 : 1024));
   if (small) launch_kernel((image_pairs_kernel<R, S, NI, 1>), grid, dim3(64), 0, s, a);
   else launch_kernel((image_pairs_kernel<R, S, NI, 4>), grid, dim3(256), 0, s, a);
   NNCV_HIP_CHECK(hipGetLastError());
