@@ -7,12 +7,15 @@
 //  * Both are split in registers, 7 vector instructions for two values: 112 of them feed the 24 products (768 clocks) of a
 //    64 x 64 tile and 16 k, and run under the products of the SIMD's other wave.
 //  * Nothing asks for alignment beyond 4 bytes.  Only the last round of the matrix can hold k >= K or leave the buffers; the
-//    group that owns it walks it first, with A masked (B's rows past the end come back as zeros from the range check).
-//    Rows m >= M read row M - 1 and columns n >= N read the next row: both only reach results that are not stored.
+//    group that owns it walks it first, with A masked (B's rows past the end come back as zeros from the range check,
+//    gemm_split_walk.hpp).
+//    Rows m >= M read row M - 1 and columns n >= N the tile's first one: both only reach results that are not stored.
 //  * KG "K groups": waves of a workgroup that share a tile of C and take every KG-th round.  Their sums meet in LDS, in a
 //    fixed order.
 #include <cmath>
+#include <type_traits>
 
+#include "gemm_split_walk.hpp"
 #include "split.hpp"
 
 namespace nncv_hip {
@@ -61,7 +64,7 @@ __global__ __launch_bounds__(64 * KG, TM * TN == 4 ? 2 : TM * TN == 2 ? 3 : 4) v
   unsigned aoff[kA];
 #pragma unroll
   for (int i = 0; i < kA; ++i) aoff[i] = ((unsigned)min((lane >> 3) + 8 * i, M - 1 - m0) * (unsigned)K + 4u * (lane & 7)) * 4u;
-  const unsigned boff = (8u * lh * (unsigned)N + (unsigned)(TN * lrow)) * 4u, brow = (unsigned)N * 4u;
+  const unsigned boff = split_b_lane(lane, TN, n0, N);
   floatx4 ra[kA];
   float rb[2][8][TN];
   // (rounds below the first read nothing: descriptors of no bytes)
@@ -72,16 +75,16 @@ __global__ __launch_bounds__(64 * KG, TM * TN == 4 ? 2 : TM * TN == 2 ? 3 : 4) v
 #pragma unroll
     for (int i = 0; i < kA; ++i) ra[i] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs, aoff[i], 0, 0));
   };
-  auto load_b = [&](int r, int k) {
-    const long long at = (32ll * r + 16 * k) * N + n0;
-    const bool in = 32 * r + 16 * k < K;
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc(B + at, in ? left((long long)K * N, at, r) : 0u);
+  auto load_b = [&](int r, int k, auto last) {
+    const SplitBRows rows = split_b_rows(r, k, n0, N, K);
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(B + rows.first, rows.bytes);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
+      const unsigned vo = split_b_vector(boff, e, N, last), so = split_b_scalar(e, N, last);
       if constexpr (TN == 1) {
-        rb[k][e][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, boff, (int)(e * brow), 0));
+        rb[k][e][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, vo, so, 0));
       } else {
-        const floatx2 v = __builtin_bit_cast(floatx2, __builtin_amdgcn_raw_buffer_load_b64(rs, boff, (int)(e * brow), 0));
+        const floatx2 v = __builtin_bit_cast(floatx2, __builtin_amdgcn_raw_buffer_load_b64(rs, vo, so, 0));
         rb[k][e][0] = v[0];
         rb[k][e][1] = v[1];
       }
@@ -114,8 +117,8 @@ __global__ __launch_bounds__(64 * KG, TM * TN == 4 ? 2 : TM * TN == 2 ? 3 : 4) v
   const int nk = (K + 31) >> 5;
   int r = nk - 1 - grp;  // this group's rounds, from the last one down
   load_a(r);
-  load_b(r, 0);
-  load_b(r, 1);
+  load_b(r, 0, std::true_type());
+  load_b(r, 1, std::true_type());
   constexpr bool kEarly = KG > 1 && TM * TN < 4;  // (the 64 x 64 forms have no registers to spare)
   vec cpre[kEarly ? kMine : 1];
   if constexpr (kEarly) {
@@ -151,7 +154,7 @@ __global__ __launch_bounds__(64 * KG, TM * TN == 4 ? 2 : TM * TN == 2 ? 3 : 4) v
 #pragma unroll
         for (int c = 0; c < 3; ++c) b[j][c] = u32x4{p[0][c], p[1][c], p[2][c], p[3][c]};
       }
-      load_b(r - KG, k);
+      load_b(r - KG, k, std::false_type());
       split_products(a, b, big, low);
     }
   }
