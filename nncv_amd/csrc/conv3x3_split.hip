@@ -11,7 +11,7 @@
 //  * Eight waves, or four where two workgroups share a CU (launch_ws1).  A wave's share of the tile is 64 slots x 32 filters (WS = 1,
 //    NI = 1: 32 x 32), its K groups take a 16-channel half of a slab each, four of them the even or the odd taps of a half; their
 //    sums meet in LDS.
-//  * A sum that is not finite is done again in plain fp32.
+//  * A wave with a sum that is not finite takes its sums again with the fp32 instructions, from memory (split.hpp).
 //  * What bounds it: the matrix pipes where tiles fill the CUs (six products, 2.7 times the fp32 instructions' rate), a slab's
 //    barrier and the LDS reads behind it where they do not: two waves a SIMD cover each other there (six 224x224 images classified by an
 //    fp32 ResNet-18: 373 us with one, 353 with two).
@@ -37,21 +37,6 @@ struct SplitCfg {
   static constexpr int buffers = WS == 4 ? 1 : 2;                     // (256 slots: layers of one slab)
   static constexpr int patch = cap * kCell, dump = buffers * patch, scale = dump + 640, smem = scale + 512;
 };
-
-// one sum in plain fp32
-__device__ __forceinline__ float plain_sum(const PatchArgs& a, int p, int f) {
-  const int HW = a.H * a.W, n = p / HW, oy = (p - n * HW) / a.W, ox = p - n * HW - oy * a.W;
-  const float* in = static_cast<const float*>(a.in);
-  const float* wt = static_cast<const float*>(a.wt) + (long long)f * 9 * a.C;
-  float sum = 0.0f;
-  for (int t = 0; t < 9; ++t) {
-    const int iy = oy + t / 3 - 1, ix = ox + t % 3 - 1;
-    if ((unsigned)iy >= (unsigned)a.H || (unsigned)ix >= (unsigned)a.W) continue;
-    const float* row = in + (long long)((n * a.H + iy) * a.W + ix) * a.pix;
-    for (int c = 0; c < a.C; ++c) sum = __builtin_fmaf(row[c], wt[t * a.C + c], sum);
-  }
-  return sum;
-}
 
 template <int WS, int NI, int KG>  // KG: K groups, waves that share a tile's sums
 __global__ __launch_bounds__(64 * KG * split_units(WS)) __attribute__((amdgpu_waves_per_eu(2, 2))) void conv3x3_split_kernel(
@@ -255,13 +240,39 @@ __global__ __launch_bounds__(64 * KG * split_units(WS)) __attribute__((amdgpu_wa
     else walk(std::integral_constant<int, 1>());
   }
 
+  if (__builtin_expect(split_sums(big, low), 0)) {
+    // a slab of this wave: 16 channels, or both halves with one K group, of its taps; two steps of eight channels each
+    const int taps = KG == 4 ? 5 - (kg >> 1) : 9, per = KG == 1 ? 2 * taps : taps, HW = a.H * a.W;
+    int py[JN], px[JN], img[JN];
+#pragma unroll
+    for (int j = 0; j < JN; ++j) {
+      const int p = max(obase[j], 0) / a.ldo, n = p / HW, rem = p - n * HW, y = rem / a.W;
+      img[j] = n * HW;
+      py[j] = obase[j] >= 0 ? y : -(1 << 20);
+      px[j] = rem - y * a.W;
+    }
+    const __amdgpu_buffer_rsrc_t rs_wt = make_rsrc(a.wt, (unsigned)a.F * 9u * (unsigned)a.C * 4u);
+    plain_products(big, 2 * per * nslab, [&](int step, u32x4 (&f)[1], u32x4 (&x)[JN]) {
+      const int t = step >> 1, slab = t / per, st = t - slab * per;
+      const int tap = KG == 1 ? st >> 1 : KG == 2 ? st : 2 * st + (kg >> 1), half16 = KG == 1 ? st & 1 : kg & 1;
+      const int c = slab * 32 + half16 * 16 + (step & 1) * 8 + 4 * lh, dy = tap / 3 - 1, dx = tap - tap / 3 * 3 - 1;
+      const bool in = slab < nslab;
+      f[0] = __builtin_amdgcn_raw_buffer_load_b128(rs_wt, in ? (unsigned)((min(f0 + lrow, a.F - 1) * 9 + tap) * a.C + c) * 4u : kOOBp, 0, 0);
+#pragma unroll
+      for (int j = 0; j < JN; ++j) {
+        const bool ok = in & ((unsigned)(py[j] + dy) < (unsigned)a.H) & ((unsigned)(px[j] + dx) < (unsigned)a.W);
+        x[j] = __builtin_amdgcn_raw_buffer_load_b128(rs_in, ok ? (unsigned)((img[j] + (py[j] + dy) * a.W + px[j] + dx) * a.pix + c) * 4u : kOOBp, 0, 0);
+      }
+    });
+  }
+
   // ---- out: quad (j, g): filters 8 g + 4 lh .. + 3 of slot block j.  K group g finishes quads g, g + KG ... ----
   constexpr int kMine = kQuads / KG;
   auto sum_of = [&](int q) {
     const int j = q / 4, g = q & 3;
     floatx4 s;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) s[e] = big[0][j][4 * g + e] + low[0][j][4 * g + e];
+    for (int e = 0; e < 4; ++e) s[e] = big[0][j][4 * g + e];
     return s;
   };
   const float* res = static_cast<const float*>(a.residual);
@@ -308,25 +319,12 @@ __global__ __launch_bounds__(64 * KG * split_units(WS)) __attribute__((amdgpu_wa
     }
     *reinterpret_cast<floatx4*>(out + at) = y;
   };
-  unsigned again = 0;
 #pragma unroll
   for (int m = 0; m < kMine; ++m) {
     const int q = KG * m + kg;
     int f;
     const long long at = at_of(q, &f);
-    if (at < 0) continue;
-    if (split_finite(sums[m])) put(q, at, sums[m], rv[m]);
-    else again |= 1u << q;
-  }
-  for (; again; again &= again - 1) {
-    const int q = __builtin_ctz(again);
-    int f;
-    const long long at = at_of(q, &f);
-    const int o = (int)(at - f);
-    floatx4 s;
-#pragma unroll 1
-    for (int e = 0; e < 4; ++e) s[e] = plain_sum(a, o / a.ldo, f + e);
-    put(q, at, s, res ? *reinterpret_cast<const floatx4*>(res + at) : floatx4{});
+    if (at >= 0) put(q, at, sums[m], rv[m]);
   }
 }
 

@@ -79,27 +79,6 @@ struct DirectArgs {
   float inv_ohw, inv_ow, inv_s, inv_cpt, inv_tiles;
 };
 
-// One sum in plain fp32, from the filters in their flat order: channel c of a tap is float c % 4 of chunk c / 4 of that tap.
-__device__ __forceinline__ float plain_sum(const DirectArgs& a, int p, int f, bool aux) {
-  int rem, ox;
-  const int n = fast_div(p, a.OHW, a.inv_ohw, &rem), oy = fast_div(rem, a.OW, a.inv_ow, &ox);
-  const int taps = aux ? 1 : a.chunks / a.cpt, rounds = ((aux ? a.cpt : a.chunks) + 7) >> 3;
-  const floatx4* wt = static_cast<const floatx4*>(aux ? a.aux_wt : a.wt) + (long long)(f >> 5) * rounds * 4 * 64 + (f & 31);
-  float sum = 0.0f;
-  for (int t = 0; t < taps; ++t) {
-    const int tap = aux ? a.aux_tap : t, r = tap / a.S, s = tap - r * a.S, iy = oy * a.stride_h - a.pad_h + r, ix = ox * a.stride_w - a.pad_w + s;
-    if ((unsigned)iy >= (unsigned)a.H || (unsigned)ix >= (unsigned)a.W) continue;
-    const floatx4* row = reinterpret_cast<const floatx4*>(static_cast<const float*>(a.in) + (long long)((n * a.H + iy) * a.W + ix) * a.pix);
-    for (int c = 0; c < a.cpt; ++c) {
-      const int k = t * a.cpt + c;
-      const floatx4 x = row[c], w = wt[(k >> 1) * 64 + (k & 1) * 32];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sum = __builtin_fmaf(x[e], w[e], sum);
-    }
-  }
-  return sum;
-}
-
 // UNI: a tap is a whole number of rounds (C elements = whole 128-byte lines), so the tap of a round is the same for all lanes
 template <typename T, typename OutT, int BT, int TM, int TN, int KG, bool UNI, int D>
 __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a) {
@@ -226,7 +205,7 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
   };
 
   // (split: the small products in sums of their own)
-    typename Block<T, BT>::acc acc[TM][TN], low[kSplit ? TM : 1][kSplit ? TN : 1];
+  typename Block<T, BT>::acc acc[TM][TN], low[kSplit ? TM : 1][kSplit ? TN : 1];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -287,12 +266,8 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
     for (int e = 0; e < 4; ++e) o[e] = (OutT)y[e];
     *reinterpret_cast<out4*>(out + q.at) = o;
   };
-  // Sums that are not finite (an operand that bf16 does not hold, or a result that is not) are marked, and done again at the end
-  unsigned again = 0;
-  auto finish = [&](int k, const Quad& q, const floatx4& sum) {
-    if (q.at < 0) return;
-    if (kSplit && !split_finite(sum)) again |= 1u << k;
-    else put(q, sum);
+  auto finish = [&](const Quad& q, const floatx4& sum) {
+    if (q.at >= 0) put(q, sum);
   };
   Quad mine[KG > 1 ? kMine : 1];
   if constexpr (KG > 1) {
@@ -334,10 +309,21 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
         split_products(wp, xp, acc, low);
       }
     }
+    if (__builtin_expect(split_sums(acc, low), 0)) {  // once more with the fp32 instructions: a step is a unit of the weights, two chunks
+      int rem, ox;
+      const int n = fast_div(min(p0 + lrow, a.P - 1), a.OHW, a.inv_ohw, &rem), oy = fast_div(rem, a.OW, a.inv_ow, &ox);
+      const int iy = oy * a.stride_h - a.pad_h, ix = ox * a.stride_w - a.pad_w;
+      plain_products(acc, 4 * ((r_n - grp + KG - 1) / KG), [&](int step, u32x4 (&f)[TM], u32x4 (&p)[TN]) {
+        const int r = rb + (step >> 2) * KG, unit = 4 * (r - r_lo) + (step & 3), kc = 8 * r + 2 * (step & 3) + lh;
+        int c, s;
+        const int tap = fast_div(kc, a.cpt, a.inv_cpt, &c), row = fast_div(tap, a.S, a.inv_s, &s);
+        const bool ok = (r < re) & (kc < a.chunks) & ((unsigned)(iy + row) < (unsigned)a.H) & ((unsigned)(ix + s) < (unsigned)a.W);
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] += low[i][j];
+        for (int i = 0; i < TM; ++i)
+          f[i] = __builtin_amdgcn_raw_buffer_load_b128(rs_wt, ((f0 + BT * i < f_end) & (r < re)) ? woff[i] + (unsigned)unit * 1024u : kOOBd, 0, 0);
+        p[0] = __builtin_amdgcn_raw_buffer_load_b128(rs_in, ok ? (unsigned)((((n * a.H + iy + row) * a.W + ix + s) * a.pix) * 4 + c * 16) : kOOBd, 0, 0);
+      });
+    }
   } else {
     for (int r = rb; r < re; r += D * KG, buf ^= D & 1) {
 #pragma unroll
@@ -376,7 +362,7 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
   };
   if constexpr (KG == 1) {
 #pragma unroll
-    for (int k = 0; k < kQuads; ++k) finish(k, quad_of(k), quad_sum(k));
+    for (int k = 0; k < kQuads; ++k) finish(quad_of(k), quad_sum(k));
   } else {
     floatx4* part = reinterpret_cast<floatx4*>(lds);  // this wave's own region: [quad][lane]
 #pragma unroll
@@ -393,18 +379,7 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
       for (int d = 1; d < KG; d *= 2)  // pairwise: a chain of log2(KG) additions
 #pragma unroll
         for (int g = 0; g + d < KG; g += 2 * d) v[g] += v[g + d];
-      finish(k, mine[k], v[0]);
-    }
-  }
-  if constexpr (kSplit) {
-    for (; again; again &= again - 1) {
-      const int k = __builtin_ctz(again);
-      const Quad q = quad_of(KG > 1 ? grp + k * KG : k);
-      const int p = (int)(q.at / ldo), f = (int)(q.at - (long long)p * ldo);
-      floatx4 sum;
-#pragma unroll 1
-      for (int e = 0; e < 4; ++e) sum[e] = plain_sum(a, p, f + e, aux);
-      put(q, sum);
+      finish(mine[k], v[0]);
     }
   }
 }

@@ -31,14 +31,6 @@ struct SplitCfg {
   static constexpr int kWave = kStage > kPart ? kStage : kPart, kLds = KG * kWave;
 };
 
-// one element in plain fp32
-__device__ __attribute__((noinline)) float plain_dot(const float* a, const float* b, int K, int N) {
-  float s = 0.0f;
-#pragma unroll 8
-  for (int k = 0; k < K; ++k) s = __builtin_fmaf(a[k], b[(long long)k * N], s);
-  return s;
-}
-
 template <int TM, int TN, int KG>
 __global__ __launch_bounds__(64 * KG, TM * TN == 4 ? 2 : TM * TN == 2 ? 3 : 4) void gemm_split_kernel(const float* __restrict__ A, const float* __restrict__ B, const float* C, float* D, int M,
                                                                int N, int K, int tiles_m, int tiles_n) {
@@ -158,14 +150,43 @@ __global__ __launch_bounds__(64 * KG, TM * TN == 4 ? 2 : TM * TN == 2 ? 3 : 4) v
       split_products(a, b, big, low);
     }
   }
+  if (__builtin_expect(split_sums(big, low), 0)) {  // once more with the fp32 instructions: eight k a step, four steps a round
+    int at_lane = lane;  // (worked out here: what is known before the loop is kept over it, in registers that it needs)
+    asm volatile("" : "+v"(at_lane));
+    const int lrow = at_lane & 31, lh = at_lane >> 5;
+    plain_products(big, 4 * ((nk - grp + KG - 1) / KG), [&](int s, u32x4 (&a)[TM], u32x4 (&b)[TN]) {
+      const int round = nk - 1 - grp - (s >> 2) * KG, k0 = 32 * round + 8 * (s & 3);
+      const long long at = (long long)m0 * K + k0, rows = (long long)k0 * N + n0;
+      const __amdgpu_buffer_rsrc_t rs_a = make_rsrc(A + at, k0 < K ? left((long long)M * K, at, round) : 0u);
+      const __amdgpu_buffer_rsrc_t rs_b = make_rsrc(B + rows, k0 < K ? left((long long)K * N, rows, round) : 0u);
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const floatx4 v = __builtin_bit_cast(
+            floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs_a, ((unsigned)min(32 * i + lrow, M - 1 - m0) * (unsigned)K + 4u * lh) * 4u, 0, 0));
+        floatx4 in;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) in[e] = k0 + 4 * lh + e < K ? v[e] : 0.0f;
+        a[i] = __builtin_bit_cast(u32x4, in);
+      }
+      const unsigned col = n0 + TN * lrow < N ? (unsigned)(TN * lrow) : 0u;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const unsigned vo = ((4u * lh + e) * (unsigned)N + col) * 4u;
+        if constexpr (TN == 1) {
+          b[0][e] = __builtin_amdgcn_raw_buffer_load_b32(rs_b, vo, 0, 0);
+        } else {
+          const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs_b, vo, 0, 0));
+          b[0][e] = v[0];
+          b[1][e] = v[1];
+        }
+      }
+    });
+  }
 
   // ---- D = C + sums ----
   auto emit = [&](int unit, const vec& c, vec sum) {
     const int m = row_of(unit), n = n0 + TN * lrow;
     if (m >= M || n >= N) return;
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-      if (n + j < N && !(__builtin_fabsf(sum[j]) < __builtin_inff())) sum[j] = plain_dot(A + (long long)m * K, B + n + j, K, N);
     sum += c;
     float* d = D + ((long long)m * N + n);
     if (TN == 1 || n + 1 < N) __builtin_memcpy(d, &sum, sizeof(sum));
@@ -176,7 +197,7 @@ __global__ __launch_bounds__(64 * KG, TM * TN == 4 ? 2 : TM * TN == 2 ? 3 : 4) v
     for (int u = 0; u < kUnits; ++u) {
       vec y;
 #pragma unroll
-      for (int j = 0; j < TN; ++j) y[j] = big[u >> 4][j][u & 15] + low[u >> 4][j][u & 15];
+      for (int j = 0; j < TN; ++j) y[j] = big[u >> 4][j][u & 15];
       emit(u, fetch(u), y);
     }
   } else {
@@ -186,7 +207,7 @@ __global__ __launch_bounds__(64 * KG, TM * TN == 4 ? 2 : TM * TN == 2 ? 3 : 4) v
     for (int u = 0; u < kUnits; ++u) {
       vec y;
 #pragma unroll
-      for (int j = 0; j < TN; ++j) y[j] = big[u >> 4][j][u & 15] + low[u >> 4][j][u & 15];
+      for (int j = 0; j < TN; ++j) y[j] = big[u >> 4][j][u & 15];
       mine[u * 64] = y;
     }
     __syncthreads();

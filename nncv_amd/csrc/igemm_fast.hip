@@ -240,41 +240,32 @@ __global__ __launch_bounds__(64 * WP * WF * WK, kSplit ? 2 : 1) void igemm_fast_
   const int fo = aux ? a.aux_f0 : 0;                     // first filter of this output tensor
   const int fend = (aux || a.aux_f0 == 0) ? a.F : a.aux_f0;  // one past its last filter
   if constexpr (kSplit) {
-    // Sums that are not finite (an operand that bf16 does not hold, or a result that is not) are done again in plain fp32
-    unsigned long long again = 0;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
+    if (__builtin_expect(split_sums(acc, low), 0)) {  // once more with the fp32 instructions: half a K step at a time, two chunks
+      int iy[2], ix[2], img[2];
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        acc[i][j] += low[i][j];
-#pragma unroll
-        for (int v = 0; v < 16; ++v) again |= __builtin_fabsf(acc[i][j][v]) < __builtin_inff() ? 0ull : 1ull << ((i * 2 + j) * 16 + v);
-      }
-    auto mend = [&](unsigned char* tile) {
-      for (; again; again &= again - 1) {
-        const int k = __builtin_ctzll(again), i = k >> 5, j = k >> 4 & 1, v = k & 15;
-        const int slot = j * 32 + lrow, chan = i * 32 + 8 * (v >> 2) + 4 * lchunk + (v & 3);
-        const int f = by * BFE + wf * 64 + chan, gp = bx * BP + wp * 64 + slot;
-        if (f >= a.F || gp >= P) continue;
         int rem, ox;
-        const int n = fast_div(gp, a.OH * a.OW, inv_ohow, &rem), oy = fast_div(rem, a.OW, inv_ow, &ox);
-        float sum = 0.0f;
-        for (int t = aux ? a.aux_tap : 0; t < (aux ? a.aux_tap + 1 : a.R * a.S); ++t) {
-          const int iy = oy * a.stride_h - a.pad_h + t / a.S, ix = ox * a.stride_w - a.pad_w + t % a.S;
-          if ((unsigned)iy >= (unsigned)a.H || (unsigned)ix >= (unsigned)a.W) continue;
-          const float* x = static_cast<const float*>(a.in) + (long long)bz * a.in_bs + (long long)((n * a.H + iy) * a.W + ix) * pix;
-          const float* y = static_cast<const float*>(a.wt) + (long long)bz * a.wt_bs + ((long long)f * a.R * a.S + t) * a.C;
-          for (int c = 0; c < a.C; ++c) sum = __builtin_fmaf(x[c], y[c], sum);
-        }
-        *reinterpret_cast<float*>(tile + slot * kTilePitch + chan * 4) = sum;
+        const int gp = bx * BP + wp * 64 + j * 32 + lrow, n = fast_div(min(gp, P - 1), a.OH * a.OW, inv_ohow, &rem), oy = fast_div(rem, a.OW, inv_ow, &ox);
+        iy[j] = oy * a.stride_h - a.pad_h;
+        ix[j] = ox * a.stride_w - a.pad_w;
+        img[j] = n * a.H * a.W;
       }
-    };
-    tile_reduce_store<OutT, WK, NI>(acc, smem + wpos * WK * kTileBytes, wk, lane, rowoff, by * BFE + wf * 64 - fo, fend - fo, ess, res, out,
-                                    aux ? a.aux_relu : a.relu, mend);
-  } else {
-    tile_reduce_store<OutT, WK, NI>(acc, smem + wpos * WK * kTileBytes, wk, lane, rowoff, by * BFE + wf * 64 - fo, fend - fo, ess, res, out,
-                                    aux ? a.aux_relu : a.relu);
+      plain_products(acc, 2 * (nk - k_begin), [&](int step, u32x4 (&w)[2], u32x4 (&x)[2]) {
+        const int k = k_begin + (step >> 1), tap = k / spt, r = tap / a.S, t = tap - r * a.S, chunk = 2 * (step & 1) + lchunk, c = (k - tap * spt) * BKE + chunk * CE;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          w[i] = __builtin_amdgcn_raw_buffer_load_b128(
+              rs_wt, k < nk ? (unsigned)((min(by * BFE + wf * 64 + i * 32 + lrow, a.F - 1) * nk_row + k) * BKE + chunk * CE) * ES : kOOB, 0, 0);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const bool ok = k < nk && (unsigned)(iy[j] + r) < (unsigned)a.H && (unsigned)(ix[j] + t) < (unsigned)a.W;
+          x[j] = __builtin_amdgcn_raw_buffer_load_b128(rs_in, ok ? (unsigned)((img[j] + (iy[j] + r) * a.W + ix[j] + t) * pix + c) * ES : kOOB, 0, 0);
+        }
+      });
+    }
   }
+  tile_reduce_store<OutT, WK, NI>(acc, smem + wpos * WK * kTileBytes, wk, lane, rowoff, by * BFE + wf * 64 - fo, fend - fo, ess, res, out,
+                                  aux ? a.aux_relu : a.relu);
 }
 
 namespace {

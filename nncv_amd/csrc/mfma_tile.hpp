@@ -113,12 +113,10 @@ struct EpiScale {
 // NI = 1: the wave tile is 64 slots x 32 channels (acc[0] only); the LDS tile keeps its 64-channel
 // rows and the lanes of the upper 32 channels simply store nothing.
 // ACT = false compiles only the ReLU form of the activation (the register-tight patch kernel).
-// `mend(tile)` runs when a wave has written its sums (row = slot, column = channel of the tile), before they are read.
-struct NoMend { __device__ __forceinline__ void operator()(unsigned char*) const {} };
-template <typename OutT, int NG, int NI = 2, bool ACT = true, typename Mend = NoMend>
+template <typename OutT, int NG, int NI = 2, bool ACT = true>
 __device__ __forceinline__ void tile_reduce_store(const floatx16 (&acc)[2][2], unsigned char* tile, int g, int lane,
                                                   const int (&rowoff)[2], int f0, int F, const EpiScale<OutT>& ss,
-                                                  const OutT* res, OutT* out, int relu, const Mend& mend = Mend()) {
+                                                  const OutT* res, OutT* out, int relu) {
   const int lrow = lane & 31, lchunk = lane >> 5;
   constexpr int FPL = EpiScale<OutT>::FPL, LPR = EpiScale<OutT>::LPR;
   constexpr int RPI = 64 / LPR;          // pixel rows per store instruction
@@ -158,7 +156,6 @@ __device__ __forceinline__ void tile_reduce_store(const floatx16 (&acc)[2][2], u
         floatx4* p = reinterpret_cast<floatx4*>(mine + (j * 32 + lrow) * kTilePitch + (i * 32 + 8 * q + 4 * lchunk) * 4);
         *p = floatx4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
       }
-  mend(mine);
   __syncthreads();
   floatx4 v[NIT][FPL / 4];
 #pragma unroll

@@ -7,7 +7,10 @@
 // and 4.2e-7 at 4608 (1.2e-6).  The first piece rounds to nearest even: cutting it off as well gives the dropped products a
 // sign (a bias of 3e-8).
 // An infinity has a NaN for its second piece, and so has a finite value that rounds to infinity in bf16: every result such an
-// operand takes part in comes out as a NaN.  A kernel recomputes results that are not finite in plain fp32.
+// operand takes part in comes out as a NaN.  A wave whose sums are not all finite takes them again with the fp32 instructions
+// (plain_products): one operand like that costs its tile's waves a second walk at a third of the rate, and inputs that are all NaN
+// every wave.  Back to back, us a call, usual / one NaN / all NaN: 1500x1001x777 40 / 53 / 75 (one lane a sum: 40 / 90 / 693), a 3x3
+// layer 6x58x78x64 -> 64 31 / 83 / 119 (30 / 360 / 2038), a 1x1 one 23x88x24x128 -> 128 36 / 59 / 77 (36 / 305 / 1918).
 #pragma once
 #include "mfma_tile.hpp"
 
@@ -64,11 +67,43 @@ __device__ __forceinline__ void split_products(const u32x4 (&a)[TM][3], const u3
       }
 }
 
-__device__ __forceinline__ bool split_finite(const floatx4& v) {
-  bool ok = true;
+// big + low -> big; whether a sum of the wave is not finite
+template <int TM, int TN>
+__device__ __forceinline__ bool split_sums(floatx16 (&big)[TM][TN], const floatx16 (&low)[TM][TN]) {
+  float t = 0.0f;  // a sum times zero is a zero or a NaN
 #pragma unroll
-  for (int e = 0; e < 4; ++e) ok &= __builtin_fabsf(v[e]) < __builtin_inff();
-  return ok;
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      big[i][j] += low[i][j];
+#pragma unroll
+      for (int v = 0; v < 16; ++v) t = __builtin_fmaf(big[i][j][v], 0.0f, t);
+    }
+  return __builtin_amdgcn_ballot_w64(!(t == 0.0f)) != 0;
+}
+
+// The sums of TM x TN blocks with the fp32 instructions, straight from memory.  load(s, a, b): step s, eight k, four of which a lane half has
+// (lanes l < 32 the first ones); zeros for a step past the last.
+template <int TM, int TN, typename Load>
+__device__ __forceinline__ void plain_products(floatx16 (&acc)[TM][TN], int steps, const Load& load) {
+  u32x4 a[2][TM], b[2][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+  load(0, a[0], b[0]);
+#pragma unroll 1
+  for (int s = 0; s < steps; s += 2)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      load(s + h + 1, a[h ^ 1], b[h ^ 1]);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) Mma<float>::run(a[h][i], b[h][j], acc[i][j]);
+    }
 }
 
 }  // namespace mt
