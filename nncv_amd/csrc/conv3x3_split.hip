@@ -216,7 +216,7 @@ __global__ __launch_bounds__(64 * KG * split_units(WS)) __attribute__((amdgpu_wa
             pstore(i, other);
             pload(i, slab + 2);
           }
-          constexpr int kMma = 6 * JN, kValu = (26 * (p1 - p0) + kMma - 1) / kMma;
+          constexpr int kMma = 6 * JN, kValu = (30 * (p1 - p0) + kMma - 1) / kMma;
 #pragma unroll
           for (int n = 0; n < kMma; ++n) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);

@@ -4,8 +4,8 @@
 //  * A (K contiguous): whole 128-byte lines, eight lanes each, a round ahead, through an LDS buffer of the wave's own, because an
 //    operand wants 16 bytes of 32 rows and read like that every lane of a load touches a line of its own.
 //  * B (N contiguous): lane l holds columns TN l .. TN l + TN - 1, so a load of row k is whole lines again.
-//  * Both are split in registers, 7 vector instructions for two values: 112 of them feed the 24 products (768 clocks) of a
-//    64 x 64 tile and 16 k, and run under the products of the SIMD's other wave.
+//  * Both are split in registers, thirteen vector instructions for two values: 208 of them (832 clocks) feed the 24 products (768 clocks)
+//    of a 64 x 64 tile and 16 k, and run under the products of the SIMD's other wave.
 //  * Nothing asks for alignment beyond 4 bytes.  Only the last round of the matrix can hold k >= K or leave the buffers; the
 //    group that owns it walks it first, with A masked (B's rows past the end come back as zeros from the range check,
 //    gemm_split_walk.hpp).
@@ -94,9 +94,9 @@ __global__ __launch_bounds__(64 * KG, TM * TN == 4 ? 2 : TM * TN == 2 ? 3 : 4) v
   // units of the tile: register u % 16 of block row u / 16, columns TN lrow .. ; the ones this wave adds to C are asked for now
   typedef float vec __attribute__((ext_vector_type(TN)));
   constexpr int kUnits = 16 * TM, kMine = kUnits / KG;
-  auto row_of = [&](int u) { return m0 + 32 * (u >> 4) + 8 * ((u & 15) >> 2) + 4 * lh + (u & 3); };
-  auto fetch = [&](int u) {
-    const int m = row_of(u), n = n0 + TN * lrow;
+  auto row_of = [&](int u, int lane) { return m0 + 32 * (u >> 4) + 8 * ((u & 15) >> 2) + 4 * (lane >> 5) + (u & 3); };
+  auto fetch = [&](int u, int lane) {
+    const int m = row_of(u, lane), n = n0 + TN * (lane & 31);
     vec v = {};
     if (m < M && n < N) {
       const float* c = C + ((long long)m * N + n);
@@ -115,7 +115,7 @@ __global__ __launch_bounds__(64 * KG, TM * TN == 4 ? 2 : TM * TN == 2 ? 3 : 4) v
   vec cpre[kEarly ? kMine : 1];
   if constexpr (kEarly) {
 #pragma unroll
-    for (int q = 0; q < kMine; ++q) cpre[q] = fetch(grp * kMine + q);
+    for (int q = 0; q < kMine; ++q) cpre[q] = fetch(grp * kMine + q, lane);
   }
   if (grp == 0) {
     const int kend = K - 32 * r - 4 * (lane & 7);  // of this lane's four k
@@ -150,10 +150,11 @@ __global__ __launch_bounds__(64 * KG, TM * TN == 4 ? 2 : TM * TN == 2 ? 3 : 4) v
       split_products(a, b, big, low);
     }
   }
+  // The lane's number once more: what follows from it is not kept over the loop, in registers that the loop needs.  (32-row forms only
+  // behind the sums: 1500x1001x777 36.4 -> 35.2 us a call; 64 x 64 tiles spill with it.)
+  const int again = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), late = TM == 1 ? again : lane;
   if (__builtin_expect(split_sums(big, low), 0)) {  // once more with the fp32 instructions: eight k a step, four steps a round
-    int at_lane = lane;  // (worked out here: what is known before the loop is kept over it, in registers that it needs)
-    asm volatile("" : "+v"(at_lane));
-    const int lrow = at_lane & 31, lh = at_lane >> 5;
+    const int lrow = again & 31, lh = again >> 5;
     plain_products(big, 4 * ((nk - grp + KG - 1) / KG), [&](int s, u32x4 (&a)[TM], u32x4 (&b)[TN]) {
       const int round = nk - 1 - grp - (s >> 2) * KG, k0 = 32 * round + 8 * (s & 3);
       const long long at = (long long)m0 * K + k0, rows = (long long)k0 * N + n0;
@@ -185,7 +186,7 @@ __global__ __launch_bounds__(64 * KG, TM * TN == 4 ? 2 : TM * TN == 2 ? 3 : 4) v
 
   // ---- D = C + sums ----
   auto emit = [&](int unit, const vec& c, vec sum) {
-    const int m = row_of(unit), n = n0 + TN * lrow;
+    const int m = row_of(unit, late), n = n0 + TN * (late & 31);
     if (m >= M || n >= N) return;
     sum += c;
     float* d = D + ((long long)m * N + n);
@@ -198,11 +199,11 @@ __global__ __launch_bounds__(64 * KG, TM * TN == 4 ? 2 : TM * TN == 2 ? 3 : 4) v
       vec y;
 #pragma unroll
       for (int j = 0; j < TN; ++j) y[j] = big[u >> 4][j][u & 15];
-      emit(u, fetch(u), y);
+      emit(u, fetch(u, late), y);
     }
   } else {
     // [group][unit][lane][TN]
-    vec* mine = reinterpret_cast<vec*>(lds) + lane;
+    vec* mine = reinterpret_cast<vec*>(lds) + late;
 #pragma unroll
     for (int u = 0; u < kUnits; ++u) {
       vec y;
@@ -214,11 +215,11 @@ __global__ __launch_bounds__(64 * KG, TM * TN == 4 ? 2 : TM * TN == 2 ? 3 : 4) v
 #pragma unroll
     for (int q = 0; q < kMine; ++q) {
       const int u = grp * kMine + q;
-      const vec* p = reinterpret_cast<const vec*>(smem) + u * 64 + lane;
+      const vec* p = reinterpret_cast<const vec*>(smem) + u * 64 + late;
       vec sum = p[0];
 #pragma unroll
       for (int g = 1; g < KG; ++g) sum += p[g * (Cfg::kWave / sizeof(vec))];
-      emit(u, kEarly ? cpre[kEarly ? q : 0] : fetch(u), sum);
+      emit(u, kEarly ? cpre[kEarly ? q : 0] : fetch(u, late), sum);
     }
   }
 }

@@ -19,7 +19,7 @@
 //  * K groups meet in an fp32 LDS tile and the epilogue reads it back so that residual reads and
 //    result stores are whole 128-byte rows (mfma_tile.hpp).
 //  * fp32 blocks without K groups multiply on the bf16 matrix pipes (three-way splits, split.hpp): a 64x64 sub-tile's 16 k are 24
-//    instructions of 32 clocks instead of 32 of 64, and 176 to split its operands, which run beside them (two waves a SIMD).
+//    instructions of 32 clocks instead of 32 of 64, and 208 to split its operands, which run beside them (two waves a SIMD).
 //  * Workgroups are renumbered so that each XCD (8 of them, round-robin over the linear workgroup
 //    id) gets a contiguous range of pixel tiles: neighbouring tiles share input rows, and each
 //    XCD has its own L2.

@@ -6,8 +6,13 @@
 // 64 bits the error of a sum of normal products is 3.1e-8 at 16 of them (fp32 instructions 7.3e-8), 1.3e-7 at 576 (4.3e-7)
 // and 4.2e-7 at 4608 (1.2e-6).  The first piece rounds to nearest even: cutting it off as well gives the dropped products a
 // sign (a bias of 3e-8).
-// An infinity has a NaN for its second piece, and so has a finite value that rounds to infinity in bf16: every result such an
-// operand takes part in comes out as a NaN.  A wave whose sums are not all finite takes them again with the fp32 instructions
+// bf16 ends at 2^-133 (its normal numbers at 2^-126), fp32 at 2^-149: what is split is 2^24 times the value, so that every piece
+// of every fp32 value is a normal number, and a sum is 2^48 times what it is worth.  (Unscaled, the error of a sum of products of one
+// operand at 2^-112 was 2.6e-7, at 2^-118 1.8e-5, at 2^-126 2.4e-3.)  The two multiplications for a pair of values cost 1.7 % of a
+// classification of six photographs (368.1 -> 374.3 us), 2 to 6 % of a product (1500x1001x777 22.6 -> 23.0, 4096^3 758 -> 796).  To look
+// for pieces that lose bits instead (an or for a pair) was slower: its register made the 64 x 64 products spill (4096^3 1142).
+// An infinity has a NaN for its second piece, and so has a value from 2^103 on that 2^24 takes to infinity; a sum from 2^80 on is
+// infinite.  Every result such an operand takes part in comes out not finite.  A wave whose sums are not all finite takes them again with the fp32 instructions
 // (plain_products): one operand like that costs its tile's waves a second walk at a third of the rate, and inputs that are all NaN
 // every wave.  Back to back, us a call, usual / one NaN / all NaN: 1500x1001x777 40 / 53 / 75 (one lane a sum: 40 / 90 / 693), a 3x3
 // layer 6x58x78x64 -> 64 31 / 83 / 119 (30 / 360 / 2038), a 1x1 one 23x88x24x128 -> 128 36 / 59 / 77 (36 / 305 / 1918).
@@ -22,10 +27,14 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
-// Two values -> their pieces, packed in pairs: eleven instructions.  The first piece is rounded to nearest even, the second is
+constexpr float kSplitScale = 0x1p24f, kSplitWorth = 0x1p-48f;
+
+// Two values -> their pieces, packed in pairs: thirteen instructions.  The first piece is rounded to nearest even, the second is
 // cut off what is left, which has eight bits to go then: the third is exact.  (v_dot2_f32_bf16 would take a piece off in
 // one instruction instead of two, but it runs in the matrix pipe: the products wait for it.)
 __device__ __forceinline__ void split_pair(float x, float y, unsigned (&p)[3]) {
+  x *= kSplitScale;
+  y *= kSplitScale;
   p[0] = __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2{x, y}), bf16x2));
   x -= __builtin_bit_cast(float, p[0] << 16);
   y -= __builtin_bit_cast(float, p[0] & 0xffff0000u);
@@ -67,7 +76,7 @@ __device__ __forceinline__ void split_products(const u32x4 (&a)[TM][3], const u3
       }
 }
 
-// big + low -> big; whether a sum of the wave is not finite
+// what big + low are worth -> big; whether a sum of the wave is not finite
 template <int TM, int TN>
 __device__ __forceinline__ bool split_sums(floatx16 (&big)[TM][TN], const floatx16 (&low)[TM][TN]) {
   float t = 0.0f;  // a sum times zero is a zero or a NaN
@@ -75,9 +84,11 @@ __device__ __forceinline__ bool split_sums(floatx16 (&big)[TM][TN], const floatx
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      big[i][j] += low[i][j];
 #pragma unroll
-      for (int v = 0; v < 16; ++v) t = __builtin_fmaf(big[i][j][v], 0.0f, t);
+      for (int v = 0; v < 16; ++v) {
+        big[i][j][v] = (big[i][j][v] + low[i][j][v]) * kSplitWorth;
+        t = __builtin_fmaf(big[i][j][v], 0.0f, t);
+      }
     }
   return __builtin_amdgcn_ballot_w64(!(t == 0.0f)) != 0;
 }
