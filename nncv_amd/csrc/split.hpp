@@ -1,21 +1,26 @@
 // fp32 products on the bf16 matrix pipes (gfx950): an fp32 value is the exact sum of three bf16 pieces, and
-//   a b = ah bh + (ah bm + am bh) + (ah bl + am bm + al bh) + what is below 2^-24 of it.
+//   a b = ah bh + (ah bm + am bh) + (ah bl + am bm + al bh) + what is below 2^-24 of it
+// (G. Henry, P. T. P. Tang, A. Heinecke, Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations, 2019).
 // The six products are v_mfma_f32_32x32x16_bf16, sixteen times the rate of the fp32 instructions for six times the
 // work; every one is exact and the sums are fp32.  The five small ones are summed in registers of their own, so the chain of
 // roundings that carries the result's magnitude has one link for 16 k, where the fp32 instructions have one for every k: against
 // 64 bits the error of a sum of normal products is 3.1e-8 at 16 of them (fp32 instructions 7.3e-8), 1.3e-7 at 576 (4.3e-7)
-// and 4.2e-7 at 4608 (1.2e-6).  The first piece rounds to nearest even: cutting it off as well gives the dropped products a
-// sign (a bias of 3e-8).
-// bf16 ends at 2^-133 (its normal numbers at 2^-126), fp32 at 2^-149: what is split is 2^24 times the value, so that every piece
+// and 4.2e-7 at 4608 (1.2e-6).  A sum that one product is all of is where the dropped ones show: off by 9.5e-8 at most, 2.6e-8 in the
+// mean, where one fp32 rounding makes 6.0e-8 and 2.5e-8.  (Pieces that are cut off instead of rounded: 1.55e-7 with the second one,
+// and with the first one the dropped products have a sign, a bias of 3e-8.)
+//
+// Range.  bf16 ends at 2^-133 (its normal numbers at 2^-126), fp32 at 2^-149: what is split is 2^24 times the value, so that every piece
 // of every fp32 value is a normal number, and a sum is 2^48 times what it is worth.  (Unscaled, the error of a sum of products of one
 // operand at 2^-112 was 2.6e-7, at 2^-118 1.8e-5, at 2^-126 2.4e-3.)  The two multiplications for a pair of values cost 1.7 % of a
 // classification of six photographs (368.1 -> 374.3 us), 2 to 6 % of a product (1500x1001x777 22.6 -> 23.0, 4096^3 758 -> 796).  To look
 // for pieces that lose bits instead (an or for a pair) was slower: its register made the 64 x 64 products spill (4096^3 1142).
-// An infinity has a NaN for its second piece, and so has a value from 2^103 on that 2^24 takes to infinity; a sum from 2^80 on is
-// infinite.  Every result such an operand takes part in comes out not finite.  A wave whose sums are not all finite takes them again with the fp32 instructions
-// (plain_products): one operand like that costs its tile's waves a second walk at a third of the rate, and inputs that are all NaN
-// every wave.  Back to back, us a call, usual / one NaN / all NaN: 1500x1001x777 40 / 53 / 75 (one lane a sum: 40 / 90 / 693), a 3x3
-// layer 6x58x78x64 -> 64 31 / 83 / 119 (30 / 360 / 2038), a 1x1 one 23x88x24x128 -> 128 36 / 59 / 77 (36 / 305 / 1918).
+//
+// What is not finite.  An infinity has a NaN for its second piece, and so has a value from 2^103 on, which 2^24 takes to infinity; a sum
+// from 2^80 on is infinite.  Every result such an operand takes part in comes out not finite, and a wave whose sums are not all finite
+// takes them again with the fp32 instructions (plain_products): one operand like that costs its tile's waves a second walk at a
+// third of the rate, and inputs that are all NaN every wave.  Back to back, us a call, usual / one NaN / all NaN: 1500x1001x777
+// 40 / 53 / 75 (one lane a sum: 40 / 90 / 693), a 3x3 layer 6x58x78x64 -> 64 31 / 83 / 119 (30 / 360 / 2038), a 1x1 one
+// 23x88x24x128 -> 128 36 / 59 / 77 (36 / 305 / 1918).
 #pragma once
 #include "mfma_tile.hpp"
 
@@ -29,19 +34,18 @@ typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr float kSplitScale = 0x1p24f, kSplitWorth = 0x1p-48f;
 
-// Two values -> their pieces, packed in pairs: thirteen instructions.  The first piece is rounded to nearest even, the second is
-// cut off what is left, which has eight bits to go then: the third is exact.  (v_dot2_f32_bf16 would take a piece off in
-// one instruction instead of two, but it runs in the matrix pipe: the products wait for it.)
+// Two values -> their pieces, packed in pairs: thirteen instructions.  Two pieces are rounded to nearest even, what is left after them
+// has eight bits: the third is exact.  (The second one cut off takes as many, and as long within 1 %.  v_dot2_f32_bf16 would take a piece off in one instruction instead of
+// two, but it runs in the matrix pipe: the products wait for it.)
 __device__ __forceinline__ void split_pair(float x, float y, unsigned (&p)[3]) {
   x *= kSplitScale;
   y *= kSplitScale;
   p[0] = __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2{x, y}), bf16x2));
   x -= __builtin_bit_cast(float, p[0] << 16);
   y -= __builtin_bit_cast(float, p[0] & 0xffff0000u);
-  const unsigned u = __builtin_bit_cast(unsigned, x), v = __builtin_bit_cast(unsigned, y);
-  p[1] = __builtin_amdgcn_perm(v, u, 0x07060302u);
-  x -= __builtin_bit_cast(float, u & 0xffff0000u);
-  y -= __builtin_bit_cast(float, v & 0xffff0000u);
+  p[1] = __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2{x, y}), bf16x2));
+  x -= __builtin_bit_cast(float, p[1] << 16);
+  y -= __builtin_bit_cast(float, p[1] & 0xffff0000u);
   p[2] = __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, y), __builtin_bit_cast(unsigned, x), 0x07060302u);
 }
 

@@ -1,5 +1,5 @@
 """fp32 kernels on the bf16 matrix pipes (split.hpp) over the whole range of fp32: operands down to the subnormal numbers and up to
-where sums are large, values of very different size in one sum; each kernel, against 64 bits, with the error of ordinary operands as the bar."""
+where sums are large, values of very different size in one sum, sums that one product is all of; each kernel, against 64 bits, with the error of ordinary operands as the bar."""
 import numpy as np
 import pytest
 import torch
@@ -74,6 +74,33 @@ def test_layer(case, sx, sw):
     scale, pick = 2.0 ** -(sx + sw), [0, N - 1]
     want = torch.nn.functional.conv2d(x[pick].double(), w.double(), stride=stride, padding=pad) * scale
     assert relative(got[pick].double() * scale, want) < (bar(R * R * C) if taken_again(sx, sw) else split_bar(R * R * C))
+
+
+# A sum that is one product: two dropped products of 2^-8 x 2^-17 at most, and a rounding of 2^-24
+LONE = 2.0 ** -23 * 1.01
+
+
+def test_a_product_that_is_a_sum_of_its_own():
+    M, N, K = 1499, 1002, 778
+    g = torch.Generator().manual_seed(8)
+    a, b = torch.zeros(M, K), torch.rand((K, N), generator=g) + 1
+    col = torch.arange(M) % K
+    a[torch.arange(M), col] = torch.rand(M, generator=g) + 1
+    got, tags = product(a, b, torch.zeros(M, N))
+    assert tags[0].startswith("gemm_split")
+    want = a[torch.arange(M), col].double().view(M, 1) * b[col].double()
+    assert ((got.double() - want).abs() / want).max().item() < LONE
+
+
+@pytest.mark.parametrize("case", LAYERS, ids=lambda c: c[8])
+def test_a_filter_of_one_weight(case):
+    N, C, F, H, W, R, stride, pad, _ = case
+    g = torch.Generator().manual_seed(9)
+    x, w = torch.rand((N, C, H, W), generator=g) + 1, torch.zeros(F, C, R, R)
+    f = torch.arange(F)
+    w[f, f % C, R // 2, R // 2] = torch.rand(F, generator=g) + 1
+    want = x[:, f % C, ::stride, ::stride].double() * w[f, f % C, R // 2, R // 2].double().view(1, F, 1, 1)
+    assert ((layer(case, x, w).double() - want).abs() / want).max().item() < LONE
 
 
 @pytest.mark.parametrize("case", LAYERS, ids=lambda c: c[8])
