@@ -723,7 +723,7 @@ void launch_conv3x3_patch(const IgemmArgs& g, int in_dt, int out_dt, hipStream_t
     else if (halves) launch_patch_cfg<half_t, half_t, 1, 4, 1>(a, flops, bytes, "conv3x3_patch<f16,1,4,half>", s);
     else launch_patch_cfg<half_t, half_t, 1, 4, 2>(a, flops, bytes, "conv3x3_patch<f16,1,4>", s);
   } else {
-    launch_conv3x3_split(a, ws, halves, ws == 4 ? "conv3x3_patch<f32,4,1>" : ws == 2 ? "conv3x3_patch<f32,2,2>" : halves ? "conv3x3_patch<f32,1,4,half>" : "conv3x3_patch<f32,1,4>",
+    launch_conv3x3_split(a, ws, halves, ws == 4 ? "conv3x3_split<f32,4,1>" : ws == 2 ? "conv3x3_split<f32,2,2>" : halves ? "conv3x3_split<f32,1,4,half>" : "conv3x3_split<f32,1,4>",
                          flops, bytes, s);
   }
   NNCV_HIP_CHECK(hipGetLastError());

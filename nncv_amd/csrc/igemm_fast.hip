@@ -281,7 +281,7 @@ void launch_fast_cfg(const IgemmArgs& a, hipStream_t s) {
   constexpr int epi = WP * WF * WK * kTileBytes;  // one output-tile copy per K group
   constexpr int smem = stage2 > epi ? stage2 : epi;
   static const std::string tag = std::string("igemm_fast<") + tn<T>() + "," + tn<OutT>() + "," + std::to_string(WP) + "," +
-                                 std::to_string(WF) + "," + std::to_string(WK) + "," + std::to_string(KS) + (NI == 1 ? ",half>" : ">");
+                                 std::to_string(WF) + "," + std::to_string(WK) + "," + std::to_string(KS) + (SPLIT ? ",split>" : NI == 1 ? ",half>" : ">");
   auto kern = igemm_fast_kernel<T, OutT, WP, WF, WK, KS, NI, SPLIT>;
   static const bool attr_set = [&] {
     NNCV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem));

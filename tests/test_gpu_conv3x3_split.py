@@ -41,7 +41,7 @@ def layer_and_reference(case, seed, spoil=None):
 @pytest.mark.parametrize("case", CASES, ids=lambda c: c[5] + "-" + "x".join(map(str, c[:5])))
 def test_every_form(case):
     got, want, tags = layer_and_reference(case, 1)
-    assert tags == ["conv3x3_patch<f32,%s>" % case[5]]
+    assert tags == ["conv3x3_split<f32,%s>" % case[5]]
     err = ((got.double() - want).norm() / want.norm()).item()
     # 9 C / 16 additions of half an ulp at most in a row, as a random walk, and a few ulp at the end
     assert err < 2.0 ** -25 * (9 * case[1] / 48) ** 0.5 + 2.0 ** -24, err

@@ -34,7 +34,7 @@ def test_matches_double(N, C, F, H, W, R, stride, pad, tag):
     want = torch.nn.functional.conv2d(x[pick].double(), w.double(), stride=stride, padding=pad)
     res = torch.randn((N, F) + tuple(want.shape[2:]), generator=g)
     got, tags = run(x, w, stride, pad)
-    assert tags == ["igemm_fast<f32,f32,%s>" % tag], tags
+    assert tags == ["igemm_fast<f32,f32,%s,split>" % tag], tags
     assert rel_l2(got[pick], want.numpy()) < 2.0 ** -24 * (R * R * C) ** 0.5
     got, _ = run(x, w, stride, pad, True, res)
     assert rel_l2(got[pick], torch.relu(want + res[pick].double()).numpy()) < 2.0 ** -24 * (R * R * C) ** 0.5
@@ -48,7 +48,7 @@ def test_not_finite():
     x[7, :, 9, 9] = 0.0
     w[5, 1], w[77, 63] = 3.4e38, float("inf")
     got, tags = run(x, w, 1, 0)
-    assert tags == ["igemm_fast<f32,f32,2,2,1,1>"], tags
+    assert tags == ["igemm_fast<f32,f32,2,2,1,1,split>"], tags
     want = torch.nn.functional.conv2d(x, w).numpy()
     fin = np.isfinite(want)
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[~fin & ~np.isnan(want)], want[~fin & ~np.isnan(want)])

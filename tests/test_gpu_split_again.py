@@ -14,11 +14,11 @@ pytestmark = pytest.mark.gpu
 HUGE = 3.4e38  # infinity in bf16: a sum with it in is a NaN there, whatever it is multiplied by
 
 # N, C, F, H, W, R, stride, pad, tag.  Taps of whole rounds and others, blocks of 128 x 128 and 256 x 64, windows over the border
-LAYERS = [(N, C, F, H, W, 3, 1, 1, "conv3x3_patch<f32,%s>" % form) for N, C, F, H, W, form in CASES] + [
+LAYERS = [(N, C, F, H, W, 3, 1, 1, "conv3x3_split<f32,%s>" % form) for N, C, F, H, W, form in CASES] + [
     (7, 96, 108, 24, 42, 3, 1, 1, "conv3x3_direct<f32,64x32,splitk4>"), (12, 88, 108, 35, 17, 3, 1, 1, "conv3x3_direct<f32,64x32,splitk4>"),
     (6, 64, 128, 58, 78, 3, 2, 1, "conv3x3_direct<f32,64x32,splitk4>"),
-    (23, 128, 128, 88, 24, 1, 1, 0, "igemm_fast<f32,f32,2,2,1,1>"), (13, 16, 128, 95, 29, 5, 1, 2, "igemm_fast<f32,f32,2,2,1,1>"),
-    (43, 16, 60, 22, 89, 5, 1, 2, "igemm_fast<f32,f32,4,1,1,1>")]
+    (23, 128, 128, 88, 24, 1, 1, 0, "igemm_fast<f32,f32,2,2,1,1,split>"), (13, 16, 128, 95, 29, 5, 1, 2, "igemm_fast<f32,f32,2,2,1,1,split>"),
+    (43, 16, 60, 22, 89, 5, 1, 2, "igemm_fast<f32,f32,4,1,1,1,split>")]
 
 
 def relative(got, want):

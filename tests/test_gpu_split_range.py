@@ -40,7 +40,7 @@ def test_product(M, N, K, sa, sb):
     assert relative(got.double() * scale, (a.double() @ b.double()) * scale) < (bar(K) if taken_again(sa, sb) else split_bar(K))
 
 
-LAYERS = [(6, 64, 64, 29, 39, 3, 1, 1, "conv3x3_patch<f32"), (6, 256, 256, 15, 20, 3, 1, 1, "conv3x3_patch<f32"), (6, 64, 128, 58, 78, 3, 2, 1, "conv3x3_direct<f32,64x32"),
+LAYERS = [(6, 64, 64, 29, 39, 3, 1, 1, "conv3x3_split<f32"), (6, 256, 256, 15, 20, 3, 1, 1, "conv3x3_split<f32"), (6, 64, 128, 58, 78, 3, 2, 1, "conv3x3_direct<f32,64x32"),
           (23, 128, 128, 88, 24, 1, 1, 0, "igemm_fast<f32,f32,2,2"), (43, 16, 60, 22, 89, 5, 1, 2, "igemm_fast<f32,f32,4,1")]
 
 
