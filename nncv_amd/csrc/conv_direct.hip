@@ -502,9 +502,10 @@ const Form* best_form(const IgemmArgs& a, int dt, double* us) {
 
 // The same for the kernel that would run the layer otherwise.  Implicit GEMM: fits over its 64 x 64 tiles, within 7-16 %.
 // fp32 3x3 stride-1 layers (conv3x3_split.hip): a start and so much for every 32 channels and tap of a CU's turns; 75 layers of 20
-// MFLOP to 20 GFLOP, within 10 %.  Half blocks of filters are the launches of up to 128 whole ones.  From 129 to 144 whole
-// blocks nearly half of the chip is idle and the layer stays here, though it would take less there (7x15x20x256 23.1 us against
-// 35.3, 5x9x25x192 -> 440 18.9 against 23.6): this is the size of layer that this kernel's test holds it to.
+// MFLOP to 20 GFLOP, within 10 %.  Half blocks of filters are the launches of up to 128 whole ones; just above, where nearly half of the
+// chip is idle, the model holds too: of 75 layers of 120 to 160 whole blocks the 15 that it gives to that kernel from 129 to 144 on
+// take 1.2 to 1.7 times as long here (7x15x20x256 32.1 against 19.7 us, 5x9x25x192 -> 440 21.2 against 16.2, 16x36x16x512 -> 64 55.6
+// against 32.1).
 double other_us(const IgemmArgs& a, int dt, DirectRival rival) {
   struct Fit { double fixed, round, tile, chain; };
   static const Fit f32[] = {{3.3, 0.642, 0.79, 0.0}, {2.7, 0.835, 0.14, 0.26}};
@@ -518,7 +519,7 @@ double other_us(const IgemmArgs& a, int dt, DirectRival rival) {
     if (p[0] == 4) return 5.0 + 1.2 * rounds * turns;
     if (p[0] == 2) return 6.0 + 0.5 * rounds * turns;
     if (wgs <= 128 && main_f % 64 == 0) return 4.9 + 0.132 * rounds;
-    return wgs > 128 && wgs <= 144 ? 1e30 : 4.3 + 0.26 * rounds * turns;
+    return 4.3 + 0.26 * rounds * turns;
   }
   if (rival == kRivalIgemmFast && dt == kF32) {
     const double split = igemm_fast_split_us(a);

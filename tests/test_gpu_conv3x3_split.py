@@ -16,7 +16,9 @@ CASES = [(8, 32, 344, 53, 47, "4,1"), (15, 32, 480, 35, 17, "4,1"), (6, 64, 64, 
          (12, 128, 200, 19, 13, "1,4"), (33, 96, 72, 31, 9, "1,4"), (5, 96, 456, 19, 13, "1,4"), (6, 256, 256, 15, 20, "1,4,half"),
          (4, 224, 256, 40, 7, "1,4,half"), (16, 512, 512, 7, 7, "1,4,half"), (5, 128, 128, 25, 17, "1,4,half"),
          # more workgroups on an XCD than it has CUs
-         (17, 224, 152, 14, 19, "1,4"), (9, 512, 896, 8, 8, "1,4,half")]
+         (17, 224, 152, 14, 19, "1,4"), (9, 512, 896, 8, 8, "1,4,half"),
+         # whole blocks of filters for little more than half of the CUs
+         (7, 256, 256, 15, 20, "1,4"), (5, 192, 440, 9, 25, "1,4")]
 
 
 def layer_and_reference(case, seed, spoil=None):
