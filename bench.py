@@ -73,7 +73,7 @@ CLOCK_WARMUP_MS = 60.0          # untimed work ahead of a timed loop (see the mo
 DOMINANT_LAYER = {
     "conv3x3_stream<f16,1x2x2>": (128, 128, 28),
     "conv3x3_stream<f16,1x4x1>": (128, 128, 28),
-    "conv3x3_stream<f16,1x1x4>": (256, 256, 14),
+    "conv3x3_stream<f16,1x1x4>": (512, 512, 7),
     "conv3x3_patch<f16,4,1>": (64, 64, 56),
     "conv3x3_patch<f16,2,2>": (128, 128, 28),
     "conv3x3_patch<f16,1,4>": (512, 512, 7),

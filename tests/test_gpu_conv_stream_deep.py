@@ -10,7 +10,9 @@ pytestmark = pytest.mark.gpu
 
 # N, H, W, C, F, tag: two images and more a tile (rows of 3 to 8 pixels), the last tile part empty, filters in 32s, 64s and 128s
 CASES = [(41, 7, 7, 512, 512, "1x2x2"), (50, 7, 7, 512, 512, "1x2x2"), (101, 7, 7, 512, 512, "1x4x1"), (41, 8, 8, 384, 512, "1x2x2"), (37, 22, 3, 384, 512, "1x2x2"),
-         (111, 3, 8, 192, 192, "1x1x4"), (33, 10, 10, 448, 512, "1x2x2"), (7, 32, 32, 320, 320, "1x2x2"), (19, 9, 11, 256, 256, "1x1x4")]
+         (111, 3, 8, 192, 192, "1x1x4"), (33, 10, 10, 448, 512, "1x2x2"), (7, 32, 32, 320, 320, "1x2x2"), (19, 9, 11, 256, 256, "1x1x4"),
+         # little more than 128 blocks of 32 filters
+         (32, 7, 7, 512, 512, "1x1x4"), (18, 5, 31, 448, 160, "1x1x4"), (46, 10, 10, 64, 96, "1x1x4"), (7, 13, 17, 256, 320, "1x1x4")]
 
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c[:5])))

@@ -95,7 +95,7 @@ def test_fp16_small_batch(blob):
 
 def test_fp16_layers_take_the_kernels_they_are_measured_on(blob):
     """The launch tags of one fp16 forward pass at 224x224: every 3x3 stride-1 layer goes through one of the two LDS-patch
-    kernels (the stream form for layers of at most 256 channels, the patch form for the deepest ones), the three stride-2
+    kernels (the stream form where its blocks of 32 filters are for more than half of the CUs, the patch form where not), the three stride-2
     ones through the patch kernel's stride-2 form with the 1x1 shortcut riding along (no separate shortcut launch), so a
     silent fall-back to the implicit-GEMM kernels shows up here and not only in the timings."""
     hb = synth.round_fp16(blob)
@@ -117,10 +117,13 @@ def test_fp16_layers_take_the_kernels_they_are_measured_on(blob):
     # batch 32, the measured configuration (input values do not matter for the route)
     _, rep, count = tags(dev(synth.round_fp16(synth.uniform(4004, (32, 3, 224, 224), 0.0, 1.0)), abi.F16))
     assert count("conv3x3_patch") + count("conv3x3_stream") == 13
-    assert count("conv3x3_stream") == 10  # layer1 (4), layer2 (3) and layer3 (3)
+    assert count("conv3x3_stream") == 13  # layer1 (4), layer2, layer3 and layer4 (3 each)
     assert count("conv3x3s2_patch") == 3
     assert count("igemm") == 0
     assert sum(v["launches"] for v in rep.values()) == 18  # + stem/pool and pool/FC
+    # batch 16: layer4 has 128 blocks
+    _, rep, count = tags(dev(synth.round_fp16(synth.uniform(4005, (16, 3, 224, 224), 0.0, 1.0)), abi.F16))
+    assert count("conv3x3_stream") == 10 and count("conv3x3_patch") == 3 and count("conv3x3s2_patch") == 3 and count("igemm") == 0
     # batch 4 against the oracle: the small launches of layer2 / layer3 stay with the patch kernel
     x = synth.round_fp16(synth.uniform(4003, (4, 3, 224, 224), 0.0, 1.0))
     got, rep, count = tags(dev(x, abi.F16))
