@@ -565,9 +565,12 @@ void launch_frag(RingArgs d, int, hipStream_t s) {
 // chain_us + t * slab_any for 64 channels (nine slabs, bound by memory); within 6 % (1 sigma) over 112 stride-2 layers of 1 to 60
 // GFLOP, and in the choice between the two 0.8 % off the better one on average.  With 64 channels, 64 pixels to a tile are up to 8 %
 // ahead to 16 such tiles a CU (80x56x56 -> 128 17.1 against 18.3 us), 128 from there (241x77x91 -> 72 91.7 against 101.9).  The
-// ring's own forms of 128 filters are level with them at best, save for 64 channels and a fourth turn of the tiles of 64 pixels: the two
-// tiles of 128 x 128 of a CU then run side by side with 16 waves (64 to 80 images of 56x56x64 -> 128: 13.7 to 14.9 against 13.8 to 15.8 us
-// on one card, 15.5 to 17.4 against 15.9 to 17.1 on another).
+// ring's own forms of 128 filters are level with them at best, save for 64 channels and more than three, up to four tiles of 64 x 128 a CU:
+// the two tiles of 128 x 128 that a CU has there run side by side with 16 waves, in one turn.  It is the number of tiles that does it, not
+// the layer: of 31 layers in that band, 72 to 384 filters on maps of 14x14 to 224x20, 28 take 0.90 to 0.995 times as long on the ring
+// and three 1.00 to 1.01 (1037x14x14 -> 72 13.3 against 14.0 us, 318x28x28 -> 96 15.1 / 16.0, 79x56x56 -> 128 15.8 / 17.6, 19x80x80 -> 256
+// 15.7 / 16.3); of 38 layers on both sides of it, 2.3 to 6.5 tiles, 36 take 1.00 to 1.19 times as long there (41x80x80 -> 96, 4.004
+// tiles: 19.9 against 17.1; 242x28x28 -> 128, 2.9: 14.8 / 13.2).
 // slab_us and chain_us grow by slab_any and chain_any where the taps are not whole slabs.  Fits over 300 layers of 1x1 to 7x7
 // windows, 8 to 1024 channels; the form they choose is within 1.5 % of the best one on average.
 struct Form {
@@ -600,6 +603,7 @@ const Form* best_form(const IgemmArgs& a, double* us) {
   const double P = (double)a.N * a.OH * a.OW, slabs = std::ceil(a.R * a.S * a.C / 64.0), main_f = a.aux_f0 ? a.aux_f0 : a.F;
   const bool any = a.R * a.S > 1 && a.C % 64 != 0, nine = slabs <= 9;
   auto per_cu = [&](const Form& f, double filters) { return std::ceil(P / f.bp) * std::ceil(filters / f.bf) / 256; };
+  // (tiles of 64 x 128 a CU: see the forms)
   const double quarters = std::ceil(P / 64) * std::ceil(main_f / 128) / 256;
   const bool frag = frag_ok(a) && !(nine && quarters > 3 && quarters <= 4);
   const Form* best = nullptr;
