@@ -83,7 +83,7 @@ struct DirectArgs {
 template <typename T, typename OutT, int BT, int TM, int TN, int KG, bool UNI, int D>
 __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a) {
   // Three-way bf16 splits (split.hpp) where two filter blocks share a split of the pixels and there are waves to hide it:
-  // 6x58x78x64 -> 128 at stride 2 17.2 -> 14.3 us, 16x28x28x128 -> 256 24.8 -> 19.9.  32 x 32 waves spend as long splitting as they
+  // 6x58x78x64 -> 128 at stride 2 15.9 -> 14.1 us, 16x28x28x128 -> 256 24.5 -> 21.2.  32 x 32 waves spend as long splitting as they
   // save (0.83 to 1.11 times), 64 x 64 ones are alone on their SIMD (0.91).
   constexpr bool kSplit = sizeof(T) == 4 && BT == 32 && TM == 2 && TN == 1;
   constexpr int kEs = sizeof(T), LG = 64 / BT, NQ = BT / 8, GL = BT * TN / 8;  // GL: pixel loads of a round

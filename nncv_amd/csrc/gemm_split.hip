@@ -241,9 +241,11 @@ void launch_cfg(const float* A, const float* B, const float* C, float* D, int M,
 // The forms, and what a launch of each takes:
 //   us = fixed + x (round_us * rounds of a wave + tile_us) + turns (turn_round_us * rounds of a wave + turn_us)
 // with x = tiles / 256 CUs and turns = ceil(x / workgroups that a CU holds): the matrix pipes' share, and a workgroup's own length.
-// Least-squares fits over 115 shapes of 30 MFLOP to 137 GFLOP, within 4-8 % of the times; the form they choose, or the fp32
-// instructions where those are the sooner ones, takes 3 % longer than the best one on average and 15 % less than the fp32 ones.
-//   1024^3 23.9 -> 16.4 us (131 TFLOP/s), 1500x1001x777 31.6 -> 24.3, 4096^3 960 -> 726 (189 TFLOP/s), 676x1382x829 21.3 -> 15.6
+// Least-squares fits over 115 shapes of 30 MFLOP to 137 GFLOP, within 4-8 % of the times without the scaling of the operands, which
+// made the 64 x 64 forms 6 to 11 % and the others 2 to 3 % longer.  The choice between these and the fp32 instructions holds all the
+// same: over 70 shapes of 60 MFLOP to 80 GFLOP it takes 0.4 % longer than the sooner one on average (4 % at most), the fp32 ones 8.7 %.
+//   fp32 instructions -> these: 1024^3 20.8 -> 16.7 us (129 TFLOP/s), 1500x1001x777 27.4 -> 23.3, 4096^3 965 -> 789 (174 TFLOP/s),
+//   676x1382x829 18.8 -> 16.0
 struct Form {
   int rows, cols, kg, resident;
   double fixed_us, round_us, tile_us, turn_round_us, turn_us;

@@ -317,8 +317,8 @@ void launch_fast_typed(const IgemmArgs& a, hipStream_t s) {
     else if (blocks(64, 64) >= 128 || a.F % 32 != 0) pick = 4;
     else pick = 5;  // fewer than 128 workgroups of 64x64: halve the filter blocks
   }
-  // fp32 blocks without K groups: on the bf16 matrix pipes from 32 k on (1.17 times at 64, 1.3 at 144, 1.4 to 1.6 at 400; the 7x7
-  // stem of 6x224x303 40.3 -> 30.8 us); a single step of 16 is bound by memory (55x9x90x16 -> 128 10.5 against 10.9).  Blocks with K
+  // fp32 blocks without K groups: on the bf16 matrix pipes from 32 k on (1.05 to 1.09 times at 32, 1.17 at 64, 1.28 at 144, 1.38 at 400; the 7x7
+  // stem of 6x224x303 40.3 -> 31.9 us); a single step of 16 is bound by memory (55x9x90x16 -> 128 10.5 against 10.9).  Blocks with K
   // groups have as many waves as their steps, and wait for memory.
   if constexpr (sizeof(T) == 4) {
     if (pick <= 2 && a.R * a.S * a.C >= 32) {

@@ -11,8 +11,9 @@
 //
 // Range.  bf16 ends at 2^-133 (its normal numbers at 2^-126), fp32 at 2^-149: what is split is 2^24 times the value, so that every piece
 // of every fp32 value is a normal number, and a sum is 2^48 times what it is worth.  (Unscaled, the error of a sum of products of one
-// operand at 2^-112 was 2.6e-7, at 2^-118 1.8e-5, at 2^-126 2.4e-3.)  The two multiplications for a pair of values cost 1.7 % of a
-// classification of six photographs (368.1 -> 374.3 us), 2 to 6 % of a product (1500x1001x777 22.6 -> 23.0, 4096^3 758 -> 796).  To look
+// operand at 2^-112 was 2.6e-7, at 2^-118 1.8e-5, at 2^-126 2.4e-3.)  The two multiplications for a pair of values cost what a kernel's
+// vector instructions bound: 2 to 11 % of a product (1024^3 14.9 -> 16.6 us, 1500x1001x777 22.7 -> 23.2, 4096^3 772 -> 817), 8 % of
+// the 64 x 32 form of conv_direct, 2 to 7 % of igemm_fast's, 0 to 3 % of conv3x3_split, 1.7 % of a classification of six photographs.  To look
 // for pieces that lose bits instead (an or for a pair) was slower: its register made the 64 x 64 products spill (4096^3 1142).
 //
 // What is not finite.  An infinity has a NaN for its second piece, and so has a value from 2^103 on, which 2^24 takes to infinity; a sum
