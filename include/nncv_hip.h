@@ -209,7 +209,9 @@ unsigned long long nncv_hip_plan_arena(int n, const int* first_op, const int* la
                                        unsigned long long align, unsigned long long* offsets);
 
 /* C += A.B, fp32 row-major, DEVICE pointers, any M, N, K >= 1 (the device form of _mlir_ciface_matmul;
- * tests/MatMulOptimization/MatMulDeafult.mlir:11-21). */
+ * tests/MatMulOptimization/MatMulDeafult.mlir:11-21).  fp32 values of any size, in and out.  Products of large K, like the fp32
+ * layers of this library, may run on the bf16 matrix pipes, three pieces to a value: the error of a sum of ordinary products is smaller than that of
+ * fp32 instructions, and a call whose operands or results are not finite, or above 2^80 or so, takes up to four times the usual. */
 int nncv_hip_matmul_f32(const float* A, const float* B, float* C, int M, int N, int K, void* stream);
 /* Measurement helper, like nncv_hip_conv_time: `reps` launches of C += A.B back to back on `stream` between one pair
  * of HIP events (after 5 untimed ones); *avg_us = elapsed / reps.  C keeps accumulating. */
