@@ -770,7 +770,7 @@ bool conv3x3_stream_applicable(const IgemmArgs& a, int in_dt, int out_dt) {
   // blocks.  Stream / patch us: 1x28x28x128 5.7 / 4.9, 4x28x28x128 5.9 / 5.0, 8x14x14x256 7.9 / 6.3, 9x10x10x128 -> 320 (90 blocks) 5.4 / 4.8,
   // 27x8x8x448 -> 256 (128) 9.4 / 8.0; just above the line 46x10x10x64 -> 96 (129) 4.4 / 4.9, 44x5x31x256 -> 64 (132) 6.8 / 7.6,
   // 7x13x17x256 -> 320 (140) 6.9 / 7.9, and further up 8x28x28x128 5.9 / 6.3, 16x14x14x256 7.9 / 8.6, 4x56x56x64 4.9 / 5.4 (216-224
-  // blocks).  Of 13 layers of up to 256 channels from 129 to 143 blocks all are 1.10 to 1.14 times as fast here.  Rows of 80 pixels fill 80
+  // blocks).  Of 10 layers of up to 256 channels from 129 to 143 blocks all are 1.10 to 1.14 times as fast here.  Rows of 80 pixels fill 80
   // of a tile's 128 slots: 16x80x80x64 18.2 / 15.7, where the patch kernel cuts the rows into column tiles.
   const long long fine_wgs = (long long)c.geo.n_tiles * (a.F / 32);
   // With three or more passes in flight (overlap_hint) a ReLU layer whose filter count rules out the 128-filter form goes
@@ -779,15 +779,17 @@ bool conv3x3_stream_applicable(const IgemmArgs& a, int in_dt, int out_dt) {
   // layer, whose 64-filter form keeps the weights in registers (204.4 k images/s with layer1 on the patch kernel,
   // 212.6 k here, same box).
   if (!all && overlap_hint() >= 3 && a.relu <= kActRelu && c.WF != 4 && !(a.C == 64 && c.WF == 2 && c.PG == 1)) return false;
-  // From five slabs up: of 37 layers of 320 to 512 channels from 129 to 325 blocks 35 are 1.01 to 1.7 times as fast here (32x7x7x512
+  // From five slabs up: of 34 layers of 320 to 512 channels from 129 to 325 blocks 32 are 1.01 to 1.7 times as fast here (32x7x7x512
   // 12.6 -> 11.6 us, 35x14x14x512 -> 96 18.2 -> 10.6, 17x20x20x320 -> 160 13.8 -> 11.7; 38x8x8x320 -> 192 6.8 against 7.8 and 61x10x10x384 -> 128
   // 10.3 against 10.7 are the other two), and 30 from 320 on 1.04 to 1.5 times (256x7x7x512 79.4 -> 62.0, 64x14x14x512 74.4 -> 58.5).
-  // In a pass of ResNet-18 over 32 images, whose layer4 has 256 blocks, 250.9 -> 244.6 us.  With passes in flight the line lies at
-  // 320: other passes fill the CUs that the patch kernel leaves, and it takes less of them.  Four in flight, us a round, stream / patch:
-  // 24 images (192 blocks) 509 / 469, 32 (256) 602 / 590, 40 (320) 715 / 717, 48 842 / 864, 64 1083 / 1129.
+  // In a pass of ResNet-18 over 32 images, whose layer4 has 256 blocks, 250.9 -> 244.6 us.
+  // With passes in flight other passes fill the CUs that the patch kernel leaves, and it takes less of them: the lines lie at 144 and,
+  // from five slabs up, 320.  Four in flight, us a round, stream / patch on the layers in question: 5 images (layer2 140 blocks) 191 / 185, 6
+  // (168) 201 / 198, 10 (layer3 136) 267 / 258, 9 to 23 with layer2 and layer3 above the line 243 / 251 to 461 / 474; layer4 at 24 images (192
+  // blocks) 509 / 469, 32 (256) 602 / 590, 40 (320) 715 / 717, 48 842 / 864, 64 1083 / 1129.
   // A tile of 96 slots is too few there: 174x19x6x384 74 against 62.
   const bool deep = a.C > 256;
-  return all || (fine_wgs >= (deep && overlap_hint() >= 3 ? 320 : 129) && c.geo.TH * a.W >= (deep ? 100 : 96));
+  return all || (fine_wgs >= (overlap_hint() < 3 ? 129 : deep ? 320 : 144) && c.geo.TH * a.W >= (deep ? 100 : 96));
 }
 
 template <int PG, int WF, int WK, bool ACT, bool RES = false>

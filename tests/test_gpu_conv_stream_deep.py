@@ -33,3 +33,25 @@ def test_deep_layers_and_tiles_of_several_images(case):
         abi.profile_enable(False)
     assert tags == ["conv3x3_stream<f16,%s>" % form]
     assert rel_l2(got, want) < 4e-4  # half an ulp of eleven bits, 2.8e-4 in the mean over a binade
+
+
+# with passes in flight the lines are 144 blocks and, from five slabs on, 320: below them the patch kernel
+@pytest.mark.parametrize("case", [(5, 28, 28, 128, 128, "conv3x3_patch<f16,1,4>"), (32, 7, 7, 512, 512, "conv3x3_patch<f16,1,4>"),
+                                  (6, 28, 28, 128, 128, "conv3x3_stream<f16,1x4x1>"), (41, 7, 7, 512, 512, "conv3x3_stream<f16,1x4x1>")],
+                         ids=lambda c: "x".join(map(str, c[:5])))
+def test_lines_with_passes_in_flight(case):
+    N, H, W, C, F, tag = case
+    g = torch.Generator().manual_seed(N)
+    x, w = torch.randn((N, C, H, W), generator=g).half().float(), (torch.randn((F, C, 3, 3), generator=g) * (2.0 / (9 * C)) ** 0.5).half().float()
+    try:
+        abi.check(abi.lib().nncv_hip_set_overlap_hint(4))
+        layer, xd = Conv(abi.F16, w.numpy(), 1, 1, relu=True), dev(nhwc(x.numpy()), abi.F16)
+        abi.profile_enable(True)
+        abi.profile_report()
+        got = nchw(host(layer(xd, abi.NHWC)))
+        tags = list(abi.profile_report())
+    finally:
+        abi.profile_enable(False)
+        abi.check(abi.lib().nncv_hip_set_overlap_hint(1))
+    assert tags == [tag]
+    assert rel_l2(got, torch.relu(torch.nn.functional.conv2d(x.double(), w.double(), padding=1)).numpy()) < 4e-4
