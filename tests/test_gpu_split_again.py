@@ -4,8 +4,9 @@ import numpy as np
 import pytest
 import torch
 
-from nncv_amd import abi
-from gpu_util import Conv, dev, host, nchw, nhwc
+import oracle
+from nncv_amd import abi, synth
+from gpu_util import Conv, Model, dev, host, max_rel, nchw, nhwc
 from test_gpu_conv3x3_split import CASES
 from test_gpu_gemm_split import SHAPES, operands, product
 
@@ -101,3 +102,24 @@ def test_a_layer_of_nan_is_not_much_slower(case):
     xd.fill_(float("nan"))
     assert microseconds(call) < SLOWEST * usual
     assert torch.isnan(out).all()
+
+
+def test_a_network_whose_sums_are_large():
+    """An fp32 ResNet-18 with one pixel of 3e31: the sums around it are above 2^80 from the first layer on, so every kernel on the bf16 pipes, the
+    shortcuts inside the stride-2 layers among them, takes them again; against the oracle, image by image."""
+    blob = synth.resnet18_params()
+    x = synth.uniform(77, (6, 3, 231, 309), 0.0, 1.0)
+    x[2, 1, 100, 140] = 3e31
+    m = Model(blob, abi.F32)
+    abi.profile_enable(True)
+    try:
+        abi.profile_report()
+        got = host(m(dev(x, abi.F32)))
+        tags = abi.profile_report()
+    finally:
+        abi.profile_enable(False)
+    assert tags["conv3x3_direct<f32,64x32,splitk4>"]["launches"] == 2 and any(t.startswith("conv3x3_split<") for t in tags), list(tags)
+    want = oracle.hwp_resnet18_forward(x, blob)
+    assert np.isfinite(want).all() and np.abs(want[2]).max() > 2.0 ** 100
+    for i in range(6):
+        assert max_rel(got[i], want[i]) < 1e-5  # 20 layers of fp32 sums, each off by 1e-6 of its largest at most; 3e-7 where none is taken again
