@@ -344,11 +344,13 @@ size_t weight_frag3x3_bytes(int dt, int F, int C);
 void launch_weight_frag3x3(const void* w, int w_dt, void* dst, int dst_dt, int F, int C, hipStream_t s);
 // 1x1 weights [F][C] in the same order with one tap per slab (IgemmArgs::aux_wt_frag)
 void launch_weight_frag1x1(const void* w, int w_dt, void* dst, int dst_dt, int F, int C, hipStream_t s);
-// stem weights [64,3,7,7] -> [64][7][4][8] over (pixel-pair, channel4); pair sp / pixel p holds
-// filter column 2*sp + p - col_shift (zero outside 0..6)
-void launch_stem_weight(const void* w, int w_dt, void* dst, int dst_dt, int F, int col_shift, hipStream_t s);
+// stem weights [F,3,7,7] -> [F][7][4][8] over (pixel-pair, channel4); pair sp / pixel p holds
+// filter column 2*sp + p (zero outside 0..6)
+void launch_stem_weight(const void* w, int w_dt, void* dst, int dst_dt, int F, hipStream_t s);
 // fused stem: conv7x7 s2 p3 + scale/shift + ReLU + maxpool 3x3 s2 p1, NCHW fp16 in, NHWC out
-// (stem_pool.hip); wt in the col_shift = 1 layout above
+// (stem_pool.hip); wt: the 64 fp16 filters as launch_stem_weight_strip lays them out
+size_t stem_weight_strip_bytes();
+void launch_stem_weight_strip(const void* w, void* dst, hipStream_t s);
 bool stem_pool_applicable(int dt, int N, int H, int W, int F);
 void launch_stem_pool(const void* in, const void* wt, const float* scale, const float* shift, void* out, int N, int H, int W,
                       hipStream_t s);

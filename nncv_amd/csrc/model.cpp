@@ -46,7 +46,8 @@ ConvLayer::Sizes ConvLayer::sizes(const Desc& d, int algo, bool bn) {
   const int Cp = round_up(d.C, d.dt == kF16 ? 8 : 4), Fp = round_up(d.F, 4), RS = d.R * d.S;
   Sizes z{};
   if (d.stem) {
-    z.wt = z.wt_shift = (size_t)d.F * 224 * es;
+    z.wt = (size_t)d.F * 224 * es;
+    if (d.dt == kF16 && d.F == 64) z.wstrip = stem_weight_strip_bytes();
     z.wflat = weight_flat_bytes(d.dt, d.F, 7, 32);
   } else if (algo == kAlgoWinograd) {
     z.U = (size_t)36 * d.F * d.C * es;
@@ -65,7 +66,7 @@ ConvLayer::Sizes ConvLayer::sizes(const Desc& d, int algo, bool bn) {
 size_t ConvLayer::device_bytes(const Desc& d, bool bn) {
   const Sizes z = sizes(d, pick_algo(d), bn);
   size_t total = 0;
-  for (const size_t b : {z.wt, z.wflat, z.wfrag, z.wfrag32, z.U, z.wt_shift, z.scale, z.scale}) total += align256(b);
+  for (const size_t b : {z.wt, z.wflat, z.wfrag, z.wfrag32, z.U, z.wstrip, z.scale, z.scale}) total += align256(b);
   return total;
 }
 
@@ -85,15 +86,15 @@ ConvLayer::ConvLayer(const Desc& d, const void* w, const void* gamma, const void
   wfrag_.reset(z.wfrag, d.pool);
   wfrag32_.reset(z.wfrag32, d.pool);
   U_.reset(z.U, d.pool);
-  wt_shift_.reset(z.wt_shift, d.pool);
+  wstrip_.reset(z.wstrip, d.pool);
   scale_.reset(z.scale, d.pool);
   shift_.reset(z.scale, d.pool);
 
   const int Cp = round_up(d.C, d.dt == kF16 ? 8 : 4), Fp = round_up(d.F, 4);
   if (d.stem) {
-    launch_stem_weight(w, d.dt, wt_.get(), d.dt, d.F, 0, s);
+    launch_stem_weight(w, d.dt, wt_.get(), d.dt, d.F, s);
     launch_weight_flat_rows(wt_.get(), wflat_.get(), d.dt, d.F, 224, s);
-    launch_stem_weight(w, d.dt, wt_shift_.get(), d.dt, d.F, 1, s);  // pairs start one column further left (fused stem)
+    if (z.wstrip) launch_stem_weight_strip(w, wstrip_.get(), s);
   } else if (algo_ == kAlgoWinograd) {
     launch_wino43_filter(w, d.dt, U_.get(), d.dt, d.F, d.C, s);
   } else {
@@ -161,7 +162,7 @@ void ConvLayer::forward(const void* in, int N, int H, int W, const void* residua
 
 bool ConvLayer::forward_stem_pool(const void* in, int N, int H, int W, void* pooled_out, hipStream_t s) const {
   if (!d_.stem || d_.relu != kActRelu || !stem_pool_applicable(d_.dt, N, H, W, d_.F)) return false;
-  launch_stem_pool(in, wt_shift_.get(), scale_.as<float>(), shift_.as<float>(), pooled_out, N, H, W, s);
+  launch_stem_pool(in, wstrip_.get(), scale_.as<float>(), shift_.as<float>(), pooled_out, N, H, W, s);
   return true;
 }
 

@@ -59,13 +59,13 @@ class ConvLayer {
 
  private:
   // bytes of each array a layer keeps, 0: not kept
-  struct Sizes { size_t wt, wflat, wfrag, wfrag32, U, wt_shift, scale; };
+  struct Sizes { size_t wt, wflat, wfrag, wfrag32, U, wstrip, scale; };
   static Sizes sizes(const Desc& d, int algo, bool bn);
   static int pick_algo(const Desc& d);
 
   Desc d_;
   int algo_;
-  DeviceBuffer wt_, wfrag_, wfrag32_, wflat_, U_, scale_, shift_, wt_shift_;
+  DeviceBuffer wt_, wfrag_, wfrag32_, wflat_, U_, scale_, shift_, wstrip_;
   DeviceBuffer wt_cat_, scale_cat_, shift_cat_;  // this layer's filters followed by the fused shortcut's
   const void* aux_wflat_ = nullptr;  // the fused shortcut layer's own wflat_
   DeviceBuffer aux_wfrag_;  // the fused shortcut's filters alone, fragment-major (stride-2 patch kernel)
