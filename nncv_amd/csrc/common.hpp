@@ -347,13 +347,17 @@ void launch_weight_frag1x1(const void* w, int w_dt, void* dst, int dst_dt, int F
 // stem weights [F,3,7,7] -> [F][7][4][8] over (pixel-pair, channel4); pair sp / pixel p holds
 // filter column 2*sp + p (zero outside 0..6)
 void launch_stem_weight(const void* w, int w_dt, void* dst, int dst_dt, int F, hipStream_t s);
-// fused stem: conv7x7 s2 p3 + scale/shift + ReLU + maxpool 3x3 s2 p1, NCHW fp16 in, NHWC out
-// (stem_pool.hip); wt: the 64 fp16 filters as launch_stem_weight_strip lays them out
+// fused stem: conv7x7 s2 p3 + scale/shift + ReLU + maxpool 3x3 s2 p1, NCHW in, NHWC out
+// (fp16: stem_pool.hip, fp32: stem_pool_split.hip); wt: the 64 filters as launch_stem_weight_strip(_split) lays them out
 size_t stem_weight_strip_bytes();
 void launch_stem_weight_strip(const void* w, void* dst, hipStream_t s);
+size_t stem_weight_strip_split_bytes();
+void launch_stem_weight_strip_split(const void* w, void* dst, hipStream_t s);
 bool stem_pool_applicable(int dt, int N, int H, int W, int F);
 void launch_stem_pool(const void* in, const void* wt, const float* scale, const float* shift, void* out, int N, int H, int W,
                       hipStream_t s);
+void launch_stem_pool_split(const void* in, const void* wt, const float* scale, const float* shift, void* out, int N, int H, int W,
+                            hipStream_t s);
 // BN fold: scale = gamma / sqrt(var + eps), shift = beta - mean*scale (fp32 out)
 void launch_bn_fold(const void* gamma, const void* beta, const void* mean, const void* var, int dt, float* scale,
                     float* shift, int C, hipStream_t s, float eps = 1e-5f);

@@ -47,7 +47,7 @@ ConvLayer::Sizes ConvLayer::sizes(const Desc& d, int algo, bool bn) {
   Sizes z{};
   if (d.stem) {
     z.wt = (size_t)d.F * 224 * es;
-    if (d.dt == kF16 && d.F == 64) z.wstrip = stem_weight_strip_bytes();
+    if (d.F == 64) z.wstrip = d.dt == kF16 ? stem_weight_strip_bytes() : stem_weight_strip_split_bytes();
     z.wflat = weight_flat_bytes(d.dt, d.F, 7, 32);
   } else if (algo == kAlgoWinograd) {
     z.U = (size_t)36 * d.F * d.C * es;
@@ -94,7 +94,7 @@ ConvLayer::ConvLayer(const Desc& d, const void* w, const void* gamma, const void
   if (d.stem) {
     launch_stem_weight(w, d.dt, wt_.get(), d.dt, d.F, s);
     launch_weight_flat_rows(wt_.get(), wflat_.get(), d.dt, d.F, 224, s);
-    if (z.wstrip) launch_stem_weight_strip(w, wstrip_.get(), s);
+    if (z.wstrip) (d.dt == kF16 ? launch_stem_weight_strip : launch_stem_weight_strip_split)(w, wstrip_.get(), s);
   } else if (algo_ == kAlgoWinograd) {
     launch_wino43_filter(w, d.dt, U_.get(), d.dt, d.F, d.C, s);
   } else {
@@ -162,7 +162,7 @@ void ConvLayer::forward(const void* in, int N, int H, int W, const void* residua
 
 bool ConvLayer::forward_stem_pool(const void* in, int N, int H, int W, void* pooled_out, hipStream_t s) const {
   if (!d_.stem || d_.relu != kActRelu || !stem_pool_applicable(d_.dt, N, H, W, d_.F)) return false;
-  launch_stem_pool(in, wstrip_.get(), scale_.as<float>(), shift_.as<float>(), pooled_out, N, H, W, s);
+  (d_.dt == kF16 ? launch_stem_pool : launch_stem_pool_split)(in, wstrip_.get(), scale_.as<float>(), shift_.as<float>(), pooled_out, N, H, W, s);
   return true;
 }
 

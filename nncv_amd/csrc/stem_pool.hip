@@ -374,8 +374,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
 bool stem_pool_applicable(int dt, int N, int H, int W, int F) {
   static const bool off = getenv("NNCV_HIP_NO_STEM_FUSION") != nullptr;
-  return !off && dt == kF16 && F == 64 && H >= 7 && W >= 7 && (long long)N * 3 * H * W * 2 < (long long)kOOBs &&
-         (long long)N * ((H + 3) / 4) * ((W + 3) / 4) * 128 < (long long)kOOBs;  // image and pooled tensor within a buffer descriptor's range check
+  return !off && F == 64 && H >= 7 && W >= 7 && (long long)N * 3 * H * W * (long long)dtype_size(dt) < (long long)kOOBs &&
+         (long long)((W + 3) / 4) * 256 < (long long)kOOBs;  // the image and a pooled row within a buffer descriptor's range check
 }
 
 size_t stem_weight_strip_bytes() { return kWtBytes; }
