@@ -80,7 +80,8 @@ struct DirectArgs {
 };
 
 // UNI: a tap is a whole number of rounds (C elements = whole 128-byte lines), so the tap of a round is the same for all lanes
-template <typename T, typename OutT, int BT, int TM, int TN, int KG, bool UNI, int D>
+// BEHIND: a workgroup takes its tile's auxiliary filters behind it, over the same pixels; there are no workgroups for them
+template <typename T, typename OutT, int BT, int TM, int TN, int KG, bool UNI, int D, bool BEHIND>
 __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a) {
   // Three-way bf16 splits (split.hpp) where two filter blocks share a split of the pixels and there are waves to hide it:
   // 6x58x78x64 -> 128 at stride 2 15.9 -> 14.1 us, 16x28x28x128 -> 256 24.5 -> 21.2.  32 x 32 waves spend as long splitting as they
@@ -110,10 +111,14 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
     tf = __builtin_amdgcn_readfirstlane(tf);
     tp = __builtin_amdgcn_readfirstlane(tp);
   }
-  const bool aux = tf >= a.main_tiles;
-  const int f0 = aux ? a.main_f + (tf - a.main_tiles) * BT * TM : tf * BT * TM, p0 = tp * BT * TN;
-  const int f_end = aux ? a.F : a.main_f;
+  const int p0 = tp * BT * TN;
   const __amdgpu_buffer_rsrc_t rs_in = make_rsrc(a.in, a.in_bytes);
+  int base[GL], iy0[GL], ix0[GL];
+  u32x4 w[D][NQ][TM], gx[D][GL];
+  for (int pass = 0;; ++pass, tf += a.main_tiles) {
+  const bool aux = tf >= a.main_tiles;
+  const int f0 = aux ? a.main_f + (tf - a.main_tiles) * BT * TM : tf * BT * TM;
+  const int f_end = aux ? a.F : a.main_f;
   const __amdgpu_buffer_rsrc_t rs_wt = aux ? make_rsrc(a.aux_wt, a.aux_wt_bytes) : make_rsrc(a.wt, a.wt_bytes);
 
   // rounds of this group; an auxiliary tile walks the rounds of its tap (UNI)
@@ -134,15 +139,16 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
 #pragma unroll
     for (int i = 0; i < TM; ++i) w[q][i] = __builtin_amdgcn_raw_buffer_load_b128(rs_wt, ((f0 + BT * i < f_end) & (r < re)) ? woff[i] + at : kOOBd, 0, 0);
   };
-  u32x4 w[D][NQ][TM];  // the first ones are asked for now: their addresses are there long before the pixels'
+  // the first ones are asked for now: their addresses are there long before the pixels' (those of the second pass are on their way)
+  if (pass == 0) {
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) load_w(rb, q, w[0]);
+    for (int q = 0; q < NQ; ++q) load_w(rb, q, w[0]);
+  }
   __builtin_amdgcn_sched_barrier(0);
 
   // pixels: this lane loads chunk lane % 8 of the rows lane / 8, + 8, ...; pixels past the end read the last one (not stored)
   // (worked out once per row, a lane each, and handed round through the LDS buffer that is still empty)
-  int base[GL], iy0[GL], ix0[GL];
-  {
+  if (pass == 0) {
     static_assert(BT * TN <= 64, "a lane per pixel row");
     int rem, ox;
     const int n = fast_div(min(p0 + lane, a.P - 1), a.OHW, a.inv_ohw, &rem);
@@ -169,17 +175,20 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
     dr = fast_div(tap, a.S, a.inv_s, &ds);
   }
   int rload = rb;
-  u32x4 gx[D][GL];
+  auto step_tap = [&]() __attribute__((always_inline)) {
+    uc += dc;
+    us += ds;
+    ur += dr;
+    if (uc >= a.cpt) uc -= a.cpt, ++us;
+    if (us >= a.S) us -= a.S, ++ur;
+    rload += KG;
+  };
   auto load_x = [&](u32x4 (&gx)[GL]) __attribute__((always_inline)) {
     int r = ur, s = us, at;
     bool in_k = rload < re;
     if constexpr (UNI) {
       at = ((ur * a.W + us) * a.pix) * kEs + uc * 16;
-      uc += dc;
-      us += ds;
-      ur += dr;
-      if (uc >= a.cpt) uc -= a.cpt, ++us;
-      if (us >= a.S) us -= a.S, ++ur;
+      step_tap();
     } else {
       const int kc = 8 * rload + (lane & 7);
       int c;
@@ -187,8 +196,8 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
       r = fast_div(tap, a.S, a.inv_s, &s);
       at = ((r * a.W + s) * a.pix) * kEs + c * 16;
       in_k &= kc < a.chunks;
+      rload += KG;
     }
-    rload += KG;
 #pragma unroll
     for (int g = 0; g < GL; ++g) {
       const bool ok = in_k & ((unsigned)(iy0[g] + r) < (unsigned)a.H) & ((unsigned)(ix0[g] + s) < (unsigned)a.W);
@@ -215,7 +224,8 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
         acc[i][j][v] = 0.0f;
         if constexpr (kSplit) low[i][j][v] = 0.0f;
       }
-  load_x(gx[0]);
+  if (pass == 0) load_x(gx[0]);
+  else step_tap();
 #pragma unroll
   for (int d = 1; d < D; ++d) {
     __builtin_amdgcn_sched_barrier(0);  // (the first requests leave before the addresses of the others are there)
@@ -353,6 +363,28 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
     }
   }
 
+  if constexpr (BEHIND) {
+    static_assert(UNI && D == 1, "one round of the second pass is asked for here, of one tap");
+    if (pass == 0) {  // under the sums and their stores
+      const int ur = fast_div(a.aux_tap, a.S, a.inv_s, &us), r = grp, at = ((ur * a.W + us) * a.pix) * kEs + 8 * grp * 16;
+      const __amdgpu_buffer_rsrc_t rs_aux = make_rsrc(a.aux_wt, a.aux_wt_bytes);
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int f = tf * BT * TM + BT * i;
+        const unsigned fb = (unsigned)(f >> 5) * (unsigned)(rpt * 4);
+        const unsigned off = BT == 32 ? (fb * 64u + lane) * 16u : ((fb + (lh >> 1)) * 64u + (lh & 1) * 32u + (f & 16) + lrow) * 16u;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+          w[0][q][i] = __builtin_amdgcn_raw_buffer_load_b128(rs_aux, ((a.main_f + f < a.F) & (r < rpt)) ? off + (unsigned)(4 * r + (BT == 32 ? q : 2 * q)) * 1024u : kOOBd, 0, 0);
+      }
+#pragma unroll
+      for (int g = 0; g < GL; ++g) {
+        const bool ok = (r < rpt) & ((unsigned)(iy0[g] + ur) < (unsigned)a.H) & ((unsigned)(ix0[g] + us) < (unsigned)a.W);
+        gx[0][g] = __builtin_amdgcn_raw_buffer_load_b128(rs_in, ok ? (unsigned)(base[g] + at) : kOOBd, 0, 0);
+      }
+    }
+  }
+
   auto quad_sum = [&](int k) {
     const int blk = k / kQuadsPerBlock, g4 = k % kQuadsPerBlock;
     floatx4 s;
@@ -382,6 +414,9 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
       finish(mine[k], v[0]);
     }
   }
+  if (!BEHIND || pass == 1) break;
+  if constexpr (KG > 1) __syncthreads();  // every sum has been read: LDS holds pixels again
+  }
 }
 
 template <typename T, typename OutT, int BT, int TM, int TN, int KG>
@@ -390,6 +425,11 @@ void launch_cfg(DirectArgs d, hipStream_t s) {
   d.main_tiles = (d.main_f + BT * TM - 1) / (BT * TM);
   d.tiles_f = d.main_tiles + (d.F - d.main_f + BT * TM - 1) / (BT * TM);
   d.tiles_p = (d.P + BT * TN - 1) / (BT * TN);
+  // Auxiliary filters, as many as the convolution's own: behind them in the same workgroups where those alone are for most of the CUs;
+  // on their own they start late and their pixels come from memory again.  Six images, us: 58x78x64 -> 128 + 128 26.0 -> BEHIND1,
+  // 29x39x128 -> 256 + 256 21.8 -> BEHIND2, 15x20x256 -> 512 + 512 29.0 -> BEHIND3.
+  const bool behind = sizeof(T) == 4 && d.cpt % 8 == 0 && d.F == 2 * d.main_f && (long long)d.main_tiles * d.tiles_p >= 200;
+  if (behind) d.tiles_f = d.main_tiles;
   d.inv_tiles = 1.0f / (float)(d.pixels_first ? d.tiles_p : d.tiles_f);
   auto go = [&](auto kern) {
     static const bool attr = [&] {
@@ -400,8 +440,8 @@ void launch_cfg(DirectArgs d, hipStream_t s) {
     launch_kernel(kern, dim3((unsigned)((long long)d.tiles_f * d.tiles_p)), dim3(64 * KG), lds, s, d);
   };
   auto depth = [&](auto dc) {
-    if (d.cpt % 8 == 0) go(conv_direct_kernel<T, OutT, BT, TM, TN, KG, true, decltype(dc)::value>);
-    else go(conv_direct_kernel<T, OutT, BT, TM, TN, KG, false, decltype(dc)::value>);
+    if (d.cpt % 8 == 0) go(conv_direct_kernel<T, OutT, BT, TM, TN, KG, true, decltype(dc)::value, false>);
+    else go(conv_direct_kernel<T, OutT, BT, TM, TN, KG, false, decltype(dc)::value, false>);
   };
   // Three rounds of operands in flight for fp16 walks of nine rounds a wave and more, up to two workgroups a CU: the weights of a
   // pass over one image come from beyond L2 (7x7x512 in such a pass: 8.1 -> 6.9 us, the pass 104.3 -> 101.2; alone, from L2, 6.4 either
@@ -410,6 +450,12 @@ void launch_cfg(DirectArgs d, hipStream_t s) {
   if constexpr (sizeof(T) == 2 && BT == 16) {
     if ((d.chunks + 7) / 8 >= 9 * KG && (long long)d.tiles_f * d.tiles_p <= 512) {
       depth(std::integral_constant<int, 3>());
+      return;
+    }
+  }
+  if constexpr (sizeof(T) == 4) {
+    if (behind) {
+      go(conv_direct_kernel<T, OutT, BT, TM, TN, KG, true, 1, true>);
       return;
     }
   }
