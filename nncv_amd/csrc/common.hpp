@@ -226,6 +226,8 @@ bool igemm_takes_direct(const IgemmArgs& a, int in_dt, int out_dt);
 // 3x3 pad-1 layers at stride 1, or 2 in fp16: direct convolution with the haloed input patch resident in LDS
 // (conv3x3_patch.hip); same arguments and epilogue as the igemm kernels.
 bool conv3x3_patch_applicable(const IgemmArgs& a, int in_dt);
+// us that the fp32 kernel takes in tiles of 32 consecutive pixels, 0: it does not (conv3x3_split.hip)
+double conv3x3_split_flat_us(int N, int H, int W, int C, int F);
 // The tile plan that kernel would use for N x OH x OW output pixels, F filters and `slabs` 128-byte
 // channel slabs: out = {WS, TN, TH, TW, NTX, rw_log, LDS cells available, loader coverage}.  Host
 // arithmetic only (no device needed); false = no plan.

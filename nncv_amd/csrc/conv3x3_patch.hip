@@ -722,6 +722,8 @@ void launch_conv3x3_patch(const IgemmArgs& g, int in_dt, int out_dt, hipStream_t
     else if (ws == 2) launch_patch_cfg<half_t, half_t, 2, 2, 2>(a, flops, bytes, "conv3x3_patch<f16,2,2>", s);
     else if (halves) launch_patch_cfg<half_t, half_t, 1, 4, 1>(a, flops, bytes, "conv3x3_patch<f16,1,4,half>", s);
     else launch_patch_cfg<half_t, half_t, 1, 4, 2>(a, flops, bytes, "conv3x3_patch<f16,1,4>", s);
+  } else if (conv3x3_split_flat_us(a.N, a.H, a.W, a.C, a.F) > 0) {
+    launch_conv3x3_split_flat(a, flops, bytes, s);
   } else {
     launch_conv3x3_split(a, ws, halves, ws == 4 ? "conv3x3_split<f32,4,1>" : ws == 2 ? "conv3x3_split<f32,2,2>" : halves ? "conv3x3_split<f32,1,4,half>" : "conv3x3_split<f32,1,4>",
                          flops, bytes, s);

@@ -426,8 +426,8 @@ void launch_cfg(DirectArgs d, hipStream_t s) {
   d.tiles_f = d.main_tiles + (d.F - d.main_f + BT * TM - 1) / (BT * TM);
   d.tiles_p = (d.P + BT * TN - 1) / (BT * TN);
   // Auxiliary filters, as many as the convolution's own: behind them in the same workgroups where those alone are for most of the CUs;
-  // on their own they start late and their pixels come from memory again.  Six images, us: 58x78x64 -> 128 + 128 26.0 -> BEHIND1,
-  // 29x39x128 -> 256 + 256 21.8 -> BEHIND2, 15x20x256 -> 512 + 512 29.0 -> BEHIND3.
+  // on their own they start late and their pixels come from memory again.  Six images, us: 58x78x64 -> 128 + 128 26.0 -> 21.8,
+  // 29x39x128 -> 256 + 256 21.8 -> 19.6, 15x20x256 -> 512 + 512 29.0 -> 19.6.
   const bool behind = sizeof(T) == 4 && d.cpt % 8 == 0 && d.F == 2 * d.main_f && (long long)d.main_tiles * d.tiles_p >= 200;
   if (behind) d.tiles_f = d.main_tiles;
   d.inv_tiles = 1.0f / (float)(d.pixels_first ? d.tiles_p : d.tiles_f);
@@ -559,6 +559,9 @@ double other_us(const IgemmArgs& a, int dt, DirectRival rival) {
   static const Fit f16_3x3[] = {{2.7, 0.097, 0.85, 0.0}, {1.5, 0.009, 2.43, 0.10}};
   const int rounds = (a.R * a.S * a.C * (int)dtype_size(dt) + 127) / 128, main_f = a.aux_f0 ? a.aux_f0 : a.F;
   if (rival == kRivalPatch && dt == kF32) {
+    // (from 257 channels: 4x8x10x512 -> 512 24.5 us here, 15.5 there, 2x14x14x384 18.5 and 13.4; at 256 what there is to gain is 1 to 3 us)
+    const double flat = a.C > 256 ? conv3x3_split_flat_us(a.N, a.OH, a.OW, a.C, main_f) : 0;
+    if (flat > 0) return flat;
     int p[8];
     if (!conv3x3_patch_plan(1, a.N, a.OH, a.OW, main_f, a.C / 32, p)) return 1e30;
     const double wgs = (double)((a.N + p[1] - 1) / p[1]) * ((a.OH + p[2] - 1) / p[2]) * p[4] * ((main_f + 63) / 64), turns = std::ceil(wgs / 256);

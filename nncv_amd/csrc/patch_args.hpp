@@ -47,5 +47,7 @@ struct PatchArgs {
 
 // The fp32 kernel (conv3x3_split.hip): 64 ws pixel slots, 64 filters (half: 32) a workgroup
 void launch_conv3x3_split(const PatchArgs& a, int ws, bool half, const char* tag, double flops, double bytes, hipStream_t s);
+// ... and 32 consecutive pixels x 32 filters
+void launch_conv3x3_split_flat(const PatchArgs& a, double flops, double bytes, hipStream_t s);
 
 }  // namespace nncv_hip
