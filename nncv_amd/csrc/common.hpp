@@ -226,6 +226,9 @@ bool igemm_takes_direct(const IgemmArgs& a, int in_dt, int out_dt);
 // 3x3 pad-1 layers at stride 1, or 2 in fp16: direct convolution with the haloed input patch resident in LDS
 // (conv3x3_patch.hip); same arguments and epilogue as the igemm kernels.
 bool conv3x3_patch_applicable(const IgemmArgs& a, int in_dt);
+// fp16 3x3 stride-2 layers of 64 channels, of those that conv_ring would run, with their filters in registers (conv3x3s2_resident.hip)
+bool conv3x3s2_resident_wins(const IgemmArgs& a);
+void launch_conv3x3s2_resident(const IgemmArgs& a, double flops, double bytes, hipStream_t s);
 // us that the fp32 kernel takes in tiles of 32 consecutive pixels, 0: it does not (conv3x3_split.hip)
 double conv3x3_split_flat_us(int N, int H, int W, int C, int F);
 // The tile plan that kernel would use for N x OH x OW output pixels, F filters and `slabs` 128-byte

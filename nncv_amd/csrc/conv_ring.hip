@@ -694,7 +694,12 @@ void launch_conv_ring(const IgemmArgs& a, hipStream_t s) {
   const Form* f = best_form(a, &us);
   d.wfrag = a.wt_frag; d.aux_wfrag = a.aux_wt_frag;
   const double flops = a.alg_flops > 0 ? a.alg_flops : 2.0 * d.P * (double)a.F * a.R * a.S * a.C;
-  ProfScope prof(f->tag, flops, 2.0 * ((double)a.N * a.H * a.W * a.C + (double)a.F * a.R * a.S * a.C + (double)d.P * a.F * (a.residual ? 2 : 1)), s);
+  const double bytes = 2.0 * ((double)a.N * a.H * a.W * a.C + (double)a.F * a.R * a.S * a.C + (double)d.P * a.F * (a.residual ? 2 : 1));
+  if (conv3x3s2_resident_wins(a)) {
+    launch_conv3x3s2_resident(a, flops, bytes, s);
+    return;
+  }
+  ProfScope prof(f->tag, flops, bytes, s);
   f->launch(d, a.R * a.S == 1 && a.pad_h == 0 && a.pad_w == 0 ? kPoint : a.C % 64 == 0 ? kLines : kAny, s);
   NNCV_HIP_CHECK(hipGetLastError());
 }
