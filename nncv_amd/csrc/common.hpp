@@ -268,7 +268,8 @@ enum DirectRival : int { kRivalPatch = 0, kRivalPatchS2 = 1, kRivalIgemmFast = 2
 bool conv_direct_serves(int dt, int F, int RS, int Cp);
 bool conv_direct_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 bool conv_direct_wins(const IgemmArgs& a, int dt, DirectRival rival);
-void launch_conv_direct(const IgemmArgs& a, int dt, hipStream_t s);
+// (store_f32: `out` is fp32, whatever dt is, at any float's address)
+void launch_conv_direct(const IgemmArgs& a, int dt, hipStream_t s, bool store_f32 = false);
 size_t weight_flat_bytes(int dt, int F, int RS, int Cp);
 // (rows: the filters are [F][K] already, K contiguous)
 void launch_weight_flat_rows(const void* w, void* dst, int dt, int F, int K, hipStream_t s);
@@ -413,6 +414,14 @@ struct SeProjectArgs {
 bool se_project_applicable(int HW, int C, int SQ, int F);
 void launch_transpose_half(const void* w, void* dst, int rows, int cols, hipStream_t s);  // [rows][cols] -> [cols][rows]
 void launch_se_project(const SeProjectArgs& a, hipStream_t s);
+// out[n][f] = mean over HW of act(scale * (wt . in) + shift), fp16 (conv_pool.hip): in [N][HW] pixels of `pix` elements, wt [F][C]
+struct ConvPoolArgs {
+  const void* in; const void* wt; const float* scale; const float* shift; void* out;
+  int N, HW, pix, C, F, act;
+  int blocks; float inv_blocks;  // filled in by the launcher
+};
+bool conv_pool_applicable(int N, int HW, int pix, int C, int F);
+void launch_conv_pool(const ConvPoolArgs& a, hipStream_t s);
 // out = act(a (+ b));  b may be null;  n elements, n a multiple of the 16-byte vector
 void launch_eltwise(const void* a, const void* b, void* out, int dt, long long n, int act, hipStream_t s);
 // the same over [P][C] tensors with row pitches lda / ldb / ldo (elements): slices of wider tensors

@@ -78,6 +78,7 @@ struct DirectArgs {
   int main_f, aux_tap;   // filters of the convolution itself; the tap the others walk
   float inv_ohw, inv_ow, inv_s, inv_cpt, inv_tiles;
 };
+constexpr int kStoreF32 = 1 << 30;  // in `act`: the result is fp32 whatever OutT (no residual, no auxiliary filters)
 
 // UNI: a tap is a whole number of rounds (C elements = whole 128-byte lines), so the tap of a round is the same for all lanes
 // BEHIND: a workgroup takes its tile's auxiliary filters behind it, over the same pixels; there are no workgroups for them
@@ -239,7 +240,9 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
   const OutT* res = aux ? nullptr : static_cast<const OutT*>(a.residual);
   OutT* out = static_cast<OutT*>(aux ? a.aux_out : a.out);
   const int ldo = aux ? a.aux_ldo : a.ldo, act = aux ? a.aux_act : a.act;
-  typedef OutT out4 __attribute__((ext_vector_type(4)));
+  typedef OutT out4_whole __attribute__((ext_vector_type(4)));
+  typedef out4_whole out4 __attribute__((aligned(sizeof(OutT) == 4 ? 4 : 8)));  // (a caller's fp32 tensor may begin at any float)
+  typedef floatx4 float4_any __attribute__((aligned(4)));
   struct Quad {
     floatx4 sc, sh;
     out4 rv;
@@ -270,6 +273,12 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
     if (res && after) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) y[e] += (float)q.rv[e];
+    }
+    if constexpr (sizeof(OutT) == 2) {
+      if (act & kStoreF32) {
+        *reinterpret_cast<float4_any*>(reinterpret_cast<float*>(out) + q.at) = float4_any{y[0], y[1], y[2], y[3]};
+        return;
+      }
     }
     out4 o;
 #pragma unroll
@@ -642,7 +651,8 @@ bool conv_direct_wins(const IgemmArgs& a, int dt, DirectRival rival) {
   return us < margin * other_us(a, dt, rival);
 }
 
-void launch_conv_direct(const IgemmArgs& a, int dt, hipStream_t s) {
+void launch_conv_direct(const IgemmArgs& a, int dt, hipStream_t s, bool store_f32) {
+  NNCV_REQUIRE(!store_f32 || (!a.residual && a.aux_f0 == 0), "conv_direct: fp32 results take no residual and no auxiliary filters");
   DirectArgs d{};
   const int es = (int)dtype_size(dt);
   d.in = a.in; d.wt = a.wt_flat; d.out = a.out; d.scale = a.scale; d.shift = a.shift; d.residual = a.residual; d.aux_out = a.aux_out;
@@ -651,7 +661,7 @@ void launch_conv_direct(const IgemmArgs& a, int dt, hipStream_t s) {
   if (a.aux_f0) d.aux_wt = a.aux_wt_flat, d.aux_wt_bytes = (unsigned)weight_flat_bytes(dt, a.F - a.aux_f0, 1, a.C);
   d.H = a.H; d.W = a.W; d.F = a.F; d.S = a.S; d.OW = a.OW; d.OHW = a.OH * a.OW; d.P = a.N * a.OH * a.OW; d.pix = a.pix_stride ? a.pix_stride : a.C;
   d.stride_h = a.stride_h; d.stride_w = a.stride_w; d.pad_h = a.pad_h; d.pad_w = a.pad_w;
-  d.act = a.relu; d.aux_act = a.aux_relu; d.ldo = a.ldo; d.aux_ldo = a.aux_ldo;
+  d.act = a.relu | (store_f32 ? kStoreF32 : 0); d.aux_act = a.aux_relu; d.ldo = a.ldo; d.aux_ldo = a.aux_ldo;
   d.chunks = a.R * a.S * a.C * es / 16; d.cpt = a.C * es / 16;
   d.main_f = a.aux_f0 ? a.aux_f0 : a.F; d.aux_tap = a.aux_tap;
   d.inv_ohw = 1.0f / (float)d.OHW; d.inv_ow = 1.0f / (float)d.OW; d.inv_s = 1.0f / (float)d.S; d.inv_cpt = 1.0f / (float)d.cpt;

@@ -332,9 +332,18 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
     launch_weight_flat(blob + (size_t)o.w * es, nodes_[i].wflat.get(), dt, o.F, logical_[o.in[0]], o.K * o.K, C, s);
   }
 
+  // a pointwise convolution that is only averaged: its result need not be stored
+  static const bool no_pool = getenv("NNCV_HIP_NO_POOL_FUSION") != nullptr;
+  for (int i = 0; !no_pool && dt == kF16 && i + 1 < n; ++i) {
+    const GraphOp &c = ops[i], &q = ops[i + 1];
+    nodes_[i].pools = c.kind == NNCV_HIP_OP_CONV && c.K == 1 && c.stride == 1 && c.pad == 0 && c.in[0] > 0 && c.in[1] < 0 && q.kind == NNCV_HIP_OP_GAVGPOOL &&
+                      q.in[0] == c.out && readers[c.out] == 1 && !nodes_[i].skip && !nodes_[i + 1].skip && !nodes_[i + 1].se_head &&
+                      logical_[c.in[0]] == channels_[c.in[0]] && !(i >= 4 && nodes_[i - 4].projects == i);
+  }
+
   for (int i = 0; i < n; ++i) {  // what rides in another launch, or carries one, does not join
     auto single = [&](int k) {
-      return !nodes_[k].skip && nodes_[k].add_out < 0 && !(k >= 4 && nodes_[k - 4].projects == k) && !(k + 1 < n && nodes_[k + 1].expands == k);
+      return !nodes_[k].pools && !nodes_[k].skip && nodes_[k].add_out < 0 && !(k >= 4 && nodes_[k - 4].projects == k) && !(k + 1 < n && nodes_[k + 1].expands == k);
     };
     if (nodes_[i].joins >= 0 && !(single(i) && single(nodes_[i].joins))) nodes_[nodes_[i].joins].joined = false, nodes_[i].joins = -1;
   }
@@ -557,6 +566,25 @@ const Graph::Plan& Graph::plan_of(int N, int H, int W) const {
         life[nodes_[i + 2].op.out].first_op = i + 1;
       }
   }
+  p.pooled.assign(n, 0);
+  for (int i = 0; i + 1 < n; ++i) {
+    const int in = nodes_[i].op.in[0], t = nodes_[i].op.out;
+    const Dims a = p.dims[in];
+    if (!nodes_[i].pools || !conv_pool_applicable(N, a.H * a.W, pitch(in), a.C, channels_[t])) continue;
+    p.pooled[i] = 1;
+    life[t] = TensorLife{i + 1, i + 1, 0, 0};
+    life[nodes_[i + 1].op.out].first_op = i + 1;
+  }
+  // A last convolution to one pixel, where its kernel can store fp32: in the order of the caller's tensor already (32x1x1x1024 -> 1000: 5.9 us
+  // behind the pass; 4.2 and as much again for the conversion before).
+  if (const Node& nd = nodes_[n - 1]; nd.op.kind == NNCV_HIP_OP_CONV && !nd.skip && !nd.joined && nd.op.in[1] < 0 && nd.op.in[0] > 0 && nd.wflat.get() &&
+                                      nd.op.F % 4 == 0 && p.dims[nd.op.out].H * p.dims[nd.op.out].W == 1 && pair_stem_ != n - 1 &&
+                                      !(n >= 5 && nodes_[n - 5].projects == n - 1))
+    p.last_f32 = igemm_takes_direct(last_args(p, nullptr, nullptr), dt_, dt_);
+  if (p.last_f32) {
+    life[nodes_[n - 1].op.out].bytes = 0;
+    life[nodes_[n - 1].op.in[0]].last_op = n + 1;
+  }
   p.head = nodes_[n - 1].op.kind == NNCV_HIP_OP_YOLO_DETECT;
   for (int k = 0; p.head && k < 3 && nodes_[n - 1].op.in[k] >= 0; ++k) {
     const Node* c = maker(nodes_[n - 1].op.in[k]);
@@ -625,6 +653,23 @@ int Graph::pitch(int t) const {
   return row_[root];
 }
 
+// The last convolution, to one pixel of `out`.
+IgemmArgs Graph::last_args(const Plan& p, const char* base, float* out) const {
+  const Node& nd = nodes_.back();
+  const GraphOp& op = nd.op;
+  const Dims a = p.dims[op.in[0]];
+  IgemmArgs g{};
+  g.in = base ? base + p.offset[op.in[0]] : nullptr; g.wt = nd.wt.get(); g.wt_flat = nd.wflat.get(); g.out = out;
+  g.scale = nd.scale.as<float>(); g.shift = nd.shift.as<float>();
+  g.N = p.N; g.H = a.H; g.W = a.W; g.C = a.C; g.F = g.ldo = op.F; g.R = g.S = op.K; g.OH = g.OW = 1;
+  g.stride_h = g.stride_w = op.stride; g.pad_h = g.pad_w = op.pad; g.relu = op.act; g.batch = 1;
+  g.pix_stride = pitch(op.in[0]);
+  const unsigned long long span = (unsigned long long)p.N * a.H * a.W * g.pix_stride * dtype_size(dt_);
+  g.in_bytes = span < 0xffffffffull ? (unsigned)span : 0xffffffffu;
+  g.alg_flops = 2.0 * p.N * op.F * (double)op.K * op.K * logical_[op.in[0]];
+  return g;
+}
+
 // The launch that computes operator i and the one it joins: filters of both, results to two tensors.
 IgemmArgs Graph::joint_args(const Plan& p, int i, char* base) const {
   const Node &nd = nodes_[i], &nj = nodes_[nd.joins];
@@ -658,6 +703,12 @@ void Graph::launch_io(const Plan& p, int i, std::vector<int>* writes, std::vecto
     return;
   }
   if (nd.joined && joint_second(p, i)) return;
+  if (i > 0 && p.pooled[i - 1]) return;
+  if (p.pooled[i] || (i == n - 1 && p.last_f32)) {
+    reads->push_back(op.in[0]);
+    if (p.pooled[i]) writes->push_back(nodes_[i + 1].op.out);
+    return;
+  }
   if (nd.joins >= 0 && p.joint[i]) {
     reads->push_back(op.in[0]);
     writes->push_back(op.out);
@@ -795,6 +846,14 @@ void Graph::forward_body(const void* src, int N, int H, int W, void* ws, hipStre
       continue;
     }
     if (nd.skip || (nd.head && p.head) || (nd.joined && joint_second(p, (int)i))) continue;
+    if ((i > 0 && p.pooled[i - 1]) || (i + 1 == nodes_.size() && p.last_f32)) continue;
+    if (p.pooled[i]) {
+      ConvPoolArgs c{};
+      c.in = at(op.in[0]); c.wt = nd.wt.get(); c.scale = nd.scale.as<float>(); c.shift = nd.shift.as<float>(); c.out = at(nodes_[i + 1].op.out);
+      c.N = N; c.HW = a.H * a.W; c.pix = pitch(op.in[0]); c.C = a.C; c.F = o.C; c.act = op.act;
+      launch_conv_pool(c, s);
+      continue;
+    }
     if (nd.joins >= 0 && p.joint[i]) {
       launch_conv_ring(joint_args(p, (int)i, base), s);
       continue;
@@ -961,6 +1020,10 @@ void Graph::forward_tail(int N, int H, int W, float* out, void* ws, hipStream_t 
       launch_yolo_detect(d, dt_, s);
       box0 += (long long)op.K * h.H * h.W;
     }
+    return;
+  }
+  if (p.last_f32) {
+    launch_conv_direct(last_args(p, base, out), dt_, s, dt_ == kF16);
     return;
   }
   const int Cl = logical_[op.out];

@@ -68,6 +68,7 @@ class Graph {
     int joins = -1;
     bool head = false;  // a 1x1 CONV that only the YOLO_DETECT reads and whose launch may compute it (Plan::head)
     bool joined = false;
+    bool pools = false;  // a 1x1 CONV whose only reader is the GAVGPOOL behind it (Plan::pooled)
     DeviceBuffer wt_t;  // the two vectors' weights of such a block, [in][out]
   };
   struct Dims { int C, H, W; };
@@ -79,6 +80,8 @@ class Graph {
     std::vector<int> dw;             // per operator: bands of a DWCONV that runs as a dw_block, 0: as its own operators
     std::vector<char> se;            // per operator: this GAVGPOOL starts a se_project launch
     bool head = false;               // the YOLO_DETECT launch computes the convolutions that it reads
+    std::vector<char> pooled;        // per operator: its launch stores the means that the next operator is after, not the result
+    bool last_f32 = false;           // the last operator is a convolution whose launch writes the caller's buffer
     std::vector<char> joint;         // per operator: its launch computes the one it joins as well
     size_t total;
   };
@@ -104,6 +107,7 @@ class Graph {
   std::vector<int> row_;  // per tensor that is no view: elements between consecutive pixels, its channel count or more
   int pitch(int t) const;  // the same for any tensor
   IgemmArgs joint_args(const Plan& p, int i, char* base) const;
+  IgemmArgs last_args(const Plan& p, const char* base, float* out) const;
   const Node* maker(int t) const;  // the operator whose result t is
   bool joint_second(const Plan& p, int i) const;  // operator i is computed by the one that joins it
   std::vector<float> detect_anchor_wh_, detect_stride_;  // YOLO_DETECT: host copies of anchors * stride, strides
