@@ -216,6 +216,13 @@ struct IgemmArgs {
   // `out`.  split_f = 0: none; otherwise a multiple of 8, and no residual.
   int split_f, split_ldo;
   long long split_ofs;
+  // With two results: a 1x1 layer of chain_f = split_f channels and filters that reads the first one, and its result; or null.
+  // chain_only: nothing else reads the first result, it is not stored.
+  const void* chain_wt;  // [chain_f][chain_f]
+  const float *chain_scale, *chain_shift;
+  void* chain_out;
+  int chain_f, chain_act, chain_ldo;
+  bool chain_only;
 };
 // in_dt: element type of in/wt (kF32 | kF16); out_dt: element type of out/residual.
 // Dispatches to the fast kernel (igemm_fast.hip) when C is a multiple of one K step and the
@@ -279,6 +286,8 @@ void launch_weight_flat(const void* w_fcrs, void* dst, int dt, int F, int C, int
 bool conv3x3_narrow_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 double conv3x3_narrow_us(const IgemmArgs& a);
 void launch_conv3x3_narrow(const IgemmArgs& a, hipStream_t s);
+// whether two 1x1 layers of C channels and F filters each over P pixels should compute the 1x1 layer behind the first one as well
+bool conv_ring_chains(long long P, int C, int F);
 bool conv_ring_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 double conv_ring_us(const IgemmArgs& a);
 bool conv_ring_beats_patch_s2(const IgemmArgs& a);

@@ -42,13 +42,19 @@ struct RingArgs {
   void* aux_out; unsigned aux_out_bytes;
   int split_f, split_ldo; unsigned ofs, split_ofs;    // filters from split_f on (F: none) go to rows of their own; bytes from `out`
   float inv_ohw, inv_ow, inv_tiles;
+  const void* chain_wt; const float* chain_scale; const float* chain_shift; void* chain_out;  // the layer behind the first result (CH > 0)
+  unsigned chain_bytes; int chain_act, chain_ldo, chain_only;
   const void* wfrag; const void* aux_wfrag; int groups, aux_groups, lead;  // the resident form's filters: 32-filter groups; bytes of padding
 };
 
 enum { kPoint = 0, kLines = 1, kAny = 2 };  // 1x1 without padding; taps of whole slabs (C % 64 == 0); any C % 8 == 0
 
-template <int WP, int WF, int PB, int FB, int S, int MODE>
+// CH > 0: of two results the first one, 16 * CH channels, is the input of a further 1x1 layer with as many filters.  Its values are in LDS on
+// their way out, rounded; the workgroups that have all its channels multiply them there.
+template <int WP, int WF, int PB, int FB, int S, int MODE, int CH = 0>
 __global__ __launch_bounds__(64 * WP * WF) void conv_ring_kernel(const RingArgs a) {
+  constexpr int kChain = 16 * CH, NB = CH / (2 * WF) > 0 ? CH / (2 * WF) : 1;  // blocks of 32 of those filters a wave takes
+  static_assert(CH == 0 || (PB == 1 && MODE == kPoint && kChain <= 32 * WF * FB), "a tile has all channels of the first result");
   constexpr int NW = WP * WF, BP = 32 * WP * PB, BF = 32 * WF * FB, LP = BP / 8 / NW, LF = BF / 8 / NW;
   static_assert(BP % (8 * NW) == 0 && BF % (8 * NW) == 0, "whole load instructions per wave");
   constexpr int kStage = (BP + BF) * 128;
@@ -205,7 +211,8 @@ __global__ __launch_bounds__(64 * WP * WF) void conv_ring_kernel(const RingArgs 
   for (int o = 0; o < kOut; ++o) {
     const int p = p0 + wp * PB * 32 + o * kRowsInstr + orow, f = f0 + wf * FB * 32 + ochan;
     oofs[o] = p < a.P && f < fend ? (unsigned)(aux ? p * a.aux_ldo + f - a.aux_f0 : p * a.ldo + f) * 2u : kOOBr;
-    if (MODE == kPoint && p < a.P && f < fend) oofs[o] = f < a.split_f ? oofs[o] + a.ofs : (unsigned)(p * a.split_ldo + f - a.split_f) * 2u + a.split_ofs;
+    if (CH > 0 && a.chain_only && f < a.split_f) oofs[o] = kOOBr;
+    else if (MODE == kPoint && p < a.P && f < fend) oofs[o] = f < a.split_f ? oofs[o] + a.ofs : (unsigned)(p * a.split_ldo + f - a.split_f) * 2u + a.split_ofs;
   }
   if (residual) {
     const __amdgpu_buffer_rsrc_t rs_res = make_rsrc(a.residual, a.out_bytes);
@@ -213,6 +220,12 @@ __global__ __launch_bounds__(64 * WP * WF) void conv_ring_kernel(const RingArgs 
     for (int o = 0; o < kOut; ++o) rv[o] = __builtin_amdgcn_raw_buffer_load_b128(rs_res, oofs[o], 0, 0);
   }
   fetch_pixels(0);
+  if constexpr (CH > 0) {
+    if ((int)threadIdx.x < kChain) {
+      ss[2 * BF + threadIdx.x] = a.chain_scale ? a.chain_scale[threadIdx.x] : 1.0f;
+      ss[2 * BF + kChain + threadIdx.x] = a.chain_shift ? a.chain_shift[threadIdx.x] : 0.0f;
+    }
+  }
   if ((int)threadIdx.x < BF) ss[threadIdx.x] = ssv, ss[BF + threadIdx.x] = shv;
 
   floatx16 acc[FB][PB];
@@ -297,10 +310,66 @@ __global__ __launch_bounds__(64 * WP * WF) void conv_ring_kernel(const RingArgs 
         *reinterpret_cast<half4*>(at + q * 16) = x;
       }
     }
+  const int cf0 = wf * NB * 32;  // this wave's filters of the chained layer
+  const bool chained = CH > 0 && tf == 0 && cf0 < kChain;
+  u32x4 cw[CH > 0 ? CH : 1][NB];
+  if constexpr (CH > 0) {
+    const __amdgpu_buffer_rsrc_t rs_c = make_rsrc(a.chain_wt, (unsigned)(kChain * kChain) * 2u);
+#pragma unroll
+    for (int k = 0; k < CH; ++k)
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+        cw[k][b] = __builtin_amdgcn_raw_buffer_load_b128(rs_c, chained ? (unsigned)((cf0 + b * 32 + lrow) * kChain + k * 16 + lh * 8) * 2u : kOOBr, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  }
 #pragma unroll
   for (int o = 0; o < kOut; ++o) {
     const u32x4 v = *reinterpret_cast<const u32x4*>(tile + (o * kRowsInstr + orow) * kPitch + ochan * 2);
     __builtin_amdgcn_raw_buffer_store_b128(v, rs_out, oofs[o], 0, 0);
+  }
+  if constexpr (CH > 0) {
+    if (tf != 0) return;  // (uniform)
+    __syncthreads();
+    floatx16 z[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) z[b][e] = 0.0f;
+#pragma unroll
+    for (int k = 0; k < CH; ++k) {  // channels 16 k + 8 lh .. of pixel lrow: in the tile of the wave whose filters they were
+      const u32x4 x = *reinterpret_cast<const u32x4*>(smem + (wp + WP * (16 * k / (32 * FB))) * (32 * kPitch) + lrow * kPitch + (16 * k % (32 * FB) + 8 * lh) * 2);
+#pragma unroll
+      for (int b = 0; b < NB; ++b) Mma<half_t>::run(cw[k][b], x, z[b]);
+    }
+    __syncthreads();
+    if (!chained) return;
+    constexpr int kLanes = 4 * NB, kRows = 64 / kLanes, kPitchC = NB * 64 + 16;
+    const float* sc = ss + 2 * BF + cf0;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      float y[16];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const floatx4 m = *reinterpret_cast<const floatx4*>(sc + b * 32 + 8 * q + 4 * lh), h = *reinterpret_cast<const floatx4*>(sc + kChain + b * 32 + 8 * q + 4 * lh);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[4 * q + e] = z[b][4 * q + e] * m[e] + h[e];
+      }
+      act_apply_n<true>(y, a.chain_act);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        half4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = (half_t)y[4 * q + e];
+        *reinterpret_cast<half4*>(tile + lrow * kPitchC + b * 64 + q * 16 + lh * 8) = v;
+      }
+    }
+    const __amdgpu_buffer_rsrc_t rs_co = make_rsrc(a.chain_out, a.chain_bytes);
+#pragma unroll
+    for (int o = 0; o < 32 / kRows; ++o) {
+      const int r = o * kRows + lane / kLanes, c = (lane % kLanes) * 8, p = p0 + wp * 32 + r;
+      const u32x4 v = *reinterpret_cast<const u32x4*>(tile + r * kPitchC + c * 2);
+      __builtin_amdgcn_raw_buffer_store_b128(v, rs_co, p < a.P ? (unsigned)(p * a.chain_ldo + cf0 + c) * 2u : kOOBr, 0, 0);
+    }
   }
 }
 
@@ -514,10 +583,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PB == 4 ? 2
 
 // ---- dispatch
 
-template <int WP, int WF, int PB, int FB, int S>
+template <int WP, int WF, int PB, int FB, int S, int CH = 0>
 void launch_cfg(RingArgs d, int mode, hipStream_t s) {
   constexpr int NW = WP * WF, BP = 32 * WP * PB, BF = 32 * WF * FB, ring = S * (BP + BF) * 128, tile = NW * PB * 32 * (FB * 64 + 16);
-  constexpr int lds = (ring > tile ? ring : tile) + BF * 8;
+  constexpr int lds = (ring > tile ? ring : tile) + BF * 8 + 128 * CH;
   const int main_f = d.aux_f0 ? d.aux_f0 : d.F;
   d.tiles_f = (main_f + BF - 1) / BF;
   d.aux_tiles = (d.F - main_f + BF - 1) / BF;
@@ -531,6 +600,7 @@ void launch_cfg(RingArgs d, int mode, hipStream_t s) {
     (void)attr;
     launch_kernel(kern, dim3((unsigned)(d.aux_f0 ? (d.tiles_p + 7) / 8 * 8 * (d.tiles_f + d.aux_tiles) : d.tiles_f * d.tiles_p)), dim3(64 * NW), lds, s, d);
   };
+  if constexpr (CH > 0) return go(conv_ring_kernel<WP, WF, PB, FB, S, kPoint, CH>);
   if (mode == kPoint) go(conv_ring_kernel<WP, WF, PB, FB, S, kPoint>);
   else if (mode == kLines) go(conv_ring_kernel<WP, WF, PB, FB, S, kLines>);
   else go(conv_ring_kernel<WP, WF, PB, FB, S, kAny>);
@@ -661,6 +731,12 @@ bool conv_ring_beats_patch_s2(const IgemmArgs& a) {
   return a.stride_h == 2 && (P + 127) / 128 * ((main_f + 127) / 128) >= 200;
 }
 
+// Blocks of two 1x1 layers with one bottleneck, us with its first layer in a launch of its own / here, MB of that layer's input: 16x160x160x64 ->
+// 32 + 32 -> 32 158.4 / 152.6 (25 MB), 4 images 73.8 / 71.5 (6), 1 image 50.7 / 49.2 (1.6); 16x80x80x128 -> 64 + 64 -> 64 112.5 / 111.8 (12.5), 4
+// images 60.2 / 59.1 (3); 2 images 50.2 / 50.3 (1.6); 4x80x80x256 -> 64 + 64 -> 64, where nothing else reads the first result, 73.3 / 70.4 (3).
+// With 128 channels the chained filters take the registers of a CU's second workgroup: 16x40x40x256 21.0 us against 11.5 + 6.7.
+bool conv_ring_chains(long long P, int C, int F) { return (F == 32 || F == 64) && C % 8 == 0 && P * F * 2 >= 2 << 20; }
+
 double conv_ring_us(const IgemmArgs& a) {
   double us = 0;
   best_form(a, &us);
@@ -695,6 +771,19 @@ void launch_conv_ring(const IgemmArgs& a, hipStream_t s) {
   d.wfrag = a.wt_frag; d.aux_wfrag = a.aux_wt_frag;
   const double flops = a.alg_flops > 0 ? a.alg_flops : 2.0 * d.P * (double)a.F * a.R * a.S * a.C;
   const double bytes = 2.0 * ((double)a.N * a.H * a.W * a.C + (double)a.F * a.R * a.S * a.C + (double)d.P * a.F * (a.residual ? 2 : 1));
+  if (a.chain_wt) {
+    d.chain_wt = a.chain_wt; d.chain_scale = a.chain_scale; d.chain_shift = a.chain_shift; d.chain_out = a.chain_out;
+    d.chain_act = a.chain_act; d.chain_ldo = a.chain_ldo; d.chain_only = a.chain_only;
+    d.chain_bytes = (unsigned)d.P * a.chain_ldo * 2u;
+    d.pixels_first = false;
+    ProfScope prof("conv_ring<chain>", flops + 2.0 * d.P * (double)a.chain_f * a.chain_f, bytes + 2.0 * d.P * (double)a.chain_f, s);
+    const bool two = d.chunks > 16;  // (slabs in the ring: one up to 128 channels, as without the chained layer)
+    if (a.chain_f == 32) launch_cfg<2, 2, 1, 1, 1, 2>(d, kPoint, s);
+    else if (two) launch_cfg<4, 2, 1, 2, 2, 4>(d, kPoint, s);
+    else launch_cfg<4, 2, 1, 2, 1, 4>(d, kPoint, s);
+    NNCV_HIP_CHECK(hipGetLastError());
+    return;
+  }
   if (conv3x3s2_resident_wins(a)) {
     launch_conv3x3s2_resident(a, flops, bytes, s);
     return;

@@ -347,6 +347,19 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
     };
     if (nodes_[i].joins >= 0 && !(single(i) && single(nodes_[i].joins))) nodes_[nodes_[i].joins].joined = false, nodes_[i].joins = -1;
   }
+  // the first pointwise layer of the bottleneck behind the first of two joined ones
+  static const bool no_chain = getenv("NNCV_HIP_NO_CHAIN") != nullptr;
+  for (int i = 0; !no_chain && i + 1 < n; ++i) {
+    if (nodes_[i].joins < 0) continue;
+    for (int k = i + 1; k < n && nodes_[i].chain < 0; ++k) {
+      const GraphOp& o = ops[k];
+      const Node& nk = nodes_[k];
+      if (o.kind == NNCV_HIP_OP_CONV && o.K == 1 && o.stride == 1 && o.pad == 0 && o.in[0] == ops[i].out && o.in[1] < 0 && o.F == ops[i].F && !nk.skip &&
+          nk.add_out < 0 && nk.joins < 0 && !nk.joined && !nk.pools && !nk.head && !(k >= 4 && nodes_[k - 4].projects == k) &&
+          !(k + 1 < n && nodes_[k + 1].expands == k) && k != n - 1)
+        nodes_[i].chain = k, nodes_[i].chain_only = readers[ops[i].out] == 1, nodes_[k].chained_by = i;
+    }
+  }
 
   // detection heads
   if (dt == kF16 && ops[n - 1].kind == NNCV_HIP_OP_YOLO_DETECT) {
@@ -359,7 +372,7 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
         if (ops[i].out == d.in[k]) h = i;
       const GraphOp& c = ops[std::max(h, 0)];
       ok = ok && h >= 0 && c.kind == NNCV_HIP_OP_CONV && c.K == 1 && c.stride == 1 && c.pad == 0 && c.in[0] > 0 && c.in[1] < 0 && c.act == kActNone &&
-           readers[d.in[k]] == 1 && !nodes_[h].skip && !nodes_[h].joined && nodes_[h].joins < 0 && logical_[c.in[0]] == channels_[c.in[0]] &&
+           readers[d.in[k]] == 1 && !nodes_[h].skip && nodes_[h].chained_by < 0 && !nodes_[h].joined && nodes_[h].joins < 0 && logical_[c.in[0]] == channels_[c.in[0]] &&
            detect_head_applicable(d.K, d.F, channels_[c.in[0]], 0);
       made.push_back(h);
     }
@@ -554,6 +567,7 @@ const Graph::Plan& Graph::plan_of(int N, int H, int W) const {
     }
     if (nodes_[i].add_out >= 0) life[nodes_[i].add_out].first_op = std::min(life[nodes_[i].add_out].first_op, i + 1);
     if (nodes_[i].joins >= 0) life[nodes_[nodes_[i].joins].op.out].first_op = i + 1;  // (also where the shape is not joined)
+    if (nodes_[i].chain >= 0) life[nodes_[nodes_[i].chain].op.out].first_op = i + 1;  // (likewise)
   }
   {
     auto pool5 = [&](int k, int in) {
@@ -624,10 +638,13 @@ const Graph::Plan& Graph::plan_of(int N, int H, int W) const {
   }
   // Joined convolutions: one launch where the LDS ring takes the doubled filters and both results lie within its reach.
   p.joint.assign(n, 0);
+  p.chained.assign(n, 0);
   for (int i = 0; i < n; ++i) {
     if (nodes_[i].joins < 0) continue;
     const IgemmArgs g = joint_args(p, i, nullptr);
     p.joint[i] = g.in_bytes < 0x7fffff00u && !igemm_takes_direct(g, dt_, dt_) && conv_ring_applicable(g, dt_, dt_);
+    const long long P = (long long)N * g.OH * g.OW;
+    p.chained[i] = p.joint[i] && nodes_[i].chain >= 0 && conv_ring_chains(P, g.C, nodes_[i].op.F) && P * pitch(nodes_[nodes_[i].chain].op.out) * 2 < 0x7fffff00ll;
   }
   check_plan(p);
   if (plans_.size() >= 8) plans_.erase(plans_.begin());
@@ -640,6 +657,8 @@ const Graph::Node* Graph::maker(int t) const {
     if (nd.op.out == t) return &nd;
   return nullptr;
 }
+
+bool Graph::chained_third(const Plan& p, int i) const { return nodes_[i].chained_by >= 0 && p.chained[nodes_[i].chained_by]; }
 
 bool Graph::joint_second(const Plan& p, int i) const {
   for (int k = 0; k < i; ++k)
@@ -684,6 +703,11 @@ IgemmArgs Graph::joint_args(const Plan& p, int i, char* base) const {
   const unsigned long long span = (unsigned long long)p.N * a.H * a.W * ldi * dtype_size(dt_);
   g.in_bytes = span < 0xffffffffull ? (unsigned)span : 0xffffffffu;
   g.out = base + p.offset[t]; g.ldo = pitch(t);
+  if (p.chained[i]) {
+    const Node& nk = nodes_[nd.chain];
+    g.chain_wt = nk.wt.get(); g.chain_scale = nk.scale.as<float>(); g.chain_shift = nk.shift.as<float>();
+    g.chain_out = base + p.offset[nk.op.out]; g.chain_f = F; g.chain_act = nk.op.act; g.chain_ldo = pitch(nk.op.out); g.chain_only = nd.chain_only;
+  }
   g.split_f = F; g.split_ldo = pitch(u); g.split_ofs = (long long)p.offset[u] - (long long)p.offset[t];
   g.alg_flops = 2.0 * p.N * a.H * a.W * 2 * F * (double)logical_[nd.op.in[0]];
   return g;
@@ -702,7 +726,7 @@ void Graph::launch_io(const Plan& p, int i, std::vector<int>* writes, std::vecto
       if (op.in[k] >= 0) reads->push_back(maker(op.in[k])->op.in[0]);
     return;
   }
-  if (nd.joined && joint_second(p, i)) return;
+  if ((nd.joined && joint_second(p, i)) || chained_third(p, i)) return;
   if (i > 0 && p.pooled[i - 1]) return;
   if (p.pooled[i] || (i == n - 1 && p.last_f32)) {
     reads->push_back(op.in[0]);
@@ -711,8 +735,9 @@ void Graph::launch_io(const Plan& p, int i, std::vector<int>* writes, std::vecto
   }
   if (nd.joins >= 0 && p.joint[i]) {
     reads->push_back(op.in[0]);
-    writes->push_back(op.out);
+    if (!(p.chained[i] && nd.chain_only)) writes->push_back(op.out);
     writes->push_back(nodes_[nd.joins].op.out);
+    if (p.chained[i]) writes->push_back(nodes_[nd.chain].op.out);
     return;
   }
   if (op.kind == NNCV_HIP_OP_CONV && i + 1 < n && nodes_[i + 1].expands == i && p.dw[i + 1]) {
@@ -845,7 +870,7 @@ void Graph::forward_body(const void* src, int N, int H, int W, void* ws, hipStre
       launch_image_pairs(image, s);
       continue;
     }
-    if (nd.skip || (nd.head && p.head) || (nd.joined && joint_second(p, (int)i))) continue;
+    if (nd.skip || (nd.head && p.head) || (nd.joined && joint_second(p, (int)i)) || chained_third(p, (int)i)) continue;
     if ((i > 0 && p.pooled[i - 1]) || (i + 1 == nodes_.size() && p.last_f32)) continue;
     if (p.pooled[i]) {
       ConvPoolArgs c{};

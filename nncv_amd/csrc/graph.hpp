@@ -66,6 +66,9 @@ class Graph {
     int expands = -1, projects = -1;
     // 1x1 convolutions that may run as one launch (Plan::joint): on the first one, the index of the second
     int joins = -1;
+    bool chain_only = false;  // nothing but `chain` reads this result
+    int chained_by = -1;
+    int chain = -1;  // with `joins`: a 1x1 CONV that reads this one's result and may be in that launch too (Plan::chained)
     bool head = false;  // a 1x1 CONV that only the YOLO_DETECT reads and whose launch may compute it (Plan::head)
     bool joined = false;
     bool pools = false;  // a 1x1 CONV whose only reader is the GAVGPOOL behind it (Plan::pooled)
@@ -82,6 +85,7 @@ class Graph {
     bool head = false;               // the YOLO_DETECT launch computes the convolutions that it reads
     std::vector<char> pooled;        // per operator: its launch stores the means that the next operator is after, not the result
     bool last_f32 = false;           // the last operator is a convolution whose launch writes the caller's buffer
+    std::vector<char> chained;       // per operator: its launch, which computes the one it joins, computes `chain` as well
     std::vector<char> joint;         // per operator: its launch computes the one it joins as well
     size_t total;
   };
@@ -109,6 +113,7 @@ class Graph {
   IgemmArgs joint_args(const Plan& p, int i, char* base) const;
   IgemmArgs last_args(const Plan& p, const char* base, float* out) const;
   const Node* maker(int t) const;  // the operator whose result t is
+  bool chained_third(const Plan& p, int i) const;  // operator i is computed by the launch of two joined ones
   bool joint_second(const Plan& p, int i) const;  // operator i is computed by the one that joins it
   std::vector<float> detect_anchor_wh_, detect_stride_;  // YOLO_DETECT: host copies of anchors * stride, strides
   std::vector<int> last_use_;  // per tensor: index of the last operator that reads it
