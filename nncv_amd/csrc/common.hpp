@@ -198,7 +198,7 @@ struct IgemmArgs {
   int pix_stride;    // elements between horizontally adjacent pixels; 0 = C (the stem reads 32
                      // contiguous elements = 4 packed pixel pairs at a pixel pitch of 8)
   unsigned in_bytes, wt_bytes;  // size of one batch slice of in / wt; 0 = derived from the geometry
-  const void* wt_frag;  // the same 3x3 filters in fragment-major order (launch_weight_frag3x3), or null
+  const void* wt_frag;  // the same 3x3 (or, for conv_ring.hip, 1x1) filters in fragment-major order (launch_weight_frag3x3, 1x1), or null
   const void* wt_frag32;  // fp16 3x3 stride-1 filters in the stream kernel's order (launch_weight_frag32), or null
   // Auxiliary filters fused into the same launch (the 1x1 stride-2 shortcut convolution of a
   // down-sampling block rides on the 3x3 stride-2 one: same input pixels, centre tap only).
@@ -272,6 +272,8 @@ void launch_image_pairs(const ImagePairsArgs& a, hipStream_t s);
 // that of the kernel which would run the layer otherwise.
 enum DirectRival : int { kRivalPatch = 0, kRivalPatchS2 = 1, kRivalIgemmFast = 2, kRivalIgemm = 3, kRivalShortK = 4, kRivalRing = 5, kRivalNarrow = 6 };
 // whether it is the kernel for a layer of F filters over RS taps of Cp channels at any size (else its order of the filters is not kept)
+// whether a 1x1 layer may run on conv_ring.hip's fragment forms, i.e. reads wt_frag (fp16)
+bool conv_ring_point_serves(int dt, int F, int RS, int C, int stride, int pad);
 bool conv_direct_serves(int dt, int F, int RS, int Cp);
 bool conv_direct_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 bool conv_direct_wins(const IgemmArgs& a, int dt, DirectRival rival);
@@ -358,6 +360,7 @@ void launch_weight_frsc(const void* w, int w_dt, void* dst, int dst_dt, int F, i
 size_t weight_frag3x3_bytes(int dt, int F, int C);
 void launch_weight_frag3x3(const void* w, int w_dt, void* dst, int dst_dt, int F, int C, hipStream_t s);
 // 1x1 weights [F][C] in the same order with one tap per slab (IgemmArgs::aux_wt_frag)
+inline size_t weight_frag1x1_bytes(int F, int C) { return (size_t)((F + 63) / 64) * 64 * C * 2; }  // fp16
 void launch_weight_frag1x1(const void* w, int w_dt, void* dst, int dst_dt, int F, int C, hipStream_t s);
 // stem weights [F,3,7,7] -> [F][7][4][8] over (pixel-pair, channel4); pair sp / pixel p holds
 // filter column 2*sp + p (zero outside 0..6)

@@ -385,7 +385,8 @@ __global__ __launch_bounds__(64 * WP * WF) void conv_ring_kernel(const RingArgs 
 //    loads, 62 without the pixels', 65 without the LDS reads, 50 without the products: a wave issues all of them in turn.
 // Times against the ring's 128 x 128 form or, below 200 tiles, conv3x3_patch.hip: 16x40x40x256 -> 512 27.1 -> 21.7 us, 16x160x160x64 ->
 // 128 29.0 -> 25.8, 16x40x40x256 -> 256 20.2 -> 13.3, 33x25x106x64 -> 128 14.0 -> 8.6.
-template <int PB, bool AUX>
+// POINT: 1x1 layers, one stage to a slab (point_us).
+template <int PB, bool AUX, bool POINT = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PB == 4 ? 2 : 3, PB == 4 ? 2 : 4))) void conv_ring_frag_kernel(const RingArgs a) {
   constexpr int BP = 32 * PB, BF = 128, kStage = BP * 128, kStages = 4, kRing = 8;
   constexpr int kPitch = 272, kLds = kStages * kStage > BP * kPitch ? kStages * kStage : BP * kPitch;
@@ -407,7 +408,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PB == 4 ? 2
   const int p0 = tp * BP, f0 = tf * BF, fend = AUX ? a.aux_f0 : a.F;
 
   // ---- filters: fragment (group g, stage st, sub-step kk) is the kilobyte ((g / 2 * stages + st) * 4 + kk) * 2 + g % 2 ----
-  const int nslab = a.cpt >> 3, T = nslab * 9;
+  const int nslab = a.cpt >> 3, T = POINT ? nslab : nslab * 9;
   const int g = min(tf * 4 + wave, a.groups - 1);  // (filters that are not there: the last ones again)
   const __amdgpu_buffer_rsrc_t rs_w = make_rsrc(a.wfrag, (unsigned)(a.groups >> 1) * T * 8192u);
   unsigned woff = (unsigned)((g >> 1) * T * 8192 + (g & 1) * 1024 + lane * 16);
@@ -432,6 +433,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PB == 4 ? 2
 #pragma unroll
   for (int i = 0; i < PB; ++i) {
     const int group = wave * PB + i, p = p0 + group * 8 + sub;
+    if constexpr (POINT) {  // result p reads pixel p
+      pbase[i] = p < a.P ? (unsigned)(p * a.pix * 2 + (pos ^ (((group & 1) << 2) + (sub >> 1))) * 16) : kOOBr;
+      valid[i] = 1u;
+      continue;
+    }
     int rem, x;
     const int n = fast_div(p < a.P ? p : 0, a.OHW, a.inv_ohw, &rem), y = fast_div(rem, a.OW, a.inv_ow, &x);
     const int yy = y * a.stride_h, xx = x * a.stride_w;
@@ -442,6 +448,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PB == 4 ? 2
   const int pixB = a.pix * 2, rowB = (a.W - 2) * pixB, turnB = 128 - (2 * a.W + 2) * pixB;
   int ptap = 0, pleft = T, poff = 0;  // the stage to fetch next
   auto fetch = [&](int buf) __attribute__((always_inline)) {
+    if constexpr (POINT) {
+#pragma unroll
+      for (int i = 0; i < PB; ++i) {
+        const unsigned at = pbase[i], v = pleft > 0 ? at : kOOBr;
+        fetch16(rs_in, smem + buf * kStage + (wave * PB + i) * 1024, v, (unsigned)poff);
+      }
+      --pleft;
+      poff += 128;
+      return;
+    }
     const unsigned bit = pleft > 0 ? 1u << ptap : 0u;
 #pragma unroll
     for (int i = 0; i < PB; ++i) {
@@ -547,7 +563,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PB == 4 ? 2
   // ---- out, through one tile [BP pixels][128 channels]: rows of 256 bytes leave as whole lines (64 bytes of a row a wave: 81
   // instead of 66 us for 256x56x56x64 -> 128 + 128, which is bound by what it writes) ----
   const int orow = wave * 4 + (lane >> 4), ochan = (lane & 15) * 8;
-  auto finish = [&](floatx16 (&sum)[PB], const float* sc, int act, __amdgpu_buffer_rsrc_t rs_out, int f, int filters, int ldo) __attribute__((always_inline)) {
+  auto finish = [&](floatx16 (&sum)[PB], const float* sc, int act, __amdgpu_buffer_rsrc_t rs_out, int f, int filters, int ldo, int from, unsigned ofs) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < PB; ++j) {
       float y[16];
@@ -571,13 +587,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PB == 4 ? 2
     for (int o = 0; o < 2 * PB; ++o) {
       const int p = p0 + o * 16 + orow;
       const u32x4 v = *reinterpret_cast<const u32x4*>(smem + (o * 16 + orow) * kPitch + ochan * 2);
-      __builtin_amdgcn_raw_buffer_store_b128(v, rs_out, p < a.P && f < filters ? (unsigned)(p * ldo + f) * 2u : kOOBr, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b128(v, rs_out, p < a.P && f < filters ? (unsigned)(p * ldo + f - from) * 2u + ofs : kOOBr, 0, 0);
     }
   };
-  finish(acc, ss + wave * 32, a.act, make_rsrc(a.out, a.out_bytes), f0 + ochan, fend, a.ldo);
+  const bool other = POINT && f0 + ochan >= a.split_f;  // (of a lane's eight filters all or none)
+  finish(acc, ss + wave * 32, a.act, make_rsrc(a.out, a.out_bytes), f0 + ochan, fend, other ? a.split_ldo : a.ldo, other ? a.split_f : 0, POINT ? (other ? a.split_ofs : a.ofs) : 0u);
   if constexpr (AUX) {
     __syncthreads();
-    finish(acc2, ss + BF + wave * 32, a.aux_act, make_rsrc(a.aux_out, a.aux_out_bytes), f0 + ochan, a.F - a.aux_f0, a.aux_ldo);
+    finish(acc2, ss + BF + wave * 32, a.aux_act, make_rsrc(a.aux_out, a.aux_out_bytes), f0 + ochan, a.F - a.aux_f0, a.aux_ldo, 0, 0u);
   }
 }
 
@@ -607,7 +624,7 @@ void launch_cfg(RingArgs d, int mode, hipStream_t s) {
 }
 
 template <int PB>
-void launch_frag(RingArgs d, int, hipStream_t s) {
+void launch_frag(RingArgs d, int mode, hipStream_t s) {
   constexpr int BP = 32 * PB, ring = 4 * BP * 128, tile = BP * 272, lds = (ring > tile ? ring : tile) + 128 * 16;
   const int main_f = d.aux_f0 ? d.aux_f0 : d.F;
   d.tiles_f = (main_f + 127) / 128;
@@ -615,7 +632,7 @@ void launch_frag(RingArgs d, int, hipStream_t s) {
   d.inv_tiles = 1.0f / (float)(d.pixels_first ? d.tiles_p : d.tiles_f);
   d.groups = (main_f + 63) / 64 * 2;
   d.aux_groups = (d.F - main_f + 63) / 64 * 2;
-  d.lead = (d.W + 1) * d.pix * 2;
+  d.lead = mode == kPoint ? 0 : (d.W + 1) * d.pix * 2;
   auto go = [&](auto kern) {
     static const bool attr = [&] {
       NNCV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
@@ -624,6 +641,8 @@ void launch_frag(RingArgs d, int, hipStream_t s) {
     (void)attr;
     launch_kernel(kern, dim3((unsigned)(d.tiles_f * d.tiles_p)), dim3(256), lds, s, d);
   };
+  if constexpr (PB == 2)
+    if (mode == kPoint) return go(conv_ring_frag_kernel<PB, false, true>);
   if (d.aux_f0) go(conv_ring_frag_kernel<PB, true>);
   else go(conv_ring_frag_kernel<PB, false>);
 }
@@ -661,6 +680,20 @@ const Form kForms[] = {
     {128, 128, 2, 1.51, 0.472, 2.537, 2.41, 6.32, 0, launch_frag<4>, "conv_ring<128x128,frag>", true},
 };
 
+// 1x1 layers of 512 channels and more, one to one and a half tiles of 64 x 128 a CU: long chains of slabs that the ring fetches one ahead and the
+// fragment form three, with filters from memory that may not be in L2.  us, ring / here: 4x28x28x512 -> 512 7.2 / 6.5, 2x40x40x768 -> 384 8.3 / 7.1,
+// 12x20x20x1024 -> 384 13.2 / 9.2, 48x20x20x1536 -> 96 22.2 / 17.5, 32x14x14x1536 -> 512 19.1 / 17.0; of 12 such layers the least gains 1.8 %
+// (32x14x14x768 -> 384, 24x10x10x640 -> 384).  With 256 and 384 channels, below 112 tiles and above 400 it is level at best (12x20x20x256 -> 96
+// 4.5 / 4.9, 16x28x28x768 -> 384 15.4 / 15.7).  The model: the same layers, within 8 %.
+bool point_serves(int dt, int F, int RS, int C, int stride, int pad) { return dt == kF16 && RS == 1 && stride == 1 && pad == 0 && C % 64 == 0 && C >= 512 && F > 64; }
+const Form kPointForm{64, 128, 4, 0, 0, 0, 0, 0, 0, launch_frag<2>, "conv_ring<64x128,point>", true};
+double point_us(const IgemmArgs& a) {  // 0: not taken
+  const double tiles = std::ceil((double)a.N * a.OH * a.OW / 64) * std::ceil(a.F / 128.0), slabs = a.C / 64;
+  if (!a.wt_frag || !point_serves(kF16, a.F, a.R * a.S, a.C, a.stride_h, a.pad_h) || a.stride_w != 1 || a.pad_w != 0 || a.residual || a.aux_f0 || a.chain_wt || tiles < 112 || tiles > 400)
+    return 0;
+  return tiles <= 256 ? 3.1 + 0.36 * slabs : 4.9 + 0.51 * slabs;
+}
+
 // What the fragment forms cover.  With auxiliary filters, whose sums take the registers of a third wave, from 256 channels on
 // (ResNet-18, 256 images: 44.3 -> 41.2 us; 47.2 -> 49.7 at 128 channels, 65.8 -> 67.8 at 64), and with 128 pixels to a tile (64: 77).
 bool frag_ok(const IgemmArgs& a) {
@@ -670,6 +703,7 @@ bool frag_ok(const IgemmArgs& a) {
 }
 
 const Form* best_form(const IgemmArgs& a, double* us) {
+  if ((*us = point_us(a)) > 0) return &kPointForm;
   const double P = (double)a.N * a.OH * a.OW, slabs = std::ceil(a.R * a.S * a.C / 64.0), main_f = a.aux_f0 ? a.aux_f0 : a.F;
   const bool any = a.R * a.S > 1 && a.C % 64 != 0, nine = slabs <= 9;
   auto per_cu = [&](const Form& f, double filters) { return std::ceil(P / f.bp) * std::ceil(filters / f.bf) / 256; };
@@ -725,6 +759,8 @@ bool conv_ring_applicable(const IgemmArgs& a, int in_dt, int out_dt) {
 // 150 tiles, is the other way round: 16.5 against 15.1).  Larger launches used to be igemm_fast's: 23 of them take 1.14 to 1.35
 // times as long there (256x28x28x128 -> 256: 52.2 against 42.0).  In a ResNet-18 pass of 256 images the three such layers with
 // their shortcuts went from 78.1 + 58.4 + 52.2 us there to 65.4 + 46.6 + 43.6, the pass from 1162 to 1133 us of launches.
+bool conv_ring_point_serves(int dt, int F, int RS, int C, int stride, int pad) { return point_serves(dt, F, RS, C, stride, pad); }
+
 bool conv_ring_beats_patch_s2(const IgemmArgs& a) {
   const long long P = (long long)a.N * a.OH * a.OW, main_f = a.aux_f0 ? a.aux_f0 : a.F;
   if (a.stride_h == 2 && frag_ok(a) && a.aux_f0 == 0 && a.F > 64 && (P + 63) / 64 * ((main_f + 127) / 128) >= 112) return true;

@@ -100,6 +100,7 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
     return blob + (size_t)off * es;
   };
 
+  std::vector<char> pixel(n_tensors_, 0);  // tensors of one pixel an image
   for (int i = 0; i < n; ++i) {
     const GraphOp& op = ops[i];
     const std::string where = "graph: operator " + std::to_string(i) + " (" + kind_name(op.kind) + "): ";
@@ -146,6 +147,12 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
         take(i, &Node::wt, (size_t)Cstored * op.K * op.K * C * es);
         if (Cstored > op.F) NNCV_HIP_CHECK(hipMemsetAsync(nd.wt.get(), 0, (size_t)Cstored * op.K * op.K * C * es, s));
         launch_weight_frsc(w, dt, nd.wt.get(), dt, op.F, Cl, op.K, op.K, C, s);
+        pixel[op.out] = pixel[op.in[0]];
+        // (1x1: not for single pixels, which are never enough; with the filters of both where two are joined, whole blocks of 64 of the first)
+        if (!pixel[op.in[0]] && Cl == C && Cstored == op.F && ((nd.joins < 0 && !nd.joined) || op.F % 64 == 0) && conv_ring_point_serves(dt, nd.joins >= 0 || nd.joined ? 2 * op.F : op.F, op.K * op.K, C, op.stride, op.pad)) {
+          take(i, &Node::wfrag, weight_frag1x1_bytes(op.F, C));
+          launch_weight_frag1x1(w, dt, nd.wfrag.get(), dt, op.F, C, s);
+        }
         if (op.K == 3 && (op.stride == 1 || (op.stride == 2 && dt == kF16)) && op.pad == 1 && Cl == C && Cstored == op.F && C % (128 / (int)es) == 0) {
           nd.wfrag.reset(weight_frag3x3_bytes(dt, op.F, C), &pool_);
           launch_weight_frag3x3(w, dt, nd.wfrag.get(), dt, op.F, C, s);
@@ -168,6 +175,7 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
       case NNCV_HIP_OP_MAXPOOL:
         NNCV_REQUIRE(op.K >= 1 && op.stride >= 1 && op.pad >= 0 && 2 * op.pad <= op.K, where + "bad geometry");
         break;
+      case NNCV_HIP_OP_GAVGPOOL: pixel[op.out] = 1; break;
       case NNCV_HIP_OP_SCALE:
       case NNCV_HIP_OP_ADD:
         NNCV_REQUIRE(channels_[op.in[1]] == C, where + "operands have different channel counts");
@@ -695,7 +703,7 @@ IgemmArgs Graph::joint_args(const Plan& p, int i, char* base) const {
   const Dims a = p.dims[nd.op.in[0]];
   const int F = nd.op.F, t = nd.op.out, u = nj.op.out, ldi = pitch(nd.op.in[0]);
   IgemmArgs g{};
-  g.in = base + p.offset[nd.op.in[0]]; g.wt = nd.wt.get(); g.wt_flat = nd.wflat.get();
+  g.in = base + p.offset[nd.op.in[0]]; g.wt = nd.wt.get(); g.wt_flat = nd.wflat.get(); g.wt_frag = nd.wfrag.get();
   g.scale = nd.scale.as<float>(); g.shift = nd.shift.as<float>();
   g.N = p.N; g.H = g.OH = a.H; g.W = g.OW = a.W; g.C = a.C; g.F = 2 * F; g.R = g.S = 1;
   g.stride_h = g.stride_w = 1; g.relu = nd.op.act; g.batch = 1;

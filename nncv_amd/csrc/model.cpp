@@ -57,6 +57,8 @@ ConvLayer::Sizes ConvLayer::sizes(const Desc& d, int algo, bool bn) {
     if (d.R == 3 && d.S == 3 && (d.stride == 1 || (d.stride == 2 && d.dt == kF16)) && d.pad == 1 && d.C % (128 / (int)es) == 0) {
       z.wfrag = weight_frag3x3_bytes(d.dt, d.F, d.C);
       if (d.dt == kF16 && d.stride == 1 && d.C % 64 == 0 && d.F % 32 == 0) z.wfrag32 = weight_frag32_bytes(d.F, d.C);
+    } else if (conv_ring_point_serves(d.dt, d.F, RS, d.C, d.stride, d.pad)) {
+      z.wfrag = weight_frag1x1_bytes(d.F, d.C);
     }
   }
   if (bn) z.scale = (size_t)Fp * 4;
@@ -101,7 +103,8 @@ ConvLayer::ConvLayer(const Desc& d, const void* w, const void* gamma, const void
     if (Fp > d.F) NNCV_HIP_CHECK(hipMemsetAsync(wt_.get(), 0, wt_.bytes(), s));  // padding filters; padding channels are written
     launch_weight_frsc(w, d.dt, wt_.get(), d.dt, d.F, d.C, d.R, d.S, Cp, s);
     if (z.wflat) launch_weight_flat(w, wflat_.get(), d.dt, d.F, d.C, d.R * d.S, Cp, s);
-    if (z.wfrag) launch_weight_frag3x3(w, d.dt, wfrag_.get(), d.dt, d.F, d.C, s);
+    if (z.wfrag && d.R == 1) launch_weight_frag1x1(w, d.dt, wfrag_.get(), d.dt, d.F, d.C, s);
+    else if (z.wfrag) launch_weight_frag3x3(w, d.dt, wfrag_.get(), d.dt, d.F, d.C, s);
     if (z.wfrag32) launch_weight_frag32(w, d.dt, wfrag32_.get(), d.F, d.C, s);
   }
   if (gamma) {
