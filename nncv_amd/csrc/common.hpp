@@ -462,9 +462,9 @@ struct DetectArgs {
 void launch_yolo_detect(const DetectArgs& a, int dt, hipStream_t s);
 // The same with the 1x1 convolutions (fp16, no activation) that make the heads, all levels in one launch (detect_head.hip).
 struct DetectHeadLevel {
-  const void* in; const void* wt; const float* scale; const float* shift;  // [N][HW] pixels of `pix` elements; [rows][C], rows >= A * F
+  const void* in; const void* wt; const float* scale; const float* shift;  // [N][HW] pixels of `pix` elements; launch_weight_frag1x1's order, rows >= A * F
   int HW, W, pix, C, rows; long long box0; float stride; float anchor_wh[8];
-  unsigned in_bytes, wt_bytes; int tiles, first; float inv_tiles, inv_w;  // filled in by the launcher
+  unsigned in_bytes, wt_bytes; int tiles, first, run; float inv_tiles, inv_w;  // filled in by the launcher
 };
 struct DetectHeadArgs { DetectHeadLevel lv[3]; float* out; int levels, N, A, F; long long boxes_total; float inv_f; };
 bool detect_head_applicable(int A, int F, int C, long long in_bytes);

@@ -384,7 +384,13 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
            detect_head_applicable(d.K, d.F, channels_[c.in[0]], 0);
       made.push_back(h);
     }
-    for (int h : made) nodes_[std::max(h, 0)].head = ok;
+    for (int h : made) {
+      Node& c = nodes_[std::max(h, 0)];
+      c.head = ok;
+      if (!ok || dry_) continue;
+      c.wfrag.reset(weight_frag1x1_bytes(c.op.F, c.C), &pool_);
+      launch_weight_frag1x1(blob + (size_t)c.op.w * es, dt, c.wfrag.get(), dt, c.op.F, c.C, s);
+    }
   }
 
   // concatenation views
@@ -1036,7 +1042,7 @@ void Graph::forward_tail(int N, int H, int W, float* out, void* ws, hipStream_t 
         const int t = c.op.in[0];
         const Dims h = p.dims[t];
         DetectHeadLevel& v = d.lv[d.levels - 1 - k];  // (the later levels are the ones with more channels)
-        v.in = at(t); v.wt = c.wt.get(); v.scale = c.scale.as<float>(); v.shift = c.shift.as<float>();
+        v.in = at(t); v.wt = c.wfrag.get(); v.scale = c.scale.as<float>(); v.shift = c.shift.as<float>();
         v.HW = h.H * h.W; v.W = h.W; v.pix = pitch(t); v.C = h.C; v.rows = channels_[c.op.out]; v.box0 = box0; v.stride = detect_stride_[k];
         for (int q = 0; q < op.K * 2; ++q) v.anchor_wh[q] = detect_anchor_wh_[k * op.K * 2 + q];
         box0 += (long long)op.K * h.H * h.W;
