@@ -223,6 +223,10 @@ struct IgemmArgs {
   void* chain_out;
   int chain_f, chain_act, chain_ldo;
   bool chain_only;
+  // With two results: the first up_c channels of a pixel are those of another tensor [N][H/2][W/2] with pixels of up_pix elements, each of
+  // its pixels four times (up-sampling by two); or null.
+  const void* up_in;
+  int up_c, up_pix;
 };
 // in_dt: element type of in/wt (kF32 | kF16); out_dt: element type of out/residual.
 // Dispatches to the fast kernel (igemm_fast.hip) when C is a multiple of one K step and the
@@ -290,6 +294,8 @@ double conv3x3_narrow_us(const IgemmArgs& a);
 void launch_conv3x3_narrow(const IgemmArgs& a, hipStream_t s);
 // whether two 1x1 layers of C channels and F filters each over P pixels should compute the 1x1 layer behind the first one as well
 bool conv_ring_chains(long long P, int C, int F);
+// whether a launch of two such layers, alone or chained, takes its first up_c channels from another tensor (IgemmArgs::up_in)
+bool conv_ring_upsamples(const IgemmArgs& a, int up_c, int up_pix);
 bool conv_ring_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 double conv_ring_us(const IgemmArgs& a);
 bool conv_ring_beats_patch_s2(const IgemmArgs& a);

@@ -44,6 +44,7 @@ struct RingArgs {
   float inv_ohw, inv_ow, inv_tiles;
   const void* chain_wt; const float* chain_scale; const float* chain_shift; void* chain_out;  // the layer behind the first result (CH > 0)
   unsigned chain_bytes; int chain_act, chain_ldo, chain_only;
+  const void* up_in; unsigned up_bytes; int up_slabs, up_pix;                                 // slabs that come from another tensor (UP)
   const void* wfrag; const void* aux_wfrag; int groups, aux_groups, lead;  // the resident form's filters: 32-filter groups; bytes of padding
 };
 
@@ -51,7 +52,8 @@ enum { kPoint = 0, kLines = 1, kAny = 2 };  // 1x1 without padding; taps of whol
 
 // CH > 0: of two results the first one, 16 * CH channels, is the input of a further 1x1 layer with as many filters.  Its values are in LDS on
 // their way out, rounded; the workgroups that have all its channels multiply them there.
-template <int WP, int WF, int PB, int FB, int S, int MODE, int CH = 0>
+// UP: the first slabs are those of a tensor of half the size, whose up-sampled copy is never made.
+template <int WP, int WF, int PB, int FB, int S, int MODE, int CH = 0, bool UP = false>
 __global__ __launch_bounds__(64 * WP * WF) void conv_ring_kernel(const RingArgs a) {
   constexpr int kChain = 16 * CH, NB = CH / (2 * WF) > 0 ? CH / (2 * WF) : 1;  // blocks of 32 of those filters a wave takes
   static_assert(CH == 0 || (PB == 1 && MODE == kPoint && kChain <= 32 * WF * FB), "a tile has all channels of the first result");
@@ -132,11 +134,18 @@ __global__ __launch_bounds__(64 * WP * WF) void conv_ring_kernel(const RingArgs 
   float shv = 0.0f;
   if ((int)threadIdx.x < BF && f0 + (int)threadIdx.x < a.F && a.shift) shv = a.shift[f0 + threadIdx.x];
 
-  unsigned pbase[LP];
+  unsigned pbase[LP], ubase[UP ? LP : 1];
   int py[LP], px[LP];
+  const __amdgpu_buffer_rsrc_t rs_up = make_rsrc(UP ? a.up_in : a.in, UP ? a.up_bytes : 0u);
 #pragma unroll
   for (int i = 0; i < LP; ++i) {
     const int group = wave * LP + i, p = p0 + group * 8 + sub;
+    if constexpr (UP) {
+      int rem, x;
+      const int n = fast_div(p < a.P ? p : 0, a.OHW, a.inv_ohw, &rem), y = fast_div(rem, a.OW, a.inv_ow, &x);
+      const int from = (n * (a.H >> 1) + (y >> 1)) * (a.W >> 1) + (x >> 1);
+      ubase[i] = p < a.P ? (unsigned)(from * a.up_pix * 2 + column(group) * 16) : kOOBr;
+    }
     if constexpr (MODE == kPoint) {
       int at = p;  // result p reads pixel p (40 layers: 1.03x on average without the divisions, 7.1 -> 6.7 us for 64 -> 64 channels at 16x80x80)
       if ((a.stride_h | a.stride_w) != 1) {  // strided windows read every stride-th pixel
@@ -186,7 +195,8 @@ __global__ __launch_bounds__(64 * WP * WF) void conv_ring_kernel(const RingArgs 
         const bool ok = (8 * slab + column(group) < a.chunks) & ((unsigned)(py[i] + r) < (unsigned)a.H) & ((unsigned)(px[i] + s) < (unsigned)a.W);
         v = ok ? pbase[i] + (unsigned)((r * a.W + s) * a.pix * 2 + c * 16) : kOOBr;
       }
-      fetch16(rs_in, dst + group * 1024, v, MODE == kPoint ? soff : 0u);
+      if (UP && slab < a.up_slabs) fetch16(rs_up, dst + group * 1024, ubase[UP ? i : 0], soff);
+      else fetch16(rs_in, dst + group * 1024, v, MODE == kPoint ? soff : 0u);
     }
     ++slab;
     if constexpr (MODE == kLines) {
@@ -600,7 +610,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PB == 4 ? 2
 
 // ---- dispatch
 
-template <int WP, int WF, int PB, int FB, int S, int CH = 0>
+template <int WP, int WF, int PB, int FB, int S, int CH = 0, bool UP = false>
 void launch_cfg(RingArgs d, int mode, hipStream_t s) {
   constexpr int NW = WP * WF, BP = 32 * WP * PB, BF = 32 * WF * FB, ring = S * (BP + BF) * 128, tile = NW * PB * 32 * (FB * 64 + 16);
   constexpr int lds = (ring > tile ? ring : tile) + BF * 8 + 128 * CH;
@@ -617,7 +627,7 @@ void launch_cfg(RingArgs d, int mode, hipStream_t s) {
     (void)attr;
     launch_kernel(kern, dim3((unsigned)(d.aux_f0 ? (d.tiles_p + 7) / 8 * 8 * (d.tiles_f + d.aux_tiles) : d.tiles_f * d.tiles_p)), dim3(64 * NW), lds, s, d);
   };
-  if constexpr (CH > 0) return go(conv_ring_kernel<WP, WF, PB, FB, S, kPoint, CH>);
+  if constexpr (CH > 0 || UP) return go(conv_ring_kernel<WP, WF, PB, FB, S, kPoint, CH, UP>);
   if (mode == kPoint) go(conv_ring_kernel<WP, WF, PB, FB, S, kPoint>);
   else if (mode == kLines) go(conv_ring_kernel<WP, WF, PB, FB, S, kLines>);
   else go(conv_ring_kernel<WP, WF, PB, FB, S, kAny>);
@@ -689,7 +699,7 @@ bool point_serves(int dt, int F, int RS, int C, int stride, int pad) { return dt
 const Form kPointForm{64, 128, 4, 0, 0, 0, 0, 0, 0, launch_frag<2>, "conv_ring<64x128,point>", true};
 double point_us(const IgemmArgs& a) {  // 0: not taken
   const double tiles = std::ceil((double)a.N * a.OH * a.OW / 64) * std::ceil(a.F / 128.0), slabs = a.C / 64;
-  if (!a.wt_frag || !point_serves(kF16, a.F, a.R * a.S, a.C, a.stride_h, a.pad_h) || a.stride_w != 1 || a.pad_w != 0 || a.residual || a.aux_f0 || a.chain_wt || tiles < 112 || tiles > 400)
+  if (!a.wt_frag || !point_serves(kF16, a.F, a.R * a.S, a.C, a.stride_h, a.pad_h) || a.stride_w != 1 || a.pad_w != 0 || a.residual || a.aux_f0 || a.chain_f || tiles < 112 || tiles > 400)
     return 0;
   return tiles <= 256 ? 3.1 + 0.36 * slabs : 4.9 + 0.51 * slabs;
 }
@@ -773,6 +783,15 @@ bool conv_ring_beats_patch_s2(const IgemmArgs& a) {
 // With 128 channels the chained filters take the registers of a CU's second workgroup: 16x40x40x256 21.0 us against 11.5 + 6.7.
 bool conv_ring_chains(long long P, int C, int F) { return (F == 32 || F == 64) && C % 8 == 0 && P * F * 2 >= 2 << 20; }
 
+// The forms that have it: two slabs in the ring, tiles of 128 x 128, where those run anyway.  A lane reads its pixel or its quarter as easily:
+// 16x40x40x(256 + 256) -> 128 + 128 15.5 us, 15.9 behind a copy of 6.1; 16x80x80x(128 + 128) -> 64 + 64 -> 64 24.6, 25.1 behind 8.8.
+bool conv_ring_upsamples(const IgemmArgs& a, int up_c, int up_pix) {
+  double us = 0;
+  const bool form = a.chain_f ? a.chain_f == 64 && a.C > 128 : best_form(a, &us)->launch == static_cast<void (*)(RingArgs, int, hipStream_t)>(launch_cfg<4, 2, 1, 2, 2>);
+  return form && up_c % 64 == 0 && up_c > 0 && up_pix % 8 == 0 && a.H % 2 == 0 && a.W % 2 == 0 && a.OH == a.H && a.OW == a.W &&
+         (long long)a.N * (a.H / 2) * (a.W / 2) * up_pix * 2 < (long long)kOOBr;
+}
+
 double conv_ring_us(const IgemmArgs& a) {
   double us = 0;
   best_form(a, &us);
@@ -807,16 +826,27 @@ void launch_conv_ring(const IgemmArgs& a, hipStream_t s) {
   d.wfrag = a.wt_frag; d.aux_wfrag = a.aux_wt_frag;
   const double flops = a.alg_flops > 0 ? a.alg_flops : 2.0 * d.P * (double)a.F * a.R * a.S * a.C;
   const double bytes = 2.0 * ((double)a.N * a.H * a.W * a.C + (double)a.F * a.R * a.S * a.C + (double)d.P * a.F * (a.residual ? 2 : 1));
-  if (a.chain_wt) {
+  if (a.up_in) {
+    d.up_in = a.up_in; d.up_slabs = a.up_c / 64; d.up_pix = a.up_pix;
+    d.up_bytes = (unsigned)((long long)a.N * (a.H / 2) * (a.W / 2) * a.up_pix * 2);
+  }
+  if (a.chain_f) {
     d.chain_wt = a.chain_wt; d.chain_scale = a.chain_scale; d.chain_shift = a.chain_shift; d.chain_out = a.chain_out;
     d.chain_act = a.chain_act; d.chain_ldo = a.chain_ldo; d.chain_only = a.chain_only;
     d.chain_bytes = (unsigned)d.P * a.chain_ldo * 2u;
     d.pixels_first = false;
     ProfScope prof("conv_ring<chain>", flops + 2.0 * d.P * (double)a.chain_f * a.chain_f, bytes + 2.0 * d.P * (double)a.chain_f, s);
     const bool two = d.chunks > 16;  // (slabs in the ring: one up to 128 channels, as without the chained layer)
-    if (a.chain_f == 32) launch_cfg<2, 2, 1, 1, 1, 2>(d, kPoint, s);
+    if (a.up_in) launch_cfg<4, 2, 1, 2, 2, 4, true>(d, kPoint, s);
+    else if (a.chain_f == 32) launch_cfg<2, 2, 1, 1, 1, 2>(d, kPoint, s);
     else if (two) launch_cfg<4, 2, 1, 2, 2, 4>(d, kPoint, s);
     else launch_cfg<4, 2, 1, 2, 1, 4>(d, kPoint, s);
+    NNCV_HIP_CHECK(hipGetLastError());
+    return;
+  }
+  if (a.up_in) {
+    ProfScope prof("conv_ring<128x128,2,up>", flops, bytes, s);
+    launch_cfg<4, 2, 1, 2, 2, 0, true>(d, kPoint, s);
     NNCV_HIP_CHECK(hipGetLastError());
     return;
   }

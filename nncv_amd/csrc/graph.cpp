@@ -472,6 +472,14 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
       }
     }
   }
+  // an up-sampled tensor that is the beginning of a concatenated one, which two joined convolutions read and nothing else
+  static const bool no_up = getenv("NNCV_HIP_NO_UP_FUSION") != nullptr;
+  for (int u = 0; !no_up && u < n; ++u) {
+    const int t = ops[u].out, cat = view_of_[t];
+    if (ops[u].kind != NNCV_HIP_OP_UPSAMPLE2X || ops[u].in[0] == 0 || cat < 0 || view_c0_[t] != 0 || readers[t] != 1 || readers[cat] != 2 || view_of_[cat] >= 0) continue;
+    for (int i = u + 1; i < n; ++i)
+      if (ops[i].in[0] == cat && nodes_[i].joins >= 0 && ops[nodes_[i].joins].in[0] == cat) nodes_[i].ups = u, nodes_[u].upped_by = i;
+  }
 }
 
 void Graph::root_of(int t, int* root, int* c0) const {
@@ -581,6 +589,7 @@ const Graph::Plan& Graph::plan_of(int N, int H, int W) const {
     }
     if (nodes_[i].add_out >= 0) life[nodes_[i].add_out].first_op = std::min(life[nodes_[i].add_out].first_op, i + 1);
     if (nodes_[i].joins >= 0) life[nodes_[nodes_[i].joins].op.out].first_op = i + 1;  // (also where the shape is not joined)
+    if (nodes_[i].ups >= 0) life[nodes_[nodes_[i].ups].op.in[0]].last_op = std::max(life[nodes_[nodes_[i].ups].op.in[0]].last_op, i + 1);
     if (nodes_[i].chain >= 0) life[nodes_[nodes_[i].chain].op.out].first_op = i + 1;  // (likewise)
   }
   {
@@ -653,12 +662,15 @@ const Graph::Plan& Graph::plan_of(int N, int H, int W) const {
   // Joined convolutions: one launch where the LDS ring takes the doubled filters and both results lie within its reach.
   p.joint.assign(n, 0);
   p.chained.assign(n, 0);
+  p.upped.assign(n, 0);
   for (int i = 0; i < n; ++i) {
     if (nodes_[i].joins < 0) continue;
     const IgemmArgs g = joint_args(p, i, nullptr);
     p.joint[i] = g.in_bytes < 0x7fffff00u && !igemm_takes_direct(g, dt_, dt_) && conv_ring_applicable(g, dt_, dt_);
     const long long P = (long long)N * g.OH * g.OW;
     p.chained[i] = p.joint[i] && nodes_[i].chain >= 0 && conv_ring_chains(P, g.C, nodes_[i].op.F) && P * pitch(nodes_[nodes_[i].chain].op.out) * 2 < 0x7fffff00ll;
+    if (const int u = nodes_[i].ups; p.joint[i] && u >= 0)
+      p.upped[i] = conv_ring_upsamples(joint_args(p, i, nullptr), channels_[nodes_[u].op.out], pitch(nodes_[u].op.in[0]));
   }
   check_plan(p);
   if (plans_.size() >= 8) plans_.erase(plans_.begin());
@@ -717,6 +729,10 @@ IgemmArgs Graph::joint_args(const Plan& p, int i, char* base) const {
   const unsigned long long span = (unsigned long long)p.N * a.H * a.W * ldi * dtype_size(dt_);
   g.in_bytes = span < 0xffffffffull ? (unsigned)span : 0xffffffffu;
   g.out = base + p.offset[t]; g.ldo = pitch(t);
+  if (p.upped[i]) {
+    const GraphOp& u = nodes_[nd.ups].op;
+    g.up_in = base + p.offset[u.in[0]]; g.up_c = channels_[u.out]; g.up_pix = pitch(u.in[0]);
+  }
   if (p.chained[i]) {
     const Node& nk = nodes_[nd.chain];
     g.chain_wt = nk.wt.get(); g.chain_scale = nk.scale.as<float>(); g.chain_shift = nk.shift.as<float>();
@@ -740,7 +756,7 @@ void Graph::launch_io(const Plan& p, int i, std::vector<int>* writes, std::vecto
       if (op.in[k] >= 0) reads->push_back(maker(op.in[k])->op.in[0]);
     return;
   }
-  if ((nd.joined && joint_second(p, i)) || chained_third(p, i)) return;
+  if ((nd.joined && joint_second(p, i)) || chained_third(p, i) || (nd.upped_by >= 0 && p.upped[nd.upped_by])) return;
   if (i > 0 && p.pooled[i - 1]) return;
   if (p.pooled[i] || (i == n - 1 && p.last_f32)) {
     reads->push_back(op.in[0]);
@@ -749,6 +765,7 @@ void Graph::launch_io(const Plan& p, int i, std::vector<int>* writes, std::vecto
   }
   if (nd.joins >= 0 && p.joint[i]) {
     reads->push_back(op.in[0]);
+    if (p.upped[i]) reads->push_back(nodes_[nd.ups].op.in[0]);
     if (!(p.chained[i] && nd.chain_only)) writes->push_back(op.out);
     writes->push_back(nodes_[nd.joins].op.out);
     if (p.chained[i]) writes->push_back(nodes_[nd.chain].op.out);
@@ -884,7 +901,7 @@ void Graph::forward_body(const void* src, int N, int H, int W, void* ws, hipStre
       launch_image_pairs(image, s);
       continue;
     }
-    if (nd.skip || (nd.head && p.head) || (nd.joined && joint_second(p, (int)i)) || chained_third(p, (int)i)) continue;
+    if (nd.skip || (nd.head && p.head) || (nd.joined && joint_second(p, (int)i)) || chained_third(p, (int)i) || (nd.upped_by >= 0 && p.upped[nd.upped_by])) continue;
     if ((i > 0 && p.pooled[i - 1]) || (i + 1 == nodes_.size() && p.last_f32)) continue;
     if (p.pooled[i]) {
       ConvPoolArgs c{};

@@ -66,6 +66,8 @@ class Graph {
     int expands = -1, projects = -1;
     // 1x1 convolutions that may run as one launch (Plan::joint): on the first one, the index of the second
     int joins = -1;
+    int ups = -1;  // with `joins`: the UPSAMPLE2X whose result is the first channels of this one's input, which nothing else reads (Plan::upped)
+    int upped_by = -1;
     bool chain_only = false;  // nothing but `chain` reads this result
     int chained_by = -1;
     int chain = -1;  // with `joins`: a 1x1 CONV that reads this one's result and may be in that launch too (Plan::chained)
@@ -85,6 +87,7 @@ class Graph {
     bool head = false;               // the YOLO_DETECT launch computes the convolutions that it reads
     std::vector<char> pooled;        // per operator: its launch stores the means that the next operator is after, not the result
     bool last_f32 = false;           // the last operator is a convolution whose launch writes the caller's buffer
+    std::vector<char> upped;         // per operator: its launch reads what `ups` would have copied
     std::vector<char> chained;       // per operator: its launch, which computes the one it joins, computes `chain` as well
     std::vector<char> joint;         // per operator: its launch computes the one it joins as well
     size_t total;
