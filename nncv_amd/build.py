@@ -16,7 +16,7 @@ LIB = os.path.join(HERE, "lib", "libnncv_hip.so")
 RT_LIB = os.path.join(HERE, "lib", "libnncv_rt.so")
 DRIVER = os.path.join(HERE, "lib", "res18_main")
 
-DEVICE_SOURCES = ["igemm.hip", "igemm_fast.hip", "conv3x3_patch.hip", "conv3x3_split.hip", "conv3x3_f16.hip", "conv3x3_narrow.hip", "conv_pairs.hip", "conv_direct.hip", "conv_pool.hip", "conv_ring.hip", "conv3x3s2_resident.hip", "stem_pool.hip", "stem_pool_split.hip", "gemm_nn.hip", "gemm_split.hip", "winograd.hip", "pool_layout.hip", "elementwise.hip", "mobile_block.hip", "detect_head.hip", "noalloc.hip", "stream_probe.hip"]
+DEVICE_SOURCES = ["igemm.hip", "igemm_fast.hip", "conv3x3_patch.hip", "conv3x3_split.hip", "conv3x3_f16.hip", "conv3x3_narrow.hip", "conv_pairs.hip", "conv_direct.hip", "conv_pool.hip", "conv_ring.hip", "conv3x3s2_resident.hip", "basic_block.hip", "stem_pool.hip", "stem_pool_split.hip", "gemm_nn.hip", "gemm_split.hip", "winograd.hip", "pool_layout.hip", "elementwise.hip", "mobile_block.hip", "detect_head.hip", "noalloc.hip", "stream_probe.hip"]
 HOST_SOURCES = ["model.cpp", "capi.cpp", "datatype.cpp", "profiler.cpp", "arena_plan.cpp", "graph.cpp", "hostcopy.cpp"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -1,0 +1,258 @@
+// A residual block of 64 channels in one launch (gfx950, fp16): relu(bn2(conv2(relu(bn1(conv1(x))))) + x), both convolutions 3x3 stride 1 pad 1
+// (tests/Nets/Res18.mlir:152-203, :205-251), for many pixels.
+//
+//  * As two launches the block writes and reads a tensor between its convolutions and reads x twice: five times the tensor over memory.
+//    Here it is two: what lies between the convolutions stays in LDS, and x is there when it is added.  At 256x56x56 (118 GFLOP, 205 MB)
+//    it takes 120.8 us, 980 TFLOP/s, where the two launches (conv3x3_f16.hip's stream form, filters resident) took 153.5.
+//  * What bounds it: the matrix pipe and LDS, which the products need for the same time.  A step's 144 products of a SIMD are 4608 of its
+//    6100 cycles (56 pixels: 112 of 128 slots), and with 32 filters of a wave each 1 KB fragment of pixels read feeds one product, 128 B a
+//    cycle over four SIMDs.  64 filters a wave would halve the reads and need 288 registers for them: one wave a SIMD, nothing to run
+//    beside its epilogues.  The rest are the second convolution's results (1900 cycles, beside the first one's products) and the first
+//    one's epilogue (1300, beside the second one's products).  Wave priority for either of them made it slower (the pass lost 8 us).
+//  * A workgroup has a CU and a strip of whole rows of an image.  It walks down two rows at a time: four waves make two rows of the first
+//    convolution, four the two rows of the second one that the rows before have completed; a step later the next two.  Nothing but a
+//    strip's first and last row is computed twice.
+//  * A wave has 32 filters of its convolution for good, 144 registers of them, and 64 of the 128 slots of two rows.  Two waves share a
+//    SIMD, one of each convolution: the second one's begin a step with the results of the step before, the first one's end it with theirs,
+//    so that the matrix pipe has work from one or the other.
+//  * x comes by DMA (buffer_load ... lds) two steps ahead into a ring of five pairs of rows; the rows between the convolutions have a ring
+//    of three.  A cell is a pixel's 64 channels in 144 bytes, a row's pitch continues the sequence of its cells' units: reads of 16
+//    neighbouring slots are free of bank conflicts, across the end of a row too (conv3x3_f16.hip).  Cells left and right of a row are zeros.
+#include <algorithm>
+#include <type_traits>
+
+#include "mfma_tile.hpp"
+
+namespace nncv_hip {
+
+using namespace mt;
+
+namespace {
+
+constexpr unsigned kOOBb = 0x7fffff00u;  // byte offset beyond any buffer this kernel accepts
+constexpr int kCell = 144, kInBlocks = 5, kMidBlocks = 3, kMostW = 64;
+constexpr int kEach = 3;  // load instructions of a wave for a pair of rows, at most
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
+__device__ __forceinline__ void fetch16(__amdgpu_buffer_rsrc_t rs, unsigned char* lds, unsigned voffset) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)lds, 16, voffset, 0, 0, 0);
+}
+constexpr int row_bytes(int W) { return (W + 2) * kCell + 224; }                       // = W * 144 modulo 256
+constexpr int in_block(int W) { return (2 * row_bytes(W) + 1023) / 1024 * 1024; }      // whole load instructions
+static_assert(2 * row_bytes(kMostW) <= kEach * 8 * 1024, "a pair of rows is three instructions a wave");
+
+struct BlockArgs {
+  const void* in; void* out; const void* wf1; const void* wf2;
+  const float* scale1; const float* shift1; const float* scale2; const float* shift2;
+  int H, W, strips, rows;  // strips of an image, their rows (even)
+  float inv_row;           // 1 / 16-byte units of a row
+};
+
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void basic_block_kernel(const BlockArgs a) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int W = a.W, H = a.H, rowB = (W + 2) * kCell + 224, inB = (2 * rowB + 1023) & ~1023, midB = 2 * rowB;
+  const int mid0 = kInBlocks * inB;
+  float* tab = reinterpret_cast<float*>(smem + mid0 + kMidBlocks * midB);  // scale and shift of both
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lrow = lane & 31, lh = lane >> 5, second = wave >> 2, fg = wave & 1, half = (wave >> 1) & 1;
+  const int n = blockIdx.x / a.strips, strip = blockIdx.x - n * a.strips;
+  const int y0 = strip * a.rows, y1 = min(y0 + a.rows, H), K = (y1 - y0 + 1) >> 1;  // pairs of rows of the result
+  const long long image = (long long)n * H * W * 128;
+  const __amdgpu_buffer_rsrc_t rs_in = make_rsrc(static_cast<const char*>(a.in) + image, (unsigned)(H * W) * 128u);
+  const __amdgpu_buffer_rsrc_t rs_out = make_rsrc(static_cast<char*>(a.out) + image, (unsigned)(H * W) * 128u);
+
+  // ---- loader: unit u of a pair of rows is part of a cell, of the spare 16 bytes behind it or of those behind the row ----
+  const int units = rowB >> 4, calls = inB >> 10;
+  unsigned from[kEach];
+  int frow[kEach];
+#pragma unroll
+  for (int i = 0; i < kEach; ++i) {
+    int v;
+    const int u = (i * 8 + wave) * 64 + lane, r = fast_div(u, units, a.inv_row, &v), cell = (v * 7282) >> 16, part = v - cell * 9;
+    const bool ok = r < 2 && part < 8 && cell >= 1 && cell <= W;
+    from[i] = (unsigned)((r * W + cell - 1) * 128 + part * 16);
+    frow[i] = ok ? r : 1 << 28;
+  }
+  auto fetch = [&](int b, int slot) __attribute__((always_inline)) {  // pair b of the input: rows y0 - 2 + 2 b ..
+    const int y = y0 - 2 + 2 * b;
+#pragma unroll
+    for (int i = 0; i < kEach; ++i)
+      if (i * 8 + wave < calls) fetch16(rs_in, smem + slot * inB + (i * 8 + wave) * 1024, (unsigned)(y + frow[i]) < (unsigned)H ? (unsigned)(y * W * 128) + from[i] : kOOBb);
+  };
+  fetch(0, 0);
+  fetch(1, 1);
+  u32x4 w[36];
+  {
+    const __amdgpu_buffer_rsrc_t rs_w = make_rsrc(second ? a.wf2 : a.wf1, 2u * 36u * 1024u);
+#pragma unroll
+    for (int q = 0; q < 36; ++q) w[q] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, (unsigned)lane * 16u, (unsigned)((fg * 36 + q) * 1024), 0);
+  }
+  if (tid < 64) {
+    tab[tid] = a.scale1[tid], tab[64 + tid] = a.shift1[tid];
+    tab[128 + tid] = a.scale2[tid], tab[192 + tid] = a.shift2[tid];
+  }
+  for (int i = tid * 16; i < kMidBlocks * midB; i += 512 * 16) *reinterpret_cast<u32x4*>(smem + mid0 + i) = u32x4{0, 0, 0, 0};
+
+  // ---- this lane's two slots: pixel x of row i of the pair; slots behind the last pixel read with one 16, 32 .. before them ----
+  int xs[2], is[2];
+  bool there[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    int s = (2 * half + u) * 32 + lrow;
+    there[u] = s < 2 * W;
+    if (s >= 2 * W) s -= (((s - 2 * W) >> 4) + 1) << 4;
+    is[u] = s >= W ? 1 : 0;
+    xs[u] = s - is[u] * W;
+  }
+  // byte of tap (r, 0) of a slot: pair t (first convolution: of the input; second: of the rows between) and the one behind it
+  const int block = second ? midB : inB, ring0 = second ? mid0 : 0, ring_end = ring0 + (second ? kMidBlocks * midB : kInBlocks * inB), ring = ring_end - ring0;
+  int base[3][2];
+#pragma unroll
+  for (int r = 0; r < 3; ++r)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int j = is[u] + r;
+      base[r][u] = ring0 + (j >> 1) * block + (j & 1) * rowB + xs[u] * kCell + lh * 16;
+    }
+  const int f0 = fg * 32 + 16 * lh;  // this lane's 16 consecutive channels
+  const float* sc = tab + second * 128 + f0;
+  floatx16 acc[2];
+  int slot_in = 2, slot_mid = 0, slot_res = 1;  // of the pair to fetch, to write between the convolutions, of the pair of x to add
+
+  auto scaled = [&](int u, float (&y)[16]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const floatx4 m = *reinterpret_cast<const floatx4*>(sc + 4 * q), h = *reinterpret_cast<const floatx4*>(sc + 64 + 4 * q);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[4 * q + e] = acc[u][4 * q + e] * m[e] + h[e];
+    }
+  };
+  auto halves = [](const float (&y)[16], int c) __attribute__((always_inline)) {
+    half8 v;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = (half_t)y[8 * c + e];
+    return __builtin_bit_cast(u32x4, v);
+  };
+  // the first convolution's rows y0 - 1 + 2 t ..: to LDS, zeros where they lie outside the image
+  auto between = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      float y[16];
+      scaled(u, y);
+      act_apply_n<true>(y, kActRelu);
+      const bool inside = (unsigned)(y0 - 1 + 2 * t + is[u]) < (unsigned)H;
+      unsigned char* to = smem + mid0 + slot_mid * midB + is[u] * rowB + (xs[u] + 1) * kCell + f0 * 2;
+      if (there[u]) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) *reinterpret_cast<u32x4*>(to + 16 * c) = inside ? halves(y, c) : u32x4{0, 0, 0, 0};
+      }
+    }
+    slot_mid = slot_mid == kMidBlocks - 1 ? 0 : slot_mid + 1;
+  };
+  // the second one's rows y0 + 2 k ..: x added, to memory (always four stores)
+  auto result = [&](int k) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      float y[16];
+      scaled(u, y);
+      const unsigned char* x = smem + slot_res * inB + is[u] * rowB + (xs[u] + 1) * kCell + f0 * 2;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const half8 v = *reinterpret_cast<const half8*>(x + 16 * c);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[8 * c + e] += (float)v[e];
+      }
+      act_apply_n<true>(y, kActRelu);
+      const int yo = y0 + 2 * k + is[u];
+      const unsigned o = there[u] && yo < y1 ? (unsigned)((yo * W + xs[u]) * 128 + f0 * 2) : kOOBb;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) __builtin_amdgcn_raw_buffer_store_b128(halves(y, c), rs_out, o + 16u * c, 0, 0);
+    }
+    slot_res = slot_res == kInBlocks - 1 ? 0 : slot_res + 1;
+  };
+  auto products = [&]() __attribute__((always_inline)) {
+    constexpr int kAhead = 2;
+    u32x4 p[36][2];
+    auto read = [&](auto q_c) __attribute__((always_inline)) {
+      constexpr int q = decltype(q_c)::value, tap = q >> 2;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) p[q][u] = *reinterpret_cast<const u32x4*>(smem + base[tap / 3][u] + (tap % 3) * kCell + (q & 3) * 32);
+    };
+    read(std::integral_constant<int, 0>());
+    read(std::integral_constant<int, 1>());
+    auto steps = [&](auto self, auto q_c) __attribute__((always_inline)) -> void {
+      constexpr int q = decltype(q_c)::value;
+      if constexpr (q < 36) {
+        if constexpr (q + kAhead < 36) read(std::integral_constant<int, q + kAhead>());
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          if constexpr (q == 0) Mma<half_t>::start(w[q], p[q][u], acc[u]);
+          else Mma<half_t>::run(w[q], p[q][u], acc[u]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        self(self, std::integral_constant<int, q + 1>());
+      }
+    };
+    steps(steps, std::integral_constant<int, 0>());
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int v = base[r][u] + block;
+        base[r][u] = v >= ring_end ? v - ring : v;
+      }
+  };
+
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // filters and the first two pairs of rows: waited for where they are used, every step would count them
+  // Step t: the first convolution's pair t (t <= K), the second one's pair t - 2, and the results of its pair t - 3.
+  for (int t = 0; t < K + 3; ++t) {
+    __builtin_amdgcn_sched_barrier(0);
+    if (second && t > 3) __builtin_amdgcn_s_waitcnt(0xc07f & (0x0f70 | 4));  // x's next pair of rows (the last step's four stores may be on their way), LDS
+    else __builtin_amdgcn_s_waitcnt(0x0070);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    if (t + 2 <= K + 1) {
+      fetch(t + 2, slot_in);
+      slot_in = slot_in == kInBlocks - 1 ? 0 : slot_in + 1;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (second && t > 2) result(t - 3);
+    if (second ? t >= 2 && t < K + 2 : t <= K) products();
+    if (!second && t <= K) between(t);
+  }
+}
+
+}  // namespace
+
+bool basic_block_applicable(int N, int H, int W) { return W >= 8 && W <= kMostW && H >= 2 && (long long)H * W * 128 < (long long)kOOBb && N < (1 << 20); }
+
+void launch_basic_block(const BasicBlockArgs& g, hipStream_t s) {
+  NNCV_REQUIRE(basic_block_applicable(g.N, g.H, g.W), "basic_block: shape not covered");
+  BlockArgs d{};
+  d.in = g.in; d.out = g.out; d.wf1 = g.wf1; d.wf2 = g.wf2; d.scale1 = g.scale1; d.shift1 = g.shift1; d.scale2 = g.scale2; d.shift2 = g.shift2;
+  d.H = g.H; d.W = g.W;
+  int strips = 1;
+  double best = 1e30;
+  for (int c = 1; c <= (g.H + 1) / 2; ++c) {
+    const int rows = ((g.H + c - 1) / c + 1) / 2 * 2;
+    if ((c - 1) * rows >= g.H) continue;
+    const double us = std::ceil((double)g.N * c / 256) * (rows / 2 + 5);
+    if (us < best) best = us, strips = c, d.rows = rows;
+  }
+  d.strips = strips;
+  d.inv_row = 1.0f / (float)(row_bytes(g.W) / 16);
+  const int lds = kInBlocks * in_block(g.W) + kMidBlocks * 2 * row_bytes(g.W) + 1024;
+  static const bool attr = [] {
+    NNCV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(basic_block_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       kInBlocks * in_block(kMostW) + kMidBlocks * 2 * row_bytes(kMostW) + 1024));
+    return true;
+  }();
+  (void)attr;
+  const double px = (double)g.N * g.H * g.W;
+  ProfScope prof("basic_block<f16,64>", 4.0 * px * 9 * 64 * 64, 2.0 * (2 * px * 64 + 2 * 9 * 64 * 64), s);
+  launch_kernel(basic_block_kernel, dim3((unsigned)(g.N * strips)), dim3(512), lds, s, d);
+  NNCV_HIP_CHECK(hipGetLastError());
+}
+
+}  // namespace nncv_hip

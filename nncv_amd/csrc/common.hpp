@@ -432,6 +432,15 @@ struct SeProjectArgs {
 bool se_project_applicable(int HW, int C, int SQ, int F);
 void launch_transpose_half(const void* w, void* dst, int rows, int cols, hipStream_t s);  // [rows][cols] -> [cols][rows]
 void launch_se_project(const SeProjectArgs& a, hipStream_t s);
+// out = relu(scale2 * conv2(relu(scale1 * conv1(in) + shift1)) + shift2 + in), both 3x3 stride 1 pad 1 over 64 channels, fp16 NHWC (basic_block.hip);
+// wf1, wf2: launch_weight_frag32's order
+struct BasicBlockArgs {
+  const void* in; void* out; const void* wf1; const void* wf2;
+  const float* scale1; const float* shift1; const float* scale2; const float* shift2;
+  int N, H, W;
+};
+bool basic_block_applicable(int N, int H, int W);
+void launch_basic_block(const BasicBlockArgs& a, hipStream_t s);
 // out[n][f] = mean over HW of act(scale * (wt . in) + shift), fp16 (conv_pool.hip): in [N][HW] pixels of `pix` elements, wt [F][C]
 struct ConvPoolArgs {
   const void* in; const void* wt; const float* scale; const float* shift; void* out;

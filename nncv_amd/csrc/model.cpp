@@ -169,6 +169,28 @@ bool ConvLayer::forward_stem_pool(const void* in, int N, int H, int W, void* poo
   return true;
 }
 
+bool ConvLayer::forward_block(const ConvLayer& second, const void* in, int N, int H, int W, void* out, hipStream_t s) const {
+  auto fits = [](const ConvLayer& c) {
+    const Desc& d = c.d_;
+    return !d.stem && c.algo_ == kAlgoIgemm && d.dt == kF16 && d.C == 64 && d.F == 64 && d.R == 3 && d.S == 3 && d.stride == 1 && d.pad == 1 && d.relu == kActRelu &&
+           c.wfrag32_.get() && c.scale_.get();
+  };
+  if (!fits(*this) || !fits(second) || !basic_block_applicable(N, H, W)) return false;
+  // Against the two launches of conv3x3_f16.hip, a whole ResNet-18 pass in microseconds, theirs first:
+  //  * W: the kernel works on 128 slots, two rows.  256 images: W = 24 328 against 350, 32 448 against 469, 40 624 against
+  //    623, 44 769 against 722, 48 887 against 837, 56 1032 against 976, 64 1440 against 1223.
+  //  * Pairs of rows for each CU: a strip pays five steps beyond its own.  W = 56: 1.8 of them (16 images) 179 against 176, 4.4 (40) 294
+  //    against 280, 7 (64) 352 against 333; four is the line, and up to 32 images of 224x224 keep the launches they had.  W > 56, where
+  //    two rows are nearly the 128 slots and the stream form's tile of a row is two thirds full: 1 image of 256x256 122 against 118, 8
+  //    165 against 155, 16 of 240x240 188 against 185, so any number.
+  //  * Three and more passes in flight, each workgroup of this kernel with a CU to itself: 48 images of 224x224 (5.3 pairs) 642 against
+  //    653 us for three passes, 64 (7) 1075 against 1044 for four, 128 1971 against 1850, 64 of 256x256 1313 against 1176.
+  const long long pairs = (long long)N * ((H + 1) / 2), cus = 256;
+  if (W < 44 || pairs < (overlap_hint() >= 3 ? 6 * cus : W > 56 ? 0 : 4 * cus)) return false;
+  launch_basic_block(BasicBlockArgs{in, out, wfrag32_.get(), second.wfrag32_.get(), scale_.as<float>(), shift_.as<float>(), second.scale_.as<float>(), second.shift_.as<float>(), N, H, W}, s);
+  return true;
+}
+
 bool ConvLayer::fuse_shortcut(const ConvLayer& ds, hipStream_t s) {
   const Desc& q = ds.d_;
   const size_t es = dtype_size(d_.dt);
@@ -391,7 +413,10 @@ void ResNet18::forward_body(const void* src, int N, int H, int W, void* ws, hipS
     char* y2 = base + p.x[nblk + 1];
     const int oh = b.c1->out_h(h), ow = b.c1->out_w(w);
     const void* shortcut = x;
-    if (b.ds && b.c1->has_shortcut()) {
+    const bool whole = !b.ds && b.c1->forward_block(*b.c2, x, N, h, w, y2, s);
+    if (whole) {
+      // y1 is never stored
+    } else if (b.ds && b.c1->has_shortcut()) {
       b.c1->forward_with_shortcut(x, N, h, w, y1, idn, cws, s);
       shortcut = idn;
     } else {
@@ -401,7 +426,7 @@ void ResNet18::forward_body(const void* src, int N, int H, int W, void* ws, hipS
         shortcut = idn;
       }
     }
-    b.c2->forward(y1, N, oh, ow, shortcut, y2, cws, s);
+    if (!whole) b.c2->forward(y1, N, oh, ow, shortcut, y2, cws, s);
     h = oh; w = ow;
     ch = b.c2->desc().F;
     ++nblk;

@@ -57,6 +57,9 @@ class ConvLayer {
   // forward() of this layer into `out` and of the fused shortcut into `shortcut_out`
   void forward_with_shortcut(const void* in, int N, int H, int W, void* out, void* shortcut_out, void* ws, hipStream_t s) const;
 
+  // this layer, `second` behind it and the sum with `in` in one launch; false: not covered, or slower
+  bool forward_block(const ConvLayer& second, const void* in, int N, int H, int W, void* out, hipStream_t s) const;
+
  private:
   // bytes of each array a layer keeps, 0: not kept
   struct Sizes { size_t wt, wflat, wfrag, wfrag32, U, wstrip, scale; };
