@@ -9,14 +9,16 @@
 //    cycle over four SIMDs.  64 filters a wave would halve the reads and need 288 registers for them: one wave a SIMD, nothing to run
 //    beside its epilogues.  The rest are the second convolution's results (1900 cycles, beside the first one's products) and the first
 //    one's epilogue (1300, beside the second one's products).  Wave priority for either of them made it slower (the pass lost 8 us).
-//  * A workgroup has a CU and a strip of whole rows of an image.  It walks down two rows at a time: four waves make two rows of the first
-//    convolution, four the two rows of the second one that the rows before have completed; a step later the next two.  Nothing but a
-//    strip's first and last row is computed twice.
-//  * A wave has 32 filters of its convolution for good, 144 registers of them, and 64 of the 128 slots of two rows.  Two waves share a
+//  * A workgroup has a CU and a strip of whole rows of an image.  It walks down in steps of two rows (W > 42), three (W > 32) or four, so that
+//    they fill most of 128 slots: four waves make a step's rows of the first convolution, four the rows of the second one that the steps
+//    before have completed; a step later the next.  Nothing but a strip's first and last row is computed twice.  With two rows a step,
+//    256 images of 128x128 lost 21 us of a pass of 448 to the two launches and 160x160 gained one; with four and three it gains 15 and 32.
+//  * A wave has 32 filters of its convolution for good, 144 registers of them, and 64 of the 128 slots.  Two waves share a
 //    SIMD, one of each convolution: the second one's begin a step with the results of the step before, the first one's end it with theirs,
 //    so that the matrix pipe has work from one or the other.
-//  * x comes by DMA (buffer_load ... lds) two steps ahead into a ring of five pairs of rows; the rows between the convolutions have a ring
-//    of three.  A cell is a pixel's 64 channels in 144 bytes, a row's pitch continues the sequence of its cells' units: reads of 16
+//  * x comes by DMA (buffer_load ... lds) two steps ahead into a ring of five steps' rows; the rows between the convolutions have a ring
+//    of three.  With two rows a step the x that results add is the second of two blocks and stays one step less; with three and four
+//    (TALL) the results read the block whose place the next one takes, so that fetch waits for them in the middle of the step.  A cell is a pixel's 64 channels in 144 bytes, a row's pitch continues the sequence of its cells' units: reads of 16
 //    neighbouring slots are free of bank conflicts, across the end of a row too (conv3x3_f16.hip).  Cells left and right of a row are zeros.
 #include <algorithm>
 #include <type_traits>
@@ -37,25 +39,35 @@ __device__ __forceinline__ void fetch16(__amdgpu_buffer_rsrc_t rs, unsigned char
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)lds, 16, voffset, 0, 0, 0);
 }
 constexpr int row_bytes(int W) { return (W + 2) * kCell + 224; }                       // = W * 144 modulo 256
-constexpr int in_block(int W) { return (2 * row_bytes(W) + 1023) / 1024 * 1024; }      // whole load instructions
-static_assert(2 * row_bytes(kMostW) <= kEach * 8 * 1024, "a pair of rows is three instructions a wave");
+constexpr int in_block(int W, int R) { return (R * row_bytes(W) + 1023) / 1024 * 1024; }  // whole load instructions
+constexpr int step_rows(int W) { return W <= 32 ? 4 : W <= 42 ? 3 : 2; }
+constexpr int lds_bytes(int W) {
+  const int R = step_rows(W);
+  return kInBlocks * in_block(W, R) + kMidBlocks * R * row_bytes(W) + (R == 2 ? 1024 : 0);
+}
+static_assert(lds_bytes(32) <= 160 * 1024 && lds_bytes(42) <= 160 * 1024 && lds_bytes(kMostW) <= 160 * 1024, "LDS of a CU");
+static_assert(in_block(32, 4) <= kEach * 8 * 1024 && in_block(42, 3) <= kEach * 8 * 1024 && in_block(kMostW, 2) <= kEach * 8 * 1024, "a step's rows are three instructions a wave");
 
 struct BlockArgs {
   const void* in; void* out; const void* wf1; const void* wf2;
   const float* scale1; const float* shift1; const float* scale2; const float* shift2;
-  int H, W, strips, rows;  // strips of an image, their rows (even)
+  int H, W, R, strips, rows;  // rows of a step, strips of an image, their rows (whole steps)
   float inv_row;           // 1 / 16-byte units of a row
 };
 
+template <bool TALL>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void basic_block_kernel(const BlockArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
-  const int W = a.W, H = a.H, rowB = (W + 2) * kCell + 224, inB = (2 * rowB + 1023) & ~1023, midB = 2 * rowB;
+  const int W = a.W, H = a.H, R = TALL ? a.R : 2, rowB = (W + 2) * kCell + 224, inB = (R * rowB + 1023) & ~1023, midB = R * rowB;
   const int mid0 = kInBlocks * inB;
-  float* tab = reinterpret_cast<float*>(smem + mid0 + kMidBlocks * midB);  // scale and shift of both
+  // scale and shift of both, in pieces of 32 channels: behind the rows; TALL: a piece in what is spare behind each of the first eight of them
+  auto tab = [&](int piece) __attribute__((always_inline)) {
+    return reinterpret_cast<float*>(smem + mid0 + (TALL ? piece * rowB + (W + 2) * kCell : kMidBlocks * midB + piece * 128));
+  };
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 31, lh = lane >> 5, second = wave >> 2, fg = wave & 1, half = (wave >> 1) & 1;
   const int n = blockIdx.x / a.strips, strip = blockIdx.x - n * a.strips;
-  const int y0 = strip * a.rows, y1 = min(y0 + a.rows, H), K = (y1 - y0 + 1) >> 1;  // pairs of rows of the result
+  const int y0 = strip * a.rows, y1 = min(y0 + a.rows, H), K = (y1 - y0 + R - 1) / R;  // steps' rows of the result
   const long long image = (long long)n * H * W * 128;
   const __amdgpu_buffer_rsrc_t rs_in = make_rsrc(static_cast<const char*>(a.in) + image, (unsigned)(H * W) * 128u);
   const __amdgpu_buffer_rsrc_t rs_out = make_rsrc(static_cast<char*>(a.out) + image, (unsigned)(H * W) * 128u);
@@ -68,12 +80,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   for (int i = 0; i < kEach; ++i) {
     int v;
     const int u = (i * 8 + wave) * 64 + lane, r = fast_div(u, units, a.inv_row, &v), cell = (v * 7282) >> 16, part = v - cell * 9;
-    const bool ok = r < 2 && part < 8 && cell >= 1 && cell <= W;
+    const bool ok = r < R && part < 8 && cell >= 1 && cell <= W;
     from[i] = (unsigned)((r * W + cell - 1) * 128 + part * 16);
     frow[i] = ok ? r : 1 << 28;
   }
-  auto fetch = [&](int b, int slot) __attribute__((always_inline)) {  // pair b of the input: rows y0 - 2 + 2 b ..
-    const int y = y0 - 2 + 2 * b;
+  auto fetch = [&](int b, int slot) __attribute__((always_inline)) {  // block b of the input: rows y0 - 2 + R b ..
+    const int y = y0 - 2 + R * b;
 #pragma unroll
     for (int i = 0; i < kEach; ++i)
       if (i * 8 + wave < calls) fetch16(rs_in, smem + slot * inB + (i * 8 + wave) * 1024, (unsigned)(y + frow[i]) < (unsigned)H ? (unsigned)(y * W * 128) + from[i] : kOOBb);
@@ -86,24 +98,27 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int q = 0; q < 36; ++q) w[q] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, (unsigned)lane * 16u, (unsigned)((fg * 36 + q) * 1024), 0);
   }
-  if (tid < 64) {
-    tab[tid] = a.scale1[tid], tab[64 + tid] = a.shift1[tid];
-    tab[128 + tid] = a.scale2[tid], tab[192 + tid] = a.shift2[tid];
-  }
   for (int i = tid * 16; i < kMidBlocks * midB; i += 512 * 16) *reinterpret_cast<u32x4*>(smem + mid0 + i) = u32x4{0, 0, 0, 0};
+  if constexpr (TALL) __syncthreads();
+  if (tid < 64) {
+    const int h = tid >> 5, f = tid & 31;
+    tab(h)[f] = a.scale1[tid], tab(2 + h)[f] = a.shift1[tid];
+    tab(4 + h)[f] = a.scale2[tid], tab(6 + h)[f] = a.shift2[tid];
+  }
 
-  // ---- this lane's two slots: pixel x of row i of the pair; slots behind the last pixel read with one 16, 32 .. before them ----
+  // ---- this lane's two slots: pixel x of row i of the block; slots behind the last pixel read with one 16, 32 .. before them ----
   int xs[2], is[2];
   bool there[2];
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     int s = (2 * half + u) * 32 + lrow;
-    there[u] = s < 2 * W;
-    if (s >= 2 * W) s -= (((s - 2 * W) >> 4) + 1) << 4;
+    there[u] = s < R * W;
+    if (s >= R * W) s -= (((s - R * W) >> 4) + 1) << 4;
     is[u] = s >= W ? 1 : 0;
+    if constexpr (TALL) is[u] += (s >= 2 * W ? 1 : 0) + (s >= 3 * W ? 1 : 0);
     xs[u] = s - is[u] * W;
   }
-  // byte of tap (r, 0) of a slot: pair t (first convolution: of the input; second: of the rows between) and the one behind it
+  // byte of tap (r, 0) of a slot: block t (first convolution: of the input; second: of the rows between) and two rows of the one behind it
   const int block = second ? midB : inB, ring0 = second ? mid0 : 0, ring_end = ring0 + (second ? kMidBlocks * midB : kInBlocks * inB), ring = ring_end - ring0;
   int base[3][2];
 #pragma unroll
@@ -111,17 +126,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int j = is[u] + r;
-      base[r][u] = ring0 + (j >> 1) * block + (j & 1) * rowB + xs[u] * kCell + lh * 16;
+      base[r][u] = ring0 + (j >= R ? block + (j - R) * rowB : j * rowB) + xs[u] * kCell + lh * 16;
     }
   const int f0 = fg * 32 + 16 * lh;  // this lane's 16 consecutive channels
-  const float* sc = tab + second * 128 + f0;
+  const float *sc = tab(second * 4 + fg) + 16 * lh, *sh = tab(second * 4 + 2 + fg) + 16 * lh;
   floatx16 acc[2];
-  int slot_in = 2, slot_mid = 0, slot_res = 1;  // of the pair to fetch, to write between the convolutions, of the pair of x to add
+  int slot_in = 2, slot_mid = 0, slot_res = TALL ? 0 : 1;  // of the block to fetch, to write between the convolutions, of the (first) block of x to add
 
   auto scaled = [&](int u, float (&y)[16]) __attribute__((always_inline)) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const floatx4 m = *reinterpret_cast<const floatx4*>(sc + 4 * q), h = *reinterpret_cast<const floatx4*>(sc + 64 + 4 * q);
+      const floatx4 m = *reinterpret_cast<const floatx4*>(sc + 4 * q), h = *reinterpret_cast<const floatx4*>(sh + 4 * q);
 #pragma unroll
       for (int e = 0; e < 4; ++e) y[4 * q + e] = acc[u][4 * q + e] * m[e] + h[e];
     }
@@ -132,14 +147,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int e = 0; e < 8; ++e) v[e] = (half_t)y[8 * c + e];
     return __builtin_bit_cast(u32x4, v);
   };
-  // the first convolution's rows y0 - 1 + 2 t ..: to LDS, zeros where they lie outside the image
+  // the first convolution's rows y0 - 1 + R t ..: to LDS, zeros where they lie outside the image
   auto between = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       float y[16];
       scaled(u, y);
       act_apply_n<true>(y, kActRelu);
-      const bool inside = (unsigned)(y0 - 1 + 2 * t + is[u]) < (unsigned)H;
+      const bool inside = (unsigned)(y0 - 1 + R * t + is[u]) < (unsigned)H;
       unsigned char* to = smem + mid0 + slot_mid * midB + is[u] * rowB + (xs[u] + 1) * kCell + f0 * 2;
       if (there[u]) {
 #pragma unroll
@@ -148,13 +163,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     slot_mid = slot_mid == kMidBlocks - 1 ? 0 : slot_mid + 1;
   };
-  // the second one's rows y0 + 2 k ..: x added, to memory (always four stores)
+  // the second one's rows y0 + R k ..: x (from row 2 of block k on) added, to memory (always four stores)
   auto result = [&](int k) __attribute__((always_inline)) {
+    const int next = slot_res == kInBlocks - 1 ? 0 : slot_res + 1;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       float y[16];
       scaled(u, y);
-      const unsigned char* x = smem + slot_res * inB + is[u] * rowB + (xs[u] + 1) * kCell + f0 * 2;
+      int xrow = slot_res * inB + is[u] * rowB;
+      if constexpr (TALL) xrow = is[u] + 2 < R ? xrow + 2 * rowB : next * inB + (is[u] + 2 - R) * rowB;
+      const unsigned char* x = smem + xrow + (xs[u] + 1) * kCell + f0 * 2;
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
         const half8 v = *reinterpret_cast<const half8*>(x + 16 * c);
@@ -162,14 +180,29 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int e = 0; e < 8; ++e) y[8 * c + e] += (float)v[e];
       }
       act_apply_n<true>(y, kActRelu);
-      const int yo = y0 + 2 * k + is[u];
+      const int yo = y0 + R * k + is[u];
       const unsigned o = there[u] && yo < y1 ? (unsigned)((yo * W + xs[u]) * 128 + f0 * 2) : kOOBb;
 #pragma unroll
       for (int c = 0; c < 2; ++c) __builtin_amdgcn_raw_buffer_store_b128(halves(y, c), rs_out, o + 16u * c, 0, 0);
     }
-    slot_res = slot_res == kInBlocks - 1 ? 0 : slot_res + 1;
+    slot_res = next;
   };
-  auto products = [&]() __attribute__((always_inline)) {
+  auto fetch_next = [&](int t) __attribute__((always_inline)) {
+    if (t + 2 <= K + 1) {
+      fetch(t + 2, slot_in);
+      slot_in = slot_in == kInBlocks - 1 ? 0 : slot_in + 1;
+    }
+  };
+  // TALL: results read x from the block whose place the next one takes
+  auto results_read = [&](int t) __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    fetch_next(t);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto products = [&](int t) __attribute__((always_inline)) {
     constexpr int kAhead = 2;
     u32x4 p[36][2];
     auto read = [&](auto q_c) __attribute__((always_inline)) {
@@ -190,6 +223,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           else Mma<half_t>::run(w[q], p[q][u], acc[u]);
         }
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (TALL && q == 24) {
+          if (!second) results_read(t);
+        }
         self(self, std::integral_constant<int, q + 1>());
       }
     };
@@ -204,54 +240,60 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   };
 
   __builtin_amdgcn_s_waitcnt(0x0f70);  // filters and the first two pairs of rows: waited for where they are used, every step would count them
-  // Step t: the first convolution's pair t (t <= K), the second one's pair t - 2, and the results of its pair t - 3.
+  // Step t: the first convolution's block t (t <= K), the second one's block t - 2, and the results of its block t - 3.
   for (int t = 0; t < K + 3; ++t) {
     __builtin_amdgcn_sched_barrier(0);
-    if (second && t > 3) __builtin_amdgcn_s_waitcnt(0xc07f & (0x0f70 | 4));  // x's next pair of rows (the last step's four stores may be on their way), LDS
+    if (!TALL && second && t > 3) __builtin_amdgcn_s_waitcnt(0xc07f & (0x0f70 | 4));  // x's next rows (the last step's four stores may be on their way), LDS
     else __builtin_amdgcn_s_waitcnt(0x0070);
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
-    if (t + 2 <= K + 1) {
-      fetch(t + 2, slot_in);
-      slot_in = slot_in == kInBlocks - 1 ? 0 : slot_in + 1;
-    }
+    if constexpr (!TALL) fetch_next(t);
     __builtin_amdgcn_sched_barrier(0);
     if (second && t > 2) result(t - 3);
-    if (second ? t >= 2 && t < K + 2 : t <= K) products();
+    const bool work = second ? t >= 2 && t < K + 2 : t <= K;
+    if constexpr (TALL) {
+      if (second || !work) results_read(t);
+    }
+    if (work) products(t);
     if (!second && t <= K) between(t);
   }
 }
 
 }  // namespace
 
-bool basic_block_applicable(int N, int H, int W) { return W >= 8 && W <= kMostW && H >= 2 && (long long)H * W * 128 < (long long)kOOBb && N < (1 << 20); }
+long long basic_block_steps(int N, int H, int W) {
+  if (W < 24 || W > kMostW || H < 2 || (long long)H * W * 128 >= (long long)kOOBb || N >= (1 << 20)) return 0;
+  return (long long)N * ((H + step_rows(W) - 1) / step_rows(W));
+}
 
 void launch_basic_block(const BasicBlockArgs& g, hipStream_t s) {
-  NNCV_REQUIRE(basic_block_applicable(g.N, g.H, g.W), "basic_block: shape not covered");
+  NNCV_REQUIRE(basic_block_steps(g.N, g.H, g.W) > 0, "basic_block: shape not covered");
+  const int R = step_rows(g.W);
   BlockArgs d{};
   d.in = g.in; d.out = g.out; d.wf1 = g.wf1; d.wf2 = g.wf2; d.scale1 = g.scale1; d.shift1 = g.shift1; d.scale2 = g.scale2; d.shift2 = g.shift2;
-  d.H = g.H; d.W = g.W;
+  d.H = g.H; d.W = g.W; d.R = R;
   int strips = 1;
   double best = 1e30;
-  for (int c = 1; c <= (g.H + 1) / 2; ++c) {
-    const int rows = ((g.H + c - 1) / c + 1) / 2 * 2;
+  for (int c = 1; c <= (g.H + R - 1) / R; ++c) {
+    const int rows = ((g.H + c - 1) / c + R - 1) / R * R;
     if ((c - 1) * rows >= g.H) continue;
-    const double us = std::ceil((double)g.N * c / 256) * (rows / 2 + 5);
+    const double us = std::ceil((double)g.N * c / 256) * (rows / R + 5);
     if (us < best) best = us, strips = c, d.rows = rows;
   }
   d.strips = strips;
   d.inv_row = 1.0f / (float)(row_bytes(g.W) / 16);
-  const int lds = kInBlocks * in_block(g.W) + kMidBlocks * 2 * row_bytes(g.W) + 1024;
+  const int lds = lds_bytes(g.W);
+  const auto kernel = R == 2 ? basic_block_kernel<false> : basic_block_kernel<true>;
   static const bool attr = [] {
-    NNCV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(basic_block_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       kInBlocks * in_block(kMostW) + kMidBlocks * 2 * row_bytes(kMostW) + 1024));
+    for (auto k : {basic_block_kernel<false>, basic_block_kernel<true>})
+      NNCV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     return true;
   }();
   (void)attr;
   const double px = (double)g.N * g.H * g.W;
   ProfScope prof("basic_block<f16,64>", 4.0 * px * 9 * 64 * 64, 2.0 * (2 * px * 64 + 2 * 9 * 64 * 64), s);
-  launch_kernel(basic_block_kernel, dim3((unsigned)(g.N * strips)), dim3(512), lds, s, d);
+  launch_kernel(kernel, dim3((unsigned)(g.N * strips)), dim3(512), lds, s, d);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 

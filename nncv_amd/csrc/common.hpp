@@ -439,7 +439,7 @@ struct BasicBlockArgs {
   const float* scale1; const float* shift1; const float* scale2; const float* shift2;
   int N, H, W;
 };
-bool basic_block_applicable(int N, int H, int W);
+long long basic_block_steps(int N, int H, int W);  // of all images together, 0: not covered
 void launch_basic_block(const BasicBlockArgs& a, hipStream_t s);
 // out[n][f] = mean over HW of act(scale * (wt . in) + shift), fp16 (conv_pool.hip): in [N][HW] pixels of `pix` elements, wt [F][C]
 struct ConvPoolArgs {

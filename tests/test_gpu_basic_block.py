@@ -53,10 +53,10 @@ def _layer(x, parts):
     return y, lambda e: F.conv2d(e, w.abs(), padding=1) * s.abs().view(1, -1, 1, 1), (b.abs() + mean.abs() * s.abs()).view(1, -1, 1, 1)
 
 
-# rows of 44, 56, 57, 63 and 64 pixels; eight and nine rows, odd heights, a strip that ends inside a pair, images in one strip and in many, more
-# workgroups than CUs
+# two rows a step: rows of 44, 56, 57, 63 and 64 pixels; three: 33, 40 and 42; four: 24, 29 and 32 (all of LDS); eight and nine rows, heights that
+# are no whole steps, images in one strip and in many, more workgroups than CUs
 @pytest.mark.parametrize("shape", [(37, 219, 227), (40, 224, 224), (48, 173, 173), (1, 32, 256), (2, 36, 228), (3, 97, 250), (1, 253, 253), (300, 33, 256),
-                                   (7, 180, 240)])
+                                   (7, 180, 240), (60, 130, 129), (37, 219, 160), (70, 91, 168), (103, 77, 96), (300, 35, 115), (65, 125, 128)])
 def test_block(net, shape):
     m, first, second = net
     N, H, W = shape
@@ -79,11 +79,13 @@ def test_block(net, shape):
     assert float(err.norm() / want.norm()) < 2.0 ** -10  # and two roundings, of 2^-11 at most, on the whole
 
 
-def test_not_finite(net):
+@pytest.mark.parametrize("shape", [(3, 99, 256), (70, 99, 160), (90, 99, 128)])
+def test_not_finite(net, shape):
     """What is not a number stays where the convolutions carry it: not beyond a strip, a row's end or an image."""
-    m, first, second = net
-    x = torch.rand((3, 3, 99, 256), generator=torch.Generator().manual_seed(5)) * 2 - 1
-    for n, yy, xx in [(0, 0, 0), (0, 98, 255), (1, 50, 255), (1, 24, 0), (2, 97, 100)]:
+    m, _, _ = net
+    N, H, W = shape
+    x = torch.rand((N, 3, H, W), generator=torch.Generator().manual_seed(5)) * 2 - 1
+    for n, yy, xx in [(0, 0, 0), (0, H - 1, W - 1), (1, 50, W - 1), (1, 24, 0), (2, 97, 100)]:
         x[n, 1, yy, xx] = float("nan")
     xd = x.half().cuda()
     t, _ = _tap(m, xd, 0)
@@ -98,9 +100,9 @@ def test_not_finite(net):
     assert torch.equal(got[keep], clean[keep])
 
 
-@pytest.mark.parametrize("shape", [(36, 224, 224), (64, 172, 172), (8, 224, 260)])
+@pytest.mark.parametrize("shape", [(36, 224, 224), (100, 92, 92), (8, 224, 260), (31, 160, 160)])
 def test_not_taken(net, shape):
-    """Too few rows, rows too short and too long: two launches, as before."""
+    """Too few steps, rows too short and too long: two launches, as before."""
     m, _, _ = net
     _, rep = _tap(m, torch.rand((shape[0], 3, shape[1], shape[2]), device="cuda").half(), 1)
     assert TAG not in rep
