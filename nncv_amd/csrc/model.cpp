@@ -179,16 +179,17 @@ bool ConvLayer::forward_block(const ConvLayer& second, const void* in, int N, in
   // Against the two launches of conv3x3_f16.hip, a whole ResNet-18 pass in microseconds, theirs first:
   //  * 256 images, rows of W: 24 319 against 313, 28 366 against 351, 32 421 against 406, 33 500 against 477, 40 592 against 559, 43 742
   //    against 707, 48 887 against 837, 56 1032 against 976, 64 1440 against 1223.
-  //  * Steps for each CU: a strip pays five beyond its own.  Three and four rows a step (W <= 42): 0.9 of them (32 images of 100x100) 157
-  //    against 158, 1.8 (32 of 160x160) 195 against 195, 2 (64 of 128x128) 202 against 200, 2.6 (48 of 160x160) 248 against 239; two is
-  //    the line.  Two rows: W = 56 1.8 (16 images) 179 against 176, 4.4 (40) 294 against 280, 7 (64) 352 against 333; four is the line, and
-  //    up to 32 images of 224x224 keep the launches they had.  W > 56, where two rows are nearly the 128 slots and the stream form's tile
-  //    of a row is two thirds full: 1 image of 256x256 122 against 118, 8 165 against 155, 16 of 240x240 188 against 185, so any number.
+  //  * Steps for each CU (replayed graphs): a strip pays five beyond its own.  Three and four rows a step (W <= 42): 1.5 of them (64 images of
+  //    96x96) 161 against 158, 2 (64 of 128x128) 187 against 185, 2.6 (48 of 160x160) 223 against 214, and few lose (2 of 128x128 108 against
+  //    114); two is the line.  Two rows: W = 56 0.1 (1 image) 94 against 99, 1.8 (16) 161 against 159, 5.3 (48) 297 against 286; four is the
+  //    line, and up to 32 images of 224x224 keep the launches they had.  W > 56, where two rows are nearly the 128 slots and the stream
+  //    form's tile of a row is two thirds full: 4 images of 256x256 (0.5) 129 against 129, 8 (1) 151 against 141, 16 200 against 179, 8
+  //    of 240x240 (0.9) 139 against 138; one is the line.
   //  * Three and more passes in flight, each workgroup of this kernel with a CU to itself: 64 images of 160x160 (3.5) 670 against 683 for
   //    four passes, 48 of 224x224 (5.3) 642 against 653 for three, 128 of 160x160 (7) 1153 against 1131, 64 of 224x224 (7) 1075 against
   //    1044, 64 of 256x256 (8) 1313 against 1176; six is the line.
   const long long steps = basic_block_steps(N, H, W);
-  if (!steps || steps < 256 * (overlap_hint() >= 3 ? 6 : W <= 42 ? 2 : W <= 56 ? 4 : 0)) return false;
+  if (!steps || steps < 256 * (overlap_hint() >= 3 ? 6 : W <= 42 ? 2 : W <= 56 ? 4 : 1)) return false;
   launch_basic_block(BasicBlockArgs{in, out, wfrag32_.get(), second.wfrag32_.get(), scale_.as<float>(), shift_.as<float>(), second.scale_.as<float>(), second.shift_.as<float>(), N, H, W}, s);
   return true;
 }
