@@ -13,6 +13,8 @@
 //    they fill most of 128 slots: four waves make a step's rows of the first convolution, four the rows of the second one that the steps
 //    before have completed; a step later the next.  Nothing but a strip's first and last row is computed twice.  With two rows a step,
 //    256 images of 128x128 lost 21 us of a pass of 448 to the two launches and 160x160 gained one; with four and three it gains 15 and 32.
+//  * A row of more than 64 pixels is cut into columns of up to 40 (WIDE), each with a pixel of the first convolution and two of x more on
+//    either side: 42 of them three rows a step, 32 four.  64 images of 320x320, a pass: 633 us with two launches a block, 568.
 //  * A wave has 32 filters of its convolution for good, 144 registers of them, and 64 of the 128 slots.  Two waves share a
 //    SIMD, one of each convolution: the second one's begin a step with the results of the step before, the first one's end it with theirs,
 //    so that the matrix pipe has work from one or the other.
@@ -32,7 +34,7 @@ using namespace mt;
 namespace {
 
 constexpr unsigned kOOBb = 0x7fffff00u;  // byte offset beyond any buffer this kernel accepts
-constexpr int kCell = 144, kInBlocks = 5, kMidBlocks = 3, kMostW = 64;
+constexpr int kCell = 144, kInBlocks = 5, kMidBlocks = 3, kMostW = 64, kMostRow = 256;  // slots of a row; pixels of a row (in columns)
 constexpr int kEach = 3;  // load instructions of a wave for a pair of rows, at most
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 __device__ __forceinline__ void fetch16(__amdgpu_buffer_rsrc_t rs, unsigned char* lds, unsigned voffset) {
@@ -41,54 +43,68 @@ __device__ __forceinline__ void fetch16(__amdgpu_buffer_rsrc_t rs, unsigned char
 constexpr int row_bytes(int W) { return (W + 2) * kCell + 224; }                       // = W * 144 modulo 256
 constexpr int in_block(int W, int R) { return (R * row_bytes(W) + 1023) / 1024 * 1024; }  // whole load instructions
 constexpr int step_rows(int W) { return W <= 32 ? 4 : W <= 42 ? 3 : 2; }
-constexpr int lds_bytes(int W) {
-  const int R = step_rows(W);
-  return kInBlocks * in_block(W, R) + kMidBlocks * R * row_bytes(W) + (R == 2 ? 1024 : 0);
+constexpr int lds_bytes(int Wi, int Wo) {  // slots of a row of the first and of the second convolution
+  const int R = step_rows(Wi);
+  return kInBlocks * in_block(Wi, R) + kMidBlocks * R * row_bytes(Wo) + (R == 2 ? 1024 : 0);
 }
-static_assert(lds_bytes(32) <= 160 * 1024 && lds_bytes(42) <= 160 * 1024 && lds_bytes(kMostW) <= 160 * 1024, "LDS of a CU");
+static_assert(lds_bytes(32, 32) <= 160 * 1024 && lds_bytes(42, 42) <= 160 * 1024 && lds_bytes(kMostW, kMostW) <= 160 * 1024, "LDS of a CU");
 static_assert(in_block(32, 4) <= kEach * 8 * 1024 && in_block(42, 3) <= kEach * 8 * 1024 && in_block(kMostW, 2) <= kEach * 8 * 1024, "a step's rows are three instructions a wave");
+
+// columns a row is cut into, their pixels (of the last one at most), slots of a row of the first convolution, rows of a step
+struct Cut { int cols, Wo, Wi, R; };
+Cut cut_of(int W) {
+  if (W <= kMostW) return Cut{1, W, W, step_rows(W)};
+  Cut best{0, 0, 0, 1};
+  for (int c = 2; c <= 8; ++c) {
+    const int Wo = (W + c - 1) / c, R = step_rows(Wo + 2);
+    if (R > 2 && (c - 1) * Wo < W && (!best.cols || c * best.R < best.cols * R)) best = Cut{c, Wo, Wo + 2, R};
+  }
+  return best;
+}
 
 struct BlockArgs {
   const void* in; void* out; const void* wf1; const void* wf2;
   const float* scale1; const float* shift1; const float* scale2; const float* shift2;
-  int H, W, R, strips, rows;  // rows of a step, strips of an image, their rows (whole steps)
+  int H, W, Wi, Wo, R, cols, strips, rows;  // Cut; strips of an image, their rows (whole steps)
   float inv_row;           // 1 / 16-byte units of a row
 };
 
-template <bool TALL>
+template <bool TALL, bool WIDE>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void basic_block_kernel(const BlockArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
-  const int W = a.W, H = a.H, R = TALL ? a.R : 2, rowB = (W + 2) * kCell + 224, inB = (R * rowB + 1023) & ~1023, midB = R * rowB;
+  static_assert(TALL || !WIDE, "columns have three or four rows a step");
+  const int W = a.W, H = a.H, R = TALL ? a.R : 2, Wi = WIDE ? a.Wi : W, Wo = WIDE ? a.Wo : W;
+  const int rowI = (Wi + 2) * kCell + 224, rowM = WIDE ? (Wo + 2) * kCell + 224 : rowI, inB = (R * rowI + 1023) & ~1023, midB = R * rowM;
   const int mid0 = kInBlocks * inB;
   // scale and shift of both, in pieces of 32 channels: behind the rows; TALL: a piece in what is spare behind each of the first eight of them
   auto tab = [&](int piece) __attribute__((always_inline)) {
-    return reinterpret_cast<float*>(smem + mid0 + (TALL ? piece * rowB + (W + 2) * kCell : kMidBlocks * midB + piece * 128));
+    return reinterpret_cast<float*>(smem + mid0 + (TALL ? piece * rowM + (Wo + 2) * kCell : kMidBlocks * midB + piece * 128));
   };
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 31, lh = lane >> 5, second = wave >> 2, fg = wave & 1, half = (wave >> 1) & 1;
-  const int n = blockIdx.x / a.strips, strip = blockIdx.x - n * a.strips;
+  const int part_of = WIDE ? blockIdx.x / a.cols : blockIdx.x, x0 = WIDE ? (blockIdx.x - part_of * a.cols) * Wo : 0;  // first column of the result
+  const int n = part_of / a.strips, strip = part_of - n * a.strips;
   const int y0 = strip * a.rows, y1 = min(y0 + a.rows, H), K = (y1 - y0 + R - 1) / R;  // steps' rows of the result
   const long long image = (long long)n * H * W * 128;
   const __amdgpu_buffer_rsrc_t rs_in = make_rsrc(static_cast<const char*>(a.in) + image, (unsigned)(H * W) * 128u);
   const __amdgpu_buffer_rsrc_t rs_out = make_rsrc(static_cast<char*>(a.out) + image, (unsigned)(H * W) * 128u);
 
   // ---- loader: unit u of a pair of rows is part of a cell, of the spare 16 bytes behind it or of those behind the row ----
-  const int units = rowB >> 4, calls = inB >> 10;
-  unsigned from[kEach];
-  int frow[kEach];
+  const int units = rowI >> 4, calls = inB >> 10;
+  unsigned from[kEach];  // row << 20 | byte behind the first row's start; all ones: zeros
 #pragma unroll
   for (int i = 0; i < kEach; ++i) {
     int v;
     const int u = (i * 8 + wave) * 64 + lane, r = fast_div(u, units, a.inv_row, &v), cell = (v * 7282) >> 16, part = v - cell * 9;
-    const bool ok = r < R && part < 8 && cell >= 1 && cell <= W;
-    from[i] = (unsigned)((r * W + cell - 1) * 128 + part * 16);
-    frow[i] = ok ? r : 1 << 28;
+    const int x = x0 + cell - (WIDE ? 2 : 1);
+    const bool ok = r < R && part < 8 && cell < Wi + 2 && (unsigned)x < (unsigned)W;
+    from[i] = ok ? (unsigned)(r << 20 | ((r * W + x) * 128 + part * 16)) : ~0u;
   }
   auto fetch = [&](int b, int slot) __attribute__((always_inline)) {  // block b of the input: rows y0 - 2 + R b ..
     const int y = y0 - 2 + R * b;
 #pragma unroll
     for (int i = 0; i < kEach; ++i)
-      if (i * 8 + wave < calls) fetch16(rs_in, smem + slot * inB + (i * 8 + wave) * 1024, (unsigned)(y + frow[i]) < (unsigned)H ? (unsigned)(y * W * 128) + from[i] : kOOBb);
+      if (i * 8 + wave < calls) fetch16(rs_in, smem + slot * inB + (i * 8 + wave) * 1024, from[i] != ~0u && (unsigned)(y + (int)(from[i] >> 20)) < (unsigned)H ? (unsigned)(y * W * 128) + (from[i] & 0xfffffu) : kOOBb);
   };
   fetch(0, 0);
   fetch(1, 1);
@@ -107,19 +123,20 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 
   // ---- this lane's two slots: pixel x of row i of the block; slots behind the last pixel read with one 16, 32 .. before them ----
+  const int Ws = WIDE && second ? Wo : Wi;
   int xs[2], is[2];
   bool there[2];
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     int s = (2 * half + u) * 32 + lrow;
-    there[u] = s < R * W;
-    if (s >= R * W) s -= (((s - R * W) >> 4) + 1) << 4;
-    is[u] = s >= W ? 1 : 0;
-    if constexpr (TALL) is[u] += (s >= 2 * W ? 1 : 0) + (s >= 3 * W ? 1 : 0);
-    xs[u] = s - is[u] * W;
+    there[u] = s < R * Ws;
+    if (s >= R * Ws) s -= (((s - R * Ws) >> 4) + 1) << 4;
+    is[u] = s >= Ws ? 1 : 0;
+    if constexpr (TALL) is[u] += (s >= 2 * Ws ? 1 : 0) + (s >= 3 * Ws ? 1 : 0);
+    xs[u] = s - is[u] * Ws;
   }
   // byte of tap (r, 0) of a slot: block t (first convolution: of the input; second: of the rows between) and two rows of the one behind it
-  const int block = second ? midB : inB, ring0 = second ? mid0 : 0, ring_end = ring0 + (second ? kMidBlocks * midB : kInBlocks * inB), ring = ring_end - ring0;
+  const int block = second ? midB : inB, rowB = second ? rowM : rowI, ring0 = second ? mid0 : 0, ring_end = ring0 + (second ? kMidBlocks * midB : kInBlocks * inB), ring = ring_end - ring0;
   int base[3][2];
 #pragma unroll
   for (int r = 0; r < 3; ++r)
@@ -128,6 +145,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       const int j = is[u] + r;
       base[r][u] = ring0 + (j >= R ? block + (j - R) * rowB : j * rowB) + xs[u] * kCell + lh * 16;
     }
+  // A slot's place in 3 bytes.  WIDE: opaque to the compiler, which would keep what follows from it in registers beyond the 256 (14 spilled)
+  unsigned place[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) place[u] = (unsigned)(xs[u] | is[u] << 8 | (there[u] ? 1 << 16 : 0));
+  auto placed = [&](int u) __attribute__((always_inline)) {
+    unsigned v = place[u];
+    if constexpr (WIDE) asm volatile("" : "+v"(v));
+    return v;
+  };
   const int f0 = fg * 32 + 16 * lh;  // this lane's 16 consecutive channels
   const float *sc = tab(second * 4 + fg) + 16 * lh, *sh = tab(second * 4 + 2 + fg) + 16 * lh;
   floatx16 acc[2];
@@ -151,12 +177,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   auto between = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
+      const unsigned v = placed(u);
+      const int x = v & 255, i = v >> 8 & 255;
       float y[16];
       scaled(u, y);
       act_apply_n<true>(y, kActRelu);
-      const bool inside = (unsigned)(y0 - 1 + R * t + is[u]) < (unsigned)H;
-      unsigned char* to = smem + mid0 + slot_mid * midB + is[u] * rowB + (xs[u] + 1) * kCell + f0 * 2;
-      if (there[u]) {
+      const bool inside = (unsigned)(y0 - 1 + R * t + i) < (unsigned)H && (!WIDE || (unsigned)(x0 - 1 + x) < (unsigned)W);
+      unsigned char* to = smem + mid0 + slot_mid * midB + i * rowM + (x + (WIDE ? 0 : 1)) * kCell + f0 * 2;
+      if (v >> 16) {
 #pragma unroll
         for (int c = 0; c < 2; ++c) *reinterpret_cast<u32x4*>(to + 16 * c) = inside ? halves(y, c) : u32x4{0, 0, 0, 0};
       }
@@ -168,20 +196,22 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int next = slot_res == kInBlocks - 1 ? 0 : slot_res + 1;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
+      const unsigned v = placed(u);
+      const int xo = v & 255, i = v >> 8 & 255;
       float y[16];
       scaled(u, y);
-      int xrow = slot_res * inB + is[u] * rowB;
-      if constexpr (TALL) xrow = is[u] + 2 < R ? xrow + 2 * rowB : next * inB + (is[u] + 2 - R) * rowB;
-      const unsigned char* x = smem + xrow + (xs[u] + 1) * kCell + f0 * 2;
+      int xrow = slot_res * inB + i * rowI;
+      if constexpr (TALL) xrow = i + 2 < R ? xrow + 2 * rowI : next * inB + (i + 2 - R) * rowI;
+      const unsigned char* x = smem + xrow + (xo + (WIDE ? 2 : 1)) * kCell + f0 * 2;
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
-        const half8 v = *reinterpret_cast<const half8*>(x + 16 * c);
+        const half8 add = *reinterpret_cast<const half8*>(x + 16 * c);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) y[8 * c + e] += (float)v[e];
+        for (int e = 0; e < 8; ++e) y[8 * c + e] += (float)add[e];
       }
       act_apply_n<true>(y, kActRelu);
-      const int yo = y0 + R * k + is[u];
-      const unsigned o = there[u] && yo < y1 ? (unsigned)((yo * W + xs[u]) * 128 + f0 * 2) : kOOBb;
+      const int yo = y0 + R * k + i;
+      const unsigned o = v >> 16 && yo < y1 && (!WIDE || x0 + xo < W) ? (unsigned)((yo * W + x0 + xo) * 128 + f0 * 2) : kOOBb;
 #pragma unroll
       for (int c = 0; c < 2; ++c) __builtin_amdgcn_raw_buffer_store_b128(halves(y, c), rs_out, o + 16u * c, 0, 0);
     }
@@ -263,37 +293,39 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 }  // namespace
 
 long long basic_block_steps(int N, int H, int W) {
-  if (W < 24 || W > kMostW || H < 2 || (long long)H * W * 128 >= (long long)kOOBb || N >= (1 << 20)) return 0;
-  return (long long)N * ((H + step_rows(W) - 1) / step_rows(W));
+  if (W < 24 || W > kMostRow || H < 2 || (long long)H * W * 128 >= (long long)kOOBb || N >= (1 << 20)) return 0;
+  const Cut c = cut_of(W);
+  return (long long)N * c.cols * ((H + c.R - 1) / c.R);
 }
 
 void launch_basic_block(const BasicBlockArgs& g, hipStream_t s) {
   NNCV_REQUIRE(basic_block_steps(g.N, g.H, g.W) > 0, "basic_block: shape not covered");
-  const int R = step_rows(g.W);
+  const Cut cut = cut_of(g.W);
+  const int R = cut.R;
   BlockArgs d{};
   d.in = g.in; d.out = g.out; d.wf1 = g.wf1; d.wf2 = g.wf2; d.scale1 = g.scale1; d.shift1 = g.shift1; d.scale2 = g.scale2; d.shift2 = g.shift2;
-  d.H = g.H; d.W = g.W; d.R = R;
+  d.H = g.H; d.W = g.W; d.R = R; d.Wi = cut.Wi; d.Wo = cut.Wo; d.cols = cut.cols;
   int strips = 1;
   double best = 1e30;
   for (int c = 1; c <= (g.H + R - 1) / R; ++c) {
     const int rows = ((g.H + c - 1) / c + R - 1) / R * R;
     if ((c - 1) * rows >= g.H) continue;
-    const double us = std::ceil((double)g.N * c / 256) * (rows / R + 5);
+    const double us = std::ceil((double)g.N * cut.cols * c / 256) * (rows / R + 5);
     if (us < best) best = us, strips = c, d.rows = rows;
   }
   d.strips = strips;
-  d.inv_row = 1.0f / (float)(row_bytes(g.W) / 16);
-  const int lds = lds_bytes(g.W);
-  const auto kernel = R == 2 ? basic_block_kernel<false> : basic_block_kernel<true>;
+  d.inv_row = 1.0f / (float)(row_bytes(cut.Wi) / 16);
+  const int lds = lds_bytes(cut.Wi, cut.Wo);
+  const auto kernel = cut.cols > 1 ? basic_block_kernel<true, true> : R == 2 ? basic_block_kernel<false, false> : basic_block_kernel<true, false>;
   static const bool attr = [] {
-    for (auto k : {basic_block_kernel<false>, basic_block_kernel<true>})
+    for (auto k : {basic_block_kernel<false, false>, basic_block_kernel<true, false>, basic_block_kernel<true, true>})
       NNCV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     return true;
   }();
   (void)attr;
   const double px = (double)g.N * g.H * g.W;
   ProfScope prof("basic_block<f16,64>", 4.0 * px * 9 * 64 * 64, 2.0 * (2 * px * 64 + 2 * 9 * 64 * 64), s);
-  launch_kernel(kernel, dim3((unsigned)(g.N * strips)), dim3(512), lds, s, d);
+  launch_kernel(kernel, dim3((unsigned)(g.N * strips * cut.cols)), dim3(512), lds, s, d);
   NNCV_HIP_CHECK(hipGetLastError());
 }
 
