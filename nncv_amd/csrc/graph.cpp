@@ -89,10 +89,16 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
       if (nodes_[k].joins == i) return &nodes_[k];
     return nullptr;
   };
+  // an array of filters; without parameters a placeholder, so that the plan is made for the kernels that a graph with them has
+  static char nothing;
+  auto keep = [&](DeviceBuffer& b, size_t bytes) {
+    if (dry_) b.borrow(&nothing, bytes);
+    else b.reset(bytes, &pool_);
+  };
   // a buffer of node i, with room behind it for the node it joins, or the second half of its joiner's
   auto take = [&](int i, DeviceBuffer Node::*b, size_t bytes) {
-    if (const Node* first = joined_by(i)) (nodes_[i].*b).borrow((first->*b).as<char>() + bytes, bytes);
-    else (nodes_[i].*b).reset(bytes * (nodes_[i].joins >= 0 ? 2 : 1), &pool_);
+    if (const Node* first = dry_ ? nullptr : joined_by(i)) (nodes_[i].*b).borrow((first->*b).as<char>() + bytes, bytes);
+    else keep(nodes_[i].*b, bytes * (nodes_[i].joins >= 0 ? 2 : 1));
   };
 
   auto param = [&](long long off, long long count, const std::string& what) -> const void* {
@@ -143,22 +149,23 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
         Cstored = round_up(op.F, vn);
         const int Cl = logical_[op.in[0]];  // channels the filters really have
         const void* w = param(op.w, (long long)op.F * Cl * op.K * op.K, where + "w");
-        if (dry_) break;
         take(i, &Node::wt, (size_t)Cstored * op.K * op.K * C * es);
-        if (Cstored > op.F) NNCV_HIP_CHECK(hipMemsetAsync(nd.wt.get(), 0, (size_t)Cstored * op.K * op.K * C * es, s));
-        launch_weight_frsc(w, dt, nd.wt.get(), dt, op.F, Cl, op.K, op.K, C, s);
+        if (!dry_) {
+          if (Cstored > op.F) NNCV_HIP_CHECK(hipMemsetAsync(nd.wt.get(), 0, (size_t)Cstored * op.K * op.K * C * es, s));
+          launch_weight_frsc(w, dt, nd.wt.get(), dt, op.F, Cl, op.K, op.K, C, s);
+        }
         pixel[op.out] = pixel[op.in[0]];
         // (1x1: not for single pixels, which are never enough; with the filters of both where two are joined, whole blocks of 64 of the first)
         if (!pixel[op.in[0]] && Cl == C && Cstored == op.F && ((nd.joins < 0 && !nd.joined) || op.F % 64 == 0) && conv_ring_point_serves(dt, nd.joins >= 0 || nd.joined ? 2 * op.F : op.F, op.K * op.K, C, op.stride, op.pad)) {
           take(i, &Node::wfrag, weight_frag1x1_bytes(op.F, C));
-          launch_weight_frag1x1(w, dt, nd.wfrag.get(), dt, op.F, C, s);
+          if (!dry_) launch_weight_frag1x1(w, dt, nd.wfrag.get(), dt, op.F, C, s);
         }
         if (op.K == 3 && (op.stride == 1 || (op.stride == 2 && dt == kF16)) && op.pad == 1 && Cl == C && Cstored == op.F && C % (128 / (int)es) == 0) {
-          nd.wfrag.reset(weight_frag3x3_bytes(dt, op.F, C), &pool_);
-          launch_weight_frag3x3(w, dt, nd.wfrag.get(), dt, op.F, C, s);
+          keep(nd.wfrag, weight_frag3x3_bytes(dt, op.F, C));
+          if (!dry_) launch_weight_frag3x3(w, dt, nd.wfrag.get(), dt, op.F, C, s);
           if (dt == kF16 && op.stride == 1 && C % 64 == 0 && op.F % 32 == 0) {
-            nd.wfrag32.reset(weight_frag32_bytes(op.F, C), &pool_);
-            launch_weight_frag32(w, dt, nd.wfrag32.get(), op.F, C, s);
+            keep(nd.wfrag32, weight_frag32_bytes(op.F, C));
+            if (!dry_) launch_weight_frag32(w, dt, nd.wfrag32.get(), op.F, C, s);
           }
         }
         break;
@@ -167,9 +174,8 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
         NNCV_REQUIRE(op.K == 3 || op.K == 5, where + "K must be 3 or 5");
         NNCV_REQUIRE(op.stride >= 1 && op.pad >= 0, where + "bad geometry");
         const void* w = param(op.w, (long long)C * op.K * op.K, where + "w");
-        if (dry_) break;
-        nd.wt.reset((size_t)C * op.K * op.K * es, &pool_);
-        launch_weight_dw(w, dt, nd.wt.get(), dt, C, op.K, s);
+        keep(nd.wt, (size_t)C * op.K * op.K * es);
+        if (!dry_) launch_weight_dw(w, dt, nd.wt.get(), dt, C, op.K, s);
         break;
       }
       case NNCV_HIP_OP_MAXPOOL:
@@ -278,8 +284,8 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
         const GraphOp& o = ops[i];
         const int Fp = channels_[o.out], S2 = (o.K + (o.pad & 1) + 1) / 2;
         pair_stem_ = i;
+        keep(nodes_[i].wt_pairs, (size_t)Fp * o.K * S2 * 8 * es);
         if (dry_) continue;
-        nodes_[i].wt_pairs.reset((size_t)Fp * o.K * S2 * 8 * es, &pool_);
         launch_weight_pairs(param(o.w, (long long)o.F * c_in_ * o.K * o.K, "pair stem w"), dt, nodes_[i].wt_pairs.get(), o.F, Fp, c_in_,
                             o.K, o.pad, s);
       }
@@ -318,10 +324,10 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
             nodes_[i + 4].add_out < 0 && logical_[pr.out] == channels_[pr.out] && se_project_applicable(1, g.in[0] >= 0 ? channels_[g.in[0]] : 0, ops[i + 1].F, pr.F))
         {
           nodes_[i].projects = i + 4;
-          for (int k = 1; k <= 2 && !dry_; ++k) {
+          for (int k = 1; k <= 2; ++k) {
             Node& f = nodes_[i + k];
-            f.wt_t.reset((size_t)f.op.F * f.C * es, &pool_);
-            launch_transpose_half(f.wt.get(), f.wt_t.get(), f.op.F, f.C, s);
+            keep(f.wt_t, (size_t)f.op.F * f.C * es);
+            if (!dry_) launch_transpose_half(f.wt.get(), f.wt_t.get(), f.op.F, f.C, s);
           }
         }
       }
@@ -330,14 +336,14 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
 
   // The filters in conv_direct.hip's order, for the layers that may run there, and for projections (mobile_block.hip).  The two
   // vectors of a squeeze-excitation block are never convolutions of their own.
-  for (int i = 0; i < n && !dry_; ++i) {
+  for (int i = 0; i < n; ++i) {
     const GraphOp& o = ops[i];
     const bool projection = i >= 4 && nodes_[i - 4].projects == i;
     if (o.kind != NNCV_HIP_OP_CONV || nodes_[i].skip) continue;
     const int C = nodes_[i].C, Fs = channels_[o.out];
     if (!projection && !conv_direct_serves(dt, Fs, o.K * o.K, C)) continue;
-    nodes_[i].wflat.reset(weight_flat_bytes(dt, Fs, o.K * o.K, C), &pool_);
-    launch_weight_flat(blob + (size_t)o.w * es, nodes_[i].wflat.get(), dt, o.F, logical_[o.in[0]], o.K * o.K, C, s);
+    keep(nodes_[i].wflat, weight_flat_bytes(dt, Fs, o.K * o.K, C));
+    if (!dry_) launch_weight_flat(blob + (size_t)o.w * es, nodes_[i].wflat.get(), dt, o.F, logical_[o.in[0]], o.K * o.K, C, s);
   }
 
   // a pointwise convolution that is only averaged: its result need not be stored
@@ -387,9 +393,9 @@ Graph::Graph(const GraphOp* ops, int n, int in_channels, const void* params, lon
     for (int h : made) {
       Node& c = nodes_[std::max(h, 0)];
       c.head = ok;
-      if (!ok || dry_) continue;
-      c.wfrag.reset(weight_frag1x1_bytes(c.op.F, c.C), &pool_);
-      launch_weight_frag1x1(blob + (size_t)c.op.w * es, dt, c.wfrag.get(), dt, c.op.F, c.C, s);
+      if (!ok) continue;
+      keep(c.wfrag, weight_frag1x1_bytes(c.op.F, c.C));
+      if (!dry_) launch_weight_frag1x1(blob + (size_t)c.op.w * es, dt, c.wfrag.get(), dt, c.op.F, c.C, s);
     }
   }
 

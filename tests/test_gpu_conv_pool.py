@@ -28,6 +28,7 @@ def test_means_and_last_layer(case, dt):
     x = synth.normal(8201, (N, 8, H, W))
     if dt == abi.F16:
         blob, x = synth.round_fp16(blob), synth.round_fp16(x)
+    launches = abi.graph_plan(ops, 8, dt, N, H, W)[2]
     g = Graph(ops, 8, blob, dt)
     out = torch.empty(N * O + 1, dtype=torch.float32, device="cuda")  # the caller's tensor at 16 bytes and one float further on
     xd = dev(x, dt)
@@ -48,6 +49,7 @@ def test_means_and_last_layer(case, dt):
             assert tags.get("conv_pool", 0) == int(pool) and tags.get("global_avgpool", 0) == int(not pool), tags
             ends = tags.get("relayout", 0) - int("image_to_nhwc" not in tags)  # (one of them may lay the input out)
             assert (O % 4 == 0 or ends == 1) and (O != 1000 or ends == 0), tags
+            assert (launches[3] == -1) == (ends == 0) and (launches[1] == 3) == (launches[2] == -1) == pool, launches  # the plan is of these launches
     finally:
         abi.profile_enable(False)
         g.close()

@@ -1,6 +1,6 @@
 """A C3 block behind [up-sampled, skip] whose launch reads the tensor of half the size itself (conv_ring.hip) where that can go wrong: with and without the
 chained layer, pixels that end inside a tile, a last slab that is not full, several images, a source that is a slice of a wider tensor; and what must keep
-the copy: another reader, the second place in the concatenation, part of a slab, a launch of other tiles.  Against the oracle's evaluator."""
+the copy: another reader, the second place in the concatenation, part of a slab, launches of other tiles.  Against the oracle's evaluator."""
 import pytest
 
 import oracle
@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 # channels up-sampled, of the skip, c_, N, H, W of the small tensor, what else, whether the copy is saved
 @pytest.mark.parametrize("case", [(128, 128, 64, 3, 41, 37, "", True), (64, 104, 64, 1, 75, 67, "", True), (256, 256, 128, 5, 33, 35, "", True), (64, 200, 128, 3, 59, 45, "", True),
                                   (128, 128, 64, 3, 41, 37, "sliced", True), (128, 128, 64, 3, 41, 37, "reader", False), (128, 128, 64, 3, 41, 37, "second", False),
-                                  (72, 128, 64, 3, 41, 37, "", False), (128, 128, 64, 1, 9, 11, "", False)])
+                                  (72, 128, 64, 3, 41, 37, "", False), (128, 128, 64, 1, 9, 11, "", False), (256, 256, 128, 7, 20, 20, "", False)])
 def test_block_behind_upsampling(case):
     cu, cs, c_, N, H, W, other, saved = case
     sizes, ops = [], []

@@ -102,3 +102,38 @@ def test_merged_bottleneck_result_is_live_from_the_convolution():
     o4, b4 = info[4][1], info[4][2]
     assert o4 + b4 <= o2 or o2 + b2 <= o4, "the merged result shares memory with the convolution's input"
     _check(ops, 8, abi.F16, 4, 40, 40)
+
+
+@pytest.mark.parametrize("dt", [abi.F16, abi.F32])
+@pytest.mark.parametrize("N", [1, 32])
+def test_a_last_layer_that_writes_the_callers_tensor(dt, N):
+    """The plan is that of the launches of a graph with parameters: MobileNetV3's last layer writes the caller's fp32 tensor itself
+    (test_gpu_conv_pool.py counts the launches), so it has no tensor of its own."""
+    ops = mobilenetv3_spec.graph_ops()
+    _, info, dst = abi.graph_plan(ops, 3, dt, N, 224, 224)
+    assert dst[-1] == -1 and info[ops[-1].out][2] == 0
+
+
+@pytest.mark.parametrize("N,joined,saved", [(1, False, False), (14, True, False), (20, True, True)])
+def test_a_folded_up_sampling_depends_on_the_kernel(N, joined, saved):
+    """[up-sampled, skip] of 512 channels in front of two layers of 64 filters: two launches of few tiles, one of the fragment form (350 tiles), which
+    reads one tensor only, and one of the ring (128 x 128), which reads the small one (test_gpu_graph_upsample.py counts the launches)."""
+    ops, off = [], [0]
+
+    def take(n):
+        o = off[0]; off[0] += n; return o
+
+    def conv(i, c, f, k=1, s=1):
+        ops.append(abi.graph_op(abi.OP_CONV, [i, -1], len(ops) + 1, F=f, K=k, stride=s, pad=k // 2, act=abi.ACT_SILU, w=take(f * c * k * k), bias=take(f)))
+        return len(ops)
+
+    skip = conv(0, 8, 256)
+    small = conv(skip, 256, 256, 3, 2)
+    ops.append(abi.graph_op(abi.OP_UPSAMPLE2X, [small], 3, stride=0))
+    ops.append(abi.graph_op(abi.OP_CONCAT, [3, skip], 4, stride=0))
+    a, b = conv(4, 512, 64), conv(4, 512, 64)
+    ops.append(abi.graph_op(abi.OP_CONCAT, [a, b], 7, stride=0))
+    conv(7, 128, 32)
+    dst = abi.graph_plan(ops, 8, abi.F16, N, 40, 40)[2]
+    assert (dst[5] == -1) == joined and (dst[2] == -1) == saved
+    _check(ops, 8, abi.F16, N, 40, 40)
