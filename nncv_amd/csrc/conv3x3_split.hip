@@ -423,9 +423,10 @@ long long flat_bytes(int H, int W) { return ((W + 30) / W + (30ll + H * W) / (H 
 // Tiles of 32 consecutive pixels where every workgroup has a CU to itself; us, back to back, to within 5 % on 20 layers of 128 to 512
 // channels, or 0.  Half the products of a 64-slot tile a workgroup and none for slots without a pixel: 6x8x10x512 -> 512 24.5 -> 17,
 // 55x3x3 25 -> 18.5, 4x15x17x256 -> 256 13 -> 11.4; with more workgroups than CUs a second turn takes as long as the first
-// (3x14x14x384, 36 workgroups on an XCD, 24).
+// (3x14x14x384, 36 workgroups on an XCD, 24).  Every layer of this file that it covers takes it: 50 layers of 192 and 256 channels, which half blocks of a
+// 64-slot tile take 10.5 to 13.4 us for, 8.1 to 11.1.  Layers of fewer channels are conv_direct.hip's at all of these sizes (237 000 of them, by the models).
 double conv3x3_split_flat_us(int N, int H, int W, int C, int F) {
-  if (C % 64 != 0 || F % 64 != 0 || flat_bytes(H, W) > kFlatCells[1] * kCell) return 0;
+  if (C < 192 || C % 64 != 0 || F % 64 != 0 || flat_bytes(H, W) > kFlatCells[1] * kCell) return 0;
   const long long tiles = ((long long)N * H * W + 31) / 32, fblocks = F / 32;
   const bool by_filter = flat_by_filter(C, F);
   const long long on_xcd = by_filter ? tiles * (fblocks / kXcdsP) : (tiles + kXcdsP - 1) / kXcdsP * fblocks;

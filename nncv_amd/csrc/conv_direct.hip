@@ -568,7 +568,9 @@ double other_us(const IgemmArgs& a, int dt, DirectRival rival) {
   static const Fit f16_3x3[] = {{2.7, 0.097, 0.85, 0.0}, {1.5, 0.009, 2.43, 0.10}};
   const int rounds = (a.R * a.S * a.C * (int)dtype_size(dt) + 127) / 128, main_f = a.aux_f0 ? a.aux_f0 : a.F;
   if (rival == kRivalPatch && dt == kF32) {
-    // (from 257 channels: 4x8x10x512 -> 512 24.5 us here, 15.5 there, 2x14x14x384 18.5 and 13.4; at 256 what there is to gain is 1 to 3 us)
+    // From 257 channels at the price of tiles of 32 pixels: 4x8x10x512 -> 512 24.5 us here, 15.5 there, 2x14x14x384 18.5 and 13.4.  Up to 256 at that of
+    // half blocks, more than those tiles take, which run there all the same: what goes there gains, and what stays here could (14.2 against 9.7 to 11.4 at
+    // 256 channels, 11.6 against 8.9 to 10.4 at 192).
     const double flat = a.C > 256 ? conv3x3_split_flat_us(a.N, a.OH, a.OW, a.C, main_f) : 0;
     if (flat > 0) return flat;
     int p[8];

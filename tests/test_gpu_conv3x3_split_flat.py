@@ -1,5 +1,5 @@
 """fp32 3x3 layers in tiles of 32 consecutive pixels (conv3x3_split.hip): tiles that end inside a row, an image, the batch; several images a
-tile; one image of exactly a tile; two slabs and many; the widest rows; against torch in 64 bits, and what is not finite."""
+tile; one image of exactly a tile; six slabs, the fewest, and many; the widest rows; against torch in 64 bits, and what is not finite."""
 import numpy as np
 import pytest
 import torch
@@ -9,7 +9,8 @@ from test_gpu_conv3x3_split import layer_and_reference
 pytestmark = pytest.mark.gpu
 
 CASES = [(6, 512, 512, 8, 10, "flat"), (7, 512, 512, 8, 9, "flat"), (9, 512, 512, 7, 8, "flat"), (20, 448, 448, 5, 5, "flat"),
-         (12, 512, 512, 4, 8, "flat"), (16, 512, 512, 4, 7, "flat"), (3, 448, 512, 10, 16, "flat"), (55, 512, 512, 3, 3, "flat"), (4, 512, 512, 5, 24, "flat")]
+         (12, 512, 512, 4, 8, "flat"), (16, 512, 512, 4, 7, "flat"), (3, 448, 512, 10, 16, "flat"), (55, 512, 512, 3, 3, "flat"), (4, 512, 512, 5, 24, "flat"),
+         (64, 192, 256, 8, 2, "flat"), (3, 192, 512, 7, 24, "flat"), (24, 192, 64, 10, 17, "flat"), (1, 256, 512, 22, 23, "flat"), (12, 256, 512, 14, 3, "flat"), (16, 256, 512, 32, 1, "flat")]
 
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c[:5])))
