@@ -185,6 +185,11 @@ int nncv_hip_conv3x3_patch_plan(int stride, int N, int OH, int OW, int F, int sl
  * bytes of one patch buffer}.  Returns 0, or 1 when the kernel does not take the shape.
  * No counterpart in the reference: it lets the CPU test suite check that a plan never outgrows the kernel's LDS. */
 int nncv_hip_conv3x3_stream_plan(int N, int H, int W, int C, int F, int* plan);
+/* Diagnostic, host arithmetic only: the launch of a down-sampling block's 3x3 stride-2 convolution C -> F and its 1x1 shortcut over N
+ * fp32 images of H x W pixels.  plan[5] = {filters, pixels and K groups of a tile, tiles of the convolution, 1: a workgroup computes its tile's
+ * shortcut filters behind it, 0: they have workgroups of their own}.  Returns 0, or 1 when conv_direct.hip does not take the block.
+ * No counterpart in the reference: both forms have one name in a profile, the test suite tells them apart by this. */
+int nncv_hip_conv_shortcut_plan(int N, int H, int W, int C, int F, int* plan);
 
 /* The reference driver's image preparation and top-1 scan on the device
  * (examples/Res18/main.cpp:38-77 and :103-111).

@@ -908,6 +908,17 @@ int nncv_hip_conv3x3_stream_plan(int N, int H, int W, int C, int F, int* plan) {
   return conv3x3_stream_plan(N, H, W, C, F, plan) ? 0 : 1;
 }
 
+int nncv_hip_conv_shortcut_plan(int N, int H, int W, int C, int F, int* plan) {
+  if (!plan || N < 1 || H < 1 || W < 1 || C < 1 || F < 1) return 1;
+  static char there;  // stands for the filters' arrays, of which only the presence counts
+  IgemmArgs a{};
+  a.in = a.wt = a.wt_flat = a.aux_wt_flat = &there;
+  a.out = a.aux_out = &there;
+  a.N = N; a.H = H; a.W = W; a.C = C; a.F = 2 * F; a.R = a.S = 3; a.OH = (H - 1) / 2 + 1; a.OW = (W - 1) / 2 + 1;
+  a.stride_h = a.stride_w = 2; a.pad_h = a.pad_w = 1; a.relu = kActRelu; a.ldo = a.aux_ldo = a.aux_f0 = F; a.aux_tap = 4; a.batch = 1;
+  return conv_direct_plan(a, kF32, plan) ? 0 : 1;
+}
+
 size_t nncv_hip_profile_report(char* buf, size_t cap) {
   std::string r;
   if (guarded([&] { r = profiler_report(); }) != 0) r = "{}";

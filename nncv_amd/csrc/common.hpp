@@ -281,6 +281,8 @@ bool conv_ring_point_serves(int dt, int F, int RS, int C, int stride, int pad);
 bool conv_direct_serves(int dt, int F, int RS, int Cp);
 bool conv_direct_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 bool conv_direct_wins(const IgemmArgs& a, int dt, DirectRival rival);
+// rows, columns, K groups and number of its tiles, and whether auxiliary filters are computed behind them; false: another kernel's
+bool conv_direct_plan(const IgemmArgs& a, int dt, int* plan);
 // (store_f32: `out` is fp32, whatever dt is, at any float's address)
 void launch_conv_direct(const IgemmArgs& a, int dt, hipStream_t s, bool store_f32 = false);
 size_t weight_flat_bytes(int dt, int F, int RS, int Cp);

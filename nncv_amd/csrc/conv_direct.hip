@@ -428,16 +428,23 @@ __global__ __launch_bounds__(64 * KG) void conv_direct_kernel(const DirectArgs a
   }
 }
 
+// Auxiliary filters, as many as the convolution's own: behind them in the same workgroups where those alone are for most of the CUs;
+// on their own they start late and their pixels come from memory again.  Six images, us: 58x78x64 -> 128 + 128 26.0 -> 21.8,
+// 29x39x128 -> 256 + 256 21.8 -> 19.6, 15x20x256 -> 512 + 512 29.0 -> 19.6.  Whole ResNet-18 passes, never / from 200 tiles on / always: one image of 224x224 144 / 143 / 144,
+// 8 279 / 270 / 268, 16 446 / 432 / 431, 32 760 / 752 / 751, 64 1421 / 1406 / 1405, 128 of 160x160 1445 / 1433 / 1429; between 150 and 199 tiles there is something left
+// (three 214 / 214 / 210, two of 231x309 217 / 216 / 212), below that nothing.
+// (fp32 only; tiles of 32 x 32 over two K groups are no down-sampling block's at any number of pixels, by the models)
+constexpr bool behind_form(size_t es, int rows, int cols, int kg) { return es == 4 && !(rows == 32 && cols == 32 && kg == 2); }
+bool aux_behind(int cpt, int F, int main_f, long long main_tiles) { return cpt % 8 == 0 && F == 2 * main_f && main_tiles >= 200; }
+
 template <typename T, typename OutT, int BT, int TM, int TN, int KG>
 void launch_cfg(DirectArgs d, hipStream_t s) {
+  constexpr bool kBehind = behind_form(sizeof(T), BT * TM, BT * TN, KG);
   constexpr int kBuf = 2 * BT * TN * 128, kPart = TM * TN * BT * BT * 4, lds = KG * (kBuf > kPart || KG == 1 ? kBuf : kPart);
   d.main_tiles = (d.main_f + BT * TM - 1) / (BT * TM);
   d.tiles_f = d.main_tiles + (d.F - d.main_f + BT * TM - 1) / (BT * TM);
   d.tiles_p = (d.P + BT * TN - 1) / (BT * TN);
-  // Auxiliary filters, as many as the convolution's own: behind them in the same workgroups where those alone are for most of the CUs;
-  // on their own they start late and their pixels come from memory again.  Six images, us: 58x78x64 -> 128 + 128 26.0 -> 21.8,
-  // 29x39x128 -> 256 + 256 21.8 -> 19.6, 15x20x256 -> 512 + 512 29.0 -> 19.6.
-  const bool behind = sizeof(T) == 4 && d.cpt % 8 == 0 && d.F == 2 * d.main_f && (long long)d.main_tiles * d.tiles_p >= 200;
+  const bool behind = kBehind && aux_behind(d.cpt, d.F, d.main_f, (long long)d.main_tiles * d.tiles_p);
   if (behind) d.tiles_f = d.main_tiles;
   d.inv_tiles = 1.0f / (float)(d.pixels_first ? d.tiles_p : d.tiles_f);
   auto go = [&](auto kern) {
@@ -462,7 +469,7 @@ void launch_cfg(DirectArgs d, hipStream_t s) {
       return;
     }
   }
-  if constexpr (sizeof(T) == 4) {
+  if constexpr (kBehind) {
     if (behind) {
       go(conv_direct_kernel<T, OutT, BT, TM, TN, KG, true, 1, true>);
       return;
@@ -651,6 +658,17 @@ bool conv_direct_wins(const IgemmArgs& a, int dt, DirectRival rival) {
   // margins cover the fits' errors: the fp16 3x3 stride-1 kernels' times are the least well fitted
   const double margin = dt == kF32 ? (rival == kRivalPatch ? 1.0 : 0.97) : rival == kRivalPatch ? 0.85 : 0.9;
   return us < margin * other_us(a, dt, rival);
+}
+
+bool conv_direct_plan(const IgemmArgs& a, int dt, int* plan) {
+  double us = 0;
+  const Form* f = igemm_takes_direct(a, dt, dt) ? best_form(a, dt, &us) : nullptr;
+  if (!f) return false;
+  const int es = (int)dtype_size(dt), main_f = a.aux_f0 ? a.aux_f0 : a.F;
+  const long long tiles = (long long)((main_f + f->rows - 1) / f->rows) * (((long long)a.N * a.OH * a.OW + f->cols - 1) / f->cols);
+  plan[0] = f->rows; plan[1] = f->cols; plan[2] = f->kg; plan[3] = (int)tiles;
+  plan[4] = behind_form(es, f->rows, f->cols, f->kg) && aux_behind(a.C * es / 16, a.F, main_f, tiles);
+  return true;
 }
 
 void launch_conv_direct(const IgemmArgs& a, int dt, hipStream_t s, bool store_f32) {
