@@ -4,6 +4,7 @@ layers; against torch."""
 import pytest
 import torch
 
+import graph_bound
 import oracle
 from nncv_amd import abi, synth
 from gpu_util import Conv, FP16_REL_L2, Graph, dev, host, nchw, nhwc, rel_l2
@@ -29,6 +30,11 @@ def test_against_torch(N, C, F, H, W, act, point):
         abi.profile_enable(False)
     assert (tags == ["conv_ring<64x128,point>"]) == point, tags
     assert rel_l2(nchw(got), f(torch.nn.functional.conv2d(x, w)).numpy()) < 2e-3 < FP16_REL_L2
+    exact, size = f(torch.nn.functional.conv2d(x.double(), w.double())), torch.nn.functional.conv2d(x.double().abs(), w.double().abs())
+    # every value: half an ulp of it, C additions in fp32 and a few for the activation
+    room = exact.abs() * (2.0 ** -11 + 2.0 ** -20) + 2.0 ** -24 + (C + 4) * 2.0 ** -24 * size
+    err = (torch.from_numpy(nchw(got)).double() - exact).abs()
+    assert (err <= room).all(), float((err / room).max())
 
 
 @pytest.mark.parametrize("c_,N,H,W", [(128, 3, 50, 51), (192, 1, 63, 65), (64, 4, 45, 47)])
@@ -58,4 +64,5 @@ def test_two_joined_layers(c_, N, H, W):
         abi.profile_enable(False)
     assert tags.get("conv_ring<64x128,point>") == 1, tags
     assert rel_l2(got, oracle.run_graph(ops, inp, blob, 16)) < FP16_REL_L2
+    assert graph_bound.worst(got, ops, inp, blob) < graph_bound.LIMIT  # every value
     g.close()

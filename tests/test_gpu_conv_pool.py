@@ -4,6 +4,7 @@ the largest map and the first one beyond it, filter counts that are whole vector
 import pytest
 import torch
 
+import graph_bound
 import oracle
 from nncv_amd import abi, synth
 from gpu_util import FP16_REL_L2, Graph, dev, host, rel_l2
@@ -46,6 +47,7 @@ def test_means_and_last_layer(case, dt):
             got = host(out)[shift:shift + N * O].reshape(want.shape)
             # fp16: three layers of rounded results, as in the other tests of merged layers; fp32: sums of up to 576 terms
             assert rel_l2(got, want) < (3e-3 if dt == abi.F16 else 1e-5) < FP16_REL_L2
+            assert dt == abi.F32 or graph_bound.worst(got.reshape(N, O, 1, 1), ops, x, blob) < graph_bound.LIMIT  # every value
             assert tags.get("conv_pool", 0) == int(pool) and tags.get("global_avgpool", 0) == int(not pool), tags
             ends = tags.get("relayout", 0) - int("image_to_nhwc" not in tags)  # (one of them may lay the input out)
             assert (O % 4 == 0 or ends == 1) and (O != 1000 or ends == 0), tags

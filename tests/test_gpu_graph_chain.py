@@ -3,6 +3,7 @@ go wrong: one slab of channels and several, a slab that is not full, pixels that
 nothing else reads, chains of bottlenecks, rows of a wider tensor, and the first size below the line; against the oracle's evaluator."""
 import pytest
 
+import graph_bound
 import oracle
 from nncv_amd import abi, synth
 from gpu_util import FP16_REL_L2, Graph, dev, host, rel_l2
@@ -50,4 +51,5 @@ def test_chained_layer(case):
     print(case, tags, flush=True)
     assert tags.get("conv_ring<chain>", 0) == int(chained) and (launches[2] == -1) == chained, tags
     assert rel_l2(got, oracle.run_graph(ops, inp, blob, 8)) < FP16_REL_L2
+    assert graph_bound.worst(got, ops, inp, blob) < graph_bound.LIMIT  # every value
     g.close()

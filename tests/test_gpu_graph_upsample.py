@@ -3,6 +3,7 @@ chained layer, pixels that end inside a tile, a last slab that is not full, seve
 the copy: another reader, the second place in the concatenation, part of a slab, launches of other tiles.  Against the oracle's evaluator."""
 import pytest
 
+import graph_bound
 import oracle
 from nncv_amd import abi, synth
 from gpu_util import FP16_REL_L2, Graph, dev, host, rel_l2
@@ -59,4 +60,5 @@ def test_block_behind_upsampling(case):
     assert tags.get("upsample2x", 0) == int(not saved) + int(other == "sliced"), tags
     assert (launches[up - 1] == -1) == saved
     assert rel_l2(got, oracle.run_graph(ops, inp, blob, 8)) < FP16_REL_L2
+    assert graph_bound.worst(got, ops, inp, blob) < graph_bound.LIMIT  # every value
     g.close()

@@ -269,7 +269,7 @@ def test_fp16_fused_stem_nan_and_inf_at_tile_borders(blob):
 @pytest.mark.parametrize("shape", [(1, 3, 32, 32), (3, 3, 33, 47), (2, 3, 225, 223), (1, 3, 330, 70), (33, 3, 64, 64)])
 def test_unusual_sizes_both_types(blob, shape):
     """Smallest image the network accepts, odd and very oblong images, a batch that is not a power of two:
-    the tile planners, the fused stem (even widths only) and its fallback all see shapes they were not tuned for."""
+    the tile planners and the fused stem all see shapes they were not tuned for."""
     x = synth.uniform(3011, shape, 0.0, 1.0)
     print("sizes", shape, flush=True)
     m32 = Model(blob, abi.F32)

@@ -1,6 +1,9 @@
 """The stem kernels (7x7 stride 2 + BN + ReLU + 3x3 stride 2 maximum, stem_pool.hip and stem_pool_split.hip) where their strips and walks
 end: the pooled activation against the same layer in 64 bits."""
 import math
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -96,3 +99,36 @@ def test_fp32_sums_taken_again(net):
     fin = torch.isfinite(want)
     t = _terms(x, parts)
     assert ((got.double() - want.double()).abs()[fin] <= 147 * 2.0 ** -24 * t[fin]).all()
+
+
+SEPARATE = """
+import oracle
+from nncv_amd import abi, synth
+from gpu_util import FP16_REL_L2, FP32_MAX_REL, Model, dev, host, max_rel, rel_l2
+for dt in (abi.F32, abi.F16):
+    half = synth.round_fp16 if dt == abi.F16 else (lambda v: v)
+    blob = half(synth.resnet18_params())
+    m = Model(blob, dt)
+    for shape in [(2, 3, 66, 64), (3, 3, 33, 47)]:
+        x = half(synth.uniform(91, shape, 0.0, 1.0))
+        abi.profile_enable(True)
+        abi.profile_report()
+        got = host(m(dev(x, dt)))
+        tags = list(abi.profile_report())
+        abi.profile_enable(False)
+        assert any(t.startswith("maxpool") for t in tags) and not any(t.startswith("stem_conv7x7_bn_relu_maxpool") for t in tags), tags
+        want = oracle.resnet18_forward(x, blob)
+        err = max_rel(got, want) if dt == abi.F32 else rel_l2(got, want)
+        assert err < (FP32_MAX_REL if dt == abi.F32 else FP16_REL_L2), (dt, shape, err)
+        print(dt, shape, err, flush=True)
+"""
+
+
+def test_the_stem_as_separate_launches():
+    """Packing, implicit GEMM and pool: what images of 2 GB in all and more, beyond the fused kernels' range, still take; here by its switch, which a process
+    reads once."""
+    here = os.path.dirname(os.path.abspath(__file__))
+    env = dict(os.environ, NNCV_HIP_NO_STEM_FUSION="1", PYTHONPATH=os.pathsep.join([here, os.path.dirname(here)]))
+    r = subprocess.run([sys.executable, "-c", SEPARATE], env=env, capture_output=True, text=True, timeout=100)
+    print(r.stdout, flush=True)
+    assert r.returncode == 0, r.stderr[-2000:]
