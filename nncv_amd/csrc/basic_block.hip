@@ -35,7 +35,7 @@ namespace {
 
 constexpr unsigned kOOBb = 0x7fffff00u;  // byte offset beyond any buffer this kernel accepts
 constexpr int kCell = 144, kInBlocks = 5, kMidBlocks = 3, kMostW = 64, kMostRow = 256;  // slots of a row; pixels of a row (in columns)
-constexpr int kEach = 3;  // load instructions of a wave for a pair of rows, at most
+constexpr int kEach = 3;  // load instructions of a wave for a step's rows, at most
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 __device__ __forceinline__ void fetch16(__amdgpu_buffer_rsrc_t rs, unsigned char* lds, unsigned voffset) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)lds, 16, voffset, 0, 0, 0);
@@ -89,7 +89,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const __amdgpu_buffer_rsrc_t rs_in = make_rsrc(static_cast<const char*>(a.in) + image, (unsigned)(H * W) * 128u);
   const __amdgpu_buffer_rsrc_t rs_out = make_rsrc(static_cast<char*>(a.out) + image, (unsigned)(H * W) * 128u);
 
-  // ---- loader: unit u of a pair of rows is part of a cell, of the spare 16 bytes behind it or of those behind the row ----
+  // ---- loader: unit u of a step's rows is part of a cell, of the spare 16 bytes behind it or of those behind the row ----
   const int units = rowI >> 4, calls = inB >> 10;
   unsigned from[kEach];  // row << 20 | byte behind the first row's start; all ones: zeros
 #pragma unroll
@@ -269,7 +269,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
   };
 
-  __builtin_amdgcn_s_waitcnt(0x0f70);  // filters and the first two pairs of rows: waited for where they are used, every step would count them
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // filters and the first two steps' rows: waited for where they are used, every step would count them
   // Step t: the first convolution's block t (t <= K), the second one's block t - 2, and the results of its block t - 3.
   for (int t = 0; t < K + 3; ++t) {
     __builtin_amdgcn_sched_barrier(0);

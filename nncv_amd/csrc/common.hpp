@@ -276,8 +276,6 @@ void launch_image_pairs(const ImagePairsArgs& a, hipStream_t s);
 // that of the kernel which would run the layer otherwise.
 enum DirectRival : int { kRivalPatch = 0, kRivalPatchS2 = 1, kRivalIgemmFast = 2, kRivalIgemm = 3, kRivalShortK = 4, kRivalRing = 5, kRivalNarrow = 6 };
 // whether it is the kernel for a layer of F filters over RS taps of Cp channels at any size (else its order of the filters is not kept)
-// whether a 1x1 layer may run on conv_ring.hip's fragment forms, i.e. reads wt_frag (fp16)
-bool conv_ring_point_serves(int dt, int F, int RS, int C, int stride, int pad);
 bool conv_direct_serves(int dt, int F, int RS, int Cp);
 bool conv_direct_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 bool conv_direct_wins(const IgemmArgs& a, int dt, DirectRival rival);
@@ -294,6 +292,8 @@ void launch_weight_flat(const void* w_fcrs, void* dst, int dt, int F, int C, int
 bool conv3x3_narrow_applicable(const IgemmArgs& a, int in_dt, int out_dt);
 double conv3x3_narrow_us(const IgemmArgs& a);
 void launch_conv3x3_narrow(const IgemmArgs& a, hipStream_t s);
+// whether a 1x1 layer may run on conv_ring.hip's fragment forms, i.e. reads wt_frag (fp16)
+bool conv_ring_point_serves(int dt, int F, int RS, int C, int stride, int pad);
 // whether two 1x1 layers of C channels and F filters each over P pixels should compute the 1x1 layer behind the first one as well
 bool conv_ring_chains(long long P, int C, int F);
 // whether a launch of two such layers, alone or chained, takes its first up_c channels from another tensor (IgemmArgs::up_in)
@@ -483,7 +483,7 @@ struct DetectHeadLevel {
   int HW, W, pix, C, rows; long long box0; float stride; float anchor_wh[8];
   unsigned in_bytes, wt_bytes; int tiles, first, run; float inv_tiles, inv_w;  // filled in by the launcher
 };
-struct DetectHeadArgs { DetectHeadLevel lv[3]; float* out; int levels, N, A, F; long long boxes_total; float inv_f; };
+struct DetectHeadArgs { DetectHeadLevel lv[3]; float* out; int levels, N, A, F; long long boxes_total; };
 bool detect_head_applicable(int A, int F, int C, long long in_bytes);
 void launch_detect_head(const DetectHeadArgs& a, hipStream_t s);
 void launch_cast(const void* src, int src_dt, void* dst, int dst_dt, long long n, hipStream_t s);

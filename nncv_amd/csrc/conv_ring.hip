@@ -758,6 +758,8 @@ bool conv_ring_applicable(const IgemmArgs& a, int in_dt, int out_dt) {
          P * a.ldo * 2 < (long long)kOOBr && ((P + 63) / 64) * ((a.F + 31) / 32) < lim && (a.relu & ~(0xff | kActResidualAfter)) == 0;
 }
 
+bool conv_ring_point_serves(int dt, int F, int RS, int C, int stride, int pad) { return point_serves(dt, F, RS, C, stride, pad); }
+
 // Stride-2 3x3 layers without auxiliary filters leave the patch kernel for the fragment forms from 112 tiles of 64 x 128 on: of 41
 // layers between there and 400 tiles 38 take 0.5 to 0.96 times as long, the others 1.0 (24x19x16x256 -> 512, 120 tiles: 19.9 -> 12.7;
 // 19x31x77x64 -> 192, 372: 9.5 -> 9.1).  Below, its smaller tiles and K groups mostly fill the chip better (6x22x86x256 -> 256, 92
@@ -769,8 +771,6 @@ bool conv_ring_applicable(const IgemmArgs& a, int in_dt, int out_dt) {
 // 150 tiles, is the other way round: 16.5 against 15.1).  Larger launches used to be igemm_fast's: 23 of them take 1.14 to 1.35
 // times as long there (256x28x28x128 -> 256: 52.2 against 42.0).  In a ResNet-18 pass of 256 images the three such layers with
 // their shortcuts went from 78.1 + 58.4 + 52.2 us there to 65.4 + 46.6 + 43.6, the pass from 1162 to 1133 us of launches.
-bool conv_ring_point_serves(int dt, int F, int RS, int C, int stride, int pad) { return point_serves(dt, F, RS, C, stride, pad); }
-
 bool conv_ring_beats_patch_s2(const IgemmArgs& a) {
   const long long P = (long long)a.N * a.OH * a.OW, main_f = a.aux_f0 ? a.aux_f0 : a.F;
   if (a.stride_h == 2 && frag_ok(a) && a.aux_f0 == 0 && a.F > 64 && (P + 63) / 64 * ((main_f + 127) / 128) >= 112) return true;

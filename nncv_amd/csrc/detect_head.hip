@@ -197,7 +197,6 @@ bool detect_head_applicable(int A, int F, int C, long long in_bytes) {
 
 void launch_detect_head(const DetectHeadArgs& a_in, hipStream_t s) {
   DetectHeadArgs a = a_in;
-  a.inv_f = 1.0f / (float)a.F;
   bool vec = (a.boxes_total * a.F) % 4 == 0 && reinterpret_cast<uintptr_t>(a.out) % 16 == 0;
   long long blocks = 0;
   double flops = 0, bytes = 0;
