@@ -231,9 +231,12 @@ void geometry(int OW, int* TW, int* ntx) {
 // Taken where a workgroup has three and a half tiles or more and four fifths of the slots hold a pixel.  us, in the ring and here: 256x56x56 -> 128
 // 57 / 38-47, 128 images 31.4 / 24-28, 16x160x160 31.6 / 25-29, 128x62x62 36.8 / 27-33, 64x56x56 -> 256 24.2 / 22-24; below that many tiles 100x56x56
 // 20.1 / 19.8, 64x56x56 14.7 / 15.6, 8x160x160 14.9 / 16.5; and with 20 of 32 slots 128x58x78 41.6 / 42, 64x58x78 19.0 / 23.3.
+// With passes in flight too, though a workgroup has a CU to itself, ResNet-18: four of 128 images 1853 / 1842, three of 192 2067 / 2044, four of 256 3715 / 3650, three of 64 images of
+// 320x320 1418 / 1423.
 bool conv3x3s2_resident_wins(const IgemmArgs& a) {
+  static const bool off = getenv("NNCV_HIP_NO_S2_RESIDENT") != nullptr;
   const int pix = a.pix_stride ? a.pix_stride : a.C, main_f = a.aux_f0 ? a.aux_f0 : a.F, aux_f = a.F - main_f;
-  if (a.stride_h != 2 || a.stride_w != 2 || a.R != 3 || a.S != 3 || a.pad_h != 1 || a.pad_w != 1 || a.C != 64 || a.residual || !a.wt_frag || a.batch != 1 ||
+  if (off || a.stride_h != 2 || a.stride_w != 2 || a.R != 3 || a.S != 3 || a.pad_h != 1 || a.pad_w != 1 || a.C != 64 || a.residual || !a.wt_frag || a.batch != 1 ||
       a.split_f || a.OH != (a.H - 1) / 2 + 1 || a.OW != (a.W - 1) / 2 + 1 || main_f % 8 != 0 || a.ldo % 8 != 0 || pix % 8 != 0 || (a.relu & ~0xff) ||
       (a.aux_f0 && (!a.aux_wt_frag || a.aux_tap != 4 || aux_f != main_f || a.aux_ldo % 8 != 0 || (a.aux_relu & ~0xff))))
     return false;

@@ -175,7 +175,8 @@ bool ConvLayer::forward_block(const ConvLayer& second, const void* in, int N, in
     return !d.stem && c.algo_ == kAlgoIgemm && d.dt == kF16 && d.C == 64 && d.F == 64 && d.R == 3 && d.S == 3 && d.stride == 1 && d.pad == 1 && d.relu == kActRelu &&
            c.wfrag32_.get() && c.scale_.get();
   };
-  if (!fits(*this) || !fits(second)) return false;
+  static const bool off = getenv("NNCV_HIP_NO_BASIC_BLOCK") != nullptr;
+  if (off || !fits(*this) || !fits(second)) return false;
   // Against the two launches of conv3x3_f16.hip, a whole ResNet-18 pass in microseconds, theirs first:
   //  * 256 images, rows of W: 24 319 against 313, 28 366 against 351, 32 421 against 406, 33 500 against 477, 40 592 against 559, 43 742
   //    against 707, 48 887 against 837, 56 1032 against 976, 64 1440 against 1223;
@@ -183,12 +184,13 @@ bool ConvLayer::forward_block(const ConvLayer& second, const void* in, int N, in
   //  * Steps for each CU (replayed graphs): a strip pays five beyond its own.  Three and four rows a step (W <= 42): 1.5 of them (64 images of
   //    96x96) 161 against 158, 2 (64 of 128x128) 187 against 185, 2.6 (48 of 160x160) 223 against 214, and few lose (2 of 128x128 108 against
   //    114); two is the line.  Two rows: W = 56 0.1 (1 image) 94 against 99, 1.8 (16) 161 against 159, 5.3 (48) 297 against 286; four is the
-  //    line, and up to 32 images of 224x224 keep the launches they had.  W > 56, where two rows are nearly the 128 slots and the stream
+  //    line, and up to 36 images of 224x224 keep the launches they had, though less than all of them need to: 2.2 (20) 195 against 187, 2.6 (24) 199 against 190,
+  //    3.5 (32) 207 against 200, 3.9 (36) 225 against 218.  W > 56, where two rows are nearly the 128 slots and the stream
   //    form's tile of a row is two thirds full: 4 images of 256x256 (0.5) 129 against 129, 8 (1) 151 against 141, 16 200 against 179, 8
   //    of 240x240 (0.9) 139 against 138; one is the line, for rows in columns too: 2 images of 320x320 (0.4) 126 against 128, 4 (0.8) 139 against 139, 8 (1.7)
   //    181 against 172.
   //  * Three and more passes in flight, each workgroup of this kernel with a CU to itself: 64 images of 160x160 (3.5) 670 against 683 for
-  //    four passes, 48 of 224x224 (5.3) 642 against 653 for three, 128 of 160x160 (7) 1153 against 1131, 64 of 224x224 (7) 1075 against
+  //    four passes, 48 of 224x224 (5.3) 642 against 653 for three, 32 (3.5) 448 against 455, for four 585 against 581, 128 of 160x160 (7) 1153 against 1131, 64 of 224x224 (7) 1075 against
   //    1044, 64 of 256x256 (8) 1313 against 1176; 8 of 320x320 (1.7) 411 against 418, 32 (6.8) 1144 against 1088; six is the line.
   const long long steps = basic_block_steps(N, H, W);
   if (!steps || steps < 256 * (overlap_hint() >= 3 ? 6 : W <= 42 ? 2 : W <= 56 ? 4 : 1)) return false;
