@@ -90,7 +90,7 @@ DOMINANT_TRAFFIC = {  # profiles/resnet18_fp16_bs32_hbm_counters.txt, launches w
 
 
 # the same for the launch plan of three or more passes in flight
-IN_FLIGHT_TRAFFIC = {  # profiles/resnet18_fp16_bs32_in_flight_plan_hbm_counters.txt, the layer alone, no residual input
+IN_FLIGHT_TRAFFIC = {  # profiles/resnet18_fp16_bs32_in_flight_plan_hbm_counters.txt, launches without a residual input
     "conv3x3_stream<f16,1x4x1>": (8835 + 6272) * 1024,
 }
 
